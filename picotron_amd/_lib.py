@@ -93,6 +93,23 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The Python extension with the host path of the hot ops (csrc/host.cpp); raises if it was never built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from picotron_amd import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"picotron_amd/_host.so cannot be loaded ({e}): build it first with "
+                               "`python -m picotron_amd.build`") from e
+        _host = module
+    return _host
+
+
 def check(rc: int) -> None:
     """Turn a negative pico_status into the RuntimeError the reference's Python would raise."""
     if rc != 0:

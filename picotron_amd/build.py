@@ -1,9 +1,10 @@
-"""Builds libpicotron_amd.so (the C-ABI library of HIP kernels) in-tree with plain hipcc.
+"""Builds libpicotron_amd.so (the C-ABI library of HIP kernels) and _host.so (the Python extension with the host path of
+the hot ops, linked against it) in-tree.
 
-    python -m picotron_amd.build          # compile every csrc/*.hip for gfx950 and link
+    python -m picotron_amd.build          # compile every csrc/*.hip for gfx950, csrc/host.cpp for the host, and link
 
-hipcc cross-compiles for gfx950 without a GPU present.  The library lands next to this file
-so that it travels with the source tree; nothing is installed into site-packages.
+hipcc cross-compiles for gfx950 without a GPU present.  Both libraries land next to this file
+so that they travel with the source tree; nothing is installed into site-packages.
 """
 from __future__ import annotations
 
@@ -16,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libpicotron_amd.so")
+HOST = os.path.join(HERE, "_host.so")
 
 SOURCES = ["common.hip", "norm.hip", "pointwise.hip", "optim.hip", "loss.hip", "attn_fwd.hip", "attn_bwd.hip"]
 FLAGS = [
@@ -41,6 +43,27 @@ def _run(cmd):
     return out
 
 
+def _compile_host() -> str:
+    """csrc/host.cpp -> build/host.o with the host compiler (it holds no device code) against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import COMMON_HIP_FLAGS, include_paths
+    obj = os.path.join(OBJ, "host.o")
+    includes = [*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    _run(["g++", "-O2", "-std=c++17", *COMMON_HIP_FLAGS, "-DTORCH_EXTENSION_NAME=_host", "-DTORCH_API_INCLUDE_EXTENSION_H",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{d}" for d in includes],
+          "-c", os.path.join(CSRC, "host.cpp"), "-o", obj])
+    return obj
+
+
+def _link_host(obj: str) -> str:
+    from torch.utils.cpp_extension import library_paths
+    dirs = library_paths()
+    return _run(["g++", "-shared", "-o", HOST, obj, *[f"-L{d}" for d in dirs], "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip",
+                 f"-L{HERE}", "-lpicotron_amd", "-Wl,-rpath,$ORIGIN"])
+
+
 def build(verbose: bool = True, extra_flags=()) -> str:
     os.makedirs(OBJ, exist_ok=True)
     hipcc = _hipcc()
@@ -52,13 +75,15 @@ def build(verbose: bool = True, extra_flags=()) -> str:
             print(out)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(compile_one, SOURCES))
-    out = _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+        out = _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+        out += _link_host(host.result())
     if verbose:
         if out.strip():
             print(out)
-        print(f"built {LIB}")
+        print(f"built {LIB} and {HOST}")
     return LIB
 
 

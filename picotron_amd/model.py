@@ -33,8 +33,9 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 import picotron_amd.process_group_manager as pgm
+from picotron_amd import _lib
 from picotron_amd.context_parallel import context_parallel
-from picotron_amd.functional import (FlashAttnFunc, FusedLinearFunc, QKVAttentionFunc, RMSNormFunc, RMSNormResidualFunc,
+from picotron_amd.functional import (FusedLinearFunc, QKVAttentionFunc, RMSNormFunc, RMSNormResidualFunc,
                                      RotaryFunc, SwiGLUFunc, SwiGLUFusedFunc, _fused_rope)
 
 
@@ -60,7 +61,7 @@ def get_cos_sin(seq_length, head_dim, base=500000.0):
 def flash_attention(q, k, v, causal=True):
     """q [B,Hq,S,D], k/v [B,Hkv,S,D] -> [B,S,Hq,D] (the layout flash_attn_func returns, ``model.py:33-37``)."""
     sm_scale = 1.0 / math.sqrt(q.size(-1))
-    return FlashAttnFunc.apply(q, k, v, sm_scale, causal).transpose(1, 2)
+    return _lib.host().flash_attention(q, k, v, sm_scale, causal, False)
 
 
 class TritonRMSNorm(nn.Module):

@@ -16,7 +16,7 @@ from typing import Iterable
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 
 class FusedAdamW:
@@ -31,6 +31,7 @@ class FusedAdamW:
         self.lr, self.betas, self.eps, self.weight_decay = lr, betas, eps, weight_decay
         self.step_count = 0
         self._plans = {}
+        self._whole = None    # the plan over all parameters, once a step has built it
         dev = self.params[0].device
         # every tensor starts on a multiple of 8 elements so that all kernel accesses are 16-byte aligned
         self.offsets, total = [], 0
@@ -96,10 +97,11 @@ class FusedAdamW:
         if self.overlap:
             self.step_count += 1
             self._open = True
+        if set_to_none:
+            _lib.host().zero_grads(self.params)
+            return
         for p in self.params:
-            if set_to_none:
-                p.grad = None
-            elif p.grad is not None:
+            if p.grad is not None:
                 p.grad.zero_()
 
     @torch.no_grad()
@@ -111,10 +113,13 @@ class FusedAdamW:
             self._open = False
             return
         self.step_count += 1
+        hyper = (self.step_count, self.lr, self.betas[0], self.betas[1], self.eps, self.weight_decay, grad_scale)
+        # the common step -- every parameter has a gradient, all of one dtype -- is one native call over the whole list
+        if self._whole is not None and self._whole.step_params(self.params, *hyper):
+            return
         live = tuple(i for i, p in enumerate(self.params) if p.grad is not None)
         if not live:
             return
-        hyper = (self.step_count, self.lr, self.betas[0], self.betas[1], self.eps, self.weight_decay, grad_scale)
         # one launch table per gradient dtype; the tables (everything but the gradients' addresses) are built once per
         # set of live parameters and reused, so the host side of a step stays far below the kernel's own time
         by_dtype = {}
@@ -125,6 +130,9 @@ class FusedAdamW:
             plan = self._plans.get(key)
             if plan is None or any(self.params[i].data_ptr() != ptr for i, ptr in zip(idx, plan.param_ptrs)):
                 plan = self._plans[key] = self._make_plan(idx)
+                # (fp32 parameters beside master weights are copied back below: those steps stay here)
+                if len(idx) == len(self.params) and not (self.master_weights and any(p.dtype == torch.float32 for p in self.params)):
+                    self._whole = plan
             plan.step([self.params[i].grad for i in idx], *hyper)
             if self.master_weights:
                 for i in idx:
