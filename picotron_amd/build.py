@@ -60,7 +60,7 @@ def _compile_host() -> str:
 def _link_host(obj: str) -> str:
     from torch.utils.cpp_extension import library_paths
     dirs = library_paths()
-    return _run(["g++", "-shared", "-o", HOST, obj, *[f"-L{d}" for d in dirs], "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip",
+    return _run(["g++", "-shared", "-o", HOST, obj, *[f"-L{d}" for d in dirs], "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-lhipblaslt",
                  f"-L{HERE}", "-lpicotron_amd", "-Wl,-rpath,$ORIGIN"])
 
 

@@ -6,10 +6,16 @@
 // kernels did.  Here a call is one C++ function: no ctypes conversions, no Python frames in the backward (the autograd
 // thread never takes the GIL), views replaced by pointer + strides.  Nothing is cached from one call to the next.
 #include <torch/extension.h>
+#include <ATen/Context.h>
+#include <ATen/autocast_mode.h>
 #include <c10/hip/HIPStream.h>
+#include <hipblaslt/hipblaslt.h>
 
 #include <array>
+#include <cstdlib>
+#include <mutex>
 #include <optional>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/picotron_amd.h"
@@ -563,7 +569,167 @@ Tensor flash_attention(const Tensor& q, const Tensor& k, const Tensor& v, double
   return FlashAttention::apply(q, k, v, sm_scale, causal, heads_first);
 }
 
-// ------------------------------------------------------------------------------------------------ fused projections
+// ------------------------------------------------------------------------------------------------ projections
+// The model's matrix products are plain library GEMMs (hipBLASLt, the library torch calls too).  torch asks the library's
+// heuristic for an algorithm on every call, which is most of the 25-30 us of host time a product costs there; here the
+// answer is kept with the shape, and a product costs its launch.  At most kMaxPlans shapes are kept; all are dropped when
+// one more is asked for.
+class GemmPlans {
+ public:
+  struct Shape {
+    int64_t device, ta, tb, m, n, k, lda, ldb, ldc;
+    bool operator==(const Shape& o) const {
+      return device == o.device && ta == o.ta && tb == o.tb && m == o.m && n == o.n && k == o.k && lda == o.lda && ldb == o.ldb && ldc == o.ldc;
+    }
+  };
+
+  // column-major C[m,n] = op(A) op(B), bf16 in and out, fp32 accumulation; false: the library has no algorithm for it
+  bool run(const Shape& s, const void* a, const void* b, void* c, const at::TensorOptions& options) {
+    std::lock_guard<std::mutex> lock(mutex_);   // (several host threads may come here with one device's handle)
+    auto it = plans_.find(s);
+    if (it == plans_.end()) {
+      if (plans_.size() >= kMaxPlans) clear();
+      it = plans_.emplace(s, make(s)).first;
+    }
+    const Plan& p = it->second;
+    if (!p.usable) return false;
+    Tensor ws;   // (from torch's allocator: reused in stream order, safe with several streams)
+    if (p.ws_bytes) ws = at::empty({static_cast<int64_t>(p.ws_bytes)}, options.dtype(at::kByte));
+    const float one = 1.f, zero = 0.f;
+    const auto rc = hipblasLtMatmul(handles_[s.device], p.desc, &one, a, p.a, b, p.b, &zero, c, p.c, c, p.c, &p.algo, ptr(ws), p.ws_bytes,
+                                    c10::hip::getCurrentHIPStream().stream());
+    TORCH_CHECK(rc == HIPBLAS_STATUS_SUCCESS, "hipblasLtMatmul failed with status ", static_cast<int>(rc));
+    return true;
+  }
+
+ private:
+  static constexpr size_t kMaxPlans = 1024;
+  static constexpr uint64_t kMaxWorkspace = 76ull << 20;
+  struct Plan {
+    hipblasLtMatmulDesc_t desc = nullptr;
+    hipblasLtMatrixLayout_t a = nullptr, b = nullptr, c = nullptr;
+    hipblasLtMatmulAlgo_t algo = {};
+    size_t ws_bytes = 0;
+    bool usable = false;
+  };
+  struct Hash {
+    size_t operator()(const Shape& s) const {
+      uint64_t h = 1469598103934665603ull;
+      for (int64_t v : {s.device, s.ta, s.tb, s.m, s.n, s.k, s.lda, s.ldb, s.ldc}) h = (h ^ static_cast<uint64_t>(v)) * 1099511628211ull;
+      return static_cast<size_t>(h ^ (h >> 29));
+    }
+  };
+
+  static void ok(hipblasStatus_t rc, const char* what) {
+    TORCH_CHECK(rc == HIPBLAS_STATUS_SUCCESS, what, " failed with status ", static_cast<int>(rc));
+  }
+  Plan make(const Shape& s) {
+    auto& handle = handles_[s.device];
+    if (!handle) ok(hipblasLtCreate(&handle), "hipblasLtCreate");
+    Plan p;
+    ok(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F), "hipblasLtMatmulDescCreate");
+    const int32_t op_a = s.ta ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_b = s.tb ? HIPBLAS_OP_T : HIPBLAS_OP_N;
+    ok(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &op_a, sizeof op_a), "TRANSA");
+    ok(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSB, &op_b, sizeof op_b), "TRANSB");
+    ok(hipblasLtMatrixLayoutCreate(&p.a, HIP_R_16BF, s.ta ? s.k : s.m, s.ta ? s.m : s.k, s.lda), "layout A");
+    ok(hipblasLtMatrixLayoutCreate(&p.b, HIP_R_16BF, s.tb ? s.n : s.k, s.tb ? s.k : s.n, s.ldb), "layout B");
+    ok(hipblasLtMatrixLayoutCreate(&p.c, HIP_R_16BF, s.m, s.n, s.ldc), "layout C");
+    hipblasLtMatmulPreference_t pref = nullptr;
+    ok(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
+    const uint64_t ws = kMaxWorkspace;
+    ok(hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof ws), "workspace preference");
+    hipblasLtMatmulHeuristicResult_t best = {};
+    int found = 0;
+    const auto rc = hipblasLtMatmulAlgoGetHeuristic(handle, p.desc, p.a, p.b, p.c, p.c, pref, 1, &best, &found);
+    hipblasLtMatmulPreferenceDestroy(pref);
+    if (rc == HIPBLAS_STATUS_SUCCESS && found > 0) {
+      p.algo = best.algo;
+      p.ws_bytes = best.workspaceSize;
+      p.usable = true;
+    }
+    return p;
+  }
+  void clear() {
+    for (auto& [shape, p] : plans_) {
+      hipblasLtMatrixLayoutDestroy(p.a);
+      hipblasLtMatrixLayoutDestroy(p.b);
+      hipblasLtMatrixLayoutDestroy(p.c);
+      hipblasLtMatmulDescDestroy(p.desc);
+    }
+    plans_.clear();
+  }
+
+  std::mutex mutex_;
+  std::unordered_map<int64_t, hipblasLtHandle_t> handles_;   // per device, kept until the process ends
+  std::unordered_map<Shape, Plan, Hash> plans_;
+};
+
+GemmPlans& gemm_plans() {
+  static GemmPlans* plans = new GemmPlans;   // never destroyed: the library may be gone before static destructors run
+  return *plans;
+}
+
+// The product is one for the plans above: bf16 on the GPU, rows of one pitch, 16-byte aligned, and no torch setting asks for
+// another route (autocast, another BLAS backend, TunableOp; PICO_TORCH_GEMM=1 sends every product through torch).
+bool torch_gemm_only() {
+  static const bool v = [] {
+    auto on = [](const char* name) { const char* e = std::getenv(name); return e && std::string(e) == "1"; };
+    return on("PICO_TORCH_GEMM") || on("PYTORCH_TUNABLEOP_ENABLED");
+  }();
+  return v || at::autocast::is_autocast_enabled(at::kCUDA) ||
+         (at::globalContext().blasPreferredBackend() != at::BlasBackend::Default &&
+          at::globalContext().blasPreferredBackend() != at::BlasBackend::Cublaslt);
+}
+bool plain(const Tensor& t) {
+  return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) &&
+         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.numel() > 0;
+}
+Tensor matrix(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
+
+// row-major products: a @ b^T, a @ b, a^T @ b
+enum class Product { NT, NN, TN };
+Tensor product(const Tensor& a, const Tensor& b, Product kind) {
+  if (plain(a) && plain(b) && !torch_gemm_only()) {
+    // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
+    const int64_t M = kind == Product::TN ? a.size(1) : a.size(0), K = kind == Product::TN ? a.size(0) : a.size(1);
+    const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
+    TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
+    Tensor c = at::empty({M, N}, a.options());
+    const GemmPlans::Shape s = {a.device().index(), kind == Product::NT, kind == Product::TN, N, M, K, b.stride(0), a.stride(0), N};
+    if (gemm_plans().run(s, b.data_ptr(), a.data_ptr(), c.data_ptr(), a.options())) return c;
+  }
+  return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
+}
+
+Tensor linear_forward(const Tensor& x, const Tensor& w) {
+  if (x.dim() < 1 || w.dim() != 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || torch_gemm_only()) return at::linear(x, w);
+  const Tensor y = product(matrix(x), w, Product::NT);
+  if (x.dim() == 2) return y;
+  auto sizes = x.sizes().vec();
+  sizes.back() = w.size(0);
+  return y.view(sizes);
+}
+
+// y = x @ w^T
+struct Linear : torch::autograd::Function<Linear> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    ctx->save_for_backward({x, w});
+    return linear_forward(x, w);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const auto s = ctx->get_saved_variables();
+    const Tensor dy = matrix(g[0]);
+    variable_list r(2);
+    if (ctx->needs_input_grad(0)) r[0] = product(dy, s[1], Product::NN).view(s[0].sizes());
+    if (ctx->needs_input_grad(1)) r[1] = product(dy, matrix(s[0]), Product::TN);
+    return r;
+  }
+};
+Tensor linear(const Tensor& x, const Tensor& w) {
+  if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || torch_gemm_only()) return at::linear(x, w);
+  return records({&x, &w}) ? Linear::apply(x, w) : linear_forward(x, w);
+}
+
 // y = x @ w^T where w is the buffer that the Parameters `parts` (rows of it, in order) alias; one GEMM for all outputs, one
 // for all weight gradients, one for the summed input gradient.
 struct FusedLinear : torch::autograd::Function<FusedLinear> {
@@ -572,19 +738,19 @@ struct FusedLinear : torch::autograd::Function<FusedLinear> {
     std::vector<int64_t> rows;
     for (const Tensor& p : parts) rows.push_back(p.size(0));
     ctx->saved_data["rows"] = rows;
-    return at::linear(x, w);
+    return linear_forward(x, w);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const auto s = ctx->get_saved_variables();
     const Tensor &x = s[0], &w = s[1];
     const auto rows = ctx->saved_data["rows"].toIntVector();
-    const Tensor dy = g[0].reshape({-1, g[0].size(-1)});
+    const Tensor dy = matrix(g[0]);
     variable_list r(2 + rows.size());
-    if (ctx->needs_input_grad(0)) r[0] = at::mm(dy, w).view(x.sizes());
+    if (ctx->needs_input_grad(0)) r[0] = product(dy, w, Product::NN).view(x.sizes());
     bool any = false;
     for (size_t i = 0; i < rows.size(); ++i) any |= ctx->needs_input_grad(2 + i);
     if (any) {
-      const Tensor dw = at::mm(dy.t(), x.reshape({-1, x.size(-1)}));
+      const Tensor dw = product(dy, matrix(x), Product::TN);
       int64_t at_row = 0;
       for (size_t i = 0; i < rows.size(); ++i, at_row += rows[i - 1]) r[2 + i] = dw.narrow(0, at_row, rows[i]);
     }
@@ -593,7 +759,7 @@ struct FusedLinear : torch::autograd::Function<FusedLinear> {
 };
 
 Tensor fused_linear(const Tensor& x, const Tensor& w, const std::vector<Tensor>& parts) {
-  if (!at::GradMode::is_enabled()) return at::linear(x, w);
+  if (!at::GradMode::is_enabled()) return linear_forward(x, w);
   return FusedLinear::apply(x, w, at::TensorList(parts));
 }
 
@@ -853,6 +1019,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_fwd", &attn_fwd, nogil());
   m.def("attn_bwd", &attn_bwd, nogil());
   m.def("flash_attention", &flash_attention, nogil());
+  m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("qkv_attention", &qkv_attention, nogil());
   m.def("cross_entropy_fwd", &cross_entropy_fwd, nogil());

@@ -161,6 +161,13 @@ def _fused_weight(owner, name, linears):
     return buf
 
 
+class Linear(nn.Linear):
+    """nn.Linear without a bias on the native host path (the same library product, its algorithm kept with the shape)."""
+
+    def forward(self, x):
+        return _lib.host().linear(x, self.weight)
+
+
 def _fan_in_uniform_(tensor):
     bound = math.sqrt(1 / tensor.size(1))
     torch.nn.init.uniform_(tensor, -bound, bound)
@@ -179,10 +186,10 @@ class Attention(nn.Module):
         self.num_local_heads = config.num_attention_heads // mgr.tp_world_size
         self.num_local_kv_heads = config.num_key_value_heads // mgr.tp_world_size
 
-        self.q_proj = nn.Linear(config.hidden_size, self.num_heads * self.head_dim, bias=False)
-        self.k_proj = nn.Linear(config.hidden_size, self.num_key_values * self.head_dim, bias=False)
-        self.v_proj = nn.Linear(config.hidden_size, self.num_key_values * self.head_dim, bias=False)
-        self.out_proj = nn.Linear(config.hidden_size, config.hidden_size, bias=False)
+        self.q_proj = Linear(config.hidden_size, self.num_heads * self.head_dim, bias=False)
+        self.k_proj = Linear(config.hidden_size, self.num_key_values * self.head_dim, bias=False)
+        self.v_proj = Linear(config.hidden_size, self.num_key_values * self.head_dim, bias=False)
+        self.out_proj = Linear(config.hidden_size, config.hidden_size, bias=False)
         self.layer_idx = layer_idx
         self.reset_parameters()
 
@@ -239,9 +246,9 @@ class Attention(nn.Module):
 class MLP(nn.Module):
     def __init__(self, config) -> None:
         super().__init__()
-        self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
-        self.gate_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
-        self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
+        self.up_proj = Linear(config.hidden_size, config.intermediate_size, bias=False)
+        self.gate_proj = Linear(config.hidden_size, config.intermediate_size, bias=False)
+        self.down_proj = Linear(config.intermediate_size, config.hidden_size, bias=False)
         self.reset_parameters()
 
     def reset_parameters(self):
@@ -273,7 +280,7 @@ class FinalProjection(nn.Module):
             torch.nn.init.uniform_(self.bias, -bound_b, bound_b)
 
     def forward(self, x):
-        return F.linear(x, self.weight, self.bias)
+        return _lib.host().linear(x, self.weight) if self.bias is None else F.linear(x, self.weight, self.bias)
 
 
 class DecoderLayer(nn.Module):
