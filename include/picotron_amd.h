@@ -319,6 +319,21 @@ int pico_cross_entropy_fwd(const void* logits, const int64_t* targets, float* lo
 int pico_cross_entropy_bwd(const void* logits, const int64_t* targets, const float* lse, const float* scale,
                            void* dlogits, int64_t rows, int64_t vocab, int64_t ld, int64_t dld, int64_t ignore_index,
                            int dtype, void* stream);
+/* The mean over the rows that count (F.cross_entropy's reduction='mean') with its gradient, without torch reductions in
+ * between.  Forward: loss / lse per row as above, mean[0] and inv_count[0] = 1 / max(rows that count, 1) (device floats).
+ * With dlogits (pitch dld; allowed where pico_cross_entropy_one_pass(vocab, dtype) is 1: bf16 rows of up to 131072
+ * entries, fp32 of up to 65536) the gradient for an upstream gradient of 1 is written in the same pass, the logits are
+ * read once, and a row that does not count gets lse = 0.  Backward: dlogits of the upstream gradient grad_out[0] (device
+ * float); with have_unit != 0 dlogits holds the forward's gradient already and is left as it is where grad_out[0] is 1
+ * (decided on the device, no synchronisation) and recomputed from the logits otherwise.
+ */
+int pico_cross_entropy_one_pass(int64_t vocab, int dtype);
+int pico_cross_entropy_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
+                                float* inv_count, void* dlogits, int64_t rows, int64_t vocab, int64_t ld, int64_t dld,
+                                int64_t ignore_index, int dtype, void* stream);
+int pico_cross_entropy_mean_bwd(const void* logits, const int64_t* targets, const float* lse, const float* inv_count,
+                                const float* grad_out, void* dlogits, int have_unit, int64_t rows, int64_t vocab, int64_t ld,
+                                int64_t dld, int64_t ignore_index, int dtype, void* stream);
 
 /* ------------------------------------------------------------------ optimizer step
  * replaces: torch.optim.AdamW(model.parameters(), lr).step()  train.py:204-209,240  for low-precision parameters

@@ -52,13 +52,15 @@ class FlashAttnFunc:
         return _lib.host().flash_attention(q, k, v, sm_scale, causal, True)
 
 
-class CrossEntropyFunc(torch.autograd.Function):
-    """Mean cross-entropy of [rows, vocab] logits against int64 targets (``train.py:46-49``), fp32 loss.
-    The backward writes dlogits in the dtype of the logits in one pass; the upstream gradient and the 1 / count
-    factor reach the kernel through a device scalar, so nothing synchronises with the host."""
+class CrossEntropyFunc:
+    """``apply(logits, targets, ignore_index)``: mean cross-entropy of [rows, vocab] logits against int64 targets
+    (``train.py:46-49``), fp32 loss.  The gradient leaves in the dtype of the logits; the upstream gradient and the
+    1 / count factor reach the kernels through device scalars, so nothing synchronises with the host.  Where a gradient
+    will be wanted the forward already writes the gradient for an upstream gradient of 1 (one pass over the logits instead
+    of two), so that buffer, as large as the logits, lives from the forward to the backward."""
 
     @staticmethod
-    def forward(ctx, logits, targets, ignore_index=-100):
+    def apply(logits, targets, ignore_index=-100):
         if os.getenv("PICO_CHECK_TARGETS", "0") == "1":
             # F.cross_entropy asserts on the device for a target outside [0, vocab) (train.py:46-49); the kernels skip such
             # a row instead (they may not index with it), which would hide a tokenizer / vocabulary mismatch.  This
@@ -67,18 +69,7 @@ class CrossEntropyFunc(torch.autograd.Function):
             if bool(bad.any()):
                 raise RuntimeError(f"cross_entropy: {int(bad.sum())} targets lie outside [0, {logits.size(-1)}) and are not "
                                    f"ignore_index={ignore_index}")
-        loss_rows, lse = ops.cross_entropy_fwd(logits, targets, ignore_index)
-        # rows that count: not ignored and a valid index (the kernels skip a target outside [0, vocab) as well)
-        count = ((targets != ignore_index) & (targets >= 0) & (targets < logits.size(-1))).sum().clamp(min=1).to(torch.float32)
-        ctx.save_for_backward(logits, targets, lse, count)
-        ctx.ignore_index = ignore_index
-        return loss_rows.sum() / count
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        logits, targets, lse, count = ctx.saved_tensors
-        scale = (grad_out.to(torch.float32) / count).reshape(1)
-        return ops.cross_entropy_bwd(logits, targets, lse, scale, ctx.ignore_index), None, None
+        return _lib.host().cross_entropy(logits, targets, ignore_index)
 
 
 def cross_entropy(logits, targets, ignore_index: int = -100):
