@@ -26,7 +26,7 @@ from typing import Any, Optional, Tuple
 import torch
 
 import picotron_amd.process_group_manager as pgm
-from picotron_amd import ops
+from picotron_amd import _lib, ops
 from picotron_amd.context_parallel.cp_communications import ContextCommunicate
 
 
@@ -107,10 +107,35 @@ def publish_chunk(ring, slot, rank, k, v, rope=None):
     chunk = ring.publish_kv(slot, rank, k, v)
     if chunk.k is chunk.src_k:
         if torch.is_grad_enabled() and (k.requires_grad or v.requires_grad):
-            chunk.k, chunk.v = _PublishKV.apply(k, v, chunk.grads, rope)
+            if k.is_cuda:
+                chunk.k, chunk.v = _lib.host().publish_kv(k, v, chunk.grads, rope[:2] if rope is not None else None, rope[2] if rope is not None else 0)
+            else:
+                chunk.k, chunk.v = _PublishKV.apply(k, v, chunk.grads, rope)
         elif rope is not None:
             chunk.k = ops.rope(k, rope[0], rope[1], pos_offset=rope[2])
     return chunk
+
+
+def _one_run(order, rank: int, is_causal: bool) -> bool:
+    """True if the chunks `order` (sorted ranks) follow each other without a gap -- up to the rank's own under a mask."""
+    return order[-1] - order[0] + 1 == len(order) and (not is_causal or order[-1] == rank)
+
+
+def _one_launch(q, chunks, sm_scale, is_causal, q_offset, rope):
+    """All ring steps of a rank on the GPU: one launch over the chunk list and one native autograd node (``RingAttention``
+    in ``csrc/host.cpp``) whose backward is one launch pair and does the bookkeeping of the chunks' sums.  None if the
+    chunks do not fit one launch."""
+    ks, vs = [c.k for c in chunks], [c.v for c in chunks]
+    if not ops.chunks_fit_one_launch(ks, vs):
+        return None
+    cs, q_pos = (rope[:2], rope[2]) if rope is not None else (None, 0)
+    records = torch.is_grad_enabled() and (q.requires_grad or any(t.requires_grad for t in ks + vs))
+    out, lse, q_rot = ops.attn_fwd_chunks(q, ks, vs, sm_scale, is_causal, q_offset, out_dtype=q.dtype, bshd_out=True, rope=cs,
+                                          q_pos_offset=q_pos, want_q_rot=records, checked=True)
+    if not records:
+        return out
+    return _lib.host().ring_node(q, ks, vs, out, lse, q_rot, [c.grads for c in chunks], sm_scale, is_causal, q_offset, cs, q_pos,
+                                 q_pos - q_offset if is_causal else 0)
 
 
 class RingAttentionFunc(torch.autograd.Function):
@@ -123,7 +148,8 @@ class RingAttentionFunc(torch.autograd.Function):
     All chunks a rank will read are at hand when its turn comes, so by default the loop over the ring steps
     (:30-45, :63-106) runs INSIDE one launch per direction: the kernels take the list of chunk tensors as it is (no
     concatenation, no hop copies), carry the online softmax across the chunks, write the output in q's dtype and add
-    each chunk's dK / dV block to that chunk's accumulator.  Chunks that do not fit one launch (see
+    each chunk's dK / dV block to that chunk's accumulator; on the GPU its autograd node is native (``_one_launch``), the
+    Python form of the same below serves the other devices.  Chunks that do not fit one launch (see
     ``ops.chunks_fit_one_launch``), or ``PICO_RING_PER_STEP=1``, take the reference's shape: one launch per ring step
     with the hop between steps."""
 
@@ -142,12 +168,17 @@ class RingAttentionFunc(torch.autograd.Function):
         for _, held, runs, _ in ring_schedule(world, rank, is_causal):
             if runs and held != rank:
                 chunks[held] = ring.fetch(slot, held, rank)
-        peers = [c for c in sorted(chunks) if c != rank]
+        order = sorted(chunks)
+        peers = [c for c in order if c != rank]
         flat = [t for c in peers for t in (chunks[c].k, chunks[c].v)]
         if torch.is_grad_enabled():
             for c in chunks.values():
                 if c.k.requires_grad or c.v.requires_grad:
                     c.grads.readers += 1
+        if q.is_cuda and not _per_step() and _one_run(order, rank, is_causal):
+            out = _one_launch(q, [chunks[c] for c in order], sm_scale, is_causal, (rank - order[0]) * Sc if is_causal else 0, table)
+            if out is not None:
+                return out
         return super().apply(q, own.k, own.v, sm_scale, is_causal, (slot, rank, world, chunks, peers), table, *flat)
 
     @staticmethod
@@ -172,8 +203,7 @@ class RingAttentionFunc(torch.autograd.Function):
         order = sorted(held for _, held, runs, _ in schedule if runs)
         ks = [k if c == rank else chunks[c].k.detach() for c in order]
         vs = [v if c == rank else chunks[c].v.detach() for c in order]
-        contiguous_positions = order == list(range(order[0], order[0] + len(order))) and (not is_causal or order[-1] == rank)
-        if not _per_step() and contiguous_positions and ops.chunks_fit_one_launch(ks, vs):
+        if not _per_step() and _one_run(order, rank, is_causal) and ops.chunks_fit_one_launch(ks, vs):
             q_off = (rank - order[0]) * Sq if is_causal else 0
             out, lse, q_rot = ops.attn_fwd_chunks(q, ks, vs, sm_scale, is_causal, q_off, out_dtype=q.dtype, bshd_out=True,
                                                   rope=cs, q_pos_offset=q_pos, want_q_rot=rope is not None, checked=True)

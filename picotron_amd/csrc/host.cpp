@@ -383,6 +383,7 @@ std::tuple<Tensor, Tensor, OptTensor> attn_fwd(const Tensor& q_in, std::vector<T
                                                bool causal, int64_t q_offset, const OptTensor& out_in, const OptTensor& lse_in, bool merge,
                                                at::ScalarType out_dtype, bool bshd_out, const Rope& rope, int64_t q_pos_offset,
                                                bool want_q_rot, const OptTensor& q_rot_in) {
+  const at::NoGradGuard no_grad;
   on_gpu(q_in);
   on_gpu(out_in);
   on_gpu(lse_in);
@@ -441,6 +442,7 @@ Tensor attn_bwd(const Tensor& dout_in, const Tensor& q_in, std::vector<Tensor> k
                 double sm_scale, bool causal, int64_t q_offset, const OptTensor& dq, const OptTensors& dks, const OptTensors& dvs,
                 bool dq_accumulate, const std::vector<bool>& dkv_accumulate, const OptTensor& out_in, const OptTensor& delta_in,
                 const Rope& rope, int64_t q_pos_offset, int64_t k_pos_offset, const OptTensors& dk_finals, const OptTensors& dv_finals) {
+  const at::NoGradGuard no_grad;
   on_gpu(dout_in);
   on_gpu(q_in);
   on_gpu(lse_in);
@@ -567,6 +569,191 @@ struct FlashAttention : torch::autograd::Function<FlashAttention> {
 Tensor flash_attention(const Tensor& q, const Tensor& k, const Tensor& v, double sm_scale, bool causal, bool heads_first) {
   on_gpu(q);
   return FlashAttention::apply(q, k, v, sm_scale, causal, heads_first);
+}
+
+// ------------------------------------------------------------------------------------------------ ring attention
+// The autograd nodes of ring attention over virtual ranks (context_parallel.py) where all ring steps of a rank are one
+// launch.  The Python objects they share -- one GradBox per published chunk -- belong to the mailbox; they are touched with
+// the GIL held, the kernels are launched without it.
+struct PyHeld : torch::CustomClassHolder {
+  std::vector<PyObject*> objects;   // strong references
+  explicit PyHeld(const std::vector<pybind11::object>& os) {
+    for (const auto& o : os) objects.push_back(pybind11::object(o).release().ptr());
+  }
+  ~PyHeld() override {
+    pybind11::gil_scoped_acquire gil;
+    for (PyObject* o : objects) Py_DECREF(o);
+  }
+};
+OptTensor tensor_attr(const pybind11::handle& o, const char* name) {
+  pybind11::object v = o.attr(name);
+  return v.is_none() ? std::nullopt : OptTensor(v.cast<Tensor>());
+}
+void set_attr(const pybind11::handle& o, const char* name, const OptTensor& t) { o.attr(name) = t ? pybind11::cast(*t) : pybind11::none(); }
+
+// the gradient of a chunk leaves in the chunk's own layout where that is dense with a unit last stride (as k and v share it)
+bool dense_layout(const Tensor& t) { return t.stride(-1) == 1 && t.is_non_overlapping_and_dense(); }
+
+Tensor convert_sum(const Tensor& src, at::ScalarType dtype, bool dense, at::IntArrayRef strides) {
+  Tensor dst = dense ? at::empty_strided(src.sizes(), strides, src.options().dtype(dtype)) : at::empty(src.sizes(), src.options().dtype(dtype));
+  check(pico_convert_f32(fptr(src), ptr(dst), src.size(0), src.size(1), src.size(2), src.size(3), dst.stride(0), dst.stride(1), dst.stride(2),
+                         dtype_code(dst, "convert_f32"), stream_now()));
+  return dst;
+}
+
+// Identity on a rank's (k, v) chunk -- with rope tables k is rotated -- that marks where the ring's dK / dV come back: the
+// native form of _PublishKV.  It keeps no saved variables: the node may run in several backward calls.
+struct PublishKV : torch::autograd::Function<PublishKV> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& v, const c10::intrusive_ptr<PyHeld>& box,
+                               const Rope& rope_cs, int64_t pos) {
+    ctx->saved_data["box"] = c10::IValue::make_capsule(box);
+    ctx->saved_data["dtypes"] = std::vector<int64_t>{static_cast<int64_t>(k.scalar_type()), static_cast<int64_t>(v.scalar_type())};
+    ctx->saved_data["k_strides"] = k.strides().vec();
+    ctx->saved_data["v_strides"] = v.strides().vec();
+    ctx->saved_data["dense"] = std::vector<int64_t>{dense_layout(k), dense_layout(v)};
+    ctx->set_materialize_grads(false);
+    if (rope_cs) {
+      ctx->saved_data["cos"] = rope_cs->first;
+      ctx->saved_data["sin"] = rope_cs->second;
+      ctx->saved_data["pos"] = pos;
+      return {rope(k, rope_cs->first, rope_cs->second, pos, false, std::nullopt), v.variable_data()};
+    }
+    return {k.variable_data(), v.variable_data()};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    OptTensor dk, dv, sum_k, sum_v;
+    {
+      pybind11::gil_scoped_acquire gil;
+      const pybind11::handle box(static_cast<PyHeld*>(ctx->saved_data["box"].toCapsule().get())->objects[0]);
+      box.attr("arrived") = 0;
+      dk = tensor_attr(box, "final_dk");
+      if (dk) {   // the last reader's kernel wrote the rounded totals itself
+        dv = tensor_attr(box, "final_dv");
+        set_attr(box, "final_dk", std::nullopt);
+        set_attr(box, "final_dv", std::nullopt);
+      } else {
+        sum_k = tensor_attr(box, "dk");
+        sum_v = tensor_attr(box, "dv");
+      }
+      set_attr(box, "dk", std::nullopt);   // the next backward through this chunk starts a fresh sum
+      set_attr(box, "dv", std::nullopt);
+    }
+    const auto dtypes = ctx->saved_data["dtypes"].toIntVector(), dense = ctx->saved_data["dense"].toIntVector();
+    if (sum_k) {
+      dk = convert_sum(*sum_k, static_cast<at::ScalarType>(dtypes[0]), dense[0], ctx->saved_data["k_strides"].toIntVector());
+      dv = convert_sum(*sum_v, static_cast<at::ScalarType>(dtypes[1]), dense[1], ctx->saved_data["v_strides"].toIntVector());
+    }
+    if (g[0].defined()) {   // a gradient that reached the (rotated) chunk some other way
+      Tensor gk = g[0];
+      if (ctx->saved_data.count("cos"))
+        gk = rope(gk, ctx->saved_data["cos"].toTensor(), ctx->saved_data["sin"].toTensor(), ctx->saved_data["pos"].toInt(), true, std::nullopt);
+      dk = dk ? *dk + gk : gk;
+    }
+    if (g[1].defined()) dv = dv ? *dv + g[1] : g[1];
+    return {dk.value_or(Tensor()), dv.value_or(Tensor()), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::pair<Tensor, Tensor> publish_kv(const Tensor& k, const Tensor& v, const pybind11::object& box, const Rope& rope_cs, int64_t pos) {
+  auto held = c10::make_intrusive<PyHeld>(std::vector<pybind11::object>{box});
+  pybind11::gil_scoped_release nogil;
+  auto r = PublishKV::apply(k, v, held, rope_cs, pos);
+  return {r[0], r[1]};
+}
+
+// What the launch of a rank's forward left behind, for its backward.
+struct RingPass {
+  Tensor out, lse, q;   // q: the rotated copy where rope tables are given
+  c10::intrusive_ptr<PyHeld> boxes;
+  Rope rope;
+  double sm_scale;
+  bool causal;
+  int64_t q_offset, q_pos, k_pos;
+};
+
+// One rank's attention over the chunks it reads (their k, v in the order of their positions).  The forward has run already;
+// this node carries its backward: one launch pair for all chunks, whose dK / dV blocks are added to the chunks' fp32 sums
+// -- or, where this is the last block a chunk waits for, leave as the chunk's rounded totals.
+struct RingAttention : torch::autograd::Function<RingAttention> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, at::TensorList kvs, const RingPass& p) {
+    variable_list saved = {p.q.defined() ? p.q : q, p.lse, p.out};
+    for (const Tensor& t : kvs) saved.push_back(t);
+    if (p.rope) {
+      saved.push_back(p.rope->first);
+      saved.push_back(p.rope->second);
+    }
+    ctx->save_for_backward(saved);
+    ctx->saved_data["boxes"] = c10::IValue::make_capsule(p.boxes);
+    ctx->saved_data["scale"] = p.sm_scale;
+    ctx->saved_data["meta"] = std::vector<int64_t>{p.causal, p.q_offset, p.q_pos, p.k_pos, static_cast<int64_t>(kvs.size() / 2), p.rope.has_value()};
+    return p.out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const auto s = ctx->get_saved_variables();
+    const auto meta = ctx->saved_data["meta"].toIntVector();
+    const size_t n = meta[4];
+    const Tensor &q = s[0], &lse = s[1], &out = s[2];
+    std::vector<Tensor> ks, vs;
+    for (size_t i = 0; i < n; ++i) {
+      ks.push_back(s[3 + 2 * i]);
+      vs.push_back(s[4 + 2 * i]);
+    }
+    Rope rope_cs;
+    if (meta[5]) rope_cs = std::make_pair(s[3 + 2 * n], s[4 + 2 * n]);
+    OptTensors dks(n), dvs(n), dk_finals(n), dv_finals(n);
+    std::vector<bool> add(n, false);
+    bool any_final = false;
+    {
+      pybind11::gil_scoped_acquire gil;
+      const auto& boxes = static_cast<PyHeld*>(ctx->saved_data["boxes"].toCapsule().get())->objects;
+      for (size_t i = 0; i < n; ++i) {
+        if (!ctx->needs_input_grad(1 + 2 * i) && !ctx->needs_input_grad(2 + 2 * i)) continue;
+        const pybind11::handle box(boxes[i]);
+        const int64_t arrived = box.attr("arrived").cast<int64_t>() + 1;
+        box.attr("arrived") = arrived;
+        dks[i] = tensor_attr(box, "dk");
+        dvs[i] = tensor_attr(box, "dv");
+        add[i] = dks[i].has_value();
+        if (arrived == box.attr("readers").cast<int64_t>()) {
+          // every other rank that read the chunk has added its block: the totals leave from this launch, and fp32 sums are
+          // only read, if earlier blocks left some
+          const Tensor &k = ks[i], &v = vs[i];
+          const bool own_layout = dense_layout(k) && k.strides() == v.strides();
+          auto total = [&] { return own_layout ? at::empty_strided(k.sizes(), k.strides(), k.options()) : at::empty(k.sizes(), k.options()); };
+          dk_finals[i] = total();
+          dv_finals[i] = total();
+          set_attr(box, "final_dk", dk_finals[i]);
+          set_attr(box, "final_dv", dv_finals[i]);
+          any_final = true;
+        } else if (!add[i]) {
+          dks[i] = at::empty(ks[i].sizes(), ks[i].options().dtype(at::kFloat));
+          dvs[i] = at::empty(ks[i].sizes(), ks[i].options().dtype(at::kFloat));
+          set_attr(box, "dk", dks[i]);
+          set_attr(box, "dv", dvs[i]);
+        }
+      }
+    }
+    OptTensor dq;
+    if (ctx->needs_input_grad(0)) dq = empty_like_layout(q, q.options());
+    attn_bwd(g[0], q, ks, vs, lse, ctx->saved_data["scale"].toDouble(), meta[0], meta[1], dq, dks, dvs, false, add, out, std::nullopt, rope_cs,
+             meta[2], meta[3], any_final ? dk_finals : OptTensors(), any_final ? dv_finals : OptTensors());
+    variable_list r(2 + 2 * n);
+    r[0] = dq.value_or(Tensor());
+    return r;
+  }
+};
+
+Tensor ring_node(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs, const Tensor& out, const Tensor& lse,
+                 const OptTensor& q_rot, const std::vector<pybind11::object>& boxes, double sm_scale, bool causal, int64_t q_offset,
+                 const Rope& rope_cs, int64_t q_pos, int64_t k_pos) {
+  RingPass p = {out, lse, q_rot.value_or(Tensor()), c10::make_intrusive<PyHeld>(boxes), rope_cs, sm_scale, causal, q_offset, q_pos, k_pos};
+  pybind11::gil_scoped_release nogil;
+  std::vector<Tensor> kvs;
+  for (size_t i = 0; i < ks.size(); ++i) {
+    kvs.push_back(ks[i]);
+    kvs.push_back(vs[i]);
+  }
+  return RingAttention::apply(q, at::TensorList(kvs), p);
 }
 
 // ------------------------------------------------------------------------------------------------ projections
@@ -1065,6 +1252,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("chunks_fit", &chunks_fit, nogil());
   m.def("attn_fwd", &attn_fwd, nogil());
   m.def("attn_bwd", &attn_bwd, nogil());
+  m.def("publish_kv", &publish_kv);
+  m.def("ring_node", &ring_node);
   m.def("flash_attention", &flash_attention, nogil());
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
