@@ -302,6 +302,12 @@ int pico_convert_f32(const float* src, void* dst, int64_t B, int64_t H, int64_t 
                      int64_t dst_stride_b, int64_t dst_stride_h, int64_t dst_stride_s,
                      int dst_dtype, void* stream);
 
+/* dst[i] = sum over p of src[p][i] for i in [0, n): the pieces of a product whose contraction was cut into `parts` pieces
+ * (fp32 each, contiguous), added in fp32 in the order of the pieces and rounded once.  n must be a multiple of 8.
+ * No counterpart in the reference (its products are torch's).
+ */
+int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int dst_dtype, void* stream);
+
 /* ------------------------------------------------------------------ loss
  * replaces: F.cross_entropy(outputs.view(S*B, V), target_ids, reduction='mean')  train.py:46-49  and its autograd.
  * logits: [rows, vocab] with row pitch ld (elements; a multiple of 8 for bf16, 4 for fp32), dtype `dtype`;

@@ -763,14 +763,16 @@ Tensor ring_node(const Tensor& q, const std::vector<Tensor>& ks, const std::vect
 // one more is asked for.
 class GemmPlans {
  public:
+  // parts > 1: k is cut into that many equal pieces whose products, each in fp32, lie one after the other in C
   struct Shape {
-    int64_t device, ta, tb, m, n, k, lda, ldb, ldc;
+    int64_t device, ta, tb, m, n, k, lda, ldb, parts;
     bool operator==(const Shape& o) const {
-      return device == o.device && ta == o.ta && tb == o.tb && m == o.m && n == o.n && k == o.k && lda == o.lda && ldb == o.ldb && ldc == o.ldc;
+      return device == o.device && ta == o.ta && tb == o.tb && m == o.m && n == o.n && k == o.k && lda == o.lda && ldb == o.ldb && parts == o.parts;
     }
   };
 
-  // column-major C[m,n] = op(A) op(B), bf16 in and out, fp32 accumulation; false: the library has no algorithm for it
+  // column-major C[m,n] = op(A) op(B), bf16 in, bf16 (or, in parts, fp32) out, fp32 accumulation; false: the library has no
+  // algorithm for it
   bool run(const Shape& s, const void* a, const void* b, void* c, const at::TensorOptions& options) {
     std::lock_guard<std::mutex> lock(mutex_);   // (several host threads may come here with one device's handle)
     auto it = plans_.find(s);
@@ -802,7 +804,7 @@ class GemmPlans {
   struct Hash {
     size_t operator()(const Shape& s) const {
       uint64_t h = 1469598103934665603ull;
-      for (int64_t v : {s.device, s.ta, s.tb, s.m, s.n, s.k, s.lda, s.ldb, s.ldc}) h = (h ^ static_cast<uint64_t>(v)) * 1099511628211ull;
+      for (int64_t v : {s.device, s.ta, s.tb, s.m, s.n, s.k, s.lda, s.ldb, s.parts}) h = (h ^ static_cast<uint64_t>(v)) * 1099511628211ull;
       return static_cast<size_t>(h ^ (h >> 29));
     }
   };
@@ -818,9 +820,18 @@ class GemmPlans {
     const int32_t op_a = s.ta ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_b = s.tb ? HIPBLAS_OP_T : HIPBLAS_OP_N;
     ok(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &op_a, sizeof op_a), "TRANSA");
     ok(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSB, &op_b, sizeof op_b), "TRANSB");
-    ok(hipblasLtMatrixLayoutCreate(&p.a, HIP_R_16BF, s.ta ? s.k : s.m, s.ta ? s.m : s.k, s.lda), "layout A");
-    ok(hipblasLtMatrixLayoutCreate(&p.b, HIP_R_16BF, s.tb ? s.n : s.k, s.tb ? s.k : s.n, s.ldb), "layout B");
-    ok(hipblasLtMatrixLayoutCreate(&p.c, HIP_R_16BF, s.m, s.n, s.ldc), "layout C");
+    const int64_t k = s.k / s.parts;
+    ok(hipblasLtMatrixLayoutCreate(&p.a, HIP_R_16BF, s.ta ? k : s.m, s.ta ? s.m : k, s.lda), "layout A");
+    ok(hipblasLtMatrixLayoutCreate(&p.b, HIP_R_16BF, s.tb ? s.n : k, s.tb ? k : s.n, s.ldb), "layout B");
+    ok(hipblasLtMatrixLayoutCreate(&p.c, s.parts > 1 ? HIP_R_32F : HIP_R_16BF, s.m, s.n, s.m), "layout C");
+    if (s.parts > 1) {
+      const int32_t count = static_cast<int32_t>(s.parts);
+      const int64_t step_a = s.ta ? k : k * s.lda, step_b = s.tb ? k * s.ldb : k, step_c = s.m * s.n;
+      for (auto [layout, step] : {std::pair(p.a, step_a), std::pair(p.b, step_b), std::pair(p.c, step_c)}) {
+        ok(hipblasLtMatrixLayoutSetAttribute(layout, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &count, sizeof count), "batch count");
+        ok(hipblasLtMatrixLayoutSetAttribute(layout, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &step, sizeof step), "batch stride");
+      }
+    }
     hipblasLtMatmulPreference_t pref = nullptr;
     ok(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
     const uint64_t ws = kMaxWorkspace;
@@ -875,14 +886,83 @@ Tensor matrix(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size
 
 // row-major products: a @ b^T, a @ b, a^T @ b
 enum class Product { NT, NN, TN };
-Tensor product(const Tensor& a, const Tensor& b, Product kind) {
+
+// How much of the GPU's 256 CUs a product keeps busy, over the library's tile shapes (256 x 256 and narrower ones, which run
+// at the given share of its rate): output / (waves of workgroups x tile).
+double tile_fit(int64_t M, int64_t N) {
+  double best = 0;
+  for (auto [side, rate] : {std::pair<int64_t, double>(256, 1.0), {192, 0.97}, {160, 0.95}, {128, 0.85}})
+    for (auto [m, n] : {std::pair<int64_t, int64_t>(side, 256), {256, side}}) {
+      const int64_t waves = (((M + m - 1) / m) * ((N + n - 1) / n) + 255) / 256;
+      best = std::max(best, rate * M * N / (256.0 * waves * m * n));
+    }
+  return best;
+}
+
+// Into how many pieces the contraction is cut (1: not at all).  The library works on output tiles and walks the whole
+// contraction in each, so a product of few tiles and a long contraction -- the input gradient of the vocabulary projection
+// or of gate / up, weight gradients of a small model -- leaves most of the GPU idle: [512 x 49152] @ [49152 x 576] took
+// 143 us and takes 53 us in 16 pieces, [2048 x 21760] @ [21760 x 4096] 447 and 291 us in two.  The pieces cost 8 bytes of
+// fp32 traffic per output element each, hence the lower bound on a piece's length and, as output grows, on its ratio to
+// the number of tiles; the lines below lie where a sweep over 128 .. 8192 rows, 576 .. 4096 columns and contractions of
+// 512 .. 49152 crossed.  Products of the forward's layout (NT), the library's best, gain only from 8192 on.
+// More than 256 tiles and a contraction from 16384 on (NN): the library is fast where one of its tile shapes fills the CUs
+// evenly ([5120 x 49152] @ [49152 x 2048]: 1200 TFLOP/s) and at half that rate elsewhere ([4500 x 49152]: 620, in four
+// pieces 1150).
+int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  if ((M * N) % 8) return 1;   // (pico_sum_parts moves 8 elements at a time)
+  auto cuts = [&](int64_t parts) { return K % parts == 0 && (K / parts) % 32 == 0; };
+  int64_t most = 1, piece = 0;
+  if (kind == Product::NN && tiles > 256) {
+    if (K < 16384 || tile_fit(M, N) >= 0.88) return 1;
+    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
+    int64_t best = 1;
+    double least = 1.8;   // (of the ideal time)
+    for (int64_t parts : {2, 4}) {
+      if (!cuts(parts)) continue;
+      const int64_t waves = (t256 * parts + 255) / 256;
+      const double cost = waves * 256.0 * 65536 / (static_cast<double>(M) * N * parts) + 1040.0 * parts / K;
+      if (cost < least && (parts > 2 || cost < 1.37)) {   // (two half-filled waves: 956 us at [6145 x 32000], 792 in four pieces)
+        least = cost;
+        best = parts;
+      }
+    }
+    return best;
+  }
+  if (kind == Product::NN && K >= 5120) {
+    most = std::min<int64_t>(16, 1024 / tiles);
+    piece = std::max<int64_t>(1280, 16 * tiles);
+  } else if (kind == Product::TN && K >= 4096) {
+    most = std::min<int64_t>(4, 512 / tiles);
+    piece = 2048;
+  } else if (kind == Product::NT && K >= 8192) {
+    most = tiles <= 64 ? 4 : tiles <= 128 ? 2 : 1;
+    piece = 4096;
+  }
+  int64_t parts = 1;
+  while (2 * parts <= most && cuts(2 * parts) && K / (2 * parts) >= piece) parts *= 2;
+  return parts;
+}
+
+Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0) {
   if (plain(a) && plain(b) && !torch_gemm_only()) {
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
     const int64_t M = kind == Product::TN ? a.size(1) : a.size(0), K = kind == Product::TN ? a.size(0) : a.size(1);
     const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
     TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
     Tensor c = at::empty({M, N}, a.options());
-    const GemmPlans::Shape s = {a.device().index(), kind == Product::NT, kind == Product::TN, N, M, K, b.stride(0), a.stride(0), N};
+    if (parts == 0) parts = contraction_parts(kind, M, N, K);
+    TORCH_CHECK(parts >= 1 && K % parts == 0, "matrix product: a contraction of ", K, " cannot be cut into ", parts, " equal pieces");
+    GemmPlans::Shape s = {a.device().index(), kind == Product::NT, kind == Product::TN, N, M, K, b.stride(0), a.stride(0), parts};
+    if (parts > 1) {
+      const Tensor sums = at::empty({parts, M, N}, a.options().dtype(at::kFloat));
+      if (gemm_plans().run(s, b.data_ptr(), a.data_ptr(), sums.data_ptr(), a.options())) {
+        check(pico_sum_parts(fptr(sums), ptr(c), parts, M * N, PICO_BF16, stream_now()));
+        return c;
+      }
+      s.parts = 1;
+    }
     if (gemm_plans().run(s, b.data_ptr(), a.data_ptr(), c.data_ptr(), a.options())) return c;
   }
   return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
@@ -1255,6 +1335,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("publish_kv", &publish_kv);
   m.def("ring_node", &ring_node);
   m.def("flash_attention", &flash_attention, nogil());
+  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts) {
+    TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
+    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts);
+  });
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("qkv_attention", &qkv_attention, nogil());

@@ -192,6 +192,40 @@ __global__ __launch_bounds__(kThreads) void convert_kernel(const float* __restri
   io<T>::store(dst + b * dsb + h * dsh + s * dss + v * V, vals);
 }
 
+// ---------------------------------------------------------------------------------- sum of fp32 pieces
+// A thread adds its 8 columns of all pieces, four pieces requested at a time; consecutive lanes read consecutive 32 bytes.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float* __restrict__ src, T* __restrict__ dst, int parts, int64_t n) {
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * 8;
+  if (i >= n) return;
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+  constexpr int U = 4;
+  int p = 0;
+  for (; p + U <= parts; p += U) {
+    f32x4 a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float* s = src + (p + u) * n + i;
+      a[u] = *reinterpret_cast<const f32x4*>(s);
+      b[u] = *reinterpret_cast<const f32x4*>(s + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) { lo += a[u]; hi += b[u]; }
+  }
+  for (; p < parts; ++p) {
+    const float* s = src + p * n + i;
+    lo += *reinterpret_cast<const f32x4*>(s);
+    hi += *reinterpret_cast<const f32x4*>(s + 4);
+  }
+  if constexpr (sizeof(T) == 2) {
+    const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    io<__bf16>::store(dst + i, v);
+  } else {
+    *reinterpret_cast<f32x4*>(dst + i) = lo;
+    *reinterpret_cast<f32x4*>(dst + i + 4) = hi;
+  }
+}
+
 unsigned blocks_for(int64_t total) { return static_cast<unsigned>((total + kThreads - 1) / kThreads); }
 bool dtype_ok(int d) { return d == PICO_BF16 || d == PICO_F32; }
 int vec_of(int d) { return d == PICO_BF16 ? 8 : 4; }
@@ -341,4 +375,19 @@ extern "C" int pico_convert_f32(const float* src, void* dst, int64_t B, int64_t 
     hipLaunchKernelGGL(convert_kernel<float>, dim3(blocks_for(total)), dim3(kThreads), 0, st, src,
                        static_cast<float*>(dst), total, (int)H, (int)S, (int)D, dsb, dsh, dss, s_outer);
   return check_launch("pico_convert_f32");
+}
+
+extern "C" int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int dst_dtype, void* stream) {
+  if (!dtype_ok(dst_dtype)) return fail(PICO_ERR_DTYPE, "pico_sum_parts: dtype code %d not supported", dst_dtype);
+  if (parts < 1 || parts > 0x7fffffff || n < 0 || n % 8 != 0)
+    return fail(PICO_ERR_SHAPE, "pico_sum_parts: parts=%lld n=%lld (n must be a multiple of 8)", (long long)parts, (long long)n);
+  if (n == 0) return PICO_OK;
+  if (!src || !dst) return fail(PICO_ERR_NULL, "pico_sum_parts: src and dst are required");
+  if (!aligned16(src) || !aligned16(dst)) return fail(PICO_ERR_ALIGN, "pico_sum_parts: pointers must be 16-byte aligned");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dst_dtype == PICO_BF16)
+    hipLaunchKernelGGL(sum_parts_kernel<__bf16>, dim3(blocks_for(n / 8)), dim3(kThreads), 0, st, src, static_cast<__bf16*>(dst), (int)parts, n);
+  else
+    hipLaunchKernelGGL(sum_parts_kernel<float>, dim3(blocks_for(n / 8)), dim3(kThreads), 0, st, src, static_cast<float*>(dst), (int)parts, n);
+  return check_launch("pico_sum_parts");
 }

@@ -1,0 +1,36 @@
+"""The projections' matrix products: the rule that cuts long contractions into pieces, and the sum of the pieces, against a
+fp32 product on the same bf16 operands."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,M,N,K", [
+    ("NN", 8, 64, 5120), ("NN", 129, 576, 49152), ("NN", 512, 576, 49152), ("NN", 300, 1024, 5376), ("NN", 2100, 2048, 16384),
+    ("NT", 31, 576, 8192), ("NT", 200, 2048, 16384), ("TN", 576, 960, 4096), ("TN", 64, 8, 8192), ("NN", 7, 9, 8192), ("TN", 72, 40, 333)])
+def test_products_in_pieces(device, kind, M, N, K):
+    from picotron_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, b = (torch.randn(*s, generator=g, device=device).to(torch.bfloat16)
+            for s in (((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))))
+    want = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float())
+    for parts in (0, 1, 2, 4, 16):           # 0: the rule's own choice
+        if parts > 1 and (K % (32 * parts) or M * N % 8):
+            continue
+        got = _lib.host().product(a, b, kind, parts)
+        assert got.shape == (M, N) and got.dtype == torch.bfloat16
+        assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, parts
+
+
+def test_linear_layer_gradients_match_torch(device):
+    from picotron_amd.model import Linear
+    g = torch.Generator(device="cuda").manual_seed(3)
+    layer = Linear(5376, 1024, bias=False, device=device, dtype=torch.bfloat16)
+    x = torch.randn(3, 107, 5376, generator=g, device=device).to(torch.bfloat16).requires_grad_()
+    dy = torch.randn(3, 107, 1024, generator=g, device=device).to(torch.bfloat16)
+    got = torch.autograd.grad(layer(x), (x, layer.weight), dy)
+    xf, wf = x.detach().float().requires_grad_(), layer.weight.detach().float().requires_grad_()
+    want = torch.autograd.grad(torch.nn.functional.linear(xf, wf), (xf, wf), dy.float())
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and ((a.float() - b).norm() / b.norm()).item() <= 3e-3
