@@ -249,8 +249,8 @@ int pico_attn_bwd_rope(const pico_attn_desc* desc, const void* q_rot, const void
  *           chunks a rank would receive step by step are all in this GPU's memory already (virtual ranks).
  * K / V are `count` chunks of chunk_len keys each, given by their base pointers; every chunk is addressed with the
  * descriptor's k_stride / v_stride (and dkv_stride), desc->Sk must equal count * chunk_len, and with count > 1
- * chunk_len must be a multiple of 128 (otherwise PICO_ERR_SHAPE: run the ring step by step with pico_attn_fwd(merge)
- * / pico_attn_bwd(accumulate)).  Key j of the launch is row j % chunk_len of chunk j / chunk_len and sits at position
+ * chunk_len must be over 64 (otherwise PICO_ERR_SHAPE: run the ring step by step with pico_attn_fwd(merge)
+ * / pico_attn_bwd(accumulate)); multiples of 128 leave no partly filled key tile at the end of a chunk.  Key j of the launch is row j % chunk_len of chunk j / chunk_len and sits at position
  * j: list the chunks in the order of their positions (for a causal ring: the chunks of ranks 0 .. r, q_offset =
  * r * chunk_len).  The online softmax runs across the chunks inside the kernel -- no per-step partial result, no
  * merge pass, no fp32 running out.
@@ -293,6 +293,26 @@ int pico_attn_bwd_chunks(const pico_attn_desc* desc, const void* q, const pico_k
                          void* dq, const int64_t* dq_stride, int dq_dtype, int dq_accumulate,
                          const int64_t* dkv_stride, int dkv_dtype,
                          const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset, void* stream);
+
+/* The same two calls with device scratch memory, for launches that leave much of the GPU idle -- few heads, short
+ * sequences, GQA groups (whose query heads one dK/dV workgroup otherwise walks one after the other).  Where that pays, the
+ * key or query range of an output tile is dealt to several workgroups, whose fp32 accumulators go through the workspace to
+ * a second small launch that adds them in a fixed order.  *_workspace_bytes says what such a launch needs (0: none; at most
+ * PICO_ATTN_MAX_WORKSPACE) for the descriptor and number of chunks; with less, or NULL, the call runs as without.  Contents
+ * are undefined on entry and exit; calls that overlap in time need workspaces of their own.
+ */
+#define PICO_ATTN_MAX_WORKSPACE (256ll << 20)
+int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count);
+int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count);
+int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out, float* lse,
+                            int out_dtype, int merge, const pico_rope_tables* rope, int q_pos_offset, void* q_rot,
+                            const int64_t* q_rot_stride, void* workspace, int64_t workspace_bytes, void* stream);
+int pico_attn_bwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
+                            const void* out, int out_dtype, const float* lse, float* delta,
+                            void* dq, const int64_t* dq_stride, int dq_dtype, int dq_accumulate,
+                            const int64_t* dkv_stride, int dkv_dtype,
+                            const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 
 /* fp32 -> bf16/fp32 conversion with layout change: src [B,H,S,D] contiguous fp32,
  * dst addressed by dst_stride (b,h,s).  Used to hand dq_acc back in the dtype / layout of q.

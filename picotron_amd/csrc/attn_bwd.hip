@@ -86,8 +86,59 @@ struct KvCfg {
   static_assert(!PAIR || kKeyWaves * kPairExchangeBytes <= kTileBytes, "the pair exchange reuses the tile buffers");
 };
 
+// key tile `ktile` (counted chunk by chunk): its chunk, its first row there and that row's position in the launch
+struct KeyTile {
+  int chunk, row0, key0;
+};
+__host__ __device__ inline KeyTile key_tile(const KvChunks& kv, int ktile, int BN) {
+  if (kv.count == 1) return {0, ktile * BN, ktile * BN};
+  const int per = (kv.len + BN - 1) / BN, chunk = ktile / per, row0 = (ktile - chunk * per) * BN;
+  return {chunk, row0, chunk * kv.len + row0};
+}
+// first query tile of BM queries that sees position key0
+__host__ __device__ inline int first_query_tile(const AttnParams& a, int key0, int BM) {
+  const int first_q = a.causal ? key0 - a.q_offset : 0;
+  return first_q > 0 ? first_q / BM : 0;
+}
+// trips of a key tile: (query heads of the group) x (query tiles that see it)
+__host__ __device__ inline int dkdv_trips(const AttnParams& a, int ktile, int BN, int BM) {
+  const int n = (a.Sq + BM - 1) / BM, start = first_query_tile(a, key_tile(a.kv, ktile, BN).key0, BM);
+  return n > start ? (n - start) * (a.Hq / a.Hkv) : 0;
+}
+
+// the rows of dK (kDk) or dV that a wave's accumulators hold: 32 keys from row `row0` of their chunk, position `key0`
+template <int D, bool kDk>
+__device__ __forceinline__ void dkdv_store(const BwdParams& p, unsigned char* region, f32x16 (&acc)[D / 32], int chunk, int b, int hkv,
+                                           int row0, int key0, int lane) {
+  const AttnParams& a = p.a;
+  const int n = lane % 32, h = lane / 32;
+  const int rows_live = a.kv.len - row0;
+  const int64_t off = b * p.dks[0] + hkv * p.dks[1] + static_cast<int64_t>(row0) * p.dks[2];
+  // gradient w.r.t. the un-rotated k: rotate the lane's row of dK back (linear, so the scale and the sum can follow)
+  if constexpr (kDk) {
+    if (p.rope.cos != nullptr) rope_unrotate_acc<D>(acc, p.rope, n < rows_live ? p.rope.k_pos0 + key0 + n : 0, h);
+  }
+  const float scale = kDk ? a.sm_scale : 1.f;
+  void* const dst = kDk ? p.dk[chunk] : p.dv[chunk];
+  __bf16* const total = kDk ? p.dk_final[chunk] : p.dv_final[chunk];
+  const bool accumulate = (p.dkv_accumulate >> chunk) & 1u;
+  if (total != nullptr) {
+    // the last block this chunk's gradient was waiting for: total = travelling sums + this block, rounded once
+    const int64_t foff = b * p.dkfs[0] + hkv * p.dkfs[1] + static_cast<int64_t>(row0) * p.dkfs[2];
+    wave_store_rows_total<D>(region, acc, scale, accumulate ? static_cast<const float*>(dst) + off : nullptr, p.dks[2], total + foff,
+                             p.dkfs[2], rows_live, lane);
+  } else if (p.dkv_f32) {
+    wave_store_rows<D, true>(region, acc, scale, static_cast<float*>(dst) + off, p.dks[2], rows_live, lane, accumulate, false);
+  } else {
+    wave_store_rows<D, false>(region, acc, scale, static_cast<__bf16*>(dst) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
+  }
+}
+
+// what a wave of a piece leaves: its dK and dV accumulators
+__host__ __device__ constexpr int dkdv_piece_floats(int D) { return 2 * (D / 32) * 16 * kWave; }
+
 template <int D, bool PAIR = false>
-__device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int ktile) {
+__device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int ktile, const int part = 0, const int parts = 1) {
   using C = KvCfg<D, PAIR>;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -96,9 +147,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   const AttnParams& a = p.a;
   const int hkv = blockIdx.x % a.Hkv, b = blockIdx.x / a.Hkv;
   const int group = a.Hq / a.Hkv;
-  const int key0 = ktile * BN;                     // position of the tile's first key in the launch
-  const int chunk = a.kv.count > 1 ? key0 / a.kv.len : 0;
-  const int crow0 = key0 - chunk * a.kv.len;       // ... and its row in the chunk that holds it
+  const KeyTile kt_at = key_tile(a.kv, ktile, BN);
+  const int key0 = kt_at.key0, chunk = kt_at.chunk, crow0 = kt_at.row0;
   if (p.dk[chunk] == nullptr && p.dk_final[chunk] == nullptr) return;   // this chunk's gradient is not wanted (uniform over the workgroup)
   const int tid = threadIdx.x, wave_id = tid / 64, lane = tid % 64;
   // wave: which 32 keys of the tile; pair_sb (PAIR only): which 32-query sub-block of every query tile
@@ -136,13 +186,16 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 
   // ---- trip space: (query head of the group) x (query tiles that can see key0)
   const int n_qtiles = (a.Sq + BM - 1) / BM;
-  int qt_start = 0;
-  if (a.causal) {
-    const int first_q = key0 - a.q_offset;  // first query index that sees key0
-    qt_start = first_q > 0 ? first_q / BM : 0;
-  }
+  const int qt_start = first_query_tile(a, key0, BM);
   const int tiles_per_head = n_qtiles > qt_start ? n_qtiles - qt_start : 0;
-  const int n_iter = tiles_per_head * group;
+  int n_iter = tiles_per_head * group, head_first = hkv * group, tile_first = qt_start;
+  if (parts > 1) {   // this workgroup's share of the trips
+    const int t0 = n_iter * part / parts;
+    n_iter = n_iter * (part + 1) / parts - t0;
+    const int skip = t0 / tiles_per_head;
+    head_first += skip;
+    tile_first += t0 - skip * tiles_per_head;
+  }
 
   // Global -> register prefetch of a Q / dO tile (+ lse, delta) with buffer loads.  A cursor (wave-uniform:
   // it lives in scalar registers) walks the trip space; stepping to the next tile of the same head is a few
@@ -222,7 +275,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   };
 
   if (n_iter > 0) {
-    seek(hkv * group, qt_start);
+    seek(head_first, tile_first);
     prefetch();
   }
   if (loads_kv) {
@@ -259,7 +312,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   }
 
   const int kw0 = key0 + 32 * wave;
-  int tile = qt_start;       // query tile (within its head) of the trip being computed
+  int tile = tile_first;     // query tile (within its head) of the trip being computed
   uint32_t buf_off = 0;      // byte offset of the LDS buffer being read
   for (int it = 0; it < n_iter; ++it) {
     // tile it+1 travels global -> registers while this trip computes; it goes to the other LDS buffer at
@@ -538,27 +591,15 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     }
   }
   if (!PAIR || pair_sb == 0) {
-    unsigned char* region = smem_raw + wave * kRowRegionBytes;
-    const int row0 = crow0 + 32 * wave;          // first row of the wave inside its chunk
-    const int rows_live = a.kv.len - row0;
-    const int64_t off = b * p.dks[0] + hkv * p.dks[1] + static_cast<int64_t>(row0) * p.dks[2];
-    // gradient w.r.t. the un-rotated k: rotate the lane's row of dK back (linear, so the scale and the sum can follow)
-    if (p.rope.cos != nullptr) rope_unrotate_acc<D>(dk_acc, p.rope, n < rows_live ? p.rope.k_pos0 + kw0 + n : 0, h);
-    const bool accumulate = (p.dkv_accumulate >> chunk) & 1u;
-    if (p.dk_final[chunk] != nullptr) {
-      // the last block this chunk's gradient was waiting for: total = travelling sums + this block, rounded once
-      const int64_t foff = b * p.dkfs[0] + hkv * p.dkfs[1] + static_cast<int64_t>(row0) * p.dkfs[2];
-      wave_store_rows_total<D>(region, dk_acc, a.sm_scale, accumulate ? static_cast<const float*>(p.dk[chunk]) + off : nullptr, p.dks[2],
-                               p.dk_final[chunk] + foff, p.dkfs[2], rows_live, lane);
-      wave_store_rows_total<D>(region, dv_acc, 1.f, accumulate ? static_cast<const float*>(p.dv[chunk]) + off : nullptr, p.dks[2],
-                               p.dv_final[chunk] + foff, p.dkfs[2], rows_live, lane);
-    } else if (p.dkv_f32) {
-      wave_store_rows<D, true>(region, dk_acc, a.sm_scale, static_cast<float*>(p.dk[chunk]) + off, p.dks[2], rows_live, lane, accumulate, false);
-      wave_store_rows<D, true>(region, dv_acc, 1.f, static_cast<float*>(p.dv[chunk]) + off, p.dks[2], rows_live, lane, accumulate, false);
-    } else {
-      wave_store_rows<D, false>(region, dk_acc, a.sm_scale, static_cast<__bf16*>(p.dk[chunk]) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
-      wave_store_rows<D, false>(region, dv_acc, 1.f, static_cast<__bf16*>(p.dv[chunk]) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
+    if (parts > 1) {   // one piece of several: the sums leave as they are
+      float* dst = a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kKeyWaves + wave) * dkdv_piece_floats(D);
+      put_acc<D / 32>(dst, dk_acc, lane);
+      put_acc<D / 32>(dst + dkdv_piece_floats(D) / 2, dv_acc, lane);
+      return;
     }
+    unsigned char* region = smem_raw + wave * kRowRegionBytes;
+    dkdv_store<D, true>(p, region, dk_acc, chunk, b, hkv, crow0 + 32 * wave, kw0, lane);
+    dkdv_store<D, false>(p, region, dv_acc, chunk, b, hkv, crow0 + 32 * wave, kw0, lane);
   }
 }
 
@@ -570,7 +611,13 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 // workgroup (kernel arguments, first loads) half as often.
 template <int D, bool PAIR = false>
 __device__ __forceinline__ void attn_bwd_dkdv_body(const BwdParams& p) {
-  const int n_ktiles = (p.a.Sk + KvCfg<D, PAIR>::BN - 1) / KvCfg<D, PAIR>::BN;
+  using C = KvCfg<D, PAIR>;
+  const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN);
+  if (p.a.pieces.len > 0) {
+    const Piece at = find_piece(blockIdx.y, n_ktiles, p.a.pieces.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
+    attn_bwd_dkdv_tile<D, PAIR>(p, at.tile, at.part, at.parts);
+    return;
+  }
   const int first = blockIdx.y;
   attn_bwd_dkdv_tile<D, PAIR>(p, first);
   const int second = n_ktiles - 1 - first;
@@ -588,6 +635,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // D = 128: eight waves, two per key block (see KvCfg), 256 registers each
 __global__ __launch_bounds__(512) void attn_bwd_dkdv_kernel_d128(const BwdParams p) {
   attn_bwd_dkdv_body<128, true>(p);
+}
+
+// The pieces of every cut key tile put together: grid.z 0 sums dK, 1 dV; a wave per 32 keys adds the pieces' accumulators in
+// their order and ends as the kernel above does.
+template <int D>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_join_kernel(const BwdParams p, const int pieces_per_head) {
+  using C = KvCfg<D, D == 128>;
+  __shared__ __attribute__((aligned(16))) unsigned char smem_raw[C::kKeyWaves * kRowRegionBytes];
+  const AttnParams& a = p.a;
+  const int tile = static_cast<int>(blockIdx.y);
+  auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
+  const int parts = pieces_of(trips_of(tile), a.pieces.len);
+  const KeyTile at = key_tile(a.kv, tile, C::BN);
+  if (parts == 1 || (p.dk[at.chunk] == nullptr && p.dk_final[at.chunk] == nullptr)) return;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int hkv = blockIdx.x % a.Hkv, b = blockIdx.x / a.Hkv;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * pieces_per_head + first_piece(tile, a.pieces.len, trips_of);
+  const float* src = a.pieces.ws + (first * C::kKeyWaves + wave) * dkdv_piece_floats(D) + (blockIdx.z ? dkdv_piece_floats(D) / 2 : 0);
+  constexpr int64_t kStep = static_cast<int64_t>(C::kKeyWaves) * dkdv_piece_floats(D);
+  f32x16 acc[D / 32];
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
+  for (int j = 0; j < parts; ++j) {
+    f32x4 raw[D / 32][4];
+    get_acc<D / 32>(src + j * kStep, raw, lane);
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[db][i] += raw[db][i / 4][i % 4];
+  }
+  unsigned char* region = smem_raw + wave * kRowRegionBytes;
+  if (blockIdx.z == 0) dkdv_store<D, true>(p, region, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
+  else dkdv_store<D, false>(p, region, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
 }
 
 template <int D> struct KvKernel;
@@ -616,6 +698,22 @@ struct DqCfg {
   static_assert(KS == 1 || NW * kExchangeBytes <= kLdsBytes, "the exchange reuses the tile buffers");
 };
 
+// what a wave of a piece leaves: its dQ^T accumulators
+__host__ __device__ constexpr int dq_piece_floats(int D) { return (D / 32) * 16 * kWave; }
+
+// the wave's 32 dQ rows leave through its piece of LDS as whole lines
+template <int D>
+__device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* region, f32x16 (&dq)[D / 32], int b, int hq, int row0, int lane) {
+  const AttnParams& a = p.a;
+  const int qrow = row0 + lane % 32, h = lane / 32;
+  const int64_t off = b * p.dqs[0] + hq * p.dqs[1] + static_cast<int64_t>(row0) * p.dqs[2];
+  if (p.rope.cos != nullptr) rope_unrotate_acc<D>(dq, p.rope, qrow < a.Sq ? p.rope.q_pos0 + qrow : 0, h);
+  if (p.dq_f32)
+    wave_store_rows<D, true>(region, dq, a.sm_scale, static_cast<float*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, p.dq_accumulate, false);
+  else
+    wave_store_rows<D, false>(region, dq, a.sm_scale, static_cast<__bf16*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, false, kStreamGrads);
+}
+
 // (small workgroups are built for two of them per CU: at most 256 registers per lane)
 template <int D, int NW, int KT, bool kDelta, int KS = 1>
 __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bwd_dq_kernel(const BwdParams p) {
@@ -627,7 +725,10 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
   // same dispatch order as the forward kernel: every head's last (longest) query tile first
-  const int qtile = n_qtiles - 1 - static_cast<int>(blockIdx.y);
+  Piece piece = {static_cast<int>(blockIdx.y), 0, 1};
+  if (a.pieces.len > 0)
+    piece = find_piece(blockIdx.y, n_qtiles, a.pieces.len, [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, BM, KT); });
+  const int qtile = n_qtiles - 1 - piece.tile;
   const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
   const int hkv = hq / (a.Hq / a.Hkv);
   const int q0 = qtile * BM;
@@ -673,7 +774,7 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
 #pragma unroll
         for (int e = 0; e < 8; ++e) part += static_cast<float>(dof[s][e]) * static_cast<float>(of[s][e]);
       delta = half_sum(part);
-      if (qlive && h == 0 && ks == 0) p.delta_w[gi] = delta;
+      if (qlive && h == 0 && ks == 0 && piece.part == 0) p.delta_w[gi] = delta;
     }
   }
 
@@ -691,7 +792,11 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
     kv_end = vis < a.Sk ? vis : a.Sk;
     if (kv_end < 0) kv_end = 0;
   }
-  const int ntiles = (kv_end + KT - 1) / KT;
+  int t_first = 0, ntiles = tiles_before(a.kv, kv_end, KT);
+  if (piece.parts > 1) {
+    t_first = ntiles * piece.part / piece.parts;
+    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
+  }
 
   // K / V tiles travel global -> registers -> LDS with buffer loads (wave-uniform resource per tile, per-lane
   // byte offsets computed once, rows past Sk read as zeros)
@@ -706,7 +811,9 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
   }
   // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
   KvCursor<D> cur;
-  cur.open(a, 0, b, hkv, KT);
+  cur.open(a, t_first, b, hkv, KT);
+  KvPosition pos;
+  pos.open(a.kv, t_first, KT);
   auto load_tile = [&]() {  // the next tile of KT keys
     const buffer_rsrc kb = make_buffer(cur.k, cur.k_left), vb = make_buffer(cur.v, cur.v_left);
 #pragma unroll
@@ -738,8 +845,8 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
   __syncthreads();
 
   const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
-  const int qpos = a.q_offset + qrow;
-  for (int t = 0; t < ntiles; ++t) {
+  const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
+  for (int t = 0; t < ntiles; ++t, pos.next(a.kv, KT)) {
     if (t + 1 < ntiles) {
       store_tile((t + 1) & 1);
       if (t + 2 < ntiles) load_tile();
@@ -749,8 +856,8 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
-      const int k0 = t * KT + sub * BN;
-      if (k0 >= kv_end) break;
+      const int k0 = pos.key0 + sub * BN;
+      if (k0 >= kv_end || k0 >= pos.end) break;
       if (a.causal && k0 > blk_q_lo + 31) continue;  // the wave's whole 32x64 block is in the future
       const __bf16* sKs = sK + sub * BN * LDK;
       const __bf16* sVs = sV + sub * BN * LDK;
@@ -771,9 +878,10 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
           dp_acc[mb] = mfma32(va, dof[s], dp_acc[mb]);
         }
       }
-      // dS^T = P^T * (dP^T - delta); keys past the diagonal are masked only in tiles that straddle it
-      // (rows of K / V past Sk are zero, so those keys add nothing to dQ)
-      const bool need_mask = a.causal && (k0 + BN - 1 > blk_q_lo);
+      // dS^T = P^T * (dP^T - delta); keys past the diagonal or the end of their chunk are masked only in tiles that
+      // straddle it (the rows read past a chunk are zero, but P of a zero score need not be finite beside a very
+      // negative lse)
+      const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || k0 + BN > pos.end;
       if (need_mask) {
         // the asm statement keeps this a real (wave-uniform) branch instead of per-element selects
         asm volatile("; masked tile" ::: "memory");
@@ -782,7 +890,7 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const int key = k0 + 32 * mb + 8 * (i / 4) + 4 * h + (i % 4);
-            if (key > qpos) s_acc[mb][i] = -INFINITY;   // exp2(-inf) = 0
+            if (key > qpos || key >= pos.end) s_acc[mb][i] = -INFINITY;   // exp2(-inf) = 0
           }
       }
 #pragma unroll
@@ -834,17 +942,42 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
     static_assert(kRowRegionBytes <= C::kExchangeBytes, "store pieces lie below the exchange areas read above");
   }
 
-  // ---- epilogue: the wave's 32 dQ rows leave through its piece of LDS as whole lines (the loop ended on a barrier)
-  {
-    unsigned char* region = smem_raw + wave * kRowRegionBytes;
-    const int row0 = q0 + qw * 32;
-    const int64_t off = b * p.dqs[0] + hq * p.dqs[1] + static_cast<int64_t>(row0) * p.dqs[2];
-    if (p.rope.cos != nullptr) rope_unrotate_acc<D>(dq, p.rope, qlive ? p.rope.q_pos0 + qrow : 0, h);
-    if (p.dq_f32)
-      wave_store_rows<D, true>(region, dq, a.sm_scale, static_cast<float*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, p.dq_accumulate, false);
-    else
-      wave_store_rows<D, false>(region, dq, a.sm_scale, static_cast<__bf16*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, false, kStreamGrads);
+  if (piece.parts > 1) {   // one piece of several: the sums leave as they are
+    put_acc<D / 32>(a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * dq_piece_floats(D), dq, lane);
+    return;
   }
+  dq_store<D>(p, smem_raw + wave * kRowRegionBytes, dq, b, hq, q0 + qw * 32, lane);
+}
+
+// The pieces of every cut query tile put together (see attn_bwd_dkdv_join_kernel).
+template <int D, int QW, int KT>
+__global__ __launch_bounds__(64 * QW) void attn_bwd_dq_join_kernel(const BwdParams p, const int pieces_per_head) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem_raw[QW * kRowRegionBytes];
+  const AttnParams& a = p.a;
+  constexpr int BM = 32 * QW;
+  const int n_qtiles = (a.Sq + BM - 1) / BM, tile = static_cast<int>(blockIdx.y);
+  auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, BM, KT); };
+  const int parts = pieces_of(trips_of(tile), a.pieces.len);
+  if (parts == 1) return;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * pieces_per_head + first_piece(tile, a.pieces.len, trips_of);
+  const float* src = a.pieces.ws + (first * QW + wave) * dq_piece_floats(D);
+  constexpr int64_t kStep = static_cast<int64_t>(QW) * dq_piece_floats(D);
+  f32x16 dq[D / 32];
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dq[db][i] = 0.f;
+  for (int j = 0; j < parts; ++j) {
+    f32x4 raw[D / 32][4];
+    get_acc<D / 32>(src + j * kStep, raw, lane);
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dq[db][i] += raw[db][i / 4][i % 4];
+  }
+  dq_store<D>(p, smem_raw + wave * kRowRegionBytes, dq, b, hq, (n_qtiles - 1 - tile) * BM + wave * 32, lane);
 }
 
 // delta[row] = sum_d dO * O, one 16-byte vector of each per lane, D/8 lanes per row.
@@ -890,21 +1023,52 @@ __global__ __launch_bounds__(256) void attn_bwd_preprocess_kernel(const __bf16* 
   if (row < rows && v == 0) delta[row] = part;
 }
 
+// How the dK/dV launch is run: key tiles singly, in pairs, or cut into pieces.
+struct DkdvPlan {
+  bool pair = false;
+  int len = 0;
+  int64_t ws_bytes = 0;
+};
 template <int D>
-int launch_dkdv(const BwdParams& p, hipStream_t s) {
+DkdvPlan plan_dkdv(const AttnParams& a, int64_t ws_bytes) {
+  using C = KvCfg<D, D == 128>;
+  DkdvPlan plan;
+  const int64_t heads = static_cast<int64_t>(a.Hkv) * a.B;
+  const int n_ktiles = tiles_before(a.kv, a.Sk, C::BN);
+  // pairs only when they still fill most of the GPU (two workgroups per CU for D = 64, one for D = 128; at D = 64 three
+  // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
+  // are up to 30 % faster)
+  plan.pair = a.causal && n_ktiles >= 2 && heads * ((n_ktiles + 1) / 2) >= (D == 64 ? 384 : 256);
+  if (ws_bytes <= 0) return plan;
+  TripCost cost = {1.1, 1.0, 4.0, 0.0};
+  if (D == 128) cost = {1.65, 2.05, 4.0, 0.0};
+  cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
+  auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
+  plan.len = choose_pieces(heads, n_ktiles, cost, ws_bytes, trips_of);
+  if (plan.len > 0) {
+    const int n = count_pieces(n_ktiles, plan.len, trips_of);
+    if (n == n_ktiles) plan.len = 0;
+    else plan.ws_bytes = static_cast<int64_t>(heads * n * cost.piece_bytes);
+  }
+  return plan;
+}
+
+template <int D>
+int launch_dkdv(const BwdParams& p, float* ws, int64_t ws_bytes, hipStream_t s) {
   using C = KvCfg<D, D == 128>;
   static LdsOnce lds_reserved;
   if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(KvKernel<D>::fn), C::kLdsBytes))
     return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dk/dv): cannot reserve %zu bytes of LDS", C::kLdsBytes);
-  const int n_ktiles = (p.a.Sk + C::BN - 1) / C::BN;
-  // pairs only when they still fill most of the GPU (two workgroups per CU for D = 64, one for D = 128; at D = 64 three
-  // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
-  // are up to 30 % faster)
+  const DkdvPlan plan = plan_dkdv<D>(p.a, ws ? ws_bytes : 0);
+  const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN), heads = p.a.Hkv * p.a.B;
   BwdParams q = p;
-  const int64_t slots = D == 64 ? 384 : 256;
-  q.pair_ktiles = p.a.causal && n_ktiles >= 2 && static_cast<int64_t>(p.a.Hkv) * p.a.B * ((n_ktiles + 1) / 2) >= slots;
-  const int grid_y = q.pair_ktiles ? (n_ktiles + 1) / 2 : n_ktiles;
-  hipLaunchKernelGGL(KvKernel<D>::fn, dim3(p.a.Hkv * p.a.B, grid_y), dim3(C::kThreads), C::kLdsBytes, s, q);
+  q.pair_ktiles = plan.pair;
+  q.a.pieces = Pieces{plan.len, ws};
+  int grid_y = plan.pair ? (n_ktiles + 1) / 2 : n_ktiles;
+  if (plan.len > 0) grid_y = count_pieces(n_ktiles, plan.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
+  hipLaunchKernelGGL(KvKernel<D>::fn, dim3(heads, grid_y), dim3(C::kThreads), C::kLdsBytes, s, q);
+  if (plan.len > 0)
+    hipLaunchKernelGGL(attn_bwd_dkdv_join_kernel<D>, dim3(heads, n_ktiles, 2), dim3(256), 0, s, q, grid_y);
   return PICO_OK;
 }
 
@@ -915,13 +1079,68 @@ int launch_dq_impl(const BwdParams& p, hipStream_t s) {
   if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, NW, KT, kDelta, KS>), C::kLdsBytes))
     return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dq): cannot reserve %zu bytes of LDS", C::kLdsBytes);
   const int n_qtiles = (p.a.Sq + C::BM - 1) / C::BM;
-  hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NW, KT, kDelta, KS>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(C::kThreads), C::kLdsBytes, s, p);
+  BwdParams q = p;
+  int n = n_qtiles;
+  if (q.a.pieces.len > 0) {
+    n = count_pieces(n_qtiles, q.a.pieces.len, [&](int i) { return query_tile_trips(q.a, n_qtiles - 1 - i, C::BM, KT); });
+    if (n == n_qtiles) q.a.pieces.len = 0;
+  }
+  hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NW, KT, kDelta, KS>), dim3(p.a.Hq * p.a.B, n), dim3(C::kThreads), C::kLdsBytes, s, q);
+  if (q.a.pieces.len > 0)
+    hipLaunchKernelGGL((attn_bwd_dq_join_kernel<D, C::kQWaves, KT>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(64 * C::kQWaves), 0, s, q, n);
   return PICO_OK;
 }
 
 template <int D, int NW, int KT, int KS = 1>
 int launch_dq(const BwdParams& p, hipStream_t s) {
   return p.out ? launch_dq_impl<D, NW, KT, true, KS>(p, s) : launch_dq_impl<D, NW, KT, false, KS>(p, s);
+}
+
+// How the dQ launch is run: which kernel, and whether its query tiles are cut into pieces.
+struct DqPlan {
+  enum { kWaves4, kWaves8, kSplit4, kSplit8 } kernel;
+  int len = 0;
+  int64_t ws_bytes = 0;
+};
+DqPlan plan_dq(const AttnParams& a, int D, int64_t ws_bytes) {
+  DqPlan plan;
+  const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
+  auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
+  TripCost cost = {1.65, 1.8, 4.0, 0.0};
+  int bm = 128, kt = 64;
+  if (D == 64) {
+    const int64_t visible_keys = a.causal ? std::min<int64_t>(a.Sk, static_cast<int64_t>(a.q_offset) + a.Sq) : a.Sk;
+    // the forward's rules: eight waves per workgroup also for rectangular launches (every query sees at least as many
+    // keys as there are queries) with fewer workgroups than the square ones need
+    const bool rectangular = !a.causal || a.q_offset >= a.Sq;
+    // several generations of workgroups over short key ranges (a few trips each): two four-wave workgroups per CU hide
+    // each other's prologues and epilogues, which one eight-wave workgroup per CU cannot (B8 S768 51.3 -> 44.3 us,
+    // B16 S512 54.4 -> 48.1, B8 S1024 78.5 -> 72.9, B8 S1536 147.8 -> 144.3; from S2048 on, and with 512 workgroups,
+    // the eight-wave kernel is level or ahead)
+    if (groups(256) >= 768 && visible_keys <= 1536) plan.kernel = DqPlan::kWaves4;
+    else if (groups(256) >= 512) plan.kernel = DqPlan::kWaves8;
+    else if (groups(128) >= 512) plan.kernel = rectangular && groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
+    // few waves in all: two waves per 32 queries, 64 keys of every 128 each (rank 3 of 4 at configs[1] with eight waves
+    // per workgroup: 18.8 -> 17.9 us)
+    else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
+    bm = plan.kernel == DqPlan::kWaves8 ? 256 : plan.kernel == DqPlan::kSplit4 ? 64 : 128;
+    kt = plan.kernel >= DqPlan::kSplit4 ? 128 : 64;
+    cost = plan.kernel == DqPlan::kWaves8 ? TripCost{1.7, 1.5, 4.0, 0.0} : plan.kernel == DqPlan::kWaves4 ? TripCost{1.3, 0.78, 4.0, 0.0}
+         : plan.kernel == DqPlan::kSplit8 ? TripCost{1.6, 1.5, 4.0, 0.0} : TripCost{1.25, 0.8, 4.0, 0.0};
+  } else {
+    plan.kernel = groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
+    if (plan.kernel == DqPlan::kWaves8) {
+      bm = 256;
+      cost = {2.0, 2.87, 4.0, 0.0};
+    }
+  }
+  if (ws_bytes <= 0) return plan;
+  const int n_qtiles = (a.Sq + bm - 1) / bm;
+  cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);
+  auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, bm, kt); };
+  plan.len = choose_pieces(heads, n_qtiles, cost, ws_bytes, trips_of);
+  if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_qtiles, plan.len, trips_of) * cost.piece_bytes);
+  return plan;
 }
 
 }  // namespace
@@ -960,7 +1179,7 @@ namespace {
 int run_bwd(const char* fn, const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
             const float* lse, const float* delta, const void* out, float* delta_w, void* dq, const int64_t* dq_stride,
             int dq_dtype, int dq_accumulate, const int64_t* dkv_stride, int dkv_dtype, void* stream,
-            const RopeArgs* rope = nullptr) {
+            const RopeArgs* rope = nullptr, float* ws = nullptr, int64_t ws_bytes = 0) {
   if ((dkv_dtype != PICO_BF16 && dkv_dtype != PICO_F32) || (dq_dtype != PICO_BF16 && dq_dtype != PICO_F32))
     return fail(PICO_ERR_DTYPE, "%s: gradient dtype codes %d / %d not supported", fn, dq_dtype, dkv_dtype);
   if (dq_accumulate && dq_dtype != PICO_F32) return fail(PICO_ERR_DTYPE, "%s: accumulate needs fp32 gradients", fn);
@@ -1037,37 +1256,23 @@ int run_bwd(const char* fn, const pico_attn_desc* desc, const void* q, const pic
   auto run_dkdv = [&]() -> int {
     if (!have_k) return PICO_OK;
     // without queries the dK/dV kernel still runs: it writes (or adds) zeros
-    if (int rc = desc->D == 64 ? launch_dkdv<64>(p, s) : launch_dkdv<128>(p, s)) return rc;
+    if (int rc = desc->D == 64 ? launch_dkdv<64>(p, ws, ws_bytes, s) : launch_dkdv<128>(p, ws, ws_bytes, s)) return rc;
     return check_launch("pico_attn_bwd(dk/dv)");
   };
   auto run_dq = [&]() -> int {
     if (!have_q) return PICO_OK;
     // without keys the dQ kernel still runs: it writes (or adds) zeros
+    const DqPlan plan = plan_dq(p.a, desc->D, ws ? ws_bytes : 0);
+    BwdParams p_dq = p;
+    p_dq.a.pieces = Pieces{plan.len, ws};
     int rc;
-    const int64_t heads = static_cast<int64_t>(desc->B) * desc->Hq;
     if (desc->D == 64) {
-      auto groups = [&](int bm) { return heads * ((desc->Sq + bm - 1) / bm); };
-      const int64_t visible_keys = desc->causal ? std::min<int64_t>(desc->Sk, static_cast<int64_t>(desc->q_offset) + desc->Sq) : desc->Sk;
-      // the forward's rules: eight waves per workgroup also for rectangular launches (every query sees at least as many
-      // keys as there are queries) with fewer workgroups than the square ones need
-      const bool rectangular = !desc->causal || desc->q_offset >= desc->Sq;
-      // several generations of workgroups over short key ranges (a few trips each): two four-wave workgroups per CU hide
-      // each other's prologues and epilogues, which one eight-wave workgroup per CU cannot (B8 S768 51.3 -> 44.3 us,
-      // B16 S512 54.4 -> 48.1, B8 S1024 78.5 -> 72.9, B8 S1536 147.8 -> 144.3; from S2048 on, and with 512 workgroups,
-      // the eight-wave kernel is level or ahead)
-      if (groups(256) >= 768 && visible_keys <= 1536) rc = launch_dq<64, 4, 64>(p, s);
-      else if (groups(256) >= 512) rc = launch_dq<64, 8, 64>(p, s);
-      else if (groups(128) >= 512) {
-        if (rectangular && groups(256) >= 256) rc = launch_dq<64, 8, 64>(p, s);
-        else rc = launch_dq<64, 4, 64>(p, s);
-      }
-      // few waves in all: two waves per 32 queries, 64 keys of every 128 each (rank 3 of 4 at configs[1] with eight waves
-      // per workgroup: 18.8 -> 17.9 us)
-      else if (groups(128) >= 256 && rectangular && visible_keys >= 512) rc = launch_dq<64, 8, 128, 2>(p, s);
-      else rc = launch_dq<64, 4, 128, 2>(p, s);
+      if (plan.kernel == DqPlan::kWaves8) rc = launch_dq<64, 8, 64>(p_dq, s);
+      else if (plan.kernel == DqPlan::kWaves4) rc = launch_dq<64, 4, 64>(p_dq, s);
+      else if (plan.kernel == DqPlan::kSplit8) rc = launch_dq<64, 8, 128, 2>(p_dq, s);
+      else rc = launch_dq<64, 4, 128, 2>(p_dq, s);
     } else {
-      if (heads * ((desc->Sq + 255) / 256) >= 256) rc = launch_dq<128, 8, 64>(p, s);
-      else rc = launch_dq<128, 4, 64>(p, s);
+      rc = plan.kernel == DqPlan::kWaves8 ? launch_dq<128, 8, 64>(p_dq, s) : launch_dq<128, 4, 64>(p_dq, s);
     }
     if (rc) return rc;
     return check_launch("pico_attn_bwd(dq)");
@@ -1096,7 +1301,7 @@ pico_kv_chunks one_chunk(const pico_attn_desc* desc, const void* k, const void* 
 int run_bwd_with_out(const char* fn, const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
                      const void* out, int out_dtype, const float* lse, float* delta, void* dq, const int64_t* dq_stride,
                      int dq_dtype, int dq_accumulate, const int64_t* dkv_stride, int dkv_dtype, void* stream,
-                     const RopeArgs* rope) {
+                     const RopeArgs* rope, float* ws = nullptr, int64_t ws_bytes = 0) {
   if (out_dtype != PICO_BF16 && out_dtype != PICO_F32)
     return fail(PICO_ERR_DTYPE, "%s: out dtype code %d not supported", fn, out_dtype);
   if (desc->B == 0) return PICO_OK;
@@ -1105,10 +1310,10 @@ int run_bwd_with_out(const char* fn, const pico_attn_desc* desc, const void* q, 
   if (!in_kernel) {
     if (int rc = pico_attn_bwd_preprocess(desc, dout, out, out_dtype, delta, nullptr, stream)) return rc;
     return run_bwd(fn, desc, q, kv, dout, lse, delta, nullptr, nullptr, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride,
-                   dkv_dtype, stream, rope);
+                   dkv_dtype, stream, rope, ws, ws_bytes);
   }
   return run_bwd(fn, desc, q, kv, dout, lse, delta, out, delta, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride, dkv_dtype,
-                 stream, rope);
+                 stream, rope, ws, ws_bytes);
 }
 
 int rope_args(const char* fn, const pico_attn_desc* desc, const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset,
@@ -1162,22 +1367,44 @@ extern "C" int pico_attn_bwd_rope(const pico_attn_desc* desc, const void* q_rot,
                           dkv_stride, dkv_dtype, stream, &r);
 }
 
-extern "C" int pico_attn_bwd_chunks(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
-                                    const void* out, int out_dtype, const float* lse, float* delta, void* dq,
-                                    const int64_t* dq_stride, int dq_dtype, int dq_accumulate, const int64_t* dkv_stride,
-                                    int dkv_dtype, const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset,
-                                    void* stream) {
+extern "C" int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
+  if (!desc || chunk_count < 1 || (desc->D != 64 && desc->D != 128) || desc->B <= 0 || desc->Hkv <= 0 || desc->Hq % desc->Hkv != 0 ||
+      desc->Hq <= 0 || desc->Sq <= 0 || desc->Sk <= 0)
+    return 0;
+  AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
+  a.kv.count = chunk_count;
+  a.kv.len = desc->Sk / chunk_count;
+  const int64_t dkdv = desc->D == 64 ? plan_dkdv<64>(a, PICO_ATTN_MAX_WORKSPACE).ws_bytes : plan_dkdv<128>(a, PICO_ATTN_MAX_WORKSPACE).ws_bytes;
+  return std::max(dkdv, plan_dq(a, desc->D, PICO_ATTN_MAX_WORKSPACE).ws_bytes);   // (the two kernels run one after the other)
+}
+
+extern "C" int pico_attn_bwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
+                                       const void* out, int out_dtype, const float* lse, float* delta, void* dq,
+                                       const int64_t* dq_stride, int dq_dtype, int dq_accumulate, const int64_t* dkv_stride,
+                                       int dkv_dtype, const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset,
+                                       void* workspace, int64_t workspace_bytes, void* stream) {
   const char* fn = "pico_attn_bwd_chunks";
   if (int rc = check_attn_desc(fn, desc)) return rc;
   if (!kv) return fail(PICO_ERR_NULL, "%s: the chunk list is NULL", fn);
+  if (!aligned16(workspace)) return fail(PICO_ERR_ALIGN, "%s: the workspace must be 16-byte aligned", fn);
   if (desc->B == 0) return PICO_OK;
   RopeArgs r;
   if (rope) {
     if (int rc = rope_args(fn, desc, rope, q_pos_offset, k_pos_offset, r)) return rc;
   }
+  float* ws = static_cast<float*>(workspace);
   if (out)
     return run_bwd_with_out(fn, desc, q, kv, dout, out, out_dtype, lse, delta, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride,
-                            dkv_dtype, stream, rope ? &r : nullptr);
-  return run_bwd(fn, desc, q, kv, dout, lse, delta, nullptr, nullptr, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride,
-                 dkv_dtype, stream, rope ? &r : nullptr);
+                            dkv_dtype, stream, rope ? &r : nullptr, ws, workspace_bytes);
+  return run_bwd(fn, desc, q, kv, dout, lse, delta, nullptr, nullptr, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride, dkv_dtype,
+                 stream, rope ? &r : nullptr, ws, workspace_bytes);
+}
+
+extern "C" int pico_attn_bwd_chunks(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,
+                                    const void* out, int out_dtype, const float* lse, float* delta, void* dq,
+                                    const int64_t* dq_stride, int dq_dtype, int dq_accumulate, const int64_t* dkv_stride,
+                                    int dkv_dtype, const pico_rope_tables* rope, int q_pos_offset, int k_pos_offset,
+                                    void* stream) {
+  return pico_attn_bwd_chunks_ws(desc, q, kv, dout, out, out_dtype, lse, delta, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride,
+                                 dkv_dtype, rope, q_pos_offset, k_pos_offset, nullptr, 0, stream);
 }

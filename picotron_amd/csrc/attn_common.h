@@ -302,13 +302,23 @@ __device__ __forceinline__ void rope_unrotate_acc(f32x16 (&acc)[D / 32], const R
 }
 
 // K / V as a list of equally long chunks that lie one after another along the key axis: key j of the launch is row
-// j % len of chunk j / len.  One chunk of len = Sk is the plain case.  With several chunks len is a multiple of every
-// kernel's staged key tile (128), so no tile straddles two chunks.
+// j % len of chunk j / len.  One chunk of len = Sk is the plain case.  A staged key tile belongs to one chunk: with a len
+// that is no multiple of the tile the last tile of every chunk is a partial one (its rows past the chunk read as zeros and
+// are masked), and tiles are counted chunk by chunk.
 constexpr int kMaxChunks = PICO_MAX_KV_CHUNKS;
 struct KvChunks {
   const __bf16* k[kMaxChunks];
   const __bf16* v[kMaxChunks];
   int count, len;
+};
+
+// A launch that is cut into pieces: too few workgroups for the GPU, or a few long ones among many short (under a causal
+// mask, and with the query heads of a GQA group walked by one workgroup in dK/dV).  The trips of an output tile are dealt
+// to ceil(trips / len) workgroups; where that is more than one, each leaves its accumulators in `ws` as they lie in its
+// registers, and a second launch adds the pieces of a tile in their order and runs the kernel's own epilogue on the sum.
+struct Pieces {
+  int len;     // most trips of a piece; 0: tiles are not cut
+  float* ws;
 };
 
 struct AttnParams {
@@ -318,7 +328,127 @@ struct AttnParams {
   int causal, q_offset;
   float sm_scale;
   int64_t qs[3], ks[3], vs[3], os[3];
+  Pieces pieces;
 };
+
+__host__ __device__ inline int pieces_of(int trips, int len) { return len <= 0 || trips <= len ? 1 : (trips + len - 1) / len; }
+
+// Which (tile, piece) workgroup `y` of a head is, tiles in order, and how many pieces its tile has.  64 tiles at a time, one
+// per lane: a prefix sum over their numbers of pieces and a ballot.  All lanes of the wave take part.
+struct Piece {
+  int tile, part, parts;
+};
+template <typename F>
+__device__ __forceinline__ Piece find_piece(int y, int n_tiles, int len, const F& trips_of) {
+  const int lane = threadIdx.x % kWave;
+  for (int base = 0; base < n_tiles; base += kWave) {
+    const int mine = base + lane < n_tiles ? pieces_of(trips_of(base + lane), len) : 0;
+    int sum = mine;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int left = __shfl_up(sum, off, kWave);
+      if (lane >= off) sum += left;
+    }
+    const uint64_t past = __ballot(sum > y);
+    if (past != 0) {
+      const int at = __builtin_ctzll(past);
+      const int parts = __builtin_amdgcn_readlane(mine, at), upto = __builtin_amdgcn_readlane(sum, at);
+      return {base + at, y - (upto - parts), parts};
+    }
+    y -= __builtin_amdgcn_readlane(sum, kWave - 1);
+  }
+  return {n_tiles - 1, 0, 0};   // (not reached: the grid has as many workgroups as there are pieces)
+}
+// the number of pieces in front of `tile`, i.e. the y of its first one
+template <typename F>
+__device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of) {
+  const int lane = threadIdx.x % kWave;
+  int sum = 0;
+  for (int i = lane; i < tile; i += kWave) sum += pieces_of(trips_of(i), len);
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+
+// Host: the piece length for a launch, from what a trip and a workgroup cost.  `alone_us` is a trip of a workgroup that has
+// its CU to itself, `full_us` the CU's time per trip where it is shared, `fixed_us` a workgroup's start and end.  Not cutting
+// (0) stands as one of the choices; cutting has to win by its second launch and by the traffic of the pieces.
+struct TripCost {
+  double alone_us, full_us, fixed_us, piece_bytes;
+};
+template <typename F>
+int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, int64_t ws_bytes, const F& trips_of, double uncut_us = -1.0) {
+  constexpr double kCus = 256.0, kSecondLaunchUs = 5.0, kBytesPerUs = 4e6;
+  auto estimate = [&](int len, int64_t* pieces) {
+    int longest = 0;
+    int64_t total = 0, n = 0, cut = 0;
+    for (int i = 0; i < n_tiles; ++i) {
+      const int t = trips_of(i), k = pieces_of(t, len);
+      longest = std::max(longest, (t + k - 1) / k);
+      total += t;
+      n += k;
+      if (k > 1) cut += k;
+    }
+    *pieces = n;
+    const double span = longest * c.alone_us + c.fixed_us, load = heads * (total * c.full_us + n * c.fixed_us * 0.5) / kCus;
+    return std::max(span, load) + 0.25 * std::min(span, load) + (cut ? kSecondLaunchUs + 2.0 * heads * cut * c.piece_bytes / kBytesPerUs : 0.0);
+  };
+  if (heads * n_tiles > 4 * 512) return 0;   // enough workgroups that their lengths even out
+  int64_t n = 0;
+  double best_us = estimate(0, &n);
+  if (uncut_us >= 0.0) best_us = uncut_us;
+  int best = 0;
+  for (int len : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+    const double us = estimate(len, &n);
+    if (n > 65535 || heads * n * c.piece_bytes > static_cast<double>(ws_bytes)) continue;
+    if (us < 0.95 * best_us) {
+      best_us = us;
+      best = len;
+    }
+  }
+  return best;
+}
+template <typename F>
+int count_pieces(int n_tiles, int len, const F& trips_of) {
+  int n = 0;
+  for (int i = 0; i < n_tiles; ++i) n += pieces_of(trips_of(i), len);
+  return n;
+}
+
+// accumulators in register order, 16 bytes per lane and piece of a row block: what a cut tile's pieces leave in memory
+template <int N>
+__device__ __forceinline__ void put_acc(float* dst, const f32x16 (&acc)[N], int lane) {
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<f32x4*>(dst + ((db * 4 + j) * kWave + lane) * 4) =
+          f32x4{acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]};
+}
+template <int N>
+__device__ __forceinline__ void get_acc(const float* src, f32x4 (&raw)[N][4], int lane) {
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) raw[db][j] = *reinterpret_cast<const f32x4*>(src + ((db * 4 + j) * kWave + lane) * 4);
+}
+
+// How many key tiles of KT keys lie in front of position `end`, counted chunk by chunk.
+__host__ __device__ inline int tiles_before(const KvChunks& kv, int end, int KT) {
+  if (kv.count == 1) return (end + KT - 1) / KT;
+  const int whole = end / kv.len, rest = end - whole * kv.len;
+  return whole * ((kv.len + KT - 1) / KT) + (rest + KT - 1) / KT;
+}
+
+// Key tiles of KT keys that query tile `qtile` of BM queries sees: the trips of a forward or dQ workgroup.
+__host__ __device__ inline int query_tile_trips(const AttnParams& a, int qtile, int BM, int KT) {
+  int end = a.Sk;
+  if (a.causal) {
+    const int hi = (qtile + 1) * BM < a.Sq ? (qtile + 1) * BM : a.Sq, vis = a.q_offset + hi;
+    end = vis < a.Sk ? vis : a.Sk;
+  }
+  return tiles_before(a.kv, end, KT);
+}
 
 // A cursor over the key tiles of KT keys, in order, across the chunks: wave-uniform, so it lives in scalar registers;
 // stepping inside a chunk is four adds, a new chunk re-reads its base addresses from the kernel arguments.
@@ -329,14 +459,22 @@ struct KvCursor {
   uint32_t k_step, v_step;
   int tiles_left, chunk, tiles_per_chunk;
   int64_t k_head, v_head;       // element offset of the (batch, kv head) inside every chunk
-  __device__ __forceinline__ void open(const AttnParams& a, int chunk_, int b, int hkv, int KT) {
-    chunk = chunk_;
+  // opens at the tile `tile` of the launch
+  __device__ __forceinline__ void open(const AttnParams& a, int tile, int b, int hkv, int KT) {
     k_head = b * a.ks[0] + hkv * a.ks[1];
     v_head = b * a.vs[0] + hkv * a.vs[1];
     k_step = static_cast<uint32_t>(KT * a.ks[2] * 2);
     v_step = static_cast<uint32_t>(KT * a.vs[2] * 2);
     tiles_per_chunk = (a.kv.len + KT - 1) / KT;
+    chunk = 0;
+    if (tile > 0 && a.kv.count > 1) chunk = tile / tiles_per_chunk;
     enter(a);
+    if (tile > 0) {
+      const int skip = tile - chunk * tiles_per_chunk;
+      k += static_cast<int64_t>(skip) * k_step;  k_left -= static_cast<uint32_t>(skip) * k_step;
+      v += static_cast<int64_t>(skip) * v_step;  v_left -= static_cast<uint32_t>(skip) * v_step;
+      tiles_left -= skip;
+    }
   }
   __device__ __forceinline__ void enter(const AttnParams& a) {
     k = reinterpret_cast<const char*>(a.kv.k[chunk] + k_head);
@@ -352,6 +490,22 @@ struct KvCursor {
     } else {
       k += k_step;  k_left -= k_step;
       v += v_step;  v_left -= v_step;
+    }
+  }
+};
+// The positions of the tile being computed: its first key, and the end of its chunk (keys from there on do not exist).
+struct KvPosition {
+  int key0, end;
+  __device__ __forceinline__ void open(const KvChunks& kv, int tile, int KT) {
+    const int per = (kv.len + KT - 1) / KT, chunk = tile > 0 && kv.count > 1 ? tile / per : 0;
+    key0 = chunk * kv.len + (tile - chunk * per) * KT;
+    end = (chunk + 1) * kv.len;
+  }
+  __device__ __forceinline__ void next(const KvChunks& kv, int KT) {
+    key0 += KT;
+    if (key0 >= end) {   // (also where the tile ended exactly with its chunk)
+      key0 = end;
+      end += kv.len;
     }
   }
 };

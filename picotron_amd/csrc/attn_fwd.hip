@@ -55,6 +55,31 @@ struct FwdCfg {
   static_assert(KT % BN == 0 && (KT * kVecPerRow) % kThreads == 0, "tile must split evenly over the threads");
 };
 
+// what a wave of a piece leaves: O^T accumulators, m and l per lane
+constexpr int fwd_piece_floats(int D) { return (D / 32) * 16 * kWave + 2 * kWave; }
+
+// lse per query; the wave's 32 output rows leave through its piece of LDS as whole lines
+template <int D>
+__device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* region, f32x16 (&o)[D / 32], float m_run, float l_run,
+                                             int b, int hq, int row0, int lane) {
+  const AttnParams& a = p.a;
+  const int row = row0 + lane % 32;
+  const float l_tot = half_sum(l_run);
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  if (row < a.Sq && lane < 32)
+    p.lse[(static_cast<int64_t>(b) * a.Hq + hq) * a.Sq + row] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
+  // normalise in place: 1 / l differs per lane (row), the store helper applies one scale to all
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[db][i] *= inv;
+  const int64_t off = b * a.os[0] + hq * a.os[1] + static_cast<int64_t>(row0) * a.os[2];
+  if (p.out_f32)
+    wave_store_rows<D, true>(region, o, 1.f, static_cast<float*>(p.out) + off, a.os[2], a.Sq - row0, lane, false, false);
+  else
+    wave_store_rows<D, false>(region, o, 1.f, static_cast<__bf16*>(p.out) + off, a.os[2], a.Sq - row0, lane, false, false);
+}
+
 template <int D, int QB, int NW, int KT, int KS = 1>
 __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
@@ -64,12 +89,16 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
 
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
+  // key tiles that the queries of a tile see (the last of a head's query tiles comes first in the order below)
+  auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, BM, KT); };
   // grid = (Hq * B, query tiles): x runs fastest in dispatch order, so every head's last query tile (the
   // longest under a causal mask) starts first and the short tiles fill in behind.  When the whole launch is
   // resident at once (pair_order), workgroups j and j + (half the grid) share a CU, so the second half runs
   // the short tiles in ASCENDING order: every CU then holds a long and a short tile of equal total length.
   const int y = static_cast<int>(blockIdx.y), half = (n_qtiles + 1) / 2;
-  const int qtile = (p.pair_order && y >= half) ? y - half : n_qtiles - 1 - y;
+  Piece piece = {y, 0, 1};
+  if (a.pieces.len > 0) piece = find_piece(y, n_qtiles, a.pieces.len, trips_of);
+  const int qtile = (p.pair_order && y >= half) ? y - half : n_qtiles - 1 - piece.tile;
   const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
   const int hkv = hq / (a.Hq / a.Hkv);
   const int q0 = qtile * BM;
@@ -96,7 +125,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
       // RoPE on the wave's own queries, once per query in the whole launch (every query belongs to one wave)
       const bool qlive = qrow[qb] < a.Sq;
       rope_rotate_fragments<D>(qf[qb], p.rope, qlive ? p.rope.q_pos0 + qrow[qb] : 0, h);
-      if (p.q_rot != nullptr && qlive && (KS == 1 || ks == 0)) {
+      if (p.q_rot != nullptr && qlive && (KS == 1 || ks == 0) && piece.part == 0) {
         __bf16* dst = p.q_rot + b * p.qrs[0] + hq * p.qrs[1] + static_cast<int64_t>(qrow[qb]) * p.qrs[2];
 #pragma unroll
         for (int s = 0; s < D / 16; ++s) *reinterpret_cast<bf16x8*>(dst + 16 * s + 8 * h) = qf[qb][s];
@@ -117,7 +146,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[qb][db][i] = 0.f;
-    if (p.merge && ks == 0 && qrow[qb] < a.Sq) {
+    if (p.merge && ks == 0 && piece.part == 0 && qrow[qb] < a.Sq) {
       // continue from (out, lse) of the earlier blocks: m = lse, l = 1, acc = out
       const float prev = p.lse[lse_row0 + qrow[qb]];
       if (prev != -INFINITY) {
@@ -145,7 +174,11 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
     kv_end = vis < a.Sk ? vis : a.Sk;
     if (kv_end < 0) kv_end = 0;
   }
-  const int ntiles = (kv_end + KT - 1) / KT;
+  int t_first = 0, ntiles = tiles_before(a.kv, kv_end, KT);
+  if (piece.parts > 1) {
+    t_first = ntiles * piece.part / piece.parts;
+    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
+  }
 
   // ---- global -> register -> LDS staging of one K/V tile of KT keys, with buffer loads: a wave-uniform
   //      resource per tile (first key row, bytes left in the sequence) plus per-lane byte offsets that are
@@ -162,7 +195,9 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   }
   // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
   KvCursor<D> cur;
-  cur.open(a, 0, b, hkv, KT);
+  cur.open(a, t_first, b, hkv, KT);
+  KvPosition pos;
+  pos.open(a.kv, t_first, KT);
   auto load_tile = [&]() {  // the next tile of KT keys
     const buffer_rsrc kb = make_buffer(cur.k, cur.k_left), vb = make_buffer(cur.v, cur.v_left);
 #pragma unroll
@@ -195,7 +230,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   if (ntiles > 1) load_tile();
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t) {
+  for (int t = 0; t < ntiles; ++t, pos.next(a.kv, KT)) {
     // stage tile t+1 into the other buffer (its readers finished before the barrier that ended trip t-1)
     if (t + 1 < ntiles) {
       store_tile((t + 1) & 1);
@@ -207,8 +242,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
-      const int k0 = t * KT + sub * BN;
-      if (k0 >= kv_end) break;
+      const int k0 = pos.key0 + sub * BN;
+      if (k0 >= kv_end || k0 >= pos.end) break;
       const __bf16* sKs = sK + sub * BN * LDK;
       const __bf16* sVs = sV + sub * BN * LDV;
 #pragma unroll
@@ -257,8 +292,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
             }
           }
         }
-        // ---- mask (only for tiles that straddle the diagonal or the end of K)
-        const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || (k0 + BN > a.Sk);
+        // ---- mask (only for tiles that straddle the diagonal or the end of their chunk)
+        const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || (k0 + BN > pos.end);
         if (need_mask) {
           // the asm statement keeps this a real (wave-uniform) branch: without it the compiler turns the
           // block into per-element selects that every tile pays for
@@ -269,7 +304,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
               const int key = k0 + 32 * mb + 8 * (i / 4) + 4 * h + (i % 4);
-              if (key > qpos || key >= a.Sk) s_acc[mb][i] = -INFINITY;
+              if (key > qpos || key >= pos.end) s_acc[mb][i] = -INFINITY;
             }
         }
         // ---- online softmax.  The running maximum is only raised (and O, l rescaled) when some query of
@@ -368,28 +403,58 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
     static_assert(C::kQWaves * kRowRegionBytes <= C::kQWaves * C::kExchangeBytes, "store pieces lie below the exchange areas read above");
   }
 
-  // ---- epilogue: lse per query; the wave's 32 output rows leave through its piece of LDS as whole lines
-  //      (the loop ended on a barrier, so the tile buffers are free)
+  if constexpr (QB == 1) {
+    if (piece.parts > 1) {   // one piece of several: the state leaves as it is (l per wave half)
+      float* dst = a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * fwd_piece_floats(D);
+      put_acc<D / 32>(dst, o[0], lane);
+      dst[(D / 32) * 16 * kWave + lane] = m_run[0];
+      dst[(D / 32) * 16 * kWave + kWave + lane] = l_run[0];
+      return;
+    }
+  }
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    const float l_tot = half_sum(l_run[qb]);
-    const bool live = qrow[qb] < a.Sq;
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (live && h == 0)
-      p.lse[lse_row0 + qrow[qb]] = l_tot > 0.f ? (m_run[qb] + fast_log2(l_tot)) * kLn2 : -INFINITY;
-    // normalise in place: 1 / l differs per lane (row), the store helper applies one scale to all
+  for (int qb = 0; qb < QB; ++qb)
+    fwd_epilogue<D>(p, smem_raw + (wave * QB + qb) * kRowRegionBytes, o[qb], m_run[qb], l_run[qb], b, hq, q0 + (qw * QB + qb) * 32, lane);
+}
+
+// The pieces of every cut query tile put together: a wave per 32 queries merges the pieces' states, which lie as the pieces'
+// registers held them, and ends as the kernel above does.
+template <int D, int QW, int KT>
+__global__ __launch_bounds__(64 * QW) void attn_fwd_join_kernel(const FwdParams p, const int pieces_per_head) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem_raw[QW * kRowRegionBytes];
+  const AttnParams& a = p.a;
+  constexpr int BM = 32 * QW;
+  const int n_qtiles = (a.Sq + BM - 1) / BM, tile = static_cast<int>(blockIdx.y);
+  auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, BM, KT); };
+  const int parts = pieces_of(trips_of(tile), a.pieces.len);
+  if (parts == 1) return;   // (its workgroup has written the tile)
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
+  const int row0 = (n_qtiles - 1 - tile) * BM + wave * 32;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * pieces_per_head + first_piece(tile, a.pieces.len, trips_of);
+  constexpr int kAcc = (D / 32) * 16 * kWave;
+  const float* src = a.pieces.ws + (first * QW + wave) * fwd_piece_floats(D);
+  constexpr int64_t kStep = static_cast<int64_t>(QW) * fwd_piece_floats(D);
+  float m = -INFINITY, l = 0.f;
+  for (int j = 0; j < parts; ++j) m = fmaxf(m, src[j * kStep + kAcc + lane]);
+  f32x16 o[D / 32];
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
+  for (int j = 0; j < parts; ++j) {
+    const float* sj = src + j * kStep;
+    const float mj = sj[kAcc + lane], lj = sj[kAcc + kWave + lane];
+    f32x4 raw[D / 32][4];
+    get_acc<D / 32>(sj, raw, lane);
+    const float aj = mj == -INFINITY ? 0.f : fast_exp2(mj - m);
+    l += aj * lj;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[qb][db][i] *= inv;
-    unsigned char* region = smem_raw + (wave * QB + qb) * kRowRegionBytes;
-    const int row0 = q0 + (qw * QB + qb) * 32;
-    const int64_t off = b * a.os[0] + hq * a.os[1] + static_cast<int64_t>(row0) * a.os[2];
-    if (p.out_f32)
-      wave_store_rows<D, true>(region, o[qb], 1.f, static_cast<float*>(p.out) + off, a.os[2], a.Sq - row0, lane, false, false);
-    else
-      wave_store_rows<D, false>(region, o[qb], 1.f, static_cast<__bf16*>(p.out) + off, a.os[2], a.Sq - row0, lane, false, false);
+      for (int i = 0; i < 16; ++i) o[db][i] += aj * raw[db][i / 4][i % 4];
   }
+  fwd_epilogue<D>(p, smem_raw + wave * kRowRegionBytes, o, m, l, b, hq, row0, lane);
 }
 
 template <int D, int QB, int NW, int KT, int KS = 1>
@@ -404,7 +469,15 @@ int launch(const FwdParams& p, hipStream_t s) {
   // generations of workgroups and longest-first is the better order -- 160 -> 137 us at B1 H32 S4096)
   constexpr bool kTwoPerCu = !(D >= 128 && NW == 8);
   q.pair_order = kTwoPerCu && p.a.causal && n_qtiles >= 2 && static_cast<int64_t>(p.a.Hq) * p.a.B * n_qtiles <= 512;
-  hipLaunchKernelGGL((attn_fwd_kernel<D, QB, NW, KT, KS>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(C::kThreads), C::kLdsBytes, s, q);
+  int n = n_qtiles;
+  if (q.a.pieces.len > 0) {
+    n = count_pieces(n_qtiles, q.a.pieces.len, [&](int i) { return query_tile_trips(q.a, n_qtiles - 1 - i, C::BM, KT); });
+    q.pair_order = 0;
+    if (n == n_qtiles) q.a.pieces.len = 0;
+  }
+  hipLaunchKernelGGL((attn_fwd_kernel<D, QB, NW, KT, KS>), dim3(p.a.Hq * p.a.B, n), dim3(C::kThreads), C::kLdsBytes, s, q);
+  if (q.a.pieces.len > 0)
+    hipLaunchKernelGGL((attn_fwd_join_kernel<D, C::kQWaves, KT>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(64 * C::kQWaves), 0, s, q, n);
   return PICO_OK;
 }
 
@@ -455,6 +528,7 @@ AttnParams make_params(const pico_attn_desc* d, const void* q, const void* k, co
   a.causal = d->causal != 0;
   a.q_offset = d->q_offset;
   a.sm_scale = d->sm_scale;
+  a.pieces = Pieces{0, nullptr};
   for (int i = 0; i < 3; ++i) {
     a.qs[i] = d->q_stride[i]; a.ks[i] = d->k_stride[i]; a.vs[i] = d->v_stride[i]; a.os[i] = d->o_stride[i];
   }
@@ -467,8 +541,9 @@ int set_chunks(const char* fn, const pico_attn_desc* d, const pico_kv_chunks* kv
     return fail(PICO_ERR_SHAPE, "%s: %d chunks (1 to %d supported)", fn, kv->count, kMaxChunks);
   if (kv->chunk_len < 0 || static_cast<int64_t>(kv->count) * kv->chunk_len != d->Sk)
     return fail(PICO_ERR_SHAPE, "%s: %d chunks of %d keys do not make Sk=%d", fn, kv->count, kv->chunk_len, d->Sk);
-  if (kv->count > 1 && kv->chunk_len % 128 != 0)
-    return fail(PICO_ERR_SHAPE, "%s: with several chunks the chunk length (%d) must be a multiple of 128", fn, kv->chunk_len);
+  // a tile belongs to one chunk: chunks of one 64-key step or less would leave most of every tile empty
+  if (kv->count > 1 && kv->chunk_len <= 64)
+    return fail(PICO_ERR_SHAPE, "%s: with several chunks the chunk length (%d) must be over 64 (best a multiple of 128)", fn, kv->chunk_len);
   // a chunk is addressed through the same 32-bit window as a whole tensor
   if (((kv->chunk_len - 1) * std::max(d->k_stride[2], d->v_stride[2]) + d->D) * 2 >= (1LL << 32))
     return fail(PICO_ERR_STRIDE, "%s: the rows of one head must span less than 4 GiB", fn);
@@ -503,9 +578,58 @@ bool rows_disjoint(const int64_t* st, int B, int H, int S, int D) {
   return true;
 }
 
+// How a launch is run: which kernel, and whether its query tiles are cut into pieces (see Pieces).
+struct FwdPlan {
+  enum { kWaves4, kWaves8, kSplit4, kSplit8 } kernel;
+  int len = 0;               // piece length in staged key tiles, 0: not cut
+  int64_t ws_bytes = 0;      // what the pieces need
+};
+
+FwdPlan plan_fwd(const AttnParams& a, int D, int64_t ws_bytes) {
+  FwdPlan plan;
+  const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
+  auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
+  TripCost cost = {1.5, 1.1, 4.0, 0.0};
+  int bm = 128, kt = 64;
+  // Tile choice for D = 64: more waves per workgroup share each staged K/V tile (fewer barriers and
+  // global loads per MFMA), but the launch still has to fill 256 CUs, so small problems get small tiles.
+  if (D == 64) {
+    const int64_t visible_keys = a.causal ? std::min<int64_t>(a.Sk, static_cast<int64_t>(a.q_offset) + a.Sq) : a.Sk;
+    // a launch whose queries all see at least as many keys as they are themselves (a rank's share of a ring, a dense
+    // block): the waves of a workgroup then do nearly equal work, and workgroups of eight waves, which share every
+    // staged tile among twice as many waves, pay even where the launch has few of them
+    const bool rectangular = !a.causal || a.q_offset >= a.Sq;
+    if (groups(256) >= 512) plan.kernel = FwdPlan::kWaves8;
+    // (measured at B8, 256 queries x 1024 keys of every head: 26.9 us with eight waves, 30.1 us with four)
+    else if (groups(128) >= 512) plan.kernel = rectangular && groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
+    // few waves in all: two waves per 32 queries, 64 keys of every 128 each -- in workgroups of eight waves (128 queries)
+    // when those still cover the CUs and the launch is rectangular (one rank's share of configs[1]: 19.8 -> 16.9 us for
+    // rank 3 of 4; on a whole causal sequence, or with 256 keys, the smaller workgroups are a few percent faster)
+    else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? FwdPlan::kSplit8 : FwdPlan::kSplit4;
+    bm = plan.kernel == FwdPlan::kWaves8 ? 256 : plan.kernel == FwdPlan::kSplit4 ? 64 : 128;
+    kt = plan.kernel >= FwdPlan::kSplit4 ? 128 : 64;
+    cost = plan.kernel == FwdPlan::kWaves8 ? TripCost{1.6, 1.28, 4.0, 0.0} : plan.kernel == FwdPlan::kWaves4 ? TripCost{1.2, 0.66, 4.0, 0.0}
+         : plan.kernel == FwdPlan::kSplit8 ? TripCost{1.5, 1.3, 4.0, 0.0} : TripCost{1.35, 0.7, 4.0, 0.0};
+  } else {
+    // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
+    plan.kernel = groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
+    if (plan.kernel == FwdPlan::kWaves8) {
+      bm = 256;
+      cost = {1.6, 2.13, 4.0, 0.0};
+    }
+  }
+  if (ws_bytes <= 0) return plan;
+  const int n_qtiles = (a.Sq + bm - 1) / bm;
+  cost.piece_bytes = 4.0 * (bm / 32) * fwd_piece_floats(D);
+  auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, bm, kt); };
+  plan.len = choose_pieces(heads, n_qtiles, cost, ws_bytes, trips_of);
+  if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_qtiles, plan.len, trips_of) * cost.piece_bytes);
+  return plan;
+}
+
 int run_fwd(const char* fn, const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out, float* lse,
             int out_dtype, int merge, const pico_rope_tables* rope, int q_pos_offset, void* q_rot,
-            const int64_t* q_rot_stride, void* stream) {
+            const int64_t* q_rot_stride, void* stream, float* workspace = nullptr, int64_t ws_bytes = 0) {
   if (int rc = check_attn_desc(fn, desc)) return rc;
   if (out_dtype != PICO_BF16 && out_dtype != PICO_F32)
     return fail(PICO_ERR_DTYPE, "%s: out dtype code %d not supported", fn, out_dtype);
@@ -541,33 +665,16 @@ int run_fwd(const char* fn, const pico_attn_desc* desc, const void* q, const pic
     }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // Tile choice for D = 64: more waves per workgroup share each staged K/V tile (fewer barriers and
-  // global loads per MFMA), but the launch still has to fill 256 CUs, so small problems get small tiles.
+  const FwdPlan plan = plan_fwd(p.a, desc->D, workspace ? ws_bytes : 0);
+  p.a.pieces = Pieces{plan.len, workspace};
   int rc;
   if (desc->D == 64) {
-    const int64_t heads = static_cast<int64_t>(desc->B) * desc->Hq;
-    auto groups = [&](int bm) { return heads * ((desc->Sq + bm - 1) / bm); };
-    const int64_t visible_keys = desc->causal ? std::min<int64_t>(desc->Sk, static_cast<int64_t>(desc->q_offset) + desc->Sq) : desc->Sk;
-    // a launch whose queries all see at least as many keys as they are themselves (a rank's share of a ring, a dense
-    // block): the waves of a workgroup then do nearly equal work, and workgroups of eight waves, which share every
-    // staged tile among twice as many waves, pay even where the launch has few of them
-    const bool rectangular = !desc->causal || desc->q_offset >= desc->Sq;
-    if (groups(256) >= 512) rc = launch<64, 1, 8, 64>(p, s);
-    else if (groups(128) >= 512) {
-      // (measured at B8, 256 queries x 1024 keys of every head: 26.9 us with eight waves, 30.1 us with four)
-      if (rectangular && groups(256) >= 256) rc = launch<64, 1, 8, 64>(p, s);
-      else rc = launch<64, 1, 4, 64>(p, s);
-    }
-    // few waves in all: two waves per 32 queries, 64 keys of every 128 each -- in workgroups of eight waves (128 queries)
-    // when those still cover the CUs and the launch is rectangular (one rank's share of configs[1]: 19.8 -> 16.9 us for
-    // rank 3 of 4; on a whole causal sequence, or with 256 keys, the smaller workgroups are a few percent faster)
-    else if (groups(128) >= 256 && rectangular && visible_keys >= 512) rc = launch<64, 1, 8, 128, 2>(p, s);
+    if (plan.kernel == FwdPlan::kWaves8) rc = launch<64, 1, 8, 64>(p, s);
+    else if (plan.kernel == FwdPlan::kWaves4) rc = launch<64, 1, 4, 64>(p, s);
+    else if (plan.kernel == FwdPlan::kSplit8) rc = launch<64, 1, 8, 128, 2>(p, s);
     else rc = launch<64, 1, 4, 128, 2>(p, s);
   } else {
-    const int64_t heads = static_cast<int64_t>(desc->B) * desc->Hq;
-    // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
-    if (heads * ((desc->Sq + 255) / 256) >= 256) rc = launch<128, 1, 8, 64>(p, s);
-    else rc = launch<128, 1, 4, 64>(p, s);
+    rc = plan.kernel == FwdPlan::kWaves8 ? launch<128, 1, 8, 64>(p, s) : launch<128, 1, 4, 64>(p, s);
   }
   if (rc) return rc;
   return check_launch(fn);
@@ -596,6 +703,22 @@ extern "C" int pico_attn_fwd_rope(const pico_attn_desc* desc, const void* q, con
   if (!rope) return fail(PICO_ERR_NULL, "pico_attn_fwd_rope: the tables are required");
   const pico_kv_chunks kv = one_chunk(desc, k_rot, v);
   return run_fwd("pico_attn_fwd_rope", desc, q, &kv, out, lse, out_dtype, merge, rope, q_pos_offset, q_rot, q_rot_stride, stream);
+}
+
+extern "C" int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
+  if (!desc || chunk_count < 1 || (desc->D != 64 && desc->D != 128) || desc->B <= 0 || desc->Hq <= 0 || desc->Sq <= 0 || desc->Sk <= 0) return 0;
+  AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
+  a.kv.count = chunk_count;
+  a.kv.len = desc->Sk / chunk_count;
+  return plan_fwd(a, desc->D, PICO_ATTN_MAX_WORKSPACE).ws_bytes;
+}
+
+extern "C" int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out,
+                                       float* lse, int out_dtype, int merge, const pico_rope_tables* rope, int q_pos_offset,
+                                       void* q_rot, const int64_t* q_rot_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!aligned16(workspace)) return fail(PICO_ERR_ALIGN, "pico_attn_fwd_chunks_ws: the workspace must be 16-byte aligned");
+  return run_fwd("pico_attn_fwd_chunks_ws", desc, q, kv, out, lse, out_dtype, merge, rope, q_pos_offset, q_rot, q_rot_stride, stream,
+                 static_cast<float*>(workspace), workspace_bytes);
 }
 
 extern "C" int pico_attn_fwd_chunks(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out,

@@ -330,6 +330,25 @@ Tensor attn_in(const Tensor& t, const char* what) {
 }
 Operand operand(const Tensor& t) { return {ptr(t), strides3(t)}; }
 
+// The two launches with the scratch memory they ask for, from torch's allocator (reused in stream order).
+Tensor scratch(int64_t bytes, const at::TensorOptions& o) { return bytes > 0 ? at::empty({bytes}, o.dtype(at::kByte)) : Tensor(); }
+void launch_fwd(const pico_attn_desc& d, const void* q, const pico_kv_chunks& kv, void* out, float* lse, int out_dtype, bool merge,
+                const pico_rope_tables* rope, int64_t q_pos, void* q_rot, const int64_t* q_rot_stride, const at::TensorOptions& o) {
+  const int64_t bytes = pico_attn_fwd_workspace_bytes(&d, kv.count);
+  const Tensor ws = scratch(bytes, o);
+  check(pico_attn_fwd_chunks_ws(&d, q, &kv, out, lse, out_dtype, merge, rope, static_cast<int>(q_pos), q_rot, q_rot_stride, ptr(ws), bytes,
+                                stream_now()));
+}
+void launch_bwd(const pico_attn_desc& d, const void* q, const pico_kv_chunks& kv, const void* dout, const void* out, int out_dtype,
+                const float* lse, float* delta, void* dq, const int64_t* dq_stride, int dq_dtype, bool dq_accumulate,
+                const int64_t* dkv_stride, int dkv_dtype, const pico_rope_tables* rope, int64_t q_pos, int64_t k_pos,
+                const at::TensorOptions& o) {
+  const int64_t bytes = pico_attn_bwd_workspace_bytes(&d, kv.count);
+  const Tensor ws = scratch(bytes, o);
+  check(pico_attn_bwd_chunks_ws(&d, q, &kv, dout, out, out_dtype, lse, delta, dq, dq_stride, dq_dtype, dq_accumulate, dkv_stride, dkv_dtype,
+                                rope, static_cast<int>(q_pos), static_cast<int>(k_pos), ptr(ws), bytes, stream_now()));
+}
+
 struct AttnShape {
   int64_t B, Hq, Hkv, Sq, Sk, D;
 };
@@ -355,11 +374,11 @@ pico_attn_desc attn_desc(const AttnShape& n, const Stride3& q, const Stride3& k,
 
 // The chunk tensors can go to the chunk-list entry points as they are: at most PICO_MAX_KV_CHUNKS bf16 chunks of one shape
 // and one stride triple (k's may differ from v's), unit D stride, strides that are multiples of 8, and -- with several
-// chunks -- a length that is a multiple of 128 (no staged key tile straddles two chunks).
+// chunks -- a length over 64 (every chunk ends with a partly filled key tile unless its length is a multiple of 128).
 bool chunks_fit(const std::vector<Tensor>& ks, const std::vector<Tensor>& vs) {
   if (ks.empty() || ks.size() != vs.size() || ks.size() > PICO_MAX_KV_CHUNKS) return false;
   const Tensor &k0 = ks[0], &v0 = vs[0];
-  if (k0.dim() != 4 || v0.dim() != 4 || (ks.size() > 1 && k0.size(2) % 128 != 0)) return false;
+  if (k0.dim() != 4 || v0.dim() != 4 || (ks.size() > 1 && k0.size(2) <= 64)) return false;
   for (const Tensor* t : {&k0, &v0})
     if (t->stride(3) != 1 || t->stride(0) % 8 || t->stride(1) % 8 || t->stride(2) % 8) return false;
   auto fits = [&](const Tensor& t, const Tensor& first) {
@@ -421,8 +440,8 @@ std::tuple<Tensor, Tensor, OptTensor> attn_fwd(const Tensor& q_in, std::vector<T
     if (want_q_rot && !q_rot) q_rot = empty_bhsd(B, Hq, Sq, D, true, q.options());
     if (q_rot) qrs = strides3(*q_rot);
   }
-  check(pico_attn_fwd_chunks(&d, ptr(q), &kv, ptr(out), fptr(lse), dtype_code(out, "attention out"), merge, rope ? &tables : nullptr,
-                             static_cast<int>(q_pos_offset), rope ? ptr(q_rot) : nullptr, rope && q_rot ? qrs.data() : nullptr, stream_now()));
+  launch_fwd(d, ptr(q), kv, ptr(out), fptr(lse), dtype_code(out, "attention out"), merge, rope ? &tables : nullptr, q_pos_offset,
+             rope ? ptr(q_rot) : nullptr, rope && q_rot ? qrs.data() : nullptr, q.options());
   return {out, lse, rope ? q_rot : std::nullopt};
 }
 
@@ -521,10 +540,9 @@ Tensor attn_bwd(const Tensor& dout_in, const Tensor& q_in, std::vector<Tensor> k
                                strides3(dout), sm_scale, causal, q_offset);
   pico_rope_tables tables;
   if (rope) tables = rope_tables(rope->first, rope->second);
-  check(pico_attn_bwd_chunks(&d, ptr(q), &kv, ptr(dout), ptr(out), out.defined() ? dtype_code(out, "out") : PICO_BF16, fptr(lse),
-                             fptr(delta), ptr(dq), dqs3.data(), dq ? dtype_code(*dq, "dq") : PICO_F32, dq_accumulate,
-                             g0 ? dks3.data() : nullptr, g0 ? dtype_code(*g0, "dk/dv") : PICO_F32, rope ? &tables : nullptr,
-                             static_cast<int>(q_pos_offset), static_cast<int>(k_pos_offset), stream_now()));
+  launch_bwd(d, ptr(q), kv, ptr(dout), ptr(out), out.defined() ? dtype_code(out, "out") : PICO_BF16, fptr(lse), fptr(delta), ptr(dq),
+             dqs3.data(), dq ? dtype_code(*dq, "dq") : PICO_F32, dq_accumulate, g0 ? dks3.data() : nullptr,
+             g0 ? dtype_code(*g0, "dk/dv") : PICO_F32, rope ? &tables : nullptr, q_pos_offset, k_pos_offset, q.options());
   return delta;
 }
 
@@ -1087,11 +1105,11 @@ QKVForward qkv_forward(const Tensor& qkv, const Tensor& cos, const Tensor& sin, 
     rope_heads(m.k, k_rot, cos, sin, B, Hkv, S, D, false);
     pico_rope_tables tables = rope_tables(cos, sin);
     pico_attn_desc d = attn_desc(m.n, m.q.s, k_rot.s, m.v.s, o, sm_scale, causal, 0);
-    check(pico_attn_fwd_chunks(&d, m.q.p, &kv, ptr(r.out), fptr(r.lse), PICO_BF16, 0, &tables, 0, q_rot.p, q_rot.s.data(), stream_now()));
+    launch_fwd(d, m.q.p, kv, ptr(r.out), fptr(r.lse), PICO_BF16, false, &tables, 0, q_rot.p, q_rot.s.data(), qkv.options());
   } else {
     rope_heads(m.q, q_rot, cos, sin, B, Hq + Hkv, S, D, false);
     pico_attn_desc d = attn_desc(m.n, q_rot.s, k_rot.s, m.v.s, o, sm_scale, causal, 0);
-    check(pico_attn_fwd_chunks(&d, q_rot.p, &kv, ptr(r.out), fptr(r.lse), PICO_BF16, 0, nullptr, 0, nullptr, nullptr, stream_now()));
+    launch_fwd(d, q_rot.p, kv, ptr(r.out), fptr(r.lse), PICO_BF16, false, nullptr, 0, nullptr, nullptr, qkv.options());
   }
   return r;
 }
@@ -1127,8 +1145,8 @@ struct QKVAttention : torch::autograd::Function<QKVAttention> {
     pico_kv_chunks kv = one_chunk(m.n, base + 2 * Hq * D, m.v.p, dm.k.p, dm.v.p);
     pico_rope_tables tables;
     if (in_kernel) tables = rope_tables(cos, sin);
-    check(pico_attn_bwd_chunks(&d, base, &kv, ptr(dout), ptr(out), PICO_BF16, fptr(lse), fptr(delta), dm.q.p, dm.q.s.data(), PICO_BF16, 0,
-                               dm.k.s.data(), PICO_BF16, in_kernel ? &tables : nullptr, 0, 0, stream_now()));
+    launch_bwd(d, base, kv, ptr(dout), ptr(out), PICO_BF16, fptr(lse), fptr(delta), dm.q.p, dm.q.s.data(), PICO_BF16, false, dm.k.s.data(),
+               PICO_BF16, in_kernel ? &tables : nullptr, 0, 0, qkv.options());
     if (!in_kernel) rope_heads(dm.q, dm.q, cos, sin, B, Hq + Hkv, S, D, true);
     return {dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }

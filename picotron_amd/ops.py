@@ -163,7 +163,7 @@ FINAL_TOTAL_DTYPES = (torch.bfloat16,)   # dtypes attn_bwd_chunks can write a ch
 def chunks_fit_one_launch(ks, vs) -> bool:
     """True if the chunk tensors can go to the chunk-list entry points as they are: at most 16 bf16 chunks of one shape
     and one stride triple (k's may differ from v's), unit D stride, strides that are multiples of 8, and -- with several
-    chunks -- a chunk length that is a multiple of 128 (no staged key tile straddles two chunks)."""
+    chunks -- a chunk length over 64 (multiples of 128 leave no partly filled key tile at the end of a chunk)."""
     return _lib.host().chunks_fit(ks, vs)
 
 
