@@ -38,7 +38,7 @@ struct BwdParams {
   uint32_t dkv_accumulate;   // bit c: chunk c's dk / dv are added to (fp32)
   int dq_f32, dq_accumulate;
   int dkv_f32;
-  int pair_ktiles;  // dK/dV kernel: a workgroup takes key tile t and then tile n-1-t (equal work under a causal mask)
+  int pair_ktiles;                  // > 0: every workgroup does key tile blockIdx.y and this number - 1 - blockIdx.y
   int64_t dqs[3];  // element strides (b, h, s) of dq
   int64_t dks[3];  // element strides (b, h, s) of dk and dv
   RopeArgs rope;   // rope.cos != nullptr: q and k are rotated tensors; dq and dk leave un-rotated (RoPE's backward)
@@ -106,38 +106,39 @@ __host__ __device__ inline int dkdv_trips(const AttnParams& a, int ktile, int BN
   return n > start ? (n - start) * (a.Hq / a.Hkv) : 0;
 }
 
-// the rows of dK (kDk) or dV that a wave's accumulators hold: 32 keys from row `row0` of their chunk, position `key0`
-template <int D, bool kDk>
-__device__ __forceinline__ void dkdv_store(const BwdParams& p, unsigned char* region, f32x16 (&acc)[D / 32], int chunk, int b, int hkv,
-                                           int row0, int key0, int lane) {
+// the rows of dK (kDk) and / or dV (kDv) that a wave's accumulators hold: 32 keys from row `row0` of their chunk, position
+// `key0`, through the wave's piece of LDS.  bf16 gradients are written with streaming stores: nothing on this GPU reads them
+// back soon, and lines left dirty in L2 are only written back when the kernel ends.
+template <int D, bool kDk, bool kDv>
+__device__ __forceinline__ void dkdv_store(const BwdParams& p, unsigned char* region, f32x16 (&dk_acc)[D / 32], f32x16 (&dv_acc)[D / 32],
+                                           int chunk, int b, int hkv, int row0, int key0, int lane) {
   const AttnParams& a = p.a;
   const int n = lane % 32, h = lane / 32;
   const int rows_live = a.kv.len - row0;
   const int64_t off = b * p.dks[0] + hkv * p.dks[1] + static_cast<int64_t>(row0) * p.dks[2];
   // gradient w.r.t. the un-rotated k: rotate the lane's row of dK back (linear, so the scale and the sum can follow)
-  if constexpr (kDk) {
-    if (p.rope.cos != nullptr) rope_unrotate_acc<D>(acc, p.rope, n < rows_live ? p.rope.k_pos0 + key0 + n : 0, h);
-  }
-  const float scale = kDk ? a.sm_scale : 1.f;
-  void* const dst = kDk ? p.dk[chunk] : p.dv[chunk];
-  __bf16* const total = kDk ? p.dk_final[chunk] : p.dv_final[chunk];
+  if (kDk && p.rope.cos != nullptr) rope_unrotate_acc<D>(dk_acc, p.rope, n < rows_live ? p.rope.k_pos0 + key0 + n : 0, h);
   const bool accumulate = (p.dkv_accumulate >> chunk) & 1u;
-  if (total != nullptr) {
+  if (p.dk_final[chunk] != nullptr) {
     // the last block this chunk's gradient was waiting for: total = travelling sums + this block, rounded once
     const int64_t foff = b * p.dkfs[0] + hkv * p.dkfs[1] + static_cast<int64_t>(row0) * p.dkfs[2];
-    wave_store_rows_total<D>(region, acc, scale, accumulate ? static_cast<const float*>(dst) + off : nullptr, p.dks[2], total + foff,
-                             p.dkfs[2], rows_live, lane);
+    if (kDk) wave_store_rows_total<D>(region, dk_acc, a.sm_scale, accumulate ? static_cast<const float*>(p.dk[chunk]) + off : nullptr,
+                                      p.dks[2], p.dk_final[chunk] + foff, p.dkfs[2], rows_live, lane);
+    if (kDv) wave_store_rows_total<D>(region, dv_acc, 1.f, accumulate ? static_cast<const float*>(p.dv[chunk]) + off : nullptr,
+                                      p.dks[2], p.dv_final[chunk] + foff, p.dkfs[2], rows_live, lane);
   } else if (p.dkv_f32) {
-    wave_store_rows<D, true>(region, acc, scale, static_cast<float*>(dst) + off, p.dks[2], rows_live, lane, accumulate, false);
+    if (kDk) wave_store_rows<D, true>(region, dk_acc, a.sm_scale, static_cast<float*>(p.dk[chunk]) + off, p.dks[2], rows_live, lane, accumulate, false);
+    if (kDv) wave_store_rows<D, true>(region, dv_acc, 1.f, static_cast<float*>(p.dv[chunk]) + off, p.dks[2], rows_live, lane, accumulate, false);
   } else {
-    wave_store_rows<D, false>(region, acc, scale, static_cast<__bf16*>(dst) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
+    if (kDk) wave_store_rows<D, false>(region, dk_acc, a.sm_scale, static_cast<__bf16*>(p.dk[chunk]) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
+    if (kDv) wave_store_rows<D, false>(region, dv_acc, 1.f, static_cast<__bf16*>(p.dv[chunk]) + off, p.dks[2], rows_live, lane, false, kStreamGrads);
   }
 }
 
 // what a wave of a piece leaves: its dK and dV accumulators
 __host__ __device__ constexpr int dkdv_piece_floats(int D) { return 2 * (D / 32) * 16 * kWave; }
 
-template <int D, bool PAIR = false>
+template <int D, bool PAIR, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int ktile, const int part = 0, const int parts = 1) {
   using C = KvCfg<D, PAIR>;
   constexpr int BM = C::BM, BN = C::BN;
@@ -189,7 +190,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   const int qt_start = first_query_tile(a, key0, BM);
   const int tiles_per_head = n_qtiles > qt_start ? n_qtiles - qt_start : 0;
   int n_iter = tiles_per_head * group, head_first = hkv * group, tile_first = qt_start;
-  if (parts > 1) {   // this workgroup's share of the trips
+  if (kCut && parts > 1) {   // this workgroup's share of the trips
     const int t0 = n_iter * part / parts;
     n_iter = n_iter * (part + 1) / parts - t0;
     const int skip = t0 / tiles_per_head;
@@ -560,9 +561,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     __syncthreads();  // all waves are done with the buffer just read (refilled in the next trip) and the next tile is visible
   }
 
-  // ---- epilogue: dK (scaled) and dV rows of this wave's 32 keys, through the wave's piece of LDS (free now:
-  //      the loop ended on a barrier).  bf16 gradients are written with streaming stores: nothing on this
-  //      GPU reads them back soon, and lines left dirty in L2 are only written back when the kernel ends.
+  // ---- epilogue (LDS is free now: the loop ended on a barrier)
   if constexpr (PAIR) {
     // the second wave of each pair hands its sums over, dK then dV (the loop ended on a barrier, or never ran)
     float* xch = reinterpret_cast<float*>(smem_raw + wave * C::kPairExchangeBytes);
@@ -591,15 +590,14 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     }
   }
   if (!PAIR || pair_sb == 0) {
-    if (parts > 1) {   // one piece of several: the sums leave as they are
+    if (kCut && parts > 1) {   // one piece of several: the sums leave as they are
       float* dst = a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kKeyWaves + wave) * dkdv_piece_floats(D);
       put_acc<D / 32>(dst, dk_acc, lane);
       put_acc<D / 32>(dst + dkdv_piece_floats(D) / 2, dv_acc, lane);
       return;
     }
     unsigned char* region = smem_raw + wave * kRowRegionBytes;
-    dkdv_store<D, true>(p, region, dk_acc, chunk, b, hkv, crow0 + 32 * wave, kw0, lane);
-    dkdv_store<D, false>(p, region, dv_acc, chunk, b, hkv, crow0 + 32 * wave, kw0, lane);
+    dkdv_store<D, true, true>(p, region, dk_acc, dv_acc, chunk, b, hkv, crow0 + 32 * wave, kw0, lane);
   }
 }
 
@@ -609,32 +607,35 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 // workgroup takes tile t and then tile n-1-t: under a causal mask every pair is the same amount of work, so a
 // launch whose pairs fill the GPU once ends without a tail of short workgroups and pays the start-up of a
 // workgroup (kernel arguments, first loads) half as often.
-template <int D, bool PAIR = false>
+// kCut: the launch deals its trips out in pieces (see Pieces); a kernel of its own, because the loop of the whole-tile kernel
+// is 1 to 2 % slower with the pieces' bookkeeping around it (in the forward and in dQ up to 10 %).
+template <int D, bool PAIR, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_body(const BwdParams& p) {
   using C = KvCfg<D, PAIR>;
-  const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN);
-  if (p.a.pieces.len > 0) {
-    const Piece at = find_piece(blockIdx.y, n_ktiles, p.a.pieces.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
-    attn_bwd_dkdv_tile<D, PAIR>(p, at.tile, at.part, at.parts);
-    return;
-  }
-  const int first = blockIdx.y;
-  attn_bwd_dkdv_tile<D, PAIR>(p, first);
-  const int second = n_ktiles - 1 - first;
-  if (p.pair_ktiles && second != first) {
-    __syncthreads();  // the epilogue's pieces of LDS are the next tile's buffers
-    attn_bwd_dkdv_tile<D, PAIR>(p, second);
+  if constexpr (kCut) {
+    const Piece at = find_piece(blockIdx.y, tiles_before(p.a.kv, p.a.Sk, C::BN), p.a.pieces.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
+    attn_bwd_dkdv_tile<D, PAIR, true>(p, at.tile, at.part, at.parts);
+  } else {
+    const int first = blockIdx.y;
+    attn_bwd_dkdv_tile<D, PAIR, false>(p, first);
+    const int second = p.pair_ktiles - 1 - first;
+    if (p.pair_ktiles > 0 && second != first) {
+      __syncthreads();  // the epilogue's pieces of LDS are the next tile's buffers
+      attn_bwd_dkdv_tile<D, PAIR, false>(p, second);
+    }
   }
 }
 
 // D = 64 fits two workgroups per CU (<= 256 registers per lane), which lets one workgroup's MFMA
 // work overlap the other's softmax / LDS phases; D = 128 needs the full register file.
+template <bool kCut>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dkdv_kernel_d64(const BwdParams p) {
-  attn_bwd_dkdv_body<64>(p);
+  attn_bwd_dkdv_body<64, false, kCut>(p);
 }
 // D = 128: eight waves, two per key block (see KvCfg), 256 registers each
+template <bool kCut>
 __global__ __launch_bounds__(512) void attn_bwd_dkdv_kernel_d128(const BwdParams p) {
-  attn_bwd_dkdv_body<128, true>(p);
+  attn_bwd_dkdv_body<128, true, kCut>(p);
 }
 
 // The pieces of every cut key tile put together: grid.z 0 sums dK, 1 dV; a wave per 32 keys adds the pieces' accumulators in
@@ -668,13 +669,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_join_kernel(const BwdParams
       for (int i = 0; i < 16; ++i) acc[db][i] += raw[db][i / 4][i % 4];
   }
   unsigned char* region = smem_raw + wave * kRowRegionBytes;
-  if (blockIdx.z == 0) dkdv_store<D, true>(p, region, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
-  else dkdv_store<D, false>(p, region, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
+  if (blockIdx.z == 0) dkdv_store<D, true, false>(p, region, acc, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
+  else dkdv_store<D, false, true>(p, region, acc, acc, at.chunk, b, hkv, at.row0 + 32 * wave, at.key0 + 32 * wave, lane);
 }
 
-template <int D> struct KvKernel;
-template <> struct KvKernel<64> { static constexpr auto fn = &attn_bwd_dkdv_kernel_d64; };
-template <> struct KvKernel<128> { static constexpr auto fn = &attn_bwd_dkdv_kernel_d128; };
+template <int D, bool kCut> struct KvKernel;
+template <bool kCut> struct KvKernel<64, kCut> { static constexpr auto fn = &attn_bwd_dkdv_kernel_d64<kCut>; };
+template <bool kCut> struct KvKernel<128, kCut> { static constexpr auto fn = &attn_bwd_dkdv_kernel_d128<kCut>; };
 
 // =====================================================================================  dQ
 // KS > 1: KS waves share the same 32 queries and each takes one 64-key step of every staged tile (see the forward
@@ -715,7 +716,7 @@ __device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* regi
 }
 
 // (small workgroups are built for two of them per CU: at most 256 registers per lane)
-template <int D, int NW, int KT, bool kDelta, int KS = 1>
+template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bwd_dq_kernel(const BwdParams p) {
   using C = DqCfg<D, NW, KT, KS>;
   constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK;
@@ -726,13 +727,14 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
   const int n_qtiles = (a.Sq + BM - 1) / BM;
   // same dispatch order as the forward kernel: every head's last (longest) query tile first
   Piece piece = {static_cast<int>(blockIdx.y), 0, 1};
-  if (a.pieces.len > 0)
+  if (kCut && a.pieces.len > 0)
     piece = find_piece(blockIdx.y, n_qtiles, a.pieces.len, [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, BM, KT); });
   const int qtile = n_qtiles - 1 - piece.tile;
   const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
   const int hkv = hq / (a.Hq / a.Hkv);
   const int q0 = qtile * BM;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);   // (a scalar: the buffer windows below are built in scalar registers)
   const int n = lane % 32, h = lane / 32;
   const int qw = wave % C::kQWaves, ks = wave / C::kQWaves;   // which queries, which 64-key step of a staged tile
   const float c = a.sm_scale * kLog2e;
@@ -792,8 +794,8 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
     kv_end = vis < a.Sk ? vis : a.Sk;
     if (kv_end < 0) kv_end = 0;
   }
-  int t_first = 0, ntiles = tiles_before(a.kv, kv_end, KT);
-  if (piece.parts > 1) {
+  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
+  if (kCut && piece.parts > 1) {
     t_first = ntiles * piece.part / piece.parts;
     ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
   }
@@ -846,7 +848,9 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
 
   const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
   const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
-  for (int t = 0; t < ntiles; ++t, pos.next(a.kv, KT)) {
+  for (int t = 0; t < ntiles; ++t) {
+    const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
+    if constexpr (kCut) pos.next(a.kv, KT);
     if (t + 1 < ntiles) {
       store_tile((t + 1) & 1);
       if (t + 2 < ntiles) load_tile();
@@ -856,8 +860,8 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
-      const int k0 = pos.key0 + sub * BN;
-      if (k0 >= kv_end || k0 >= pos.end) break;
+      const int k0 = tile_key0 + sub * BN;
+      if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
       if (a.causal && k0 > blk_q_lo + 31) continue;  // the wave's whole 32x64 block is in the future
       const __bf16* sKs = sK + sub * BN * LDK;
       const __bf16* sVs = sV + sub * BN * LDK;
@@ -881,17 +885,16 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
       // dS^T = P^T * (dP^T - delta); keys past the diagonal or the end of their chunk are masked only in tiles that
       // straddle it (the rows read past a chunk are zero, but P of a zero score need not be finite beside a very
       // negative lse)
-      const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || k0 + BN > pos.end;
+      const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || k0 + BN > keys_end;
       if (need_mask) {
         // the asm statement keeps this a real (wave-uniform) branch instead of per-element selects
         asm volatile("; masked tile" ::: "memory");
+        const int last = (qpos < keys_end ? qpos : keys_end - 1) - k0 - 4 * h;   // (one compare with a constant per element)
 #pragma unroll
         for (int mb = 0; mb < BN / 32; ++mb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = k0 + 32 * mb + 8 * (i / 4) + 4 * h + (i % 4);
-            if (key > qpos || key >= pos.end) s_acc[mb][i] = -INFINITY;   // exp2(-inf) = 0
-          }
+          for (int i = 0; i < 16; ++i)
+            if (32 * mb + 8 * (i / 4) + i % 4 > last) s_acc[mb][i] = -INFINITY;   // exp2(-inf) = 0
       }
 #pragma unroll
       for (int mb = 0; mb < BN / 32; ++mb)
@@ -942,7 +945,7 @@ __global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bw
     static_assert(kRowRegionBytes <= C::kExchangeBytes, "store pieces lie below the exchange areas read above");
   }
 
-  if (piece.parts > 1) {   // one piece of several: the sums leave as they are
+  if (kCut && piece.parts > 1) {   // one piece of several: the sums leave as they are
     put_acc<D / 32>(a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * dq_piece_floats(D), dq, lane);
     return;
   }
@@ -1030,7 +1033,7 @@ struct DkdvPlan {
   int64_t ws_bytes = 0;
 };
 template <int D>
-DkdvPlan plan_dkdv(const AttnParams& a, int64_t ws_bytes) {
+DkdvPlan make_dkdv_plan(const AttnParams& a) {
   using C = KvCfg<D, D == 128>;
   DkdvPlan plan;
   const int64_t heads = static_cast<int64_t>(a.Hkv) * a.B;
@@ -1039,61 +1042,65 @@ DkdvPlan plan_dkdv(const AttnParams& a, int64_t ws_bytes) {
   // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
   // are up to 30 % faster)
   plan.pair = a.causal && n_ktiles >= 2 && heads * ((n_ktiles + 1) / 2) >= (D == 64 ? 384 : 256);
-  if (ws_bytes <= 0) return plan;
-  TripCost cost = {1.1, 1.0, 4.0, 0.0};
-  if (D == 128) cost = {1.65, 2.05, 4.0, 0.0};
+  TripCost cost = {1.1, 1.0, 2, 0.0};
+  if (D == 128) cost = {1.65, 2.05, 1, 0.0};
   cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
   auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
-  plan.len = choose_pieces(heads, n_ktiles, cost, ws_bytes, trips_of);
-  if (plan.len > 0) {
-    const int n = count_pieces(n_ktiles, plan.len, trips_of);
-    if (n == n_ktiles) plan.len = 0;
-    else plan.ws_bytes = static_cast<int64_t>(heads * n * cost.piece_bytes);
-  }
+  plan.len = choose_pieces(heads, n_ktiles, cost, plan.pair, trips_of);
+  if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_ktiles, plan.len, trips_of) * cost.piece_bytes);
   return plan;
 }
+template <int D>
+const DkdvPlan& plan_dkdv(const AttnParams& a) {
+  static thread_local PlanTable<DkdvPlan> table;
+  return table.get(a, D, [&] { return make_dkdv_plan<D>(a); });
+}
 
+template <int D, bool kCut>
+int launch_dkdv_impl(const BwdParams& p, int grid_y, hipStream_t s) {
+  using C = KvCfg<D, D == 128>;
+  static LdsOnce lds_reserved;
+  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(KvKernel<D, kCut>::fn), C::kLdsBytes))
+    return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dk/dv): cannot reserve %zu bytes of LDS", C::kLdsBytes);
+  hipLaunchKernelGGL((KvKernel<D, kCut>::fn), dim3(p.a.Hkv * p.a.B, grid_y), dim3(C::kThreads), C::kLdsBytes, s, p);
+  return PICO_OK;
+}
 template <int D>
 int launch_dkdv(const BwdParams& p, float* ws, int64_t ws_bytes, hipStream_t s) {
   using C = KvCfg<D, D == 128>;
-  static LdsOnce lds_reserved;
-  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(KvKernel<D>::fn), C::kLdsBytes))
-    return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dk/dv): cannot reserve %zu bytes of LDS", C::kLdsBytes);
-  const DkdvPlan plan = plan_dkdv<D>(p.a, ws ? ws_bytes : 0);
-  const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN), heads = p.a.Hkv * p.a.B;
+  const DkdvPlan& plan = plan_dkdv<D>(p.a);
+  const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN);
   BwdParams q = p;
-  q.pair_ktiles = plan.pair;
+  if (plan.len == 0 || !ws || ws_bytes < plan.ws_bytes) {
+    q.pair_ktiles = plan.pair ? n_ktiles : 0;
+    return launch_dkdv_impl<D, false>(q, plan.pair ? (n_ktiles + 1) / 2 : n_ktiles, s);
+  }
   q.a.pieces = Pieces{plan.len, ws};
-  int grid_y = plan.pair ? (n_ktiles + 1) / 2 : n_ktiles;
-  if (plan.len > 0) grid_y = count_pieces(n_ktiles, plan.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
-  hipLaunchKernelGGL(KvKernel<D>::fn, dim3(heads, grid_y), dim3(C::kThreads), C::kLdsBytes, s, q);
-  if (plan.len > 0)
-    hipLaunchKernelGGL(attn_bwd_dkdv_join_kernel<D>, dim3(heads, n_ktiles, 2), dim3(256), 0, s, q, grid_y);
+  const int n = count_pieces(n_ktiles, plan.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
+  if (int rc = launch_dkdv_impl<D, true>(q, n, s)) return rc;
+  hipLaunchKernelGGL(attn_bwd_dkdv_join_kernel<D>, dim3(p.a.Hkv * p.a.B, n_ktiles, 2), dim3(256), 0, s, q, n);
   return PICO_OK;
 }
 
-template <int D, int NW, int KT, bool kDelta, int KS>
+template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
 int launch_dq_impl(const BwdParams& p, hipStream_t s) {
   using C = DqCfg<D, NW, KT, KS>;
   static LdsOnce lds_reserved;
-  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, NW, KT, kDelta, KS>), C::kLdsBytes))
+  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, NW, KT, kDelta, KS, kCut>), C::kLdsBytes))
     return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dq): cannot reserve %zu bytes of LDS", C::kLdsBytes);
-  const int n_qtiles = (p.a.Sq + C::BM - 1) / C::BM;
-  BwdParams q = p;
-  int n = n_qtiles;
-  if (q.a.pieces.len > 0) {
-    n = count_pieces(n_qtiles, q.a.pieces.len, [&](int i) { return query_tile_trips(q.a, n_qtiles - 1 - i, C::BM, KT); });
-    if (n == n_qtiles) q.a.pieces.len = 0;
-  }
-  hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NW, KT, kDelta, KS>), dim3(p.a.Hq * p.a.B, n), dim3(C::kThreads), C::kLdsBytes, s, q);
-  if (q.a.pieces.len > 0)
-    hipLaunchKernelGGL((attn_bwd_dq_join_kernel<D, C::kQWaves, KT>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(64 * C::kQWaves), 0, s, q, n);
+  const int heads = p.a.Hq * p.a.B, n_qtiles = (p.a.Sq + C::BM - 1) / C::BM, len = p.a.pieces.len;
+  const int n = count_pieces(n_qtiles, len, [&](int i) { return query_tile_trips(p.a, n_qtiles - 1 - i, C::BM, KT); });
+  hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NW, KT, kDelta, KS, kCut>), dim3(heads, n), dim3(C::kThreads), C::kLdsBytes, s, p);
+  if (kCut && len > 0)
+    hipLaunchKernelGGL((attn_bwd_dq_join_kernel<D, C::kQWaves, KT>), dim3(heads, n_qtiles), dim3(64 * C::kQWaves), 0, s, p, n);
   return PICO_OK;
 }
 
 template <int D, int NW, int KT, int KS = 1>
 int launch_dq(const BwdParams& p, hipStream_t s) {
-  return p.out ? launch_dq_impl<D, NW, KT, true, KS>(p, s) : launch_dq_impl<D, NW, KT, false, KS>(p, s);
+  const bool cut = p.a.pieces.len > 0 || ends_inside_tile(p.a.kv, KT);
+  if (p.out) return cut ? launch_dq_impl<D, NW, KT, true, KS, true>(p, s) : launch_dq_impl<D, NW, KT, true, KS, false>(p, s);
+  return cut ? launch_dq_impl<D, NW, KT, false, KS, true>(p, s) : launch_dq_impl<D, NW, KT, false, KS, false>(p, s);
 }
 
 // How the dQ launch is run: which kernel, and whether its query tiles are cut into pieces.
@@ -1102,11 +1109,11 @@ struct DqPlan {
   int len = 0;
   int64_t ws_bytes = 0;
 };
-DqPlan plan_dq(const AttnParams& a, int D, int64_t ws_bytes) {
+DqPlan make_dq_plan(const AttnParams& a, int D) {
   DqPlan plan;
   const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
-  TripCost cost = {1.65, 1.8, 4.0, 0.0};
+  TripCost cost = {1.65, 1.8, 2, 0.0};
   int bm = 128, kt = 64;
   if (D == 64) {
     const int64_t visible_keys = a.causal ? std::min<int64_t>(a.Sk, static_cast<int64_t>(a.q_offset) + a.Sq) : a.Sk;
@@ -1125,22 +1132,25 @@ DqPlan plan_dq(const AttnParams& a, int D, int64_t ws_bytes) {
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
     bm = plan.kernel == DqPlan::kWaves8 ? 256 : plan.kernel == DqPlan::kSplit4 ? 64 : 128;
     kt = plan.kernel >= DqPlan::kSplit4 ? 128 : 64;
-    cost = plan.kernel == DqPlan::kWaves8 ? TripCost{1.7, 1.5, 4.0, 0.0} : plan.kernel == DqPlan::kWaves4 ? TripCost{1.3, 0.78, 4.0, 0.0}
-         : plan.kernel == DqPlan::kSplit8 ? TripCost{1.6, 1.5, 4.0, 0.0} : TripCost{1.25, 0.8, 4.0, 0.0};
+    cost = plan.kernel == DqPlan::kWaves8 ? TripCost{1.7, 1.5, 1, 0.0} : plan.kernel == DqPlan::kWaves4 ? TripCost{1.3, 0.78, 2, 0.0}
+         : plan.kernel == DqPlan::kSplit8 ? TripCost{1.6, 1.5, 1, 0.0} : TripCost{1.25, 0.8, 2, 0.0};
   } else {
     plan.kernel = groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
     if (plan.kernel == DqPlan::kWaves8) {
       bm = 256;
-      cost = {2.0, 2.87, 4.0, 0.0};
+      cost = {2.0, 2.87, 1, 0.0};
     }
   }
-  if (ws_bytes <= 0) return plan;
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);
   auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, bm, kt); };
-  plan.len = choose_pieces(heads, n_qtiles, cost, ws_bytes, trips_of);
+  plan.len = choose_pieces(heads, n_qtiles, cost, false, trips_of);
   if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_qtiles, plan.len, trips_of) * cost.piece_bytes);
   return plan;
+}
+const DqPlan& plan_dq(const AttnParams& a, int D) {
+  static thread_local PlanTable<DqPlan> table;
+  return table.get(a, D, [&] { return make_dq_plan(a, D); });
 }
 
 }  // namespace
@@ -1262,9 +1272,9 @@ int run_bwd(const char* fn, const pico_attn_desc* desc, const void* q, const pic
   auto run_dq = [&]() -> int {
     if (!have_q) return PICO_OK;
     // without keys the dQ kernel still runs: it writes (or adds) zeros
-    const DqPlan plan = plan_dq(p.a, desc->D, ws ? ws_bytes : 0);
+    const DqPlan& plan = plan_dq(p.a, desc->D);
     BwdParams p_dq = p;
-    p_dq.a.pieces = Pieces{plan.len, ws};
+    p_dq.a.pieces = Pieces{ws && ws_bytes >= plan.ws_bytes ? plan.len : 0, ws};
     int rc;
     if (desc->D == 64) {
       if (plan.kernel == DqPlan::kWaves8) rc = launch_dq<64, 8, 64>(p_dq, s);
@@ -1374,8 +1384,8 @@ extern "C" int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int
   AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
   a.kv.count = chunk_count;
   a.kv.len = desc->Sk / chunk_count;
-  const int64_t dkdv = desc->D == 64 ? plan_dkdv<64>(a, PICO_ATTN_MAX_WORKSPACE).ws_bytes : plan_dkdv<128>(a, PICO_ATTN_MAX_WORKSPACE).ws_bytes;
-  return std::max(dkdv, plan_dq(a, desc->D, PICO_ATTN_MAX_WORKSPACE).ws_bytes);   // (the two kernels run one after the other)
+  const int64_t dkdv = desc->D == 64 ? plan_dkdv<64>(a).ws_bytes : plan_dkdv<128>(a).ws_bytes;
+  return std::max(dkdv, plan_dq(a, desc->D).ws_bytes);   // (the two kernels run one after the other)
 }
 
 extern "C" int pico_attn_bwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,

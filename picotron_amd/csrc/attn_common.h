@@ -316,6 +316,8 @@ struct KvChunks {
 // mask, and with the query heads of a GQA group walked by one workgroup in dK/dV).  The trips of an output tile are dealt
 // to ceil(trips / len) workgroups; where that is more than one, each leaves its accumulators in `ws` as they lie in its
 // registers, and a second launch adds the pieces of a tile in their order and runs the kernel's own epilogue on the sum.
+// Before and after, us: dK/dV of B1 H8/2 S2048 D64 144 -> 31, B2 H32/8 S1531 D128 143 -> 97, B8 H4/1 S7729 D64 655 -> 505,
+// B1 H12/4 S3000 D128 200 -> 87; forward and dQ of one head of 4000 rows 48 -> 21 and 44 -> 19.
 struct Pieces {
   int len;     // most trips of a piece; 0: tiles are not cut
   float* ws;
@@ -370,38 +372,92 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
   return __builtin_amdgcn_readfirstlane(sum);
 }
 
-// Host: the piece length for a launch, from what a trip and a workgroup cost.  `alone_us` is a trip of a workgroup that has
-// its CU to itself, `full_us` the CU's time per trip where it is shared, `fixed_us` a workgroup's start and end.  Not cutting
-// (0) stands as one of the choices; cutting has to win by its second launch and by the traffic of the pieces.
+// Host: the piece length for a launch, from what its workgroups cost.  A trip takes `alone_us` in a workgroup that has its
+// CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each; `fixed_us` is a workgroup's start and end.
+// (Fitted to launches from 1 to 300 heads and 200 to 8000 rows; over 27 such shapes the piece lengths chosen ran within
+// 0.7 % of the best ones in the geometric mean, 5 % at worst.)
 struct TripCost {
-  double alone_us, full_us, fixed_us, piece_bytes;
+  double alone_us, full_us;
+  int per_cu;
+  double piece_bytes;
+};
+// When the last of a launch's workgroups ends: they are dealt in grid order, tile by tile, to whichever place is free first.
+struct Places {
+  static constexpr int kMost = 64;   // groups of places that become free together (beyond that the latest two are merged)
+  double at[kMost];
+  int64_t count[kMost];
+  int n;
+  explicit Places(int64_t places) : n(1) { at[0] = 0.0; count[0] = places; }
+  void run(int64_t workgroups, double us) {
+    while (workgroups > 0) {
+      const double start = at[0];
+      const int64_t k = std::min(count[0], workgroups);
+      workgroups -= k;
+      count[0] -= k;
+      if (count[0] == 0) {
+        --n;
+        for (int i = 0; i < n; ++i) { at[i] = at[i + 1]; count[i] = count[i + 1]; }
+      }
+      const double end = start + us;
+      int i = n;
+      while (i > 0 && at[i - 1] > end + 1e-6) --i;
+      if (i > 0 && at[i - 1] > end - 1e-6) { count[i - 1] += k; continue; }
+      if (n == kMost) { count[n - 1] += k; at[n - 1] = std::max(at[n - 1], end); continue; }
+      for (int j = n; j > i; --j) { at[j] = at[j - 1]; count[j] = count[j - 1]; }
+      at[i] = end;
+      count[i] = k;
+      ++n;
+    }
+  }
+  double last() const { return at[n - 1]; }
 };
 template <typename F>
-int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, int64_t ws_bytes, const F& trips_of, double uncut_us = -1.0) {
-  constexpr double kCus = 256.0, kSecondLaunchUs = 5.0, kBytesPerUs = 4e6;
-  auto estimate = [&](int len, int64_t* pieces) {
-    int longest = 0;
-    int64_t total = 0, n = 0, cut = 0;
+double launch_us(int64_t heads, int n_tiles, const TripCost& c, int len, bool pairs, const F& trips_of) {
+  constexpr int64_t kCus = 256;
+  constexpr double kFixedUs = 4.0, kPairFixedUs = 5.2, kJoinUs = 3.0, kJoinPartUs = 1.0, kBytesPerUs = 4e6;
+  int64_t workgroups = 0, cut = 0;
+  int most = 1;
+  for (int i = 0; i < n_tiles; ++i) {
+    const int k = pieces_of(trips_of(i), len);
+    workgroups += heads * k;
+    if (k > 1) { cut += heads * k; most = std::max(most, k); }
+  }
+  if (pairs) workgroups = heads * ((n_tiles + 1) / 2);
+  const double shared = c.per_cu > 1 ? std::min(1.0, std::max(0.0, (workgroups - kCus) / static_cast<double>(kCus)))
+                                     : std::min(1.0, workgroups / static_cast<double>(kCus));
+  const double trip = c.alone_us + (std::max(c.alone_us, c.full_us * c.per_cu) - c.alone_us) * shared;
+  Places places(kCus * c.per_cu);
+  if (pairs) {
+    for (int i = 0; i < (n_tiles + 1) / 2; ++i) {
+      const int j = n_tiles - 1 - i;
+      places.run(heads, (trips_of(i) + (j != i ? trips_of(j) : 0)) * trip + kPairFixedUs);
+    }
+  } else {
     for (int i = 0; i < n_tiles; ++i) {
       const int t = trips_of(i), k = pieces_of(t, len);
-      longest = std::max(longest, (t + k - 1) / k);
-      total += t;
-      n += k;
-      if (k > 1) cut += k;
+      places.run(heads * k, t * trip / k + kFixedUs);
     }
-    *pieces = n;
-    const double span = longest * c.alone_us + c.fixed_us, load = heads * (total * c.full_us + n * c.fixed_us * 0.5) / kCus;
-    return std::max(span, load) + 0.25 * std::min(span, load) + (cut ? kSecondLaunchUs + 2.0 * heads * cut * c.piece_bytes / kBytesPerUs : 0.0);
-  };
+  }
+  return places.last() + (cut ? kJoinUs + kJoinPartUs * most + 2.0 * cut * c.piece_bytes / kBytesPerUs : 0.0);
+}
+template <typename F>
+int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, bool pairs, const F& trips_of) {
   if (heads * n_tiles > 4 * 512) return 0;   // enough workgroups that their lengths even out
-  int64_t n = 0;
-  double best_us = estimate(0, &n);
-  if (uncut_us >= 0.0) best_us = uncut_us;
-  int best = 0;
+  // a cut has to win 5 %, the most the estimate was found to be off by, and the time in which a host launches the second
+  // kernel: where the host is the slower side a shorter kernel gains nothing (B2 H9/3 S256 D64, forward and backward: 33 us
+  // of kernels cut to 29 took 38 us for 35)
+  constexpr double kLaunchUs = 5.0;
+  const double uncut_us = launch_us(heads, n_tiles, c, 0, pairs, trips_of);
+  double best_us = std::min(0.95 * uncut_us, uncut_us - kLaunchUs);
+  int best = 0, longest = 0;
+  for (int i = 0; i < n_tiles; ++i) longest = std::max(longest, trips_of(i));
   for (int len : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
-    const double us = estimate(len, &n);
-    if (n > 65535 || heads * n * c.piece_bytes > static_cast<double>(ws_bytes)) continue;
-    if (us < 0.95 * best_us) {
+    if (len >= longest) break;
+    int64_t n = 0;
+    for (int i = 0; i < n_tiles; ++i) n += pieces_of(trips_of(i), len);
+    if (n > 65535 || heads * n * c.piece_bytes > static_cast<double>(PICO_ATTN_MAX_WORKSPACE)) continue;
+    const double us = launch_us(heads, n_tiles, c, len, false, trips_of);
+    if (us < best_us) {
       best_us = us;
       best = len;
     }
@@ -410,10 +466,35 @@ int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, int64_t ws_byte
 }
 template <typename F>
 int count_pieces(int n_tiles, int len, const F& trips_of) {
+  if (len <= 0) return n_tiles;
   int n = 0;
   for (int i = 0; i < n_tiles; ++i) n += pieces_of(trips_of(i), len);
   return n;
 }
+
+// A launch's plan depends on its sizes alone and is worked out once per thread and shape (some microseconds): `make` for the
+// sizes in `key`, kept in a small direct-mapped table.
+template <typename Plan>
+struct PlanTable {
+  struct Entry {
+    int key[10];
+    bool used = false;
+    Plan plan;
+  } entries[64];
+  template <typename Make>
+  const Plan& get(const AttnParams& a, int D, const Make& make) {
+    const int key[10] = {a.B, a.Hq, a.Hkv, a.Sq, a.Sk, D, a.causal, a.q_offset, a.kv.count, a.kv.len};
+    uint32_t h = 2166136261u;
+    for (int v : key) h = (h ^ static_cast<uint32_t>(v)) * 16777619u;
+    Entry& e = entries[(h ^ (h >> 15)) % 64];
+    if (!e.used || !std::equal(key, key + 10, e.key)) {
+      e.plan = make();
+      std::copy(key, key + 10, e.key);
+      e.used = true;
+    }
+    return e.plan;
+  }
+};
 
 // accumulators in register order, 16 bytes per lane and piece of a row block: what a cut tile's pieces leave in memory
 template <int N>
@@ -449,6 +530,9 @@ __host__ __device__ inline int query_tile_trips(const AttnParams& a, int qtile, 
   }
   return tiles_before(a.kv, end, KT);
 }
+
+// do chunks end inside key tiles of KT rows that further chunks follow?
+inline bool ends_inside_tile(const KvChunks& kv, int KT) { return kv.count > 1 && kv.len % KT != 0; }
 
 // A cursor over the key tiles of KT keys, in order, across the chunks: wave-uniform, so it lives in scalar registers;
 // stepping inside a chunk is four adds, a new chunk re-reads its base addresses from the kernel arguments.

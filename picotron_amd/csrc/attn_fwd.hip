@@ -58,16 +58,16 @@ struct FwdCfg {
 // what a wave of a piece leaves: O^T accumulators, m and l per lane
 constexpr int fwd_piece_floats(int D) { return (D / 32) * 16 * kWave + 2 * kWave; }
 
-// lse per query; the wave's 32 output rows leave through its piece of LDS as whole lines
+// lse per query (the head's rows start at lse_row0); the wave's 32 output rows leave through its piece of LDS as whole lines
 template <int D>
 __device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* region, f32x16 (&o)[D / 32], float m_run, float l_run,
-                                             int b, int hq, int row0, int lane) {
+                                             int b, int hq, int64_t lse_row0, int row0, int lane) {
   const AttnParams& a = p.a;
   const int row = row0 + lane % 32;
   const float l_tot = half_sum(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row < a.Sq && lane < 32)
-    p.lse[(static_cast<int64_t>(b) * a.Hq + hq) * a.Sq + row] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
+    p.lse[lse_row0 + row] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
   // normalise in place: 1 / l differs per lane (row), the store helper applies one scale to all
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
@@ -80,7 +80,9 @@ __device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* 
     wave_store_rows<D, false>(region, o, 1.f, static_cast<__bf16*>(p.out) + off, a.os[2], a.Sq - row0, lane, false, false);
 }
 
-template <int D, int QB, int NW, int KT, int KS = 1>
+// kCut: tiles may be cut into pieces (see Pieces) and chunks may end inside a key tile; a kernel of its own, because the loop
+// of the plain one loses up to 10 % to that bookkeeping (B4 H32 S1024 D64 29.9 -> 33.0 us, B1 H32 S4096 D128 137 -> 144).
+template <int D, int QB, int NW, int KT, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
   constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK, LDV = C::LDV;
@@ -97,8 +99,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   // the short tiles in ASCENDING order: every CU then holds a long and a short tile of equal total length.
   const int y = static_cast<int>(blockIdx.y), half = (n_qtiles + 1) / 2;
   Piece piece = {y, 0, 1};
-  if (a.pieces.len > 0) piece = find_piece(y, n_qtiles, a.pieces.len, trips_of);
-  const int qtile = (p.pair_order && y >= half) ? y - half : n_qtiles - 1 - piece.tile;
+  if (kCut && a.pieces.len > 0) piece = find_piece(y, n_qtiles, a.pieces.len, trips_of);
+  const int qtile = (!kCut && p.pair_order && y >= half) ? y - half : n_qtiles - 1 - piece.tile;
   const int hq = blockIdx.x % a.Hq, b = blockIdx.x / a.Hq;
   const int hkv = hq / (a.Hq / a.Hkv);
   const int q0 = qtile * BM;
@@ -174,8 +176,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
     kv_end = vis < a.Sk ? vis : a.Sk;
     if (kv_end < 0) kv_end = 0;
   }
-  int t_first = 0, ntiles = tiles_before(a.kv, kv_end, KT);
-  if (piece.parts > 1) {
+  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
+  if (kCut && piece.parts > 1) {
     t_first = ntiles * piece.part / piece.parts;
     ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
   }
@@ -230,7 +232,9 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   if (ntiles > 1) load_tile();
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t, pos.next(a.kv, KT)) {
+  for (int t = 0; t < ntiles; ++t) {
+    const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
+    if constexpr (kCut) pos.next(a.kv, KT);
     // stage tile t+1 into the other buffer (its readers finished before the barrier that ended trip t-1)
     if (t + 1 < ntiles) {
       store_tile((t + 1) & 1);
@@ -242,8 +246,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
-      const int k0 = pos.key0 + sub * BN;
-      if (k0 >= kv_end || k0 >= pos.end) break;
+      const int k0 = tile_key0 + sub * BN;
+      if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
       const __bf16* sKs = sK + sub * BN * LDK;
       const __bf16* sVs = sV + sub * BN * LDV;
 #pragma unroll
@@ -293,19 +297,18 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
           }
         }
         // ---- mask (only for tiles that straddle the diagonal or the end of their chunk)
-        const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || (k0 + BN > pos.end);
+        const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || (k0 + BN > keys_end);
         if (need_mask) {
           // the asm statement keeps this a real (wave-uniform) branch: without it the compiler turns the
           // block into per-element selects that every tile pays for
           asm volatile("; masked tile" ::: "memory");
           const int qpos = a.causal ? a.q_offset + qrow[qb] : 0x7fffffff;
+          const int last = (qpos < keys_end ? qpos : keys_end - 1) - k0 - 4 * h;   // (one compare with a constant per element)
 #pragma unroll
           for (int mb = 0; mb < BN / 32; ++mb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int key = k0 + 32 * mb + 8 * (i / 4) + 4 * h + (i % 4);
-              if (key > qpos || key >= pos.end) s_acc[mb][i] = -INFINITY;
-            }
+            for (int i = 0; i < 16; ++i)
+              if (32 * mb + 8 * (i / 4) + i % 4 > last) s_acc[mb][i] = -INFINITY;
         }
         // ---- online softmax.  The running maximum is only raised (and O, l rescaled) when some query of
         //      the wave saw its maximum grow by more than 2^kTau; until then exp2(s - m) may exceed 1 by at
@@ -403,7 +406,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
     static_assert(C::kQWaves * kRowRegionBytes <= C::kQWaves * C::kExchangeBytes, "store pieces lie below the exchange areas read above");
   }
 
-  if constexpr (QB == 1) {
+  if constexpr (QB == 1 && kCut) {
     if (piece.parts > 1) {   // one piece of several: the state leaves as it is (l per wave half)
       float* dst = a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * fwd_piece_floats(D);
       put_acc<D / 32>(dst, o[0], lane);
@@ -414,7 +417,8 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
   }
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb)
-    fwd_epilogue<D>(p, smem_raw + (wave * QB + qb) * kRowRegionBytes, o[qb], m_run[qb], l_run[qb], b, hq, q0 + (qw * QB + qb) * 32, lane);
+    fwd_epilogue<D>(p, smem_raw + (wave * QB + qb) * kRowRegionBytes, o[qb], m_run[qb], l_run[qb], b, hq, lse_row0,
+                    q0 + (qw * QB + qb) * 32, lane);
 }
 
 // The pieces of every cut query tile put together: a wave per 32 queries merges the pieces' states, which lie as the pieces'
@@ -454,31 +458,30 @@ __global__ __launch_bounds__(64 * QW) void attn_fwd_join_kernel(const FwdParams 
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[db][i] += aj * raw[db][i / 4][i % 4];
   }
-  fwd_epilogue<D>(p, smem_raw + wave * kRowRegionBytes, o, m, l, b, hq, row0, lane);
+  fwd_epilogue<D>(p, smem_raw + wave * kRowRegionBytes, o, m, l, b, hq, (static_cast<int64_t>(b) * a.Hq + hq) * a.Sq, row0, lane);
 }
 
-template <int D, int QB, int NW, int KT, int KS = 1>
-int launch(const FwdParams& p, hipStream_t s) {
+template <int D, int QB, int NW, int KT, int KS, bool kCut>
+int launch_impl(const FwdParams& p, hipStream_t s) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
   static LdsOnce lds_reserved;
-  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(&attn_fwd_kernel<D, QB, NW, KT, KS>), C::kLdsBytes))
+  if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(&attn_fwd_kernel<D, QB, NW, KT, KS, kCut>), C::kLdsBytes))
     return fail(PICO_ERR_LAUNCH, "pico_attn_fwd: cannot reserve %zu bytes of LDS", C::kLdsBytes);
-  const int n_qtiles = (p.a.Sq + C::BM - 1) / C::BM;
+  const int heads = p.a.Hq * p.a.B, n_qtiles = (p.a.Sq + C::BM - 1) / C::BM, len = p.a.pieces.len;
   FwdParams q = p;
   // (the pairing needs two workgroups per CU: at head_dim 128 the eight-wave kernel has one, the launch is two
   // generations of workgroups and longest-first is the better order -- 160 -> 137 us at B1 H32 S4096)
   constexpr bool kTwoPerCu = !(D >= 128 && NW == 8);
-  q.pair_order = kTwoPerCu && p.a.causal && n_qtiles >= 2 && static_cast<int64_t>(p.a.Hq) * p.a.B * n_qtiles <= 512;
-  int n = n_qtiles;
-  if (q.a.pieces.len > 0) {
-    n = count_pieces(n_qtiles, q.a.pieces.len, [&](int i) { return query_tile_trips(q.a, n_qtiles - 1 - i, C::BM, KT); });
-    q.pair_order = 0;
-    if (n == n_qtiles) q.a.pieces.len = 0;
-  }
-  hipLaunchKernelGGL((attn_fwd_kernel<D, QB, NW, KT, KS>), dim3(p.a.Hq * p.a.B, n), dim3(C::kThreads), C::kLdsBytes, s, q);
-  if (q.a.pieces.len > 0)
-    hipLaunchKernelGGL((attn_fwd_join_kernel<D, C::kQWaves, KT>), dim3(p.a.Hq * p.a.B, n_qtiles), dim3(64 * C::kQWaves), 0, s, q, n);
+  q.pair_order = !kCut && kTwoPerCu && p.a.causal && n_qtiles >= 2 && static_cast<int64_t>(heads) * n_qtiles <= 512;
+  const int n = count_pieces(n_qtiles, len, [&](int i) { return query_tile_trips(p.a, n_qtiles - 1 - i, C::BM, KT); });
+  hipLaunchKernelGGL((attn_fwd_kernel<D, QB, NW, KT, KS, kCut>), dim3(heads, n), dim3(C::kThreads), C::kLdsBytes, s, q);
+  if (kCut && len > 0)
+    hipLaunchKernelGGL((attn_fwd_join_kernel<D, C::kQWaves, KT>), dim3(heads, n_qtiles), dim3(64 * C::kQWaves), 0, s, q, n);
   return PICO_OK;
+}
+template <int D, int QB, int NW, int KT, int KS = 1>
+int launch(const FwdParams& p, hipStream_t s) {
+  return p.a.pieces.len > 0 || ends_inside_tile(p.a.kv, KT) ? launch_impl<D, QB, NW, KT, KS, true>(p, s) : launch_impl<D, QB, NW, KT, KS, false>(p, s);
 }
 
 }  // namespace
@@ -585,11 +588,11 @@ struct FwdPlan {
   int64_t ws_bytes = 0;      // what the pieces need
 };
 
-FwdPlan plan_fwd(const AttnParams& a, int D, int64_t ws_bytes) {
+FwdPlan make_fwd_plan(const AttnParams& a, int D) {
   FwdPlan plan;
   const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
-  TripCost cost = {1.5, 1.1, 4.0, 0.0};
+  TripCost cost = {1.5, 1.1, 2, 0.0};
   int bm = 128, kt = 64;
   // Tile choice for D = 64: more waves per workgroup share each staged K/V tile (fewer barriers and
   // global loads per MFMA), but the launch still has to fill 256 CUs, so small problems get small tiles.
@@ -608,23 +611,26 @@ FwdPlan plan_fwd(const AttnParams& a, int D, int64_t ws_bytes) {
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? FwdPlan::kSplit8 : FwdPlan::kSplit4;
     bm = plan.kernel == FwdPlan::kWaves8 ? 256 : plan.kernel == FwdPlan::kSplit4 ? 64 : 128;
     kt = plan.kernel >= FwdPlan::kSplit4 ? 128 : 64;
-    cost = plan.kernel == FwdPlan::kWaves8 ? TripCost{1.6, 1.28, 4.0, 0.0} : plan.kernel == FwdPlan::kWaves4 ? TripCost{1.2, 0.66, 4.0, 0.0}
-         : plan.kernel == FwdPlan::kSplit8 ? TripCost{1.5, 1.3, 4.0, 0.0} : TripCost{1.35, 0.7, 4.0, 0.0};
+    cost = plan.kernel == FwdPlan::kWaves8 ? TripCost{1.6, 1.28, 2, 0.0} : plan.kernel == FwdPlan::kWaves4 ? TripCost{1.2, 0.66, 2, 0.0}
+         : plan.kernel == FwdPlan::kSplit8 ? TripCost{1.5, 1.3, 1, 0.0} : TripCost{1.35, 0.7, 2, 0.0};
   } else {
     // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
     plan.kernel = groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
     if (plan.kernel == FwdPlan::kWaves8) {
       bm = 256;
-      cost = {1.6, 2.13, 4.0, 0.0};
+      cost = {1.6, 2.13, 1, 0.0};
     }
   }
-  if (ws_bytes <= 0) return plan;
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * fwd_piece_floats(D);
   auto trips_of = [&](int i) { return query_tile_trips(a, n_qtiles - 1 - i, bm, kt); };
-  plan.len = choose_pieces(heads, n_qtiles, cost, ws_bytes, trips_of);
+  plan.len = choose_pieces(heads, n_qtiles, cost, false, trips_of);
   if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_qtiles, plan.len, trips_of) * cost.piece_bytes);
   return plan;
+}
+const FwdPlan& plan_fwd(const AttnParams& a, int D) {
+  static thread_local PlanTable<FwdPlan> table;
+  return table.get(a, D, [&] { return make_fwd_plan(a, D); });
 }
 
 int run_fwd(const char* fn, const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out, float* lse,
@@ -665,8 +671,8 @@ int run_fwd(const char* fn, const pico_attn_desc* desc, const void* q, const pic
     }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const FwdPlan plan = plan_fwd(p.a, desc->D, workspace ? ws_bytes : 0);
-  p.a.pieces = Pieces{plan.len, workspace};
+  const FwdPlan& plan = plan_fwd(p.a, desc->D);
+  p.a.pieces = Pieces{workspace && ws_bytes >= plan.ws_bytes ? plan.len : 0, workspace};
   int rc;
   if (desc->D == 64) {
     if (plan.kernel == FwdPlan::kWaves8) rc = launch<64, 1, 8, 64>(p, s);
@@ -710,7 +716,7 @@ extern "C" int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int
   AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
   a.kv.count = chunk_count;
   a.kv.len = desc->Sk / chunk_count;
-  return plan_fwd(a, desc->D, PICO_ATTN_MAX_WORKSPACE).ws_bytes;
+  return plan_fwd(a, desc->D).ws_bytes;
 }
 
 extern "C" int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out,

@@ -1,0 +1,114 @@
+"""Attention where the launch cuts a tile's walk into pieces (fp32 partial accumulators, summed by a second kernel), and over
+chunk lists whose chunks end inside a key tile: against an fp32 reference, in every form the epilogues have (plain, merged
+into a running result, accumulated into fp32 sums, rounded totals)."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from oracle import layers as OL
+from test_gpu_sweep import reference, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(device, B, Hq, Hkv, Sq, Sk, D):
+    g = torch.Generator(device="cuda").manual_seed(Sq + 7 * Sk + D)
+    make = lambda *s: torch.randn(*s, generator=g, device=device).to(torch.bfloat16)  # noqa: E731
+    return make(B, Hq, Sq, D), make(B, Hkv, Sk, D), make(B, Hkv, Sk, D), make(B, Hq, Sq, D)
+
+
+def check(got, want, what):
+    out, lse, dq, dk, dv = got
+    w_out, w_lse, w_dq, w_dk, w_dv = want
+    assert (out.float() - w_out).abs().max().item() <= 2e-2, what
+    assert torch.equal(torch.isinf(lse), torch.isinf(w_lse)), what
+    assert (lse - w_lse).masked_fill(torch.isinf(w_lse), 0.0).abs().max().item() <= 1e-3, what
+    for a, b, name in ((dq, w_dq, "dq"), (dk, w_dk, "dk"), (dv, w_dv, "dv")):
+        assert rel_l2(a, b) <= 1e-2, (what, name)
+
+
+# B, Hq, Hkv, Sq, Sk, D, causal, q_offset, cut (forward, backward): whether the launches are expected to cut
+CASES = [
+    (1, 1, 1, 4000, 4000, 64, True, 0, (True, True)),       # one head, ragged
+    (1, 8, 2, 2048, 2048, 64, True, 0, (False, True)),       # GQA
+    (2, 9, 3, 1057, 1057, 64, True, 0, (False, True)),
+    (2, 32, 8, 1531, 1531, 128, True, 0, (False, True)),     # head_dim 128, ragged, GQA
+    (1, 12, 4, 3000, 3000, 128, True, 0, (True, True)),
+    (1, 2, 2, 300, 5001, 64, False, 0, (True, True)),       # few queries, many keys, no mask
+    (1, 2, 1, 5001, 300, 128, False, 0, (False, True)),      # the other way round
+    (1, 2, 2, 2100, 2500, 128, True, 400, (True, True)),    # shifted diagonal
+    (1, 2, 2, 5100, 3500, 64, True, 0, (True, True)),       # keys end before the last queries
+    (1, 2, 2, 40, 40, 64, True, 0, (False, False)),         # one tile: nothing to cut
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,q_offset,cut", CASES)
+def test_attention_in_pieces(device, B, Hq, Hkv, Sq, Sk, D, causal, q_offset, cut):
+    from picotron_amd import _lib, ops
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, Sk, D)
+    scale = 1 / math.sqrt(D)
+    d = ops._desc(q, k, v, q, scale, causal, q_offset)
+    for need, expected in zip((_lib.lib().pico_attn_fwd_workspace_bytes(ctypes.byref(d), 1),
+                               _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1)), cut):
+        assert (need > 0) == expected
+    want = reference(q, k, v, scale, q_offset, causal, do)
+
+    out, lse = ops.attn_fwd(q, k, v, scale, causal, q_offset)
+    dq, dk, dv = (torch.empty_like(t) for t in (q, k, v))
+    ops.attn_bwd(do, q, k, v, lse, None, scale, causal, q_offset, dq=dq, dk=dk, dv=dv, out=out)
+    check((out, lse, dq, dk, dv), want, "bf16 results")
+
+    # a second half of the keys merged into the first half's running result; sums accumulated in fp32
+    if not causal:
+        h = Sk // 2
+        o32, l32 = ops.attn_fwd(q, k[:, :, :h].contiguous(), v[:, :, :h].contiguous(), scale, False, out_dtype=torch.float32)
+        ops.attn_fwd(q, k[:, :, h:].contiguous(), v[:, :, h:].contiguous(), scale, False, out=o32, lse=l32, merge=True)
+        assert (o32 - want[0]).abs().max().item() <= 2e-2 and (l32 - want[1]).abs().max().item() <= 1e-3
+    base = [torch.randn(t.shape, device=device, generator=torch.Generator(device="cuda").manual_seed(5)) for t in (q, k, v)]
+    sums = [t.clone() for t in base]
+    ops.attn_bwd(do, q, k, v, lse, None, scale, causal, q_offset, dq=sums[0], dk=sums[1], dv=sums[2], dq_accumulate=True,
+                 dkv_accumulate=True, out=out)
+    check((out, lse, *(s - b for s, b in zip(sums, base))), want, "accumulated")
+    # the launches of one call on two inputs in a row share nothing: same inputs, same bits
+    again, lse2 = ops.attn_fwd(q, k, v, scale, causal, q_offset)
+    assert torch.equal(out, again) and torch.equal(lse, lse2)
+
+
+# B, Hq, Hkv, chunks, chunk length, D, causal
+RAGGED = [(1, 4, 2, 3, 65, 64, True), (1, 2, 2, 4, 113, 128, True), (2, 4, 4, 2, 174, 64, False), (1, 2, 1, 16, 200, 128, True),
+          (1, 8, 2, 4, 1000, 64, True), (1, 2, 2, 5, 127, 64, True), (2, 32, 32, 3, 129, 64, True)]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,W,Sc,D,causal", RAGGED)
+def test_ragged_chunk_lists(device, B, Hq, Hkv, W, Sc, D, causal):
+    """The last rank of a ring whose chunk length is no multiple of a key tile, RoPE inside, dk / dv both as accumulated fp32
+    sums and as totals rounded to bf16."""
+    from picotron_amd import ops
+    S, off, scale = W * Sc, (W - 1) * Sc, 1 / math.sqrt(D)
+    _, k, v, _ = inputs(device, B, Hq, Hkv, Sc, S, D)
+    q, _, _, do = inputs(device, B, Hq, Hkv, Sc, Sc, D)
+    cos, sin = (t.to(device) for t in OL.get_cos_sin(S, D, 10000.0, torch.float32))
+    k_rot = ops.rope(k, cos, sin)
+    q_rot_want = ops.rope(q, cos, sin, pos_offset=off)
+    w_out, w_lse, w_dq, w_dk, w_dv = reference(q_rot_want, k_rot, v, scale, off, causal, do)
+    turn_back = lambda t, o: ops.rope(t.to(torch.bfloat16), cos, -sin, pos_offset=o).float()  # noqa: E731
+    want = (w_out, w_lse, turn_back(w_dq, off), turn_back(w_dk, 0), w_dv)
+
+    ks, vs = ([c.contiguous() for c in t.chunk(W, dim=2)] for t in (k_rot, v))
+    assert ops.chunks_fit_one_launch(ks, vs)
+    out, lse, q_rot = ops.attn_fwd_chunks(q, ks, vs, scale, causal, off, rope=(cos, sin), q_pos_offset=off, want_q_rot=True)
+    assert rel_l2(q_rot.float(), q_rot_want.float()) <= 2e-3
+    base = [torch.randn(B, Hkv, Sc, D, device=device) for _ in range(2 * W)]
+    sums = [t.clone() for t in base]
+    finals = [torch.empty(B, Hkv, Sc, D, dtype=torch.bfloat16, device=device) for _ in range(2 * W)]
+    dq = torch.empty(q.shape, dtype=torch.float32, device=device)
+    for final in (None, finals):             # the second call adds the block once more to the sums the first one left
+        ops.attn_bwd_chunks(do, q_rot, ks, vs, lse, scale, causal, off, dq, sums[:W], sums[W:], dkv_accumulate=[True] * W, out=out,
+                            rope=(cos, sin), q_pos_offset=off, dk_finals=final and final[:W], dv_finals=final and final[W:])
+    added = [s - b for s, b in zip(sums, base)]
+    check((out, lse, dq, torch.cat(added[:W], 2), torch.cat(added[W:], 2)), want, "accumulated")
+    totals = [2 * w + torch.cat(b, 2) for w, b in ((want[3], base[:W]), (want[4], base[W:]))]
+    for got, total in zip((torch.cat(finals[:W], 2), torch.cat(finals[W:], 2)), totals):
+        assert rel_l2(got.float(), total) <= 1e-2
