@@ -328,6 +328,13 @@ int pico_convert_f32(const float* src, void* dst, int64_t B, int64_t H, int64_t 
  */
 int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int dst_dtype, void* stream);
 
+/* y[c][r] = x[r][c] for bf16 x [rows, cols] with row pitch x_pitch and y [cols, rows] with row pitch y_pitch (elements).  cols
+ * and both pitches must be multiples of 8, pointers 16-byte aligned; where rows is no multiple of 8, zeros follow a row of y
+ * up to the next multiple.  Lays an operand of a weight gradient out as the GEMM library reads it faster.
+ * No counterpart in the reference (its products are torch's).
+ */
+int pico_transpose(const void* x, void* y, int64_t rows, int64_t cols, int64_t x_pitch, int64_t y_pitch, void* stream);
+
 /* ------------------------------------------------------------------ loss
  * replaces: F.cross_entropy(outputs.view(S*B, V), target_ids, reduction='mean')  train.py:46-49  and its autograd.
  * logits: [rows, vocab] with row pitch ld (elements; a multiple of 8 for bf16, 4 for fp32), dtype `dtype`;

@@ -226,6 +226,50 @@ __global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float* __rest
   }
 }
 
+// ---------------------------------------------------------------------------------- transposition
+// y[c][r] = x[r][c] over tiles of 128 rows x 64 columns: whole 128-byte lines of x are read and whole 256-byte pieces of y's
+// rows written, 16 bytes a lane.  A lane reads its 8 columns of two rows and leaves them in LDS as 8 (row, row + 1) pairs, a
+// word each, so that a column's words lie side by side; the pitch of 65 words keeps both the writes (banks 8 * vector + row
+// pair) and the reads (column + 4 * vector) free of conflicts.  Bound by memory traffic.
+constexpr int kTurnRows = 128, kTurnCols = 64, kTurnPitch = kTurnRows / 2 + 1;
+__global__ __launch_bounds__(kThreads) void transpose_kernel(const __bf16* __restrict__ x, __bf16* __restrict__ y, int64_t rows, int64_t cols,
+                                                             int64_t x_pitch, int64_t y_pitch) {
+  __shared__ uint32_t tile[kTurnCols * kTurnPitch];
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kTurnRows, col0 = static_cast<int64_t>(blockIdx.y) * kTurnCols;
+  constexpr int kVecs = kTurnCols / 8, kPairs = kTurnRows / 2, kLoads = kPairs * kVecs / kThreads;
+  u32x4 a[kLoads], b[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int idx = static_cast<int>(threadIdx.x) + i * kThreads, vec = idx % kVecs, pair = idx / kVecs;
+    const int64_t r = row0 + 2 * pair, c = col0 + 8 * vec;
+    a[i] = b[i] = u32x4{0, 0, 0, 0};
+    if (c < cols && r < rows) {
+      a[i] = *reinterpret_cast<const u32x4*>(x + r * x_pitch + c);
+      if (r + 1 < rows) b[i] = *reinterpret_cast<const u32x4*>(x + (r + 1) * x_pitch + c);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int idx = static_cast<int>(threadIdx.x) + i * kThreads, vec = idx % kVecs, pair = idx / kVecs;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t lo = a[i][e / 2] >> (16 * (e % 2)), hi = b[i][e / 2] >> (16 * (e % 2));
+      tile[(8 * vec + e) * kTurnPitch + pair] = (lo & 0xffffu) | (hi << 16);
+    }
+  }
+  __syncthreads();
+  constexpr int kOut = kTurnRows / 8, kStores = kTurnCols * kOut / kThreads;
+#pragma unroll
+  for (int i = 0; i < kStores; ++i) {
+    const int idx = static_cast<int>(threadIdx.x) + i * kThreads, vec = idx % kOut, c = idx / kOut;
+    if (col0 + c >= cols || row0 + 8 * vec >= y_pitch) continue;
+    u32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = tile[c * kTurnPitch + 4 * vec + j];
+    *reinterpret_cast<u32x4*>(y + (col0 + c) * y_pitch + row0 + 8 * vec) = v;
+  }
+}
+
 unsigned blocks_for(int64_t total) { return static_cast<unsigned>((total + kThreads - 1) / kThreads); }
 bool dtype_ok(int d) { return d == PICO_BF16 || d == PICO_F32; }
 int vec_of(int d) { return d == PICO_BF16 ? 8 : 4; }
@@ -390,4 +434,18 @@ extern "C" int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_
   else
     hipLaunchKernelGGL(sum_parts_kernel<float>, dim3(blocks_for(n / 8)), dim3(kThreads), 0, st, src, static_cast<float*>(dst), (int)parts, n);
   return check_launch("pico_sum_parts");
+}
+
+extern "C" int pico_transpose(const void* x, void* y, int64_t rows, int64_t cols, int64_t x_pitch, int64_t y_pitch, void* stream) {
+  if (rows < 0 || cols < 0 || cols % 8 != 0 || x_pitch < cols || x_pitch % 8 != 0 || y_pitch < rows || y_pitch % 8 != 0)
+    return fail(PICO_ERR_SHAPE, "pico_transpose: rows=%lld cols=%lld pitches %lld, %lld (columns and pitches must be multiples of 8)",
+                (long long)rows, (long long)cols, (long long)x_pitch, (long long)y_pitch);
+  if (rows == 0 || cols == 0) return PICO_OK;
+  const int64_t gx = (rows + kTurnRows - 1) / kTurnRows, gy = (cols + kTurnCols - 1) / kTurnCols;
+  if (gx > 0x7fffffff || gy > 65535) return fail(PICO_ERR_SHAPE, "pico_transpose: matrix too large");
+  if (!x || !y) return fail(PICO_ERR_NULL, "pico_transpose: x and y are required");
+  if (!aligned16(x) || !aligned16(y)) return fail(PICO_ERR_ALIGN, "pico_transpose: pointers must be 16-byte aligned");
+  hipLaunchKernelGGL(transpose_kernel, dim3(static_cast<unsigned>(gx), static_cast<unsigned>(gy)), dim3(kThreads), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const __bf16*>(x), static_cast<__bf16*>(y), rows, cols, x_pitch, y_pitch);
+  return check_launch("pico_transpose");
 }

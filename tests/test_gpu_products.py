@@ -23,6 +23,23 @@ def test_products_in_pieces(device, kind, M, N, K):
         assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, parts
 
 
+@pytest.mark.parametrize("K,M,N", [(1, 8, 16), (127, 72, 64), (130, 64, 520), (1000, 1000, 248), (1025, 16384, 1032), (1111, 1024, 32000)])
+def test_weight_gradients_with_transposed_operands(device, K, M, N):
+    from picotron_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randn(K, n, generator=g, device=device).to(torch.bfloat16) for n in (M, N))
+    want = a.float().t() @ b.float()
+    for turn in (-1, 0, 1, 2, 3):            # -1: the rule's own choice
+        got = _lib.host().product(a, b, "TN", 0, turn)
+        assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, turn
+    # columns of a wider matrix; the padding behind a row of the result is zero
+    wide = torch.randn(K, M + 24, generator=g, device=device).to(torch.bfloat16)
+    pitch = (K + 7) // 8 * 8
+    y = torch.full((M, pitch), 3.0, dtype=torch.bfloat16, device=device)
+    rc = _lib.lib().pico_transpose(wide[:, 8:].data_ptr(), y.data_ptr(), K, M, M + 24, pitch, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(y[:, :K], wide[:, 8:8 + M].t()) and not y[:, K:].any()
+
+
 def test_linear_layer_gradients_match_torch(device):
     from picotron_amd.model import Linear
     g = torch.Generator(device="cuda").manual_seed(3)
