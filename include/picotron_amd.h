@@ -335,6 +335,18 @@ int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int ds
  */
 int pico_transpose(const void* x, void* y, int64_t rows, int64_t cols, int64_t x_pitch, int64_t y_pitch, void* stream);
 
+/* ------------------------------------------------------------------ embedding
+ * replaces: the backward of F.embedding in Embedding.forward  model.py:237-251.
+ * dw[v] = sum over the tokens t with ids[t] == v of dy[t] (added in fp32 in the order of the tokens, rounded once), zero for
+ * every other row and for row skip_id (-1: none).  ids: int32 or int64 (id_bytes 4 or 8); ids outside [0, vocab) add nothing.
+ * dy [tokens, hidden] and dw [vocab, hidden] are contiguous, of dtype `dtype`; hidden a multiple of 8, at most
+ * PICO_EMBEDDING_MAX_TOKENS tokens.  workspace: pico_embedding_bwd_workspace_bytes(tokens, hidden) bytes (-1: too large).
+ */
+#define PICO_EMBEDDING_MAX_TOKENS 32768
+int64_t pico_embedding_bwd_workspace_bytes(int64_t tokens, int64_t hidden);
+int pico_embedding_bwd(const void* ids, int id_bytes, const void* dy, void* dw, void* workspace, int64_t tokens, int64_t vocab,
+                       int64_t hidden, int64_t skip_id, int dtype, void* stream);
+
 /* ------------------------------------------------------------------ loss
  * replaces: F.cross_entropy(outputs.view(S*B, V), target_ids, reduction='mean')  train.py:46-49  and its autograd.
  * logits: [rows, vocab] with row pitch ld (elements; a multiple of 8 for bf16, 4 for fp32), dtype `dtype`;

@@ -27,6 +27,15 @@ class RMSNormResidualFunc:
         return _lib.host().rms_norm_residual(x, residual, weight, eps)
 
 
+class RMSNormHeadFunc:
+    """``apply(x, weight, eps)``: returns (rmsnorm(x) * w, x): RMSNormResidualFunc where there is nothing to add yet.  The
+    gradients of both outputs meet inside the backward kernel."""
+
+    @staticmethod
+    def apply(x, weight, eps):
+        return _lib.host().rms_norm_head(x, weight, eps)
+
+
 class RotaryFunc:
     """``apply(x, cos, sin, pos_offset)``: non-interleaved RoPE on [B,H,S,D]; the backward is the rotation by -theta."""
 

@@ -35,7 +35,7 @@ import torch.nn.functional as F
 import picotron_amd.process_group_manager as pgm
 from picotron_amd import _lib
 from picotron_amd.context_parallel import context_parallel
-from picotron_amd.functional import (FusedLinearFunc, QKVAttentionFunc, RMSNormFunc, RMSNormResidualFunc,
+from picotron_amd.functional import (FusedLinearFunc, QKVAttentionFunc, RMSNormFunc, RMSNormHeadFunc, RMSNormResidualFunc,
                                      RotaryFunc, SwiGLUFunc, SwiGLUFusedFunc, _fused_rope)
 
 
@@ -87,8 +87,9 @@ class TritonRMSNorm(nn.Module):
         of the norm kernel."""
         if dropout_p == 0.0 and not return_dropout_mask and not residual_in_fp32:
             if residual is None:
-                y = RMSNormFunc.apply(hidden_states, self.weight, self.eps, False)
-                return (y, hidden_states) if prenorm else y
+                if prenorm:
+                    return RMSNormHeadFunc.apply(hidden_states, self.weight, self.eps)
+                return RMSNormFunc.apply(hidden_states, self.weight, self.eps, False)
             y, h = RMSNormResidualFunc.apply(hidden_states, residual, self.weight, self.eps)
             return (y, h) if prenorm else y
         x = hidden_states
@@ -331,7 +332,9 @@ class Embedding(nn.Module):
         torch.nn.init.normal_(self.weight, mean=0.0, std=1.0)
 
     def forward(self, x):
-        return F.embedding(x, self.weight, self.padding_idx)
+        if not self.weight.is_cuda or (self.padding_idx is not None and not 0 <= self.padding_idx < self.num_embeddings):
+            return F.embedding(x, self.weight, self.padding_idx)
+        return _lib.host().embedding(x, self.weight, -1 if self.padding_idx is None else self.padding_idx)
 
 
 class Llama(nn.Module):
