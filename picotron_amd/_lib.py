@@ -110,12 +110,7 @@ _host = None
 
 
 def host():
-    """The Python extension with the host path of the hot ops (csrc/host.cpp); raises if it was never built.
-
-    The first call also turns off autograd's device threads for the calling thread (a thread-local torch setting, see
-    ``torch.autograd.set_multithreading_enabled``): one process drives one GPU here, so a backward pass gains nothing
-    from a second thread and pays for two thread wake-ups -- 35 us of a 73 us RMSNorm forward + backward, 270 us of a
-    1465 us training step of the two-layer 135M shape.  ``PICO_AUTOGRAD_THREADS=1`` leaves the setting alone."""
+    """The Python extension with the host path of the hot ops (csrc/host.cpp); raises if it was never built."""
     global _host
     if _host is None:
         lib()
@@ -125,9 +120,6 @@ def host():
             raise RuntimeError(f"picotron_amd/_host.so cannot be loaded ({e}): build it first with "
                                "`python -m picotron_amd.build`") from e
         _host = module
-        if os.getenv("PICO_AUTOGRAD_THREADS", "0") != "1":
-            import torch
-            torch.autograd.set_multithreading_enabled(False)
     return _host
 
 
