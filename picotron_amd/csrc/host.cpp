@@ -185,7 +185,7 @@ Tensor rms_norm(const Tensor& x, const Tensor& weight, double eps, bool cast_the
 }
 
 std::pair<Tensor, Tensor> rms_norm_head(const Tensor& x, const Tensor& weight, double eps) {
-  if (!records({&x, &weight})) return {rmsnorm_forward(x, weight, eps, false, std::nullopt, false, false).y, x};
+  if (!records({&x})) return {rms_norm(x, weight, eps, false), x};   // (x has no gradient: it passes as it is)
   auto o = RMSNormHead::apply(x, weight, eps);
   return {o[0], o[1]};
 }
@@ -926,6 +926,21 @@ bool plain(const Tensor& t) {
 }
 Tensor matrix(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
 
+// Ordinary tensors in ordinary code: no forward-mode tangent, no wrapper (vmap, torch.func transforms, functionalization,
+// __torch_dispatch__ subclasses, lazy conj / neg) and no dispatch mode or tracer that has to see the operators.  Where this is
+// not so an op that torch has goes through torch.
+bool ordinary(std::initializer_list<const Tensor*> inputs) {
+  using K = c10::DispatchKey;
+  static constexpr c10::DispatchKeySet wrapped({K::Python, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::BatchedNestedTensor,
+                                                K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor});
+  static constexpr c10::DispatchKeySet modes({K::Python, K::PythonTLSSnapshot, K::FuncTorchDynamicLayerFrontMode, K::FuncTorchVmapMode,
+                                              K::Functionalize, K::Tracer});
+  if (c10::impl::tls_local_dispatch_key_set().included_.has_any(modes)) return false;
+  for (const Tensor* t : inputs)
+    if (t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
+  return true;
+}
+
 // row-major products: a @ b^T, a @ b, a^T @ b
 enum class Product { NT, NN, TN };
 
@@ -1012,7 +1027,10 @@ Tensor turned(const Tensor& t) {
 
 // parts 0, turn -1: by the rules above
 Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1) {
-  if (plain(a) && plain(b) && !torch_gemm_only()) {
+  // (a backward that is itself to be differentiated, create_graph, stays with torch)
+  const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
+  if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && !torch_gemm_only()) {
+    const c10::OptionalDeviceGuard device(a.device());
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
     const int64_t M = kind == Product::TN ? a.size(1) : a.size(0), K = kind == Product::TN ? a.size(0) : a.size(1);
     const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
@@ -1038,7 +1056,8 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
 }
 
 Tensor linear_forward(const Tensor& x, const Tensor& w) {
-  if (x.dim() < 1 || w.dim() != 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || torch_gemm_only()) return at::linear(x, w);
+  if (x.dim() < 1 || w.dim() != 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || torch_gemm_only() || !ordinary({&x, &w}))
+    return at::linear(x, w);
   const Tensor y = product(matrix(x), w, Product::NT);
   if (x.dim() == 2) return y;
   auto sizes = x.sizes().vec();
@@ -1046,23 +1065,25 @@ Tensor linear_forward(const Tensor& x, const Tensor& w) {
   return y.view(sizes);
 }
 
-// y = x @ w^T
+// y = x @ w^T; each operand is kept only for the other's gradient (a frozen weight keeps no activations)
 struct Linear : torch::autograd::Function<Linear> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
-    ctx->save_for_backward({x, w});
+    ctx->save_for_backward({w.requires_grad() ? x : Tensor(), x.requires_grad() ? w : Tensor()});
+    ctx->saved_data["sizes"] = x.sizes().vec();
     return linear_forward(x, w);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const auto s = ctx->get_saved_variables();
     const Tensor dy = matrix(g[0]);
     variable_list r(2);
-    if (ctx->needs_input_grad(0)) r[0] = product(dy, s[1], Product::NN).view(s[0].sizes());
+    if (ctx->needs_input_grad(0)) r[0] = product(dy, s[1], Product::NN).view(ctx->saved_data["sizes"].toIntVector());
     if (ctx->needs_input_grad(1)) r[1] = product(dy, matrix(s[0]), Product::TN);
     return r;
   }
 };
 Tensor linear(const Tensor& x, const Tensor& w) {
-  if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || torch_gemm_only()) return at::linear(x, w);
+  if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || torch_gemm_only() || !ordinary({&x, &w}))
+    return at::linear(x, w);
   return records({&x, &w}) ? Linear::apply(x, w) : linear_forward(x, w);
 }
 
@@ -1125,7 +1146,8 @@ struct Embedding : torch::autograd::Function<Embedding> {
   }
 };
 Tensor embedding(const Tensor& ids, const Tensor& weight, int64_t padding_idx) {
-  if (!records({&weight}) || !weight.is_cuda() || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt))
+  if (!records({&weight}) || !weight.is_cuda() || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) ||
+      !ordinary({&ids, &weight}))
     return at::embedding(weight, ids, padding_idx);
   return Embedding::apply(ids, weight, padding_idx);
 }

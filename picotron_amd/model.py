@@ -162,10 +162,17 @@ def _fused_weight(owner, name, linears):
     return buf
 
 
+def _native(*tensors):
+    """False where torch itself has to see the operator: under torch.compile and for __torch_function__ overrides."""
+    return not (torch.compiler.is_compiling() or torch.overrides.has_torch_function(tensors))
+
+
 class Linear(nn.Linear):
     """nn.Linear without a bias on the native host path (the same library product, its algorithm kept with the shape)."""
 
     def forward(self, x):
+        if self.bias is not None or not _native(x, self.weight):
+            return F.linear(x, self.weight, self.bias)
         return _lib.host().linear(x, self.weight)
 
 
@@ -281,7 +288,9 @@ class FinalProjection(nn.Module):
             torch.nn.init.uniform_(self.bias, -bound_b, bound_b)
 
     def forward(self, x):
-        return _lib.host().linear(x, self.weight) if self.bias is None else F.linear(x, self.weight, self.bias)
+        if self.bias is not None or not _native(x, self.weight):
+            return F.linear(x, self.weight, self.bias)
+        return _lib.host().linear(x, self.weight)
 
 
 class DecoderLayer(nn.Module):
@@ -332,7 +341,7 @@ class Embedding(nn.Module):
         torch.nn.init.normal_(self.weight, mean=0.0, std=1.0)
 
     def forward(self, x):
-        if not self.weight.is_cuda or (self.padding_idx is not None and not 0 <= self.padding_idx < self.num_embeddings):
+        if not _native(x, self.weight) or not self.weight.is_cuda or (self.padding_idx is not None and not 0 <= self.padding_idx < self.num_embeddings):
             return F.embedding(x, self.weight, self.padding_idx)
         return _lib.host().embedding(x, self.weight, -1 if self.padding_idx is None else self.padding_idx)
 

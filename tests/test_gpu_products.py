@@ -51,3 +51,39 @@ def test_linear_layer_gradients_match_torch(device):
     want = torch.autograd.grad(torch.nn.functional.linear(xf, wf), (xf, wf), dy.float())
     for a, b in zip(got, want):
         assert a.shape == b.shape and ((a.float() - b).norm() / b.norm()).item() <= 3e-3
+
+
+def test_linear_layer_where_torch_has_to_see_it(device):
+    """Second derivatives, forward-mode tangents and a frozen weight: as torch's own linear has them."""
+    from picotron_amd.model import Linear
+    F, rel = torch.nn.functional.linear, lambda a, b: ((a.float() - b).norm() / b.norm()).item()
+    g = torch.Generator(device="cuda").manual_seed(5)
+    layer = Linear(64, 48, bias=False, device=device, dtype=torch.bfloat16)
+    x, t = (torch.randn(24, 64, generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    xg, xf, wf = x.clone().requires_grad_(), x.float().requires_grad_(), layer.weight.detach().float().requires_grad_()
+
+    def second(y, inp, w):
+        (dx,) = torch.autograd.grad(y.float().square().sum(), inp, create_graph=True)
+        return torch.autograd.grad(dx.float().square().sum(), (inp, w))
+    for a, b in zip(second(layer(xg), xg, layer.weight), second(F(xf, wf), xf, wf)):
+        assert rel(a, b) <= 1.5e-2                # three chained products, each rounded to bf16 (2^-9 each way)
+
+    with torch.autograd.forward_ad.dual_level():
+        dual = layer(torch.autograd.forward_ad.make_dual(x, t))
+        tangent = torch.autograd.forward_ad.unpack_dual(dual).tangent
+    assert rel(tangent, F(t.float(), wf.detach())) <= 3e-3
+
+    layer.weight.requires_grad_(False)
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda s: kept.append(s) or s, lambda s: s):
+        y = layer(xg)
+    assert [s.shape for s in kept] == [layer.weight.shape]
+    assert rel(torch.autograd.grad(y, xg, y.detach())[0], y.float() @ wf.detach()) <= 3e-3
+
+
+def test_norm_passes_a_frozen_stream_through(device):
+    from picotron_amd.model import TritonRMSNorm
+    norm = TritonRMSNorm(64).to(device, torch.bfloat16)
+    x = torch.randn(8, 64, device=device).to(torch.bfloat16)
+    y, h = norm(x, prenorm=True)
+    assert h is x and not h.requires_grad and y.requires_grad
