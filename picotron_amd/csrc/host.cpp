@@ -1025,8 +1025,28 @@ Tensor turned(const Tensor& t) {
   return y;
 }
 
-// parts 0, turn -1: by the rules above
-Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1) {
+// Whether a product goes to the package's own kernel (pico_product), and with how many groups of waves: 0 no.  Its 64 x 64
+// tiles win where the library's leave most CUs idle, until either there are more tiles than CUs -- the library's larger ones
+// then do more per byte -- or the walk along the contraction is so long that its steps, and not its start, are the time.
+// Weight gradients (TN, the library's slowest layout) stay with it longest: [512 x 960]^T [512 x 576] 9.0 -> 6.0 us, [2331 x
+// 576]^T [2331 x 1536] 22.5 -> 14.3, but [1024 x 5440]^T [1024 x 1024], 1360 tiles, 20.6 and 27.6.  Input gradients (NN): [512 x 576] @ [576 x
+// 1536] 7.4 -> 6.1, [512 x 1024] @ [1024 x 1024] 8.9 -> 7.4, [512 x 3072] @ [3072 x 576] 15.6 and 14.8.  Forward (NT, its best):
+// [512 x 1024] @ [1024 x 1024]^T 8.5 -> 6.9, [512 x 1536] @ [1536 x 576]^T 8.0 and 9.4.  The lines lie where a sweep over 128 ..
+// 4096 rows, 576 .. 8192 columns and 128 .. 8192 of contraction crossed.
+int64_t small_product(Product kind, int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (N % 8 || (kind == Product::TN ? M : K) % 8 || tiles > 1400) return 0;
+  if (kind == Product::TN) {
+    if (tiles <= 256) return K <= 384 ? 1 : K <= 3072 ? 2 : K <= 4096 ? 4 : 0;
+    return K <= (tiles <= 512 ? 2560 : tiles <= 700 ? 800 : 320);
+  }
+  if (tiles > 256) return 0;
+  if (kind == Product::NN) return K <= 1024 || (K <= 1536 && tiles >= 64) || (K <= 2048 && tiles >= 128) ? 2 : 0;
+  return K <= 1024 && tiles >= 75 ? 2 : 0;
+}
+
+// parts 0, turn -1, groups -1: by the rules above
+Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1) {
   // (a backward that is itself to be differentiated, create_graph, stays with torch)
   const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
   if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && !torch_gemm_only()) {
@@ -1036,6 +1056,12 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
     const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
     TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
     Tensor c = at::empty({M, N}, a.options());
+    if (groups < 0) groups = parts == 0 && turn < 0 ? small_product(kind, M, N, K) : 0;
+    if (groups > 0) {
+      check(pico_product(ptr(a), ptr(b), ptr(c), M, N, K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
+                         static_cast<int>(groups), stream_now()));
+      return c;
+    }
     if (parts == 0) parts = contraction_parts(kind, M, N, K);
     TORCH_CHECK(parts >= 1 && K % parts == 0, "matrix product: a contraction of ", K, " cannot be cut into ", parts, " equal pieces");
     if (turn < 0) turn = turned_operand(kind, a, b);
@@ -1458,10 +1484,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("publish_kv", &publish_kv);
   m.def("ring_node", &ring_node);
   m.def("flash_attention", &flash_attention, nogil());
-  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn) {
+  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups) {
     TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
-    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts, turn);
-  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1);
+    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts, turn, groups);
+  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
+        pybind11::arg("groups") = -1);
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("embedding", &embedding, nogil());
