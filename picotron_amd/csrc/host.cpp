@@ -799,7 +799,7 @@ Tensor ring_node(const Tensor& q, const std::vector<Tensor>& ks, const std::vect
 }
 
 // ------------------------------------------------------------------------------------------------ projections
-// The model's matrix products are plain library GEMMs (hipBLASLt, the library torch calls too).  torch asks the library's
+// The model's large matrix products are plain library GEMMs (hipBLASLt, the library torch calls too).  torch asks the library's
 // heuristic for an algorithm on every call, which is most of the 25-30 us of host time a product costs there; here the
 // answer is kept with the shape, and a product costs its launch.  At most kMaxPlans shapes are kept; all are dropped when
 // one more is asked for.
@@ -1025,28 +1025,43 @@ Tensor turned(const Tensor& t) {
   return y;
 }
 
-// Whether a product goes to the package's own kernel (pico_product), and with how many groups of waves: 0 no.  Its 64 x 64
-// tiles win where the library's leave most CUs idle, until either there are more tiles than CUs -- the library's larger ones
-// then do more per byte -- or the walk along the contraction is so long that its steps, and not its start, are the time.
-// Weight gradients (TN, the library's slowest layout) stay with it longest: [512 x 960]^T [512 x 576] 9.0 -> 6.0 us, [2331 x
-// 576]^T [2331 x 1536] 22.5 -> 14.3, but [1024 x 5440]^T [1024 x 1024], 1360 tiles, 20.6 and 27.6.  Input gradients (NN): [512 x 576] @ [576 x
-// 1536] 7.4 -> 6.1, [512 x 1024] @ [1024 x 1024] 8.9 -> 7.4, [512 x 3072] @ [3072 x 576] 15.6 and 14.8.  Forward (NT, its best):
-// [512 x 1024] @ [1024 x 1024]^T 8.5 -> 6.9, [512 x 1536] @ [1536 x 576]^T 8.0 and 9.4.  The lines lie where a sweep over 128 ..
-// 4096 rows, 576 .. 8192 columns and 128 .. 8192 of contraction crossed.
-int64_t small_product(Product kind, int64_t M, int64_t N, int64_t K) {
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (N % 8 || (kind == Product::TN ? M : K) % 8 || tiles > 1400) return 0;
+// Whether a product goes to the package's own kernel (pico_product), with tiles of which side and how many groups of waves
+// (0: no).  It wins where the library's tiles leave most CUs idle, until either there are more tiles than CUs -- the
+// library's larger ones then do more per byte -- or the walk along the contraction is so long that its steps, and not its
+// start, are the time.  Weight gradients (TN, the library's slowest layout) stay with it longest.  Library and own kernel, us:
+//   TN, tiles of 64 while they are at most 256, or 512 and the walk short: [512 x 960]^T [512 x 576] 9.0, 6.0;
+//      [2331 x 576]^T [2331 x 1536] 22.5, 14.3; [3072 x 576] from 1024 rows 14.2, 13.1, from 4096 35, 37;
+//   TN, up to 256 tiles of 128, two groups: [2048 x 2048] from 512 rows 13.6, 11.3, from 4096 47, 43; [3072 x 1024] from 2630
+//      40, 29; [1024 x 2688] from 4096 41, 40, from 8192 70, 76;
+//   TN, more tiles of 128: few rows.  [49152 x 576] from 512 69, 48, from 1024 93, 89.  The library runs an even number of
+//      its tiles side by side best and a ragged contraction a quarter slower: [32000 x 1024] from 512 46, 48, [2048 x 8192]
+//      26, 36, but [32000 x 1152] 61, 50 and [8192 x 1024] from 443 20, 14;
+//   NN: [512 x 576] @ [576 x 1536] 7.4, 6.1; [512 x 1024] @ [1024 x 1024] 8.9, 7.4; [512 x 3072] @ [3072 x 576] 15.6, 14.8;
+//   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.5, 6.9; [512 x 1536] @ [1536 x 576]^T 8.0, 9.4.
+// Over 240 drawn shapes that these lines send here the geometric mean of the time over the library's is 0.70 for weight
+// gradients, 0.78 and 0.82 for NN and NT; the worst are 3 % slower.  The lines lie where sweeps over 100 .. 8192 rows, 128 ..
+// 49152 columns and 128 .. 8192 of contraction crossed.
+struct OwnProduct {
+  int64_t groups, tile;
+};
+OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), wide_tiles = ((M + 127) / 128) * ((N + 127) / 128), narrow = std::min(M, N);
+  constexpr OwnProduct no = {0, 64};
+  if (N % 8 || (kind == Product::TN ? M : K) % 8) return no;
   if (kind == Product::TN) {
-    if (tiles <= 256) return K <= 384 ? 1 : K <= 3072 ? 2 : K <= 4096 ? 4 : 0;
-    return K <= (tiles <= 512 ? 2560 : tiles <= 700 ? 800 : 320);
+    if (tiles <= 256) return K <= 384 ? OwnProduct{1, 64} : K <= 3072 ? OwnProduct{2, 64} : K <= 4096 ? OwnProduct{4, 64} : no;
+    if (wide_tiles <= 128) return K <= 2560 ? OwnProduct{1, 64} : no;
+    if (wide_tiles <= 256) return K <= 384 ? OwnProduct{1, 128} : K <= (wide_tiles >= 230 ? 8192 : 4096) ? OwnProduct{2, 128} : no;
+    const int64_t most = narrow % 512 ? (K % 64 ? 1000 : 768) : (K % 64 ? 576 : 320);
+    return K <= most && wide_tiles <= 3500 ? OwnProduct{1, 128} : no;
   }
-  if (tiles > 256) return 0;
-  if (kind == Product::NN) return K <= 1024 || (K <= 1536 && tiles >= 64) || (K <= 2048 && tiles >= 128) ? 2 : 0;
-  return K <= 1024 && tiles >= 75 ? 2 : 0;
+  if (tiles > 256) return no;
+  if (kind == Product::NN) return K <= 1024 || (K <= 1536 && tiles >= 64) || (K <= 2048 && tiles >= 128) ? OwnProduct{2, 64} : no;
+  return K <= 1024 && tiles >= 75 ? OwnProduct{2, 64} : no;
 }
 
 // parts 0, turn -1, groups -1: by the rules above
-Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1) {
+Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64) {
   // (a backward that is itself to be differentiated, create_graph, stays with torch)
   const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
   if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && !torch_gemm_only()) {
@@ -1056,10 +1071,14 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
     const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
     TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
     Tensor c = at::empty({M, N}, a.options());
-    if (groups < 0) groups = parts == 0 && turn < 0 ? small_product(kind, M, N, K) : 0;
+    if (groups < 0) {
+      const OwnProduct own = parts == 0 && turn < 0 ? own_product(kind, M, N, K) : OwnProduct{0, 64};
+      groups = own.groups;
+      tile = own.tile;
+    }
     if (groups > 0) {
       check(pico_product(ptr(a), ptr(b), ptr(c), M, N, K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
-                         static_cast<int>(groups), stream_now()));
+                         static_cast<int>(tile), static_cast<int>(groups), stream_now()));
       return c;
     }
     if (parts == 0) parts = contraction_parts(kind, M, N, K);
@@ -1484,11 +1503,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("publish_kv", &publish_kv);
   m.def("ring_node", &ring_node);
   m.def("flash_attention", &flash_attention, nogil());
-  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups) {
+  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile) {
     TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
-    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts, turn, groups);
+    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts, turn, groups, tile);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
-        pybind11::arg("groups") = -1);
+        pybind11::arg("groups") = -1, pybind11::arg("tile") = 64);
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("embedding", &embedding, nogil());

@@ -94,18 +94,18 @@ def test_norm_passes_a_frozen_stream_through(device):
     ("NN", 1, 8, 8), ("NN", 63, 72, 64), ("NN", 65, 64, 200), ("NN", 512, 576, 960), ("NN", 300, 520, 3072),
     ("TN", 8, 8, 1), ("TN", 72, 64, 63), ("TN", 64, 72, 197), ("TN", 576, 960, 512), ("TN", 520, 136, 2331)])
 def test_small_products(device, kind, M, N, K):
-    """The package's own kernel: edges of its 64 x 64 x 64 tiles, contractions shorter than a group's share, wider row pitches."""
+    """The package's own kernel: edges of its tiles of 64 and 128 and its steps of 64, contractions shorter than a group's share, wider row pitches."""
     from picotron_amd import _lib
     g = torch.Generator(device="cuda").manual_seed(M * N + K)
     shapes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     for pad in (0, 24):
         a, b = (torch.randn(r, c + pad, generator=g, device=device).to(torch.bfloat16)[:, :c] for r, c in shapes)
         want = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float())
-        for groups in (1, 2, 4):
-            got = _lib.host().product(a, b, kind, groups=groups)
+        for tile, groups in ((64, 1), (64, 2), (64, 4), (128, 1), (128, 2)):
+            got = _lib.host().product(a, b, kind, groups=groups, tile=tile)
             assert got.shape == (M, N) and got.dtype == torch.bfloat16
-            assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (pad, groups)
-            assert torch.equal(got, _lib.host().product(a, b, kind, groups=groups))
+            assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (pad, tile, groups)
+            assert torch.equal(got, _lib.host().product(a, b, kind, groups=groups, tile=tile))
     exact = _lib.host().product(a.round(), b.round(), kind, groups=4)     # small integers: sums are exact in fp32
     want = (a.round().float().t() if kind == "TN" else a.round().float()) @ (b.round().float().t() if kind == "NT" else b.round().float())
     assert torch.equal(exact, want.to(torch.bfloat16))
