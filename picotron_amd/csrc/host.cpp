@@ -1029,18 +1029,19 @@ Tensor turned(const Tensor& t) {
 // (0: no).  It wins where the library's tiles leave most CUs idle, until either there are more tiles than CUs -- the
 // library's larger ones then do more per byte -- or the walk along the contraction is so long that its steps, and not its
 // start, are the time.  Weight gradients (TN, the library's slowest layout) stay with it longest.  Library and own kernel, us:
-//   TN, tiles of 64 while they are at most 256, or 512 and the walk short: [512 x 960]^T [512 x 576] 9.0, 6.0;
-//      [2331 x 576]^T [2331 x 1536] 22.5, 14.3; [3072 x 576] from 1024 rows 14.2, 13.1, from 4096 35, 37;
-//   TN, up to 256 tiles of 128, two groups: [2048 x 2048] from 512 rows 13.6, 11.3, from 4096 47, 43; [3072 x 1024] from 2630
-//      40, 29; [1024 x 2688] from 4096 41, 40, from 8192 70, 76;
+//   TN, tiles of 64 while they are at most 256, or 512 and the walk short: [512 x 960]^T [512 x 576] 9.2, 6.0;
+//      [2331 x 1024]^T [2331 x 1024] 24, 15; [3072 x 576] from 1024 rows 14.2, 13.1, from 4096 35, 37;
+//   TN, up to 256 tiles of 128, two groups: [2048 x 2048] from 512 rows 13.6, 11.3, from 4096 49, 42; [3072 x 1024] from 2630
+//      41, 27; [1024 x 2688] from 4096 41, 40, from 8192 70, 76;
 //   TN, more tiles of 128: few rows.  [49152 x 576] from 512 69, 48, from 1024 93, 89.  The library runs an even number of
-//      its tiles side by side best and a ragged contraction a quarter slower: [32000 x 1024] from 512 46, 48, [2048 x 8192]
-//      26, 36, but [32000 x 1152] 61, 50 and [8192 x 1024] from 443 20, 14;
-//   NN: [512 x 576] @ [576 x 1536] 7.4, 6.1; [512 x 1024] @ [1024 x 1024] 8.9, 7.4; [512 x 3072] @ [3072 x 576] 15.6, 14.8;
-//   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.5, 6.9; [512 x 1536] @ [1536 x 576]^T 8.0, 9.4.
-// Over 240 drawn shapes that these lines send here the geometric mean of the time over the library's is 0.70 for weight
-// gradients, 0.78 and 0.82 for NN and NT; the worst are 3 % slower.  The lines lie where sweeps over 100 .. 8192 rows, 128 ..
-// 49152 columns and 128 .. 8192 of contraction crossed.
+//      its tiles side by side best and a ragged contraction a quarter slower: [32000 x 1024] from 512 46, 48, but [32000 x
+//      1152] 61, 50 and [8192 x 1024] from 443 20, 14;
+//   NN: [512 x 1024] @ [1024 x 1024] 9.2, 7.4; [512 x 3072] @ [3072 x 576] 17.0, 14.2; [512 x 2048] @ [2048 x 2048] 15, 12;
+//      tiles of 128: [4096 x 1536] @ [1536 x 1024] 21, 19, but with 512 of them [4096 x 2048] @ [2048 x 2048] 37, 41;
+//   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.4, 6.8; [512 x 1536] @ [1536 x 576]^T 8.4, 8.8.
+// Over 16000 drawn NN and NT products the time over the library's was, by classes of tiles and contraction, 0.62 - 0.96 in
+// the geometric mean where these lines choose the kernel (no class with a case more than 4 % slower) and mostly over 1 beyond;
+// over 150 drawn TN ones 0.70 (worst 1.03).  100 .. 8192 rows, 128 .. 49152 columns, contractions of 128 .. 8192.
 struct OwnProduct {
   int64_t groups, tile;
 };
@@ -1055,9 +1056,13 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
     const int64_t most = narrow % 512 ? (K % 64 ? 1000 : 768) : (K % 64 ? 576 : 320);
     return K <= most && wide_tiles <= 3500 ? OwnProduct{1, 128} : no;
   }
-  if (tiles > 256) return no;
-  if (kind == Product::NN) return K <= 1024 || (K <= 1536 && tiles >= 64) || (K <= 2048 && tiles >= 128) ? OwnProduct{2, 64} : no;
-  return K <= 1024 && tiles >= 75 ? OwnProduct{2, 64} : no;
+  if (tiles > 512) {
+    if (wide_tiles > 256) return no;
+    return K <= 600 ? OwnProduct{1, 128} : kind == Product::NN && K <= 4096 ? OwnProduct{2, 128} : no;
+  }
+  if (tiles > 256) return K <= 600 ? OwnProduct{1, 64} : no;
+  if (kind == Product::NN) return K <= (tiles <= 32 ? 1088 : tiles <= 64 ? 2112 : 4096) ? OwnProduct{2, 64} : no;
+  return K <= (tiles > 128 ? 3072 : tiles > 60 ? 1088 : 0) ? OwnProduct{2, 64} : no;
 }
 
 // parts 0, turn -1, groups -1: by the rules above

@@ -4,8 +4,8 @@
 // What bounds them is latency: [512 x 576] @ [576 x 576] moves 2 MB and takes 0.3 GFLOP, half a microsecond of either, but
 // every step of a walk waits for memory.  So: tiles of 64 x 64 (enough workgroups from few rows), three steps of 64 requested
 // ahead in registers, two LDS buffers, and the walk dealt to KS groups of four waves inside the workgroup, whose fp32 sums
-// meet in LDS in the order of the groups (the same result on every run, no second launch).  A step costs 0.4 us in one group
-// and start plus end 2.5 us: [512 x 960]^T [512 x 576] takes 6.0 us (library 9.0).
+// meet in LDS in the order of the groups (the same result on every run, no second launch).  A step costs 0.3 us in one group
+// and start plus end 3 us: [512 x 960]^T [512 x 576] takes 6.0 us (library 9.2).
 // With more tiles than CUs the reads of LDS are the bound, 3 KiB per MFMA of a tile of 64; tiles of 128 take 2 KiB, and two
 // workgroups fit a CU: [512 x 49152]^T [512 x 576] 48 us = 600 TFLOP/s (tiles of 64: 61, library 69).  The error against 64
 // bits is the library's (1.66e-3, the rounding to bf16).
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256 * KS, 2) void product_kernel(const ProductParam
   B b;
   a.open(p.a, p.lda, m0, p.M, p.K, tid);
   b.open(p.b, p.ldb, n0, p.N, p.K, tid);
-  constexpr int kDeep = W == 1 ? kAhead : 2;   // (steps requested ahead: registers allow the larger tile two)
+  constexpr int kDeep = W == 1 || KS == 1 ? kAhead : 2;   // (steps requested ahead; two groups of a tile of 128 gain nothing from a third)
   u32x4 ra[kDeep][A::kPieces], rb[kDeep][B::kPieces];
 #pragma unroll
   for (int u = 0; u < kDeep; ++u) {
@@ -124,46 +124,52 @@ __global__ __launch_bounds__(256 * KS, 2) void product_kernel(const ProductParam
     for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  for (int t0 = 0; t0 < trips; t0 += kDeep) {
+  constexpr int kSub = kStep / 16;
+  constexpr int kEarly = W == 1 ? kSub : 1;   // fragments requested before the next step's tile is written: LDS answers in order
+  bf16x8 fa[kSub][W], fb[kSub][W];
+  unsigned char* now = buf;
+  auto request = [&](int s) {
 #pragma unroll
-    for (int u = 0; u < kDeep; ++u) {
-      const int t = t0 + u;
-      if (t < trips) {   // (uniform over the workgroup)
-        const int next = (u + 1) % kDeep;
-        unsigned char *now = buf + (t & 1) * S::kBuffer, *then = buf + (~t & 1) * S::kBuffer;
-        constexpr int kSub = kStep / 16;
-        constexpr int kEarly = W == 1 ? kSub : 1;   // fragments requested before the next step's tile is written: LDS answers in order
-        bf16x8 fa[kSub][W], fb[kSub][W];
-        auto request = [&](int s) {
+    for (int i = 0; i < W; ++i) {
+      fa[s][i] = A::fragment(now, wm + 32 * i, s, lane);
+      fb[s][i] = B::fragment(now + A::kBytes, wn + 32 * i, s, lane);
+    }
+  };
+  auto multiply = [&] {
 #pragma unroll
-          for (int i = 0; i < W; ++i) {
-            fa[s][i] = A::fragment(now, wm + 32 * i, s, lane);
-            fb[s][i] = B::fragment(now + A::kBytes, wn + 32 * i, s, lane);
-          }
-        };
+    for (int s = 0; s < kSub; ++s) {
+      if (s + kEarly < kSub) request(s + kEarly);
 #pragma unroll
-        for (int s = 0; s < kEarly; ++s) request(s);
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + 1 < trips) {
-          A::stage(then, tid, ra[next]);
-          B::stage(then + A::kBytes, tid, rb[next]);
-        }
-        if (t + kDeep < trips) {
-          a.load(k_first + (t + kDeep) * kStep, k_end, ra[u]);
-          b.load(k_first + (t + kDeep) * kStep, k_end, rb[u]);
-        }
+      for (int i = 0; i < W; ++i)
 #pragma unroll
-        for (int s = 0; s < kSub; ++s) {
-          if (s + kEarly < kSub) request(s + kEarly);
+        for (int j = 0; j < W; ++j) acc[i][j] = mfma32(fb[s][j], fa[s][i], acc[i][j]);   // C^T: a lane holds one row of C, its registers columns 8 q + 4 h ..+3
+    }
+  };
+  // Straight-line code with nothing but one exit: requests are not skipped towards the walk's end (past it they read no
+  // memory).  Skipped under a condition they would leave the compiler unsure how many are in flight, and it would wait for all
+  // of them in every step instead of for the oldest ([2331 x 1024]^T [2331 x 1024] 15.8 us, as it is 14.8; [512 x 3072] @ [3072
+  // x 576] 16.9, 14.4).
+  for (int t = 0;;) {
 #pragma unroll
-          for (int i = 0; i < W; ++i)
+    for (int u = 0; u < 2 * kDeep; ++u) {
+      const int next = (u + 1) % kDeep, here = u % kDeep;
+      now = buf + (u & 1) * S::kBuffer;
+      unsigned char* then = buf + (~u & 1) * S::kBuffer;
 #pragma unroll
-            for (int j = 0; j < W; ++j) acc[i][j] = mfma32(fb[s][j], fa[s][i], acc[i][j]);   // C^T: a lane holds one row of C, its registers columns 8 q + 4 h ..+3
-        }
-        __syncthreads();   // `now` may be filled again, `then` is complete
-      }
+      for (int s = 0; s < kEarly; ++s) request(s);
+      if (++t >= trips) goto last;   // (uniform over the workgroup)
+      __builtin_amdgcn_sched_barrier(0);
+      A::stage(then, tid, ra[next]);
+      B::stage(then + A::kBytes, tid, rb[next]);
+      a.load(k_first + (t + kDeep - 1) * kStep, k_end, ra[here]);
+      b.load(k_first + (t + kDeep - 1) * kStep, k_end, rb[here]);
+      multiply();
+      __syncthreads();   // `now` may be filled again, `then` is complete
     }
   }
+last:
+  multiply();
+  __syncthreads();
   if constexpr (KS > 1) {
     float* sums = reinterpret_cast<float*>(lds);
     auto place = [&](int w, int i, int j, int q) { return sums + ((((w * W + i) * W + j) * 4 + q) * kWave + lane) * 4; };
