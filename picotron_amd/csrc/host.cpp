@@ -1070,7 +1070,8 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
 Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64) {
   // (a backward that is itself to be differentiated, create_graph, stays with torch)
   const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
-  if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && !torch_gemm_only()) {
+  // (and torch refuses operands on two devices)
+  if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && a.device() == b.device() && !torch_gemm_only()) {
     const c10::OptionalDeviceGuard device(a.device());
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
     const int64_t M = kind == Product::TN ? a.size(1) : a.size(0), K = kind == Product::TN ? a.size(0) : a.size(1);
