@@ -334,6 +334,8 @@ int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int ds
  * fp32 sums are added in a fixed order.  N, the pitches and the contiguous axis of a and b must be multiples of 8, pointers
  * 16-byte aligned.  Counterpart of torch's F.linear and its gradients in the reference (model.py:105-108,183-184).
  */
+/* 1 where pico_product takes operands of these sizes and row pitches, 0 where it refuses them. */
+int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow);
 int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
                  int tile, int groups, void* stream);
 

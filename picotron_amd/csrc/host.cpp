@@ -1014,7 +1014,7 @@ int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
 int64_t turned_operand(Product kind, const Tensor& a, const Tensor& b) {
   if (kind != Product::TN) return 0;
   const int64_t K = a.size(0), M = a.size(1), N = b.size(1), narrow = std::min(M, N), wide = std::max(M, N);
-  if (narrow % 8 || (K < 1024 && (K < 512 || narrow >= 1024))) return 0;
+  if (narrow % 8 || (M < N ? a : b).stride(0) % 8 || (K < 1024 && (K < 512 || narrow >= 1024))) return 0;
   if (wide <= 5000 + 1e10 / (static_cast<double>(K) * narrow)) return 0;
   return M < N ? 1 : 2;
 }
@@ -1066,20 +1066,38 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
   return K <= (tiles > 128 ? 3072 : tiles > 60 ? 1088 : 0) ? OwnProduct{2, 64} : no;
 }
 
-// parts 0, turn -1, groups -1: by the rules above
-Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64) {
+struct ProductSizes {
+  int64_t M, N, K;
+};
+ProductSizes product_sizes(const Tensor& a, const Tensor& b, Product kind) {
+  const ProductSizes n = {kind == Product::TN ? a.size(1) : a.size(0), kind == Product::NT ? b.size(0) : b.size(1),
+                          kind == Product::TN ? a.size(0) : a.size(1)};
+  TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == n.K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
+  return n;
+}
+// What torch would do differently, or refuse (operands on two devices), stays with torch.
+bool stays_with_torch(const Tensor& a, const Tensor& b) {
   // (a backward that is itself to be differentiated, create_graph, stays with torch)
   const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
-  // (and torch refuses operands on two devices)
-  if (!recorded && ordinary({&a, &b}) && plain(a) && plain(b) && a.device() == b.device() && !torch_gemm_only()) {
+  return recorded || !ordinary({&a, &b}) || !plain(a) || !plain(b) || a.device() != b.device() || torch_gemm_only();
+}
+// own_product's choice where the kernel takes the operands as they lie in memory; the library takes any row pitch
+OwnProduct own_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b) {
+  const OwnProduct own = own_product(kind, n.M, n.N, n.K);
+  if (own.groups > 0 && !pico_product_takes(n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT)) return {0, 64};
+  return own;
+}
+
+// parts 0, turn -1, groups -1: by the rules above
+Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64) {
+  if (!stays_with_torch(a, b)) {
     const c10::OptionalDeviceGuard device(a.device());
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
-    const int64_t M = kind == Product::TN ? a.size(1) : a.size(0), K = kind == Product::TN ? a.size(0) : a.size(1);
-    const int64_t N = kind == Product::NT ? b.size(0) : b.size(1);
-    TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
+    const ProductSizes n = product_sizes(a, b, kind);
+    const auto [M, N, K] = n;
     Tensor c = at::empty({M, N}, a.options());
     if (groups < 0) {
-      const OwnProduct own = parts == 0 && turn < 0 ? own_product(kind, M, N, K) : OwnProduct{0, 64};
+      const OwnProduct own = parts == 0 && turn < 0 ? own_product(kind, n, a, b) : OwnProduct{0, 64};
       groups = own.groups;
       tile = own.tile;
     }
@@ -1105,6 +1123,13 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
     if (gemm_plans().run(s, bt.data_ptr(), at_.data_ptr(), c.data_ptr(), a.options())) return c;
   }
   return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
+}
+
+// the route of a product, for tests: "torch", "own" or "library", "turned" where the library's product has an operand transposed first
+std::string product_route(const Tensor& a, const Tensor& b, Product kind) {
+  if (stays_with_torch(a, b)) return "torch";
+  if (own_product(kind, product_sizes(a, b, kind), a, b).groups > 0) return "own";
+  return turned_operand(kind, a, b) ? "turned" : "library";
 }
 
 Tensor linear_forward(const Tensor& x, const Tensor& w) {
@@ -1510,9 +1535,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("publish_kv", &publish_kv);
   m.def("ring_node", &ring_node);
   m.def("flash_attention", &flash_attention, nogil());
-  m.def("product", [](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile) {
+  const auto product_kind = [](const std::string& kind) {
     TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
-    return product(a, b, kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN, parts, turn, groups, tile);
+    return kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN;
+  };
+  m.def("product_route", [=](const Tensor& a, const Tensor& b, const std::string& kind) { return product_route(a, b, product_kind(kind)); },
+        pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"));
+  m.def("product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile) {
+    return product(a, b, product_kind(kind), parts, turn, groups, tile);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
         pybind11::arg("groups") = -1, pybind11::arg("tile") = 64);
   m.def("linear", &linear, nogil());

@@ -246,22 +246,27 @@ int launch_shape(const ProductParams& p, int tile, int groups, hipStream_t s) {
 
 using namespace pico;
 
-extern "C" int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow,
-                            int b_slow, int tile, int groups, void* stream) {
+extern "C" int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow) {
   constexpr int64_t kMost = 0x7fffffff;
   if (M < 1 || N < 1 || K < 1 || M > kMost || N > kMost || K > kMost - 4096 || N % 8 != 0 || (a_slow ? M : K) % 8 != 0 ||
       (b_slow ? N : K) % 8 != 0 || lda % 8 != 0 || ldb % 8 != 0 || lda < (a_slow ? M : K) || ldb < (b_slow ? N : K))
-    return fail(PICO_ERR_SHAPE, "pico_product: M=%lld N=%lld K=%lld row pitches %lld, %lld (rows of a, b and c must be multiples of 8 elements)",
-                (long long)M, (long long)N, (long long)K, (long long)lda, (long long)ldb);
+    return 0;
   // the windows of the buffer loads: a tile's rows, or the whole contraction where that is the slow axis
   if (lda > kMost / 2 || ldb > kMost / 2 || ((a_slow ? K + 1024 : 128) * lda + K) * 2 > kMost || ((b_slow ? K + 1024 : 128) * ldb + K) * 2 > kMost)
-    return fail(PICO_ERR_SHAPE, "pico_product: an operand is too large");
+    return 0;
+  return ((M + 63) / 64) * ((N + 63) / 64) <= kMost;
+}
+
+extern "C" int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow,
+                            int b_slow, int tile, int groups, void* stream) {
+  if (!pico_product_takes(M, N, K, lda, ldb, a_slow, b_slow))
+    return fail(PICO_ERR_SHAPE, "pico_product: M=%lld N=%lld K=%lld row pitches %lld, %lld (rows of a, b and c and the pitches must be multiples of 8 elements, a tile's rows span less than 2 GiB)",
+                (long long)M, (long long)N, (long long)K, (long long)lda, (long long)ldb);
   if (!(tile == 64 && (groups == 1 || groups == 2 || groups == 4)) && !(tile == 128 && (groups == 1 || groups == 2)))
     return fail(PICO_ERR_SHAPE, "pico_product: tile=%d groups=%d (64 with 1, 2 or 4 groups, 128 with 1 or 2)", tile, groups);
   if (!a || !b || !c) return fail(PICO_ERR_NULL, "pico_product: a, b and c are required");
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return fail(PICO_ERR_ALIGN, "pico_product: pointers must be 16-byte aligned");
   const int64_t tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
-  if (tm * tn > kMost) return fail(PICO_ERR_SHAPE, "pico_product: too many tiles");
   const ProductParams p = {static_cast<const __bf16*>(a), static_cast<const __bf16*>(b), static_cast<__bf16*>(c), (int)M, (int)N, (int)K, lda, ldb, (int)tm, (int)tn};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a_slow) return b_slow ? launch_shape<true, true>(p, tile, groups, s) : launch_shape<true, false>(p, tile, groups, s);

@@ -109,3 +109,21 @@ def test_small_products(device, kind, M, N, K):
     exact = _lib.host().product(a.round(), b.round(), kind, groups=4)     # small integers: sums are exact in fp32
     want = (a.round().float().t() if kind == "TN" else a.round().float()) @ (b.round().float().t() if kind == "NT" else b.round().float())
     assert torch.equal(exact, want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("pad", [1, 4, 8])
+@pytest.mark.parametrize("rows,cin,cout", [(512, 576, 576), (300, 520, 1536), (1024, 1024, 32000)])
+def test_linear_on_columns_of_a_wider_buffer(device, rows, cin, cout, pad):
+    """Rows that lie `pad` elements further apart than they are long, where the dense sizes go to the package's kernel (and,
+    for the last shape's weight gradient, to the library with a transposed operand)."""
+    from picotron_amd.model import Linear
+    g = torch.Generator(device="cuda").manual_seed(rows + pad)
+    layer = Linear(cin, cout, bias=False, device=device, dtype=torch.bfloat16)
+    x = torch.randn(rows, cin + pad, generator=g, device=device).to(torch.bfloat16)[:, :cin].requires_grad_()
+    dy = torch.randn(rows, cout + pad, generator=g, device=device).to(torch.bfloat16)[:, :cout]
+    y = layer(x)
+    got = (y, *torch.autograd.grad(y, (x, layer.weight), dy))
+    xf, wf = x.detach().float().requires_grad_(), layer.weight.detach().float().requires_grad_()
+    yf = torch.nn.functional.linear(xf, wf)
+    for a, b in zip(got, (yf, *torch.autograd.grad(yf, (xf, wf), dy.float()))):
+        assert a.shape == b.shape and ((a.float() - b).norm() / b.norm()).item() <= 3e-3

@@ -67,3 +67,39 @@ for rows, wide in ((512, 576), (4096, 2048)):
                  message(host.product, dy, w, "NN"), message(host.product, operand(rows, wide, device=1), x, "TN")):
         assert "same device" in what, what
 ''')
+
+
+def test_the_predicate_is_what_the_kernel_refuses():
+    """pico_product_takes against pico_product itself: with NULL operands an accepted shape ends at the pointers (-1)."""
+    from picotron_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    lib, seen = _lib.lib(), set()
+    for M, N, K in ((1, 8, 8), (512, 576, 576), (512, 576, 580), (516, 576, 576), (512, 580, 576), (2331, 1024, 2331)):
+        for a_slow in (0, 1):
+            for b_slow in (0, 1):
+                for pad_a in (0, 4, 8, -8, 1 << 23, 1 << 31):
+                    for pad_b in (0, 4, 8, 1 << 23):
+                        lda, ldb = (M if a_slow else K) + pad_a, (N if b_slow else K) + pad_b
+                        takes = lib.pico_product_takes(M, N, K, lda, ldb, a_slow, b_slow)
+                        rc = lib.pico_product(None, None, None, M, N, K, lda, ldb, a_slow, b_slow, 64, 1, None)
+                        assert rc == (-1 if takes else -3), (M, N, K, lda, ldb, a_slow, b_slow)
+                        seen.add(takes)
+    assert seen == {0, 1}
+
+
+def test_row_pitches_the_kernels_refuse_go_to_the_library():
+    """The sizes route to the package's kernels; the pitch (no multiple of 8, or rows too far apart) sends them past."""
+    run('''
+for kind, M, N, K, want in (("NT", 512, 576, 576, "own"), ("NN", 512, 1024, 1024, "own"), ("TN", 576, 960, 512, "own"),
+                            ("TN", 49152, 2048, 4096, "turned"), ("TN", 2048, 49152, 4096, "turned")):
+    (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    for pad_a, pad_b in ((0, 0), (8, 0), (0, 24), (4, 0), (0, 4), (1, 1), (4, 24), (0, 1 << 24), (1 << 24, 0)):
+        got = host.product_route(operand(ra, ca, ca + pad_a), operand(rb, cb, cb + pad_b), kind)
+        if want == "own":
+            fits = pad_a % 8 == 0 and pad_b % 8 == 0 and max(pad_a, pad_b) < 1 << 24
+        else:                                     # only the operand that is transposed, the narrower one, has to fit
+            fits = (pad_a if M < N else pad_b) % 8 == 0
+        assert got == (want if fits else "library"), (kind, M, N, K, pad_a, pad_b, got)
+    assert host.product_route(operand(ra, ca, address=(1 << 20) + 2), operand(rb, cb), kind) == "torch"
+''')
