@@ -140,7 +140,8 @@ __global__ __launch_bounds__(kThreads) void ce_bwd_kernel(const T* __restrict__ 
 // ---- forward and backward in one pass over the logits.  Bound by HBM: the row (96 KiB at vocab 49152 in bf16) is read
 // once into registers, 16 bytes per lane and piece, reduced, turned into its gradient and written: 2 x rows x vocab
 // elements of traffic where forward and backward apart move 3 x.  NT threads hold NV pieces each; with at most 8 pieces
-// (32 registers, 64 in all) two 1024-thread workgroups share a CU and one reads while the other writes.  Measured, forward
+// (32 registers for the row, 64 in all, none in scratch) two 1024-thread workgroups share a CU and one reads while the other
+// writes.  Measured, forward
 // + backward through autograd, against the two streaming kernels and torch's reductions between them: [4096, 49152] bf16
 // 232 -> 146 us (5.5 TB/s), [4096, 49152] fp32 414 -> 301, [16384, 2000] bf16 63 -> 40 (kernels alone).
 template <typename T>
@@ -218,11 +219,16 @@ __global__ __launch_bounds__(NT, NV <= 8 ? 8 : 4) void ce_one_pass_kernel(const 
   const int wave = threadIdx.x / kWave;
   if (threadIdx.x % kWave == 0) { red_m[wave] = wm; red_s[wave] = s; }
   __syncthreads();
-  float bm = red_m[0], bs = 0.f;
+  // one wave's share per lane, reduced by exchanges: read whole by every lane the shares take 2 W registers beside the row,
+  // and rows of eight pieces went to scratch ([4096, 32000] bf16 forward + backward 110 -> 103 us, [2048, 65536] 114 -> 105,
+  // [8192, 20000] 139 -> 132, fp32 the same)
+  const float pm = red_m[threadIdx.x % W];
+  float bm = pm;
 #pragma unroll
-  for (int w = 1; w < W; ++w) bm = fmaxf(bm, red_m[w]);
+  for (int off = W / 2; off > 0; off >>= 1) bm = fmaxf(bm, __shfl_xor(bm, off, kWave));
+  float bs = pm == -INFINITY ? 0.f : red_s[threadIdx.x % W] * fast_exp2(pm - bm);
 #pragma unroll
-  for (int w = 0; w < W; ++w) bs += red_m[w] == -INFINITY ? 0.f : red_s[w] * fast_exp2(red_m[w] - bm);
+  for (int off = W / 2; off > 0; off >>= 1) bs += __shfl_xor(bs, off, kWave);
   const float l2 = bm + fast_log2(bs);
   if (threadIdx.x == 0) {
     const float lse = l2 * kLn2;
