@@ -381,12 +381,18 @@ int pico_cross_entropy_bwd(const void* logits, const int64_t* targets, const flo
  * entries, fp32 of up to 65536) the gradient for an upstream gradient of 1 is written in the same pass, the logits are
  * read once, and a row that does not count gets lse = 0.  Backward: dlogits of the upstream gradient grad_out[0] (device
  * float); with have_unit != 0 dlogits holds the forward's gradient already and is left as it is where grad_out[0] is 1
- * (decided on the device, no synchronisation) and recomputed from the logits otherwise.
+ * (decided on the device, no synchronisation) and recomputed from the logits otherwise: forward and backward then make four
+ * passes over the logits' size instead of two, where forward and backward apart make three.  A loss that will be divided by a
+ * number of accumulation steps (train.py:29-55) is therefore asked for as pico_cross_entropy_scaled_mean_fwd with scale = 1 /
+ * steps: mean[0] and inv_count[0] carry the factor, the upstream gradient stays 1, and _mean_bwd is called as before.
  */
 int pico_cross_entropy_one_pass(int64_t vocab, int dtype);
 int pico_cross_entropy_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
                                 float* inv_count, void* dlogits, int64_t rows, int64_t vocab, int64_t ld, int64_t dld,
                                 int64_t ignore_index, int dtype, void* stream);
+int pico_cross_entropy_scaled_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
+                                       float* inv_count, void* dlogits, float scale, int64_t rows, int64_t vocab, int64_t ld,
+                                       int64_t dld, int64_t ignore_index, int dtype, void* stream);
 int pico_cross_entropy_mean_bwd(const void* logits, const int64_t* targets, const float* lse, const float* inv_count,
                                 const float* grad_out, void* dlogits, int have_unit, int64_t rows, int64_t vocab, int64_t ld,
                                 int64_t dld, int64_t ignore_index, int dtype, void* stream);

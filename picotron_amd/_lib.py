@@ -75,6 +75,7 @@ SIGNATURES = {
     "pico_cross_entropy_bwd": (c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, _P]),
     "pico_cross_entropy_one_pass": (c_int, [_I64, c_int]),
     "pico_cross_entropy_mean_fwd": (c_int, [_P] * 7 + [_I64] * 5 + [c_int, _P]),
+    "pico_cross_entropy_scaled_mean_fwd": (c_int, [_P] * 7 + [c_float] + [_I64] * 5 + [c_int, _P]),
     "pico_cross_entropy_mean_bwd": (c_int, [_P] * 6 + [c_int] + [_I64] * 5 + [c_int, _P]),
     "pico_adamw": (c_int, [_P, _P, _P, c_int, _P, _P, _I64] + [ctypes.c_float] * 5 + [_I64, ctypes.c_float, _P]),
     "pico_adamw_lp": (c_int, [_P, _P, c_int, _P, _P, _I64, c_int, c_int] + [ctypes.c_float] * 5 + [_I64, ctypes.c_float, _P]),

@@ -1379,11 +1379,12 @@ Tensor cross_entropy_bwd(const Tensor& logits, const Tensor& targets, const Tens
 // Mean cross-entropy of [rows, vocab] logits against int64 targets (train.py:46-49), fp32 loss.  Where a gradient will be
 // wanted and the row fits (pico_cross_entropy_one_pass) the forward writes the gradient for a unit upstream gradient while
 // it holds the row: forward and backward then read the logits once.  The backward hands that buffer over; the kernel it
-// launches looks at the upstream gradient on the device and recomputes only if it is not 1.
+// launches looks at the upstream gradient on the device and recomputes only if it is not 1.  `scale` is a factor of the loss
+// that the caller knows beforehand (1 / accumulation steps): part of the loss and of the gradient written in the forward.
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, int64_t ignore_index) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, int64_t ignore_index, double scale) {
     Tensor unit;
-    const auto [mean, lse, inv_count] = run(logits, targets, ignore_index, &unit);
+    const auto [mean, lse, inv_count] = run(logits, targets, ignore_index, scale, &unit);
     ctx->save_for_backward({logits, targets, lse, inv_count, unit});
     ctx->saved_data["ignore"] = ignore_index;
     ctx->saved_data["spent"] = false;
@@ -1400,27 +1401,27 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
     check(pico_cross_entropy_mean_bwd(ptr(logits), targets.data_ptr<int64_t>(), fptr(lse), fptr(inv_count), fptr(up), ptr(d), have_unit,
                                       logits.size(0), logits.size(1), pitch_of(logits), pitch_of(d), ctx->saved_data["ignore"].toInt(),
                                       dtype_code(logits, "logits"), stream_now()));
-    return {d, Tensor(), Tensor()};
+    return {d, Tensor(), Tensor(), Tensor()};
   }
   // same row pitch as the logits (a view into a padded buffer keeps its 16-byte-aligned rows)
   static Tensor empty_like_rows(const Tensor& logits) { return at::empty_strided(logits.sizes(), logits.strides(), logits.options()); }
-  static std::tuple<Tensor, Tensor, Tensor> run(const Tensor& logits, const Tensor& targets, int64_t ignore_index, Tensor* unit) {
+  static std::tuple<Tensor, Tensor, Tensor> run(const Tensor& logits, const Tensor& targets, int64_t ignore_index, double scale, Tensor* unit) {
     check_loss(logits, targets);
     const int64_t rows = logits.size(0), vocab = logits.size(1);
     const int dt = dtype_code(logits, "logits");
     const auto f32 = logits.options().dtype(at::kFloat);
     const Tensor loss = at::empty({rows}, f32), lse = at::empty({rows}, f32), mean = at::empty({}, f32), inv_count = at::empty({}, f32);
     if (unit && rows > 0 && pico_cross_entropy_one_pass(vocab, dt)) *unit = empty_like_rows(logits);
-    check(pico_cross_entropy_mean_fwd(ptr(logits), targets.data_ptr<int64_t>(), fptr(loss), fptr(lse), fptr(mean), fptr(inv_count),
-                                      unit ? ptr(*unit) : nullptr, rows, vocab, pitch_of(logits),
-                                      unit && unit->defined() ? pitch_of(*unit) : 0, ignore_index, dt, stream_now()));
+    check(pico_cross_entropy_scaled_mean_fwd(ptr(logits), targets.data_ptr<int64_t>(), fptr(loss), fptr(lse), fptr(mean), fptr(inv_count),
+                                             unit ? ptr(*unit) : nullptr, static_cast<float>(scale), rows, vocab, pitch_of(logits),
+                                             unit && unit->defined() ? pitch_of(*unit) : 0, ignore_index, dt, stream_now()));
     return {mean, lse, inv_count};
   }
 };
 
-Tensor cross_entropy(const Tensor& logits, const Tensor& targets, int64_t ignore_index) {
-  if (!records({&logits})) return std::get<0>(CrossEntropy::run(logits, targets, ignore_index, nullptr));
-  return CrossEntropy::apply(logits, targets, ignore_index);
+Tensor cross_entropy(const Tensor& logits, const Tensor& targets, int64_t ignore_index, double scale) {
+  if (!records({&logits})) return std::get<0>(CrossEntropy::run(logits, targets, ignore_index, scale, nullptr));
+  return CrossEntropy::apply(logits, targets, ignore_index, scale);
 }
 
 // ------------------------------------------------------------------------------------------------ AdamW
@@ -1549,7 +1550,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_linear", &fused_linear, nogil());
   m.def("embedding", &embedding, nogil());
   m.def("qkv_attention", &qkv_attention, nogil());
-  m.def("cross_entropy", &cross_entropy, nogil());
+  m.def("cross_entropy", &cross_entropy, pybind11::arg("logits"), pybind11::arg("targets"), pybind11::arg("ignore_index"),
+        pybind11::arg("scale") = 1.0, nogil());
   m.def("cross_entropy_fwd", &cross_entropy_fwd, nogil());
   m.def("cross_entropy_bwd", &cross_entropy_bwd, nogil());
   m.def("zero_grads", &zero_grads);

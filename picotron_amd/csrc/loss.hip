@@ -258,13 +258,13 @@ __global__ __launch_bounds__(NT, NV <= 8 ? 8 : 4) void ce_one_pass_kernel(const 
   if (tail < vocab) d[tail] = static_cast<T>((fast_exp2(xe * kLog2e - l2) - (tail == t ? 1.f : 0.f)) * scale);
 }
 
-// inv_count = 1 / max(rows that count, 1) and, with `loss`, mean = sum(loss) / count: one workgroup, a fixed order of
-// summation.  (A few microseconds of launch and latency; the eight elementwise and reduction launches torch needs for
+// inv_count = scale / max(rows that count, 1) and, with `loss`, mean = scale * sum(loss) / count: one workgroup, a fixed order
+// of summation.  (A few microseconds of launch and latency; the eight elementwise and reduction launches torch needs for
 // the same took 30.)
 constexpr int kMeanThreads = 1024;
 __global__ __launch_bounds__(kMeanThreads) void ce_mean_kernel(const float* __restrict__ loss, const int64_t* __restrict__ targets,
-                                                               float* __restrict__ mean, float* __restrict__ inv_count, int64_t rows,
-                                                               int64_t vocab, int64_t ignore_index) {
+                                                               float* __restrict__ mean, float* __restrict__ inv_count, float scale,
+                                                               int64_t rows, int64_t vocab, int64_t ignore_index) {
   __shared__ float red_s[kMeanThreads / kWave];
   __shared__ int red_n[kMeanThreads / kWave];
   float s = 0.f;
@@ -284,8 +284,8 @@ __global__ __launch_bounds__(kMeanThreads) void ce_mean_kernel(const float* __re
     int count = 0;
     for (int w = 0; w < kMeanThreads / kWave; ++w) { total += red_s[w]; count += red_n[w]; }
     const float c = static_cast<float>(count > 0 ? count : 1);
-    *inv_count = 1.f / c;
-    if (loss != nullptr) *mean = total / c;
+    *inv_count = scale / c;
+    if (loss != nullptr) *mean = total / c * scale;
   }
 }
 
@@ -379,23 +379,23 @@ extern "C" int pico_cross_entropy_one_pass(int64_t vocab, int dtype) {
   return (dtype == PICO_BF16 || dtype == PICO_F32) && vocab > 0 && one_pass_fits(vocab, dtype);
 }
 
-extern "C" int pico_cross_entropy_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
-                                           float* inv_count, void* dlogits, int64_t rows, int64_t vocab, int64_t ld, int64_t dld,
-                                           int64_t ignore_index, int dtype, void* stream) {
-  const char* fn = "pico_cross_entropy_mean_fwd";
+namespace {
+int run_mean_fwd(const char* fn, const void* logits, const int64_t* targets, float* loss, float* lse, float* mean, float* inv_count,
+                 void* dlogits, float scale, int64_t rows, int64_t vocab, int64_t ld, int64_t dld, int64_t ignore_index, int dtype,
+                 void* stream) {
   if (int rc = check_ce(fn, rows, vocab, ld, dtype)) return rc;
   if (!mean || !inv_count) return fail(PICO_ERR_NULL, "%s: mean and inv_count are required", fn);
   if (rows > 0 && (!logits || !targets || !loss || !lse)) return fail(PICO_ERR_NULL, "%s: logits, targets, loss and lse are required", fn);
   if (!aligned16(logits) || !aligned16(dlogits)) return fail(PICO_ERR_ALIGN, "%s: logits and dlogits must be 16-byte aligned", fn);
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto finish = [&](const float* l) {
-    hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(kMeanThreads), 0, s, l, targets, mean, inv_count, rows, vocab, ignore_index);
+    hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(kMeanThreads), 0, s, l, targets, mean, inv_count, scale, rows, vocab, ignore_index);
   };
   if (dlogits != nullptr && rows > 0) {
     if (int rc = check_ce(fn, rows, vocab, dld, dtype)) return rc;
     if (!one_pass_fits(vocab, dtype))
       return fail(PICO_ERR_SHAPE, "%s: vocab=%lld does not fit one pass (see pico_cross_entropy_one_pass)", fn, static_cast<long long>(vocab));
-    finish(nullptr);   // the gradient needs 1 / count
+    finish(nullptr);   // the gradient needs scale / count
     if (dtype == PICO_BF16)
       launch_one_pass<__bf16, true>(logits, targets, loss, lse, inv_count, dlogits, rows, static_cast<int>(vocab), ld, dld, ignore_index, s);
     else
@@ -405,6 +405,22 @@ extern "C" int pico_cross_entropy_mean_fwd(const void* logits, const int64_t* ta
   }
   finish(loss != nullptr ? loss : lse);   // (no rows: nothing is read, the mean is 0)
   return check_launch(fn);
+}
+
+}  // namespace
+
+extern "C" int pico_cross_entropy_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
+                                           float* inv_count, void* dlogits, int64_t rows, int64_t vocab, int64_t ld, int64_t dld,
+                                           int64_t ignore_index, int dtype, void* stream) {
+  return run_mean_fwd("pico_cross_entropy_mean_fwd", logits, targets, loss, lse, mean, inv_count, dlogits, 1.f, rows, vocab, ld, dld,
+                      ignore_index, dtype, stream);
+}
+
+extern "C" int pico_cross_entropy_scaled_mean_fwd(const void* logits, const int64_t* targets, float* loss, float* lse, float* mean,
+                                                  float* inv_count, void* dlogits, float scale, int64_t rows, int64_t vocab, int64_t ld,
+                                                  int64_t dld, int64_t ignore_index, int dtype, void* stream) {
+  return run_mean_fwd("pico_cross_entropy_scaled_mean_fwd", logits, targets, loss, lse, mean, inv_count, dlogits, scale, rows, vocab, ld,
+                      dld, ignore_index, dtype, stream);
 }
 
 extern "C" int pico_cross_entropy_mean_bwd(const void* logits, const int64_t* targets, const float* lse, const float* inv_count,

@@ -38,3 +38,31 @@ def test_one_pass_rows_at_the_edges(device, dtype, pieces, extra):
         assert got[2].abs().max().item() == 0.0
     (got,) = torch.autograd.grad(cross_entropy(x, t), x, torch.full_like(loss, -3.0))
     assert rel(got, gw * -3.0) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1003, 32000, 49152, 8 * 1024 * 17])   # (the last: two passes)
+def test_a_factor_of_the_loss(device, dtype, vocab):
+    """`scale` is part of the loss and of its gradient: as the division behind the loss, with an upstream gradient of 1 (the
+    forward's own gradient, the same buffer) and of something else, without a gradient, and with nothing to average."""
+    from picotron_amd.functional import cross_entropy
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    x = torch.zeros(6, (vocab + 7) // 8 * 8, dtype=dtype, device=device)[:, :vocab]
+    x.copy_(torch.randn(6, vocab, generator=g, device=device) * 3).requires_grad_()
+    t = torch.randint(0, vocab, (6,), generator=g, device=device)
+    t[2] = -100
+    xd = x.detach().double().requires_grad_()
+    want = torch.nn.functional.cross_entropy(xd, t)
+    (gw,) = torch.autograd.grad(want, xd)
+    tol = 4e-3 if dtype == torch.bfloat16 else 1e-5                     # one rounding to the logits' type
+    for scale in (1.0, 0.25, 1 / 3, 128.0):
+        loss = cross_entropy(x, t, scale=scale)
+        assert abs(loss.item() - scale * want.item()) <= 2e-5 * abs(scale * want.item())
+        for up in (1.0, 0.37):
+            (got,) = torch.autograd.grad(loss, x, torch.full_like(loss, up), retain_graph=True)
+            assert rel(got, gw * scale * up) <= tol, (scale, up)
+        with torch.no_grad():
+            assert abs(cross_entropy(x, t, scale=scale).item() - loss.item()) <= 2e-5 * abs(loss.item())
+    (one,), (div,) = (torch.autograd.grad(l, x) for l in (cross_entropy(x, t, scale=0.25), cross_entropy(x, t) / 4))
+    assert rel(one, div.double()) <= tol
+    assert cross_entropy(x, torch.full_like(t, -100), scale=0.5).item() == 0.0
