@@ -79,6 +79,8 @@ struct KvCfg {
   // PAIR: the K and V fragments of the four key waves stay in LDS behind the tile buffers instead of in registers
   static constexpr size_t kKvBytes = PAIR ? static_cast<size_t>(kKeyWaves) * 2 * WaveTile<D>::kRegionBytes : 0;
   static constexpr size_t kLdsBytes = kTileBytes + kKvBytes;
+  static constexpr int kPerCu = PAIR ? 1 : 2;         // workgroups that share a CU
+  static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   static_assert(NW * kRowRegionBytes <= kTileBytes, "the epilogue reuses the tile buffers");
   static_assert(PAIR || NW * WaveTile<D>::kRegionBytes <= kBufBytes, "the K / V fragments pass through the second tile buffer");
   // PAIR: one accumulator set (D/32 x 16 registers x 64 lanes of fp32) per key wave passes through LDS at a time
@@ -687,11 +689,16 @@ struct DqCfg {
   static constexpr int BM = 32 * kQWaves;  // queries per workgroup (32 per query wave)
   static_assert(NW % KS == 0 && (KS == 1 || KT == 64 * KS), "one 64-key step of every staged tile per key-split wave");
   static constexpr int BN = 64;            // keys per compute step
+  static constexpr int kKT = KT;
   static constexpr int LDK = D + 8;        // pitch of the K and V tiles
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;
   static constexpr int kTileElems = 2 * KT * LDK;
   static constexpr size_t kLdsBytes = 2 * kTileElems * sizeof(__bf16);  // double-buffered
+  // workgroups that share a CU: the register budget and the plan go by it (at head_dim 128 a lane needs more than the 256
+  // registers that two would leave it: with some in scratch 77 -> 121 us at one head of 3000 rows)
+  static constexpr int kPerCu = NW <= 4 && D <= 64 ? 2 : 1;
+  static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   static_assert(NW * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
   static_assert(NW * WaveTile<D>::kRegionBytes <= kLdsBytes, "the Q / dO fragments pass through the tile buffers");
   static_assert(KT % BN == 0 && (KT * kVecPerRow) % kThreads == 0, "tile must split evenly over the threads");
@@ -715,9 +722,8 @@ __device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* regi
     wave_store_rows<D, false>(region, dq, a.sm_scale, static_cast<__bf16*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, false, kStreamGrads);
 }
 
-// (small workgroups are built for two of them per CU: at most 256 registers per lane)
 template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
-__global__ __launch_bounds__(64 * NW, (NW <= 4 && D <= 64) ? 2 : 1) void attn_bwd_dq_kernel(const BwdParams p) {
+__global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) void attn_bwd_dq_kernel(const BwdParams p) {
   using C = DqCfg<D, NW, KT, KS>;
   constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -1042,8 +1048,8 @@ DkdvPlan make_dkdv_plan(const AttnParams& a) {
   // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
   // are up to 30 % faster)
   plan.pair = a.causal && n_ktiles >= 2 && heads * ((n_ktiles + 1) / 2) >= (D == 64 ? 384 : 256);
-  TripCost cost = {1.1, 1.0, 2, 0.0};
-  if (D == 128) cost = {1.65, 2.05, 1, 0.0};
+  TripCost cost = {1.1, 1.0, C::kPerCu, 0.0};
+  if (D == 128) cost = {1.65, 2.05, C::kPerCu, 0.0};
   cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
   auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
   plan.len = choose_pieces(heads, n_ktiles, cost, plan.pair, trips_of);
@@ -1113,8 +1119,14 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
   DqPlan plan;
   const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
-  TripCost cost = {1.65, 1.8, 2, 0.0};
+  TripCost cost;
   int bm = 128, kt = 64;
+  auto use = [&](auto cfg, double alone_us, double full_us) {
+    using C = decltype(cfg);
+    bm = C::BM;
+    kt = C::kKT;
+    cost = {alone_us, full_us, C::kPerCu, 0.0};
+  };
   if (D == 64) {
     const int64_t visible_keys = a.causal ? std::min<int64_t>(a.Sk, static_cast<int64_t>(a.q_offset) + a.Sq) : a.Sk;
     // the forward's rules: eight waves per workgroup also for rectangular launches (every query sees at least as many
@@ -1130,16 +1142,16 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     // few waves in all: two waves per 32 queries, 64 keys of every 128 each (rank 3 of 4 at configs[1] with eight waves
     // per workgroup: 18.8 -> 17.9 us)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
-    bm = plan.kernel == DqPlan::kWaves8 ? 256 : plan.kernel == DqPlan::kSplit4 ? 64 : 128;
-    kt = plan.kernel >= DqPlan::kSplit4 ? 128 : 64;
-    cost = plan.kernel == DqPlan::kWaves8 ? TripCost{1.7, 1.5, 1, 0.0} : plan.kernel == DqPlan::kWaves4 ? TripCost{1.3, 0.78, 2, 0.0}
-         : plan.kernel == DqPlan::kSplit8 ? TripCost{1.6, 1.5, 1, 0.0} : TripCost{1.25, 0.8, 2, 0.0};
+    switch (plan.kernel) {
+      case DqPlan::kWaves8: use(DqCfg<64, 8, 64>(), 1.7, 1.5); break;
+      case DqPlan::kWaves4: use(DqCfg<64, 4, 64>(), 1.3, 0.78); break;
+      case DqPlan::kSplit8: use(DqCfg<64, 8, 128, 2>(), 1.6, 1.5); break;
+      case DqPlan::kSplit4: use(DqCfg<64, 4, 128, 2>(), 1.25, 0.8); break;
+    }
   } else {
     plan.kernel = groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
-    if (plan.kernel == DqPlan::kWaves8) {
-      bm = 256;
-      cost = {2.0, 2.87, 1, 0.0};
-    }
+    if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 2.0, 2.87);
+    else use(DqCfg<128, 4, 64>(), 1.65, 1.8);
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);

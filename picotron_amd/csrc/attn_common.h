@@ -373,7 +373,8 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
 }
 
 // Host: the piece length for a launch, from what its workgroups cost.  A trip takes `alone_us` in a workgroup that has its
-// CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each; `fixed_us` is a workgroup's start and end.
+// CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each: as many as its registers and LDS are
+// budgeted for.
 // (Fitted to launches from 1 to 300 heads and 200 to 8000 rows; over 27 such shapes the piece lengths chosen ran within
 // 0.7 % of the best ones in the geometric mean, 5 % at worst.)
 struct TripCost {

@@ -48,6 +48,12 @@ struct FwdCfg {
   static constexpr int kTileElems = KT * (LDK + LDV);
   static constexpr size_t kLdsBytes = 2 * kTileElems * sizeof(__bf16);
   static_assert(NW * QB * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
+  // workgroups that share a CU: eight waves at head_dim 128 and with split keys have it to themselves.  The kernel's register
+  // budget is this number's, and the plan counts on it.  (Left to the whole file, four waves at head_dim 128 took 290 and one
+  // workgroup fitted: B1 H20 S3000 100 -> 68 us with the budget, 0.84 in the geometric mean of 93 drawn launches; at head_dim
+  // 64 accumulators no longer move between the two halves of the file, 0.88 of 107.)
+  static constexpr int kPerCu = NW == 8 && (D >= 128 || KS > 1) ? 1 : 2;
+  static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   // exchange of partial states between key-split waves: per wave O^T accumulators (D/32 x 16 registers x 64 lanes) + m + l
   static constexpr size_t kExchangeBytes = (D / 32) * 16 * 64 * 4 + 2 * 64 * 4;
   static_assert(KS == 1 || NW * kExchangeBytes <= kLdsBytes, "the exchange reuses the tile buffers");
@@ -83,7 +89,7 @@ __device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* 
 // kCut: tiles may be cut into pieces (see Pieces) and chunks may end inside a key tile; a kernel of its own, because the loop
 // of the plain one loses up to 10 % to that bookkeeping (B4 H32 S1024 D64 29.9 -> 33.0 us, B1 H32 S4096 D128 137 -> 144).
 template <int D, int QB, int NW, int KT, int KS, bool kCut>
-__global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(const FwdParams p) {
+__global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 4)) void attn_fwd_kernel(const FwdParams p) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
   constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK, LDV = C::LDV;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -592,8 +598,14 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
   FwdPlan plan;
   const int64_t heads = static_cast<int64_t>(a.B) * a.Hq;
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
-  TripCost cost = {1.5, 1.1, 2, 0.0};
+  TripCost cost;
   int bm = 128, kt = 64;
+  auto use = [&](auto cfg, double alone_us, double full_us) {
+    using C = decltype(cfg);
+    bm = C::BM;
+    kt = C::kKT;
+    cost = {alone_us, full_us, C::kPerCu, 0.0};
+  };
   // Tile choice for D = 64: more waves per workgroup share each staged K/V tile (fewer barriers and
   // global loads per MFMA), but the launch still has to fill 256 CUs, so small problems get small tiles.
   if (D == 64) {
@@ -609,17 +621,17 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
     // when those still cover the CUs and the launch is rectangular (one rank's share of configs[1]: 19.8 -> 16.9 us for
     // rank 3 of 4; on a whole causal sequence, or with 256 keys, the smaller workgroups are a few percent faster)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? FwdPlan::kSplit8 : FwdPlan::kSplit4;
-    bm = plan.kernel == FwdPlan::kWaves8 ? 256 : plan.kernel == FwdPlan::kSplit4 ? 64 : 128;
-    kt = plan.kernel >= FwdPlan::kSplit4 ? 128 : 64;
-    cost = plan.kernel == FwdPlan::kWaves8 ? TripCost{1.6, 1.28, 2, 0.0} : plan.kernel == FwdPlan::kWaves4 ? TripCost{1.2, 0.66, 2, 0.0}
-         : plan.kernel == FwdPlan::kSplit8 ? TripCost{1.5, 1.3, 1, 0.0} : TripCost{1.35, 0.7, 2, 0.0};
+    switch (plan.kernel) {
+      case FwdPlan::kWaves8: use(FwdCfg<64, 1, 8, 64>(), 1.6, 1.28); break;
+      case FwdPlan::kWaves4: use(FwdCfg<64, 1, 4, 64>(), 1.2, 0.66); break;
+      case FwdPlan::kSplit8: use(FwdCfg<64, 1, 8, 128, 2>(), 1.5, 1.3); break;
+      case FwdPlan::kSplit4: use(FwdCfg<64, 1, 4, 128, 2>(), 1.35, 0.7); break;
+    }
   } else {
     // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
     plan.kernel = groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
-    if (plan.kernel == FwdPlan::kWaves8) {
-      bm = 256;
-      cost = {1.6, 2.13, 1, 0.0};
-    }
+    if (plan.kernel == FwdPlan::kWaves8) use(FwdCfg<128, 1, 8, 64>(), 1.6, 2.13);
+    else use(FwdCfg<128, 1, 4, 64>(), 1.5, 1.1);
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * fwd_piece_floats(D);

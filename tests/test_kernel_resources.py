@@ -30,3 +30,28 @@ def test_loss_kernels_keep_the_row_in_registers(tmp_path):
     assert sum("ce_one_pass_kernel" in name for name in kernels) == 22
     for name, r in kernels.items():
         assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0, (name, r)
+
+
+def test_attention_kernels_fit_a_cu_as_often_as_their_plans_count_on(tmp_path):
+    """Registers: waves per SIMD x 4 SIMDs hold the workgroups of a CU (LDS is asserted where the tiles are laid out), and
+    none of them are in scratch.  Eight waves have a CU to themselves at head_dim 128 and with split keys, and in dQ; the
+    four waves of dQ at head_dim 128 do as well."""
+    per_cu = {}
+    for source in ("attn_fwd.hip", "attn_bwd.hip"):
+        for name, r in resources(source, tmp_path).items():
+            assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0, (name, r)
+            numbers = [int(n) for n in re.findall(r"L[ib](\d+)E", name)]
+            if "attn_fwd_kernel" in name:
+                D, _, NW, _, KS, _ = numbers
+                want = 1 if NW == 8 and (D == 128 or KS == 2) else 2
+            elif "attn_bwd_dq_kernel" in name:
+                D, NW, _, _, KS, _ = numbers
+                want = 2 if NW == 4 and D == 64 else 1
+            elif "dkdv_kernel" in name:
+                NW, want = (4, 2) if "_d64" in name else (8, 1)
+            else:
+                continue
+            assert r["Occupancy"] * 4 >= want * NW, (name, r)
+            per_cu[name] = want
+    assert len(per_cu) == 12 + 24 + 4
+
