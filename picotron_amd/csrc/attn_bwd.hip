@@ -1048,8 +1048,8 @@ DkdvPlan make_dkdv_plan(const AttnParams& a) {
   // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
   // are up to 30 % faster)
   plan.pair = a.causal && n_ktiles >= 2 && heads * ((n_ktiles + 1) / 2) >= (D == 64 ? 384 : 256);
-  TripCost cost = {1.1, 1.0, C::kPerCu, 0.0};
-  if (D == 128) cost = {1.65, 2.05, C::kPerCu, 0.0};
+  TripCost cost = {1.1, 1.0, 1.0, C::kPerCu, 0.0};
+  if (D == 128) cost = {1.65, 2.05, 1.0, C::kPerCu, 0.0};
   cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
   auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
   plan.len = choose_pieces(heads, n_ktiles, cost, plan.pair, trips_of);
@@ -1121,11 +1121,11 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
   TripCost cost;
   int bm = 128, kt = 64;
-  auto use = [&](auto cfg, double alone_us, double full_us) {
+  auto use = [&](auto cfg, double alone_us, double full_us, double cut) {
     using C = decltype(cfg);
     bm = C::BM;
     kt = C::kKT;
-    cost = {alone_us, full_us, C::kPerCu, 0.0};
+    cost = {alone_us, full_us, ends_inside_tile(a.kv, kt) ? 1.0 : cut, C::kPerCu, 0.0};   // (such chunks run the cutting kernel in any case)
   };
   if (D == 64) {
     const int64_t visible_keys = a.causal ? std::min<int64_t>(a.Sk, static_cast<int64_t>(a.q_offset) + a.Sq) : a.Sk;
@@ -1143,15 +1143,15 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     // per workgroup: 18.8 -> 17.9 us)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
     switch (plan.kernel) {
-      case DqPlan::kWaves8: use(DqCfg<64, 8, 64>(), 1.7, 1.5); break;
-      case DqPlan::kWaves4: use(DqCfg<64, 4, 64>(), 1.3, 0.78); break;
-      case DqPlan::kSplit8: use(DqCfg<64, 8, 128, 2>(), 1.6, 1.5); break;
-      case DqPlan::kSplit4: use(DqCfg<64, 4, 128, 2>(), 1.25, 0.8); break;
+      case DqPlan::kWaves8: use(DqCfg<64, 8, 64>(), 1.7, 1.5, 1.0); break;
+      case DqPlan::kWaves4: use(DqCfg<64, 4, 64>(), 0.79, 0.5, 1.02); break;
+      case DqPlan::kSplit8: use(DqCfg<64, 8, 128, 2>(), 1.6, 1.5, 1.0); break;
+      case DqPlan::kSplit4: use(DqCfg<64, 4, 128, 2>(), 1.25, 0.8, 1.0); break;
     }
   } else {
     plan.kernel = groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
-    if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 2.0, 2.87);
-    else use(DqCfg<128, 4, 64>(), 1.65, 1.8);
+    if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 1.15, 2.81, 1.01);
+    else use(DqCfg<128, 4, 64>(), 2.45, 0.78, 1.05);
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);

@@ -373,12 +373,15 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
 }
 
 // Host: the piece length for a launch, from what its workgroups cost.  A trip takes `alone_us` in a workgroup that has its
-// CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each: as many as its registers and LDS are
-// budgeted for.
-// (Fitted to launches from 1 to 300 heads and 200 to 8000 rows; over 27 such shapes the piece lengths chosen ran within
-// 0.7 % of the best ones in the geometric mean, 5 % at worst.)
+// CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each, `cut` times that in the kernel that can cut
+// (see kCut of the forward); `per_cu` is the number the kernel's registers and LDS are budgeted for.
+// (Fitted to every piece length of 1098 forward, dQ and dK/dV launches each, 1 to 256 heads and 200 to 8192 rows.  The
+// lengths chosen ran within 0.1 to 1.6 % of the best ones in the geometric mean -- dQ with split keys 3 %, dK/dV at head_dim
+// 64 6 % -- and at worst 3.2 % slower than the whole launch.  The four-wave kernels of head_dim 128 were once planned as two
+// per CU where their registers let one run, and the cutting kernel's own loss was not counted: at one sequence of 3000 rows
+// and 20 heads the forward, whole 100 us, was cut to 95 and is 68 whole now that two fit; dQ, whole 94, was cut to 109.)
 struct TripCost {
-  double alone_us, full_us;
+  double alone_us, full_us, cut;
   int per_cu;
   double piece_bytes;
 };
@@ -426,7 +429,7 @@ double launch_us(int64_t heads, int n_tiles, const TripCost& c, int len, bool pa
   if (pairs) workgroups = heads * ((n_tiles + 1) / 2);
   const double shared = c.per_cu > 1 ? std::min(1.0, std::max(0.0, (workgroups - kCus) / static_cast<double>(kCus)))
                                      : std::min(1.0, workgroups / static_cast<double>(kCus));
-  const double trip = c.alone_us + (std::max(c.alone_us, c.full_us * c.per_cu) - c.alone_us) * shared;
+  const double trip = (c.alone_us + (std::max(c.alone_us, c.full_us * c.per_cu) - c.alone_us) * shared) * (len > 0 ? c.cut : 1.0);
   Places places(kCus * c.per_cu);
   if (pairs) {
     for (int i = 0; i < (n_tiles + 1) / 2; ++i) {
@@ -444,8 +447,8 @@ double launch_us(int64_t heads, int n_tiles, const TripCost& c, int len, bool pa
 template <typename F>
 int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, bool pairs, const F& trips_of) {
   if (heads * n_tiles > 4 * 512) return 0;   // enough workgroups that their lengths even out
-  // a cut has to win 5 %, the most the estimate was found to be off by, and the time in which a host launches the second
-  // kernel: where the host is the slower side a shorter kernel gains nothing (B2 H9/3 S256 D64, forward and backward: 33 us
+  // a cut has to win 5 % by the estimate (with that, none of the launches above lost more than 3.2 %) and the time in which a
+  // host launches the second kernel: where the host is the slower side a shorter kernel gains nothing (B2 H9/3 S256 D64, forward and backward: 33 us
   // of kernels cut to 29 took 38 us for 35)
   constexpr double kLaunchUs = 5.0;
   const double uncut_us = launch_us(heads, n_tiles, c, 0, pairs, trips_of);

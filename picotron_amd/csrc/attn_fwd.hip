@@ -600,11 +600,11 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
   auto groups = [&](int bm) { return heads * ((a.Sq + bm - 1) / bm); };
   TripCost cost;
   int bm = 128, kt = 64;
-  auto use = [&](auto cfg, double alone_us, double full_us) {
+  auto use = [&](auto cfg, double alone_us, double full_us, double cut) {
     using C = decltype(cfg);
     bm = C::BM;
     kt = C::kKT;
-    cost = {alone_us, full_us, C::kPerCu, 0.0};
+    cost = {alone_us, full_us, ends_inside_tile(a.kv, kt) ? 1.0 : cut, C::kPerCu, 0.0};   // (such chunks run the cutting kernel in any case)
   };
   // Tile choice for D = 64: more waves per workgroup share each staged K/V tile (fewer barriers and
   // global loads per MFMA), but the launch still has to fill 256 CUs, so small problems get small tiles.
@@ -622,16 +622,16 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
     // rank 3 of 4; on a whole causal sequence, or with 256 keys, the smaller workgroups are a few percent faster)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? FwdPlan::kSplit8 : FwdPlan::kSplit4;
     switch (plan.kernel) {
-      case FwdPlan::kWaves8: use(FwdCfg<64, 1, 8, 64>(), 1.6, 1.28); break;
-      case FwdPlan::kWaves4: use(FwdCfg<64, 1, 4, 64>(), 1.2, 0.66); break;
-      case FwdPlan::kSplit8: use(FwdCfg<64, 1, 8, 128, 2>(), 1.5, 1.3); break;
-      case FwdPlan::kSplit4: use(FwdCfg<64, 1, 4, 128, 2>(), 1.35, 0.7); break;
+      case FwdPlan::kWaves8: use(FwdCfg<64, 1, 8, 64>(), 1.55, 0.84, 1.15); break;
+      case FwdPlan::kWaves4: use(FwdCfg<64, 1, 4, 64>(), 0.8, 0.4, 1.09); break;
+      case FwdPlan::kSplit8: use(FwdCfg<64, 1, 8, 128, 2>(), 1.5, 1.3, 1.0); break;
+      case FwdPlan::kSplit4: use(FwdCfg<64, 1, 4, 128, 2>(), 1.6, 0.5, 1.19); break;
     }
   } else {
     // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
     plan.kernel = groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
-    if (plan.kernel == FwdPlan::kWaves8) use(FwdCfg<128, 1, 8, 64>(), 1.6, 2.13);
-    else use(FwdCfg<128, 1, 4, 64>(), 1.5, 1.1);
+    if (plan.kernel == FwdPlan::kWaves8) use(FwdCfg<128, 1, 8, 64>(), 1.6, 2.13, 1.0);
+    else use(FwdCfg<128, 1, 4, 64>(), 1.66, 0.96, 1.19);
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * fwd_piece_floats(D);

@@ -55,3 +55,19 @@ def test_attention_kernels_fit_a_cu_as_often_as_their_plans_count_on(tmp_path):
             per_cu[name] = want
     assert len(per_cu) == 12 + 24 + 4
 
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(1, 20, 20, 2500, 128), (1, 20, 20, 3000, 128), (1, 32, 32, 4000, 64), (1, 16, 16, 8000, 64)])
+def test_launches_that_fill_the_gpu_run_whole(B, Hq, Hkv, S, D):
+    """Attention launches that every piece length slows down, by 1 to 16 %, ask for no scratch memory: neither the forward
+    nor dQ and dK/dV are cut."""
+    import ctypes
+    import math
+
+    import torch
+    from picotron_amd import _lib, ops
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    q, k = (torch.empty(B, h, S, D, dtype=torch.bfloat16) for h in (Hq, Hkv))
+    d = ops._desc(q, k, k, q, 1 / math.sqrt(D), True, 0)
+    assert _lib.lib().pico_attn_fwd_workspace_bytes(ctypes.byref(d), 1) == 0
+    assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == 0
