@@ -72,7 +72,6 @@ class _PublishKV(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         # layout only, no saved tensors: the node may run in several backward calls (one rank's loss at a time)
         ctx.layout = tuple((t.dtype, t.stride() if ops._dense(t) and t.stride(-1) == 1 else None) for t in (k, v))
-        box.layout = ctx.layout
         if rope is not None:
             cos, sin, pos0 = rope
             return ops.rope(k, cos, sin, pos_offset=pos0), v.view_as(v)
@@ -80,18 +79,12 @@ class _PublishKV(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gk, gv):
-        box = ctx.box
-        dk = dv = None
-        box.arrived = 0
-        if box.final_dk is not None:
-            # the last reader's kernel wrote the rounded totals itself
-            dk, dv = box.final_dk, box.final_dv
-            box.final_dk = box.final_dv = box.dk = box.dv = None
-        elif box.dk is not None:
+        left = ctx.box.take()
+        dk, dv = left.final_dk, left.final_dv      # (the last reader's kernel wrote the rounded totals itself)
+        if left.dk is not None:
             (k_dtype, k_strides), (v_dtype, v_strides) = ctx.layout
-            dk = ops.convert_f32(box.dk, k_dtype, strides=k_strides)
-            dv = ops.convert_f32(box.dv, v_dtype, strides=v_strides)
-            box.dk = box.dv = None      # the next backward through this chunk starts a fresh sum
+            dk = ops.convert_f32(left.dk, k_dtype, strides=k_strides)
+            dv = ops.convert_f32(left.dv, v_dtype, strides=v_strides)
         if gk is not None:
             if ctx.rope is not None:    # a gradient that reached the rotated chunk some other way
                 cos, sin, pos0 = ctx.rope
@@ -148,8 +141,8 @@ class RingAttentionFunc(torch.autograd.Function):
     All chunks a rank will read are at hand when its turn comes, so by default the loop over the ring steps
     (:30-45, :63-106) runs INSIDE one launch per direction: the kernels take the list of chunk tensors as it is (no
     concatenation, no hop copies), carry the online softmax across the chunks, write the output in q's dtype and add
-    each chunk's dK / dV block to that chunk's accumulator; on the GPU its autograd node is native (``_one_launch``), the
-    Python form of the same below serves the other devices.  Chunks that do not fit one launch (see
+    each chunk's dK / dV block to that chunk's accumulator; on the GPU its autograd node is native (``_one_launch``), and
+    the Python form of the same below, on the same bookkeeping of the sums, is what stand-ins for the kernels run under.  Chunks that do not fit one launch (see
     ``ops.chunks_fit_one_launch``), or ``PICO_RING_PER_STEP=1``, take the reference's shape: one launch per ring step
     with the hop between steps."""
 
@@ -263,51 +256,25 @@ class RingAttentionFunc(torch.autograd.Function):
             wants[c] = ctx.needs_input_grad[7 + 2 * i] or ctx.needs_input_grad[8 + 2 * i]
         nothing = (None,) * (7 + 2 * len(peers))
 
-        def boxes(c):
-            """(dk, dv, add?) of chunk c's travelling accumulators; the first block to reach them writes."""
-            box = chunks[c].grads
-            fresh = box.dk is None
-            if fresh:
-                shape = chunks[c].k.shape
-                box.dk = torch.empty(shape, dtype=torch.float32, device=q.device)
-                box.dv = torch.empty(shape, dtype=torch.float32, device=q.device)
-            return box.dk, box.dv, not fresh
-
-        def finals(c):
-            """bf16 buffers for chunk c's totals if this rank's block is the last one they wait for (every rank that
-            read the chunk has added its block), in the chunk's own layout; else None."""
-            box = chunks[c].grads
-            box.arrived += 1
-            (k_dtype, k_strides), (v_dtype, v_strides) = box.layout if box.layout is not None else ((None, None), (None, None))
-            if box.arrived != box.readers or k_dtype not in ops.FINAL_TOTAL_DTYPES or v_dtype != k_dtype:
-                return None
-            shape = chunks[c].k.shape
-            if k_strides is not None and k_strides == v_strides:
-                box.final_dk = torch.empty_strided(shape, k_strides, dtype=k_dtype, device=q.device)
-                box.final_dv = torch.empty_strided(shape, k_strides, dtype=k_dtype, device=q.device)
-            else:   # chunks that are views with gaps (or k and v laid out differently): contiguous gradients
-                box.final_dk = torch.empty(shape, dtype=k_dtype, device=q.device)
-                box.final_dv = torch.empty(shape, dtype=k_dtype, device=q.device)
-            return box.final_dk, box.final_dv
+        def claim(c, whole):
+            """Where this rank's block of chunk c's dK / dV goes (``GradBox`` in ``csrc/host.cpp``)."""
+            k, v = chunks[c].k.detach(), chunks[c].v.detach()
+            return chunks[c].grads.claim(k, v, whole, k.dtype in ops.FINAL_TOTAL_DTYPES)
 
         if ctx.one_launch is not None:
             order, q_off = ctx.one_launch
             ks = [chunks[c].k.detach() for c in order]
             vs = [chunks[c].v.detach() for c in order]
-            fin = {c: finals(c) if wants[c] else None for c in order}
-            # a chunk whose totals leave from this launch needs fp32 sums only if earlier blocks left some
-            got = [(None, None, False) if not wants[c] else
-                   ((chunks[c].grads.dk, chunks[c].grads.dv, chunks[c].grads.dk is not None) if fin[c] is not None else boxes(c))
-                   for c in order]
+            got = [claim(c, True) if wants[c] else None for c in order]
             dq = None
             if ctx.needs_input_grad[0]:
                 dq = (torch.empty_strided(q.shape, q.stride(), dtype=q.dtype, device=q.device)
                       if ops._dense(q) and q.stride(-1) == 1 else torch.empty(q.shape, dtype=q.dtype, device=q.device))
-            ops.attn_bwd_chunks(dout, q, ks, vs, softmax_lse, sm_scale, is_causal, q_off, dq, [g[0] for g in got],
-                                [g[1] for g in got], dkv_accumulate=[g[2] for g in got], out=out, rope=cs,
+            of = lambda name: [getattr(g, name) if g is not None else None for g in got]  # noqa: E731
+            ops.attn_bwd_chunks(dout, q, ks, vs, softmax_lse, sm_scale, is_causal, q_off, dq, of("dk"), of("dv"),
+                                dkv_accumulate=[g is not None and g.add for g in got], out=out, rope=cs,
                                 q_pos_offset=q_pos, k_pos_offset=q_pos - q_off if is_causal else 0,
-                                dk_finals=[fin[c][0] if fin[c] is not None else None for c in order],
-                                dv_finals=[fin[c][1] if fin[c] is not None else None for c in order],
+                                dk_finals=of("final_dk"), dv_finals=of("final_dv"),
                                 checked=True)   # (the forward asked chunks_fit_one_launch about these same tensors)
             return (dq,) + nothing[1:]
 
@@ -326,7 +293,8 @@ class RingAttentionFunc(torch.autograd.Function):
             if runs and (wants[held] or ctx.needs_input_grad[0]):
                 # dq += block_dq (:85-93) and the chunk's travelling dk / dv += block_dk / block_dv, all inside the
                 # kernels; the first block to reach an accumulator writes it instead of adding
-                dk_c, dv_c, add = boxes(held) if wants[held] else (None, None, False)
+                g = claim(held, False) if wants[held] else None
+                dk_c, dv_c, add = (g.dk, g.dv, g.add) if g is not None else (None, None, False)
                 first = dq is None
                 if first:
                     dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)

@@ -11,7 +11,7 @@ receive buffers, which is the hop.  At ring step s rank r receives the chunk pub
 
 The reference's third ring (``d_kv_comm``, :61) moves the fp32 dK / dV accumulators from rank to rank.  Virtual
 ranks share one address space, so the accumulators do not travel: they live with the published chunk
-(``process_group_manager.GradBox``), every rank's backward adds its block there inside the kernel, and the chunk's
+(``GradBox`` in ``csrc/host.cpp``), every rank's backward adds its block there inside the kernel, and the chunk's
 autograd node returns the total after the last rank has added its part.
 """
 from __future__ import annotations

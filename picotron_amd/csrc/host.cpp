@@ -616,26 +616,58 @@ Tensor flash_attention(const Tensor& q, const Tensor& k, const Tensor& v, double
 
 // ------------------------------------------------------------------------------------------------ ring attention
 // The autograd nodes of ring attention over virtual ranks (context_parallel.py) where all ring steps of a rank are one
-// launch.  The Python objects they share -- one GradBox per published chunk -- belong to the mailbox; they are touched with
-// the GIL held, the kernels are launched without it.
-struct PyHeld : torch::CustomClassHolder {
-  std::vector<PyObject*> objects;   // strong references
-  explicit PyHeld(const std::vector<pybind11::object>& os) {
-    for (const auto& o : os) objects.push_back(pybind11::object(o).release().ptr());
-  }
-  ~PyHeld() override {
-    pybind11::gil_scoped_acquire gil;
-    for (PyObject* o : objects) Py_DECREF(o);
-  }
-};
-OptTensor tensor_attr(const pybind11::handle& o, const char* name) {
-  pybind11::object v = o.attr(name);
-  return v.is_none() ? std::nullopt : OptTensor(v.cast<Tensor>());
-}
-void set_attr(const pybind11::handle& o, const char* name, const OptTensor& t) { o.attr(name) = t ? pybind11::cast(*t) : pybind11::none(); }
-
+// launch.  They share one GradBox per published chunk, which belongs to the mailbox's chunk.
 // the gradient of a chunk leaves in the chunk's own layout where that is dense with a unit last stride (as k and v share it)
 bool dense_layout(const Tensor& t) { return t.stride(-1) == 1 && t.is_non_overlapping_and_dense(); }
+
+// fp32 dK / dV accumulators of one published chunk: what travels round the ring in the reference (context_parallel.py:85-106).
+// Every rank's backward adds its block here; the chunk's own autograd node hands the total back once all of them have run.
+// All bookkeeping of the sums is here, for the native nodes and for the Python ones (one launch per ring step) alike.
+struct GradBox : torch::CustomClassHolder {
+  OptTensor dk, dv;               // sums so far; the first block to reach them writes
+  OptTensor final_dk, final_dv;   // totals in the chunk's dtype, written by the kernel that completes them
+  int64_t readers = 0;            // ranks whose forward read the chunk and will add a block in their backward
+  int64_t arrived = 0;            // ... and how many of them have done so since the sums were last handed back
+  std::mutex mutex;
+
+  // Where a rank's block goes: added to (add) or written into dk, dv; with final_dk the launch writes bf16(sums so far + block)
+  // there instead and reads dk, dv only where there are any.
+  struct Share {
+    OptTensor dk, dv;
+    bool add = false;
+    OptTensor final_dk, final_dv;
+  };
+  // `whole`: the rank's whole block arrives in this launch (not one ring step of it), so that the block every other reader has
+  // waited for may leave as the total; `rounds`: the launch can write totals in the chunk's dtype
+  Share claim(const Tensor& k, const Tensor& v, bool whole, bool rounds) {
+    std::lock_guard<std::mutex> lock(mutex);
+    Share s{dk, dv, dk.has_value(), {}, {}};
+    if (whole && ++arrived == readers && rounds && k.scalar_type() == v.scalar_type()) {
+      const bool own_layout = dense_layout(k) && k.strides() == v.strides();
+      auto total = [&] { return own_layout ? at::empty_strided(k.sizes(), k.strides(), k.options()) : at::empty(k.sizes(), k.options()); };
+      final_dk = s.final_dk = total();
+      final_dv = s.final_dv = total();
+    } else if (!s.add) {
+      dk = s.dk = at::empty(k.sizes(), k.options().dtype(at::kFloat));
+      dv = s.dv = at::empty(k.sizes(), k.options().dtype(at::kFloat));
+    }
+    return s;
+  }
+  // What this backward pass left, the totals or else the sums; the next backward through the chunk starts afresh.
+  Share take() {
+    std::lock_guard<std::mutex> lock(mutex);
+    Share s{dk, dv, false, final_dk, final_dv};
+    if (final_dk) s.dk = s.dv = std::nullopt;
+    dk = dv = final_dk = final_dv = std::nullopt;
+    arrived = 0;
+    return s;
+  }
+};
+using GradBoxPtr = c10::intrusive_ptr<GradBox>;
+struct GradBoxes : torch::CustomClassHolder {
+  std::vector<GradBoxPtr> boxes;
+  explicit GradBoxes(std::vector<GradBoxPtr> b) : boxes(std::move(b)) {}
+};
 
 Tensor convert_sum(const Tensor& src, at::ScalarType dtype, bool dense, at::IntArrayRef strides) {
   Tensor dst = dense ? at::empty_strided(src.sizes(), strides, src.options().dtype(dtype)) : at::empty(src.sizes(), src.options().dtype(dtype));
@@ -647,7 +679,7 @@ Tensor convert_sum(const Tensor& src, at::ScalarType dtype, bool dense, at::IntA
 // Identity on a rank's (k, v) chunk -- with rope tables k is rotated -- that marks where the ring's dK / dV come back: the
 // native form of _PublishKV.  It keeps no saved variables: the node may run in several backward calls.
 struct PublishKV : torch::autograd::Function<PublishKV> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& v, const c10::intrusive_ptr<PyHeld>& box,
+  static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& v, const GradBoxPtr& box,
                                const Rope& rope_cs, int64_t pos) {
     ctx->saved_data["box"] = c10::IValue::make_capsule(box);
     ctx->saved_data["dtypes"] = std::vector<int64_t>{static_cast<int64_t>(k.scalar_type()), static_cast<int64_t>(v.scalar_type())};
@@ -664,27 +696,12 @@ struct PublishKV : torch::autograd::Function<PublishKV> {
     return {k.variable_data(), v.variable_data()};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    OptTensor dk, dv, sum_k, sum_v;
-    {
-      pybind11::gil_scoped_acquire gil;
-      const pybind11::handle box(static_cast<PyHeld*>(ctx->saved_data["box"].toCapsule().get())->objects[0]);
-      box.attr("arrived") = 0;
-      dk = tensor_attr(box, "final_dk");
-      if (dk) {   // the last reader's kernel wrote the rounded totals itself
-        dv = tensor_attr(box, "final_dv");
-        set_attr(box, "final_dk", std::nullopt);
-        set_attr(box, "final_dv", std::nullopt);
-      } else {
-        sum_k = tensor_attr(box, "dk");
-        sum_v = tensor_attr(box, "dv");
-      }
-      set_attr(box, "dk", std::nullopt);   // the next backward through this chunk starts a fresh sum
-      set_attr(box, "dv", std::nullopt);
-    }
+    const GradBox::Share left = static_cast<GradBox*>(ctx->saved_data["box"].toCapsule().get())->take();
+    OptTensor dk = left.final_dk, dv = left.final_dv;   // (the last reader's kernel wrote the rounded totals itself)
     const auto dtypes = ctx->saved_data["dtypes"].toIntVector(), dense = ctx->saved_data["dense"].toIntVector();
-    if (sum_k) {
-      dk = convert_sum(*sum_k, static_cast<at::ScalarType>(dtypes[0]), dense[0], ctx->saved_data["k_strides"].toIntVector());
-      dv = convert_sum(*sum_v, static_cast<at::ScalarType>(dtypes[1]), dense[1], ctx->saved_data["v_strides"].toIntVector());
+    if (left.dk) {
+      dk = convert_sum(*left.dk, static_cast<at::ScalarType>(dtypes[0]), dense[0], ctx->saved_data["k_strides"].toIntVector());
+      dv = convert_sum(*left.dv, static_cast<at::ScalarType>(dtypes[1]), dense[1], ctx->saved_data["v_strides"].toIntVector());
     }
     if (g[0].defined()) {   // a gradient that reached the (rotated) chunk some other way
       Tensor gk = g[0];
@@ -697,17 +714,15 @@ struct PublishKV : torch::autograd::Function<PublishKV> {
   }
 };
 
-std::pair<Tensor, Tensor> publish_kv(const Tensor& k, const Tensor& v, const pybind11::object& box, const Rope& rope_cs, int64_t pos) {
-  auto held = c10::make_intrusive<PyHeld>(std::vector<pybind11::object>{box});
-  pybind11::gil_scoped_release nogil;
-  auto r = PublishKV::apply(k, v, held, rope_cs, pos);
+std::pair<Tensor, Tensor> publish_kv(const Tensor& k, const Tensor& v, const GradBoxPtr& box, const Rope& rope_cs, int64_t pos) {
+  auto r = PublishKV::apply(k, v, box, rope_cs, pos);
   return {r[0], r[1]};
 }
 
 // What the launch of a rank's forward left behind, for its backward.
 struct RingPass {
   Tensor out, lse, q;   // q: the rotated copy where rope tables are given
-  c10::intrusive_ptr<PyHeld> boxes;
+  c10::intrusive_ptr<GradBoxes> boxes;
   Rope rope;
   double sm_scale;
   bool causal;
@@ -746,35 +761,16 @@ struct RingAttention : torch::autograd::Function<RingAttention> {
     OptTensors dks(n), dvs(n), dk_finals(n), dv_finals(n);
     std::vector<bool> add(n, false);
     bool any_final = false;
-    {
-      pybind11::gil_scoped_acquire gil;
-      const auto& boxes = static_cast<PyHeld*>(ctx->saved_data["boxes"].toCapsule().get())->objects;
-      for (size_t i = 0; i < n; ++i) {
-        if (!ctx->needs_input_grad(1 + 2 * i) && !ctx->needs_input_grad(2 + 2 * i)) continue;
-        const pybind11::handle box(boxes[i]);
-        const int64_t arrived = box.attr("arrived").cast<int64_t>() + 1;
-        box.attr("arrived") = arrived;
-        dks[i] = tensor_attr(box, "dk");
-        dvs[i] = tensor_attr(box, "dv");
-        add[i] = dks[i].has_value();
-        if (arrived == box.attr("readers").cast<int64_t>()) {
-          // every other rank that read the chunk has added its block: the totals leave from this launch, and fp32 sums are
-          // only read, if earlier blocks left some
-          const Tensor &k = ks[i], &v = vs[i];
-          const bool own_layout = dense_layout(k) && k.strides() == v.strides();
-          auto total = [&] { return own_layout ? at::empty_strided(k.sizes(), k.strides(), k.options()) : at::empty(k.sizes(), k.options()); };
-          dk_finals[i] = total();
-          dv_finals[i] = total();
-          set_attr(box, "final_dk", dk_finals[i]);
-          set_attr(box, "final_dv", dv_finals[i]);
-          any_final = true;
-        } else if (!add[i]) {
-          dks[i] = at::empty(ks[i].sizes(), ks[i].options().dtype(at::kFloat));
-          dvs[i] = at::empty(ks[i].sizes(), ks[i].options().dtype(at::kFloat));
-          set_attr(box, "dk", dks[i]);
-          set_attr(box, "dv", dvs[i]);
-        }
-      }
+    const auto& boxes = static_cast<GradBoxes*>(ctx->saved_data["boxes"].toCapsule().get())->boxes;
+    for (size_t i = 0; i < n; ++i) {
+      if (!ctx->needs_input_grad(1 + 2 * i) && !ctx->needs_input_grad(2 + 2 * i)) continue;
+      const GradBox::Share s = boxes[i]->claim(ks[i], vs[i], true, true);
+      dks[i] = s.dk;
+      dvs[i] = s.dv;
+      add[i] = s.add;
+      dk_finals[i] = s.final_dk;
+      dv_finals[i] = s.final_dv;
+      any_final |= s.final_dk.has_value();
     }
     OptTensor dq;
     if (ctx->needs_input_grad(0)) dq = empty_like_layout(q, q.options());
@@ -787,10 +783,9 @@ struct RingAttention : torch::autograd::Function<RingAttention> {
 };
 
 Tensor ring_node(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs, const Tensor& out, const Tensor& lse,
-                 const OptTensor& q_rot, const std::vector<pybind11::object>& boxes, double sm_scale, bool causal, int64_t q_offset,
+                 const OptTensor& q_rot, const std::vector<GradBoxPtr>& boxes, double sm_scale, bool causal, int64_t q_offset,
                  const Rope& rope_cs, int64_t q_pos, int64_t k_pos) {
-  RingPass p = {out, lse, q_rot.value_or(Tensor()), c10::make_intrusive<PyHeld>(boxes), rope_cs, sm_scale, causal, q_offset, q_pos, k_pos};
-  pybind11::gil_scoped_release nogil;
+  RingPass p = {out, lse, q_rot.value_or(Tensor()), c10::make_intrusive<GradBoxes>(boxes), rope_cs, sm_scale, causal, q_offset, q_pos, k_pos};
   std::vector<Tensor> kvs;
   for (size_t i = 0; i < ks.size(); ++i) {
     kvs.push_back(ks[i]);
@@ -1533,8 +1528,22 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("chunks_fit", &chunks_fit, nogil());
   m.def("attn_fwd", &attn_fwd, nogil());
   m.def("attn_bwd", &attn_bwd, nogil());
-  m.def("publish_kv", &publish_kv);
-  m.def("ring_node", &ring_node);
+  py::class_<GradBox, GradBoxPtr>(m, "GradBox", "fp32 dK / dV sums of one published chunk; see csrc/host.cpp")
+      .def(py::init([] { return c10::make_intrusive<GradBox>(); }))
+      .def_readonly("dk", &GradBox::dk)
+      .def_readonly("dv", &GradBox::dv)
+      .def_readwrite("readers", &GradBox::readers)
+      .def_readonly("arrived", &GradBox::arrived)
+      .def("claim", &GradBox::claim, py::arg("k"), py::arg("v"), py::arg("whole"), py::arg("rounds"))
+      .def("take", &GradBox::take);
+  py::class_<GradBox::Share>(m, "GradShare")
+      .def_readonly("dk", &GradBox::Share::dk)
+      .def_readonly("dv", &GradBox::Share::dv)
+      .def_readonly("add", &GradBox::Share::add)
+      .def_readonly("final_dk", &GradBox::Share::final_dk)
+      .def_readonly("final_dv", &GradBox::Share::final_dv);
+  m.def("publish_kv", &publish_kv, nogil());
+  m.def("ring_node", &ring_node, nogil());
   m.def("flash_attention", &flash_attention, nogil());
   const auto product_kind = [](const std::string& kind) {
     TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
