@@ -103,3 +103,21 @@ for kind, M, N, K, want in (("NT", 512, 576, 576, "own"), ("NN", 512, 1024, 1024
         assert got == (want if fits else "library"), (kind, M, N, K, pad_a, pad_b, got)
     assert host.product_route(operand(ra, ca, address=(1 << 20) + 2), operand(rb, cb), kind) == "torch"
 ''')
+
+
+def test_long_contractions_are_cut_where_pieces_are_faster():
+    """Sizes at which a cut was up to 1.44 times as slow as the whole product, or as another number of pieces, us: whole, in the
+    number it was cut into, in the one expected now."""
+    run('''
+for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 28.7 in 2
+                            ("NT", 256, 4096, 10880, "library"),        # 1.23 times in 2
+                            ("NT", 128, 2048, 8192, "library in 8"),    # 17.2, 22.1 in 2, 14.9
+                            ("NT", 256, 3072, 12288, "library in 4"),   # 37.2, 53.7 in 2, 30.3
+                            ("NN", 3584, 3072, 16384, "library"),       # 292, 332 in 4
+                            ("NN", 3200, 2048, 32000, "library in 4"),  # 395, 522 in 2, 376
+                            ("NN", 4608, 768, 49152, "library in 8"),   # 432, 540 in 4, 346
+                            ("NN", 512, 576, 49152, "library in 16"), ("NN", 2048, 4096, 21760, "library in 2"), ("NT", 640, 2048, 8192, "library in 2")):
+    (ra, ca), (rb, cb) = (M, K), ((N, K) if kind == "NT" else (K, N))
+    got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
+    assert got == want, (kind, M, N, K, got)
+''')
