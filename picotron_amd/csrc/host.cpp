@@ -1014,11 +1014,19 @@ int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
 // lies where a sweep over contractions of 512 .. 8192 crossed ([4096 x 6144]^T [4096 x 2048]: 88 and 89 us).  Under 1024 rows
 // the product is bound by writing the result unless the narrower side leaves the library's tiles half empty.
 // (Transposing the wider operand too costs more than the second 13 %.)
+// Outputs of fewer than 384 of the library's 256 x 256 tiles stay as they are unless one side is the vocabulary's or the
+// contraction is long: its choice for the transposed layout fills the GPU worse there ([4096 x 10880]^T [4096 x 2048] 172 us,
+// transposed 273; [1280 x 12288]^T [1280 x 1536] 64 and 73), and so do short contractions that are no multiple of its step of
+// 64 ([1262 x 12288]^T [1262 x 4096] 1.06 times).  201 drawn products that are transposed took 0.90 of the library's time, five over
+// 1.04 and none over 1.13.
 int64_t turned_operand(Product kind, const Tensor& a, const Tensor& b) {
   if (kind != Product::TN) return 0;
   const int64_t K = a.size(0), M = a.size(1), N = b.size(1), narrow = std::min(M, N), wide = std::max(M, N);
-  if (narrow % 8 || (M < N ? a : b).stride(0) % 8 || (K < 1024 && (K < 512 || narrow >= 1024))) return 0;
+  if (narrow % 8 || (M < N ? a : b).stride(0) % 8 || (K < 1024 && (K < 768 || narrow >= 1024))) return 0;
   if (wide <= 5000 + 1e10 / (static_cast<double>(K) * narrow)) return 0;
+  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
+  if (t256 < 384 && wide < 24576 && (t256 < 256 || K < 4608)) return 0;
+  if (K % 64 && K < 1408 && t256 < 1024) return 0;
   return M < N ? 1 : 2;
 }
 // [K, N] -> [N, K], rows padded to 16 bytes

@@ -121,3 +121,18 @@ for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 
     got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
     assert got == want, (kind, M, N, K, got)
 ''')
+
+
+def test_weight_gradients_are_transposed_where_that_is_faster():
+    """Us whole and with the narrower operand transposed; with few output tiles or a short ragged contraction it lost up to 58 %."""
+    run('''
+for K, M, N, want in ((4096, 10880, 2048, "library"),      # 172, 273
+                      (1152, 10880, 2048, "library"),      # 67, 80
+                      (1280, 12288, 1536, "library"),      # 64, 73
+                      (1262, 12288, 4096, "library"),      # 1.06 times
+                      (4096, 49152, 2048, "turned"),       # 732, 616
+                      (4096, 2048, 16384, "turned"),       # 227, 202
+                      (5504, 12288, 1536, "turned"), (4096, 49152, 576, "turned")):
+    got = host.product_route(operand(K, M), operand(K, N), "TN")
+    assert got == want, (K, M, N, got)
+''')
