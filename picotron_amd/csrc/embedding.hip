@@ -12,6 +12,8 @@
 // 576 18 us (44), 8192 of 2048 52 us (213); 8192 times the same token 129 us (344).
 #include "common.h"
 
+#include <type_traits>
+
 namespace pico {
 namespace {
 
@@ -19,6 +21,8 @@ constexpr int kPlaces = 8;            // sorted places of a workgroup of the sec
 constexpr int kRankWaves = 8;         // waves that share the counting for 64 tokens
 constexpr int kFillBytes = 32768;     // of dw that a workgroup of the first kernel clears
 constexpr int kRankThreads = 64 * kRankWaves;
+
+typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 struct EmbeddingParams {
   const void* ids;
@@ -29,10 +33,19 @@ struct EmbeddingParams {
   int tokens, vocab, hidden, skip;    // skip: an id whose row stays zero (-1: none)
 };
 
+// ids outside [0, vocab) are all one, -1, which no row belongs to (as they stand, wide ones would alias rows of the vocabulary
+// when they are narrowed, and the largest would leave a place of the order unwritten)
+template <typename I>
+__device__ __forceinline__ int id_at(const I* ids, int t, int vocab) {
+  const I id = ids[t];
+  return static_cast<std::make_unsigned_t<I>>(id) < static_cast<std::make_unsigned_t<I>>(vocab) ? static_cast<int>(id) : -1;
+}
+
 template <typename I>
 __global__ __launch_bounds__(kRankThreads) void embedding_rank_fill_kernel(const EmbeddingParams p, const I* __restrict__ ids, int rank_blocks,
                                                                            int64_t dw_bytes) {
   __shared__ int counts[kRankWaves][64];
+  __shared__ __attribute__((aligned(16))) int shared_ids[kRankWaves][64];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   if (static_cast<int>(blockIdx.x) >= rank_blocks) {
     const int64_t from = static_cast<int64_t>(blockIdx.x - rank_blocks) * kFillBytes;
@@ -45,26 +58,31 @@ __global__ __launch_bounds__(kRankThreads) void embedding_rank_fill_kernel(const
     return;
   }
   const int t0 = static_cast<int>(blockIdx.x) * 64, mine = t0 + lane;
-  const int my_id = mine < p.tokens ? static_cast<int>(ids[mine]) : 0x7fffffff;
-  // every wave counts a share of the tokens; the ids it compares with are the same for all lanes
-  const int groups = (p.tokens + 63) / 64;
-  int below = 0;
-  for (int g = groups * wave / kRankWaves; g < groups * (wave + 1) / kRankWaves; ++g) {
-    const int j0 = g * 64, n = p.tokens - j0 < 64 ? p.tokens - j0 : 64;
-    if (j0 == t0) {
-      for (int j = 0; j < n; ++j) {
-        const int id = static_cast<int>(ids[j0 + j]);
-        below += id < my_id || (id == my_id && j < lane);
-      }
-    } else {
-      const int bound = my_id + (j0 < t0 && my_id != 0x7fffffff);   // of equal ids the earlier token comes first
-      if (n == 64) {
-#pragma unroll 16
-        for (int j = 0; j < 64; ++j) below += static_cast<int>(ids[j0 + j]) < bound;
-      } else {
-        for (int j = 0; j < n; ++j) below += static_cast<int>(ids[j0 + j]) < bound;
-      }
+  const int my_id = mine < p.tokens ? id_at(ids, mine, p.vocab) : p.vocab;
+  // every wave counts a share of the tokens, 64 at a time: a lane fetches one of them (the next 64 while these are counted), the
+  // wave's piece of LDS hands all of them to every lane
+  const int groups = (p.tokens + 63) / 64, g_end = groups * (wave + 1) / kRankWaves;
+  auto fetch = [&](int g) {
+    const int j = g * 64 + lane;
+    return g < g_end && j < p.tokens ? id_at(ids, j, p.vocab) : 0x7fffffff;   // (past the end: below nothing)
+  };
+  int* const share = shared_ids[wave];
+  int below = 0, next = fetch(groups * wave / kRankWaves);
+  for (int g = groups * wave / kRankWaves; g < g_end; ++g) {
+    __builtin_amdgcn_wave_barrier();   // (LDS answers a wave in order)
+    share[lane] = next;
+    __builtin_amdgcn_wave_barrier();
+    next = fetch(g + 1);
+    const int j0 = g * 64;
+    const int bound = my_id + (j0 < t0);   // of equal ids the earlier token comes first
+#pragma unroll
+    for (int j = 0; j < 64; j += 4) {
+      const i32x4 id = *reinterpret_cast<const i32x4*>(share + j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) below += id[e] < bound;
     }
+    if (j0 == t0)
+      for (int j = 0; j < 64; ++j) below += share[j] == my_id && j < lane;
   }
   counts[wave][lane] = below;
   __syncthreads();

@@ -39,6 +39,29 @@ def test_embedding_gradient(device, tokens, vocab, hidden, ids_of, dtype, id_dty
         assert not got[~hit].any()
 
 
+
+@pytest.mark.parametrize("id_dtype,beyond", [(torch.int32, (2**31 - 1, -1, -2**31, 100)),
+                                             (torch.int64, (2**31 - 1, 2**32 + 5, 2**63 - 1, -1, -2**63, 100, -2**32 + 7))])
+@pytest.mark.parametrize("tokens", [130, 1000])
+def test_ids_outside_the_vocabulary_add_nothing(device, id_dtype, beyond, tokens):
+    """Through the C ABI, as torch's own lookup refuses such ids in the forward: the largest, ones that narrow to an id of the
+    vocabulary, negative ones, many of each among many groups of tokens."""
+    from picotron_amd import _lib
+    lib, vocab, hidden = _lib.lib(), 100, 72
+    g = torch.Generator().manual_seed(tokens)
+    ids = torch.randint(0, vocab, (tokens,), generator=g)
+    out = torch.rand(tokens, generator=g) < 0.5
+    ids[out] = torch.tensor(beyond)[torch.randint(0, len(beyond), (int(out.sum()),), generator=g)]
+    dy = torch.randn(tokens, hidden, generator=g).to(device, torch.bfloat16)
+    want = torch.zeros(vocab, hidden, dtype=torch.float64, device=device).index_add_(0, ids[~out].to(device), dy[~out.to(device)].double())
+    dev_ids = ids.to(device, id_dtype)
+    dw = torch.empty(vocab, hidden, dtype=torch.bfloat16, device=device)
+    ws = torch.empty(lib.pico_embedding_bwd_workspace_bytes(tokens, hidden), dtype=torch.uint8, device=device)
+    _lib.check(lib.pico_embedding_bwd(dev_ids.data_ptr(), dev_ids.element_size(), dy.data_ptr(), dw.data_ptr(), ws.data_ptr(), tokens, vocab,
+                                      hidden, -1, _lib.PICO_BF16, torch.cuda.current_stream().cuda_stream))
+    assert (dw.double() - want).abs().max().item() <= 4e-3 * want.abs().max().item()
+
+
 def test_norm_at_the_head_of_a_residual_stream(device):
     from picotron_amd.model import TritonRMSNorm
     g = torch.Generator(device="cuda").manual_seed(1)
