@@ -306,7 +306,7 @@ def ring_api_extra(torch, ops, rb, iters=20, eager_only=False):
     torch.cuda.synchronize()
     ms = (time.perf_counter() - t0) * 1e3 / iters
     res["eager"] = {"ms_per_step": round(ms, 4), "TFLOP/s": round(total_flops / (ms * 1e-3) / 1e12, 2),
-                    "note": "host-bound: Python, autograd and ctypes per call"}
+                    "note": "host-bound: autograd's hand-over to its device thread"}
     pgm.setup_process_group_manager(1, 1, 1, 1)
     return res
 
@@ -493,7 +493,7 @@ def train_step_extra(torch, which="smollm_1p7b", steps=10, warmup=3, adamw="fp32
            "mfu_vs_2.5PF": round(tok_s * fpt / MI355X_BF16_DENSE_FLOPS, 4), "steps": steps,
            "adamw_state": layouts[adamw][1],
            "note": "attention / RMSNorm with the residual adds / RoPE / SwiGLU / cross-entropy / AdamW on the HIP kernels; "
-                   "embedding and projections on torch"}
+                   "projections on hipBLASLt and the package's own products"}
     del model, opt
     torch.cuda.empty_cache()
     return res
