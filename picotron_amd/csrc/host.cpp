@@ -958,31 +958,32 @@ double tile_fit(int64_t M, int64_t N) {
 // 143 us and takes 53 us in 16 pieces, [2048 x 21760] @ [21760 x 4096] 447 and 291 us in two.  The pieces cost 8 bytes of
 // fp32 traffic per output element each, hence the lower bound on a piece's length and, as output grows, on its ratio to
 // the number of tiles.  The lines lie where sweeps over 100 .. 8192 rows, 192 .. 4096 columns and contractions of 4096 ..
-// 49152 crossed, on the side where no class loses: of 2400 drawn products the cut ones took 0.52 (NN), 0.81 (NT) and 0.77 (TN)
-// of the library's time in the geometric mean, four of 604 over 1.04 and none over 1.12.
+// 49152 crossed, on the side where no class loses: of 2400 drawn products the 548 that are cut took 0.54 (NN), 0.82 (NT) and
+// 0.74 (TN) of the library's time in the geometric mean, four over 1.06 (1.25 at most: [1076 x 49152] @ [49152 x 3072]).
 // Products of the forward's layout (NT), the library's best, gain only from 8192 on; up to 32 tiles in pieces of 1024 ([128 x
 // 2048] of 8192 17.2 us whole, 22.1 in two, 14.9 in eight), up to 56 of 2048, and at 57 .. 64 not where the library's own
 // split fills the GPU ([512 x 2048] of 8192 27 us, 28.7 in two; [256 x 4096] of 10880 1.23 times).
 // More than 256 tiles and a contraction from 16384 on (NN): the library is fast where one of its tile shapes fills the CUs
 // evenly ([5120 x 49152] @ [49152 x 2048]: 1200 TFLOP/s) and at half that rate elsewhere ([4500 x 49152]: 620, in four
-// pieces 1150).  Shorter contractions are cut less readily into four and more so into two ([3584 x 16384] @ [16384 x 3072] 292
-// us, in four 332; [3200 x 32000] @ [32000 x 2048] 395, in two 522, in four 376).
+// pieces 1150).  Contractions under 24576 are never faster in four pieces than in two, and two of 129 .. 192 tiles fill two waves of
+// workgroups badly ([5465 x 16384] @ [16384 x 2048] 286 us, in two 316, in four 440; [4096 x 16384] @ [16384 x 2048] 255 and 230);
+// two of a longer one have to fill the GPU well ([3200 x 32000] @ [32000 x 2048] 395, in two 522, in four 376).
 int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   if ((M * N) % 8) return 1;   // (pico_sum_parts moves 8 elements at a time)
   auto cuts = [&](int64_t parts) { return K % parts == 0 && (K / parts) % 32 == 0; };
   int64_t most = 1, piece = 0;
   if (kind == Product::NN && tiles > 256) {
-    const bool longer = K >= 24576;
-    if (K < 16384 || tile_fit(M, N) >= (K >= 20480 ? 0.88 : 0.84)) return 1;
+    if (K < 16384 || tile_fit(M, N) >= 0.88) return 1;
     const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
+    if (K < 24576) return cuts(2) && (t256 <= 128 || t256 > 192) ? 2 : 1;
     int64_t best = 1;
     double least = 1.8;   // (of the ideal time)
     for (int64_t parts : {2, 4}) {
       if (!cuts(parts)) continue;
       const int64_t waves = (t256 * parts + 255) / 256;
       const double cost = waves * 256.0 * 65536 / (static_cast<double>(M) * N * parts) + 1040.0 * parts / K;
-      if (cost < least && (parts > 2 || cost < (longer ? 1.28 : 1.37))) {   // (two half-filled waves: 956 us at [6145 x 32000], 792 in four pieces)
+      if (cost < least && (parts > 2 || cost < 1.28)) {   // (two half-filled waves: 956 us at [6145 x 32000], 792 in four pieces)
         least = cost;
         best = parts;
       }
@@ -991,7 +992,7 @@ int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
   }
   if (kind == Product::NN && K >= 5120) {
     // (narrow outputs of the vocabulary's contraction: [4608 x 49152] @ [49152 x 768] 432 us, in four 540, in eight 346)
-    most = std::min<int64_t>(16, (N < 1024 && K >= 40000 && tiles > 128 ? 2048 : 1024) / tiles);
+    most = std::min<int64_t>(16, (N < 1024 && N % 256 == 0 && K >= 40000 && tiles > 128 ? 2048 : 1024) / tiles);
     piece = std::max<int64_t>(1280, 16 * tiles);
   } else if (kind == Product::TN && K >= 4096) {
     most = tiles < 256 ? std::min<int64_t>(K >= 16384 ? 4 : 2, 512 / tiles) : 1;
@@ -1052,8 +1053,8 @@ Tensor turned(const Tensor& t) {
 //      tiles of 128: [4096 x 1536] @ [1536 x 1024] 21, 19, but with 512 of them [4096 x 2048] @ [2048 x 2048] 37, 41;
 //   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.4, 6.8; [512 x 1536] @ [1536 x 576]^T 8.4, 8.8.
 // Over 2400 drawn products of 100 .. 8192 rows, 192 .. 49152 columns and contractions of 100 .. 49152 the time over the
-// library's was, where these lines choose the kernel, 0.76 (NN, 181 products), 0.81 (NT, 96) and 0.69 (TN, 302) in the geometric
-// mean, one over 1.03 (1.06).
+// library's was, where these lines choose the kernel, 0.75 (NN, 211 products), 0.81 (NT, 115) and 0.70 (TN, 316) in the geometric
+// mean and 1.04 at most.
 struct OwnProduct {
   int64_t groups, tile;
 };

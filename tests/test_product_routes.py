@@ -113,7 +113,9 @@ for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 
                             ("NT", 256, 4096, 10880, "library"),        # 1.23 times in 2
                             ("NT", 128, 2048, 8192, "library in 8"),    # 17.2, 22.1 in 2, 14.9
                             ("NT", 256, 3072, 12288, "library in 4"),   # 37.2, 53.7 in 2, 30.3
-                            ("NN", 3584, 3072, 16384, "library"),       # 292, 332 in 4
+                            ("NN", 4096, 2048, 16384, "library in 2"),  # 1.11 times whole
+                            ("NN", 5465, 2048, 16384, "library"),       # 286, 440 in 4
+                            ("NN", 6144, 3072, 16384, "library in 2"),  # 900, 684 in 4, 558
                             ("NN", 3200, 2048, 32000, "library in 4"),  # 395, 522 in 2, 376
                             ("NN", 4608, 768, 49152, "library in 8"),   # 432, 540 in 4, 346
                             ("NN", 512, 576, 49152, "library in 16"), ("NN", 2048, 4096, 21760, "library in 2"), ("NT", 640, 2048, 8192, "library in 2")):
