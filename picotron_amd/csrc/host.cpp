@@ -1015,19 +1015,25 @@ int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
 // lies where a sweep over contractions of 512 .. 8192 crossed ([4096 x 6144]^T [4096 x 2048]: 88 and 89 us).  Under 1024 rows
 // the product is bound by writing the result unless the narrower side leaves the library's tiles half empty.
 // (Transposing the wider operand too costs more than the second 13 %.)
-// Outputs of fewer than 384 of the library's 256 x 256 tiles stay as they are unless one side is the vocabulary's or the
-// contraction is long: its choice for the transposed layout fills the GPU worse there ([4096 x 10880]^T [4096 x 2048] 172 us,
-// transposed 273; [1280 x 12288]^T [1280 x 1536] 64 and 73), and so do short contractions that are no multiple of its step of
-// 64 ([1262 x 12288]^T [1262 x 4096] 1.06 times).  201 drawn products that are transposed took 0.90 of the library's time, five over
-// 1.04 and none over 1.13.
+// The library runs the transposed layout in tiles of 256 x 256.  With fewer than 384 of them its gain depends on how they fill
+// the GPU, unless one side is the vocabulary's: over 330 its other layout has better tiles ([4096 x 10880]^T [4096 x 2048] 172
+// us, transposed 273), up to 330 it wins outside 1152 .. 2048 rows ([1280 x 12288]^T [1280 x 1536] 64, 73; from 4096 rows 166,
+// 159), up to 256 from 1536 rows on ([4096 x 8192]^T [4096 x 2048] 124, 112), up to 230 with longer contractions and a side of
+// 8192 at least ([3266 x 9216]^T [3266 x 1152] 0.82 times, [2944 x 8192]^T [2944 x 1024] 1.03).  Short contractions that are no
+// multiple of its step of 64 lose ([1262 x 12288]^T [1262 x 4096] 1.06 times).  Of 212 drawn products that are transposed ten took
+// over 1.04 of the library's time and none over 1.13, 0.91 in the geometric mean.
 int64_t turned_operand(Product kind, const Tensor& a, const Tensor& b) {
   if (kind != Product::TN) return 0;
   const int64_t K = a.size(0), M = a.size(1), N = b.size(1), narrow = std::min(M, N), wide = std::max(M, N);
   if (narrow % 8 || (M < N ? a : b).stride(0) % 8 || (K < 1024 && (K < 768 || narrow >= 1024))) return 0;
   if (wide <= 5000 + 1e10 / (static_cast<double>(K) * narrow)) return 0;
   const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-  if (t256 < 384 && wide < 24576 && (t256 < 256 || K < 4608)) return 0;
+  const bool vocabulary = wide >= 24576;
   if (K % 64 && K < 1408 && t256 < 1024) return 0;
+  if (t256 <= 230 && !vocabulary && (wide < 8192 || K < (t256 > 160 ? 3072 : 4800))) return 0;
+  if (t256 > 230 && t256 <= 256 && !vocabulary && K < (K % 64 ? 2048 : 1536)) return 0;
+  if (t256 > 256 && t256 <= 330 && K > 1152 && K < 2048) return 0;
+  if (t256 > 330 && t256 < 384 && !vocabulary && K > 1024) return 0;
   return M < N ? 1 : 2;
 }
 // [K, N] -> [N, K], rows padded to 16 bytes

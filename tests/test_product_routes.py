@@ -126,12 +126,17 @@ for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 
 
 
 def test_weight_gradients_are_transposed_where_that_is_faster():
-    """Us whole and with the narrower operand transposed; with few output tiles or a short ragged contraction it lost up to 58 %."""
+    """Us whole and with the narrower operand transposed; in the wrong one of the two it lost up to 58 %."""
     run('''
 for K, M, N, want in ((4096, 10880, 2048, "library"),      # 172, 273
                       (1152, 10880, 2048, "library"),      # 67, 80
                       (1280, 12288, 1536, "library"),      # 64, 73
                       (1262, 12288, 4096, "library"),      # 1.06 times
+                      (4096, 6144, 2048, "library"),       # level
+                      (4096, 8192, 2048, "turned"), (4096, 2048, 8192, "turned"),   # 124, 112
+                      (1024, 10880, 2048, "turned"),       # 1.43 times whole
+                      (3266, 9216, 1152, "turned"),        # 1.23 times whole
+                      (2944, 8192, 1024, "library"),       # 1.03 times
                       (4096, 49152, 2048, "turned"),       # 732, 616
                       (4096, 2048, 16384, "turned"),       # 227, 202
                       (5504, 12288, 1536, "turned"), (4096, 49152, 576, "turned")):
