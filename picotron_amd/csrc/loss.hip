@@ -219,16 +219,27 @@ __global__ __launch_bounds__(NT, NV <= 8 ? 8 : 4) void ce_one_pass_kernel(const 
   const int wave = threadIdx.x / kWave;
   if (threadIdx.x % kWave == 0) { red_m[wave] = wm; red_s[wave] = s; }
   __syncthreads();
-  // one wave's share per lane, reduced by exchanges: read whole by every lane the shares take 2 W registers beside the row,
-  // and rows of eight pieces went to scratch ([4096, 32000] bf16 forward + backward 110 -> 103 us, [2048, 65536] 114 -> 105,
-  // [8192, 20000] 139 -> 132, fp32 the same)
-  const float pm = red_m[threadIdx.x % W];
-  float bm = pm;
+  // Rows of eight pieces and more in eight waves and more: one wave's share per lane, reduced by exchanges.  Read whole by every
+  // lane the shares take 2 W registers beside the row, and those rows went to scratch ([4096, 32000] bf16 forward + backward
+  // 110 -> 103 us, [2048, 65536] 114 -> 105, [8192, 20000] 139 -> 132, fp32 the same).  Elsewhere there is room, and reading
+  // them is 2 to 3 % faster (kernel alone, 4096 rows of 2040 pieces 54.4 us, by exchanges 56.1).
+  float bm, bs;
+  if constexpr (NV >= 8 && W >= 8) {
+    const float pm = red_m[threadIdx.x % W];
+    bm = pm;
 #pragma unroll
-  for (int off = W / 2; off > 0; off >>= 1) bm = fmaxf(bm, __shfl_xor(bm, off, kWave));
-  float bs = pm == -INFINITY ? 0.f : red_s[threadIdx.x % W] * fast_exp2(pm - bm);
+    for (int off = W / 2; off > 0; off >>= 1) bm = fmaxf(bm, __shfl_xor(bm, off, kWave));
+    bs = pm == -INFINITY ? 0.f : red_s[threadIdx.x % W] * fast_exp2(pm - bm);
 #pragma unroll
-  for (int off = W / 2; off > 0; off >>= 1) bs += __shfl_xor(bs, off, kWave);
+    for (int off = W / 2; off > 0; off >>= 1) bs += __shfl_xor(bs, off, kWave);
+  } else {
+    bm = red_m[0];
+    bs = 0.f;
+#pragma unroll
+    for (int w = 1; w < W; ++w) bm = fmaxf(bm, red_m[w]);
+#pragma unroll
+    for (int w = 0; w < W; ++w) bs += red_m[w] == -INFINITY ? 0.f : red_s[w] * fast_exp2(red_m[w] - bm);
+  }
   const float l2 = bm + fast_log2(bs);
   if (threadIdx.x == 0) {
     const float lse = l2 * kLn2;
