@@ -339,6 +339,14 @@ int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb
 int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
                  int tile, int groups, void* stream);
 
+/* The same for products that fill the GPU, in tiles of tile_m x tile_n: 256 x 256, or one side 192 or 128.  parts > 1: the
+ * contraction is cut into that many pieces, whose fp32 sums go to c [parts, M, N] (see pico_sum_parts).  Operands as above, but
+ * not with a_slow = 1 and b_slow = 0; two steps of 64 of contraction per piece at least.
+ */
+int pico_product_large_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow, int parts);
+int pico_product_large(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow,
+                       int b_slow, int tile_m, int tile_n, int parts, void* stream);
+
 /* y[c][r] = x[r][c] for bf16 x [rows, cols] with row pitch x_pitch and y [cols, rows] with row pitch y_pitch (elements).  cols
  * and both pitches must be multiples of 8, pointers 16-byte aligned; where rows is no multiple of 8, zeros follow a row of y
  * up to the next multiple.  Lays an operand of a weight gradient out as the GEMM library reads it faster.

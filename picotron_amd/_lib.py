@@ -83,6 +83,8 @@ SIGNATURES = {
     "pico_sum_parts": (c_int, [_P, _P, _I64, _I64, c_int, _P]),
     "pico_product_takes": (c_int, [_I64] * 5 + [c_int, c_int]),
     "pico_product": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
+    "pico_product_large_takes": (c_int, [_I64] * 5 + [c_int, c_int, c_int]),
+    "pico_product_large": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, c_int, _P]),
     "pico_transpose": (c_int, [_P, _P, _I64, _I64, _I64, _I64, _P]),
     "pico_embedding_bwd_workspace_bytes": (_I64, [_I64, _I64]),
     "pico_embedding_bwd": (c_int, [_P, c_int, _P, _P, _P, _I64, _I64, _I64, _I64, c_int, _P]),

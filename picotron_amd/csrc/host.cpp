@@ -1084,6 +1084,85 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
   return K <= (tiles > 128 ? 3072 : tiles > 60 ? 1088 : 0) ? OwnProduct{2, 64} : no;
 }
 
+// Whether a product goes to the package's kernel for products that fill the GPU (pico_product_large), in which tiles and in how
+// many pieces of the contraction (parts 0: no).
+//
+// The kernel's own time follows from its rounds: 256 workgroups take a tile each, a step of 64 of contraction costs 1.0 .. 1.4
+// us (less while part of the GPU idles), a tile's end 2 .. 5 us.  The estimate below has an error of 7 % (standard deviation)
+// over 20000 timed (shape, tile, pieces); the tile it takes is on average 0.7 % slower than the best one.  Against that stands
+// an estimate of the time without it, of the same form, whose error is 11 .. 34 %: the library's choices are not monotone in
+// any size.  So the lines ask for a margin where the library is good, and for none where it never is.  Of 2100 drawn products of
+// 100 .. 8192 rows those that go here took, in the geometric mean of the time without it,
+//   TN: 0.69 where the library ran them as they are (217 products, 0.99 at most; [4096 x 4096]^T [4096 x 4096] 137 -> 103
+//     us), 0.83 where it had an operand transposed first (91, 1.03 at most; [4096 x 16384]^T [4096 x 2048] 216 -> 199), 0.86 where
+//     pico_product did (13); under 640 of contraction that one stays ahead ([512 x 49152]^T [512 x 576] 45 us, here 52), and the
+//     library where the vocabulary meets fewer than 256 columns ([7358 x 49152]^T [7358 x 128] 161 us, here 179);
+//   NN: 0.80 (143, 1.06 at most; [2242 x 10880] @ [10880 x 4096] 248 -> 178, [608 x 49152] @ [49152 x 576] 84 -> 55); a margin is
+//     asked for pieces of four and up, whose rows of a large pitch come more slowly than the estimate has it, and for short
+//     products ([4548 x 1024] @ [1024 x 1024] 17 us, here 20);
+//   NT: 0.77 (42, 1.02 at most): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
+//     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
+//     16384]^T 424 -> 206).
+struct LargeProduct {
+  int64_t tile_m = 0, tile_n = 0, parts = 0;
+};
+double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
+  struct Form {
+    int64_t m, n;
+    double step, end;
+  };
+  static constexpr Form forms[] = {{256, 256, 1.43, 4.8}, {256, 192, 1.2, 4.4}, {192, 256, 1.2, 3.2}, {256, 128, 0.99, 2.4}, {128, 256, 1.0, 1.6}};
+  const int64_t steps = (K + 63) / 64;
+  double least = 1e30;
+  for (const Form& f : forms) {
+    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
+    for (int64_t parts : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+      if (parts > 1 && (tiles * parts > 300 || steps < 8 * parts)) break;
+      const int64_t full = tiles * parts / 256, rest = tiles * parts % 256, length = (steps + parts - 1) / parts;
+      const double used = rest / 256.0;   // of the GPU, in the last round
+      double t = 5 + full * (length * f.step + f.end);
+      if (rest) t += length * f.step * (0.7 + 0.3 * used) + f.end * (0.45 + 0.55 * used);
+      if (parts > 1) t += 3.8 + 1e-6 * M * N * (0.63 * parts + 0.16);   // the pieces in fp32, and their sum
+      if (t < least) {
+        least = t;
+        best = {f.m, f.n, parts};
+      }
+    }
+  }
+  return least;
+}
+// the same without it: the library's tiles (NT, NN), or pico_product's (TN)
+double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
+  struct Form {
+    int64_t m, n;
+    double step[3];   // NT, NN, TN
+  };
+  static constexpr Form forms[] = {{256, 256, {1.37, 1.45, 3.0}}, {256, 192, {1.16, 1.2, 2.0}}, {192, 256, {1.16, 1.2, 2.0}}, {256, 128, {0.72, 0.83, 1.7}},
+                                   {128, 256, {0.72, 0.83, 1.7}}, {128, 128, {0.41, 0.51, 0.88}}, {64, 128, {0.22, 0.19, 0.27}}, {128, 64, {0.22, 0.19, 0.27}}};
+  static constexpr double start[3] = {-1.6, 8.6, 2.2}, end[3] = {8.8, 2.3, 2.4};
+  const int k = static_cast<int>(kind);
+  double least = 1e30;
+  for (const Form& f : forms) {
+    const int64_t rounds = (((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n) + 255) / 256;
+    least = std::min(least, rounds * (K / 64.0 * f.step[k] + end[k]));
+  }
+  return start[k] + least;
+}
+LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
+  static_assert(static_cast<int>(Product::NT) == 0 && static_cast<int>(Product::NN) == 1 && static_cast<int>(Product::TN) == 2);
+  const int64_t narrow = std::min(M, N), wide = std::max(M, N);
+  LargeProduct best;
+  if (M < 1 || N < 1 || K < 128 || narrow < 192 || (wide >= 24576 && narrow < 256)) return {};
+  const double time = large_time(M, N, K, best), ideal = 2e-9 * M * N * K;   // (us at 1 PFLOP/s)
+  const bool small = own_product(kind, M, N, K).groups > 0;
+  bool take = false;
+  if (kind == Product::TN) take = !small || (K >= 640 && time < 0.9 * other_time(kind, M, N, K));
+  else if (small || time < 14) take = false;
+  else if (kind == Product::NN) take = time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05);
+  else take = time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal);
+  return take ? best : LargeProduct{};
+}
+
 struct ProductSizes {
   int64_t M, N, K;
 };
@@ -1106,14 +1185,31 @@ OwnProduct own_product(Product kind, const ProductSizes& n, const Tensor& a, con
   return own;
 }
 
-// parts 0, turn -1, groups -1: by the rules above
-Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64) {
+LargeProduct large_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b) {
+  const LargeProduct large = large_product(kind, n.M, n.N, n.K);
+  const bool takes = large.parts > 0 && pico_product_large_takes(n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
+                                                                 static_cast<int>(large.parts));
+  return takes ? large : LargeProduct{};
+}
+
+// parts 0, turn -1, groups -1, tile_n 0: by the rules above
+Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64, int64_t tile_n = 0) {
   if (!stays_with_torch(a, b)) {
     const c10::OptionalDeviceGuard device(a.device());
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
     const ProductSizes n = product_sizes(a, b, kind);
     const auto [M, N, K] = n;
     Tensor c = at::empty({M, N}, a.options());
+    LargeProduct large = {tile, tile_n, std::max<int64_t>(parts, 1)};
+    if (tile_n == 0) large = parts == 0 && turn < 0 && groups < 0 ? large_product(kind, n, a, b) : LargeProduct{};
+    if (large.tile_n > 0) {
+      parts = large.parts;
+      const Tensor sums = parts > 1 ? at::empty({parts, M, N}, a.options().dtype(at::kFloat)) : Tensor();
+      check(pico_product_large(ptr(a), ptr(b), parts > 1 ? ptr(sums) : ptr(c), M, N, K, a.stride(0), b.stride(0), kind == Product::TN,
+                               kind != Product::NT, static_cast<int>(large.tile_m), static_cast<int>(large.tile_n), static_cast<int>(parts), stream_now()));
+      if (parts > 1) check(pico_sum_parts(fptr(sums), ptr(c), parts, M * N, PICO_BF16, stream_now()));
+      return c;
+    }
     if (groups < 0) {
       const OwnProduct own = parts == 0 && turn < 0 ? own_product(kind, n, a, b) : OwnProduct{0, 64};
       groups = own.groups;
@@ -1143,7 +1239,7 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
   return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
 }
 
-// the route of a product, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
+// the route of a product that large_product leaves alone, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
 // "library in N" pieces
 std::string product_route(const Tensor& a, const Tensor& b, Product kind) {
   if (stays_with_torch(a, b)) return "torch";
@@ -1578,10 +1674,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   };
   m.def("product_route", [=](const Tensor& a, const Tensor& b, const std::string& kind) { return product_route(a, b, product_kind(kind)); },
         pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"));
-  m.def("product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile) {
-    return product(a, b, product_kind(kind), parts, turn, groups, tile);
+  m.def("large_product", [=](const Tensor& a, const Tensor& b, const std::string& kind) {
+    const LargeProduct large = stays_with_torch(a, b) ? LargeProduct{} : large_product(product_kind(kind), product_sizes(a, b, product_kind(kind)), a, b);
+    return std::make_tuple(large.tile_m, large.tile_n, large.parts);
+  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"));
+  m.def("product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile, int64_t tile_n) {
+    return product(a, b, product_kind(kind), parts, turn, groups, tile, tile_n);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
-        pybind11::arg("groups") = -1, pybind11::arg("tile") = 64);
+        pybind11::arg("groups") = -1, pybind11::arg("tile") = 64, pybind11::arg("tile_n") = 0);
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("embedding", &embedding, nogil());

@@ -127,3 +127,28 @@ def test_linear_on_columns_of_a_wider_buffer(device, rows, cin, cout, pad):
     yf = torch.nn.functional.linear(xf, wf)
     for a, b in zip(got, (yf, *torch.autograd.grad(yf, (xf, wf), dy.float()))):
         assert a.shape == b.shape and ((a.float() - b).norm() / b.norm()).item() <= 3e-3
+
+
+@pytest.mark.parametrize("kind,M,N,K", [
+    ("NT", 1, 8, 72), ("NT", 257, 264, 128), ("NT", 255, 200, 136), ("NT", 700, 520, 1000), ("NT", 2100, 4360, 328),
+    ("NN", 1, 8, 72), ("NN", 257, 264, 128), ("NN", 255, 200, 136), ("NN", 700, 520, 1000), ("NN", 2100, 4360, 328),
+    ("TN", 8, 8, 65), ("TN", 264, 256, 129), ("TN", 248, 200, 133), ("TN", 704, 520, 1001), ("TN", 4360, 2104, 331)])
+def test_large_products(device, kind, M, N, K):
+    """The kernel for products that fill the GPU: edges of its tiles and steps, more tiles than workgroups, pieces of unequal
+    length, wider row pitches."""
+    from picotron_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(M * N + K)
+    shapes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    for pad in (0, 24):
+        a, b = (torch.randn(r, c + pad, generator=g, device=device).to(torch.bfloat16)[:, :c] for r, c in shapes)
+        ai, bi = a.round(), b.round()            # small integers: sums are exact in fp32
+        want, exact = ((x.float().t() if kind == "TN" else x.float()) @ (y.float().t() if kind == "NT" else y.float()) for x, y in ((a, b), (ai, bi)))
+        for tile, tile_n in ((256, 256), (256, 192), (192, 256), (256, 128), (128, 256)):
+            for parts in (1, 2, 5):
+                if (K + 63) // 64 < 2 * parts:
+                    continue
+                got = _lib.host().product(a, b, kind, parts, tile=tile, tile_n=tile_n)
+                assert got.shape == (M, N) and got.dtype == torch.bfloat16
+                assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (pad, tile, tile_n, parts)
+                assert torch.equal(got, _lib.host().product(a, b, kind, parts, tile=tile, tile_n=tile_n))
+                assert torch.equal(_lib.host().product(ai, bi, kind, parts, tile=tile, tile_n=tile_n), exact.to(torch.bfloat16))

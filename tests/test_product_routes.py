@@ -143,3 +143,51 @@ for K, M, N, want in ((4096, 10880, 2048, "library"),      # 172, 273
     got = host.product_route(operand(K, M), operand(K, N), "TN")
     assert got == want, (K, M, N, got)
 ''')
+
+
+def test_the_large_predicate_is_what_the_kernel_refuses():
+    """pico_product_large_takes against pico_product_large itself: with NULL operands an accepted shape ends at the pointers."""
+    from picotron_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    lib, seen = _lib.lib(), set()
+    for M, N, K in ((1, 8, 64), (1, 8, 72), (512, 576, 576), (512, 576, 580), (516, 576, 576), (512, 580, 576), (2331, 1024, 2331)):
+        for a_slow, b_slow in ((0, 0), (0, 1), (1, 0), (1, 1)):
+            for pad_a in (0, 4, 8, -8, 1 << 23, 1 << 31):
+                for pad_b in (0, 4, 8, 1 << 23):
+                    for parts in (0, 1, 4, 5, 65):
+                        lda, ldb = (M if a_slow else K) + pad_a, (N if b_slow else K) + pad_b
+                        takes = lib.pico_product_large_takes(M, N, K, lda, ldb, a_slow, b_slow, parts)
+                        rc = lib.pico_product_large(None, None, None, M, N, K, lda, ldb, a_slow, b_slow, 256, 256, parts, None)
+                        assert rc == (-1 if takes else -3), (M, N, K, lda, ldb, a_slow, b_slow, parts)
+                        seen.add(takes)
+    assert seen == {0, 1}
+    assert lib.pico_product_large(1 << 20, 1 << 20, 1 << 20, 512, 576, 576, 576, 576, 0, 0, 128, 128, 1, None) == -3
+
+
+def test_products_that_fill_the_gpu_go_to_their_kernel_where_it_is_faster():
+    """(rows and columns of a tile, pieces of the contraction), or none; us without and with the kernel."""
+    run('''
+none = (0, 0, 0)
+for kind, M, N, K, want in (("TN", 4096, 4096, 4096, (256, 256, 1)),       # 137, 103
+                            ("TN", 6144, 2048, 4096, (192, 256, 1)),       # 101, 91
+                            ("TN", 16384, 2048, 4096, (256, 256, 1)),      # 216, 199
+                            ("TN", 49152, 576, 512, none),                 # 45, 52
+                            ("TN", 49152, 128, 7358, none),                # 161, 179
+                            ("TN", 2048, 2048, 4096, none),                # 42, 51
+                            ("NN", 2242, 10880, 4096, (256, 256, 1)),      # 248, 178
+                            ("NN", 608, 576, 49152, (256, 192, 24)),       # 84, 55
+                            ("NN", 4548, 1024, 1024, none),                # 17, 20
+                            ("NN", 2886, 3072, 49152, none),               # 785, 846
+                            ("NT", 3832, 49152, 512, (256, 256, 1)),       # 315, 218
+                            ("NT", 5856, 6144, 768, (192, 256, 1)),        # 79, 52
+                            ("NT", 4096, 16384, 2048, none),               # 194, 203
+                            ("NT", 512, 576, 576, none)):
+    (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    got = host.large_product(operand(ra, ca), operand(rb, cb), kind)
+    assert got == want, (kind, M, N, K, got)
+    if want != none:                                  # pitches that the kernel refuses
+        assert host.large_product(operand(ra, ca, ca + 4), operand(rb, cb), kind) == none
+        assert host.large_product(operand(ra, ca), operand(rb, cb, cb + (1 << 24)), kind) == none
+        assert host.large_product(operand(ra, ca, ca + 8), operand(rb, cb, cb + 24), kind) == want
+''')
