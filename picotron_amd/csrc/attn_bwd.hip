@@ -51,7 +51,9 @@ constexpr bool kStreamGrads = true;
 // 64-query tile between them, one 32-query sub-block each, with accumulators of their own that are added through LDS
 // at the end of the key tile.  A wave then holds one sub-block's S / dP tiles instead of two, which is what lets the
 // head_dim 128 kernel fit 256 registers, i.e. two waves per SIMD.
-constexpr int kPairKRegs = 4;   // PAIR: K fragments (of D / 16) that stay in registers; the others are read from LDS
+// PAIR: K fragments (of D / 16) that stay in registers; the others are read from LDS.  As many as fit: 4 -> 7 with the registers
+// that staging the tiles took, 3 % at B1 H32 S4096.
+constexpr int kPairKRegs = 7;
 
 template <int D, bool PAIR = false>
 struct KvCfg {
@@ -67,8 +69,13 @@ struct KvCfg {
   // pieces of 4 consecutive rows tile the banks (transposed reads at their minimum of 2 requests per bank; at a pitch
   // of D + 8 they take 3-4), and the 4-word skew per 4 rows spreads 16 consecutive rows over all multiples of 4 words
   // (row reads at their minimum of 4).
-  static constexpr int LDQ = D + 32;
-  static constexpr int kSkew = 8;
+  // PAIR: the tiles are filled by loads that go to LDS directly, 1 KiB of consecutive addresses per wave, so their rows are
+  // dense; the 16-byte pieces of a row change places instead (tile_twist), which spreads both kinds of read as evenly.
+  // (The loop is paced by LDS reads and their latency, the matrix cores are busy for half of it: without the LDS writes and
+  // with more of K in registers B1 H32 S4096 281 -> 271 us, H32/8 S8192 1000 -> 950.  At head_dim 64 a wave's two sub-blocks take
+  // all 256 registers, and the flipped addresses of this layout end up in scratch: S4096 143 -> 156 us, so it keeps the pitch.)
+  static constexpr int LDQ = PAIR ? D : D + 32;
+  static constexpr int kSkew = PAIR ? 0 : 8;
   static constexpr int kTileElems = BM * LDQ + kSkew * (BM / 4);       // one tile
   static constexpr int kTrStep = 8 * LDQ + 2 * kSkew;                  // 8 rows further down
   static constexpr int kVecPerRow = D / 8;
@@ -200,7 +207,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     tile_first += t0 - skip * tiles_per_head;
   }
 
-  // Global -> register prefetch of a Q / dO tile (+ lse, delta) with buffer loads.  A cursor (wave-uniform:
+  // Loads of a Q / dO tile (+ lse, delta) into registers, PAIR: of the tile straight to LDS.  A cursor (wave-uniform:
   // it lives in scalar registers) walks the trip space; stepping to the next tile of the same head is a few
   // scalar adds, only a change of head recomputes addresses.  The per-lane byte offsets are computed once,
   // and rows past Sq read as zeros because they lie past the end of the buffer window.  Every instruction
@@ -211,7 +218,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
   for (int i = 0; i < C::kQLoads; ++i) {
     const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
+    const int r = idx / C::kVecPerRow, cv = PAIR ? idx % C::kVecPerRow ^ tile_twist<D>(r) : idx % C::kVecPerRow;
     q_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.qs[2] + cv * 8) * 2);
     do_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.os[2] + cv * 8) * 2);
   }
@@ -246,13 +253,25 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       cur.lse += BM;  cur.delta += BM;  cur.rows_left -= BM * 4;
     }
   };
+  // PAIR: the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
+  auto request_tile = [&](uint32_t buf_off) {
+    const u32x4 qb = request_window(reinterpret_cast<uint64_t>(cur.q), cur.q_left), dob = request_window(reinterpret_cast<uint64_t>(cur.dout), cur.do_left);
+    const uint32_t to = buf_off + __builtin_amdgcn_readfirstlane(wave_id) * 1024;
+    static_assert(!PAIR || C::kQLoads == 2);
+    request16_to<0>(to, qb, q_off[0]);
+    request16_to<C::kThreads * 16>(to, qb, q_off[C::kQLoads - 1]);
+    request16_to<C::kTileElems * 2>(to, dob, do_off[0]);
+    request16_to<C::kTileElems * 2 + C::kThreads * 16>(to, dob, do_off[C::kQLoads - 1]);
+  };
   auto prefetch = [&]() {  // the tile under the cursor
-    const buffer_rsrc qb = make_buffer(cur.q, cur.q_left), dob = make_buffer(cur.dout, cur.do_left);
     const buffer_rsrc lb = make_buffer(cur.lse, cur.rows_left), db = make_buffer(cur.delta, cur.rows_left);
+    if constexpr (!PAIR) {
+      const buffer_rsrc qb = make_buffer(cur.q, cur.q_left), dob = make_buffer(cur.dout, cur.do_left);
 #pragma unroll
-    for (int i = 0; i < C::kQLoads; ++i) {
-      qreg[i] = buffer_load_b128(qb, q_off[i]);
-      doreg[i] = buffer_load_b128(dob, do_off[i]);
+      for (int i = 0; i < C::kQLoads; ++i) {
+        qreg[i] = buffer_load_b128(qb, q_off[i]);
+        doreg[i] = buffer_load_b128(dob, do_off[i]);
+      }
     }
     lreg = buffer_load_f32(lb, row_off);
     dreg = buffer_load_f32(db, row_off);
@@ -262,13 +281,14 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     __bf16* sdO = sQ + C::kTileElems;
     float* sL = reinterpret_cast<float*>(sdO + C::kTileElems);
     float* sDelta = sL + BM;
+    if constexpr (!PAIR)
 #pragma unroll
-    for (int i = 0; i < C::kQLoads; ++i) {
-      const int idx = tid + i * C::kThreads;
-      const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-      *reinterpret_cast<u32x4*>(&sQ[tile_row(r) + cv * 8]) = qreg[i];
-      *reinterpret_cast<u32x4*>(&sdO[tile_row(r) + cv * 8]) = doreg[i];
-    }
+      for (int i = 0; i < C::kQLoads; ++i) {
+        const int idx = tid + i * C::kThreads;
+        const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
+        *reinterpret_cast<u32x4*>(&sQ[tile_row(r) + cv * 8]) = qreg[i];
+        *reinterpret_cast<u32x4*>(&sdO[tile_row(r) + cv * 8]) = doreg[i];
+      }
     if (tid < BM) {
       // rows past Sq, and rows whose lse is -inf (they saw no key), get lse = +inf so that P = 0
       const bool live = static_cast<uint32_t>(tid) * 4u < cur.rows_left && lreg != -INFINITY;
@@ -280,6 +300,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   if (n_iter > 0) {
     seek(head_first, tile_first);
     prefetch();
+    if constexpr (PAIR) request_tile(0);
   }
   if (loads_kv) {
     if constexpr (!PAIR) {
@@ -299,21 +320,11 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     for (int j = 0; j < kPairKRegs; ++j) kf[j] = *reinterpret_cast<const bf16x8*>(pair_k + n * kFragPitch + (16 * j + 8 * h) * 2);
   }
   if (n_iter > 0) stage(0);
-  // The K / V fragment loads above are complete by now on every path that enters the loop (the LDS fill
-  // waited for all loads), but not on the static path that skips the fill; saying so here keeps the compiler
-  // from putting a vmcnt(0) wait in front of the loop's first MFMAs, where it would wait for the prefetch
-  // of the NEXT tile on every trip.
+  // All loads above are complete from here on (PAIR: also the first tile, which the barrier publishes).  Saying so
+  // keeps the compiler from putting a vmcnt(0) wait in front of the loop's first MFMAs, where it would wait for the
+  // NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
-  // PAIR: the tile after the one being computed goes to LDS at the TOP of a trip, from loads that
-  // were issued at the top of the trip before; the registers are then reloaded with the tile after that.  The LDS
-  // writes are off the end of the trip (where every wave of the workgroup would wait for them in front of the barrier)
-  // and a load has a whole trip to arrive.
-  constexpr bool kStageTop = PAIR;
-  if constexpr (kStageTop) {
-    if (n_iter > 1) { advance(); prefetch(); }
-  }
-
   const int kw0 = key0 + 32 * wave;
   int tile = tile_first;     // query tile (within its head) of the trip being computed
   uint32_t buf_off = 0;      // byte offset of the LDS buffer being read
@@ -321,19 +332,22 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // tile it+1 travels global -> registers while this trip computes; it goes to the other LDS buffer at
     // the end of the trip (that buffer's readers finished before the barrier that ended trip it-1)
     const bool has_next = it + 1 < n_iter;
-    if constexpr (kStageTop) {
+    // PAIR: it goes there directly, and is requested at the top of the trip
+    if (has_next) advance();
+    if constexpr (PAIR) {
       if (has_next) {
-        stage(buf_off == 0);   // tile it+1 (the cursor is on it)
-        if (it + 2 < n_iter) { advance(); prefetch(); }
+        prefetch();
+        request_tile(buf_off ^ static_cast<uint32_t>(C::kBufBytes));
       }
-    } else {
-      if (has_next) advance();
     }
     const int q0 = tile * BM;
     const __bf16* sQ = reinterpret_cast<const __bf16*>(smem_raw + buf_off);
     const __bf16* sdO = sQ + C::kTileElems;
     const float* sL = reinterpret_cast<const float*>(sdO + C::kTileElems);
     const float* sDelta = sL + BM;
+    // (PAIR) this lane's place in the tile of this trip: other pieces are reached by flipping bits of the address
+    const uint32_t row_lane = buf_off + row_place<D>(lane), tr_lane = buf_off + column_place<D>(lane);
+    static_assert(!PAIR || C::kBufBytes % 256 == 0);
 
     // The three phases of a 32-query sub-block.
     // products(): S = Q K^T and dP = dO V^T (C tile: lane = key, registers = queries); the dP accumulator starts at
@@ -349,12 +363,12 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         // both operands of every MFMA come from LDS: they are requested kAhead steps before the MFMAs that use them, and
         // the scheduling barriers keep that order (left alone, the compiler reuses one set of registers and every MFMA
         // waits for an LDS round trip)
-        constexpr int kSteps = D / 16, kAhead = 1;
+        constexpr int kSteps = D / 16, kAhead = 2;
         bf16x8 qa[kSteps], da[kSteps], kb[kSteps], vb[kSteps];
         auto fetch = [&](int j) {
-          qa[j] = *reinterpret_cast<const bf16x8*>(&sQ[tile_row(32 * sb + n) + 16 * j + 8 * h]);
+          qa[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2);
           if (j >= kPairKRegs) kb[j] = *reinterpret_cast<const bf16x8*>(pair_k + n * kFragPitch + (16 * j + 8 * h) * 2);
-          da[j] = *reinterpret_cast<const bf16x8*>(&sdO[tile_row(32 * sb + n) + 16 * j + 8 * h]);
+          da[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2 + C::kTileElems * 2);
           vb[j] = *reinterpret_cast<const bf16x8*>(pair_v + n * kFragPitch + (16 * j + 8 * h) * 2);
         };
 #pragma unroll
@@ -407,10 +421,10 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         bf16x8 dof[kSlots], qf[kSlots];
         auto fetch = [&](int idx) {
           const int cc = idx / (D / 32), db = idx % (D / 32);
-          const int qr = 32 * sb + 16 * cc + 4 * h + (lane % 16) / 4;
-          const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
-          dof[idx] = lds_read_tr_pair_step(&sdO[tile_row(qr) + col], C::kTrStep);
-          qf[idx] = lds_read_tr_pair_step(&sQ[tile_row(qr) + col], C::kTrStep);
+          // rows 8 further down have their pieces at other places
+          const unsigned char *lo = smem_raw + (tr_lane ^ 64 * db) + (32 * sb + 16 * cc) * D * 2, *hi = smem_raw + (tr_lane ^ (64 * db + 32)) + (32 * sb + 16 * cc + 8) * D * 2;
+          dof[idx] = lds_read_tr_two(lo + C::kTileElems * 2, hi + C::kTileElems * 2);
+          qf[idx] = lds_read_tr_two(lo, hi);
         };
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) fetch(j);
@@ -445,7 +459,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     };
 
     const bool off_diagonal = !PAIR && (!a.causal || kw0 + 31 <= a.q_offset + q0);
-    if (!kStageTop && has_next && !off_diagonal) prefetch();
+    if (!PAIR && has_next && !off_diagonal) prefetch();
     if (off_diagonal) {
       // Every pair of this trip is visible to this wave (all trips off the diagonal): straight-line code in an order
       // that lets the wave's own phases overlap -- the matrix pipe works on the second sub-block's S / dP while the
@@ -558,7 +572,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
     }
     buf_off ^= static_cast<uint32_t>(C::kBufBytes);
-    if (!kStageTop && has_next) stage(buf_off != 0);
+    if (has_next) stage(buf_off != 0);
+    if constexpr (PAIR) wait_requests<0>();
     tile = tile + 1 == n_qtiles ? qt_start : tile + 1;
     __syncthreads();  // all waves are done with the buffer just read (refilled in the next trip) and the next tile is visible
   }
@@ -690,17 +705,20 @@ struct DqCfg {
   static_assert(NW % KS == 0 && (KS == 1 || KT == 64 * KS), "one 64-key step of every staged tile per key-split wave");
   static constexpr int BN = 64;            // keys per compute step
   static constexpr int kKT = KT;
-  static constexpr int LDK = D + 8;        // pitch of the K and V tiles
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;
-  static constexpr int kTileElems = 2 * KT * LDK;
-  static constexpr size_t kLdsBytes = 2 * kTileElems * sizeof(__bf16);  // double-buffered
+  static constexpr int kTileElems = 2 * KT * D;   // K, then V
   // workgroups that share a CU: the register budget and the plan go by it (at head_dim 128 a lane needs more than the 256
   // registers that two would leave it: with some in scratch 77 -> 121 us at one head of 3000 rows)
   static constexpr int kPerCu = NW <= 4 && D <= 64 ? 2 : 1;
+  // the tiles, double-buffered; the Q / dO fragments pass through LDS behind them where there is room, so that the first tile is
+  // requested at once, and through the tile buffers otherwise
+  static constexpr size_t kTiles = 2 * kTileElems * sizeof(__bf16), kFragmentBytes = NW * WaveTile<D>::kRegionBytes;
+  static constexpr bool kBehind = kPerCu * (kTiles + kFragmentBytes) <= 160 * 1024;
+  static constexpr size_t kFragments = kBehind ? kTiles : 0, kLdsBytes = kTiles + (kBehind ? kFragmentBytes : 0);
+  static_assert(kFragmentBytes <= kLdsBytes);
   static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   static_assert(NW * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
-  static_assert(NW * WaveTile<D>::kRegionBytes <= kLdsBytes, "the Q / dO fragments pass through the tile buffers");
   static_assert(KT % BN == 0 && (KT * kVecPerRow) % kThreads == 0, "tile must split evenly over the threads");
   static constexpr size_t kExchangeBytes = (D / 32) * 16 * 64 * 4;   // a wave's dQ^T accumulators
   static_assert(KS == 1 || NW * kExchangeBytes <= kLdsBytes, "the exchange reuses the tile buffers");
@@ -725,9 +743,8 @@ __device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* regi
 template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) void attn_bwd_dq_kernel(const BwdParams p) {
   using C = DqCfg<D, NW, KT, KS>;
-  constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK;
+  constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  __bf16* smem = reinterpret_cast<__bf16*>(smem_raw);
 
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
@@ -744,6 +761,51 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   const int n = lane % 32, h = lane / 32;
   const int qw = wave % C::kQWaves, ks = wave / C::kQWaves;   // which queries, which 64-key step of a staged tile
   const float c = a.sm_scale * kLog2e;
+
+  // ---- key range of this query tile
+  const int q_hi = (q0 + BM < a.Sq ? q0 + BM : a.Sq);
+  int kv_end = a.Sk;
+  if (a.causal) {
+    const int vis = a.q_offset + q_hi;
+    kv_end = vis < a.Sk ? vis : a.Sk;
+    if (kv_end < 0) kv_end = 0;
+  }
+  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
+  if (kCut && piece.parts > 1) {
+    t_first = ntiles * piece.part / piece.parts;
+    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
+  }
+
+  // K / V tiles go straight to LDS, like in the forward kernel (rows past Sk read as zeros).  Besides the LDS writes at the end
+  // of a trip this saves the registers of the tile: B1 H32 S4096 D128 212 -> 195 us, H32/8 S8192 720 -> 669; level at head_dim 64.
+  uint32_t k_off[C::kLoads], v_off[C::kLoads];
+#pragma unroll
+  for (int i = 0; i < C::kLoads; ++i) {
+    const int idx = tid + i * C::kThreads;
+    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow ^ tile_twist<D>(r);
+    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
+    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
+  }
+  // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
+  KvCursor<D> cur;
+  cur.open(a, t_first, b, hkv, KT);
+  KvPosition pos;
+  pos.open(a.kv, t_first, KT);
+  // the next tile goes to LDS buffer `buf`
+  auto request_tile = [&](int buf) {
+    const u32x4 kb = request_window(reinterpret_cast<uint64_t>(cur.k), cur.k_left), vb = request_window(reinterpret_cast<uint64_t>(cur.v), cur.v_left);
+    const uint32_t to = static_cast<uint32_t>(buf) * (C::kTileElems * 2) + wave * 1024;
+    each_load<C::kLoads>([&](auto load) {
+      constexpr int i = decltype(load)::value;
+      request16_to<i * C::kThreads * 16>(to, kb, k_off[i]);
+      request16_to<KT * D * 2 + i * C::kThreads * 16>(to, vb, v_off[i]);
+    });
+    cur.next(a);
+  };
+
+  if constexpr (C::kBehind) {
+    if (ntiles > 0) request_tile(0);
+  }
 
   // ---- per-lane query: Q and dO fragments (B operands: fetched row-major, turned into fragments through the
   //      wave's piece of LDS; the tile buffers are filled only after the barrier below), lse and delta
@@ -768,7 +830,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
       lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;  // a row that saw no key contributes nothing
       if constexpr (!kDelta) delta = p.delta[gi];
     }
-    unsigned char* region = smem_raw + wave * WaveTile<D>::kRegionBytes;
+    unsigned char* region = smem_raw + C::kFragments + wave * WaveTile<D>::kRegionBytes;
     qt.fragments(region, lane, qf);
     dt.fragments(region, lane, dof);
     if constexpr (kDelta) {
@@ -792,85 +854,38 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] = 0.f;
 
-  // ---- key range of this query tile
-  const int q_hi = (q0 + BM < a.Sq ? q0 + BM : a.Sq);
-  int kv_end = a.Sk;
-  if (a.causal) {
-    const int vis = a.q_offset + q_hi;
-    kv_end = vis < a.Sk ? vis : a.Sk;
-    if (kv_end < 0) kv_end = 0;
+  if constexpr (!C::kBehind) {
+    __syncthreads();  // every wave has its Q / dO fragments: the tile buffers may be filled
+    if (ntiles > 0) request_tile(0);
   }
-  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
-  if (kCut && piece.parts > 1) {
-    t_first = ntiles * piece.part / piece.parts;
-    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
-  }
-
-  // K / V tiles travel global -> registers -> LDS with buffer loads (wave-uniform resource per tile, per-lane
-  // byte offsets computed once, rows past Sk read as zeros)
-  u32x4 kreg[C::kLoads], vreg[C::kLoads];
-  uint32_t k_off[C::kLoads], v_off[C::kLoads];
-#pragma unroll
-  for (int i = 0; i < C::kLoads; ++i) {
-    const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
-    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
-  }
-  // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
-  KvCursor<D> cur;
-  cur.open(a, t_first, b, hkv, KT);
-  KvPosition pos;
-  pos.open(a.kv, t_first, KT);
-  auto load_tile = [&]() {  // the next tile of KT keys
-    const buffer_rsrc kb = make_buffer(cur.k, cur.k_left), vb = make_buffer(cur.v, cur.v_left);
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      kreg[i] = buffer_load_b128(kb, k_off[i]);
-      vreg[i] = buffer_load_b128(vb, v_off[i]);
-    }
-    cur.next(a);
-  };
-  auto store_tile = [&](int buf) {
-    __bf16* sK = smem + buf * C::kTileElems;
-    __bf16* sV = sK + KT * LDK;
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      const int idx = tid + i * C::kThreads;
-      const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-      *reinterpret_cast<u32x4*>(&sK[r * LDK + cv * 8]) = kreg[i];
-      *reinterpret_cast<u32x4*>(&sV[r * LDK + cv * 8]) = vreg[i];
-    }
-  };
-
-  if (ntiles > 0) load_tile();
-  __syncthreads();  // every wave has its Q / dO fragments: the tile buffers may be filled
-  if (ntiles > 0) store_tile(0);
-  // all loads so far are complete on every path into the loop (the LDS fill waited for the newest); stating
-  // it keeps a vmcnt(0) wait, which would hit the next tile's prefetch, out of the loop body
+  // all loads so far are complete, the first tile among them (the barrier publishes it); stating it also keeps a
+  // vmcnt(0) wait, which would hit the next tile's requests, out of the loop body
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-  if (ntiles > 1) load_tile();
   __syncthreads();
+
+  uint32_t row_at[D / 16], tr_at[D / 16];   // the lane's places in a tile (see the forward kernel)
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) {
+    row_at[s] = row_place<D>(lane) ^ 32 * s;
+    tr_at[s] = column_place<D>(lane) ^ 32 * s;
+    asm volatile("" : "+v"(row_at[s]), "+v"(tr_at[s]));   // (kept, not computed again in front of every read)
+  }
 
   const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
   const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
-  for (int t = 0; t < ntiles; ++t) {
+  // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
+  auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
+    constexpr uint32_t kAt = decltype(parity)::value * C::kTileElems * 2;
+    static_assert(kAt + C::kTileElems * 2 <= 65536, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
-    if (t + 1 < ntiles) {
-      store_tile((t + 1) & 1);
-      if (t + 2 < ntiles) load_tile();
-    }
-    const __bf16* sK = smem + (t & 1) * C::kTileElems;
-    const __bf16* sV = sK + KT * LDK;
+    if (t + 1 < ntiles) request_tile(1 - decltype(parity)::value);
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
       const int k0 = tile_key0 + sub * BN;
       if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
       if (a.causal && k0 > blk_q_lo + 31) continue;  // the wave's whole 32x64 block is in the future
-      const __bf16* sKs = sK + sub * BN * LDK;
-      const __bf16* sVs = sV + sub * BN * LDK;
       f32x16 s_acc[BN / 32], dp_acc[BN / 32];
       // the compiler's scheduler is asked for its MFMA / LDS-read interleaving of this block (-1 to -5 %; the key-split
       // variant is better off without)
@@ -882,8 +897,8 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
         for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }
 #pragma unroll
         for (int s = 0; s < D / 16; ++s) {
-          const bf16x8 ka = *reinterpret_cast<const bf16x8*>(&sKs[(32 * mb + n) * LDK + 16 * s + 8 * h]);
-          const bf16x8 va = *reinterpret_cast<const bf16x8*>(&sVs[(32 * mb + n) * LDK + 16 * s + 8 * h]);
+          const unsigned char* row = smem_raw + row_at[s] + (kAt + (sub * BN + 32 * mb) * D * 2);
+          const bf16x8 ka = *reinterpret_cast<const bf16x8*>(row), va = *reinterpret_cast<const bf16x8*>(row + KT * D * 2);
           s_acc[mb] = mfma32(ka, qf[s], s_acc[mb]);
           dp_acc[mb] = mfma32(va, dof[s], dp_acc[mb]);
         }
@@ -919,12 +934,18 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
 #pragma unroll
           for (int db = 0; db < D / 32; ++db) {
             const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
-            const bf16x8 ktf = lds_read_tr_pair(&sKs[krow * LDK + col], LDK);
+            const bf16x8 ktf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
             dq[db] = mfma32(ktf, dsf, dq[db]);
           }
         }
     }
+    wait_requests<0>();
     __syncthreads();
+  };
+  for (int t = 0; t < ntiles;) {
+    trip(std::integral_constant<int, 0>(), t++);
+    if (t >= ntiles) break;
+    trip(std::integral_constant<int, 1>(), t++);
   }
 
   // ---- key split: the partial sums of the waves ks > 0 are added to the wave ks == 0 of the same queries through LDS

@@ -15,6 +15,7 @@
 // tile[row0 .. row0+3][col0 + p]: a 4-deep column of a row-major tile, which is what an MFMA operand
 // needs when the contraction index is the tile's row.
 #pragma once
+#include <type_traits>
 #include "common.h"
 
 namespace pico {
@@ -50,6 +51,15 @@ __device__ __forceinline__ bf16x8 lds_read_tr_pair_step(const __bf16* p, int ste
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// the same from two addresses
+__device__ __forceinline__ bf16x8 lds_read_tr_two(const unsigned char* a, const unsigned char* b) {
+  s16x4 lo = lds_read_tr(reinterpret_cast<const __bf16*>(a));
+  s16x4 hi = lds_read_tr(reinterpret_cast<const __bf16*>(b));
+  typedef __attribute__((ext_vector_type(8))) short s16x8;
+  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
 // s_waitcnt immediate for "vmcnt(0)" with the other counters left at their maxima (gfx9 encoding:
 // vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
 constexpr int kWaitVmcnt0 = 0x0F70;
@@ -71,6 +81,66 @@ __device__ __forceinline__ u32x4 buffer_load_b128(buffer_rsrc r, uint32_t byte_o
 }
 __device__ __forceinline__ float buffer_load_f32(buffer_rsrc r, uint32_t byte_off) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(byte_off), 0, 0));
+}
+
+// ---- loads that go to LDS without passing the registers: 16 bytes per lane, lane after lane from m0 on; zeros past the window.
+// In assembly, because the compiler makes every later read of LDS wait for the builtin: the caller waits by hand
+// (wait_requests) before the barrier that publishes the tile.  The kernel's dynamic LDS has to start at 0 (no static LDS).
+template <int kPlus>
+__device__ __forceinline__ void aim_request(uint32_t lds_off) {   // one instruction has to lie between this and the request
+  asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds_off), "n"(kPlus) : "scc", "memory");
+}
+__device__ __forceinline__ void request16(u32x4 window, uint32_t off) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(window) : "memory");
+}
+template <int kPlus>
+__device__ __forceinline__ void request16_to(uint32_t lds_off, u32x4 window, uint32_t off) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds" ::"s"(lds_off), "n"(kPlus), "v"(off), "s"(window) : "scc", "memory");
+}
+// all but the wave's newest N vector memory operations are complete
+template <int N>
+__device__ __forceinline__ void wait_requests() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// a buffer resource in scalar registers, for the requests (base and bytes uniform over the wave)
+__device__ __forceinline__ u32x4 request_window(uint64_t base, uint32_t bytes) {
+  u32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
+  r[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32) & 0xffffu);
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
+  r[3] = 0x00020000;
+  return r;
+}
+
+// K, V, Q and dO tiles lie in LDS as dense rows of D elements (the direct loads write consecutive addresses), and the 16-byte pieces
+// of a row change places: piece p of row r lies at place p ^ tile_twist<D>(r).  Both kinds of read are then free of bank
+// conflicts: 16 consecutive rows put one piece at 16 different places of the 64 banks, and four consecutive rows put the four
+// pieces of 32 columns at 16 places.  Other pieces of a lane's row are reached by flipping bits 5 and up of its address, rows
+// a multiple of 16 further down by adding.
+template <int D>
+__host__ __device__ constexpr int tile_twist(int r) {
+  return D == 128 ? (r & 3) << 2 | (r >> 2 & 3) : (r >> 1 & 1) << 2 | (r >> 2 & 3);
+}
+// the lane's place in a tile for reads by rows: piece h = lane / 32 of row lane % 32 (piece 2 s + h: ^ 32 s)
+template <int D>
+__device__ __forceinline__ uint32_t row_place(int lane) {
+  return lane % 32 * D * 2 + (lane / 32 ^ tile_twist<D>(lane % 32)) * 16;
+}
+// ... and for transposing reads: row 4 h + lane % 16 / 4, its columns 16 (lane / 16 % 2) + 4 (lane % 4) ..+3 (32 columns further: ^ 64;
+// 8 rows further down: ^ 32 besides the rows)
+template <int D>
+__device__ __forceinline__ uint32_t column_place(int lane) {
+  const int r = 4 * (lane / 32) + lane % 16 / 4;
+  return r * D * 2 + (tile_twist<D>(r) ^ (2 * (lane / 16 % 2) + lane % 4 / 2)) * 16 + lane % 2 * 8;
+}
+
+// fn(integral_constant) for 0 .. N - 1
+template <int N, typename Fn, int i = 0>
+__device__ __forceinline__ void each_load(const Fn& fn) {
+  if constexpr (i < N) {
+    fn(std::integral_constant<int, i>());
+    each_load<N, Fn, i + 1>(fn);
+  }
 }
 
 __device__ __forceinline__ bf16x8 pack8(const f32x16& c, int base) {

@@ -6,6 +6,11 @@
 // O^T accumulator, and the probabilities can be fed to the second MFMA as its B operand without
 // leaving registers.  K and V tiles are staged row-major in LDS once per workgroup; K is read with
 // 16-byte loads, V with transposing LDS reads (the contraction index of P V is V's row).
+//
+// The loop is bound by issue slots: per 32 x 64 tile of scores the softmax's vector instructions take about as long as the
+// products.  The tiles are therefore loaded by requests that write LDS themselves: through registers they cost
+// 2 x KT D / 8 / threads LDS writes with their waits at the end of every trip, and as many registers of 16 bytes (B1 H32 S4096
+// D128 147 -> 142 us, H32/8 S8192 524 -> 507; level at head_dim 64, where one register per tensor and trip was enough).
 #include "attn_common.h"
 
 namespace pico {
@@ -37,27 +42,26 @@ struct FwdCfg {
   static constexpr int BN = 64;            // keys per compute step
   static constexpr int kKT = KT;           // keys per staged LDS tile (a multiple of BN), double-buffered
   static constexpr int kKDepth = D >= 128 ? 2 : 0;  // K fragments in flight from LDS ahead of the MFMA that uses them (0: compiler's order)
-  static constexpr int LDK = D + 8;        // K tile pitch: 16-byte row reads hit distinct banks
-  // V tile pitch for the 4-row transposing reads.  At head_dim 128: 16 (mod 32) words, so that the 16-word pieces of 4
-  // consecutive rows tile the 64 LDS banks (2 requests per bank, the minimum for an 8-byte read; a pitch of D + 8 gives
-  // 3-4): -3 %.  At head_dim 64 the kernel's time does not depend on it, and the smaller tile lets two key-split
-  // workgroups (128 staged keys each) share a CU.
-  static constexpr int LDV = D + (D >= 128 ? 32 : 8);
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;  // 16-byte loads per thread per tensor
-  static constexpr int kTileElems = KT * (LDK + LDV);
-  static constexpr size_t kLdsBytes = 2 * kTileElems * sizeof(__bf16);
-  static_assert(NW * QB * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
+  static constexpr int kTileElems = 2 * KT * D;   // K, then V
   // workgroups that share a CU: eight waves at head_dim 128 and with split keys have it to themselves.  The kernel's register
   // budget is this number's, and the plan counts on it.  (Left to the whole file, four waves at head_dim 128 took 290 and one
   // workgroup fitted: B1 H20 S3000 100 -> 68 us with the budget, 0.84 in the geometric mean of 93 drawn launches; at head_dim
   // 64 accumulators no longer move between the two halves of the file, 0.88 of 107.)
   static constexpr int kPerCu = NW == 8 && (D >= 128 || KS > 1) ? 1 : 2;
+  // the Q fragments pass through LDS behind the tile buffers where there is room, so that the first tile is requested at once, and
+  // through the tile buffers otherwise
+  static constexpr size_t kTiles = 2 * kTileElems * sizeof(__bf16), kFragmentBytes = NW * QB * WaveTile<D>::kRegionBytes;
+  static constexpr bool kBehind = kPerCu * (kTiles + kFragmentBytes) <= 160 * 1024;
+  static constexpr size_t kFragments = kBehind ? kTiles : 0, kLdsBytes = kTiles + (kBehind ? kFragmentBytes : 0);
+  static_assert(NW * QB * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
+  static_assert(kFragmentBytes <= kLdsBytes);
   static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   // exchange of partial states between key-split waves: per wave O^T accumulators (D/32 x 16 registers x 64 lanes) + m + l
   static constexpr size_t kExchangeBytes = (D / 32) * 16 * 64 * 4 + 2 * 64 * 4;
   static_assert(KS == 1 || NW * kExchangeBytes <= kLdsBytes, "the exchange reuses the tile buffers");
-  static_assert(NW * QB * WaveTile<D>::kRegionBytes <= kLdsBytes, "the Q fragments pass through the tile buffers");
+  static_assert(kFragments + NW * QB * WaveTile<D>::kRegionBytes <= kLdsBytes, "the Q fragments pass through LDS");
   static_assert(KT % BN == 0 && (KT * kVecPerRow) % kThreads == 0, "tile must split evenly over the threads");
 };
 
@@ -91,9 +95,8 @@ __device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* 
 template <int D, int QB, int NW, int KT, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 4)) void attn_fwd_kernel(const FwdParams p) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
-  constexpr int BM = C::BM, BN = C::BN, LDK = C::LDK, LDV = C::LDV;
+  constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  __bf16* smem = reinterpret_cast<__bf16*>(smem_raw);
 
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
@@ -117,6 +120,53 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
 
   const __bf16* qbase = a.q + b * a.qs[0] + hq * a.qs[1];
 
+  // ---- key range of this query tile
+  const int q_hi = (q0 + BM < a.Sq ? q0 + BM : a.Sq);           // one past the last live query
+  int kv_end = a.Sk;
+  if (a.causal) {
+    const int vis = a.q_offset + q_hi;                            // keys < vis can be seen by some query
+    kv_end = vis < a.Sk ? vis : a.Sk;
+    if (kv_end < 0) kv_end = 0;
+  }
+  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
+  if (kCut && piece.parts > 1) {
+    t_first = ntiles * piece.part / piece.parts;
+    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
+  }
+
+  // ---- staging of one K/V tile of KT keys: a wave-uniform window per tile (first key row, bytes left in the
+  //      sequence) plus per-lane byte offsets that are computed once; rows past Sk read as zeros.  A lane asks for the
+  //      piece that belongs at its place of LDS (tile_twist).  The loop body holds no wait for memory other than the
+  //      one in front of the barrier that ends a trip, a whole tile after the requests.
+  uint32_t k_off[C::kLoads], v_off[C::kLoads];
+#pragma unroll
+  for (int i = 0; i < C::kLoads; ++i) {
+    const int idx = tid + i * C::kThreads;
+    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow ^ tile_twist<D>(r);
+    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
+    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
+  }
+  // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
+  KvCursor<D> cur;
+  cur.open(a, t_first, b, hkv, KT);
+  KvPosition pos;
+  pos.open(a.kv, t_first, KT);
+  // the next tile goes to LDS buffer `buf`
+  auto request_tile = [&](int buf) {
+    const u32x4 kb = request_window(reinterpret_cast<uint64_t>(cur.k), cur.k_left), vb = request_window(reinterpret_cast<uint64_t>(cur.v), cur.v_left);
+    const uint32_t to = static_cast<uint32_t>(buf) * (C::kTileElems * 2) + wave * 1024;
+    each_load<C::kLoads>([&](auto load) {
+      constexpr int i = decltype(load)::value;
+      request16_to<i * C::kThreads * 16>(to, kb, k_off[i]);
+      request16_to<KT * D * 2 + i * C::kThreads * 16>(to, vb, v_off[i]);
+    });
+    cur.next(a);
+  };
+
+  if constexpr (C::kBehind) {
+    if (ntiles > 0) request_tile(0);
+  }
+
   // ---- Q fragments (B operand of S^T): lane = query, 8 consecutive d per 16-wide k step; fetched row-major and
   //      turned into fragments through the wave's piece of LDS (the tile buffers are filled only after the
   //      barrier below)
@@ -128,7 +178,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     qrow[qb] = row0 + n;
     WaveTile<D> qt;
     qt.issue(make_buffer(qbase + static_cast<int64_t>(row0) * a.qs[2], span_bytes(a.Sq - row0, a.qs[2], D)), a.qs[2], lane);
-    qt.fragments(smem_raw + (wave * QB + qb) * WaveTile<D>::kRegionBytes, lane, qf[qb]);
+    qt.fragments(smem_raw + C::kFragments + (wave * QB + qb) * WaveTile<D>::kRegionBytes, lane, qf[qb]);
     if (p.rope.cos != nullptr) {
       // RoPE on the wave's own queries, once per query in the whole launch (every query belongs to one wave)
       const bool qlive = qrow[qb] < a.Sq;
@@ -174,88 +224,40 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     }
   }
 
-  // ---- key range of this query tile
-  const int q_hi = (q0 + BM < a.Sq ? q0 + BM : a.Sq);           // one past the last live query
-  int kv_end = a.Sk;
-  if (a.causal) {
-    const int vis = a.q_offset + q_hi;                            // keys < vis can be seen by some query
-    kv_end = vis < a.Sk ? vis : a.Sk;
-    if (kv_end < 0) kv_end = 0;
+  if constexpr (!C::kBehind) {
+    __syncthreads();  // every wave has its Q fragments: the tile buffers may be filled
+    if (ntiles > 0) request_tile(0);
   }
-  int t_first = 0, ntiles = kCut ? tiles_before(a.kv, kv_end, KT) : (kv_end + KT - 1) / KT;
-  if (kCut && piece.parts > 1) {
-    t_first = ntiles * piece.part / piece.parts;
-    ntiles = ntiles * (piece.part + 1) / piece.parts - t_first;
-  }
-
-  // ---- global -> register -> LDS staging of one K/V tile of KT keys, with buffer loads: a wave-uniform
-  //      resource per tile (first key row, bytes left in the sequence) plus per-lane byte offsets that are
-  //      computed once; rows past Sk read as zeros.  The loop body holds no wait for memory other than the
-  //      one in front of the LDS fill, a whole tile after the loads were issued.
-  u32x4 kreg[C::kLoads], vreg[C::kLoads];
-  uint32_t k_off[C::kLoads], v_off[C::kLoads];
-#pragma unroll
-  for (int i = 0; i < C::kLoads; ++i) {
-    const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
-    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
-  }
-  // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
-  KvCursor<D> cur;
-  cur.open(a, t_first, b, hkv, KT);
-  KvPosition pos;
-  pos.open(a.kv, t_first, KT);
-  auto load_tile = [&]() {  // the next tile of KT keys
-    const buffer_rsrc kb = make_buffer(cur.k, cur.k_left), vb = make_buffer(cur.v, cur.v_left);
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      kreg[i] = buffer_load_b128(kb, k_off[i]);
-      vreg[i] = buffer_load_b128(vb, v_off[i]);
-    }
-    cur.next(a);
-  };
-  auto store_tile = [&](int buf) {
-    __bf16* sK = smem + buf * C::kTileElems;
-    __bf16* sV = sK + KT * LDK;
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      const int idx = tid + i * C::kThreads;
-      const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-      *reinterpret_cast<u32x4*>(&sK[r * LDK + cv * 8]) = kreg[i];
-      *reinterpret_cast<u32x4*>(&sV[r * LDV + cv * 8]) = vreg[i];
-    }
-  };
-
-  if (ntiles > 0) load_tile();
-  __syncthreads();  // every wave has its Q fragments: the tile buffers may be filled
-  if (ntiles > 0) store_tile(0);
-  // Every load issued so far (Q fragments, the merge state, tile 0) is complete on each path that enters the
-  // loop, because the LDS fill waited for the newest of them -- but not on the static path that skips the
-  // fill.  Saying so here keeps the compiler from putting a vmcnt(0) wait in front of the loop's first MFMAs,
-  // where it would wait for the prefetch of the NEXT tile on every trip.
+  // Every load issued so far (Q fragments, the merge state, tile 0) is complete from here on.  Without this the
+  // barrier would publish a tile that is still on its way, and the compiler would put a vmcnt(0) wait in front of the
+  // loop's first MFMAs, where it would wait for the NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-  if (ntiles > 1) load_tile();
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t) {
+  // the lane's places in a tile (flipping bits of one address for every read takes the issue slots that the direct loads save:
+  // B1 H32 S4096 D128 147 -> 158 us that way)
+  uint32_t row_at[D / 16], tr_at[D / 16];
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) {
+    row_at[s] = row_place<D>(lane) ^ 32 * s;
+    tr_at[s] = column_place<D>(lane) ^ 32 * s;
+    asm volatile("" : "+v"(row_at[s]), "+v"(tr_at[s]));   // (kept, not computed again in front of every read)
+  }
+
+  // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
+  auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
+    constexpr uint32_t kAt = decltype(parity)::value * C::kTileElems * 2;
+    static_assert(kAt + C::kTileElems * 2 <= 65536, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
-    // stage tile t+1 into the other buffer (its readers finished before the barrier that ended trip t-1)
-    if (t + 1 < ntiles) {
-      store_tile((t + 1) & 1);
-      if (t + 2 < ntiles) load_tile();
-    }
-    const __bf16* sK = smem + (t & 1) * C::kTileElems;
-    const __bf16* sV = sK + KT * LDK;
+    // tile t+1 goes into the other buffer (its readers finished before the barrier that ended trip t-1)
+    if (t + 1 < ntiles) request_tile(1 - decltype(parity)::value);
 
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
       const int k0 = tile_key0 + sub * BN;
       if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
-      const __bf16* sKs = sK + sub * BN * LDK;
-      const __bf16* sVs = sV + sub * BN * LDV;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
         const int blk_q_lo = a.q_offset + q0 + (qw * QB + qb) * 32;  // position of the block's first query
@@ -274,7 +276,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
           bf16x8 kf[kSteps];
 #pragma unroll
           for (int j = 0; j < kSteps; ++j)
-            kf[j] = *reinterpret_cast<const bf16x8*>(&sKs[(32 * (j / (D / 16)) + n) * LDK + 16 * (j % (D / 16)) + 8 * h]);
+            kf[j] = *reinterpret_cast<const bf16x8*>(smem_raw + row_at[j % (D / 16)] + (kAt + (sub * BN + 32 * (j / (D / 16))) * D * 2));
 #pragma unroll
           for (int mb = 0; mb < BN / 32; ++mb) {
 #pragma unroll
@@ -297,7 +299,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
             for (int i = 0; i < 16; ++i) s_acc[mb][i] = 0.f;
 #pragma unroll
             for (int s = 0; s < D / 16; ++s) {
-              const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&sKs[(32 * mb + n) * LDK + 16 * s + 8 * h]);
+              const bf16x8 kf = *reinterpret_cast<const bf16x8*>(smem_raw + row_at[s] + (kAt + (sub * BN + 32 * mb) * D * 2));
               s_acc[mb] = mfma32(kf, qf[qb][s], s_acc[mb]);
             }
           }
@@ -357,13 +359,19 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
 #pragma unroll
             for (int db = 0; db < D / 32; ++db) {
               const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
-              const bf16x8 vf = lds_read_tr_pair(&sVs[krow * LDV + col], LDV);
+              const bf16x8 vf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
               o[qb][db] = mfma32(vf, pf, o[qb][db]);
             }
           }
       }
     }
+    wait_requests<0>();
     __syncthreads();  // all waves are done with buffer t&1 (it is refilled in trip t+1) and tile t+1 is visible
+  };
+  for (int t = 0; t < ntiles;) {
+    trip(std::integral_constant<int, 0>(), t++);
+    if (t >= ntiles) break;
+    trip(std::integral_constant<int, 1>(), t++);
   }
 
   // ---- key split: the waves ks > 0 hand their partial state to the wave ks == 0 of the same queries through LDS

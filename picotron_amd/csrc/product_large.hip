@@ -36,20 +36,6 @@ struct LargeParams {
   bool streaming;     // the output is written past the caches
 };
 
-// m0: where the next request goes in LDS.  One instruction has to lie between this and the request.
-template <int kPlus>
-__device__ __forceinline__ void aim_request(uint32_t lds_off) {
-  asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds_off), "n"(kPlus) : "scc", "memory");
-}
-// 16 bytes per lane to 16 consecutive bytes per lane from m0 on; zeros past the window.  (In assembly, because the compiler
-// makes every later read of LDS wait for the builtin; the waits are counted by hand.)
-__device__ __forceinline__ void request16(u32x4 window, uint32_t off) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(window) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_requests() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // A barrier in two halves, so that products go on between a wave's arrival and the point where it needs the others: a count in
@@ -114,14 +100,7 @@ __device__ __forceinline__ void advance(Window& w, uint32_t bytes) {
   w.base += bytes;
   w.bytes = w.bytes > bytes ? w.bytes - bytes : 0;
 }
-__device__ __forceinline__ u32x4 resource(const Window& w) {
-  u32x4 r;
-  r[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(w.base));
-  r[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(w.base >> 32) & 0xffffu);
-  r[2] = __builtin_amdgcn_readfirstlane(w.bytes);
-  r[3] = 0x00020000;
-  return r;
-}
+__device__ __forceinline__ u32x4 resource(const Window& w) { return request_window(w.base, w.bytes); }
 
 // What a workgroup works on in a round of the grid: a tile of the output and a run of steps.  The workgroups of a round go
 // round the eight XCDs; each XCD takes a run of neighbouring tiles, eight tile rows deep, whose operands then meet in its L2.
