@@ -47,21 +47,24 @@ struct BwdParams {
 // =====================================================================================  dK / dV
 // bf16 gradients leave with streaming (non-temporal) stores: nothing on this GPU reads them back soon
 constexpr bool kStreamGrads = true;
-// PAIR: eight waves instead of four; waves w and w + 4 (they share a SIMD) own the same 32 keys and split every
-// 64-query tile between them, one 32-query sub-block each, with accumulators of their own that are added through LDS
-// at the end of the key tile.  A wave then holds one sub-block's S / dP tiles instead of two, which is what lets the
-// head_dim 128 kernel fit 256 registers, i.e. two waves per SIMD.
-// PAIR: K fragments (of D / 16) that stay in registers; the others are read from LDS.  As many as fit: 4 -> 7 with the registers
+// QS > 1: eight waves instead of four, QS of them own the same 32 keys and split every query tile between them, one
+// 32-query sub-block each, with accumulators of their own that are added through LDS at the end of the key tile.
+//   QS 2 (waves w and w + 4, which share a SIMD): a wave holds one sub-block's S / dP tiles instead of two, which is what
+//     lets the head_dim 128 kernel fit 256 registers, i.e. two waves per SIMD.
+//   QS 4: for launches that leave most CUs idle, whose time is that of one workgroup's chain of trips: twice the workgroups
+//     (64 keys each), and a trip takes 128 queries in the time of 32.
+// QS > 1: K fragments (of D / 16) that stay in registers; the others are read from LDS.  As many as fit: 4 -> 7 with the registers
 // that staging the tiles took, 3 % at B1 H32 S4096.
-constexpr int kPairKRegs = 7;
+constexpr int kSplitKRegs = 7;
 
-template <int D, bool PAIR = false>
+template <int D, int QS>
 struct KvCfg {
-  static constexpr int NW = PAIR ? 8 : 4;
-  static constexpr int kKeyWaves = 4;          // waves that own different keys
+  static constexpr bool kSplit = QS > 1;
+  static constexpr int NW = kSplit ? 8 : 4;
+  static constexpr int kKeyWaves = kSplit ? NW / QS : 4;   // waves that own different keys
   static constexpr int kThreads = 64 * NW;
   static constexpr int BN = 32 * kKeyWaves;  // keys per workgroup
-  static constexpr int BM = 64;       // queries per trip
+  static constexpr int BM = QS > 2 ? 32 * QS : 64;   // queries per trip
   // Q and dO tiles: rows of D elements at a pitch of LDQ elements, plus kSkew elements after every 4 rows.  Every
   // tile is read both by rows (16 bytes per lane, 32 consecutive rows per instruction) and transposed (8 bytes per
   // lane: 4 rows x 32 bytes per 16 lanes, rows 4 apart for the two wave halves).  An LDS instruction takes as many
@@ -69,13 +72,13 @@ struct KvCfg {
   // pieces of 4 consecutive rows tile the banks (transposed reads at their minimum of 2 requests per bank; at a pitch
   // of D + 8 they take 3-4), and the 4-word skew per 4 rows spreads 16 consecutive rows over all multiples of 4 words
   // (row reads at their minimum of 4).
-  // PAIR: the tiles are filled by loads that go to LDS directly, 1 KiB of consecutive addresses per wave, so their rows are
+  // QS > 1: the tiles are filled by loads that go to LDS directly, 1 KiB of consecutive addresses per wave, so their rows are
   // dense; the 16-byte pieces of a row change places instead (tile_twist), which spreads both kinds of read as evenly.
   // (The loop is paced by LDS reads and their latency, the matrix cores are busy for half of it: without the LDS writes and
   // with more of K in registers B1 H32 S4096 281 -> 271 us, H32/8 S8192 1000 -> 950.  At head_dim 64 a wave's two sub-blocks take
   // all 256 registers, and the flipped addresses of this layout end up in scratch: S4096 143 -> 156 us, so it keeps the pitch.)
-  static constexpr int LDQ = PAIR ? D : D + 32;
-  static constexpr int kSkew = PAIR ? 0 : 8;
+  static constexpr int LDQ = kSplit ? D : D + 32;
+  static constexpr int kSkew = kSplit ? 0 : 8;
   static constexpr int kTileElems = BM * LDQ + kSkew * (BM / 4);       // one tile
   static constexpr int kTrStep = 8 * LDQ + 2 * kSkew;                  // 8 rows further down
   static constexpr int kVecPerRow = D / 8;
@@ -83,17 +86,20 @@ struct KvCfg {
   static constexpr int kBufElems = 2 * kTileElems;                     // Q + dO tile of one stage (bf16)
   static constexpr size_t kBufBytes = kBufElems * sizeof(__bf16) + 2 * BM * sizeof(float);
   static constexpr size_t kTileBytes = 2 * kBufBytes;  // the two Q / dO tile buffers
-  // PAIR: the K and V fragments of the four key waves stay in LDS behind the tile buffers instead of in registers
-  static constexpr size_t kKvBytes = PAIR ? static_cast<size_t>(kKeyWaves) * 2 * WaveTile<D>::kRegionBytes : 0;
+  // QS > 1: the K and V fragments of the key waves stay in LDS behind the tile buffers instead of in registers
+  static constexpr size_t kKvBytes = kSplit ? static_cast<size_t>(kKeyWaves) * 2 * WaveTile<D>::kRegionBytes : 0;
   static constexpr size_t kLdsBytes = kTileBytes + kKvBytes;
-  static constexpr int kPerCu = PAIR ? 1 : 2;         // workgroups that share a CU
+  static constexpr int kPerCu = kSplit ? 1 : 2;         // workgroups that share a CU
   static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   static_assert(NW * kRowRegionBytes <= kTileBytes, "the epilogue reuses the tile buffers");
-  static_assert(PAIR || NW * WaveTile<D>::kRegionBytes <= kBufBytes, "the K / V fragments pass through the second tile buffer");
-  // PAIR: one accumulator set (D/32 x 16 registers x 64 lanes of fp32) per key wave passes through LDS at a time
-  static constexpr size_t kPairExchangeBytes = static_cast<size_t>(D / 32) * 16 * 64 * 4;
-  static_assert(!PAIR || kKeyWaves * kPairExchangeBytes <= kTileBytes, "the pair exchange reuses the tile buffers");
+  static_assert(kSplit || NW * WaveTile<D>::kRegionBytes <= kBufBytes, "the K / V fragments pass through the second tile buffer");
+  // QS > 1: one accumulator set (D/32 x 16 registers x 64 lanes of fp32) of every wave but the key waves' first passes through LDS at a time
+  static constexpr size_t kExchangeBytes = static_cast<size_t>(D / 32) * 16 * 64 * 4;
+  static_assert(!kSplit || (QS - 1) * kKeyWaves * kExchangeBytes <= kTileBytes, "the exchange reuses the tile buffers");
 };
+
+// (per head_dim, where the launch is not tiny)
+template <int D> constexpr int kUsualSplit = D == 128 ? 2 : 1;
 
 // key tile `ktile` (counted chunk by chunk): its chunk, its first row there and that row's position in the launch
 struct KeyTile {
@@ -147,9 +153,10 @@ __device__ __forceinline__ void dkdv_store(const BwdParams& p, unsigned char* re
 // what a wave of a piece leaves: its dK and dV accumulators
 __host__ __device__ constexpr int dkdv_piece_floats(int D) { return 2 * (D / 32) * 16 * kWave; }
 
-template <int D, bool PAIR, bool kCut>
+template <int D, int QS, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int ktile, const int part = 0, const int parts = 1) {
-  using C = KvCfg<D, PAIR>;
+  using C = KvCfg<D, QS>;
+  constexpr bool kSplit = C::kSplit;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   auto tile_row = [](int r) { return r * C::LDQ + C::kSkew * (r >> 2); };   // element offset of a tile row
@@ -161,9 +168,9 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   const int key0 = kt_at.key0, chunk = kt_at.chunk, crow0 = kt_at.row0;
   if (p.dk[chunk] == nullptr && p.dk_final[chunk] == nullptr) return;   // this chunk's gradient is not wanted (uniform over the workgroup)
   const int tid = threadIdx.x, wave_id = tid / 64, lane = tid % 64;
-  // wave: which 32 keys of the tile; pair_sb (PAIR only): which 32-query sub-block of every query tile
-  const int wave = PAIR ? __builtin_amdgcn_readfirstlane(wave_id % C::kKeyWaves) : wave_id;
-  const int pair_sb = PAIR ? __builtin_amdgcn_readfirstlane(wave_id / C::kKeyWaves) : 0;
+  // wave: which 32 keys of the tile; query_sb (QS > 1 only): which 32-query sub-block of every query tile
+  const int wave = kSplit ? __builtin_amdgcn_readfirstlane(wave_id % C::kKeyWaves) : wave_id;
+  const int query_sb = kSplit ? __builtin_amdgcn_readfirstlane(wave_id / C::kKeyWaves) : 0;
   const int n = lane % 32, h = lane / 32;
   const float c = a.sm_scale * kLog2e;
 
@@ -175,10 +182,11 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   //      else writes before the end of the first trip, a barrier later.  The loads are issued here; the first
   //      Q / dO tile's loads follow them further down before anything waits, so that the two latencies overlap.
   bf16x8 kf[D / 16], vf[D / 16];
+  constexpr int kKRegs = kSplitKRegs < D / 16 ? kSplitKRegs : D / 16;
   constexpr int kFragPitch = (D + 8) * 2;   // WaveTile's row pitch in bytes
-  unsigned char* const pair_k = smem_raw + C::kTileBytes + wave * 2 * WaveTile<D>::kRegionBytes;   // (PAIR only)
-  unsigned char* const pair_v = pair_k + WaveTile<D>::kRegionBytes;
-  const bool loads_kv = !PAIR || pair_sb == 0;
+  unsigned char* const split_k = smem_raw + C::kTileBytes + wave * 2 * WaveTile<D>::kRegionBytes;   // (QS > 1 only)
+  unsigned char* const split_v = split_k + WaveTile<D>::kRegionBytes;
+  const bool loads_kv = !kSplit || query_sb == 0;
   WaveTile<D> kt, vt;
   if (loads_kv) {
     // (the wave index read as a scalar: the buffer windows below are then built in scalar registers; from the
@@ -207,7 +215,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     tile_first += t0 - skip * tiles_per_head;
   }
 
-  // Loads of a Q / dO tile (+ lse, delta) into registers, PAIR: of the tile straight to LDS.  A cursor (wave-uniform:
+  // Loads of a Q / dO tile (+ lse, delta) into registers, QS > 1: of the tile straight to LDS.  A cursor (wave-uniform:
   // it lives in scalar registers) walks the trip space; stepping to the next tile of the same head is a few
   // scalar adds, only a change of head recomputes addresses.  The per-lane byte offsets are computed once,
   // and rows past Sq read as zeros because they lie past the end of the buffer window.  Every instruction
@@ -218,7 +226,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
   for (int i = 0; i < C::kQLoads; ++i) {
     const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = PAIR ? idx % C::kVecPerRow ^ tile_twist<D>(r) : idx % C::kVecPerRow;
+    const int r = idx / C::kVecPerRow, cv = kSplit ? idx % C::kVecPerRow ^ tile_twist<D>(r) : idx % C::kVecPerRow;
     q_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.qs[2] + cv * 8) * 2);
     do_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.os[2] + cv * 8) * 2);
   }
@@ -253,19 +261,22 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       cur.lse += BM;  cur.delta += BM;  cur.rows_left -= BM * 4;
     }
   };
-  // PAIR: the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
+  // QS > 1: the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
   auto request_tile = [&](uint32_t buf_off) {
     const u32x4 qb = request_window(reinterpret_cast<uint64_t>(cur.q), cur.q_left), dob = request_window(reinterpret_cast<uint64_t>(cur.dout), cur.do_left);
     const uint32_t to = buf_off + __builtin_amdgcn_readfirstlane(wave_id) * 1024;
-    static_assert(!PAIR || C::kQLoads == 2);
-    request16_to<0>(to, qb, q_off[0]);
-    request16_to<C::kThreads * 16>(to, qb, q_off[C::kQLoads - 1]);
-    request16_to<C::kTileElems * 2>(to, dob, do_off[0]);
-    request16_to<C::kTileElems * 2 + C::kThreads * 16>(to, dob, do_off[C::kQLoads - 1]);
+    each_load<C::kQLoads>([&](auto load) {
+      constexpr int i = decltype(load)::value;
+      request16_to<i * C::kThreads * 16>(to, qb, q_off[i]);
+    });
+    each_load<C::kQLoads>([&](auto load) {
+      constexpr int i = decltype(load)::value;
+      request16_to<C::kTileElems * 2 + i * C::kThreads * 16>(to, dob, do_off[i]);
+    });
   };
   auto prefetch = [&]() {  // the tile under the cursor
     const buffer_rsrc lb = make_buffer(cur.lse, cur.rows_left), db = make_buffer(cur.delta, cur.rows_left);
-    if constexpr (!PAIR) {
+    if constexpr (!kSplit) {
       const buffer_rsrc qb = make_buffer(cur.q, cur.q_left), dob = make_buffer(cur.dout, cur.do_left);
 #pragma unroll
       for (int i = 0; i < C::kQLoads; ++i) {
@@ -281,7 +292,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     __bf16* sdO = sQ + C::kTileElems;
     float* sL = reinterpret_cast<float*>(sdO + C::kTileElems);
     float* sDelta = sL + BM;
-    if constexpr (!PAIR)
+    if constexpr (!kSplit)
 #pragma unroll
       for (int i = 0; i < C::kQLoads; ++i) {
         const int idx = tid + i * C::kThreads;
@@ -300,27 +311,27 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   if (n_iter > 0) {
     seek(head_first, tile_first);
     prefetch();
-    if constexpr (PAIR) request_tile(0);
+    if constexpr (QS > 1) request_tile(0);
   }
   if (loads_kv) {
-    if constexpr (!PAIR) {
+    if constexpr (!kSplit) {
       unsigned char* region = smem_raw + C::kBufBytes + wave * WaveTile<D>::kRegionBytes;
       kt.fragments(region, lane, kf);
       vt.fragments(region, lane, vf);
     } else {
       // the first wave of each pair leaves both tiles in the pair's piece of LDS
-      kt.fragments(pair_k, lane, kf);
-      vt.fragments(pair_v, lane, vf);
+      kt.fragments(split_k, lane, kf);
+      vt.fragments(split_v, lane, vf);
     }
   }
-  if constexpr (PAIR) {
+  if constexpr (QS > 1) {
     __syncthreads();
     // the first few K fragments stay in registers (as many as fit beside the accumulators)
 #pragma unroll
-    for (int j = 0; j < kPairKRegs; ++j) kf[j] = *reinterpret_cast<const bf16x8*>(pair_k + n * kFragPitch + (16 * j + 8 * h) * 2);
+    for (int j = 0; j < kKRegs; ++j) kf[j] = *reinterpret_cast<const bf16x8*>(split_k + n * kFragPitch + (16 * j + 8 * h) * 2);
   }
   if (n_iter > 0) stage(0);
-  // All loads above are complete from here on (PAIR: also the first tile, which the barrier publishes).  Saying so
+  // All loads above are complete from here on (QS > 1: also the first tile, which the barrier publishes).  Saying so
   // keeps the compiler from putting a vmcnt(0) wait in front of the loop's first MFMAs, where it would wait for the
   // NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
@@ -332,9 +343,9 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // tile it+1 travels global -> registers while this trip computes; it goes to the other LDS buffer at
     // the end of the trip (that buffer's readers finished before the barrier that ended trip it-1)
     const bool has_next = it + 1 < n_iter;
-    // PAIR: it goes there directly, and is requested at the top of the trip
+    // QS > 1: it goes there directly, and is requested at the top of the trip
     if (has_next) advance();
-    if constexpr (PAIR) {
+    if constexpr (QS > 1) {
       if (has_next) {
         prefetch();
         request_tile(buf_off ^ static_cast<uint32_t>(C::kBufBytes));
@@ -345,9 +356,9 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     const __bf16* sdO = sQ + C::kTileElems;
     const float* sL = reinterpret_cast<const float*>(sdO + C::kTileElems);
     const float* sDelta = sL + BM;
-    // (PAIR) this lane's place in the tile of this trip: other pieces are reached by flipping bits of the address
+    // (QS > 1) this lane's place in the tile of this trip: other pieces are reached by flipping bits of the address
     const uint32_t row_lane = buf_off + row_place<D>(lane), tr_lane = buf_off + column_place<D>(lane);
-    static_assert(!PAIR || C::kBufBytes % 256 == 0);
+    static_assert(!kSplit || C::kBufBytes % 256 == 0);
 
     // The three phases of a 32-query sub-block.
     // products(): S = Q K^T and dP = dO V^T (C tile: lane = key, registers = queries); the dP accumulator starts at
@@ -359,7 +370,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
         for (int t = 0; t < 4; ++t) { s_acc[4 * j + t] = 0.f; dp_acc[4 * j + t] = d4[t]; }
       }
-      if constexpr (PAIR) {
+      if constexpr (QS > 1) {
         // both operands of every MFMA come from LDS: they are requested kAhead steps before the MFMAs that use them, and
         // the scheduling barriers keep that order (left alone, the compiler reuses one set of registers and every MFMA
         // waits for an LDS round trip)
@@ -367,9 +378,9 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         bf16x8 qa[kSteps], da[kSteps], kb[kSteps], vb[kSteps];
         auto fetch = [&](int j) {
           qa[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2);
-          if (j >= kPairKRegs) kb[j] = *reinterpret_cast<const bf16x8*>(pair_k + n * kFragPitch + (16 * j + 8 * h) * 2);
+          if (j >= kKRegs) kb[j] = *reinterpret_cast<const bf16x8*>(split_k + n * kFragPitch + (16 * j + 8 * h) * 2);
           da[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2 + C::kTileElems * 2);
-          vb[j] = *reinterpret_cast<const bf16x8*>(pair_v + n * kFragPitch + (16 * j + 8 * h) * 2);
+          vb[j] = *reinterpret_cast<const bf16x8*>(split_v + n * kFragPitch + (16 * j + 8 * h) * 2);
         };
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) fetch(j);
@@ -377,7 +388,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
         for (int j = 0; j < kSteps; ++j) {
           if (j + kAhead < kSteps) fetch(j + kAhead);
-          s_acc = mfma32(qa[j], j < kPairKRegs ? kf[j] : kb[j], s_acc);
+          s_acc = mfma32(qa[j], j < kKRegs ? kf[j] : kb[j], s_acc);
           dp_acc = mfma32(da[j], vb[j], dp_acc);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -416,7 +427,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // d, which is what lets the epilogue write whole 16-byte pieces of a row); P / dS come from the registers,
     // dO^T / Q^T from the row-major LDS tiles through transposing reads.
     auto accumulate = [&](int sb, const f32x16& s_acc, const f32x16& dp_acc) {
-      if constexpr (PAIR) {
+      if constexpr (QS > 1) {
         constexpr int kSlots = 2 * (D / 32), kAhead = 2;
         bf16x8 dof[kSlots], qf[kSlots];
         auto fetch = [&](int idx) {
@@ -458,8 +469,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
     };
 
-    const bool off_diagonal = !PAIR && (!a.causal || kw0 + 31 <= a.q_offset + q0);
-    if (!PAIR && has_next && !off_diagonal) prefetch();
+    const bool off_diagonal = !kSplit && (!a.causal || kw0 + 31 <= a.q_offset + q0);
+    if (!kSplit && has_next && !off_diagonal) prefetch();
     if (off_diagonal) {
       // Every pair of this trip is visible to this wave (all trips off the diagonal): straight-line code in an order
       // that lets the wave's own phases overlap -- the matrix pipe works on the second sub-block's S / dP while the
@@ -560,8 +571,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       accumulate(1, s1, d1);
     } else {
 #pragma unroll
-      for (int sbi = 0; sbi < (PAIR ? 1 : BM / 32); ++sbi) {
-        const int sb = PAIR ? pair_sb : sbi;
+      for (int sbi = 0; sbi < (kSplit ? 1 : BM / 32); ++sbi) {
+        const int sb = kSplit ? query_sb : sbi;
         const int qs_pos = a.q_offset + q0 + 32 * sb;       // position of the sub-block's first query
         if (a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
         f32x16 s_acc, dp_acc;
@@ -573,40 +584,41 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     }
     buf_off ^= static_cast<uint32_t>(C::kBufBytes);
     if (has_next) stage(buf_off != 0);
-    if constexpr (PAIR) wait_requests<0>();
+    if constexpr (QS > 1) wait_requests<0>();
     tile = tile + 1 == n_qtiles ? qt_start : tile + 1;
     __syncthreads();  // all waves are done with the buffer just read (refilled in the next trip) and the next tile is visible
   }
 
   // ---- epilogue (LDS is free now: the loop ended on a barrier)
-  if constexpr (PAIR) {
-    // the second wave of each pair hands its sums over, dK then dV (the loop ended on a barrier, or never ran)
-    float* xch = reinterpret_cast<float*>(smem_raw + wave * C::kPairExchangeBytes);
+  if constexpr (kSplit) {
+    // the other waves of these keys hand their sums over, dK then dV (the loop ended on a barrier, or never ran)
+    auto place = [&](int sb, int db, int i) { return reinterpret_cast<f32x4*>(smem_raw + ((sb - 1) * C::kKeyWaves + wave) * C::kExchangeBytes) + (db * 4 + i / 4) * 64 + lane; };
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
       f32x16 (&acc)[D / 32] = which == 0 ? dk_acc : dv_acc;
-      if (pair_sb == 1) {
+      if (query_sb > 0) {
 #pragma unroll
         for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-          for (int i = 0; i < 16; i += 4)
-            *reinterpret_cast<f32x4*>(&xch[((db * 4 + i / 4) * 64 + lane) * 4]) = f32x4{acc[db][i], acc[db][i + 1], acc[db][i + 2], acc[db][i + 3]};
+          for (int i = 0; i < 16; i += 4) *place(query_sb, db, i) = f32x4{acc[db][i], acc[db][i + 1], acc[db][i + 2], acc[db][i + 3]};
       }
       __syncthreads();
-      if (pair_sb == 0) {
+      if (query_sb == 0) {
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db)
+        for (int sb = 1; sb < QS; ++sb)
 #pragma unroll
-          for (int i = 0; i < 16; i += 4) {
-            const f32x4 o = *reinterpret_cast<const f32x4*>(&xch[((db * 4 + i / 4) * 64 + lane) * 4]);
+          for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[db][i + t] += o[t];
-          }
+            for (int i = 0; i < 16; i += 4) {
+              const f32x4 o = *place(sb, db, i);
+#pragma unroll
+              for (int t = 0; t < 4; ++t) acc[db][i + t] += o[t];
+            }
       }
       __syncthreads();
     }
   }
-  if (!PAIR || pair_sb == 0) {
+  if (!kSplit || query_sb == 0) {
     if (kCut && parts > 1) {   // one piece of several: the sums leave as they are
       float* dst = a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kKeyWaves + wave) * dkdv_piece_floats(D);
       put_acc<D / 32>(dst, dk_acc, lane);
@@ -626,19 +638,19 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 // workgroup (kernel arguments, first loads) half as often.
 // kCut: the launch deals its trips out in pieces (see Pieces); a kernel of its own, because the loop of the whole-tile kernel
 // is 1 to 2 % slower with the pieces' bookkeeping around it (in the forward and in dQ up to 10 %).
-template <int D, bool PAIR, bool kCut>
+template <int D, int QS, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_body(const BwdParams& p) {
-  using C = KvCfg<D, PAIR>;
+  using C = KvCfg<D, QS>;
   if constexpr (kCut) {
     const Piece at = find_piece(blockIdx.y, tiles_before(p.a.kv, p.a.Sk, C::BN), p.a.pieces.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
-    attn_bwd_dkdv_tile<D, PAIR, true>(p, at.tile, at.part, at.parts);
+    attn_bwd_dkdv_tile<D, QS, true>(p, at.tile, at.part, at.parts);
   } else {
     const int first = blockIdx.y;
-    attn_bwd_dkdv_tile<D, PAIR, false>(p, first);
+    attn_bwd_dkdv_tile<D, QS, false>(p, first);
     const int second = p.pair_ktiles - 1 - first;
     if (p.pair_ktiles > 0 && second != first) {
       __syncthreads();  // the epilogue's pieces of LDS are the next tile's buffers
-      attn_bwd_dkdv_tile<D, PAIR, false>(p, second);
+      attn_bwd_dkdv_tile<D, QS, false>(p, second);
     }
   }
 }
@@ -647,19 +659,21 @@ __device__ __forceinline__ void attn_bwd_dkdv_body(const BwdParams& p) {
 // work overlap the other's softmax / LDS phases; D = 128 needs the full register file.
 template <bool kCut>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dkdv_kernel_d64(const BwdParams p) {
-  attn_bwd_dkdv_body<64, false, kCut>(p);
+  attn_bwd_dkdv_body<64, 1, kCut>(p);
 }
+// D = 64, launches of few workgroups: eight waves, four per key block
+__global__ __launch_bounds__(512) void attn_bwd_dkdv_few_kernel(const BwdParams p) { attn_bwd_dkdv_body<64, 4, false>(p); }
 // D = 128: eight waves, two per key block (see KvCfg), 256 registers each
 template <bool kCut>
 __global__ __launch_bounds__(512) void attn_bwd_dkdv_kernel_d128(const BwdParams p) {
-  attn_bwd_dkdv_body<128, true, kCut>(p);
+  attn_bwd_dkdv_body<128, 2, kCut>(p);
 }
 
 // The pieces of every cut key tile put together: grid.z 0 sums dK, 1 dV; a wave per 32 keys adds the pieces' accumulators in
 // their order and ends as the kernel above does.
 template <int D>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_join_kernel(const BwdParams p, const int pieces_per_head) {
-  using C = KvCfg<D, D == 128>;
+  using C = KvCfg<D, kUsualSplit<D>>;
   __shared__ __attribute__((aligned(16))) unsigned char smem_raw[C::kKeyWaves * kRowRegionBytes];
   const AttnParams& a = p.a;
   const int tile = static_cast<int>(blockIdx.y);
@@ -1055,19 +1069,31 @@ __global__ __launch_bounds__(256) void attn_bwd_preprocess_kernel(const __bf16* 
 
 // How the dK/dV launch is run: key tiles singly, in pairs, or cut into pieces.
 struct DkdvPlan {
+  bool few = false;    // attn_bwd_dkdv_few_kernel
   bool pair = false;
   int len = 0;
   int64_t ws_bytes = 0;
 };
 template <int D>
 DkdvPlan make_dkdv_plan(const AttnParams& a) {
-  using C = KvCfg<D, D == 128>;
+  using C = KvCfg<D, kUsualSplit<D>>;
   DkdvPlan plan;
   const int64_t heads = static_cast<int64_t>(a.Hkv) * a.B;
   const int n_ktiles = tiles_before(a.kv, a.Sk, C::BN);
   // pairs only when they still fill most of the GPU (two workgroups per CU for D = 64, one for D = 128; at D = 64 three
   // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
   // are up to 30 % faster)
+  // Few workgroups with short chains: the kernel whose chain is a quarter as long.  It takes 6.6 us + 0.92 per trip (of 128
+  // queries) while its workgroups have a CU each, the usual one 5.3 + 1.25 per trip (of 64): B2 H9/3 S256 20.3 -> 12.1, B2 H32
+  // S256 (256 workgroups) 10.4 -> 8.6, B8 H9/3 S512 (12 trips) 22.1 -> 18.3.  With longer chains the usual kernel's pieces win
+  // (B3 H9/3 S777, 21 trips: 25.2, here 26.4), with more workgroups its two per CU (B4 H32 S256 10.7, here 14.0).
+  if constexpr (D == 64) {
+    using F = KvCfg<64, 4>;
+    if (heads * tiles_before(a.kv, a.Sk, F::BN) <= 256 && dkdv_trips(a, 0, F::BN, F::BM) <= 14) {
+      plan.few = true;
+      return plan;
+    }
+  }
   plan.pair = a.causal && n_ktiles >= 2 && heads * ((n_ktiles + 1) / 2) >= (D == 64 ? 384 : 256);
   TripCost cost = {1.1, 1.0, 1.0, C::kPerCu, 0.0};
   if (D == 128) cost = {1.65, 2.05, 1.0, C::kPerCu, 0.0};
@@ -1085,7 +1111,7 @@ const DkdvPlan& plan_dkdv(const AttnParams& a) {
 
 template <int D, bool kCut>
 int launch_dkdv_impl(const BwdParams& p, int grid_y, hipStream_t s) {
-  using C = KvCfg<D, D == 128>;
+  using C = KvCfg<D, kUsualSplit<D>>;
   static LdsOnce lds_reserved;
   if (!reserve_lds_once(lds_reserved, reinterpret_cast<const void*>(KvKernel<D, kCut>::fn), C::kLdsBytes))
     return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dk/dv): cannot reserve %zu bytes of LDS", C::kLdsBytes);
@@ -1094,8 +1120,20 @@ int launch_dkdv_impl(const BwdParams& p, int grid_y, hipStream_t s) {
 }
 template <int D>
 int launch_dkdv(const BwdParams& p, float* ws, int64_t ws_bytes, hipStream_t s) {
-  using C = KvCfg<D, D == 128>;
+  using C = KvCfg<D, kUsualSplit<D>>;
   const DkdvPlan& plan = plan_dkdv<D>(p.a);
+  if constexpr (D == 64) {
+    if (plan.few) {
+      using F = KvCfg<64, 4>;
+      static LdsOnce reserved;
+      if (!reserve_lds_once(reserved, reinterpret_cast<const void*>(&attn_bwd_dkdv_few_kernel), F::kLdsBytes))
+        return fail(PICO_ERR_LAUNCH, "pico_attn_bwd(dk/dv): cannot reserve %zu bytes of LDS", F::kLdsBytes);
+      BwdParams q = p;
+      q.pair_ktiles = 0;
+      hipLaunchKernelGGL(attn_bwd_dkdv_few_kernel, dim3(p.a.Hkv * p.a.B, tiles_before(p.a.kv, p.a.Sk, F::BN)), dim3(F::kThreads), F::kLdsBytes, s, q);
+      return PICO_OK;
+    }
+  }
   const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN);
   BwdParams q = p;
   if (plan.len == 0 || !ws || ws_bytes < plan.ws_bytes) {

@@ -112,3 +112,11 @@ def test_ragged_chunk_lists(device, B, Hq, Hkv, W, Sc, D, causal):
     totals = [2 * w + torch.cat(b, 2) for w, b in ((want[3], base[:W]), (want[4], base[W:]))]
     for got, total in zip((torch.cat(finals[:W], 2), torch.cat(finals[W:], 2)), totals):
         assert rel_l2(got.float(), total) <= 1e-2
+
+
+# B, Hq, Hkv, Sq, Sk, causal, q_offset: edges of the 64-key tiles and 128-query trips that launches of few workgroups take
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,q_offset", [(1, 9, 3, 1, 1, True, 0), (1, 4, 2, 63, 65, False, 0), (2, 9, 3, 128, 128, True, 0),
+                                                            (1, 4, 2, 129, 257, True, 128), (1, 2, 2, 300, 100, True, 0),
+                                                            (1, 3, 1, 127, 64, False, 0), (4, 32, 32, 96, 96, True, 0)])
+def test_short_chains(device, B, Hq, Hkv, Sq, Sk, causal, q_offset):
+    test_attention_in_pieces(device, B, Hq, Hkv, Sq, Sk, 64, causal, q_offset, (False, False))
