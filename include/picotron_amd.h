@@ -339,6 +339,13 @@ int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb
 int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
                  int tile, int groups, void* stream);
 
+/* Both gradients of y = x w^T in one launch of pico_product's tiles of 64: dx [rows, in] = dy w and dw [out, in] = dy^T x, for dy
+ * [rows, out], w [out, in] and x [rows, in] with row pitches ld_dy, ld_w, ld_x; dx and dw contiguous.  `groups`: 1 or 2.  Takes what
+ * pico_product takes for each of the two.
+ */
+int pico_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int64_t rows, int64_t out, int64_t in,
+                      int64_t ld_dy, int64_t ld_w, int64_t ld_x, int groups, void* stream);
+
 /* The same for products that fill the GPU, in tiles of tile_m x tile_n: 256 x 256, or one side 192 or 128.  parts > 1: the
  * contraction is cut into that many pieces, whose fp32 sums go to c [parts, M, N] (see pico_sum_parts).  Operands as above, but
  * not with a_slow = 1 and b_slow = 0; two steps of 64 of contraction per piece at least.
