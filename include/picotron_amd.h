@@ -339,6 +339,13 @@ int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb
 int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
                  int tile, int groups, void* stream);
 
+/* The same as pico_product in tiles of tile_m x tile_n (32 x 32, 32 x 64, 64 x 32, 64 x 64, 64 x 96, 96 x 64, 96 x 96, 64 x 128, 128 x 64,
+ * 128 x 96, 128 x 128, 128 x 192, 192 x 128, 128 x 256).
+ */
+int pico_product_mid_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow);
+int pico_product_mid(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
+                     int tile_m, int tile_n, void* stream);
+
 /* Both gradients of y = x w^T in one launch of pico_product's tiles of 64: dx [rows, in] = dy w and dw [out, in] = dy^T x, for dy
  * [rows, out], w [out, in] and x [rows, in] with row pitches ld_dy, ld_w, ld_x; dx and dw contiguous.  `groups`: 1 or 2.  Takes what
  * pico_product takes for each of the two.

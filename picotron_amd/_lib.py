@@ -82,6 +82,8 @@ SIGNATURES = {
     "pico_adamw_multi": (c_int, [c_int, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int] + [ctypes.c_float] * 5 + [_I64, ctypes.c_float, _P]),
     "pico_sum_parts": (c_int, [_P, _P, _I64, _I64, c_int, _P]),
     "pico_product_takes": (c_int, [_I64] * 5 + [c_int, c_int]),
+    "pico_product_mid_takes": (c_int, [_I64, _I64, _I64, _I64, _I64, c_int, c_int]),
+    "pico_product_mid": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
     "pico_product_pair": (c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, c_int, _P]),
     "pico_product": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
     "pico_product_large_takes": (c_int, [_I64] * 5 + [c_int, c_int, c_int]),

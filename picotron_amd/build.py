@@ -19,7 +19,7 @@ OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libpicotron_amd.so")
 HOST = os.path.join(HERE, "_host.so")
 
-SOURCES = ["common.hip", "norm.hip", "pointwise.hip", "optim.hip", "loss.hip", "embedding.hip", "product.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip"]
+SOURCES = ["common.hip", "norm.hip", "pointwise.hip", "optim.hip", "loss.hip", "embedding.hip", "product.hip", "product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
     # packed fp32 VALU forms are kept out of the generated code on purpose

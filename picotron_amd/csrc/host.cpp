@@ -1192,6 +1192,83 @@ LargeProduct large_product(Product kind, const ProductSizes& n, const Tensor& a,
   return takes ? large : LargeProduct{};
 }
 
+// Whether a product goes to pico_product_mid and in which tiles (tile_m 0: no).
+//
+// Its time follows from its rounds: 256 workgroups take a tile each, a trip (64 of contraction for each group of waves) costs `trip`,
+// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy.  Over 25000 timed (shape, tiles) the
+// estimate has an error of 2 .. 6 % (standard deviation; tiles of 32 x 32 10 %), and the tiles it takes are 0.1 % slower than the best
+// ones in the mean.  Against it stands pico_product's own time, estimated alike (4 .. 7 %), or the library's (other_time).  Of 2290 drawn
+// products (64 .. 8192 rows, 72 .. 16384 columns and contraction) the 1430 that go here take, in the geometric mean of the time without it,
+//   NN 0.85 of pico_product's ([512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.69 of the library's ([2331 x 3072] @ [3072 x 576] 27.7 -> 15.8),
+//   TN 0.80 of pico_product's ([2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.82 of pico_product_large's,
+//   NT 0.78 of the library's ([2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5) and 0.93 of pico_product's; two over 1.12, 1.19 at most (the
+// library's choice of tiles is not monotone in any size).  The forward's layout leaves pico_product only for a clear gain: tiles of
+// 64 run level there.  Contractions that the library would cut stay with it.
+struct MidProduct {
+  int64_t tile_m = 0, tile_n = 0;
+};
+double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
+  return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
+}
+double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
+  struct Form {
+    int64_t m, n, groups;
+    double start, trip, end, walk_idle, end_idle;
+  };
+  static constexpr Form forms[] = {
+      {32, 32, 4, 1.54, 0.50, 1.46, 0.47, 1.12},   {32, 64, 4, 1.37, 0.62, 1.78, 0.64, 1.09},   {64, 32, 4, 1.36, 0.68, 1.71, 0.58, 1.15},
+      {64, 64, 2, 1.51, 0.43, 1.98, 0.80, 0.83},   {64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {96, 64, 2, 1.54, 0.56, 2.29, 0.82, 0.75},
+      {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},  {128, 64, 2, 1.59, 0.67, 2.58, 0.86, 0.70},
+      {128, 96, 2, 1.31, 1.01, 2.83, 0.71, 0.79},  {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60}, {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45},
+      {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37}, {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
+  const int64_t steps = (K + 63) / 64;
+  double least = 1e30;
+  for (const Form& f : forms) {
+    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
+    if (tiles > 1024 || (f.m == 32 && f.n == 32 && steps > 48)) continue;   // (long walks along a slow axis in rows of 64 bytes take twice that)
+    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
+    const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
+    if (t < least) {
+      least = t;
+      best = {f.m, f.n};
+    }
+  }
+  return least;
+}
+double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
+  struct Form {
+    int64_t tile, groups;
+    double start, trip, end, walk_idle, end_idle;
+  };
+  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84}, {64, 4, 2.52, 0.82, 5.90, 1.20, 0.00},
+                                   {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
+  for (const Form& f : forms) {
+    if (f.tile != own.tile || f.groups != own.groups) continue;
+    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
+    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
+    return f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
+  }
+  return 0;
+}
+MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b, const LargeProduct& large, const OwnProduct& own) {
+  const auto [M, N, K] = n;
+  if (M < 1 || N < 1 || K < 1 || !pico_product_mid_takes(M, N, K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT)) return {};
+  MidProduct best;
+  LargeProduct same;
+  const double time = mid_time(M, N, K, best);
+  bool take;
+  if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
+  else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
+  else take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? 1.0 : 0.9) * other_time(kind, M, N, K);
+  return take ? best : MidProduct{};
+}
+Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {
+  Tensor c = at::empty({n.M, n.N}, a.options());
+  check(pico_product_mid(ptr(a), ptr(b), ptr(c), n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
+                         static_cast<int>(mid.tile_m), static_cast<int>(mid.tile_n), stream_now()));
+  return c;
+}
+
 // parts 0, turn -1, groups -1, tile_n 0: by the rules above
 Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64, int64_t tile_n = 0) {
   if (!stays_with_torch(a, b)) {
@@ -1199,9 +1276,15 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
     // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
     const ProductSizes n = product_sizes(a, b, kind);
     const auto [M, N, K] = n;
-    Tensor c = at::empty({M, N}, a.options());
     LargeProduct large = {tile, tile_n, std::max<int64_t>(parts, 1)};
-    if (tile_n == 0) large = parts == 0 && turn < 0 && groups < 0 ? large_product(kind, n, a, b) : LargeProduct{};
+    const bool by_rule = tile_n == 0 && parts == 0 && turn < 0 && groups < 0;
+    if (tile_n == 0) large = by_rule ? large_product(kind, n, a, b) : LargeProduct{};
+    const OwnProduct own = by_rule ? own_product(kind, n, a, b) : OwnProduct{0, 64};
+    if (by_rule) {
+      const MidProduct mid = mid_product(kind, n, a, b, large, own);
+      if (mid.tile_m > 0) return mid_product(a, b, kind, n, mid);
+    }
+    Tensor c = at::empty({M, N}, a.options());
     if (large.tile_n > 0) {
       parts = large.parts;
       const Tensor sums = parts > 1 ? at::empty({parts, M, N}, a.options().dtype(at::kFloat)) : Tensor();
@@ -1211,7 +1294,6 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
       return c;
     }
     if (groups < 0) {
-      const OwnProduct own = parts == 0 && turn < 0 ? own_product(kind, n, a, b) : OwnProduct{0, 64};
       groups = own.groups;
       tile = own.tile;
     }
@@ -1275,7 +1357,7 @@ Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x, int64_t 
   return r;
 }
 
-// the route of a product that large_product leaves alone, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
+// the route of a product that large_product and mid_product leave alone, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
 // "library in N" pieces
 std::string product_route(const Tensor& a, const Tensor& b, Product kind) {
   if (stays_with_torch(a, b)) return "torch";
@@ -1726,6 +1808,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return product(a, b, product_kind(kind), parts, turn, groups, tile, tile_n);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
         pybind11::arg("groups") = -1, pybind11::arg("tile") = 64, pybind11::arg("tile_n") = 0);
+  m.def("mid_product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t tile_m, int64_t tile_n) {
+    TORCH_CHECK(!stays_with_torch(a, b), "mid_product: operands that stay with torch");
+    const c10::OptionalDeviceGuard device(a.device());
+    const Product k = product_kind(kind);
+    const ProductSizes n = product_sizes(a, b, k);
+    const MidProduct mid = tile_m > 0 ? MidProduct{tile_m, tile_n} : mid_product(k, n, a, b, large_product(k, n, a, b), own_product(k, n, a, b));
+    if (mid.tile_m == 0) return std::make_tuple(Tensor(), mid.tile_m, mid.tile_n);
+    return std::make_tuple(mid_product(a, b, k, n, mid), mid.tile_m, mid.tile_n);
+  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m") = 0, pybind11::arg("tile_n") = 0);
   m.def("paired", &paired);
   m.def("gradients", [](const Tensor& dy, const Tensor& w, const Tensor& x, int64_t groups) {
     Gradients d = gradients(dy, w, x, groups);

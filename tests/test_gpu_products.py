@@ -174,3 +174,26 @@ def test_both_gradients_in_one_launch(device, rows, out, inner):
             again = host.gradients(dy, w, x, groups)
             assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])
     assert host.paired(torch.empty(3201, 64, dtype=torch.bfloat16, device=device), w[:64], x[:1].expand(3201, inner)) == 0
+
+
+MID_TILES = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (96, 64), (96, 96), (64, 128), (128, 64), (128, 96), (128, 128), (128, 192), (192, 128),
+             (128, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 96, 64), (72, 136, 200), (200, 328, 72), (264, 272, 584), (520, 40, 1032)])
+@pytest.mark.parametrize("kind", ["NT", "NN", "TN"])
+def test_products_of_one_round(device, kind, M, N, K):
+    """Every tile, at sizes around its edges, contractions of fewer steps than groups and of a ragged last step, operands that are
+    columns of wider matrices, against a fp32 product (rounded once: 2^-9)."""
+    from picotron_amd import _lib
+    host = _lib.host()
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    sizes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    a, b = (torch.randn(r, c + 16, generator=g, device=device).to(torch.bfloat16)[:, 8:8 + c] for r, c in sizes)
+    want = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float())
+    for tiles in MID_TILES:
+        got, tile_m, tile_n = host.mid_product(a, b, kind, *tiles)
+        assert (tile_m, tile_n) == tiles and ((got.float() - want).norm() / want.norm()).item() <= 3e-3, tiles
+        assert torch.equal(got, host.mid_product(a, b, kind, *tiles)[0]), tiles
+    with pytest.raises(RuntimeError, match="no tiles"):
+        host.mid_product(a, b, kind, 96, 128)
