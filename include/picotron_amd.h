@@ -346,12 +346,12 @@ int pico_product_mid_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t
 int pico_product_mid(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow,
                      int tile_m, int tile_n, void* stream);
 
-/* Both gradients of y = x w^T in one launch of pico_product's tiles of 64: dx [rows, in] = dy w and dw [out, in] = dy^T x, for dy
- * [rows, out], w [out, in] and x [rows, in] with row pitches ld_dy, ld_w, ld_x; dx and dw contiguous.  `groups`: 1 or 2.  Takes what
- * pico_product takes for each of the two.
+/* Both gradients of y = x w^T in one launch of pico_product_mid's tiles: dx [rows, in] = dy w and dw [out, in] = dy^T x, for dy
+ * [rows, out], w [out, in] and x [rows, in] with row pitches ld_dy, ld_w, ld_x; dx and dw contiguous.  The tiles of each: 32 x 64, 64 x
+ * 64, 64 x 96 or 64 x 128.  Takes what pico_product_mid takes for each of the two.
  */
 int pico_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int64_t rows, int64_t out, int64_t in,
-                      int64_t ld_dy, int64_t ld_w, int64_t ld_x, int groups, void* stream);
+                      int64_t ld_dy, int64_t ld_w, int64_t ld_x, int dx_tile_m, int dx_tile_n, int dw_tile_m, int dw_tile_n, void* stream);
 
 /* The same for products that fill the GPU, in tiles of tile_m x tile_n: 256 x 256, or one side 192 or 128.  parts > 1: the
  * contraction is cut into that many pieces, whose fp32 sums go to c [parts, M, N] (see pico_sum_parts).  Operands as above, but

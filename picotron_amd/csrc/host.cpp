@@ -1321,41 +1321,79 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
   return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
 }
 
-// dx = dy w and dw = dy^T x, in one launch where neither fills the GPU for long by itself: it takes pico_product's tiles of 64, all
-// of them at once, and the launch of the second product and the idle CUs of both are what it saves.  Us apart and together:
-//   [512 x 576] and [576 x 576] 9.9, 5.5; [512 x 3072] and [3072 x 576] 20.6, 15.1; [2331 x 960] and [960 x 576] 23.7, 16.4; [1024
-//   x 1024] and [1024 x 1024] 14.5, 11.9.
-// Of 1091 drawn layers (64 .. 5000 rows, 192 .. 2400 columns in, up to 5.3 times that out) the 970 with at most 1000 tiles, 3200
-// rows and 4096 columns out took 0.71 of the time in the geometric mean and 1.008 at most, whatever the two took alone (pico_product
-// or the library); among the others the longer walks lose (5388 rows of 264 and 264: 21.9, 28.0).  One group of waves per workgroup
-// where the CUs have work throughout (steps of all tiles over 256 times the longest walk; four such workgroups share a CU), two
-// otherwise: 1.2 % over the better of the two in the mean, 2.9 % with two always.
+// dx = dy w and dw = dy^T x, in one launch where neither fills the GPU for long by itself: the launch of the second product and the
+// idle CUs of both are what it saves.  Us apart and together:
+//   [512 x 576] and [576 x 576] 8.8, 5.2; [512 x 3072] and [3072 x 576] 16.2, 13.1; [2331 x 960] and [960 x 576] 17.9, 14.0; [1024
+//   x 1024] and [1024 x 1024] 15.1, 10.4.
+// The tiles of both are chosen together: their times alike mid_time's, and the workgroups dealt to 256 CUs, the longer ones first; 7.7 %
+// error over 8900 timed (layer, tiles), 2 % over the best tiles in the mean.  It is taken where it promises 0.94 of the two products'
+// estimates: of 557 drawn layers (64 .. 5000 rows, 192 .. 2400 columns in, up to 5.3 times that out) 494, which take 0.75 of the time in
+// the geometric mean, four over 1.02 and 1.15 at most; the others would take 0.95 ([1309 x 1688] and [1688 x 1688] 30.8, 37.3).
 struct Gradients {
   Tensor dx, dw;
 };
-int64_t paired(const Tensor& dy, const Tensor& w, const Tensor& x) {   // the number of groups, 0: apart
-  if (stays_with_torch(dy, w) || stays_with_torch(dy, x)) return 0;
+struct GradientTiles {
+  MidProduct dx, dw;   // (tile_m 0: apart)
+};
+// The time at which the last of n1 workgroups of t1 each, then n2 of t2 each, ends on 256 CUs
+double workgroups_end(int64_t n1, double t1, int64_t n2, double t2) {
+  const int64_t rest = n1 % 256, idle = 256 - rest;
+  const double early = n1 / 256 * t1, late = early + t1, first = rest ? late : early;   // `idle` CUs are free at `early`, `rest` at `late`
+  double end = 1e30;
+  for (const double base : {early, late})
+    for (int64_t k = 0; k <= n2 / 256 + static_cast<int64_t>(t1 / t2) + 2; ++k) {
+      const double at = base + k * t2;
+      const int64_t done = idle * static_cast<int64_t>((at - early) / t2 + 1e-9) + (at >= late ? rest * static_cast<int64_t>((at - late) / t2 + 1e-9) : 0);
+      if (at < first || done < n2) continue;
+      end = std::min(end, at);
+      break;
+    }
+  return end;
+}
+GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
+  struct Form {
+    int64_t m, n, groups;
+    double trip, end;
+  };
+  static constexpr Form forms[] = {{32, 64, 4, 0.72, 1.93}, {64, 64, 2, 0.48, 2.15}, {64, 96, 2, 0.54, 2.50}, {64, 128, 2, 0.68, 2.69}};
+  auto tiles = [](int64_t M, int64_t N, const Form& f) { return ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n); };
+  auto length = [](int64_t K, const Form& f) { return ((K + 63) / 64 + f.groups - 1) / f.groups * f.trip + f.end; };
+  if (tiles(rows, in, forms[3]) + tiles(out, in, forms[3]) > 1024) return {};
+  GradientTiles best;
+  double least = 1e30;
+  for (const Form& x : forms)
+    for (const Form& w : forms) {
+      const int64_t nx = tiles(rows, in, x), nw = tiles(out, in, w);
+      const double tx = length(out, x), tw = length(rows, w), busy = std::min(1.0, (nx + nw) / 256.0);
+      const double t = 1.02 + (0.91 + 0.09 * busy) * (rows > out ? workgroups_end(nw, tw, nx, tx) : workgroups_end(nx, tx, nw, tw));
+      if (t < least) {
+        least = t;
+        best = {{x.m, x.n}, {w.m, w.n}};
+      }
+    }
+  MidProduct alone;
+  return least < 0.94 * (mid_time(rows, in, out, alone) + mid_time(out, in, rows, alone)) ? best : GradientTiles{};
+}
+GradientTiles gradient_tiles(const Tensor& dy, const Tensor& w, const Tensor& x) {
+  if (stays_with_torch(dy, w) || stays_with_torch(dy, x)) return {};
   const auto [rows, in, out] = product_sizes(dy, w, Product::NN);
   product_sizes(dy, x, Product::TN);
-  if (rows > 3200 || out > 4096 || !pico_product_takes(rows, in, out, dy.stride(0), w.stride(0), 0, 1) ||
-      !pico_product_takes(out, in, rows, dy.stride(0), x.stride(0), 1, 1))
-    return 0;
-  auto up = [](int64_t n) { return (n + 63) / 64; };
-  const int64_t tiles_dx = up(rows) * up(in), tiles_dw = up(out) * up(in);
-  if (tiles_dx + tiles_dw > 1000) return 0;
-  return tiles_dx * up(out) + tiles_dw * up(rows) > 256 * std::max(up(out), up(rows)) ? 1 : 2;
+  if (rows < 1 || in < 1 || out < 1 || !pico_product_mid_takes(rows, in, out, dy.stride(0), w.stride(0), 0, 1) ||
+      !pico_product_mid_takes(out, in, rows, dy.stride(0), x.stride(0), 1, 1))
+    return {};
+  return gradient_tiles(rows, out, in);
 }
-Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x, int64_t groups = 0) {
-  if (groups == 0) groups = paired(dy, w, x);
-  if (groups == 0) return {product(dy, w, Product::NN), product(dy, x, Product::TN)};
-  TORCH_CHECK(!stays_with_torch(dy, w) && !stays_with_torch(dy, x), "gradients: operands that stay with torch");
+Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x, const GradientTiles& tiles) {
+  if (tiles.dx.tile_m == 0) return {product(dy, w, Product::NN), product(dy, x, Product::TN)};
   const c10::OptionalDeviceGuard device(dy.device());
   const int64_t rows = dy.size(0), out = dy.size(1), in = w.size(1);
   Gradients r = {at::empty({rows, in}, dy.options()), at::empty({out, in}, dy.options())};
   check(pico_product_pair(ptr(dy), ptr(w), ptr(x), ptr(r.dx), ptr(r.dw), rows, out, in, dy.stride(0), w.stride(0), x.stride(0),
-                          static_cast<int>(groups), stream_now()));
+                          static_cast<int>(tiles.dx.tile_m), static_cast<int>(tiles.dx.tile_n), static_cast<int>(tiles.dw.tile_m),
+                          static_cast<int>(tiles.dw.tile_n), stream_now()));
   return r;
 }
+Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x) { return gradients(dy, w, x, gradient_tiles(dy, w, x)); }
 
 // the route of a product that large_product and mid_product leave alone, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
 // "library in N" pieces
@@ -1817,11 +1855,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     if (mid.tile_m == 0) return std::make_tuple(Tensor(), mid.tile_m, mid.tile_n);
     return std::make_tuple(mid_product(a, b, k, n, mid), mid.tile_m, mid.tile_n);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m") = 0, pybind11::arg("tile_n") = 0);
-  m.def("paired", &paired);
-  m.def("gradients", [](const Tensor& dy, const Tensor& w, const Tensor& x, int64_t groups) {
-    Gradients d = gradients(dy, w, x, groups);
-    return std::make_tuple(d.dx, d.dw);
-  }, pybind11::arg("dy"), pybind11::arg("w"), pybind11::arg("x"), pybind11::arg("groups") = 0);
+  // (dx, dw, the tiles of each or 0); tiles given: in one launch of these
+  m.def("gradients", [](const Tensor& dy, const Tensor& w, const Tensor& x, std::vector<int64_t> tiles) {
+    TORCH_CHECK(tiles.empty() || (tiles.size() == 4 && !stays_with_torch(dy, w) && !stays_with_torch(dy, x)),
+                "gradients: four tile sides, operands that do not stay with torch");
+    const GradientTiles t = tiles.empty() ? gradient_tiles(dy, w, x) : GradientTiles{{tiles[0], tiles[1]}, {tiles[2], tiles[3]}};
+    Gradients d = gradients(dy, w, x, t);
+    return std::make_tuple(d.dx, d.dw, t.dx.tile_m, t.dx.tile_n, t.dw.tile_m, t.dw.tile_n);
+  }, pybind11::arg("dy"), pybind11::arg("w"), pybind11::arg("x"), pybind11::arg("tiles") = std::vector<int64_t>());
   m.def("linear", &linear, nogil());
   m.def("fused_linear", &fused_linear, nogil());
   m.def("embedding", &embedding, nogil());

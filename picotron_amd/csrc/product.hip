@@ -86,9 +86,8 @@ struct Shape {
   static constexpr int kLds = kStaging > kEnd ? kStaging : kEnd;
 };
 
-// workgroup `block` of the product's (block % 8: its XCD)
 template <bool kSlowA, bool kSlowB, int W, int KS>
-__device__ __forceinline__ void product_tile(const ProductParams& p, int block) {
+__global__ __launch_bounds__(256 * KS, 2) void product_kernel(const ProductParams p) {
   using S = Shape<kSlowA, kSlowB, W, KS>;
   using A = typename S::A;
   using B = typename S::B;
@@ -98,7 +97,7 @@ __device__ __forceinline__ void product_tile(const ProductParams& p, int block) 
   const int group = wave / 4, tid = threadIdx.x % 256, wm = (wave % 4) / 2 * 32 * W, wn = (wave % 4) % 2 * 32 * W;
   // workgroups go round the eight XCDs: each takes a run of neighbouring tiles, along the shorter side of the output, whose
   // operand then stays in its L2 ([577 x 2048]^T [577 x 8192] 42 us along the longer side, 34 along the shorter)
-  const int tiles = p.tiles_m * p.tiles_n, xcd = block % 8, id = xcd * (tiles / 8) + min(xcd, tiles % 8) + block / 8;
+  const int tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x % 8, id = xcd * (tiles / 8) + min(xcd, tiles % 8) + blockIdx.x / 8;
   const bool down = p.tiles_m < p.tiles_n;
   const int m0 = (down ? id % p.tiles_m : id / p.tiles_n) * kTile, n0 = (down ? id / p.tiles_m : id % p.tiles_n) * kTile;
   const int steps = (p.K + kStep - 1) / kStep, trips = (steps + KS - 1) / KS;   // every group makes the same number of trips
@@ -223,41 +222,6 @@ last:
 }
 
 template <bool kSlowA, bool kSlowB, int W, int KS>
-__global__ __launch_bounds__(256 * KS, 2) void product_kernel(const ProductParams p) {
-  product_tile<kSlowA, kSlowB, W, KS>(p, blockIdx.x);
-}
-
-// Both gradients of a linear layer in one launch, dX = dY W and dW = dY^T X.  Each alone leaves CUs idle and pays a launch of
-// its own: [512 x 960] @ [960 x 576] and [512 x 960]^T [512 x 576] take 6.2 and 5.1 us alone and 6.9 together, [512 x 3072] @
-// [3072 x 576] (72 workgroups, bound by what one CU loads, 85 bytes a nanosecond) and [512 x 3072]^T [512 x 576] 12.9 and 7.5, together 15.1.
-struct PairParams {
-  ProductParams dx, dw;
-  int blocks_first;   // of the product that comes first, rounded up to whole rounds of the XCDs
-  bool dw_first;
-};
-template <int KS>
-__global__ __launch_bounds__(256 * KS, 2) void product_pair_kernel(const PairParams p) {
-  const int block = blockIdx.x, rest = block - p.blocks_first;
-  if ((rest < 0) == p.dw_first) {
-    const int at = rest < 0 ? block : rest;
-    if (at < p.dw.tiles_m * p.dw.tiles_n) product_tile<true, true, 1, KS>(p.dw, at);
-  } else {
-    const int at = rest < 0 ? block : rest;
-    if (at < p.dx.tiles_m * p.dx.tiles_n) product_tile<false, true, 1, KS>(p.dx, at);
-  }
-}
-template <int KS>
-int launch_pair(const PairParams& p, hipStream_t s) {
-  constexpr int kDx = Shape<false, true, 1, KS>::kLds, kDw = Shape<true, true, 1, KS>::kLds, kLds = kDx > kDw ? kDx : kDw;
-  static LdsOnce reserved;
-  if (!reserve_lds_once(reserved, reinterpret_cast<const void*>(&product_pair_kernel<KS>), kLds))
-    return fail(PICO_ERR_LAUNCH, "pico_product_pair: cannot reserve %d bytes of LDS", kLds);
-  const ProductParams& second = p.dw_first ? p.dx : p.dw;
-  hipLaunchKernelGGL(product_pair_kernel<KS>, dim3(static_cast<unsigned>(p.blocks_first + second.tiles_m * second.tiles_n)), dim3(256 * KS), kLds, s, p);
-  return check_launch("pico_product_pair");
-}
-
-template <bool kSlowA, bool kSlowB, int W, int KS>
 int launch(const ProductParams& p, hipStream_t s) {
   constexpr int kLds = Shape<kSlowA, kSlowB, W, KS>::kLds;
   static_assert(kLds <= 160 * 1024);
@@ -307,24 +271,4 @@ extern "C" int pico_product(const void* a, const void* b, void* c, int64_t M, in
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a_slow) return b_slow ? launch_shape<true, true>(p, tile, groups, s) : launch_shape<true, false>(p, tile, groups, s);
   return b_slow ? launch_shape<false, true>(p, tile, groups, s) : launch_shape<false, false>(p, tile, groups, s);
-}
-
-extern "C" int pico_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int64_t rows, int64_t out, int64_t in,
-                                 int64_t ld_dy, int64_t ld_w, int64_t ld_x, int groups, void* stream) {
-  if (!pico_product_takes(rows, in, out, ld_dy, ld_w, 0, 1) || !pico_product_takes(out, in, rows, ld_dy, ld_x, 1, 1))
-    return fail(PICO_ERR_SHAPE, "pico_product_pair: rows=%lld out=%lld in=%lld row pitches %lld, %lld, %lld (out, in and the pitches must be multiples of 8 elements, a tile's rows span less than 2 GiB)",
-                (long long)rows, (long long)out, (long long)in, (long long)ld_dy, (long long)ld_w, (long long)ld_x);
-  if (groups != 1 && groups != 2) return fail(PICO_ERR_SHAPE, "pico_product_pair: groups=%d (1 or 2)", groups);
-  if (!dy || !w || !x || !dx || !dw) return fail(PICO_ERR_NULL, "pico_product_pair: dy, w, x, dx and dw are required");
-  if (!aligned16(dy) || !aligned16(w) || !aligned16(x) || !aligned16(dx) || !aligned16(dw)) return fail(PICO_ERR_ALIGN, "pico_product_pair: pointers must be 16-byte aligned");
-  auto tiles = [](int64_t n) { return static_cast<int>((n + 63) / 64); };
-  PairParams p;
-  p.dx = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(w), static_cast<__bf16*>(dx), (int)rows, (int)in, (int)out, ld_dy, ld_w, tiles(rows), tiles(in)};
-  p.dw = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(x), static_cast<__bf16*>(dw), (int)out, (int)in, (int)rows, ld_dy, ld_x, tiles(out), tiles(in)};
-  const int64_t n_dx = static_cast<int64_t>(p.dx.tiles_m) * p.dx.tiles_n, n_dw = static_cast<int64_t>(p.dw.tiles_m) * p.dw.tiles_n;
-  if (n_dx + n_dw + 8 > 0x7fffffff) return fail(PICO_ERR_SHAPE, "pico_product_pair: too many tiles");
-  p.dw_first = rows > out;   // the longer walks start first
-  p.blocks_first = static_cast<int>(((p.dw_first ? n_dw : n_dx) + 7) / 8 * 8);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return groups == 1 ? launch_pair<1>(p, s) : launch_pair<2>(p, s);
 }

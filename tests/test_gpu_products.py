@@ -154,26 +154,27 @@ def test_large_products(device, kind, M, N, K):
                 assert torch.equal(_lib.host().product(ai, bi, kind, parts, tile=tile, tile_n=tile_n), exact.to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("rows,out,inner", [(1, 8, 8), (64, 64, 64), (65, 72, 136), (63, 1000, 200), (512, 960, 576), (333, 3072, 576), (3200, 128, 72),
-                                            (700, 4096, 192)])
+@pytest.mark.parametrize("rows,out,inner", [(1, 8, 8), (64, 64, 64), (65, 72, 136), (63, 1000, 200), (512, 960, 576), (333, 3072, 576), (2100, 520, 328)])
 def test_both_gradients_in_one_launch(device, rows, out, inner):
-    """Edges of the tiles and of the rule, each number of groups, operands that are columns of wider matrices, and the two
-    products by themselves (the same kernel, rounded once: 2^-9 each way)."""
+    """Edges of the tiles, every pair of tiles, operands that are columns of wider matrices, against fp32 products (rounded once:
+    2^-9); the rule takes small layers and leaves large ones apart."""
     from picotron_amd import _lib
     host = _lib.host()
     g = torch.Generator(device="cuda").manual_seed(rows + out)
     wide = torch.randn(rows, out + 24, generator=g, device=device).to(torch.bfloat16)
     w, x = (torch.randn(n, inner, generator=g, device=device).to(torch.bfloat16) for n in (out, rows))
+    tiles = [(32, 64), (64, 64), (64, 96), (64, 128)]
     for dy in (wide[:, 8:8 + out], wide[:, 16:16 + out].contiguous()):
-        assert host.paired(dy, w, x) in (1, 2)
         want = (dy.float() @ w.float(), dy.float().t() @ x.float())
-        for groups in (0, 1, 2):
-            got = host.gradients(dy, w, x, groups)
+        assert host.gradients(dy, w, x)[2] > 0
+        for choice in [[]] + [[*a, *b] for a in tiles for b in tiles]:
+            got = host.gradients(dy, w, x, choice)
             for a, b in zip(got, want):
-                assert a.shape == b.shape and a.is_contiguous() and ((a.float() - b).norm() / b.norm()).item() <= 3e-3, groups
-            again = host.gradients(dy, w, x, groups)
-            assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])
-    assert host.paired(torch.empty(3201, 64, dtype=torch.bfloat16, device=device), w[:64], x[:1].expand(3201, inner)) == 0
+                assert a.shape == b.shape and a.is_contiguous() and ((a.float() - b).norm() / b.norm()).item() <= 3e-3, choice
+            again = host.gradients(dy, w, x, choice)
+            assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1]), choice
+    big = torch.zeros(4096, 2048, dtype=torch.bfloat16, device=device)
+    assert host.gradients(big, big[:2048], big)[2] == 0
 
 
 MID_TILES = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (96, 64), (96, 96), (64, 128), (128, 64), (128, 96), (128, 128), (128, 192), (192, 128),
