@@ -1095,7 +1095,7 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
 // 100 .. 8192 rows those that go here took, in the geometric mean of the time without it,
 //   TN: 0.69 where the library ran them as they are (217 products, 0.99 at most; [4096 x 4096]^T [4096 x 4096] 137 -> 103
 //     us), 0.83 where it had an operand transposed first (91, 1.03 at most; [4096 x 16384]^T [4096 x 2048] 216 -> 199), 0.86 where
-//     pico_product did (13); under 640 of contraction that one stays ahead ([512 x 49152]^T [512 x 576] 45 us, here 52), and the
+//     pico_product did (13); under 640 of contraction that one stays ahead but for a vocabulary's width, see below, and the
 //     library where the vocabulary meets fewer than 256 columns ([7358 x 49152]^T [7358 x 128] 161 us, here 179);
 //   NN: 0.80 (143, 1.06 at most; [2242 x 10880] @ [10880 x 4096] 248 -> 178, [608 x 49152] @ [49152 x 576] 84 -> 55); a margin is
 //     asked for pieces of four and up, whose rows of a large pitch come more slowly than the estimate has it, and for short
@@ -1103,6 +1103,14 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
 //   NT: 0.77 (42, 1.02 at most): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
 //     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
 //     16384]^T 424 -> 206).
+// A vocabulary's side (24576 and up) is in every step, so its products were swept by themselves (600 of 128 .. 8192 rows, 192 .. 4096
+// columns, vocabularies of 32000 and 49152): they come here
+//   NT up to 768 of contraction, 0.81 of the library's time, none slower ([680 x 576] @ [32000 x 576]^T 57 -> 29 us, [512 x 576] @ [49152
+//     x 576]^T 41 -> 35; with 1024 0.96, and 1.10 at most);
+//   TN under 640 of contraction with 384 columns and up, 0.87 of pico_product's (1.09 at most; [464 x 32000]^T [464 x 1024] 43.6 ->
+//     34.1; with 192 and 256 columns level);
+//   NN where the library would cut the contraction, under 3072 columns, 0.83 (1.12 at most; [4548 x 49152] @ [49152 x 576] 418 ->
+//     258; with 4096 columns 1.00, and 1.21 at most).
 struct LargeProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 0;
 };
@@ -1111,7 +1119,7 @@ double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
     int64_t m, n;
     double step, end;
   };
-  static constexpr Form forms[] = {{256, 256, 1.43, 4.8}, {256, 192, 1.2, 4.4}, {192, 256, 1.2, 3.2}, {256, 128, 0.99, 2.4}, {128, 256, 1.0, 1.6}};
+  static constexpr Form forms[] = {{256, 256, 1.43, 4.8}, {256, 192, 1.18, 5.6}, {192, 256, 1.2, 3.2}, {256, 128, 0.99, 2.4}, {128, 256, 1.0, 1.6}};
   const int64_t steps = (K + 63) / 64;
   double least = 1e30;
   for (const Form& f : forms) {
@@ -1156,7 +1164,9 @@ LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
   const double time = large_time(M, N, K, best), ideal = 2e-9 * M * N * K;   // (us at 1 PFLOP/s)
   const bool small = own_product(kind, M, N, K).groups > 0;
   bool take = false;
-  if (kind == Product::TN) take = !small || (K >= 640 && time < 0.9 * other_time(kind, M, N, K));
+  const bool vocabulary = std::max(wide, K) >= 24576;   // (see above)
+  if (vocabulary && (kind == Product::TN ? narrow >= 384 && K >= 200 && K < 640 : kind == Product::NT ? K <= 768 : K == std::max(wide, K) && N < 3072 && contraction_parts(kind, M, N, K) > 1)) take = true;
+  else if (kind == Product::TN) take = !small || (K >= 640 && time < 0.9 * other_time(kind, M, N, K));
   else if (small || time < 14) take = false;
   else if (kind == Product::NN) take = time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05);
   else take = time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal);
@@ -1259,7 +1269,7 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
   else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
-  else take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? 1.0 : 0.9) * other_time(kind, M, N, K);
+  else take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? 1.0 : 2e-9 * M * N * K < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
   return take ? best : MidProduct{};
 }
 Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {

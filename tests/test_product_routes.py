@@ -172,7 +172,8 @@ none = (0, 0, 0)
 for kind, M, N, K, want in (("TN", 4096, 4096, 4096, (256, 256, 1)),       # 137, 103
                             ("TN", 6144, 2048, 4096, (192, 256, 1)),       # 101, 91
                             ("TN", 16384, 2048, 4096, (256, 256, 1)),      # 216, 199
-                            ("TN", 49152, 576, 512, none),                 # 45, 52
+                            ("TN", 49152, 576, 512, (192, 256, 1)),        # 45, 40
+                            ("TN", 32000, 256, 512, none),                 # level
                             ("TN", 49152, 128, 7358, none),                # 161, 179
                             ("TN", 2048, 2048, 4096, none),                # 42, 51
                             ("NN", 2242, 10880, 4096, (256, 256, 1)),      # 248, 178
@@ -182,6 +183,7 @@ for kind, M, N, K, want in (("TN", 4096, 4096, 4096, (256, 256, 1)),       # 137
                             ("NT", 3832, 49152, 512, (256, 256, 1)),       # 315, 218
                             ("NT", 5856, 6144, 768, (192, 256, 1)),        # 79, 52
                             ("NT", 4096, 16384, 2048, none),               # 194, 203
+                            ("NT", 512, 49152, 576, (128, 256, 1)),        # 41, 34
                             ("NT", 512, 576, 576, none)):
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     got = host.large_product(operand(ra, ca), operand(rb, cb), kind)
