@@ -396,6 +396,122 @@ void launch_dw_reduce(const float* partial, void* dweight, int dweight_dtype, in
     hipLaunchKernelGGL(rmsnorm_dw_reduce_kernel<float>, grid, block, 0, s, partial, static_cast<float*>(dweight), nparts, hidden);
 }
 
+// Few rows: dx and dweight in one launch.  There a backward takes the time of its two launches (the second one waits for the
+// partial sums of the first), so dweight has workgroups of its own, which read dy and x once more instead
+// of waiting for anybody: 32 columns of all rows each, they come first in the grid, the rows' waves after them.  The same fp32 products
+// as above, added in the order of 128 interleaved row lists.  bf16 with residual, us: [512 x 576] 6.3 -> 3.2, [64 x 2048] 7.4 -> 3.7,
+// [1024 x 576] 6.6 -> 4.3, [1024 x 4096] 13.5 -> 11.5.  Up to 1024 rows nothing loses (64 .. 1024 rows of 192 .. 4096, both types); with 1536 rows of
+// 2048 the second reading costs what the launch saves (11.6, 11.8), with 2048 of 192 as well (6.0, 6.4).
+constexpr int kFewThreads = 512, kFewCols = 32, kFewRows = 1024;
+template <typename T, typename TW, int NV, bool kRes>
+__global__ __launch_bounds__(kFewThreads) void rmsnorm_bwd_few_kernel(
+    const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ rstd, const T* dres, T* dx,
+    TW* __restrict__ dweight, int rows, int hidden, int dw_blocks) {
+  constexpr int V = io<T>::kVec;
+  auto unpack = [](const u32x4& raw, float (&out)[V]) {
+    if constexpr (V == 8) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        out[2 * i] = __uint_as_float(raw[i] << 16);
+        out[2 * i + 1] = __uint_as_float(raw[i] & 0xffff0000u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[i] = __uint_as_float(raw[i]);
+    }
+  };
+  const int tid = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) < dw_blocks) {   // (uniform over the workgroup)
+    constexpr int kPieces = kFewCols / V, kLists = kFewThreads / kPieces, kUnroll = 4;
+    __shared__ float red[kLists][kFewCols + 1];
+    const int list = tid / kPieces, c0 = (tid % kPieces) * V, col = blockIdx.x * kFewCols + c0, from = col < hidden ? col : 0;
+    float sum[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) sum[e] = 0.f;
+    for (int r0 = list; r0 < rows; r0 += kLists * kUnroll) {
+      u32x4 xr[kUnroll], dr[kUnroll];
+      float rs[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const int64_t r = min(r0 + u * kLists, rows - 1);
+        xr[u] = *reinterpret_cast<const u32x4*>(x + r * hidden + from);
+        dr[u] = *reinterpret_cast<const u32x4*>(dy + r * hidden + from);
+        rs[u] = rstd[r];
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        if (r0 + u * kLists >= rows) break;
+        float xv[V], dv[V];
+        unpack(xr[u], xv);
+        unpack(dr[u], dv);
+#pragma unroll
+        for (int e = 0; e < V; ++e) sum[e] += dv[e] * (xv[e] * rs[u]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) red[list][c0 + e] = sum[e];
+    __syncthreads();
+    constexpr int kGroups = kFewThreads / kFewCols, kOf = kLists / kGroups;
+    const int c = tid % kFewCols, g = tid / kFewCols;
+    float part = 0.f;
+#pragma unroll
+    for (int i = 0; i < kOf; ++i) part += red[g * kOf + i][c];
+    __syncthreads();
+    red[g][c] = part;
+    __syncthreads();
+    if (g == 0 && static_cast<int>(blockIdx.x) * kFewCols + c < hidden) {
+      float total = 0.f;
+#pragma unroll
+      for (int i = 0; i < kGroups; ++i) total += red[i][c];
+      dweight[blockIdx.x * kFewCols + c] = static_cast<TW>(total);
+    }
+    return;
+  }
+  const int t = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave), nvec = hidden / V;
+  const int64_t row = static_cast<int64_t>(blockIdx.x - dw_blocks) * (kFewThreads / kWave) + wave;
+  if (row >= rows) return;
+  u32x4 xr[NV], dr[NV], wr[NV], rr[kRes ? NV : 1];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int v = t + j * kWave < nvec ? t + j * kWave : 0;
+    xr[j] = *reinterpret_cast<const u32x4*>(x + row * hidden + v * V);
+    dr[j] = *reinterpret_cast<const u32x4*>(dy + row * hidden + v * V);
+    if constexpr (kRes) rr[j] = *reinterpret_cast<const u32x4*>(dres + row * hidden + v * V);
+    wr[j] = *reinterpret_cast<const u32x4*>(w + v * V);
+  }
+  const float r = rstd[row];
+  float c = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if (t + j * kWave >= nvec) continue;
+    float xv[V], dv[V], wv[V];
+    unpack(xr[j], xv);
+    unpack(dr[j], dv);
+    unpack(wr[j], wv);
+#pragma unroll
+    for (int e = 0; e < V; ++e) c += dv[e] * wv[e] * (xv[e] * r);
+  }
+  c = wave_sum(c) * (1.f / static_cast<float>(hidden));
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int v = t + j * kWave;
+    if (v >= nvec) continue;
+    float xv[V], dv[V], wv[V], o[V];
+    unpack(xr[j], xv);
+    unpack(dr[j], dv);
+    unpack(wr[j], wv);
+#pragma unroll
+    for (int e = 0; e < V; ++e) o[e] = r * (dv[e] * wv[e] - xv[e] * r * c);
+    if constexpr (kRes) {   // dx may alias dres: this lane read its part of the row before it writes it
+      float rv[V];
+      unpack(rr[j], rv);
+#pragma unroll
+      for (int e = 0; e < V; ++e) o[e] += rv[e];
+    }
+    store_as<T, kStreamBwdStores>(dx + row * hidden + v * V, o);
+  }
+}
+
 // Blocks of the backward: as many as the rows need, up to a cap that shrinks with the row length -- every block ends by
 // writing (and the reduce kernel by reading) one row of the workspace, and at hidden 4096 the 512 blocks that are right
 // for hidden 2048 cost 19 % (measured at 4096 rows: 48.7 us with 512 blocks, 39.3 us with 256).
@@ -520,6 +636,27 @@ int dispatch_bwd(const void* dy, const void* x, const void* w, const float* rstd
   return fail(PICO_ERR_SHAPE, "pico_rmsnorm_bwd: hidden=%d too large", hidden);
 }
 
+// rmsnorm_bwd_few_kernel, where it is taken: 1, nothing launched otherwise.
+template <typename T, typename TW>
+bool launch_bwd_few(const void* dy, const void* x, const void* w, const float* rstd, const void* dres, void* dx, void* dweight, int64_t rows,
+                    int hidden, hipStream_t s) {
+  const int nv = pick_nv((hidden / io<T>::kVec + 63) / 64, 8);
+  if (!nv || rows > kFewRows || dx == dy || dx == x) return false;
+  const int dw_blocks = (hidden + kFewCols - 1) / kFewCols, row_blocks = static_cast<int>((rows + kFewThreads / kWave - 1) / (kFewThreads / kWave));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(dw_blocks + row_blocks), dim3(kFewThreads), 0, s, static_cast<const T*>(dy), static_cast<const T*>(x),
+                       static_cast<const T*>(w), rstd, static_cast<const T*>(dres), static_cast<T*>(dx), static_cast<TW*>(dweight),
+                       static_cast<int>(rows), hidden, dw_blocks);
+  };
+  switch (nv) {
+    case 1: dres ? go(rmsnorm_bwd_few_kernel<T, TW, 1, true>) : go(rmsnorm_bwd_few_kernel<T, TW, 1, false>); break;
+    case 2: dres ? go(rmsnorm_bwd_few_kernel<T, TW, 2, true>) : go(rmsnorm_bwd_few_kernel<T, TW, 2, false>); break;
+    case 4: dres ? go(rmsnorm_bwd_few_kernel<T, TW, 4, true>) : go(rmsnorm_bwd_few_kernel<T, TW, 4, false>); break;
+    default: dres ? go(rmsnorm_bwd_few_kernel<T, TW, 8, true>) : go(rmsnorm_bwd_few_kernel<T, TW, 8, false>); break;
+  }
+  return true;
+}
+
 // Bytes of partial sums one backward launch writes: (blocks it will use) x hidden floats -- the same choice of
 // kernel and grid as dispatch_bwd.
 int64_t bwd_partial_bytes(int64_t rows, int64_t hidden, int dtype) {
@@ -592,6 +729,13 @@ int rmsnorm_bwd_impl(const char* fn, const void* dy, const void* x, const void* 
   if (!aligned16(dy) || !aligned16(x) || !aligned16(weight) || !aligned16(dx) || !aligned16(partial) ||
       !aligned16(dresidual))
     return fail(PICO_ERR_ALIGN, "%s: pointers must be 16-byte aligned", fn);
+  const int h = static_cast<int>(hidden);
+  const bool few = dtype == PICO_BF16
+                       ? (dweight_dtype == PICO_BF16 ? launch_bwd_few<__bf16, __bf16>(dy, x, weight, rstd, dresidual, dx, dweight, rows, h, s)
+                                                     : launch_bwd_few<__bf16, float>(dy, x, weight, rstd, dresidual, dx, dweight, rows, h, s))
+                       : (dweight_dtype == PICO_BF16 ? launch_bwd_few<float, __bf16>(dy, x, weight, rstd, dresidual, dx, dweight, rows, h, s)
+                                                     : launch_bwd_few<float, float>(dy, x, weight, rstd, dresidual, dx, dweight, rows, h, s));
+  if (few) return check_launch(fn);
   int blocks = 0;
   int rc = dtype == PICO_BF16
                ? dispatch_bwd<__bf16>(dy, x, weight, rstd, dresidual, dx, partial, rows, static_cast<int>(hidden), s, &blocks)

@@ -102,6 +102,21 @@ def test_rmsnorm_bwd_adds_residual_gradient_and_rounds_dweight(ops, device, rows
         assert ((dx.double().cpu() - exact).abs() <= exact.abs() * 2.0 ** -8 + want_dx.double().abs() * 2.0 ** -7 + 1e-6).all()
 
 
+@pytest.mark.parametrize("rows,hidden", [(1, 40), (8, 584), (9, 2056), (512, 576), (1023, 200), (1024, 4096), (1025, 1000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rmsnorm_bwd_of_few_rows(ops, device, rows, hidden, dtype):
+    """Around the sizes where dx and dweight share a launch (1024 rows, rows in eights, columns in 32s), with the residual's gradient."""
+    x, dy, dr = (rnd(rows, hidden, seed=s_, dtype=dtype) for s_ in (6, 7, 12))
+    w = (1 + 0.1 * rnd(hidden, seed=8)).to(dtype)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1) + 1e-5)
+    dev = lambda t: t.to(device)  # noqa: E731
+    want_dx, want_dw = OL.rmsnorm_backward(dy, x, w, 1e-5)
+    got = [ops.rmsnorm_bwd(dev(dy), dev(x), dev(w), dev(rstd), dresidual=dev(dr), dw_dtype=torch.float32) for _ in range(2)]
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert rel_l2(got[0][0], want_dx.float() + dr.float()) <= (1e-5 if dtype == torch.float32 else 4e-3)
+    assert rel_l2(got[0][1], want_dw) <= 1e-5
+
+
 def test_rmsnorm_bwd_is_bit_reproducible_at_every_row_length_class(ops, device):
     """dweight is summed without atomics: two runs give the same bits, for the row-per-wave kernels, for the rows a
     256-thread group owns (two groups per block meet in LDS, in group order) and for the longest rows."""
