@@ -66,3 +66,26 @@ def test_a_factor_of_the_loss(device, dtype, vocab):
     (one,), (div,) = (torch.autograd.grad(l, x) for l in (cross_entropy(x, t, scale=0.25), cross_entropy(x, t) / 4))
     assert rel(one, div.double()) <= tol
     assert cross_entropy(x, torch.full_like(t, -100), scale=0.5).item() == 0.0
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 800), (64, 800), (65, 800), (255, 8192), (257, 8192), (1024, 40000), (1025, 40000)])
+def test_rows_that_count(device, rows, vocab):
+    """Around the number of rows up to which every workgroup counts for itself (one per thread of it); ignored rows, a class that is
+    ignored, no row that counts."""
+    from picotron_amd.functional import cross_entropy
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = (torch.randn(rows, vocab, generator=g, device=device) * 2).to(torch.bfloat16).requires_grad_()
+    t = torch.randint(0, vocab, (rows,), generator=g, device=device)
+    t[::3] = 7
+    for targets, ignored in ((t, 7), (t, -100), (torch.full_like(t, -100), -100)):
+        loss = cross_entropy(x, targets, ignored)
+        (got,) = torch.autograd.grad(loss, x)
+        live = targets != ignored
+        if not live.any():
+            assert loss.item() == 0.0 and not got.any()
+            continue
+        xd = x.detach()[live].float().requires_grad_()
+        want = torch.nn.functional.cross_entropy(xd, targets[live])
+        (gw,) = torch.autograd.grad(want, xd)
+        assert abs(loss.item() - want.item()) <= 2e-5 * abs(want.item())
+        assert rel(got[live], gw) <= 4e-3 and not got[~live].any()     # (rounded once: 2^-9)
