@@ -1269,7 +1269,10 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
   else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
-  else take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? 1.0 : 2e-9 * M * N * K < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
+  else {   // (a margin that grows with the work: a wrong choice between two full GPUs costs more than it can gain)
+    const double gflop = 2e-9 * M * N * K;
+    take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? (gflop < 20 ? 1.0 : 0.9) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
+  }
   return take ? best : MidProduct{};
 }
 Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {
