@@ -83,7 +83,7 @@ SIGNATURES = {
     "pico_sum_parts": (c_int, [_P, _P, _I64, _I64, c_int, _P]),
     "pico_product_takes": (c_int, [_I64] * 5 + [c_int, c_int]),
     "pico_product_mid_takes": (c_int, [_I64, _I64, _I64, _I64, _I64, c_int, c_int]),
-    "pico_product_mid": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
+    "pico_product_mid": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, c_int, _P]),
     "pico_product_pair": (c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
     "pico_product": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, c_int, c_int, c_int, c_int, _P]),
     "pico_product_large_takes": (c_int, [_I64] * 5 + [c_int, c_int, c_int]),

@@ -1213,9 +1213,13 @@ LargeProduct large_product(Product kind, const ProductSizes& n, const Tensor& a,
 //   TN 0.80 of pico_product's ([2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.82 of pico_product_large's,
 //   NT 0.78 of the library's ([2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5) and 0.93 of pico_product's; two over 1.12, 1.19 at most (the
 // library's choice of tiles is not monotone in any size).  The forward's layout leaves pico_product only for a clear gain: tiles of
-// 64 run level there.  Contractions that the library would cut stay with it.
+// 64 run level there.
+// Contractions that the library or pico_product_large would cut are cut here where that promises 0.95 (0.88) of pico_product_large's estimate: of 1020 drawn
+// input gradients (100 .. 4096 rows, 192 .. 3072 columns, contractions of 5504 .. 49152) 0.69 of the library's time in its pieces (ten of
+// 347 over 1.02, 1.22 at most) and 0.76 of pico_product_large's (246, 0.98 at most): [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [375 x 11008] @ [11008 x
+// 3072] 51 -> 38, [145 x 49152] @ [49152 x 576] 37 -> 23.
 struct MidProduct {
-  int64_t tile_m = 0, tile_n = 0;
+  int64_t tile_m = 0, tile_n = 0, parts = 1;
 };
 double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
   return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
@@ -1240,7 +1244,34 @@ double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
     const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
     if (t < least) {
       least = t;
-      best = {f.m, f.n};
+      best = {f.m, f.n, 1};
+    }
+  }
+  return least;
+}
+// The same for an input gradient whose contraction is cut into pieces, one round of workgroups of one piece each, and the pieces'
+// sum: 8 % error over 7600 timed (shape, tiles, pieces), 1.3 % over the best ones in the mean.
+double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
+  struct Form {
+    int64_t m, n, groups;
+    double start, trip, end, walk_idle, end_idle;
+  };
+  static constexpr Form forms[] = {{64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},
+                                   {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60},
+                                   {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45}, {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37},
+                                   {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
+  const int64_t steps = (K + 63) / 64;
+  double least = 1e30;
+  for (const Form& f : forms) {
+    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n), most = 256 / tiles;
+    for (const int64_t parts : {most, 2 * most / 3, most / 2}) {
+      if (parts < 2 || parts > 64 || steps < 2 * parts) continue;
+      const double walk = ((steps + parts - 1) / parts + f.groups - 1) / f.groups * f.trip;
+      const double t = f.start + last_round(0.93 * walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 4.8 + 1e-6 * M * N * (1.41 * parts - 2.43);
+      if (t < least) {
+        least = t;
+        best = {f.m, f.n, parts};
+      }
     }
   }
   return least;
@@ -1266,6 +1297,11 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
   MidProduct best;
   LargeProduct same;
   const double time = mid_time(M, N, K, best);
+  if (kind == Product::NN && (large.parts > 0 || (own.groups == 0 && contraction_parts(kind, M, N, K) > 1))) {
+    MidProduct cut;
+    const double other = large_time(M, N, K, same), pieces = mid_parts_time(M, N, K, cut);
+    if (pieces < time && pieces < (large.parts > 0 ? 0.88 : 0.95) * other) return cut;
+  }
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
   else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
@@ -1277,8 +1313,10 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
 }
 Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {
   Tensor c = at::empty({n.M, n.N}, a.options());
-  check(pico_product_mid(ptr(a), ptr(b), ptr(c), n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
-                         static_cast<int>(mid.tile_m), static_cast<int>(mid.tile_n), stream_now()));
+  const Tensor sums = mid.parts > 1 ? at::empty({mid.parts, n.M, n.N}, a.options().dtype(at::kFloat)) : Tensor();
+  check(pico_product_mid(ptr(a), ptr(b), mid.parts > 1 ? ptr(sums) : ptr(c), n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN,
+                         kind != Product::NT, static_cast<int>(mid.tile_m), static_cast<int>(mid.tile_n), static_cast<int>(mid.parts), stream_now()));
+  if (mid.parts > 1) check(pico_sum_parts(fptr(sums), ptr(c), mid.parts, n.M * n.N, PICO_BF16, stream_now()));
   return c;
 }
 
@@ -1381,7 +1419,7 @@ GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
       const double t = 1.02 + (0.91 + 0.09 * busy) * (rows > out ? workgroups_end(nw, tw, nx, tx) : workgroups_end(nx, tx, nw, tw));
       if (t < least) {
         least = t;
-        best = {{x.m, x.n}, {w.m, w.n}};
+        best = {{x.m, x.n, 1}, {w.m, w.n, 1}};
       }
     }
   MidProduct alone;
@@ -1859,20 +1897,20 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return product(a, b, product_kind(kind), parts, turn, groups, tile, tile_n);
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
         pybind11::arg("groups") = -1, pybind11::arg("tile") = 64, pybind11::arg("tile_n") = 0);
-  m.def("mid_product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t tile_m, int64_t tile_n) {
+  m.def("mid_product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t tile_m, int64_t tile_n, int64_t parts) {
     TORCH_CHECK(!stays_with_torch(a, b), "mid_product: operands that stay with torch");
     const c10::OptionalDeviceGuard device(a.device());
     const Product k = product_kind(kind);
     const ProductSizes n = product_sizes(a, b, k);
-    const MidProduct mid = tile_m > 0 ? MidProduct{tile_m, tile_n} : mid_product(k, n, a, b, large_product(k, n, a, b), own_product(k, n, a, b));
+    const MidProduct mid = tile_m > 0 ? MidProduct{tile_m, tile_n, parts} : mid_product(k, n, a, b, large_product(k, n, a, b), own_product(k, n, a, b));
     if (mid.tile_m == 0) return std::make_tuple(Tensor(), mid.tile_m, mid.tile_n);
     return std::make_tuple(mid_product(a, b, k, n, mid), mid.tile_m, mid.tile_n);
-  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m") = 0, pybind11::arg("tile_n") = 0);
+  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m") = 0, pybind11::arg("tile_n") = 0, pybind11::arg("parts") = 1);
   // (dx, dw, the tiles of each or 0); tiles given: in one launch of these
   m.def("gradients", [](const Tensor& dy, const Tensor& w, const Tensor& x, std::vector<int64_t> tiles) {
     TORCH_CHECK(tiles.empty() || (tiles.size() == 4 && !stays_with_torch(dy, w) && !stays_with_torch(dy, x)),
                 "gradients: four tile sides, operands that do not stay with torch");
-    const GradientTiles t = tiles.empty() ? gradient_tiles(dy, w, x) : GradientTiles{{tiles[0], tiles[1]}, {tiles[2], tiles[3]}};
+    const GradientTiles t = tiles.empty() ? gradient_tiles(dy, w, x) : GradientTiles{{tiles[0], tiles[1], 1}, {tiles[2], tiles[3], 1}};
     Gradients d = gradients(dy, w, x, t);
     return std::make_tuple(d.dx, d.dw, t.dx.tile_m, t.dx.tile_n, t.dw.tile_m, t.dw.tile_n);
   }, pybind11::arg("dy"), pybind11::arg("w"), pybind11::arg("x"), pybind11::arg("tiles") = std::vector<int64_t>());

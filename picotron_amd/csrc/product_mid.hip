@@ -19,10 +19,10 @@ namespace {
 
 struct MidParams {
   const __bf16 *a, *b;
-  __bf16* c;
+  void* c;            // bf16 [M, N], or fp32 [parts, M, N]
   int M, N, K;
   int64_t lda, ldb;   // elements between the rows of a and b as they lie in memory
-  int tiles_m, tiles_n;
+  int tiles_m, tiles_n, parts;
 };
 
 // Eight waves: KS groups deal the steps of the contraction between them, and the WM x WN waves of a group take 16 I x 16 J of the
@@ -40,7 +40,7 @@ struct Form {
   static_assert(kLds <= 160 * 1024);
 };
 
-template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN>
+template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN, bool kParts = false>
 __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
   using F = Form<kSlowA, kSlowB, I, J, WM, WN>;
   using A = typename F::A;
@@ -51,12 +51,14 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
   const int group = wave / (WM * WN), in_group = wave % (WM * WN), gtid = in_group * kWave + lane;
   const int wm = in_group / WN * 16 * I, wn = in_group % WN * 16 * J;
   // workgroups go round the eight XCDs: each takes a run of neighbouring tiles, along the shorter side of the output
-  const int tiles = p.tiles_m * p.tiles_n, xcd = block % 8, id = xcd * (tiles / 8) + min(xcd, tiles % 8) + block / 8;
+  const int tiles = p.tiles_m * p.tiles_n, units = kParts ? tiles * p.parts : tiles, xcd = block % 8;
+  const int unit = xcd * (units / 8) + min(xcd, units % 8) + block / 8, part = kParts ? unit / tiles : 0, id = kParts ? unit % tiles : unit;
   const bool down = p.tiles_m < p.tiles_n;
   const int m0 = (down ? id % p.tiles_m : id / p.tiles_n) * TM, n0 = (down ? id / p.tiles_m : id % p.tiles_n) * TN;
 
   // ---- requests: the group's steps are group, group + KS, ...
-  const int steps = (p.K + kStep - 1) / kStep, trips = (steps + KS - 1) / KS;
+  const int all = (p.K + kStep - 1) / kStep, from = kParts ? static_cast<int>(static_cast<int64_t>(part) * all / p.parts) : 0;
+  const int steps = kParts ? static_cast<int>(static_cast<int64_t>(part + 1) * all / p.parts) - from : all, trips = (steps + KS - 1) / KS;   // (one at least)
   uint32_t oa[kPA], ob[kPB];
 #pragma unroll
   for (int i = 0; i < kPA; ++i) oa[i] = A::offset(p.lda, gtid, i);
@@ -64,10 +66,10 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
   for (int i = 0; i < kPB; ++i) ob[i] = B::offset(p.ldb, gtid, i);
   const uint32_t step_a = static_cast<uint32_t>(KS * (kSlowA ? kStep * p.lda * 2 : kStep * 2)), step_b = static_cast<uint32_t>(KS * (kSlowB ? kStep * p.ldb * 2 : kStep * 2));
   const int first = min(group, steps - 1);   // (a group without steps requests nothing)
-  Window wa = open_window<kSlowA>(p.a, p.lda, m0, TM, p.M, first * kStep, p.K);
-  Window wb = open_window<kSlowB>(p.b, p.ldb, n0, TN, p.N, first * kStep, p.K);
+  Window wa = open_window<kSlowA>(p.a, p.lda, m0, TM, p.M, (from + first) * kStep, p.K);
+  Window wb = open_window<kSlowB>(p.b, p.ldb, n0, TN, p.N, (from + first) * kStep, p.K);
   int load = group;   // the step that is requested next
-  const int k_piece = (gtid % 8 ^ (gtid / 16 & 7)) * 8, k_last = p.K - (steps - 1) * kStep;
+  const int k_piece = (gtid % 8 ^ (gtid / 16 & 7)) * 8, k_last = p.K - (from + steps - 1) * kStep;   // (a part that ends before the contraction does has whole steps)
   auto request_step = [&](uint32_t to) __attribute__((always_inline)) {
     if (load >= steps) wa.bytes = wb.bytes = 0;   // requests past the contraction's end read no memory
     if constexpr (!(kSlowA && kSlowB)) {
@@ -152,6 +154,21 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
           for (int j = 0; j < J; ++j) acc[i][j] += *place(g, i, j);
     }
   }
+  if constexpr (kParts) {   // a lane's four columns at a time
+    if (group == 0) {
+      float* c = static_cast<float*>(p.c) + static_cast<int64_t>(part) * p.M * p.N;
+#pragma unroll
+      for (int i = 0; i < I; ++i) {
+        const int row = m0 + wm + 16 * i + lane % 16;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int col = n0 + wn + 16 * j + 4 * (lane / 16);
+          if (row < p.M && col < p.N) *reinterpret_cast<f32x4*>(c + static_cast<int64_t>(row) * p.N + col) = acc[i][j];
+        }
+      }
+    }
+    return;
+  }
   // ---- the tile leaves through LDS as whole lines (behind the groups' sums, which may still be read)
   unsigned char* out = lds + F::kSums;
   if (group == 0) {
@@ -170,24 +187,24 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
   for (int idx = tid; idx < TM * TN / 8; idx += 512) {
     const int r = idx / (TN / 8), cv = idx % (TN / 8);
     if (m0 + r < p.M && n0 + cv * 8 < p.N)
-      *reinterpret_cast<u32x4*>(p.c + static_cast<int64_t>(m0 + r) * p.N + n0 + cv * 8) = *reinterpret_cast<const u32x4*>(out + r * F::kOutPitch * 2 + cv * 16);
+      *reinterpret_cast<u32x4*>(static_cast<__bf16*>(p.c) + static_cast<int64_t>(m0 + r) * p.N + n0 + cv * 8) = *reinterpret_cast<const u32x4*>(out + r * F::kOutPitch * 2 + cv * 16);
   }
 }
 
-template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN>
+template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN, bool kParts>
 __global__ __launch_bounds__(512, 2) void product_mid_kernel(const MidParams p) {
-  mid_tile<kSlowA, kSlowB, I, J, WM, WN>(p, blockIdx.x);
+  mid_tile<kSlowA, kSlowB, I, J, WM, WN, kParts>(p, blockIdx.x);
 }
 
-template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN>
+template <bool kSlowA, bool kSlowB, int I, int J, int WM, int WN, bool kParts = false>
 int launch(MidParams p, hipStream_t s) {
   using F = Form<kSlowA, kSlowB, I, J, WM, WN>;
   p.tiles_m = (p.M + F::TM - 1) / F::TM;
   p.tiles_n = (p.N + F::TN - 1) / F::TN;
   static LdsOnce reserved;
-  if (!reserve_lds_once(reserved, reinterpret_cast<const void*>(&product_mid_kernel<kSlowA, kSlowB, I, J, WM, WN>), F::kLds))
+  if (!reserve_lds_once(reserved, reinterpret_cast<const void*>(&product_mid_kernel<kSlowA, kSlowB, I, J, WM, WN, kParts>), F::kLds))
     return fail(PICO_ERR_LAUNCH, "pico_product_mid: cannot reserve %d bytes of LDS", F::kLds);
-  hipLaunchKernelGGL((product_mid_kernel<kSlowA, kSlowB, I, J, WM, WN>), dim3(static_cast<unsigned>(p.tiles_m) * p.tiles_n), dim3(512), F::kLds, s, p);
+  hipLaunchKernelGGL((product_mid_kernel<kSlowA, kSlowB, I, J, WM, WN, kParts>), dim3(static_cast<unsigned>(p.tiles_m) * p.tiles_n * (kParts ? p.parts : 1)), dim3(512), F::kLds, s, p);
   return check_launch("pico_product_mid");
 }
 template <bool kSlowA, bool kSlowB>
@@ -208,6 +225,21 @@ int launch_form(const MidParams& p, int tm, int tn, hipStream_t s) {
     case 192 << 16 | 128: return launch<kSlowA, kSlowB, 6, 2, 2, 4>(p, s);
     case 128 << 16 | 256: return launch<kSlowA, kSlowB, 4, 4, 2, 4>(p, s);
     default: return fail(PICO_ERR_SHAPE, "pico_product_mid: no tiles of %d x %d", tm, tn);
+  }
+}
+
+// The contraction of an input gradient in parts, as fp32 pieces: few tiles and a long contraction, where one round of workgroups takes
+// pieces of tiles ([1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [726 x 8192] @ [8192 x 1024] 29.8 -> 24.8).
+int launch_parts(const MidParams& p, int tm, int tn, hipStream_t s) {
+  switch (tm << 16 | tn) {
+    case 64 << 16 | 96: return launch<false, true, 2, 3, 2, 2, true>(p, s);
+    case 64 << 16 | 128: return launch<false, true, 2, 4, 2, 2, true>(p, s);
+    case 96 << 16 | 96: return launch<false, true, 3, 3, 2, 2, true>(p, s);
+    case 128 << 16 | 128: return launch<false, true, 4, 4, 2, 2, true>(p, s);
+    case 128 << 16 | 192: return launch<false, true, 4, 3, 2, 4, true>(p, s);
+    case 192 << 16 | 128: return launch<false, true, 6, 2, 2, 4, true>(p, s);
+    case 128 << 16 | 256: return launch<false, true, 4, 4, 2, 4, true>(p, s);
+    default: return fail(PICO_ERR_SHAPE, "pico_product_mid: no tiles of %d x %d in parts", tm, tn);
   }
 }
 
@@ -283,14 +315,17 @@ extern "C" int pico_product_mid_takes(int64_t M, int64_t N, int64_t K, int64_t l
 }
 
 extern "C" int pico_product_mid(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow,
-                                int b_slow, int tile_m, int tile_n, void* stream) {
+                                int b_slow, int tile_m, int tile_n, int parts, void* stream) {
   if (!pico_product_mid_takes(M, N, K, lda, ldb, a_slow, b_slow))
     return fail(PICO_ERR_SHAPE, "pico_product_mid: M=%lld N=%lld K=%lld row pitches %lld, %lld (rows of a, b and c and the pitches must be multiples of 8 elements, a tile's rows span less than 2 GiB, no a^T b^T)",
                 (long long)M, (long long)N, (long long)K, (long long)lda, (long long)ldb);
   if (!a || !b || !c) return fail(PICO_ERR_NULL, "pico_product_mid: a, b and c are required");
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return fail(PICO_ERR_ALIGN, "pico_product_mid: pointers must be 16-byte aligned");
-  const MidParams p = {static_cast<const __bf16*>(a), static_cast<const __bf16*>(b), static_cast<__bf16*>(c), (int)M, (int)N, (int)K, lda, ldb, 0, 0};
+  const MidParams p = {static_cast<const __bf16*>(a), static_cast<const __bf16*>(b), c, (int)M, (int)N, (int)K, lda, ldb, 0, 0, parts};
+  if (parts < 1 || parts > 64 || (K + kStep - 1) / kStep < parts || (parts > 1 && (a_slow || !b_slow)))
+    return fail(PICO_ERR_SHAPE, "pico_product_mid: %d parts (1 .. 64, a step of 64 each, input gradients only)", parts);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (parts > 1) return launch_parts(p, tile_m, tile_n, s);
   if (a_slow) return launch_form<true, true>(p, tile_m, tile_n, s);
   return b_slow ? launch_form<false, true>(p, tile_m, tile_n, s) : launch_form<false, false>(p, tile_m, tile_n, s);
 }
@@ -303,8 +338,8 @@ extern "C" int pico_product_pair(const void* dy, const void* w, const void* x, v
   if (!dy || !w || !x || !dx || !dw) return fail(PICO_ERR_NULL, "pico_product_pair: dy, w, x, dx and dw are required");
   if (!aligned16(dy) || !aligned16(w) || !aligned16(x) || !aligned16(dx) || !aligned16(dw)) return fail(PICO_ERR_ALIGN, "pico_product_pair: pointers must be 16-byte aligned");
   MidPairParams p;
-  p.dx = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(w), static_cast<__bf16*>(dx), (int)rows, (int)in, (int)out, ld_dy, ld_w, 0, 0};
-  p.dw = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(x), static_cast<__bf16*>(dw), (int)out, (int)in, (int)rows, ld_dy, ld_x, 0, 0};
+  p.dx = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(w), dx, (int)rows, (int)in, (int)out, ld_dy, ld_w, 0, 0, 1};
+  p.dw = {static_cast<const __bf16*>(dy), static_cast<const __bf16*>(x), dw, (int)out, (int)in, (int)rows, ld_dy, ld_x, 0, 0, 1};
   p.dw_first = rows > out;   // the longer walks start first
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dx_tile_m << 16 | dx_tile_n) {
