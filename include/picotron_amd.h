@@ -340,7 +340,7 @@ int pico_product(const void* a, const void* b, void* c, int64_t M, int64_t N, in
                  int tile, int groups, void* stream);
 
 /* The same as pico_product in tiles of tile_m x tile_n (32 x 32, 32 x 64, 64 x 32, 64 x 64, 64 x 96, 96 x 64, 96 x 96, 64 x 128, 128 x 64,
- * 128 x 96, 128 x 128, 128 x 192, 192 x 128, 128 x 256).  parts > 1 (a_slow 0, b_slow 1, up to 64; 64 x 96, 64 x 128, 96 x 96, 128 x 128, 128 x
+ * 128 x 96, 128 x 128, 128 x 192, 192 x 128, 128 x 256).  parts > 1 (up to 64; 64 x 96, 64 x 128, 96 x 96, 128 x 128, 128 x
  * 192, 192 x 128 and 128 x 256): c is fp32 [parts, M, N], the sums over one piece of the contraction each (see pico_sum_parts).
  */
 int pico_product_mid_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow);

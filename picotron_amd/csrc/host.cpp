@@ -1217,7 +1217,9 @@ LargeProduct large_product(Product kind, const ProductSizes& n, const Tensor& a,
 // Contractions that the library or pico_product_large would cut are cut here where that promises 0.95 (0.88) of pico_product_large's estimate: of 1020 drawn
 // input gradients (100 .. 4096 rows, 192 .. 3072 columns, contractions of 5504 .. 49152) 0.69 of the library's time in its pieces (ten of
 // 347 over 1.02, 1.22 at most) and 0.76 of pico_product_large's (246, 0.98 at most): [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [375 x 11008] @ [11008 x
-// 3072] 51 -> 38, [145 x 49152] @ [49152 x 576] 37 -> 23.
+// 3072] 51 -> 38, [145 x 49152] @ [49152 x 576] 37 -> 23.  The other layouts alike (1000 drawn, contractions of 1500 .. 16384): 0.81 of the
+// library's pieces in the forward's (1.18 at most), 0.77 and 0.73 of pico_product_large's; and where a whole walk goes here, pieces that
+// promise 0.95 of it take 0.82 (1.23 at most; [208 x 5440] @ [256 x 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9).
 struct MidProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 1;
 };
@@ -1249,7 +1251,7 @@ double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
   }
   return least;
 }
-// The same for an input gradient whose contraction is cut into pieces, one round of workgroups of one piece each, and the pieces'
+// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces'
 // sum: 8 % error over 7600 timed (shape, tiles, pieces), 1.3 % over the best ones in the mean.
 double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
   struct Form {
@@ -1297,11 +1299,10 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
   MidProduct best;
   LargeProduct same;
   const double time = mid_time(M, N, K, best);
-  if (kind == Product::NN && (large.parts > 0 || (own.groups == 0 && contraction_parts(kind, M, N, K) > 1))) {
-    MidProduct cut;
-    const double other = large_time(M, N, K, same), pieces = mid_parts_time(M, N, K, cut);
-    if (pieces < time && pieces < (large.parts > 0 ? 0.88 : 0.95) * other) return cut;
-  }
+  MidProduct cut;
+  const double pieces = mid_parts_time(M, N, K, cut);
+  const bool cut_elsewhere = large.parts > 0 || (own.groups == 0 && contraction_parts(kind, M, N, K) > 1);
+  if (cut_elsewhere && pieces < time && pieces < (kind == Product::NN && large.parts == 0 ? 0.95 : 0.88) * large_time(M, N, K, same)) return cut;
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
   else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
@@ -1309,7 +1310,8 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, con
     const double gflop = 2e-9 * M * N * K;
     take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? (gflop < 20 ? 1.0 : 0.9) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
   }
-  return take ? best : MidProduct{};
+  if (!take) return {};
+  return pieces < 0.95 * time ? cut : best;
 }
 Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {
   Tensor c = at::empty({n.M, n.N}, a.options());

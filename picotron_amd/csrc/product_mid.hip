@@ -228,17 +228,18 @@ int launch_form(const MidParams& p, int tm, int tn, hipStream_t s) {
   }
 }
 
-// The contraction of an input gradient in parts, as fp32 pieces: few tiles and a long contraction, where one round of workgroups takes
+// The contraction in parts, as fp32 pieces: few tiles and a long contraction, where one round of workgroups takes
 // pieces of tiles ([1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [726 x 8192] @ [8192 x 1024] 29.8 -> 24.8).
+template <bool kSlowA, bool kSlowB>
 int launch_parts(const MidParams& p, int tm, int tn, hipStream_t s) {
   switch (tm << 16 | tn) {
-    case 64 << 16 | 96: return launch<false, true, 2, 3, 2, 2, true>(p, s);
-    case 64 << 16 | 128: return launch<false, true, 2, 4, 2, 2, true>(p, s);
-    case 96 << 16 | 96: return launch<false, true, 3, 3, 2, 2, true>(p, s);
-    case 128 << 16 | 128: return launch<false, true, 4, 4, 2, 2, true>(p, s);
-    case 128 << 16 | 192: return launch<false, true, 4, 3, 2, 4, true>(p, s);
-    case 192 << 16 | 128: return launch<false, true, 6, 2, 2, 4, true>(p, s);
-    case 128 << 16 | 256: return launch<false, true, 4, 4, 2, 4, true>(p, s);
+    case 64 << 16 | 96: return launch<kSlowA, kSlowB, 2, 3, 2, 2, true>(p, s);
+    case 64 << 16 | 128: return launch<kSlowA, kSlowB, 2, 4, 2, 2, true>(p, s);
+    case 96 << 16 | 96: return launch<kSlowA, kSlowB, 3, 3, 2, 2, true>(p, s);
+    case 128 << 16 | 128: return launch<kSlowA, kSlowB, 4, 4, 2, 2, true>(p, s);
+    case 128 << 16 | 192: return launch<kSlowA, kSlowB, 4, 3, 2, 4, true>(p, s);
+    case 192 << 16 | 128: return launch<kSlowA, kSlowB, 6, 2, 2, 4, true>(p, s);
+    case 128 << 16 | 256: return launch<kSlowA, kSlowB, 4, 4, 2, 4, true>(p, s);
     default: return fail(PICO_ERR_SHAPE, "pico_product_mid: no tiles of %d x %d in parts", tm, tn);
   }
 }
@@ -322,10 +323,11 @@ extern "C" int pico_product_mid(const void* a, const void* b, void* c, int64_t M
   if (!a || !b || !c) return fail(PICO_ERR_NULL, "pico_product_mid: a, b and c are required");
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return fail(PICO_ERR_ALIGN, "pico_product_mid: pointers must be 16-byte aligned");
   const MidParams p = {static_cast<const __bf16*>(a), static_cast<const __bf16*>(b), c, (int)M, (int)N, (int)K, lda, ldb, 0, 0, parts};
-  if (parts < 1 || parts > 64 || (K + kStep - 1) / kStep < parts || (parts > 1 && (a_slow || !b_slow)))
-    return fail(PICO_ERR_SHAPE, "pico_product_mid: %d parts (1 .. 64, a step of 64 each, input gradients only)", parts);
+  if (parts < 1 || parts > 64 || (K + kStep - 1) / kStep < parts)
+    return fail(PICO_ERR_SHAPE, "pico_product_mid: %d parts (1 .. 64, a step of 64 each)", parts);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (parts > 1) return launch_parts(p, tile_m, tile_n, s);
+  if (parts > 1)
+    return a_slow ? launch_parts<true, true>(p, tile_m, tile_n, s) : b_slow ? launch_parts<false, true>(p, tile_m, tile_n, s) : launch_parts<false, false>(p, tile_m, tile_n, s);
   if (a_slow) return launch_form<true, true>(p, tile_m, tile_n, s);
   return b_slow ? launch_form<false, true>(p, tile_m, tile_n, s) : launch_form<false, false>(p, tile_m, tile_n, s);
 }

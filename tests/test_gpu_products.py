@@ -200,19 +200,21 @@ def test_products_of_one_round(device, kind, M, N, K):
         host.mid_product(a, b, kind, 96, 128)
 
 
-@pytest.mark.parametrize("M,N,K", [(72, 136, 1000), (300, 200, 4096), (64, 96, 256), (129, 264, 8200)])
-def test_input_gradients_in_pieces_of_one_round(device, M, N, K):
+@pytest.mark.parametrize("M,N,K", [(72, 136, 1000), (304, 200, 4096), (64, 96, 256), (136, 264, 8200)])
+@pytest.mark.parametrize("kind", ["NT", "NN", "TN"])
+def test_products_in_pieces_of_one_round(device, kind, M, N, K):
     """Every tile that takes pieces, as many as the steps allow at most, a ragged last step, and the rule's own choice."""
     from picotron_amd import _lib
     host = _lib.host()
     g = torch.Generator(device="cuda").manual_seed(K)
-    a, b = (torch.randn(r, c + 16, generator=g, device=device).to(torch.bfloat16)[:, 8:8 + c] for r, c in ((M, K), (K, N)))
-    want, steps = a.float() @ b.float(), (K + 63) // 64
+    sizes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    a, b = (torch.randn(r, c + 16, generator=g, device=device).to(torch.bfloat16)[:, 8:8 + c] for r, c in sizes)
+    want, steps = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float()), (K + 63) // 64
     for tiles in [(64, 96), (64, 128), (96, 96), (128, 128), (128, 192), (192, 128), (128, 256)]:
         for parts in {2, 3, min(steps, 15), min(steps, 64)}:
-            got = host.mid_product(a, b, "NN", *tiles, parts)[0]
+            got = host.mid_product(a, b, kind, *tiles, parts)[0]
             assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (tiles, parts)
-    assert ((host.product(a, b, "NN").float() - want).norm() / want.norm()).item() <= 3e-3
+    assert ((host.product(a, b, kind).float() - want).norm() / want.norm()).item() <= 3e-3
     for bad in ((64, 64, 2), (64, 96, 65), (64, 96, steps + 1)):
         with pytest.raises(RuntimeError):
-            host.mid_product(a, b, "NN", *bad)
+            host.mid_product(a, b, kind, *bad)
