@@ -85,17 +85,23 @@ __device__ __forceinline__ float buffer_load_f32(buffer_rsrc r, uint32_t byte_of
 
 // ---- loads that go to LDS without passing the registers: 16 bytes per lane, lane after lane from m0 on; zeros past the window.
 // In assembly, because the compiler makes every later read of LDS wait for the builtin: the caller waits by hand
-// (wait_requests) before the barrier that publishes the tile.  The kernel's dynamic LDS has to start at 0 (no static LDS).
+// (wait_requests) before the barrier that publishes the tile.  The kernel's dynamic LDS has to start at 0 (no static LDS).  m0 is an
+// output of what writes it and an operand of what reads it, so that the compiler keeps nothing of its own there across a request
+// and puts nothing there between the two statements.
 template <int kPlus>
-__device__ __forceinline__ void aim_request(uint32_t lds_off) {   // one instruction has to lie between this and the request
-  asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds_off), "n"(kPlus) : "scc", "memory");
+__device__ __forceinline__ uint32_t aim_request(uint32_t lds_off) {   // one instruction has to lie between this and the request
+  uint32_t aim;
+  asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(aim) : "s"(lds_off), "n"(kPlus) : "scc", "memory");
+  return aim;
 }
-__device__ __forceinline__ void request16(u32x4 window, uint32_t off) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(window) : "memory");
+__device__ __forceinline__ void request16(uint32_t aim, u32x4 window, uint32_t off) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(window), "{m0}"(aim) : "memory");
 }
 template <int kPlus>
 __device__ __forceinline__ void request16_to(uint32_t lds_off, u32x4 window, uint32_t off) {
-  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds" ::"s"(lds_off), "n"(kPlus), "v"(off), "s"(window) : "scc", "memory");
+  uint32_t aim;
+  asm volatile("s_add_u32 %0, %1, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds"
+               : "=&{m0}"(aim) : "s"(lds_off), "n"(kPlus), "v"(off), "s"(window) : "scc", "memory");
 }
 // all but the wave's newest N vector memory operations are complete
 template <int N>

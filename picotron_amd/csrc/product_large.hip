@@ -142,12 +142,12 @@ __global__ __launch_bounds__(512, 2) void product_large_kernel(const LargeParams
   const uint32_t lds_wave = wave * 1024;   // (dynamic LDS starts at 0)
   auto aim = [&](auto piece, uint32_t buffer) __attribute__((always_inline)) {
     constexpr int i = decltype(piece)::value;
-    aim_request<(i < kPA ? i * S::kThreads * 16 : A::kBytes + (i - kPA) * S::kThreads * 16)>(lds_wave + buffer);
+    return aim_request<(i < kPA ? i * S::kThreads * 16 : A::kBytes + (i - kPA) * S::kThreads * 16)>(lds_wave + buffer);
   };
-  auto request = [&](auto piece) __attribute__((always_inline)) {
+  auto request = [&](auto piece, uint32_t aimed) __attribute__((always_inline)) {
     constexpr int i = decltype(piece)::value;
-    if constexpr (i < kPA) request16(ra, oa[i]);
-    else request16(rb, ob[i - kPA]);
+    if constexpr (i < kPA) request16(aimed, ra, oa[i]);
+    else request16(aimed, rb, ob[i - kPA]);
   };
 
   // ---- half a step: its products, and behind each at most one other thing: a fragment of the half step that follows, a
@@ -171,7 +171,8 @@ __global__ __launch_bounds__(512, 2) void product_large_kernel(const LargeParams
       constexpr int first = here ? (place * kPieces + kPlaces - 1) / kPlaces : 0, last = here ? ((place + 1) * kPieces + kPlaces - 1) / kPlaces : 0;
       static_assert(last <= first + 1);
       using Piece = std::integral_constant<int, first>;
-      if constexpr (last > first) aim(Piece(), free);
+      [[maybe_unused]] uint32_t aimed = 0;
+      if constexpr (last > first) aimed = aim(Piece(), free);
       __builtin_amdgcn_sched_barrier(0);
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);   // C^T: a lane holds four columns of a row of C
       __builtin_amdgcn_sched_barrier(0);
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(512, 2) void product_large_kernel(const LargeParams
         wait_lds();
         arrive(kFree);
       }
-      if constexpr (last > first) request(Piece());
+      if constexpr (last > first) request(Piece(), aimed);
       if constexpr (s == 0 && m % (kProducts / 4) == 1) go_on(m / (kProducts / 4));
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -192,9 +193,9 @@ __global__ __launch_bounds__(512, 2) void product_large_kernel(const LargeParams
 
   auto all_requests = [&](uint32_t buffer) __attribute__((always_inline)) {
     each(std::make_integer_sequence<int, kPieces>(), [&](auto piece) __attribute__((always_inline)) {
-      aim(piece, buffer);
+      const uint32_t aimed = aim(piece, buffer);
       asm volatile("s_nop 0");
-      request(piece);
+      request(piece, aimed);
     });
   };
   all_requests(0);

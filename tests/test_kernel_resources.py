@@ -1,4 +1,6 @@
-"""What the compiler reports for kernels whose speed rests on it: no register of the loss kernels lives in scratch memory."""
+"""What the compiler makes of kernels whose speed or safety rests on it: registers, scratch memory, and the requests that go to LDS
+without passing the registers."""
+import functools
 import os
 import re
 import shutil
@@ -9,36 +11,47 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def resources(source, tmp_path):
-    """{mangled kernel name: {remark: value}} of csrc/<source>, compiled with the package's own flags."""
+@functools.lru_cache(maxsize=None)
+def compiled(path):
+    """({mangled kernel name: {remark: value}}, device assembly) of a source, compiled with the package's own flags."""
     from picotron_amd import build
     if shutil.which(build._hipcc()) is None:
         pytest.skip("no hipcc")
-    out = subprocess.run([build._hipcc(), *build.FLAGS, "-c", os.path.join(build.CSRC, source), "-o", str(tmp_path / "out.o"),
-                          "-Rpass-analysis=kernel-resource-usage"], capture_output=True, text=True, timeout=600, check=True).stderr
+    res = subprocess.run([build._hipcc(), *build.FLAGS, f"-I{build.CSRC}", "--cuda-device-only", "-S", path, "-o", "-",
+                          "-Rpass-analysis=kernel-resource-usage"], capture_output=True, text=True, timeout=600)
+    assert res.returncode == 0, res.stderr
     kernels, now = {}, None
-    for key, value in re.findall(r"remark: (?:\S+:\d+:\d+: )?\s*([A-Za-z ]+?)(?: \[[^\]]*\])?: (\S+) \[-Rpass", out):
+    for key, value in re.findall(r"remark: (?:\S+:\d+:\d+: )?\s*([A-Za-z ]+?)(?: \[[^\]]*\])?: (\S+) \[-Rpass", res.stderr):
         if key == "Function Name":
             now = kernels.setdefault(value, {})
         else:
             now[key] = int(value) if value.isdigit() else value
-    return kernels
+    return kernels, res.stdout
 
 
-def test_loss_kernels_keep_the_row_in_registers(tmp_path):
-    kernels = resources("loss.hip", tmp_path)
+def csrc(source):
+    from picotron_amd import build
+    return os.path.join(build.CSRC, source)
+
+
+def resources(source):
+    return compiled(csrc(source))[0]
+
+
+def test_loss_kernels_keep_the_row_in_registers():
+    kernels = resources("loss.hip")
     assert sum("ce_one_pass_kernel" in name for name in kernels) == 22
     for name, r in kernels.items():
         assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0, (name, r)
 
 
-def test_attention_kernels_fit_a_cu_as_often_as_their_plans_count_on(tmp_path):
+def test_attention_kernels_fit_a_cu_as_often_as_their_plans_count_on():
     """Registers: waves per SIMD x 4 SIMDs hold the workgroups of a CU (LDS is asserted where the tiles are laid out), and
     none of them are in scratch.  Eight waves have a CU to themselves at head_dim 128 and with split keys, and in dQ; the
     four waves of dQ at head_dim 128 do as well."""
     per_cu = {}
     for source in ("attn_fwd.hip", "attn_bwd.hip"):
-        for name, r in resources(source, tmp_path).items():
+        for name, r in resources(source).items():
             assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0, (name, r)
             numbers = [int(n) for n in re.findall(r"L[ib](\d+)E", name)]
             if "attn_fwd_kernel" in name:
@@ -71,3 +84,59 @@ def test_launches_that_fill_the_gpu_run_whole(B, Hq, Hkv, S, D):
     d = ops._desc(q, k, k, q, 1 / math.sqrt(D), True, 0)
     assert _lib.lib().pico_attn_fwd_workspace_bytes(ctypes.byref(d), 1) == 0
     assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == 0
+
+
+REQUESTING = ("product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip")   # tiles go to LDS without passing the registers
+
+
+@pytest.mark.parametrize("source", REQUESTING)
+def test_requests_find_their_aim_in_m0(source):
+    """m0 is written by nothing but the statement that aims a request, in the same straight run of code, and one instruction at least
+    lies between the two (the hardware asks for one, and the compiler does not look into the statements)."""
+    lines = [l.split(";")[0].strip() for l in compiled(csrc(source))[1].splitlines()]
+    lines = [l for l in lines if l and not l.startswith((".", "//", "#"))]
+    requests, aimed = 0, None                       # instructions since m0 was written; None: not in this run of code
+    for line in lines:
+        if "pico_wait_" in line:                    # (a wait that goes round by itself: entered from above only, and m0 stays)
+            continue
+        if line.endswith(":"):
+            aimed = None
+            continue
+        if re.search(r"\bm0\b", line):
+            assert line.startswith("s_add_u32 m0,"), line
+            assert aimed is None or aimed < 0, line  # (the aim before has been used)
+            aimed = 0
+            continue
+        if line.startswith("buffer_load") and line.endswith(" lds"):
+            assert aimed is not None and aimed >= 1, line
+            requests, aimed = requests + 1, -1
+        elif aimed is not None and aimed >= 0:
+            aimed = None if line.startswith(("s_cbranch", "s_branch", "s_setpc", "s_endpgm")) else aimed + 1
+    assert requests > 100
+
+
+def test_the_compiler_keeps_nothing_in_m0_across_a_request(tmp_path):
+    """A value that the compiler has in m0 before a request is written there again after it (never run: compiled only)."""
+    source = tmp_path / "around.hip"
+    source.write_text('''#include "attn_common.h"
+using namespace pico;
+extern "C" __global__ void whole(uint64_t base, uint32_t bytes, uint32_t to) {
+  const u32x4 window = request_window(base, bytes);
+  __builtin_amdgcn_s_sendmsg(1, 40);
+  request16_to<16>(to, window, threadIdx.x * 16);
+  __builtin_amdgcn_s_sendmsg(1, 40);
+}
+extern "C" __global__ void parted(uint64_t base, uint32_t bytes, uint32_t to) {
+  const u32x4 window = request_window(base, bytes);
+  __builtin_amdgcn_s_sendmsg(1, 40);
+  const uint32_t aim = aim_request<16>(to);
+  asm volatile("s_nop 0");
+  request16(aim, window, threadIdx.x * 16);
+  __builtin_amdgcn_s_sendmsg(1, 40);
+}
+''')
+    assembly = compiled(str(source))[1]
+    for name in ("whole", "parted"):
+        body = assembly[assembly.index(f"\n{name}:"):]
+        seen = re.findall(r"s_mov_b32 m0, 40|s_sendmsg|s_add_u32 m0|offen lds", body[:body.index("s_endpgm")])
+        assert seen == ["s_mov_b32 m0, 40", "s_sendmsg", "s_add_u32 m0", "offen lds", "s_mov_b32 m0, 40", "s_sendmsg"], (name, seen)
