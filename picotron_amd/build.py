@@ -9,6 +9,7 @@ so that they travel with the source tree; nothing is installed into site-package
 from __future__ import annotations
 
 import os
+import re
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
@@ -26,6 +27,31 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
+
+# Kernels that wait for a count of their own memory operations: an access to scratch memory would be counted with them, and the wait
+# would end before what it waits for is there.
+COUNTED_WAITS = ("product_mid.hip", "product_large.hip")
+RESOURCES = "-Rpass-analysis=kernel-resource-usage"
+
+
+def kernel_resources(remarks: str) -> dict:
+    """{mangled kernel name: {remark: value}} of what the compiler prints with RESOURCES."""
+    kernels, now = {}, None
+    for key, value in re.findall(r"remark: (?:\S+:\d+:\d+: )?\s*([A-Za-z ]+?)(?: \[[^\]]*\])?: (\S+) \[-Rpass", remarks):
+        if key == "Function Name":
+            now = kernels.setdefault(value, {})
+        else:
+            now[key] = int(value) if value.isdigit() else value
+    return kernels
+
+
+def require_no_scratch(source: str, remarks: str) -> None:
+    kernels = kernel_resources(remarks)
+    if not kernels:
+        raise RuntimeError(f"{source}: the compiler reported no kernel's resources")
+    for name, r in kernels.items():
+        if r["ScratchSize"] or r["VGPRs Spill"] or r["Dynamic Stack"] != "False":
+            raise RuntimeError(f"{source}: {name} keeps registers in scratch memory ({r}), and its counted waits would be wrong")
 
 
 def _hipcc() -> str:
@@ -70,8 +96,11 @@ def build(verbose: bool = True, extra_flags=()) -> str:
 
     def compile_one(src):
         obj = os.path.join(OBJ, src.replace(".hip", ".o"))
-        out = _run([hipcc, *FLAGS, *extra_flags, "-c", os.path.join(CSRC, src), "-o", obj])
-        if verbose and out.strip():
+        counted = src in COUNTED_WAITS
+        out = _run([hipcc, *FLAGS, *extra_flags, *([RESOURCES] if counted else []), "-c", os.path.join(CSRC, src), "-o", obj])
+        if counted:
+            require_no_scratch(src, out)
+        elif verbose and out.strip():
             print(out)
         return obj
 

@@ -17,16 +17,10 @@ def compiled(path):
     from picotron_amd import build
     if shutil.which(build._hipcc()) is None:
         pytest.skip("no hipcc")
-    res = subprocess.run([build._hipcc(), *build.FLAGS, f"-I{build.CSRC}", "--cuda-device-only", "-S", path, "-o", "-",
-                          "-Rpass-analysis=kernel-resource-usage"], capture_output=True, text=True, timeout=600)
+    res = subprocess.run([build._hipcc(), *build.FLAGS, f"-I{build.CSRC}", "--cuda-device-only", "-S", path, "-o", "-", build.RESOURCES],
+                         capture_output=True, text=True, timeout=600)
     assert res.returncode == 0, res.stderr
-    kernels, now = {}, None
-    for key, value in re.findall(r"remark: (?:\S+:\d+:\d+: )?\s*([A-Za-z ]+?)(?: \[[^\]]*\])?: (\S+) \[-Rpass", res.stderr):
-        if key == "Function Name":
-            now = kernels.setdefault(value, {})
-        else:
-            now[key] = int(value) if value.isdigit() else value
-    return kernels, res.stdout
+    return build.kernel_resources(res.stderr), res.stdout
 
 
 def csrc(source):
@@ -62,11 +56,14 @@ def test_attention_kernels_fit_a_cu_as_often_as_their_plans_count_on():
                 want = 2 if NW == 4 and D == 64 else 1
             elif "dkdv_kernel" in name:
                 NW, want = (4, 2) if "_d64" in name else (8, 1)
+            elif "dkdv_few_kernel" in name:
+                NW, want = 8, 1
             else:
+                assert "_kernel" in name and not re.search("dkdv|dq|attn_fwd", name) or "join" in name, name
                 continue
             assert r["Occupancy"] * 4 >= want * NW, (name, r)
             per_cu[name] = want
-    assert len(per_cu) == 12 + 24 + 4
+    assert len(per_cu) == 12 + 24 + 5
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,S,D", [(1, 20, 20, 2500, 128), (1, 20, 20, 3000, 128), (1, 32, 32, 4000, 64), (1, 16, 16, 8000, 64)])
@@ -84,6 +81,34 @@ def test_launches_that_fill_the_gpu_run_whole(B, Hq, Hkv, S, D):
     d = ops._desc(q, k, k, q, 1 / math.sqrt(D), True, 0)
     assert _lib.lib().pico_attn_fwd_workspace_bytes(ctypes.byref(d), 1) == 0
     assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == 0
+
+
+def test_kernels_with_counted_waits_use_no_scratch(tmp_path):
+    """A spill counts among the memory operations of which product_mid and product_large wait for all but the newest few, so the
+    build refuses one; a workgroup of theirs has a CU to itself, two waves per SIMD."""
+    from picotron_amd import build
+    for source, kernels in (("product_mid.hip", 79), ("product_large.hip", 30)):
+        found = resources(source)
+        assert source in build.COUNTED_WAITS and len(found) == kernels
+        for name, r in found.items():
+            assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0 and r["Occupancy"] >= 2, (name, r)
+    spilling = tmp_path / "spilling.hip"
+    spilling.write_text('''#include <hip/hip_runtime.h>
+extern "C" __global__ __launch_bounds__(1024) void spilling(const float* x, float* y) {
+  float v[200];
+#pragma unroll
+  for (int i = 0; i < 200; ++i) v[i] = x[i * 1024 + threadIdx.x];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 200; ++i) y[(i * 7 % 200) * 1024 + threadIdx.x] = v[i] * v[(i * 13 + 5) % 200];
+}
+''')
+    remarks = subprocess.run([build._hipcc(), *build.FLAGS, "--cuda-device-only", "-c", str(spilling), "-o", str(tmp_path / "o"), build.RESOURCES],
+                             capture_output=True, text=True, timeout=600).stderr
+    with pytest.raises(RuntimeError, match="spilling keeps registers in scratch"):
+        build.require_no_scratch("spilling.hip", remarks)
+    with pytest.raises(RuntimeError, match="no kernel"):
+        build.require_no_scratch("silent.hip", "")
 
 
 REQUESTING = ("product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip")   # tiles go to LDS without passing the registers
