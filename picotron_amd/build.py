@@ -28,9 +28,12 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-# Kernels that wait for a count of their own memory operations: an access to scratch memory would be counted with them, and the wait
-# would end before what it waits for is there.
-COUNTED_WAITS = ("product_mid.hip", "product_large.hip")
+# Kernels whose tiles go to LDS without passing the registers, by file and name.  Their dynamic LDS has to start at 0 (no static
+# LDS): the requests count their places from there (an address from the compiler is known too late to fold into them, and costs
+# an addition per request).  And they wait for a count of their own memory operations: an access to scratch memory would be
+# counted with them, and the wait would end before what it waits for is there.
+REQUESTING = {"product_mid.hip": "_kernel", "product_large.hip": "_kernel", "attn_fwd.hip": "attn_fwd_kernel",
+              "attn_bwd.hip": "dkdv_kernel|dkdv_few_kernel|dq_kernel"}
 RESOURCES = "-Rpass-analysis=kernel-resource-usage"
 
 
@@ -45,13 +48,15 @@ def kernel_resources(remarks: str) -> dict:
     return kernels
 
 
-def require_no_scratch(source: str, remarks: str) -> None:
-    kernels = kernel_resources(remarks)
+def check_requesting(source: str, remarks: str) -> None:
+    kernels = {name: r for name, r in kernel_resources(remarks).items() if re.search(REQUESTING[source], name)}
     if not kernels:
-        raise RuntimeError(f"{source}: the compiler reported no kernel's resources")
+        raise RuntimeError(f"{source}: the compiler reported no such kernel's resources")
     for name, r in kernels.items():
         if r["ScratchSize"] or r["VGPRs Spill"] or r["Dynamic Stack"] != "False":
             raise RuntimeError(f"{source}: {name} keeps registers in scratch memory ({r}), and its counted waits would be wrong")
+        if r["LDS Size"]:
+            raise RuntimeError(f"{source}: {name} has LDS of its own ({r}), and its requests would go there")
 
 
 def _hipcc() -> str:
@@ -96,10 +101,10 @@ def build(verbose: bool = True, extra_flags=()) -> str:
 
     def compile_one(src):
         obj = os.path.join(OBJ, src.replace(".hip", ".o"))
-        counted = src in COUNTED_WAITS
-        out = _run([hipcc, *FLAGS, *extra_flags, *([RESOURCES] if counted else []), "-c", os.path.join(CSRC, src), "-o", obj])
-        if counted:
-            require_no_scratch(src, out)
+        requesting = src in REQUESTING
+        out = _run([hipcc, *FLAGS, *extra_flags, *([RESOURCES] if requesting else []), "-c", os.path.join(CSRC, src), "-o", obj])
+        if requesting:
+            check_requesting(src, out)
         elif verbose and out.strip():
             print(out)
         return obj

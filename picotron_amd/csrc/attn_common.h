@@ -85,10 +85,10 @@ __device__ __forceinline__ float buffer_load_f32(buffer_rsrc r, uint32_t byte_of
 
 // ---- loads that go to LDS without passing the registers: 16 bytes per lane, lane after lane from m0 on; zeros past the window.
 // In assembly, because the compiler makes every later read of LDS wait for the builtin: the caller waits by hand
-// (wait_requests) before the barrier that publishes the tile; a spill to scratch would be counted in its place, so the build refuses
-// one where the waits are for less than everything.  The kernel's dynamic LDS has to start at 0 (no static LDS).  m0 is an
-// output of what writes it and an operand of what reads it, so that the compiler keeps nothing of its own there across a request
-// and puts nothing there between the two statements.
+// (wait_requests) before the barrier that publishes the tile.  A spill to scratch would be counted in a request's place, and
+// the kernel's dynamic LDS has to start at 0 (no static LDS): the build refuses kernels that have either.  m0 is an output of what
+// writes it and an operand of what reads it, so that the compiler keeps nothing of its own there across a request and puts nothing
+// there between the two statements.
 template <int kPlus>
 __device__ __forceinline__ uint32_t aim_request(uint32_t lds_off) {   // one instruction has to lie between this and the request
   uint32_t aim;

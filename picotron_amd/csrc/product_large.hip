@@ -139,7 +139,7 @@ __global__ __launch_bounds__(512, 2) void product_large_kernel(const LargeParams
       rb = resource(wb);
     }
   };
-  const uint32_t lds_wave = wave * 1024;   // (dynamic LDS starts at 0)
+  const uint32_t lds_wave = wave * 1024;   // (dynamic LDS starts at 0: the build looks)
   auto aim = [&](auto piece, uint32_t buffer) __attribute__((always_inline)) {
     constexpr int i = decltype(piece)::value;
     return aim_request<(i < kPA ? i * S::kThreads * 16 : A::kBytes + (i - kPA) * S::kThreads * 16)>(lds_wave + buffer);

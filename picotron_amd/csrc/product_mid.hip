@@ -82,7 +82,7 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, int block) {
       }
     }
     const u32x4 ra = resource(wa), rb = resource(wb);
-    const uint32_t at = to + in_group * 1024;   // (dynamic LDS starts at 0)
+    const uint32_t at = to + in_group * 1024;   // (dynamic LDS starts at 0: the build looks)
     each_load<kPA>([&](auto piece) {
       constexpr int i = decltype(piece)::value;
       request16_to<i * F::kGroup * 16>(at, ra, oa[i]);

@@ -83,18 +83,25 @@ def test_launches_that_fill_the_gpu_run_whole(B, Hq, Hkv, S, D):
     assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == 0
 
 
-def test_kernels_with_counted_waits_use_no_scratch(tmp_path):
-    """A spill counts among the memory operations of which product_mid and product_large wait for all but the newest few, so the
-    build refuses one; a workgroup of theirs has a CU to itself, two waves per SIMD."""
+def test_kernels_that_make_requests_have_no_scratch_and_no_lds_of_their_own(tmp_path):
+    """A spill counts among the memory operations of which product_mid and product_large wait for all but the newest few, and the
+    requests' places in LDS are counted from 0: the build refuses both.  A workgroup of the products has a CU to itself, two
+    waves per SIMD.  The kernels that the build looks at are those with requests in their code."""
     from picotron_amd import build
-    for source, kernels in (("product_mid.hip", 79), ("product_large.hip", 30)):
-        found = resources(source)
-        assert source in build.COUNTED_WAITS and len(found) == kernels
-        for name, r in found.items():
-            assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0 and r["Occupancy"] >= 2, (name, r)
-    spilling = tmp_path / "spilling.hip"
-    spilling.write_text('''#include <hip/hip_runtime.h>
-extern "C" __global__ __launch_bounds__(1024) void spilling(const float* x, float* y) {
+    for source, count in (("product_mid.hip", 79), ("product_large.hip", 30), ("attn_fwd.hip", 12), ("attn_bwd.hip", 29)):
+        kernels, assembly = compiled(csrc(source))
+        looked_at = {name for name in kernels if re.search(build.REQUESTING[source], name)}
+        assert len(looked_at) == count
+        for name, r in kernels.items():
+            body = assembly[assembly.index(f"\n{name}:"):]
+            requests = " lds\n" in body[:body.index("s_endpgm")] or " lds\n" in body[:body.index(".Lfunc_end")]
+            assert not requests or name in looked_at, name
+            if name in looked_at:
+                assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0 and r["LDS Size"] == 0, (name, r)
+                assert not source.startswith("product") or r["Occupancy"] >= 2, (name, r)
+    both = tmp_path / "both.hip"
+    both.write_text('''#include <hip/hip_runtime.h>
+extern "C" __global__ __launch_bounds__(1024) void spilling_kernel(const float* x, float* y) {
   float v[200];
 #pragma unroll
   for (int i = 0; i < 200; ++i) v[i] = x[i * 1024 + threadIdx.x];
@@ -102,19 +109,25 @@ extern "C" __global__ __launch_bounds__(1024) void spilling(const float* x, floa
 #pragma unroll
   for (int i = 0; i < 200; ++i) y[(i * 7 % 200) * 1024 + threadIdx.x] = v[i] * v[(i * 13 + 5) % 200];
 }
+extern "C" __global__ void static_kernel(const float* x, float* y) {
+  __shared__ float lds[64];
+  lds[threadIdx.x] = x[threadIdx.x];
+  __syncthreads();
+  y[threadIdx.x] = lds[63 - threadIdx.x];
+}
 ''')
-    remarks = subprocess.run([build._hipcc(), *build.FLAGS, "--cuda-device-only", "-c", str(spilling), "-o", str(tmp_path / "o"), build.RESOURCES],
+    remarks = subprocess.run([build._hipcc(), *build.FLAGS, "--cuda-device-only", "-c", str(both), "-o", str(tmp_path / "o"), build.RESOURCES],
                              capture_output=True, text=True, timeout=600).stderr
-    with pytest.raises(RuntimeError, match="spilling keeps registers in scratch"):
-        build.require_no_scratch("spilling.hip", remarks)
-    with pytest.raises(RuntimeError, match="no kernel"):
-        build.require_no_scratch("silent.hip", "")
+    spilling, static = (remarks[remarks.index(f"Function Name: {name}") - 60:] for name in ("spilling_kernel", "static_kernel"))
+    with pytest.raises(RuntimeError, match="spilling_kernel keeps registers in scratch"):
+        build.check_requesting("product_mid.hip", spilling)
+    with pytest.raises(RuntimeError, match="static_kernel has LDS of its own"):
+        build.check_requesting("product_mid.hip", static)
+    with pytest.raises(RuntimeError, match="no such kernel"):
+        build.check_requesting("product_mid.hip", "")
 
 
-REQUESTING = ("product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip")   # tiles go to LDS without passing the registers
-
-
-@pytest.mark.parametrize("source", REQUESTING)
+@pytest.mark.parametrize("source", ["product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip"])
 def test_requests_find_their_aim_in_m0(source):
     """m0 is written by nothing but the statement that aims a request, in the same straight run of code, and one instruction at least
     lies between the two (the hardware asks for one, and the compiler does not look into the statements)."""
