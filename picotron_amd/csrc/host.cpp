@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/picotron_amd.h"
+#include "product_route.h"
 
 namespace {
 
@@ -937,105 +938,6 @@ bool ordinary(std::initializer_list<const Tensor*> inputs) {
   return true;
 }
 
-// row-major products: a @ b^T, a @ b, a^T @ b
-enum class Product { NT, NN, TN };
-
-// How much of the GPU's 256 CUs a product keeps busy, over the library's tile shapes (256 x 256 and narrower ones, which run
-// at the given share of its rate): output / (waves of workgroups x tile).
-double tile_fit(int64_t M, int64_t N) {
-  double best = 0;
-  for (auto [side, rate] : {std::pair<int64_t, double>(256, 1.0), {192, 0.97}, {160, 0.95}, {128, 0.85}})
-    for (auto [m, n] : {std::pair<int64_t, int64_t>(side, 256), {256, side}}) {
-      const int64_t waves = (((M + m - 1) / m) * ((N + n - 1) / n) + 255) / 256;
-      best = std::max(best, rate * M * N / (256.0 * waves * m * n));
-    }
-  return best;
-}
-
-// Into how many pieces the contraction is cut (1: not at all).  The library works on output tiles and walks the whole
-// contraction in each, so a product of few tiles and a long contraction -- the input gradient of the vocabulary projection
-// or of gate / up, weight gradients of a small model -- leaves most of the GPU idle: [512 x 49152] @ [49152 x 576] took
-// 143 us and takes 53 us in 16 pieces, [2048 x 21760] @ [21760 x 4096] 447 and 291 us in two.  The pieces cost 8 bytes of
-// fp32 traffic per output element each, hence the lower bound on a piece's length and, as output grows, on its ratio to
-// the number of tiles.  The lines lie where sweeps over 100 .. 8192 rows, 192 .. 4096 columns and contractions of 4096 ..
-// 49152 crossed, on the side where no class loses: of 2400 drawn products the 548 that are cut took 0.54 (NN), 0.82 (NT) and
-// 0.74 (TN) of the library's time in the geometric mean, four over 1.06 (1.25 at most: [1076 x 49152] @ [49152 x 3072]).
-// Products of the forward's layout (NT), the library's best, gain only from 8192 on; up to 32 tiles in pieces of 1024 ([128 x
-// 2048] of 8192 17.2 us whole, 22.1 in two, 14.9 in eight), up to 56 of 2048, and at 57 .. 64 not where the library's own
-// split fills the GPU ([512 x 2048] of 8192 27 us, 28.7 in two; [256 x 4096] of 10880 1.23 times).
-// More than 256 tiles and a contraction from 16384 on (NN): the library is fast where one of its tile shapes fills the CUs
-// evenly ([5120 x 49152] @ [49152 x 2048]: 1200 TFLOP/s) and at half that rate elsewhere ([4500 x 49152]: 620, in four
-// pieces 1150).  Contractions under 24576 are never faster in four pieces than in two, and two of 129 .. 192 tiles fill two waves of
-// workgroups badly ([5465 x 16384] @ [16384 x 2048] 286 us, in two 316, in four 440; [4096 x 16384] @ [16384 x 2048] 255 and 230);
-// two of a longer one have to fill the GPU well ([3200 x 32000] @ [32000 x 2048] 395, in two 522, in four 376).
-int64_t contraction_parts(Product kind, int64_t M, int64_t N, int64_t K) {
-  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  if ((M * N) % 8) return 1;   // (pico_sum_parts moves 8 elements at a time)
-  auto cuts = [&](int64_t parts) { return K % parts == 0 && (K / parts) % 32 == 0; };
-  int64_t most = 1, piece = 0;
-  if (kind == Product::NN && tiles > 256) {
-    if (K < 16384 || tile_fit(M, N) >= 0.88) return 1;
-    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-    if (K < 24576) return cuts(2) && (t256 <= 128 || t256 > 192) ? 2 : 1;
-    int64_t best = 1;
-    double least = 1.8;   // (of the ideal time)
-    for (int64_t parts : {2, 4}) {
-      if (!cuts(parts)) continue;
-      const int64_t waves = (t256 * parts + 255) / 256;
-      const double cost = waves * 256.0 * 65536 / (static_cast<double>(M) * N * parts) + 1040.0 * parts / K;
-      if (cost < least && (parts > 2 || cost < 1.28)) {   // (two half-filled waves: 956 us at [6145 x 32000], 792 in four pieces)
-        least = cost;
-        best = parts;
-      }
-    }
-    return best;
-  }
-  if (kind == Product::NN && K >= 5120) {
-    // (narrow outputs of the vocabulary's contraction: [4608 x 49152] @ [49152 x 768] 432 us, in four 540, in eight 346)
-    most = std::min<int64_t>(16, (N < 1024 && N % 256 == 0 && K >= 40000 && tiles > 128 ? 2048 : 1024) / tiles);
-    piece = std::max<int64_t>(1280, 16 * tiles);
-  } else if (kind == Product::TN && K >= 4096) {
-    most = tiles < 256 ? std::min<int64_t>(K >= 16384 ? 4 : 2, 512 / tiles) : 1;
-    piece = 2048;
-  } else if (kind == Product::NT && K >= 8192) {
-    const bool whole = K < 10240 || (M % 256 == 0 && K < 12288);   // (57 .. 64 tiles)
-    most = tiles <= 32 ? 8 : tiles <= 56 || (tiles <= 64 && !whole) ? 4 : tiles > 64 && tiles <= 128 ? 2 : 1;
-    piece = tiles <= 32 ? 1024 : tiles <= 56 ? 2048 : 4096;
-  }
-  int64_t parts = 1;
-  while (2 * parts <= most && cuts(2 * parts) && K / (2 * parts) >= piece) parts *= 2;
-  return parts;
-}
-
-// Which operand of a weight gradient (a^T b, both with the contraction as their slow axis) is transposed first, 1: a, 2: b, 0:
-// none.  The library runs the product at 1000 - 1100 TFLOP/s as it is and 13 % faster where one operand has the contraction
-// as its fast axis, and the narrower operand is small beside the work: [4096 x 49152]^T [4096 x 2048] 732 -> 616 us, the
-// transposition included, [4096 x 16384]^T [4096 x 2048] 227 -> 202, [4096 x 49152]^T [4096 x 576] 289 -> 229.  The gain is
-// proportional to the wider side and to the narrower operand's size, the transposition to the latter plus a launch: the line
-// lies where a sweep over contractions of 512 .. 8192 crossed ([4096 x 6144]^T [4096 x 2048]: 88 and 89 us).  Under 1024 rows
-// the product is bound by writing the result unless the narrower side leaves the library's tiles half empty.
-// (Transposing the wider operand too costs more than the second 13 %.)
-// The library runs the transposed layout in tiles of 256 x 256.  With fewer than 384 of them its gain depends on how they fill
-// the GPU, unless one side is the vocabulary's: over 330 its other layout has better tiles ([4096 x 10880]^T [4096 x 2048] 172
-// us, transposed 273), up to 330 it wins outside 1152 .. 2048 rows ([1280 x 12288]^T [1280 x 1536] 64, 73; from 4096 rows 166,
-// 159), up to 256 from 1536 rows on ([4096 x 8192]^T [4096 x 2048] 124, 112), up to 230 with longer contractions and a side of
-// 8192 at least ([3266 x 9216]^T [3266 x 1152] 0.82 times, [2944 x 8192]^T [2944 x 1024] 1.03).  Short contractions that are no
-// multiple of its step of 64 lose ([1262 x 12288]^T [1262 x 4096] 1.06 times).  Of 212 drawn products that are transposed ten took
-// over 1.04 of the library's time and none over 1.13, 0.91 in the geometric mean.
-int64_t turned_operand(Product kind, const Tensor& a, const Tensor& b) {
-  if (kind != Product::TN) return 0;
-  const int64_t K = a.size(0), M = a.size(1), N = b.size(1), narrow = std::min(M, N), wide = std::max(M, N);
-  if (narrow % 8 || (M < N ? a : b).stride(0) % 8 || (K < 1024 && (K < 768 || narrow >= 1024))) return 0;
-  if (wide <= 5000 + 1e10 / (static_cast<double>(K) * narrow)) return 0;
-  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-  const bool vocabulary = wide >= 24576;
-  if (K % 64 && K < 1408 && t256 < 1024) return 0;
-  if (t256 <= 230 && !vocabulary && (wide < 8192 || K < (t256 > 160 ? 3072 : 4800))) return 0;
-  if (t256 > 230 && t256 <= 256 && !vocabulary && K < (K % 64 ? 2048 : 1536)) return 0;
-  if (t256 > 256 && t256 <= 330 && K > 1152 && K < 2048) return 0;
-  if (t256 > 330 && t256 < 384 && !vocabulary && K > 1024) return 0;
-  return M < N ? 1 : 2;
-}
 // [K, N] -> [N, K], rows padded to 16 bytes
 Tensor turned(const Tensor& t) {
   const int64_t K = t.size(0), N = t.size(1), pitch = (K + 7) / 8 * 8;
@@ -1044,143 +946,14 @@ Tensor turned(const Tensor& t) {
   return y;
 }
 
-// Whether a product goes to the package's own kernel (pico_product), with tiles of which side and how many groups of waves
-// (0: no).  It wins where the library's tiles leave most CUs idle, until either there are more tiles than CUs -- the
-// library's larger ones then do more per byte -- or the walk along the contraction is so long that its steps, and not its
-// start, are the time.  Weight gradients (TN, the library's slowest layout) stay with it longest.  Library and own kernel, us:
-//   TN, tiles of 64 while they are at most 256, or 512 and the walk short: [512 x 960]^T [512 x 576] 9.2, 6.0;
-//      [2331 x 1024]^T [2331 x 1024] 24, 15; [3072 x 576] from 1024 rows 14.2, 13.1, from 4096 35, 37;
-//   TN, up to 256 tiles of 128, two groups: [2048 x 2048] from 512 rows 13.6, 11.3, from 4096 49, 42; [3072 x 1024] from 2630
-//      41, 27; [1024 x 2688] from 4096 41, 40, from 8192 70, 76;
-//   TN, more tiles of 128: few rows.  [49152 x 576] from 512 69, 48, from 1024 93, 89.  The library runs an even number of
-//      its tiles side by side best and a ragged contraction a quarter slower: [32000 x 1024] from 512 46, 48, but [32000 x
-//      1152] 61, 50 and [8192 x 1024] from 443 20, 14;
-//   NN: [512 x 1024] @ [1024 x 1024] 9.2, 7.4; [512 x 3072] @ [3072 x 576] 17.0, 14.2; [512 x 2048] @ [2048 x 2048] 15, 12;
-//      tiles of 128: [4096 x 1536] @ [1536 x 1024] 21, 19, but with 512 of them [4096 x 2048] @ [2048 x 2048] 37, 41;
-//   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.4, 6.8; [512 x 1536] @ [1536 x 576]^T 8.4, 8.8.
-// Over 2400 drawn products of 100 .. 8192 rows, 192 .. 49152 columns and contractions of 100 .. 49152 the time over the
-// library's was, where these lines choose the kernel, 0.75 (NN, 211 products), 0.81 (NT, 115) and 0.70 (TN, 316) in the geometric
-// mean and 1.04 at most.
-struct OwnProduct {
-  int64_t groups, tile;
-};
-OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), wide_tiles = ((M + 127) / 128) * ((N + 127) / 128), narrow = std::min(M, N);
-  constexpr OwnProduct no = {0, 64};
-  if (N % 8 || (kind == Product::TN ? M : K) % 8) return no;
-  if (kind == Product::TN) {
-    if (tiles <= 256) return K <= 384 ? OwnProduct{1, 64} : K <= 3072 ? OwnProduct{2, 64} : K <= 4096 ? OwnProduct{4, 64} : no;
-    if (wide_tiles <= 128) return K <= 2560 ? OwnProduct{1, 64} : no;
-    if (wide_tiles <= 256) return K <= 384 ? OwnProduct{1, 128} : K <= (wide_tiles >= 230 ? 8192 : 4096) ? OwnProduct{2, 128} : no;
-    const int64_t most = narrow % 512 ? (K % 64 ? 1000 : 768) : (K % 64 ? 576 : 320);
-    return K <= most && wide_tiles <= 3500 ? OwnProduct{1, 128} : no;
-  }
-  if (tiles > 512) {
-    if (wide_tiles > 256) return no;
-    return K <= 600 ? OwnProduct{1, 128} : kind == Product::NN && K <= 4096 ? OwnProduct{2, 128} : no;
-  }
-  if (tiles > 256) return K <= 600 ? OwnProduct{1, 64} : no;
-  if (kind == Product::NN) return K <= (tiles <= 32 ? 1088 : tiles <= 64 ? 2112 : 4096) ? OwnProduct{2, 64} : no;
-  return K <= (tiles > 128 ? 3072 : tiles > 60 ? 1088 : 0) ? OwnProduct{2, 64} : no;
-}
-
-// Whether a product goes to the package's kernel for products that fill the GPU (pico_product_large), in which tiles and in how
-// many pieces of the contraction (parts 0: no).
-//
-// The kernel's own time follows from its rounds: 256 workgroups take a tile each, a step of 64 of contraction costs 1.0 .. 1.4
-// us (less while part of the GPU idles), a tile's end 2 .. 5 us.  The estimate below has an error of 7 % (standard deviation)
-// over 20000 timed (shape, tile, pieces); the tile it takes is on average 0.7 % slower than the best one.  Against that stands
-// an estimate of the time without it, of the same form, whose error is 11 .. 34 %: the library's choices are not monotone in
-// any size.  So the lines ask for a margin where the library is good, and for none where it never is.  Of 2100 drawn products of
-// 100 .. 8192 rows those that go here took, in the geometric mean of the time without it,
-//   TN: 0.69 where the library ran them as they are (217 products, 0.99 at most; [4096 x 4096]^T [4096 x 4096] 137 -> 103
-//     us), 0.83 where it had an operand transposed first (91, 1.03 at most; [4096 x 16384]^T [4096 x 2048] 216 -> 199), 0.86 where
-//     pico_product did (13); under 640 of contraction that one stays ahead but for a vocabulary's width, see below, and the
-//     library where the vocabulary meets fewer than 256 columns ([7358 x 49152]^T [7358 x 128] 161 us, here 179);
-//   NN: 0.80 (143, 1.06 at most; [2242 x 10880] @ [10880 x 4096] 248 -> 178, [608 x 49152] @ [49152 x 576] 84 -> 55); a margin is
-//     asked for pieces of four and up, whose rows of a large pitch come more slowly than the estimate has it, and for short
-//     products ([4548 x 1024] @ [1024 x 1024] 17 us, here 20);
-//   NT: 0.77 (42, 1.02 at most): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
-//     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
-//     16384]^T 424 -> 206).
-// A vocabulary's side (24576 and up) is in every step, so its products were swept by themselves (600 of 128 .. 8192 rows, 192 .. 4096
-// columns, vocabularies of 32000 and 49152): they come here
-//   NT up to 768 of contraction, 0.81 of the library's time, none slower ([680 x 576] @ [32000 x 576]^T 57 -> 29 us, [512 x 576] @ [49152
-//     x 576]^T 41 -> 35; with 1024 0.96, and 1.10 at most);
-//   TN under 640 of contraction with 384 columns and up, 0.87 of pico_product's (1.09 at most; [464 x 32000]^T [464 x 1024] 43.6 ->
-//     34.1; with 192 and 256 columns level);
-//   NN where the library would cut the contraction, under 3072 columns, 0.83 (1.12 at most; [4548 x 49152] @ [49152 x 576] 418 ->
-//     258; with 4096 columns 1.00, and 1.21 at most).
-struct LargeProduct {
-  int64_t tile_m = 0, tile_n = 0, parts = 0;
-};
-double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
-  struct Form {
-    int64_t m, n;
-    double step, end;
-  };
-  static constexpr Form forms[] = {{256, 256, 1.43, 4.8}, {256, 192, 1.18, 5.6}, {192, 256, 1.2, 3.2}, {256, 128, 0.99, 2.4}, {128, 256, 1.0, 1.6}};
-  const int64_t steps = (K + 63) / 64;
-  double least = 1e30;
-  for (const Form& f : forms) {
-    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
-    for (int64_t parts : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
-      if (parts > 1 && (tiles * parts > 300 || steps < 8 * parts)) break;
-      const int64_t full = tiles * parts / 256, rest = tiles * parts % 256, length = (steps + parts - 1) / parts;
-      const double used = rest / 256.0;   // of the GPU, in the last round
-      double t = 5 + full * (length * f.step + f.end);
-      if (rest) t += length * f.step * (0.7 + 0.3 * used) + f.end * (0.45 + 0.55 * used);
-      if (parts > 1) t += 3.8 + 1e-6 * M * N * (0.63 * parts + 0.16);   // the pieces in fp32, and their sum
-      if (t < least) {
-        least = t;
-        best = {f.m, f.n, parts};
-      }
-    }
-  }
-  return least;
-}
-// the same without it: the library's tiles (NT, NN), or pico_product's (TN)
-double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
-  struct Form {
-    int64_t m, n;
-    double step[3];   // NT, NN, TN
-  };
-  static constexpr Form forms[] = {{256, 256, {1.37, 1.45, 3.0}}, {256, 192, {1.16, 1.2, 2.0}}, {192, 256, {1.16, 1.2, 2.0}}, {256, 128, {0.72, 0.83, 1.7}},
-                                   {128, 256, {0.72, 0.83, 1.7}}, {128, 128, {0.41, 0.51, 0.88}}, {64, 128, {0.22, 0.19, 0.27}}, {128, 64, {0.22, 0.19, 0.27}}};
-  static constexpr double start[3] = {-1.6, 8.6, 2.2}, end[3] = {8.8, 2.3, 2.4};
-  const int k = static_cast<int>(kind);
-  double least = 1e30;
-  for (const Form& f : forms) {
-    const int64_t rounds = (((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n) + 255) / 256;
-    least = std::min(least, rounds * (K / 64.0 * f.step[k] + end[k]));
-  }
-  return start[k] + least;
-}
-LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
-  static_assert(static_cast<int>(Product::NT) == 0 && static_cast<int>(Product::NN) == 1 && static_cast<int>(Product::TN) == 2);
-  const int64_t narrow = std::min(M, N), wide = std::max(M, N);
-  LargeProduct best;
-  if (M < 1 || N < 1 || K < 128 || narrow < 192 || (wide >= 24576 && narrow < 256)) return {};
-  const double time = large_time(M, N, K, best), ideal = 2e-9 * M * N * K;   // (us at 1 PFLOP/s)
-  const bool small = own_product(kind, M, N, K).groups > 0;
-  bool take = false;
-  const bool vocabulary = std::max(wide, K) >= 24576;   // (see above)
-  if (vocabulary && (kind == Product::TN ? narrow >= 384 && K >= 200 && K < 640 : kind == Product::NT ? K <= 768 : K == std::max(wide, K) && N < 3072 && contraction_parts(kind, M, N, K) > 1)) take = true;
-  else if (kind == Product::TN) take = !small || (K >= 640 && time < 0.9 * other_time(kind, M, N, K));
-  else if (small || time < 14) take = false;
-  else if (kind == Product::NN) take = time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05);
-  else take = time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal);
-  return take ? best : LargeProduct{};
-}
-
-struct ProductSizes {
-  int64_t M, N, K;
-};
 ProductSizes product_sizes(const Tensor& a, const Tensor& b, Product kind) {
   const ProductSizes n = {kind == Product::TN ? a.size(1) : a.size(0), kind == Product::NT ? b.size(0) : b.size(1),
-                          kind == Product::TN ? a.size(0) : a.size(1)};
+                          kind == Product::TN ? a.size(0) : a.size(1), a.stride(0), b.stride(0)};
   TORCH_CHECK((kind == Product::NT ? b.size(1) : b.size(0)) == n.K, "matrix product: shapes ", a.sizes(), " and ", b.sizes(), " do not match");
   return n;
+}
+Tensor torch_product(const Tensor& a, const Tensor& b, Product kind) {
+  return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
 }
 // What torch would do differently, or refuse (operands on two devices), stays with torch.
 bool stays_with_torch(const Tensor& a, const Tensor& b) {
@@ -1188,190 +961,45 @@ bool stays_with_torch(const Tensor& a, const Tensor& b) {
   const bool recorded = at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
   return recorded || !ordinary({&a, &b}) || !plain(a) || !plain(b) || a.device() != b.device() || torch_gemm_only();
 }
-// own_product's choice where the kernel takes the operands as they lie in memory; the library takes any row pitch
-OwnProduct own_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b) {
-  const OwnProduct own = own_product(kind, n.M, n.N, n.K);
-  if (own.groups > 0 && !pico_product_takes(n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT)) return {0, 64};
-  return own;
-}
 
-LargeProduct large_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b) {
-  const LargeProduct large = large_product(kind, n.M, n.N, n.K);
-  const bool takes = large.parts > 0 && pico_product_large_takes(n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
-                                                                 static_cast<int>(large.parts));
-  return takes ? large : LargeProduct{};
-}
-
-// Whether a product goes to pico_product_mid and in which tiles (tile_m 0: no).
-//
-// Its time follows from its rounds: 256 workgroups take a tile each, a trip (64 of contraction for each group of waves) costs `trip`,
-// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy.  Over 25000 timed (shape, tiles) the
-// estimate has an error of 2 .. 6 % (standard deviation; tiles of 32 x 32 10 %), and the tiles it takes are 0.1 % slower than the best
-// ones in the mean.  Against it stands pico_product's own time, estimated alike (4 .. 7 %), or the library's (other_time).  Of 2290 drawn
-// products (64 .. 8192 rows, 72 .. 16384 columns and contraction) the 1430 that go here take, in the geometric mean of the time without it,
-//   NN 0.85 of pico_product's ([512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.69 of the library's ([2331 x 3072] @ [3072 x 576] 27.7 -> 15.8),
-//   TN 0.80 of pico_product's ([2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.82 of pico_product_large's,
-//   NT 0.78 of the library's ([2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5) and 0.93 of pico_product's; two over 1.12, 1.19 at most (the
-// library's choice of tiles is not monotone in any size).  The forward's layout leaves pico_product only for a clear gain: tiles of
-// 64 run level there.
-// Contractions that the library or pico_product_large would cut are cut here where that promises 0.95 (0.88) of pico_product_large's estimate: of 1020 drawn
-// input gradients (100 .. 4096 rows, 192 .. 3072 columns, contractions of 5504 .. 49152) 0.69 of the library's time in its pieces (ten of
-// 347 over 1.02, 1.22 at most) and 0.76 of pico_product_large's (246, 0.98 at most): [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [375 x 11008] @ [11008 x
-// 3072] 51 -> 38, [145 x 49152] @ [49152 x 576] 37 -> 23.  The other layouts alike (1000 drawn, contractions of 1500 .. 16384): 0.81 of the
-// library's pieces in the forward's (1.18 at most), 0.77 and 0.73 of pico_product_large's; and where a whole walk goes here, pieces that
-// promise 0.95 of it take 0.82 (1.23 at most; [208 x 5440] @ [256 x 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9).
-struct MidProduct {
-  int64_t tile_m = 0, tile_n = 0, parts = 1;
-};
-double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
-  return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
-}
-double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
-  struct Form {
-    int64_t m, n, groups;
-    double start, trip, end, walk_idle, end_idle;
-  };
-  static constexpr Form forms[] = {
-      {32, 32, 4, 1.54, 0.50, 1.46, 0.47, 1.12},   {32, 64, 4, 1.37, 0.62, 1.78, 0.64, 1.09},   {64, 32, 4, 1.36, 0.68, 1.71, 0.58, 1.15},
-      {64, 64, 2, 1.51, 0.43, 1.98, 0.80, 0.83},   {64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {96, 64, 2, 1.54, 0.56, 2.29, 0.82, 0.75},
-      {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},  {128, 64, 2, 1.59, 0.67, 2.58, 0.86, 0.70},
-      {128, 96, 2, 1.31, 1.01, 2.83, 0.71, 0.79},  {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60}, {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45},
-      {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37}, {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
-  const int64_t steps = (K + 63) / 64;
-  double least = 1e30;
-  for (const Form& f : forms) {
-    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
-    if (tiles > 1024 || (f.m == 32 && f.n == 32 && steps > 48)) continue;   // (long walks along a slow axis in rows of 64 bytes take twice that)
-    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
-    const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
-    if (t < least) {
-      least = t;
-      best = {f.m, f.n, 1};
+// a product in the kernel of its route; the operands do not stay with torch
+Tensor product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const ProductRoute& route) {
+  const c10::OptionalDeviceGuard device(a.device());
+  const auto [M, N, K, lda, ldb] = n;
+  const int a_slow = kind == Product::TN, b_slow = kind != Product::NT, tile_m = static_cast<int>(route.tile_m), tile_n = static_cast<int>(route.tile_n);
+  const int parts = static_cast<int>(route.parts);
+  TORCH_CHECK(parts >= 1 && (route.kernel != ProductRoute::Library || K % parts == 0), "matrix product: a contraction of ", K, " cannot be cut into ", parts, " equal pieces");
+  Tensor c = at::empty({M, N}, a.options());
+  const Tensor sums = parts > 1 ? at::empty({parts, M, N}, a.options().dtype(at::kFloat)) : Tensor();
+  void* out = parts > 1 ? ptr(sums) : ptr(c);
+  switch (route.kernel) {
+    case ProductRoute::Own:
+      check(pico_product(ptr(a), ptr(b), ptr(c), M, N, K, lda, ldb, a_slow, b_slow, tile_m, static_cast<int>(route.groups), stream_now()));
+      return c;
+    case ProductRoute::Mid:
+      check(pico_product_mid(ptr(a), ptr(b), out, M, N, K, lda, ldb, a_slow, b_slow, tile_m, tile_n, parts, stream_now()));
+      break;
+    case ProductRoute::Large:
+      check(pico_product_large(ptr(a), ptr(b), out, M, N, K, lda, ldb, a_slow, b_slow, tile_m, tile_n, parts, stream_now()));
+      break;
+    case ProductRoute::Library: {
+      // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
+      const Tensor at_ = route.turn & 1 ? turned(a) : a, bt = route.turn & 2 ? turned(b) : b;
+      GemmPlans::Shape s = {a.device().index(), kind == Product::NT || (route.turn & 2), kind == Product::TN && !(route.turn & 1), N, M, K,
+                            bt.stride(0), at_.stride(0), parts};
+      if (gemm_plans().run(s, bt.data_ptr(), at_.data_ptr(), out, a.options())) break;
+      s.parts = 1;
+      if (parts > 1 && gemm_plans().run(s, bt.data_ptr(), at_.data_ptr(), c.data_ptr(), a.options())) return c;
+      return torch_product(a, b, kind);
     }
   }
-  return least;
-}
-// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces'
-// sum: 8 % error over 7600 timed (shape, tiles, pieces), 1.3 % over the best ones in the mean.
-double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
-  struct Form {
-    int64_t m, n, groups;
-    double start, trip, end, walk_idle, end_idle;
-  };
-  static constexpr Form forms[] = {{64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},
-                                   {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60},
-                                   {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45}, {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37},
-                                   {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
-  const int64_t steps = (K + 63) / 64;
-  double least = 1e30;
-  for (const Form& f : forms) {
-    const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n), most = 256 / tiles;
-    for (const int64_t parts : {most, 2 * most / 3, most / 2}) {
-      if (parts < 2 || parts > 64 || steps < 2 * parts) continue;
-      const double walk = ((steps + parts - 1) / parts + f.groups - 1) / f.groups * f.trip;
-      const double t = f.start + last_round(0.93 * walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 4.8 + 1e-6 * M * N * (1.41 * parts - 2.43);
-      if (t < least) {
-        least = t;
-        best = {f.m, f.n, parts};
-      }
-    }
-  }
-  return least;
-}
-double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
-  struct Form {
-    int64_t tile, groups;
-    double start, trip, end, walk_idle, end_idle;
-  };
-  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84}, {64, 4, 2.52, 0.82, 5.90, 1.20, 0.00},
-                                   {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
-  for (const Form& f : forms) {
-    if (f.tile != own.tile || f.groups != own.groups) continue;
-    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
-    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
-    return f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
-  }
-  return 0;
-}
-MidProduct mid_product(Product kind, const ProductSizes& n, const Tensor& a, const Tensor& b, const LargeProduct& large, const OwnProduct& own) {
-  const auto [M, N, K] = n;
-  if (M < 1 || N < 1 || K < 1 || !pico_product_mid_takes(M, N, K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT)) return {};
-  MidProduct best;
-  LargeProduct same;
-  const double time = mid_time(M, N, K, best);
-  MidProduct cut;
-  const double pieces = mid_parts_time(M, N, K, cut);
-  const bool cut_elsewhere = large.parts > 0 || (own.groups == 0 && contraction_parts(kind, M, N, K) > 1);
-  if (cut_elsewhere && pieces < time && pieces < (kind == Product::NN && large.parts == 0 ? 0.95 : 0.88) * large_time(M, N, K, same)) return cut;
-  bool take;
-  if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
-  else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
-  else {   // (a margin that grows with the work: a wrong choice between two full GPUs costs more than it can gain)
-    const double gflop = 2e-9 * M * N * K;
-    take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? (gflop < 20 ? 1.0 : 0.9) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
-  }
-  if (!take) return {};
-  return pieces < 0.95 * time ? cut : best;
-}
-Tensor mid_product(const Tensor& a, const Tensor& b, Product kind, const ProductSizes& n, const MidProduct& mid) {
-  Tensor c = at::empty({n.M, n.N}, a.options());
-  const Tensor sums = mid.parts > 1 ? at::empty({mid.parts, n.M, n.N}, a.options().dtype(at::kFloat)) : Tensor();
-  check(pico_product_mid(ptr(a), ptr(b), mid.parts > 1 ? ptr(sums) : ptr(c), n.M, n.N, n.K, a.stride(0), b.stride(0), kind == Product::TN,
-                         kind != Product::NT, static_cast<int>(mid.tile_m), static_cast<int>(mid.tile_n), static_cast<int>(mid.parts), stream_now()));
-  if (mid.parts > 1) check(pico_sum_parts(fptr(sums), ptr(c), mid.parts, n.M * n.N, PICO_BF16, stream_now()));
+  if (parts > 1) check(pico_sum_parts(fptr(sums), ptr(c), parts, M * N, PICO_BF16, stream_now()));
   return c;
 }
-
-// parts 0, turn -1, groups -1, tile_n 0: by the rules above
-Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0, int64_t turn = -1, int64_t groups = -1, int64_t tile = 64, int64_t tile_n = 0) {
-  if (!stays_with_torch(a, b)) {
-    const c10::OptionalDeviceGuard device(a.device());
-    // row-major C = op(a) op(b) is column-major C^T = op(b)^T op(a)^T: the operands change places
-    const ProductSizes n = product_sizes(a, b, kind);
-    const auto [M, N, K] = n;
-    LargeProduct large = {tile, tile_n, std::max<int64_t>(parts, 1)};
-    const bool by_rule = tile_n == 0 && parts == 0 && turn < 0 && groups < 0;
-    if (tile_n == 0) large = by_rule ? large_product(kind, n, a, b) : LargeProduct{};
-    const OwnProduct own = by_rule ? own_product(kind, n, a, b) : OwnProduct{0, 64};
-    if (by_rule) {
-      const MidProduct mid = mid_product(kind, n, a, b, large, own);
-      if (mid.tile_m > 0) return mid_product(a, b, kind, n, mid);
-    }
-    Tensor c = at::empty({M, N}, a.options());
-    if (large.tile_n > 0) {
-      parts = large.parts;
-      const Tensor sums = parts > 1 ? at::empty({parts, M, N}, a.options().dtype(at::kFloat)) : Tensor();
-      check(pico_product_large(ptr(a), ptr(b), parts > 1 ? ptr(sums) : ptr(c), M, N, K, a.stride(0), b.stride(0), kind == Product::TN,
-                               kind != Product::NT, static_cast<int>(large.tile_m), static_cast<int>(large.tile_n), static_cast<int>(parts), stream_now()));
-      if (parts > 1) check(pico_sum_parts(fptr(sums), ptr(c), parts, M * N, PICO_BF16, stream_now()));
-      return c;
-    }
-    if (groups < 0) {
-      groups = own.groups;
-      tile = own.tile;
-    }
-    if (groups > 0) {
-      check(pico_product(ptr(a), ptr(b), ptr(c), M, N, K, a.stride(0), b.stride(0), kind == Product::TN, kind != Product::NT,
-                         static_cast<int>(tile), static_cast<int>(groups), stream_now()));
-      return c;
-    }
-    if (parts == 0) parts = contraction_parts(kind, M, N, K);
-    TORCH_CHECK(parts >= 1 && K % parts == 0, "matrix product: a contraction of ", K, " cannot be cut into ", parts, " equal pieces");
-    if (turn < 0) turn = turned_operand(kind, a, b);
-    const Tensor at_ = turn & 1 ? turned(a) : a, bt = turn & 2 ? turned(b) : b;
-    GemmPlans::Shape s = {a.device().index(), kind == Product::NT || (turn & 2), kind == Product::TN && !(turn & 1), N, M, K,
-                          bt.stride(0), at_.stride(0), parts};
-    if (parts > 1) {
-      const Tensor sums = at::empty({parts, M, N}, a.options().dtype(at::kFloat));
-      if (gemm_plans().run(s, bt.data_ptr(), at_.data_ptr(), sums.data_ptr(), a.options())) {
-        check(pico_sum_parts(fptr(sums), ptr(c), parts, M * N, PICO_BF16, stream_now()));
-        return c;
-      }
-      s.parts = 1;
-    }
-    if (gemm_plans().run(s, bt.data_ptr(), at_.data_ptr(), c.data_ptr(), a.options())) return c;
-  }
-  return kind == Product::NT ? at::mm(a, b.t()) : kind == Product::NN ? at::mm(a, b) : at::mm(a.t(), b);
+Tensor product(const Tensor& a, const Tensor& b, Product kind) {
+  if (stays_with_torch(a, b)) return torch_product(a, b, kind);
+  const ProductSizes n = product_sizes(a, b, kind);
+  return product(a, b, kind, n, product_route(kind, n));
 }
 
 // dx = dy w and dw = dy^T x, in one launch where neither fills the GPU for long by itself: the launch of the second product and the
@@ -1385,51 +1013,10 @@ Tensor product(const Tensor& a, const Tensor& b, Product kind, int64_t parts = 0
 struct Gradients {
   Tensor dx, dw;
 };
-struct GradientTiles {
-  MidProduct dx, dw;   // (tile_m 0: apart)
-};
-// The time at which the last of n1 workgroups of t1 each, then n2 of t2 each, ends on 256 CUs
-double workgroups_end(int64_t n1, double t1, int64_t n2, double t2) {
-  const int64_t rest = n1 % 256, idle = 256 - rest;
-  const double early = n1 / 256 * t1, late = early + t1, first = rest ? late : early;   // `idle` CUs are free at `early`, `rest` at `late`
-  double end = 1e30;
-  for (const double base : {early, late})
-    for (int64_t k = 0; k <= n2 / 256 + static_cast<int64_t>(t1 / t2) + 2; ++k) {
-      const double at = base + k * t2;
-      const int64_t done = idle * static_cast<int64_t>((at - early) / t2 + 1e-9) + (at >= late ? rest * static_cast<int64_t>((at - late) / t2 + 1e-9) : 0);
-      if (at < first || done < n2) continue;
-      end = std::min(end, at);
-      break;
-    }
-  return end;
-}
-GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
-  struct Form {
-    int64_t m, n, groups;
-    double trip, end;
-  };
-  static constexpr Form forms[] = {{32, 64, 4, 0.72, 1.93}, {64, 64, 2, 0.48, 2.15}, {64, 96, 2, 0.54, 2.50}, {64, 128, 2, 0.68, 2.69}};
-  auto tiles = [](int64_t M, int64_t N, const Form& f) { return ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n); };
-  auto length = [](int64_t K, const Form& f) { return ((K + 63) / 64 + f.groups - 1) / f.groups * f.trip + f.end; };
-  if (tiles(rows, in, forms[3]) + tiles(out, in, forms[3]) > 1024) return {};
-  GradientTiles best;
-  double least = 1e30;
-  for (const Form& x : forms)
-    for (const Form& w : forms) {
-      const int64_t nx = tiles(rows, in, x), nw = tiles(out, in, w);
-      const double tx = length(out, x), tw = length(rows, w), busy = std::min(1.0, (nx + nw) / 256.0);
-      const double t = 1.02 + (0.91 + 0.09 * busy) * (rows > out ? workgroups_end(nw, tw, nx, tx) : workgroups_end(nx, tx, nw, tw));
-      if (t < least) {
-        least = t;
-        best = {{x.m, x.n, 1}, {w.m, w.n, 1}};
-      }
-    }
-  MidProduct alone;
-  return least < 0.94 * (mid_time(rows, in, out, alone) + mid_time(out, in, rows, alone)) ? best : GradientTiles{};
-}
 GradientTiles gradient_tiles(const Tensor& dy, const Tensor& w, const Tensor& x) {
   if (stays_with_torch(dy, w) || stays_with_torch(dy, x)) return {};
-  const auto [rows, in, out] = product_sizes(dy, w, Product::NN);
+  const ProductSizes n = product_sizes(dy, w, Product::NN);
+  const int64_t rows = n.M, in = n.N, out = n.K;
   product_sizes(dy, x, Product::TN);
   if (rows < 1 || in < 1 || out < 1 || !pico_product_mid_takes(rows, in, out, dy.stride(0), w.stride(0), 0, 1) ||
       !pico_product_mid_takes(out, in, rows, dy.stride(0), x.stride(0), 1, 1))
@@ -1447,17 +1034,6 @@ Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x, const Gr
   return r;
 }
 Gradients gradients(const Tensor& dy, const Tensor& w, const Tensor& x) { return gradients(dy, w, x, gradient_tiles(dy, w, x)); }
-
-// the route of a product that large_product and mid_product leave alone, for tests: "torch", "own", "turned" (the library's with an operand transposed first), "library" or
-// "library in N" pieces
-std::string product_route(const Tensor& a, const Tensor& b, Product kind) {
-  if (stays_with_torch(a, b)) return "torch";
-  const ProductSizes n = product_sizes(a, b, kind);
-  if (own_product(kind, n, a, b).groups > 0) return "own";
-  if (turned_operand(kind, a, b)) return "turned";
-  const int64_t parts = contraction_parts(kind, n.M, n.N, n.K);
-  return parts > 1 ? "library in " + std::to_string(parts) : "library";
-}
 
 Tensor linear_forward(const Tensor& x, const Tensor& w) {
   if (x.dim() < 1 || w.dim() != 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || torch_gemm_only() || !ordinary({&x, &w}))
@@ -1889,25 +1465,29 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     TORCH_CHECK(kind == "NT" || kind == "NN" || kind == "TN", "product: kind must be NT, NN or TN");
     return kind == "NT" ? Product::NT : kind == "NN" ? Product::NN : Product::TN;
   };
-  m.def("product_route", [=](const Tensor& a, const Tensor& b, const std::string& kind) { return product_route(a, b, product_kind(kind)); },
-        pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"));
-  m.def("large_product", [=](const Tensor& a, const Tensor& b, const std::string& kind) {
-    const LargeProduct large = stays_with_torch(a, b) ? LargeProduct{} : large_product(product_kind(kind), product_sizes(a, b, product_kind(kind)), a, b);
-    return std::make_tuple(large.tile_m, large.tile_n, large.parts);
+  m.def("product_route", [=](const Tensor& a, const Tensor& b, const std::string& kind) {
+    const Product k = product_kind(kind);
+    return stays_with_torch(a, b) ? std::string("torch") : route_name(product_route(k, product_sizes(a, b, k)));
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"));
+  m.def("gradient_route", [](const Tensor& dy, const Tensor& w, const Tensor& x) {
+    return route_name(gradient_tiles(dy, w, x));
+  }, pybind11::arg("dy"), pybind11::arg("w"), pybind11::arg("x"));
+  // by the rules; tile_n > 0: in pico_product_large; groups > 0: in pico_product; anything else given: in the library, parts 0 and
+  // turn -1 by the rules
   m.def("product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t parts, int64_t turn, int64_t groups, int64_t tile, int64_t tile_n) {
-    return product(a, b, product_kind(kind), parts, turn, groups, tile, tile_n);
+    const Product k = product_kind(kind);
+    if (stays_with_torch(a, b) || (parts == 0 && turn < 0 && groups < 0 && tile_n == 0)) return product(a, b, k);
+    const ProductSizes n = product_sizes(a, b, k);
+    if (tile_n > 0) return product(a, b, k, n, {ProductRoute::Large, tile, tile_n, 0, std::max<int64_t>(parts, 1), 0});
+    if (groups > 0) return product(a, b, k, n, {ProductRoute::Own, tile, tile, groups, 1, 0});
+    return product(a, b, k, n, {ProductRoute::Library, 0, 0, 0, parts == 0 ? contraction_parts(k, n.M, n.N, n.K) : parts, turn < 0 ? turned_operand(k, n) : turn});
   }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("parts") = 0, pybind11::arg("turn") = -1,
         pybind11::arg("groups") = -1, pybind11::arg("tile") = 64, pybind11::arg("tile_n") = 0);
   m.def("mid_product", [=](const Tensor& a, const Tensor& b, const std::string& kind, int64_t tile_m, int64_t tile_n, int64_t parts) {
     TORCH_CHECK(!stays_with_torch(a, b), "mid_product: operands that stay with torch");
-    const c10::OptionalDeviceGuard device(a.device());
     const Product k = product_kind(kind);
-    const ProductSizes n = product_sizes(a, b, k);
-    const MidProduct mid = tile_m > 0 ? MidProduct{tile_m, tile_n, parts} : mid_product(k, n, a, b, large_product(k, n, a, b), own_product(k, n, a, b));
-    if (mid.tile_m == 0) return std::make_tuple(Tensor(), mid.tile_m, mid.tile_n);
-    return std::make_tuple(mid_product(a, b, k, n, mid), mid.tile_m, mid.tile_n);
-  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m") = 0, pybind11::arg("tile_n") = 0, pybind11::arg("parts") = 1);
+    return std::make_tuple(product(a, b, k, product_sizes(a, b, k), {ProductRoute::Mid, tile_m, tile_n, 0, parts, 0}), tile_m, tile_n);
+  }, pybind11::arg("a"), pybind11::arg("b"), pybind11::arg("kind"), pybind11::arg("tile_m"), pybind11::arg("tile_n"), pybind11::arg("parts") = 1);
   // (dx, dw, the tiles of each or 0); tiles given: in one launch of these
   m.def("gradients", [](const Tensor& dy, const Tensor& w, const Tensor& x, std::vector<int64_t> tiles) {
     TORCH_CHECK(tiles.empty() || (tiles.size() == 4 && !stays_with_torch(dy, w) && !stays_with_torch(dy, x)),

@@ -89,25 +89,24 @@ def test_the_predicate_is_what_the_kernel_refuses():
 
 
 def test_row_pitches_the_kernels_refuse_go_to_the_library():
-    """The sizes route to the package's kernels; the pitch (no multiple of 8, or rows too far apart) sends them past."""
+    """The sizes route to the package's kernels; the pitch (no multiple of 8, or rows too far apart) sends them past, to the library
+    or, where only the operand that stays as it is does not fit, to the library with the other one transposed."""
     run('''
-for kind, M, N, K, want in (("NT", 512, 576, 576, "own"), ("NN", 512, 1024, 1024, "own"), ("TN", 576, 960, 512, "own"),
-                            ("TN", 49152, 2048, 4096, "turned"), ("TN", 2048, 49152, 4096, "turned")):
+for kind, M, N, K, want in (("NT", 512, 576, 576, "own 64 in 2 groups"), ("NN", 512, 1024, 1024, "mid 32x64"), ("TN", 576, 960, 512, "own 64 in 2 groups"),
+                            ("TN", 49152, 2048, 4096, "large 256x256"), ("TN", 2048, 49152, 4096, "large 256x256")):
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     for pad_a, pad_b in ((0, 0), (8, 0), (0, 24), (4, 0), (0, 4), (1, 1), (4, 24), (0, 1 << 24), (1 << 24, 0)):
         got = host.product_route(operand(ra, ca, ca + pad_a), operand(rb, cb, cb + pad_b), kind)
-        if want == "own":
-            fits = pad_a % 8 == 0 and pad_b % 8 == 0 and max(pad_a, pad_b) < 1 << 24
-        else:                                     # only the operand that is transposed, the narrower one, has to fit
-            fits = (pad_a if M < N else pad_b) % 8 == 0
-        assert got == (want if fits else "library"), (kind, M, N, K, pad_a, pad_b, got)
+        fits = pad_a % 8 == 0 and pad_b % 8 == 0 and max(pad_a, pad_b) < 1 << 24
+        turns = max(M, N) == 49152 and (pad_a if M < N else pad_b) % 8 == 0
+        assert got == (want if fits else "turned" if turns else "library"), (kind, M, N, K, pad_a, pad_b, got)
     assert host.product_route(operand(ra, ca, address=(1 << 20) + 2), operand(rb, cb), kind) == "torch"
 ''')
 
 
 def test_long_contractions_are_cut_where_pieces_are_faster():
-    """Sizes at which a cut was up to 1.44 times as slow as the whole product, or as another number of pieces, us: whole, in the
-    number it was cut into, in the one expected now."""
+    """Operands whose pitch leaves them to the library.  Sizes at which a cut was up to 1.44 times as slow as the whole product, or as
+    another number of pieces, us: whole, in the number it was cut into, in the one expected now."""
     run('''
 for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 28.7 in 2
                             ("NT", 256, 4096, 10880, "library"),        # 1.23 times in 2
@@ -120,13 +119,14 @@ for kind, M, N, K, want in (("NT", 512, 2048, 8192, "library"),         # 27.0, 
                             ("NN", 4608, 768, 49152, "library in 8"),   # 432, 540 in 4, 346
                             ("NN", 512, 576, 49152, "library in 16"), ("NN", 2048, 4096, 21760, "library in 2"), ("NT", 640, 2048, 8192, "library in 2")):
     (ra, ca), (rb, cb) = (M, K), ((N, K) if kind == "NT" else (K, N))
-    got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
+    got = host.product_route(operand(ra, ca), operand(rb, cb, cb + 4), kind)
     assert got == want, (kind, M, N, K, got)
 ''')
 
 
 def test_weight_gradients_are_transposed_where_that_is_faster():
-    """Us whole and with the narrower operand transposed; in the wrong one of the two it lost up to 58 %."""
+    """Operands of which the wider one's pitch leaves them to the library.  Us whole and with the narrower operand transposed; in the
+    wrong one of the two it lost up to 58 %."""
     run('''
 for K, M, N, want in ((4096, 10880, 2048, "library"),      # 172, 273
                       (1152, 10880, 2048, "library"),      # 67, 80
@@ -140,7 +140,7 @@ for K, M, N, want in ((4096, 10880, 2048, "library"),      # 172, 273
                       (4096, 49152, 2048, "turned"),       # 732, 616
                       (4096, 2048, 16384, "turned"),       # 227, 202
                       (5504, 12288, 1536, "turned"), (4096, 49152, 576, "turned")):
-    got = host.product_route(operand(K, M), operand(K, N), "TN")
+    got = host.product_route(operand(K, M, M + 4 * (M > N)), operand(K, N, N + 4 * (N > M)), "TN")
     assert got == want, (K, M, N, got)
 ''')
 
@@ -165,31 +165,54 @@ def test_the_large_predicate_is_what_the_kernel_refuses():
     assert lib.pico_product_large(1 << 20, 1 << 20, 1 << 20, 512, 576, 576, 576, 576, 0, 0, 128, 128, 1, None) == -3
 
 
-def test_products_that_fill_the_gpu_go_to_their_kernel_where_it_is_faster():
-    """(rows and columns of a tile, pieces of the contraction), or none; us without and with the kernel."""
+def test_the_route_of_a_product():
+    """Each route where it is taken and, beside it, where it is not: us without and with it."""
     run('''
-none = (0, 0, 0)
-for kind, M, N, K, want in (("TN", 4096, 4096, 4096, (256, 256, 1)),       # 137, 103
-                            ("TN", 6144, 2048, 4096, (192, 256, 1)),       # 101, 91
-                            ("TN", 16384, 2048, 4096, (256, 256, 1)),      # 216, 199
-                            ("TN", 49152, 576, 512, (192, 256, 1)),        # 45, 40
-                            ("TN", 32000, 256, 512, none),                 # level
-                            ("TN", 49152, 128, 7358, none),                # 161, 179
-                            ("TN", 2048, 2048, 4096, none),                # 42, 51
-                            ("NN", 2242, 10880, 4096, (256, 256, 1)),      # 248, 178
-                            ("NN", 608, 576, 49152, (256, 192, 24)),       # 84, 55
-                            ("NN", 4548, 1024, 1024, none),                # 17, 20
-                            ("NN", 2886, 3072, 49152, none),               # 785, 846
-                            ("NT", 3832, 49152, 512, (256, 256, 1)),       # 315, 218
-                            ("NT", 5856, 6144, 768, (192, 256, 1)),        # 79, 52
-                            ("NT", 4096, 16384, 2048, none),               # 194, 203
-                            ("NT", 512, 49152, 576, (128, 256, 1)),        # 41, 34
-                            ("NT", 512, 576, 576, none)):
+for kind, M, N, K, want in (("TN", 4096, 4096, 4096, "large 256x256"),       # 137, 103
+                            ("TN", 6144, 2048, 4096, "large 192x256"),       # 101, 91
+                            ("TN", 16384, 2048, 4096, "large 256x256"),      # 216, 199
+                            ("TN", 49152, 576, 512, "large 192x256"),        # 45, 40
+                            ("TN", 32000, 256, 512, "mid 128x256"),          # (the large kernel is level with pico_product)
+                            ("TN", 49152, 128, 7358, "turned"),              # 161, large 179
+                            ("TN", 2048, 2048, 4096, "mid 128x128"),         # 42, large 51
+                            ("NN", 2242, 10880, 4096, "large 256x256"),      # 248, 178
+                            ("NN", 608, 576, 49152, "mid 128x192 in 17"),    # 84, large 55
+                            ("NN", 4548, 1024, 1024, "mid 128x192"),         # 17, large 20
+                            ("NN", 2886, 3072, 49152, "library in 4"),       # 785, large 846
+                            ("NT", 3832, 49152, 512, "large 256x256"),       # 315, 218
+                            ("NT", 5856, 6144, 768, "large 192x256"),        # 79, 52
+                            ("NT", 4096, 16384, 2048, "library"),            # 194, large 203
+                            ("NT", 512, 49152, 576, "large 128x256"),        # 41, 34
+                            ("NT", 512, 576, 576, "own 64 in 2 groups"),
+                            ("NN", 512, 576, 3072, "mid 32x64"),             # own 12.9, 8.7
+                            ("NN", 2331, 576, 3072, "mid 64x96"),            # 27.7, 15.8
+                            ("TN", 3072, 576, 2331, "mid 64x128"),
+                            ("NT", 2331, 576, 1536, "mid 64x96"),            # 12.0, 9.5
+                            ("NT", 128, 2048, 8192, "mid 64x128 in 8")):     # 14.9 in the library
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
-    got = host.large_product(operand(ra, ca), operand(rb, cb), kind)
+    got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
     assert got == want, (kind, M, N, K, got)
-    if want != none:                                  # pitches that the kernel refuses
-        assert host.large_product(operand(ra, ca, ca + 4), operand(rb, cb), kind) == none
-        assert host.large_product(operand(ra, ca), operand(rb, cb, cb + (1 << 24)), kind) == none
-        assert host.large_product(operand(ra, ca, ca + 8), operand(rb, cb, cb + 24), kind) == want
+    if not want.startswith(("library", "turned")):    # pitches that the kernels refuse, and pitches that they take
+        for a, b in ((operand(ra, ca, ca + 4), operand(rb, cb)), (operand(ra, ca), operand(rb, cb, cb + (1 << 24)))):
+            assert host.product_route(a, b, kind).startswith(("library", "turned"))
+        assert host.product_route(operand(ra, ca, ca + 8), operand(rb, cb, cb + 24), kind) == want
+''')
+
+
+def test_both_gradients_of_a_small_layer_go_together():
+    """(rows, columns out, columns in): the tiles of dx and dw in one launch, or apart; us apart and together."""
+    run('''
+for rows, out, inner, want in ((512, 576, 576, "32x64 64x64"),     # 8.8, 5.2
+                               (512, 3072, 576, "64x64 64x64"),    # 16.2, 13.1
+                               (2331, 960, 576, "64x96 64x64"),    # 17.9, 14.0
+                               (1024, 1024, 1024, "64x128 64x128"), # 15.1, 10.4
+                               (1309, 1688, 1688, "apart"),        # 30.8, 37.3
+                               (4096, 2048, 2048, "apart"), (512, 49152, 576, "apart"), (512, 580, 576, "apart")):
+    got = host.gradient_route(operand(rows, out), operand(out, inner), operand(rows, inner))
+    assert got == want, (rows, out, inner, got)
+    if want != "apart":
+        for a, b, c in ((operand(rows, out, out + 4), operand(out, inner), operand(rows, inner)),
+                        (operand(rows, out), operand(out, inner), operand(rows, inner, inner + 4)),
+                        (operand(rows, out), operand(out, inner), operand(rows, inner, device=1))):
+            assert host.gradient_route(a, b, c) == "apart"
 ''')
