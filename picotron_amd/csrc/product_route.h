@@ -1,6 +1,7 @@
 // Which kernel a projection's product goes to, in which tiles and pieces: rules on its kind, sizes and row pitches alone.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <string>
 #include <utility>
@@ -152,36 +153,51 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
   return K <= (tiles > 128 ? 3072 : tiles > 60 ? 1088 : 0) ? OwnProduct{2, 64} : no;
 }
 
+double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
+  return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
+}
+double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
+  struct Form {
+    int64_t tile, groups;
+    double start, trip, end, walk_idle, end_idle;
+  };
+  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84}, {64, 4, 2.52, 0.82, 5.90, 1.20, 0.00},
+                                   {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
+  for (const Form& f : forms) {
+    if (f.tile != own.tile || f.groups != own.groups) continue;
+    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
+    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
+    return f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
+  }
+  return 0;
+}
 // Whether a product goes to the package's kernel for products that fill the GPU (pico_product_large), in which tiles and in how
 // many pieces of the contraction (parts 0: no).
 //
 // The kernel's own time follows from its rounds: 256 workgroups take a tile each, a step of 64 of contraction costs 1.0 .. 1.4
-// us (less while part of the GPU idles), a tile's end 2 .. 5 us.  The estimate below has an error of 7 % (standard deviation)
-// over 20000 timed (shape, tile, pieces); the tile it takes is on average 0.7 % slower than the best one.  Against that stands
-// an estimate of the time without it, of the same form, whose error is 11 .. 34 %: the library's choices are not monotone in
-// any size.  So the lines ask for a margin where the library is good, and for none where it never is.  Of 2100 drawn products of
-// 100 .. 8192 rows those that go here took, in the geometric mean of the time without it,
-//   TN: 0.69 where the library ran them as they are (217 products, 0.99 at most; [4096 x 4096]^T [4096 x 4096] 137 -> 103
-//     us), 0.83 where it had an operand transposed first (91, 1.03 at most; [4096 x 16384]^T [4096 x 2048] 216 -> 199), 0.86 where
-//     pico_product did (13); under 640 of contraction that one stays ahead but for a vocabulary's width, see below, and the
-//     library where the vocabulary meets fewer than 256 columns ([7358 x 49152]^T [7358 x 128] 161 us, here 179);
-//   NN: 0.80 (143, 1.06 at most; [2242 x 10880] @ [10880 x 4096] 248 -> 178, [608 x 49152] @ [49152 x 576] 84 -> 55); a margin is
-//     asked for pieces of four and up, whose rows of a large pitch come more slowly than the estimate has it, and for short
-//     products ([4548 x 1024] @ [1024 x 1024] 17 us, here 20);
-//   NT: 0.77 (42, 1.02 at most): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
+// us (less while part of the GPU idles), a tile's end 2 .. 5 us; and from what it reads and writes, at 4.8 TB/s.  Over 39000 timed
+// (shape, tile, pieces) the estimate has an error of 7 % (standard deviation).  Against it stands what the product would take
+// otherwise: pico_product's time, estimated to 3 .. 8 %, or the library's, whose choices are not monotone in any size and cannot be estimated
+// to better than 11 .. 34 %.  So the lines ask for a margin where the library is good, and for none where it never is.  Layers drawn over 64 .. 8192
+// rows, 64 .. 4096 columns on one side, up to 22016 on the other, and vocabularies of 24576 .. 151936, other ones than those that the lines were
+// drawn from, took, over the time without this kernel, in the geometric mean (slower than 1.05, at most):
+//   TN: 0.71 of the library's time (1713 products; 7, 1.10; [4096 x 4096]^T [4096 x 4096] 137 -> 103 us), 0.83 of pico_product's (206; 2, 1.06; under
+//     640 of contraction that one stays ahead but for a vocabulary's width).  A vocabulary's weight gradient of up to 768 columns over
+//     4000 rows (576: 3000) stays in the library, with an operand transposed: 0.95 .. 1.03 of that, one in four over 1.05 ([6080 x 49152]^T
+//     [6080 x 576] 333 us, here 387);
+//   NN: 0.82 whole (269; 0, 1.03; [2242 x 10880] @ [10880 x 4096] 248 -> 178) and 0.69 in pieces (441; 8, 1.18), see cut_limit;
+//   NT: 0.74 (912; 1, 1.08): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
 //     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
-//     16384]^T 424 -> 206).
-// A vocabulary's side (24576 and up) is in every step, so its products were swept by themselves (600 of 128 .. 8192 rows, 192 .. 4096
-// columns, vocabularies of 32000 and 49152): they come here
-//   NT up to 768 of contraction, 0.81 of the library's time, none slower ([680 x 576] @ [32000 x 576]^T 57 -> 29 us, [512 x 576] @ [49152
-//     x 576]^T 41 -> 35; with 1024 0.96, and 1.10 at most);
-//   TN under 640 of contraction with 384 columns and up, 0.87 of pico_product's (1.09 at most; [464 x 32000]^T [464 x 1024] 43.6 ->
-//     34.1; with 192 and 256 columns level);
-//   NN where the library would cut the contraction, under 3072 columns, 0.83 (1.12 at most; [4548 x 49152] @ [49152 x 576] 418 ->
-//     258; with 4096 columns 1.00, and 1.21 at most).
+//     16384]^T 424 -> 206).  Logits of up to 768 columns always ([680 x 576] @ [32000 x 576]^T 57 -> 29 us), unless they are short (256)
+//     and their rows no whole lines ([6912 x 192] @ [73448 x 192]^T 419, here 508).
 struct LargeProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 0;
 };
+// `work` us of products beside a walk through the operands and the result at `rate` TB/s: the longer one, and more where both are long
+double with_memory(double work, int64_t M, int64_t N, int64_t K, double rate) {
+  const double memory = 2e-6 / rate * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N);
+  return std::sqrt(std::sqrt(work * work * work * work + memory * memory * memory * memory));
+}
 double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
   struct Form {
     int64_t m, n;
@@ -205,7 +221,7 @@ double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
       }
     }
   }
-  return least;
+  return with_memory(least, M, N, K, 4.8);
 }
 // the same without it: the library's tiles (NT, NN), or pico_product's (TN)
 double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
@@ -224,20 +240,49 @@ double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
   }
   return start[k] + least;
 }
+// The library's time for an input gradient that it would get in `parts` pieces (contraction_parts), at its best: whole tiles of a
+// contraction that divides evenly.
+double cut_time(int64_t M, int64_t N, int64_t K, int64_t parts) {
+  struct Form {
+    int64_t m, n;
+    double step;
+  };
+  static constexpr Form forms[] = {{256, 256, 1.44}, {256, 128, 0.71}, {128, 256, 0.71}, {128, 128, 0.35}};
+  double least = 1e30;
+  for (const Form& f : forms) {
+    const int64_t rounds = (((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n) * parts + 255) / 256;
+    least = std::min(least, rounds * (K / 64.0 / parts * f.step + 1.6));
+  }
+  return 2 + with_memory(least, M, N, K, 6.8) + 1.53e-6 * M * N * parts;
+}
+// What a kernel of the package's has to promise to get it.  Over 4000 timed products the library took, over cut_time, 0.98 .. 1.48 (a tenth and
+// nine tenths of them) with columns a multiple of 256 and a contraction of 1024, elsewhere 1.1 .. 2.0: there few kernels of its
+// do not fit.  A line of its own for vocabularies had [1536 x 49152] @ [49152 x 2048] at 262 -> 314 us, [3584 x 32768] @ [32768 x 512]
+// 120 -> 158; now 0.69 (large) and 0.54 (mid) of the library's time, as before, and 15 of 1604 over 1.05.
+double cut_limit(int64_t M, int64_t N, int64_t K, int64_t parts) {
+  return (N % 256 == 0 && K % 1024 == 0 ? 0.92 : 1.3) * cut_time(M, N, K, parts);
+}
 LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
   static_assert(static_cast<int>(Product::NT) == 0 && static_cast<int>(Product::NN) == 1 && static_cast<int>(Product::TN) == 2);
   const int64_t narrow = std::min(M, N), wide = std::max(M, N);
   LargeProduct best;
   if (M < 1 || N < 1 || K < 128 || narrow < 192 || (wide >= 24576 && narrow < 256)) return {};
   const double time = large_time(M, N, K, best), ideal = 2e-9 * M * N * K;   // (us at 1 PFLOP/s)
-  const bool small = own_product(kind, M, N, K).groups > 0;
+  const OwnProduct own = own_product(kind, M, N, K);
   bool take = false;
-  const bool vocabulary = std::max(wide, K) >= 24576;   // (see above)
-  if (vocabulary && (kind == Product::TN ? narrow >= 384 && K >= 200 && K < 640 : kind == Product::NT ? K <= 768 : K == std::max(wide, K) && N < 3072 && contraction_parts(kind, M, N, K) > 1)) take = true;
-  else if (kind == Product::TN) take = !small || (K >= 640 && time < 0.9 * other_time(kind, M, N, K));
-  else if (small || time < 14) take = false;
-  else if (kind == Product::NN) take = time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05);
-  else take = time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal);
+  const bool vocabulary = wide >= 24576;
+  if (own.groups > 0) {
+    take = kind == Product::TN && (vocabulary ? narrow >= 384 && K >= 200 : K >= 640) && time < 0.9 * own_time(own, M, N, K);
+  } else if (kind == Product::TN) {
+    take = !vocabulary || narrow > 768 || K < (narrow > 576 ? 4000 : 3000);
+  } else if (kind == Product::NT) {
+    if (vocabulary && K <= 768) take = N % 64 == 0 || K > 256;
+    else take = time >= 14 && (time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal));
+  } else if (const int64_t parts = contraction_parts(kind, M, N, K); parts > 1) {
+    take = time < cut_limit(M, N, K, parts);
+  } else {
+    take = time >= 14 && (time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05));
+  }
   return take ? best : LargeProduct{};
 }
 
@@ -258,28 +303,23 @@ LargeProduct large_product(Product kind, const ProductSizes& n) {
 // Whether a product goes to pico_product_mid and in which tiles (tile_m 0: no).
 //
 // Its time follows from its rounds: 256 workgroups take a tile each, a trip (64 of contraction for each group of waves) costs `trip`,
-// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy.  Over 25000 timed (shape, tiles) the
-// estimate has an error of 2 .. 6 % (standard deviation; tiles of 32 x 32 10 %), and the tiles it takes are 0.1 % slower than the best
-// ones in the mean.  Against it stands pico_product's own time, estimated alike (4 .. 7 %), or the library's (other_time).  Of 2290 drawn
-// products (64 .. 8192 rows, 72 .. 16384 columns and contraction) the 1430 that go here take, in the geometric mean of the time without it,
-//   NN 0.85 of pico_product's ([512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.69 of the library's ([2331 x 3072] @ [3072 x 576] 27.7 -> 15.8),
-//   TN 0.80 of pico_product's ([2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.82 of pico_product_large's,
-//   NT 0.78 of the library's ([2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5) and 0.93 of pico_product's; two over 1.12, 1.19 at most (the
-// library's choice of tiles is not monotone in any size).  The forward's layout leaves pico_product only for a clear gain: tiles of
-// 64 run level there.
-// Contractions that the library or pico_product_large would cut are cut here where that promises 0.95 (0.88) of pico_product_large's estimate: of 1020 drawn
-// input gradients (100 .. 4096 rows, 192 .. 3072 columns, contractions of 5504 .. 49152) 0.69 of the library's time in its pieces (ten of
-// 347 over 1.02, 1.22 at most) and 0.76 of pico_product_large's (246, 0.98 at most): [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [375 x 11008] @ [11008 x
-// 3072] 51 -> 38, [145 x 49152] @ [49152 x 576] 37 -> 23.  The other layouts alike (1000 drawn, contractions of 1500 .. 16384): 0.81 of the
-// library's pieces in the forward's (1.18 at most), 0.77 and 0.73 of pico_product_large's; and where a whole walk goes here, pieces that
-// promise 0.95 of it take 0.82 (1.23 at most; [208 x 5440] @ [256 x 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9).
+// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy; reading and writing go on beside, at 5.6 TB/s.
+// Over 27000 timed (shape, tiles) the estimate has an error of 7 .. 10 % (standard deviation), the larger one along a slow axis.  Against
+// it stands pico_product's or pico_product_large's own time, estimated alike, or the library's (other_time).  Of the drawn layers above those that
+// go here take, over the time without it, in the geometric mean (slower than 1.05, at most),
+//   NN 0.86 of pico_product's (3046 products; 5, 1.09; [512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.63 of the library's (1273; 0, 1.04; [2331 x
+//     3072] @ [3072 x 576] 27.7 -> 15.8),
+//   TN 0.74 of pico_product's (3419; 1, 1.09; [2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.56 of the library's (499; 0),
+//   NT 0.93 of pico_product's (373; 0, 1.03) and 0.70 of the library's (3359; 15, 1.20; [2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5).  The forward's layout
+//     leaves pico_product only for a clear gain: tiles of 64 run level there.
+// Contractions that the library or pico_product_large would cut are cut here where that promises more than cut_limit (NN) or 0.88 of
+// pico_product_large's estimate: 0.54 of the library's time in its pieces (NN, 1163; 7, 1.15; [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [145 x 49152] @
+// [49152 x 576] 37 -> 23) and 0.33 (TN, 386; 0).  And where a whole walk goes here, pieces that promise 0.9 of it ([208 x 5440] @ [256 x
+// 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9; with 0.95 two pieces of large outputs lost, [3584 x 3072]^T [3584 x 1024] 29.7 -> 35.8).
 struct MidProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 1;
 };
-double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
-  return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
-}
-double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
+double mid_time(Product kind, int64_t M, int64_t N, int64_t K, MidProduct& best) {
   struct Form {
     int64_t m, n, groups;
     double start, trip, end, walk_idle, end_idle;
@@ -294,7 +334,8 @@ double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
   double least = 1e30;
   for (const Form& f : forms) {
     const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
-    if (tiles > 1024 || (f.m == 32 && f.n == 32 && steps > 48)) continue;   // (long walks along a slow axis in rows of 64 bytes take twice that)
+    // (long walks along a slow axis in rows of 64 or 128 bytes take up to twice that)
+    if (tiles > 1024 || (f.m == 32 && ((f.n == 32 && steps > 48) || (kind != Product::NT && steps > 64)))) continue;
     const double walk = (steps + f.groups - 1) / f.groups * f.trip;
     const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
     if (t < least) {
@@ -302,19 +343,19 @@ double mid_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
       best = {f.m, f.n, 1};
     }
   }
-  return least;
+  return with_memory(least, M, N, K, 5.6);
 }
-// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces'
-// sum: 8 % error over 7600 timed (shape, tiles, pieces), 1.3 % over the best ones in the mean.
+// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces' sum: 10 % error over
+// 11000 timed (shape, tiles, pieces).
 double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
   struct Form {
     int64_t m, n, groups;
-    double start, trip, end, walk_idle, end_idle;
+    double start, trip, end, walk_idle, end_idle, share;   // (share: of a trip's time in mid_time)
   };
-  static constexpr Form forms[] = {{64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},
-                                   {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60},
-                                   {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45}, {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37},
-                                   {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
+  static constexpr Form forms[] = {{64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81, 0.86},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73, 0.90},
+                                   {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75, 0.88},   {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60, 0.93},
+                                   {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45, 0.95}, {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37, 0.93},
+                                   {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36, 0.95}};
   const int64_t steps = (K + 63) / 64;
   double least = 1e30;
   for (const Form& f : forms) {
@@ -322,49 +363,39 @@ double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
     for (const int64_t parts : {most, 2 * most / 3, most / 2}) {
       if (parts < 2 || parts > 64 || steps < 2 * parts) continue;
       const double walk = ((steps + parts - 1) / parts + f.groups - 1) / f.groups * f.trip;
-      const double t = f.start + last_round(0.93 * walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 4.8 + 1e-6 * M * N * (1.41 * parts - 2.43);
+      const double t = f.start + last_round(f.share * walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 4.8 + 1e-6 * M * N * (1.41 * parts - 0.9);
       if (t < least) {
         least = t;
         best = {f.m, f.n, parts};
       }
     }
   }
-  return least;
-}
-double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
-  struct Form {
-    int64_t tile, groups;
-    double start, trip, end, walk_idle, end_idle;
-  };
-  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84}, {64, 4, 2.52, 0.82, 5.90, 1.20, 0.00},
-                                   {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
-  for (const Form& f : forms) {
-    if (f.tile != own.tile || f.groups != own.groups) continue;
-    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
-    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
-    return f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
-  }
-  return 0;
+  return with_memory(least, M, N, K, 5.6);
 }
 MidProduct mid_product(Product kind, const ProductSizes& n, const LargeProduct& large, const OwnProduct& own) {
   const auto [M, N, K, lda, ldb] = n;
   if (M < 1 || N < 1 || K < 1 || !pico_product_mid_takes(M, N, K, lda, ldb, kind == Product::TN, kind != Product::NT)) return {};
-  MidProduct best;
+  // With few tiles the library deals out a contraction that divides evenly: [128 x 3328] @ [832 x 3328]^T 6.9 us, here 9.0; over 300 such
+  // products whole walks here took 1.06 .. 1.3 of its time, and 0.6 .. 0.9 with other contractions or more tiles.
+  const bool dealt = kind == Product::NT && K > 3072 && (K % 256 == 0 ? K <= 8192 : K % 128 == 0 && K <= 4352) && ((M + 31) / 32) * ((N + 63) / 64) <= 128;
+  MidProduct best, cut;
   LargeProduct same;
-  const double time = mid_time(M, N, K, best);
-  MidProduct cut;
-  const double pieces = mid_parts_time(M, N, K, cut);
-  const bool cut_elsewhere = large.parts > 0 || (own.groups == 0 && contraction_parts(kind, M, N, K) > 1);
-  if (cut_elsewhere && pieces < time && pieces < (kind == Product::NN && large.parts == 0 ? 0.95 : 0.88) * large_time(M, N, K, same)) return cut;
+  const double time = mid_time(kind, M, N, K, best), pieces = mid_parts_time(M, N, K, cut), least = std::min(time, pieces);
+  const int64_t library_parts = own.groups > 0 ? 1 : contraction_parts(kind, M, N, K);
+  if (kind == Product::NN && library_parts > 1) {
+    const bool take = large.parts > 0 ? least < large_time(M, N, K, same) : least < cut_limit(M, N, K, library_parts);
+    return !take ? MidProduct{} : pieces < time ? cut : best;
+  }
+  if ((large.parts > 0 || library_parts > 1) && pieces < time && pieces < 0.88 * large_time(M, N, K, same)) return cut;
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
-  else if (own.groups > 0) take = time < (kind == Product::NT ? 0.92 : 0.97) * own_time(own, M, N, K);
+  else if (own.groups > 0) take = time < (kind == Product::NT || best.tile_m * best.tile_n >= 6144 ? (kind == Product::TN ? 0.92 : 0.9) : 0.97) * own_time(own, M, N, K);
   else {   // (a margin that grows with the work: a wrong choice between two full GPUs costs more than it can gain)
     const double gflop = 2e-9 * M * N * K;
-    take = contraction_parts(kind, M, N, K) == 1 && time < (kind == Product::NN ? (gflop < 20 ? 1.0 : 0.9) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
+    take = library_parts == 1 && turned_operand(kind, n) == 0 && time < (kind == Product::NN ? (gflop < 20 ? 0.97 : 0.87) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
   }
   if (!take) return {};
-  return pieces < 0.95 * time ? cut : best;
+  return pieces < 0.9 * time ? cut : dealt ? MidProduct{} : best;
 }
 
 // The route of a product: the library whole or in `parts` pieces of the contraction, with operand `turn` (1: a, 2: b) transposed first;
@@ -434,7 +465,7 @@ GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
       }
     }
   MidProduct alone;
-  return least < 0.94 * (mid_time(rows, in, out, alone) + mid_time(out, in, rows, alone)) ? best : GradientTiles{};
+  return least < 0.94 * (mid_time(Product::NN, rows, in, out, alone) + mid_time(Product::TN, out, in, rows, alone)) ? best : GradientTiles{};
 }
 std::string route_name(const GradientTiles& t) {   // "32x64 64x96" (of dx, of dw) or "apart"
   auto tiles = [](const MidProduct& m) { return std::to_string(m.tile_m) + "x" + std::to_string(m.tile_n); };

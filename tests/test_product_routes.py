@@ -172,9 +172,9 @@ for kind, M, N, K, want in (("TN", 4096, 4096, 4096, "large 256x256"),       # 1
                             ("TN", 6144, 2048, 4096, "large 192x256"),       # 101, 91
                             ("TN", 16384, 2048, 4096, "large 256x256"),      # 216, 199
                             ("TN", 49152, 576, 512, "large 192x256"),        # 45, 40
-                            ("TN", 32000, 256, 512, "mid 128x256"),          # (the large kernel is level with pico_product)
+                            ("TN", 32000, 256, 512, "own 128 in 1 group"),   # (level in the large kernel)
                             ("TN", 49152, 128, 7358, "turned"),              # 161, large 179
-                            ("TN", 2048, 2048, 4096, "mid 128x128"),         # 42, large 51
+                            ("TN", 2048, 2048, 4096, "own 128 in 2 groups"), # 42, large 51
                             ("NN", 2242, 10880, 4096, "large 256x256"),      # 248, 178
                             ("NN", 608, 576, 49152, "mid 128x192 in 17"),    # 84, large 55
                             ("NN", 4548, 1024, 1024, "mid 128x192"),         # 17, large 20
@@ -188,7 +188,7 @@ for kind, M, N, K, want in (("TN", 4096, 4096, 4096, "large 256x256"),       # 1
                             ("NN", 2331, 576, 3072, "mid 64x96"),            # 27.7, 15.8
                             ("TN", 3072, 576, 2331, "mid 64x128"),
                             ("NT", 2331, 576, 1536, "mid 64x96"),            # 12.0, 9.5
-                            ("NT", 128, 2048, 8192, "mid 64x128 in 8")):     # 14.9 in the library
+                            ("NT", 128, 2048, 8192, "mid 64x96 in 5")):      # 14.9 in the library
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
     assert got == want, (kind, M, N, K, got)
@@ -215,4 +215,27 @@ for rows, out, inner, want in ((512, 576, 576, "32x64 64x64"),     # 8.8, 5.2
                         (operand(rows, out), operand(out, inner), operand(rows, inner, inner + 4)),
                         (operand(rows, out), operand(out, inner), operand(rows, inner, device=1))):
             assert host.gradient_route(a, b, c) == "apart"
+''')
+
+
+def test_products_stay_where_the_other_kernels_lose():
+    """Sizes of every kind that an own kernel, or another one, took and lost at: us where they go, us where they had gone."""
+    run('''
+for kind, M, N, K, want in (("NN", 1536, 2048, 49152, "library in 4"),       # 262, large 314
+                            ("NN", 3584, 512, 32768, "library in 8"),        # 120, large 158
+                            ("NN", 1974, 1536, 12288, "library in 4"),       # 82, mid in pieces 90
+                            ("NN", 3274, 920, 2384, "own 128 in 2 groups"),  # 25.3, mid 28.5
+                            ("NN", 64, 1784, 5376, "mid 64x96 in 6"),        # 11, mid 32x64 18
+                            ("TN", 49152, 576, 6080, "turned"),              # 333, large 387
+                            ("TN", 50304, 384, 243, "own 128 in 1 group"),   # 19.4, large 23.6
+                            ("TN", 3072, 1024, 3584, "own 128 in 2 groups"), # 31.9, mid in pieces 35.8
+                            ("TN", 2048, 2048, 5624, "own 128 in 2 groups"), # 56, mid 61
+                            ("TN", 9792, 3264, 451, "own 128 in 1 group"),   # 43.9, mid 50.4
+                            ("NT", 128, 832, 3328, "library"),               # 6.9, mid 9.0
+                            ("NT", 6912, 73448, 192, "library"),             # 419, large 508
+                            ("NT", 256, 2112, 2112, "own 64 in 2 groups"),   # 9.0, mid 9.8
+                            ("NT", 64, 2688, 8064, "mid 64x96 in 9")):       # 0.57 of the library's time
+    (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
+    assert got == want, (kind, M, N, K, got)
 ''')
