@@ -330,9 +330,9 @@ int pico_sum_parts(const float* src, void* dst, int64_t parts, int64_t n, int ds
 
 /* c = op(a) op(b) for bf16 operands, fp32 accumulation, one rounding; c [M, N] contiguous.  a_slow = 0: a is [M, K] with row
  * pitch lda; a_slow = 1: a is [K, M], op(a) = a^T.  b_slow = 0: b is [N, K], op(b) = b^T; b_slow = 1: b is [K, N].  For layers whose
- * output has few tiles.  `tile` (64 or 128): rows and columns of an output tile.  `groups` (1, 2, and 4 at tile 64): into how many groups of waves of a workgroup the contraction is dealt; their
- * fp32 sums are added in a fixed order.  N, the pitches and the contiguous axis of a and b must be multiples of 8, pointers
- * 16-byte aligned.  Counterpart of torch's F.linear and its gradients in the reference (model.py:105-108,183-184).
+ * output has few tiles.  `tile` (64 or 128): rows and columns of an output tile.  `groups` (1 or 2; 4 at tile 64 is taken as 2): into
+ * how many groups of waves of a workgroup the contraction is dealt; their fp32 sums are added in a fixed order.  N, the pitches and
+ * the contiguous axis of a and b must be multiples of 8, pointers 16-byte aligned.  Counterpart of torch's F.linear and its gradients in the reference (model.py:105-108,183-184).
  */
 /* 1 where pico_product takes operands of these sizes and row pitches, 0 where it refuses them. */
 int pico_product_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_slow, int b_slow);

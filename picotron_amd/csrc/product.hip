@@ -7,7 +7,8 @@
 // meet in LDS in the order of the groups (the same result on every run, no second launch).  A step costs 0.3 us in one group
 // and start plus end 3 us: [512 x 960]^T [512 x 576] takes 6.0 us (library 9.2).
 // With more tiles than CUs the reads of LDS are the bound, 3 KiB per MFMA of a tile of 64; tiles of 128 take 2 KiB, and two
-// workgroups fit a CU: [512 x 49152]^T [512 x 576] 48 us = 600 TFLOP/s (tiles of 64: 61, library 69).  The error against 64
+// workgroups fit a CU: [451 x 9792]^T [451 x 3264] 44 us = 655 TFLOP/s.  (A walk dealt to four groups was level with two or behind
+// where pico_product_mid leaves it here: [3950 x 15800]^T [3950 x 40] 22.7 us, in two 21.3.)  The error against 64
 // bits is the library's (1.66e-3, the rounding to bf16).
 #include "attn_common.h"
 
@@ -234,11 +235,7 @@ int launch(const ProductParams& p, hipStream_t s) {
 template <bool kSlowA, bool kSlowB>
 int launch_shape(const ProductParams& p, int tile, int groups, hipStream_t s) {
   if (tile == 128) return groups == 1 ? launch<kSlowA, kSlowB, 2, 1>(p, s) : launch<kSlowA, kSlowB, 2, 2>(p, s);
-  switch (groups) {
-    case 1: return launch<kSlowA, kSlowB, 1, 1>(p, s);
-    case 2: return launch<kSlowA, kSlowB, 1, 2>(p, s);
-    default: return launch<kSlowA, kSlowB, 1, 4>(p, s);
-  }
+  return groups == 1 ? launch<kSlowA, kSlowB, 1, 1>(p, s) : launch<kSlowA, kSlowB, 1, 2>(p, s);   // (4: as 2)
 }
 
 }  // namespace

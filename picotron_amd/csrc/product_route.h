@@ -121,7 +121,7 @@ int64_t turned_operand(Product kind, const ProductSizes& n) {
 //      [2331 x 1024]^T [2331 x 1024] 24, 15; [3072 x 576] from 1024 rows 14.2, 13.1, from 4096 35, 37;
 //   TN, up to 256 tiles of 128, two groups: [2048 x 2048] from 512 rows 13.6, 11.3, from 4096 49, 42; [3072 x 1024] from 2630
 //      41, 27; [1024 x 2688] from 4096 41, 40, from 8192 70, 76;
-//   TN, more tiles of 128: few rows.  [49152 x 576] from 512 69, 48, from 1024 93, 89.  The library runs an even number of
+//   TN, more tiles of 128: few rows.  [49152 x 576] from 512 69, 48 (pico_product_large 40), from 1024 93, 89.  The library runs an even number of
 //      its tiles side by side best and a ragged contraction a quarter slower: [32000 x 1024] from 512 46, 48, but [32000 x
 //      1152] 61, 50 and [8192 x 1024] from 443 20, 14;
 //   NN: [512 x 1024] @ [1024 x 1024] 9.2, 7.4; [512 x 3072] @ [3072 x 576] 17.0, 14.2; [512 x 2048] @ [2048 x 2048] 15, 12;
@@ -129,7 +129,7 @@ int64_t turned_operand(Product kind, const ProductSizes& n) {
 //   NT, its best: [512 x 1024] @ [1024 x 1024]^T 8.4, 6.8; [512 x 1536] @ [1536 x 576]^T 8.4, 8.8.
 // Over 2400 drawn products of 100 .. 8192 rows, 192 .. 49152 columns and contractions of 100 .. 49152 the time over the
 // library's was, where these lines choose the kernel, 0.75 (NN, 211 products), 0.81 (NT, 115) and 0.70 (TN, 316) in the geometric
-// mean and 1.04 at most.
+// mean and 1.04 at most.  Half of them go to pico_product_mid or pico_product_large, see their rules.
 struct OwnProduct {
   int64_t groups, tile;
 };
@@ -138,7 +138,7 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
   constexpr OwnProduct no = {0, 64};
   if (N % 8 || (kind == Product::TN ? M : K) % 8) return no;
   if (kind == Product::TN) {
-    if (tiles <= 256) return K <= 384 ? OwnProduct{1, 64} : K <= 3072 ? OwnProduct{2, 64} : K <= 4096 ? OwnProduct{4, 64} : no;
+    if (tiles <= 256) return K <= 384 ? OwnProduct{1, 64} : K <= 4096 ? OwnProduct{2, 64} : no;
     if (wide_tiles <= 128) return K <= 2560 ? OwnProduct{1, 64} : no;
     if (wide_tiles <= 256) return K <= 384 ? OwnProduct{1, 128} : K <= (wide_tiles >= 230 ? 8192 : 4096) ? OwnProduct{2, 128} : no;
     const int64_t most = narrow % 512 ? (K % 64 ? 1000 : 768) : (K % 64 ? 576 : 320);
@@ -161,7 +161,7 @@ double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
     int64_t tile, groups;
     double start, trip, end, walk_idle, end_idle;
   };
-  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84}, {64, 4, 2.52, 0.82, 5.90, 1.20, 0.00},
+  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84},
                                    {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
   for (const Form& f : forms) {
     if (f.tile != own.tile || f.groups != own.groups) continue;
