@@ -5,7 +5,7 @@
 // 40 us of GPU time, and with torch.autograd.Function classes and ctypes in Python a pass took 180 us, whatever the
 // kernels did.  Here a call is one C++ function: no ctypes conversions, no Python frames in the backward (the autograd
 // thread never takes the GIL), views replaced by pointer + strides.  Nothing is kept from one call
-// for the next but the GEMM library's plans, by shape.
+// for the next but the GEMM library's plans, by shape, and which kernel a product of given sizes goes to.
 #include <torch/extension.h>
 #include <ATen/Context.h>
 #include <ATen/autocast_mode.h>

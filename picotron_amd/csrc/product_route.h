@@ -404,7 +404,7 @@ struct ProductRoute {
   enum Kernel { Library, Own, Mid, Large } kernel = Library;
   int64_t tile_m = 0, tile_n = 0, groups = 0, parts = 1, turn = 0;
 };
-ProductRoute product_route(Product kind, const ProductSizes& n) {
+ProductRoute choose_route(Product kind, const ProductSizes& n) {
   const LargeProduct large = large_product(kind, n);
   const OwnProduct own = own_product(kind, n);
   const MidProduct mid = mid_product(kind, n, large, own);
@@ -412,6 +412,33 @@ ProductRoute product_route(Product kind, const ProductSizes& n) {
   if (large.parts > 0) return {ProductRoute::Large, large.tile_m, large.tile_n, 0, large.parts, 0};
   if (own.groups > 0) return {ProductRoute::Own, own.tile, own.tile, own.groups, 1, 0};
   return {ProductRoute::Library, 0, 0, 0, contraction_parts(kind, n.M, n.N, n.K), turned_operand(kind, n)};
+}
+
+// The rules go through some thirty tiles each, 0.4 .. 1.3 us a call on the side that paces a small model's step (13 us of a two-layer
+// 135M step), so what they say is kept by the numbers they were asked with: per thread, and dropped for whatever comes to the same place.
+template <typename Answer>
+struct RouteTable {
+  struct Entry {
+    int64_t key[6] = {};
+    bool used = false;
+    Answer answer;
+  } entries[256];
+  template <typename Make>
+  const Answer& get(const int64_t (&key)[6], const Make& make) {
+    uint64_t h = 1469598103934665603ull;
+    for (const int64_t v : key) h = (h ^ static_cast<uint64_t>(v)) * 1099511628211ull;
+    Entry& e = entries[(h ^ (h >> 29)) % 256];
+    if (!e.used || !std::equal(key, key + 6, e.key)) {
+      e.answer = make();
+      std::copy(key, key + 6, e.key);
+      e.used = true;
+    }
+    return e.answer;
+  }
+};
+ProductRoute product_route(Product kind, const ProductSizes& n) {
+  static thread_local RouteTable<ProductRoute> table;
+  return table.get({static_cast<int64_t>(kind), n.M, n.N, n.K, n.lda, n.ldb}, [&] { return choose_route(kind, n); });
 }
 // for tests: "mid 64x96", "large 256x192 in 24", "own 64 in 2 groups", "library", "library in 4", "turned" (the library with an
 // operand transposed first)
@@ -443,7 +470,7 @@ double workgroups_end(int64_t n1, double t1, int64_t n2, double t2) {
     }
   return end;
 }
-GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
+GradientTiles choose_gradient_tiles(int64_t rows, int64_t out, int64_t in) {
   struct Form {
     int64_t m, n, groups;
     double trip, end;
@@ -466,6 +493,10 @@ GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
     }
   MidProduct alone;
   return least < 0.94 * (mid_time(Product::NN, rows, in, out, alone) + mid_time(Product::TN, out, in, rows, alone)) ? best : GradientTiles{};
+}
+GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
+  static thread_local RouteTable<GradientTiles> table;
+  return table.get({rows, out, in, 0, 0, 0}, [&] { return choose_gradient_tiles(rows, out, in); });
 }
 std::string route_name(const GradientTiles& t) {   // "32x64 64x96" (of dx, of dw) or "apart"
   auto tiles = [](const MidProduct& m) { return std::to_string(m.tile_m) + "x" + std::to_string(m.tile_n); };

@@ -239,3 +239,30 @@ for kind, M, N, K, want in (("NN", 1536, 2048, 49152, "library in 4"),       # 2
     got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
     assert got == want, (kind, M, N, K, got)
 ''')
+
+
+def test_routes_that_are_kept_are_those_of_their_sizes():
+    """More sizes than a thread keeps, with pitches that send some past the kernels, in one order and in the other, from two threads."""
+    run('''
+import threading
+asked = [(kind, 64 + 40 * i, 64 + 8 * (i * 37 % 300), 64 + 8 * (i * 53 % 500), 4 * (i % 3)) for i in range(400) for kind in ("NT", "NN", "TN")]
+
+
+def route(kind, M, N, K, pad):
+    (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    return host.product_route(operand(ra, ca, ca + pad), operand(rb, cb), kind), host.gradient_route(operand(M, K), operand(K, N), operand(M, N))
+
+
+def ask(into, order):
+    for q in order:
+        into.append((q, route(*q), route(*q)))
+
+
+answers = [[], []]
+threads = [threading.Thread(target=ask, args=a) for a in zip(answers, (asked, asked[::-1]))]
+for t in threads: t.start()
+for t in threads: t.join()
+first, second = ({q: r for q, r, again in a if r == again} for a in answers)
+assert len(first) == len(set(asked)) and first == second
+assert len(set(first.values())) > 20
+''')
