@@ -1203,7 +1203,7 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
     switch (plan.kernel) {
       case DqPlan::kWaves8: use(DqCfg<64, 8, 64>(), 1.7, 1.5, 1.0); break;
-      case DqPlan::kWaves4: use(DqCfg<64, 4, 64>(), 0.79, 0.5, 1.02); break;
+      case DqPlan::kWaves4: use(DqCfg<64, 4, 64>(), 0.89, 0.44, 1.18); break;
       case DqPlan::kSplit8: use(DqCfg<64, 8, 128, 2>(), 1.6, 1.5, 1.0); break;
       case DqPlan::kSplit4: use(DqCfg<64, 4, 128, 2>(), 1.25, 0.8, 1.0); break;
     }

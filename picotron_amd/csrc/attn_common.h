@@ -452,11 +452,11 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
 // Host: the piece length for a launch, from what its workgroups cost.  A trip takes `alone_us` in a workgroup that has its
 // CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each, `cut` times that in the kernel that can cut
 // (see kCut of the forward); `per_cu` is the number the kernel's registers and LDS are budgeted for.
-// (Fitted to every piece length of 1098 forward, dQ and dK/dV launches each, 1 to 256 heads and 200 to 8192 rows.  The
-// lengths chosen ran within 0.1 to 1.6 % of the best ones in the geometric mean -- dQ with split keys 3 %, dK/dV at head_dim
-// 64 6 % -- and at worst 3.2 % slower than the whole launch.  The four-wave kernels of head_dim 128 were once planned as two
-// per CU where their registers let one run, and the cutting kernel's own loss was not counted: at one sequence of 3000 rows
-// and 20 heads the forward, whole 100 us, was cut to 95 and is 68 whole now that two fit; dQ, whole 94, was cut to 109.)
+// (Fitted to every piece length of some thousand launches, 1 to 256 heads and 200 to 8192 rows, and held against 5752 others with today's
+// kernels: of 16714 launches 22 run over 1.03 of the whole launch's time, 1.07 at worst, where they would be level.  The lengths chosen
+// run within 0.5 to 1.8 % of the best ones in the geometric mean, dK/dV at head_dim 64 4 %: constants that come nearer there make every
+// twentieth launch 3 to 12 % slower than these do.  The four-wave dQ at head_dim 64 is never faster cut, which its own loss, 1.18, says: with
+// 1.02 it was cut eight times in 218, B2 H8 S4096 64.1 whole, 71.1.)
 struct TripCost {
   double alone_us, full_us, cut;
   int per_cu;
@@ -524,7 +524,7 @@ double launch_us(int64_t heads, int n_tiles, const TripCost& c, int len, bool pa
 template <typename F>
 int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, bool pairs, const F& trips_of) {
   if (heads * n_tiles > 4 * 512) return 0;   // enough workgroups that their lengths even out
-  // a cut has to win 5 % by the estimate (with that, none of the launches above lost more than 3.2 %) and the time in which a
+  // a cut has to win 5 % by the estimate (so that few of the launches above lose) and the time in which a
   // host launches the second kernel: where the host is the slower side a shorter kernel gains nothing (B2 H9/3 S256 D64, forward and backward: 33 us
   // of kernels cut to 29 took 38 us for 35)
   constexpr double kLaunchUs = 5.0;

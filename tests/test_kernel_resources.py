@@ -83,6 +83,21 @@ def test_launches_that_fill_the_gpu_run_whole(B, Hq, Hkv, S, D):
     assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == 0
 
 
+@pytest.mark.parametrize("Hq,S,dkdv_pieces", [(16, 4096, 272), (12, 5888, 288)])
+def test_dq_of_four_waves_at_head_dim_64_runs_whole(Hq, S, dkdv_pieces):
+    """It is never faster in pieces (B2 H8 S4096 64.1 us, cut 71.1).  With one key head the scratch memory that dQ's pieces would ask for is
+    larger than that of dK/dV's (four key waves, 2 x 32 x 64 floats each), which is what the call asks for."""
+    import ctypes
+
+    import torch
+    from picotron_amd import _lib, ops
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    q, k = (torch.empty(1, h, S, 64, dtype=torch.bfloat16) for h in (Hq, 1))
+    d = ops._desc(q, k, k, q, 0.125, True, 0)
+    assert _lib.lib().pico_attn_bwd_workspace_bytes(ctypes.byref(d), 1) == dkdv_pieces * 4 * 2 * 32 * 64 * 4
+
+
 def test_kernels_that_make_requests_have_no_scratch_and_no_lds_of_their_own(tmp_path):
     """A spill counts among the memory operations of which product_mid and product_large wait for all but the newest few, and the
     requests' places in LDS are counted from 0: the build refuses both.  A workgroup of the products has a CU to itself, two
