@@ -258,9 +258,10 @@ double cut_time(int64_t M, int64_t N, int64_t K, int64_t parts) {
 // What a kernel of the package's has to promise to get it.  Over 4000 timed products the library took, over cut_time, 0.98 .. 1.48 (a tenth and
 // nine tenths of them) with columns a multiple of 256 and a contraction of 1024, elsewhere 1.1 .. 2.0: there few kernels of its
 // do not fit.  A line of its own for vocabularies had [1536 x 49152] @ [49152 x 2048] at 262 -> 314 us, [3584 x 32768] @ [32768 x 512]
-// 120 -> 158; now 0.69 (large) and 0.54 (mid) of the library's time, as before, and 15 of 1604 over 1.05.
+// 120 -> 158; now 0.69 (large) and 0.54 (mid) of the library's time, as before, and 15 of 1604 over 1.05.  (Two pieces
+// need no margin: 20 of those products, none over 1.05; [4096 x 16384] @ [16384 x 2048] with operands from memory 225 us, here 218.)
 double cut_limit(int64_t M, int64_t N, int64_t K, int64_t parts) {
-  return (N % 256 == 0 && K % 1024 == 0 ? 0.92 : 1.3) * cut_time(M, N, K, parts);
+  return (N % 256 != 0 || K % 1024 != 0 ? 1.3 : parts == 2 ? 1.0 : 0.92) * cut_time(M, N, K, parts);
 }
 LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
   static_assert(static_cast<int>(Product::NT) == 0 && static_cast<int>(Product::NN) == 1 && static_cast<int>(Product::TN) == 2);
@@ -389,7 +390,10 @@ MidProduct mid_product(Product kind, const ProductSizes& n, const LargeProduct& 
   if ((large.parts > 0 || library_parts > 1) && pieces < time && pieces < 0.88 * large_time(M, N, K, same)) return cut;
   bool take;
   if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
-  else if (own.groups > 0) take = time < (kind == Product::NT || best.tile_m * best.tile_n >= 6144 ? (kind == Product::TN ? 0.92 : 0.9) : 0.97) * own_time(own, M, N, K);
+  else if (own.groups > 0) {   // (margins that the estimates' errors need: along one slow axis and in tiles of 128 x 256 they are larger)
+    const int64_t area = best.tile_m * best.tile_n;
+    take = time < (kind == Product::NT ? 0.9 : area < 6144 ? 0.97 : kind == Product::NN ? 0.9 : area < 32768 ? 0.94 : 0.92) * own_time(own, M, N, K);
+  }
   else {   // (a margin that grows with the work: a wrong choice between two full GPUs costs more than it can gain)
     const double gflop = 2e-9 * M * N * K;
     take = library_parts == 1 && turned_operand(kind, n) == 0 && time < (kind == Product::NN ? (gflop < 20 ? 0.97 : 0.87) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);

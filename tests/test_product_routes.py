@@ -174,7 +174,7 @@ for kind, M, N, K, want in (("TN", 4096, 4096, 4096, "large 256x256"),       # 1
                             ("TN", 49152, 576, 512, "large 192x256"),        # 45, 40
                             ("TN", 32000, 256, 512, "own 128 in 1 group"),   # (level in the large kernel)
                             ("TN", 49152, 128, 7358, "turned"),              # 161, large 179
-                            ("TN", 2048, 2048, 4096, "own 128 in 2 groups"), # 42, large 51
+                            ("TN", 2048, 2048, 4096, "mid 128x128"),         # 42, 39, large 51
                             ("NN", 2242, 10880, 4096, "large 256x256"),      # 248, 178
                             ("NN", 608, 576, 49152, "mid 128x192 in 17"),    # 84, large 55
                             ("NN", 4548, 1024, 1024, "mid 128x192"),         # 17, large 20
