@@ -181,12 +181,12 @@ double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
 // to better than 11 .. 34 %.  So the lines ask for a margin where the library is good, and for none where it never is.  Layers drawn over 64 .. 8192
 // rows, 64 .. 4096 columns on one side, up to 22016 on the other, and vocabularies of 24576 .. 151936, other ones than those that the lines were
 // drawn from, took, over the time without this kernel, in the geometric mean (slower than 1.05, at most):
-//   TN: 0.71 of the library's time (1713 products; 7, 1.10; [4096 x 4096]^T [4096 x 4096] 137 -> 103 us), 0.83 of pico_product's (206; 2, 1.06; under
+//   TN: 0.71 of the library's time (1768 products; 1, 1.07; [4096 x 4096]^T [4096 x 4096] 137 -> 103 us), 0.84 of pico_product's (216; 0, 1.01; under
 //     640 of contraction that one stays ahead but for a vocabulary's width).  A vocabulary's weight gradient of up to 768 columns over
 //     4000 rows (576: 3000) stays in the library, with an operand transposed: 0.95 .. 1.03 of that, one in four over 1.05 ([6080 x 49152]^T
 //     [6080 x 576] 333 us, here 387);
-//   NN: 0.82 whole (269; 0, 1.03; [2242 x 10880] @ [10880 x 4096] 248 -> 178) and 0.69 in pieces (441; 8, 1.18), see cut_limit;
-//   NT: 0.74 (912; 1, 1.08): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
+//   NN: 0.82 whole (399; 0, 1.01; [2242 x 10880] @ [10880 x 4096] 248 -> 178) and 0.71 in pieces (421; 2, 1.08), see cut_limit;
+//   NT: 0.74 (912; 1, 1.07): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
 //     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
 //     16384]^T 424 -> 206).  Logits of up to 768 columns always ([680 x 576] @ [32000 x 576]^T 57 -> 29 us), unless they are short (256)
 //     and their rows no whole lines ([6912 x 192] @ [73448 x 192]^T 419, here 508).
@@ -258,7 +258,7 @@ double cut_time(int64_t M, int64_t N, int64_t K, int64_t parts) {
 // What a kernel of the package's has to promise to get it.  Over 4000 timed products the library took, over cut_time, 0.98 .. 1.48 (a tenth and
 // nine tenths of them) with columns a multiple of 256 and a contraction of 1024, elsewhere 1.1 .. 2.0: there few kernels of its
 // do not fit.  A line of its own for vocabularies had [1536 x 49152] @ [49152 x 2048] at 262 -> 314 us, [3584 x 32768] @ [32768 x 512]
-// 120 -> 158; now 0.69 (large) and 0.54 (mid) of the library's time, as before, and 15 of 1604 over 1.05.  (Two pieces
+// 120 -> 158; now 0.71 (large) and 0.55 (mid) of the library's time, as before, and 10 of 1460 over 1.05.  (Two pieces
 // need no margin: 20 of those products, none over 1.05; [4096 x 16384] @ [16384 x 2048] with operands from memory 225 us, here 218.)
 double cut_limit(int64_t M, int64_t N, int64_t K, int64_t parts) {
   return (N % 256 != 0 || K % 1024 != 0 ? 1.3 : parts == 2 ? 1.0 : 0.92) * cut_time(M, N, K, parts);
@@ -308,14 +308,14 @@ LargeProduct large_product(Product kind, const ProductSizes& n) {
 // Over 27000 timed (shape, tiles) the estimate has an error of 7 .. 10 % (standard deviation), the larger one along a slow axis.  Against
 // it stands pico_product's or pico_product_large's own time, estimated alike, or the library's (other_time).  Of the drawn layers above those that
 // go here take, over the time without it, in the geometric mean (slower than 1.05, at most),
-//   NN 0.86 of pico_product's (3046 products; 5, 1.09; [512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.63 of the library's (1273; 0, 1.04; [2331 x
+//   NN 0.87 of pico_product's (2978 products; 1, 1.05; [512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.66 of the library's (1221; 4, 1.06; [2331 x
 //     3072] @ [3072 x 576] 27.7 -> 15.8),
-//   TN 0.74 of pico_product's (3419; 1, 1.09; [2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.56 of the library's (499; 0),
-//   NT 0.93 of pico_product's (373; 0, 1.03) and 0.70 of the library's (3359; 15, 1.20; [2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5).  The forward's layout
+//   TN 0.75 of pico_product's (3570; 0, 1.05; [2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.57 of the library's (503; 0),
+//   NT 0.94 of pico_product's (362; 0, 1.03) and 0.69 of the library's (3554; 10, 1.18; [2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5).  The forward's layout
 //     leaves pico_product only for a clear gain: tiles of 64 run level there.
 // Contractions that the library or pico_product_large would cut are cut here where that promises more than cut_limit (NN) or 0.88 of
-// pico_product_large's estimate: 0.54 of the library's time in its pieces (NN, 1163; 7, 1.15; [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [145 x 49152] @
-// [49152 x 576] 37 -> 23) and 0.33 (TN, 386; 0).  And where a whole walk goes here, pieces that promise 0.9 of it ([208 x 5440] @ [256 x
+// pico_product_large's estimate: 0.54 of the library's time in its pieces (NN, 1039; 8, 1.28; [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [145 x 49152] @
+// [49152 x 576] 37 -> 23) and 0.31 (TN, 424; 0).  And where a whole walk goes here, pieces that promise 0.9 of it ([208 x 5440] @ [256 x
 // 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9; with 0.95 two pieces of large outputs lost, [3584 x 3072]^T [3584 x 1024] 29.7 -> 35.8).
 struct MidProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 1;
