@@ -223,7 +223,7 @@ double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
   }
   return with_memory(least, M, N, K, 4.8);
 }
-// the same without it: the library's tiles (NT, NN), or pico_product's (TN)
+// the same in the library (TN: 1.5 times this at the median, hardly ever less)
 double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
   struct Form {
     int64_t m, n;

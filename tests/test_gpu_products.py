@@ -218,3 +218,23 @@ def test_products_in_pieces_of_one_round(device, kind, M, N, K):
     for bad in ((64, 64, 2), (64, 96, 65), (64, 96, steps + 1)):
         with pytest.raises(RuntimeError):
             host.mid_product(a, b, kind, *bad)
+
+
+@pytest.mark.parametrize("kind,M,N,K", [
+    ("NN", 64, 1784, 5376), ("NN", 577, 192, 24576), ("NN", 300, 512, 32768), ("NN", 1320, 2240, 3360), ("NN", 3274, 920, 2384), ("NN", 2048, 2048, 16384),
+    ("NT", 128, 832, 3328), ("NT", 64, 2688, 8064), ("NT", 129, 640, 4096), ("NT", 700, 24584, 192), ("NT", 700, 24584, 320), ("NT", 256, 2112, 2112),
+    ("TN", 24576, 384, 243), ("TN", 24584, 576, 3001), ("TN", 3072, 1024, 3584), ("TN", 2048, 2048, 1111), ("TN", 48, 9000, 3950)])
+def test_products_by_the_rule(device, kind, M, N, K):
+    """On both sides of the lines between the kernels, as dense operands and as columns of wider ones whose pitch the package's kernels
+    take or refuse, against a fp32 product (rounded once: 2^-9); the package's kernels give the same on every call."""
+    from picotron_amd import _lib
+    host = _lib.host()
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    sizes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
+    for pad in (0, 16, 4):
+        a, b = (torch.randn(r, c + pad, generator=g, device=device).to(torch.bfloat16)[:, :c] for r, c in sizes)
+        want = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float())
+        got, route = host.product(a, b, kind), host.product_route(a, b, kind)
+        assert got.shape == (M, N) and ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (pad, route)
+        if not route.startswith(("library", "turned")):
+            assert pad != 4 and torch.equal(got, host.product(a, b, kind)), (pad, route)
