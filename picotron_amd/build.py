@@ -105,7 +105,8 @@ def build(verbose: bool = True, extra_flags=()) -> str:
         out = _run([hipcc, *FLAGS, *extra_flags, *([RESOURCES] if requesting else []), "-c", os.path.join(CSRC, src), "-o", obj])
         if requesting:
             check_requesting(src, out)
-        elif verbose and out.strip():
+            out = "\n".join(l for l in out.splitlines() if "warning:" in l)   # (of the rest all but warnings are the remarks just read)
+        if verbose and out.strip():
             print(out)
         return obj
 
