@@ -636,12 +636,13 @@ int dispatch_bwd(const void* dy, const void* x, const void* w, const float* rstd
   return fail(PICO_ERR_SHAPE, "pico_rmsnorm_bwd: hidden=%d too large", hidden);
 }
 
-// rmsnorm_bwd_few_kernel, where it is taken: 1, nothing launched otherwise.
+// Launches rmsnorm_bwd_few_kernel where it is taken; false: nothing is launched.  An output that takes an input's place needs the two launches: here
+// workgroups of the other gradient may still read what is written (dresidual is read by the lanes that write dx, so it may be dx).
 template <typename T, typename TW>
 bool launch_bwd_few(const void* dy, const void* x, const void* w, const float* rstd, const void* dres, void* dx, void* dweight, int64_t rows,
                     int hidden, hipStream_t s) {
   const int nv = pick_nv((hidden / io<T>::kVec + 63) / 64, 8);
-  if (!nv || rows > kFewRows || dx == dy || dx == x) return false;
+  if (!nv || rows > kFewRows || dx == dy || dx == x || dweight == w) return false;
   const int dw_blocks = (hidden + kFewCols - 1) / kFewCols, row_blocks = static_cast<int>((rows + kFewThreads / kWave - 1) / (kFewThreads / kWave));
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(dw_blocks + row_blocks), dim3(kFewThreads), 0, s, static_cast<const T*>(dy), static_cast<const T*>(x),

@@ -117,6 +117,37 @@ def test_rmsnorm_bwd_of_few_rows(ops, device, rows, hidden, dtype):
     assert rel_l2(got[0][1], want_dw) <= 1e-5
 
 
+@pytest.mark.parametrize("rows", [1, 64, 1024, 1100])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rmsnorm_bwd_in_the_place_of_an_input(ops, device, rows, dtype):
+    """Through the C ABI: dx written over dy or dresidual, and dweight over weight, on both sides of the 1024 rows up to which the two
+    gradients share a launch.  Where that launch is left for two, dweight is added in another order: 1e-5 of it in fp32, one rounding in bf16."""
+    from picotron_amd import _lib
+    hidden, code = 576, 0 if dtype == torch.bfloat16 else 1
+    dy, x, dr = (rnd(rows, hidden, seed=s_, dtype=dtype).to(device) for s_ in (31, 32, 33))
+    w = (1 + 0.1 * rnd(hidden, seed=34)).to(dtype).to(device)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1) + 1e-5)
+    lib = _lib.lib()
+    ws = torch.empty(lib.pico_rmsnorm_bwd_workspace_bytes(rows, hidden), dtype=torch.uint8, device=device)
+
+    def backward(place):
+        t = {"dy": dy.clone(), "x": x.clone(), "dr": dr.clone(), "w": w.clone()}
+        dx = t.get(place) if place != "w" else None
+        dx, dw = dx if dx is not None else torch.empty_like(x), t["w"] if place == "w" else torch.empty_like(w)
+        rc = lib.pico_rmsnorm_bwd(t["dy"].data_ptr(), t["x"].data_ptr(), t["w"].data_ptr(), rstd.data_ptr(), t["dr"].data_ptr(), dx.data_ptr(),
+                                  dw.data_ptr(), code, ws.data_ptr(), ws.numel(), rows, hidden, code, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.lib().pico_last_error()
+        return dx, dw
+
+    dx0, dw0 = backward(None)
+    for place in ("dy", "dr", "w"):
+        dx, dw = backward(place)
+        assert rel_l2(dx, dx0.float()) <= (1e-6 if dtype == torch.float32 else 2.0 ** -8), place
+        assert rel_l2(dw, dw0.float()) <= (1e-5 if dtype == torch.float32 else 2.0 ** -8), place
+    dx, dw = backward("dr")
+    assert torch.equal(dx, dx0) and torch.equal(dw, dw0)
+
+
 def test_rmsnorm_bwd_is_bit_reproducible_at_every_row_length_class(ops, device):
     """dweight is summed without atomics: two runs give the same bits, for the row-per-wave kernels, for the rows a
     256-thread group owns (two groups per block meet in LDS, in group order) and for the longest rows."""
