@@ -150,17 +150,22 @@ def test_rmsnorm_bwd_in_the_place_of_an_input(ops, device, rows, dtype):
 
 def test_rmsnorm_bwd_is_bit_reproducible_at_every_row_length_class(ops, device):
     """dweight is summed without atomics: two runs give the same bits, for the row-per-wave kernels, for the rows a
-    256-thread group owns (two groups per block meet in LDS, in group order) and for the longest rows."""
+    256-thread group owns (two groups per block meet in LDS, in group order) and for the longest rows.  Up to 1024 rows of up to
+    4096 (fp32: 2048) the two gradients share a launch, so the row-per-wave kernels are the sizes above; with the residual's gradient
+    a wave keeps two rows in flight where it owns several (4096 x 2048)."""
     for rows, hidden, dtype in ((1000, 2048, torch.bfloat16), (1000, 4096, torch.bfloat16), (700, 8192, torch.bfloat16),
-                                (300, 16384, torch.bfloat16), (500, 8192, torch.float32), (900, 1000, torch.float32)):
+                                (300, 16384, torch.bfloat16), (500, 8192, torch.float32), (900, 1000, torch.float32),
+                                (1100, 512, torch.bfloat16), (1100, 2048, torch.bfloat16), (1100, 4096, torch.bfloat16), (4096, 2048, torch.bfloat16),
+                                (1100, 1000, torch.float32), (4096, 1024, torch.float32)):
         x = rnd(rows, hidden, seed=70, dtype=dtype).to(device)
         dy = rnd(rows, hidden, seed=71, dtype=dtype).to(device)
         w = (1 + 0.1 * rnd(hidden, seed=72)).to(dtype).to(device)
         _, rstd, _ = ops.rmsnorm_fwd(x, w, 1e-5, False)
-        a = ops.rmsnorm_bwd(dy, x, w, rstd)
-        for _ in range(3):
-            b = ops.rmsnorm_bwd(dy, x, w, rstd)
-            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]), (rows, hidden, dtype)
+        for dr in (None, dy.flip(0)):
+            a = ops.rmsnorm_bwd(dy, x, w, rstd, dresidual=dr)
+            for _ in range(3):
+                b = ops.rmsnorm_bwd(dy, x, w, rstd, dresidual=dr)
+                assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]), (rows, hidden, dtype)
 
 
 # ------------------------------------------------------------------------------------ RoPE
