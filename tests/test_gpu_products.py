@@ -114,8 +114,8 @@ def test_small_products(device, kind, M, N, K):
 @pytest.mark.parametrize("pad", [1, 4, 8])
 @pytest.mark.parametrize("rows,cin,cout", [(512, 576, 576), (300, 520, 1536), (1024, 1024, 32000)])
 def test_linear_on_columns_of_a_wider_buffer(device, rows, cin, cout, pad):
-    """Rows that lie `pad` elements further apart than they are long, where the dense sizes go to the package's kernel (and,
-    for the last shape's weight gradient, to the library with a transposed operand)."""
+    """Rows that lie `pad` elements further apart than they are long, where the dense sizes go to the package's kernels; with
+    a pitch that is no multiple of 8 the product that reads it goes to the library."""
     from picotron_amd.model import Linear
     g = torch.Generator(device="cuda").manual_seed(rows + pad)
     layer = Linear(cin, cout, bias=False, device=device, dtype=torch.bfloat16)
@@ -181,21 +181,24 @@ MID_TILES = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (96, 64), (96, 96
              (128, 256)]
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 96, 64), (72, 136, 200), (200, 328, 72), (264, 272, 584), (520, 40, 1032)])
-@pytest.mark.parametrize("kind", ["NT", "NN", "TN"])
+@pytest.mark.parametrize("kind,M,N,K", [(kind, *size) for size in [(8, 8, 8), (64, 96, 64), (72, 136, 200), (200, 328, 72), (264, 272, 584), (520, 40, 1032)]
+                                        for kind in ("NT", "NN", "TN")] +
+                         [("NT", 1, 8, 8), ("NN", 1, 8, 8), ("NT", 33, 72, 136), ("NN", 33, 72, 136), ("TN", 72, 40, 1), ("TN", 72, 40, 333)])
 def test_products_of_one_round(device, kind, M, N, K):
-    """Every tile, at sizes around its edges, contractions of fewer steps than groups and of a ragged last step, operands that are
-    columns of wider matrices, against a fp32 product (rounded once: 2^-9)."""
+    """Every tile, at sizes around its edges, one row, contractions of fewer steps than groups and of a ragged last step, operands that are
+    columns of wider matrices, against a fp32 product (rounded once: 2^-9) and, with small integers, whose sums are exact in fp32, bit for bit."""
     from picotron_amd import _lib
     host = _lib.host()
     g = torch.Generator(device="cuda").manual_seed(M + K)
     sizes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     a, b = (torch.randn(r, c + 16, generator=g, device=device).to(torch.bfloat16)[:, 8:8 + c] for r, c in sizes)
-    want = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float())
+    ai, bi = a.round(), b.round()
+    want, exact = ((x.float().t() if kind == "TN" else x.float()) @ (y.float().t() if kind == "NT" else y.float()) for x, y in ((a, b), (ai, bi)))
     for tiles in MID_TILES:
         got, tile_m, tile_n = host.mid_product(a, b, kind, *tiles)
         assert (tile_m, tile_n) == tiles and ((got.float() - want).norm() / want.norm()).item() <= 3e-3, tiles
         assert torch.equal(got, host.mid_product(a, b, kind, *tiles)[0]), tiles
+        assert torch.equal(host.mid_product(ai, bi, kind, *tiles)[0], exact.to(torch.bfloat16)), tiles
     with pytest.raises(RuntimeError, match="no tiles"):
         host.mid_product(a, b, kind, 96, 128)
 
@@ -209,11 +212,14 @@ def test_products_in_pieces_of_one_round(device, kind, M, N, K):
     g = torch.Generator(device="cuda").manual_seed(K)
     sizes = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     a, b = (torch.randn(r, c + 16, generator=g, device=device).to(torch.bfloat16)[:, 8:8 + c] for r, c in sizes)
-    want, steps = (a.float().t() if kind == "TN" else a.float()) @ (b.float().t() if kind == "NT" else b.float()), (K + 63) // 64
+    ai, bi = a.round(), b.round()    # small integers: sums are exact in fp32
+    want, exact = ((x.float().t() if kind == "TN" else x.float()) @ (y.float().t() if kind == "NT" else y.float()) for x, y in ((a, b), (ai, bi)))
+    steps = (K + 63) // 64
     for tiles in [(64, 96), (64, 128), (96, 96), (128, 128), (128, 192), (192, 128), (128, 256)]:
         for parts in {2, 3, min(steps, 15), min(steps, 64)}:
             got = host.mid_product(a, b, kind, *tiles, parts)[0]
             assert ((got.float() - want).norm() / want.norm()).item() <= 3e-3, (tiles, parts)
+            assert torch.equal(host.mid_product(ai, bi, kind, *tiles, parts)[0], exact.to(torch.bfloat16)), (tiles, parts)
     assert ((host.product(a, b, kind).float() - want).norm() / want.norm()).item() <= 3e-3
     for bad in ((64, 64, 2), (64, 96, 65), (64, 96, steps + 1)):
         with pytest.raises(RuntimeError):

@@ -165,6 +165,38 @@ def test_the_large_predicate_is_what_the_kernel_refuses():
     assert lib.pico_product_large(1 << 20, 1 << 20, 1 << 20, 512, 576, 576, 576, 576, 0, 0, 128, 128, 1, None) == -3
 
 
+def test_the_predicate_of_the_products_of_one_round_is_what_the_kernels_refuse():
+    """pico_product_mid_takes against pico_product_mid and pico_product_pair themselves: with NULL operands an accepted shape ends at the pointers."""
+    from picotron_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    lib, seen = _lib.lib(), set()
+    sizes = ((1, 8, 8), (1, 8, 72), (512, 576, 576), (512, 576, 580), (516, 576, 576), (512, 580, 576), (2331, 1024, 2331), (0, 8, 8))
+    pads = (0, 4, 8, -8, 1 << 23, 1 << 31)
+    for M, N, K in sizes:
+        for a_slow, b_slow in ((0, 0), (0, 1), (1, 0), (1, 1)):
+            for pad_a in pads:
+                for pad_b in pads:
+                    lda, ldb = (M if a_slow else K) + pad_a, (N if b_slow else K) + pad_b
+                    takes = lib.pico_product_mid_takes(M, N, K, lda, ldb, a_slow, b_slow)
+                    rc = lib.pico_product_mid(None, None, None, M, N, K, lda, ldb, a_slow, b_slow, 64, 64, 1, None)
+                    assert rc == (-1 if takes else -3), (M, N, K, lda, ldb, a_slow, b_slow)
+                    seen.add(takes)
+    for rows, out, inner in sizes:
+        for pads_here in [(a, b, c) for a in pads for b in pads for c in pads]:
+            ld_dy, ld_w, ld_x = (n + pad for n, pad in zip((out, inner, inner), pads_here))
+            takes = lib.pico_product_mid_takes(rows, inner, out, ld_dy, ld_w, 0, 1) and lib.pico_product_mid_takes(out, inner, rows, ld_dy, ld_x, 1, 1)
+            rc = lib.pico_product_pair(None, None, None, None, None, rows, out, inner, ld_dy, ld_w, ld_x, 64, 64, 64, 64, None)
+            assert rc == (-1 if takes else -3), (rows, out, inner, pads_here)
+            seen.add(2 + takes)
+    assert seen == {0, 1, 2, 3}
+    p = 1 << 20    # (refused before anything is launched: tiles that there are none of, more pieces than steps)
+    for tile_m, tile_n, parts in ((96, 128, 1), (64, 64, 2), (64, 96, 10), (64, 96, 0)):
+        assert lib.pico_product_mid(p, p, p, 512, 576, 576, 576, 576, 0, 0, tile_m, tile_n, parts, None) == -3
+    for dx, dw in (((32, 32), (64, 64)), ((64, 64), (128, 128))):
+        assert lib.pico_product_pair(p, p, p, p, p, 512, 576, 576, 576, 576, 576, *dx, *dw, None) == -3
+
+
 def test_the_route_of_a_product():
     """Each route where it is taken and, beside it, where it is not: us without and with it."""
     run('''
