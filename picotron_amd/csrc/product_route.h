@@ -156,54 +156,44 @@ OwnProduct own_product(Product kind, int64_t M, int64_t N, int64_t K) {
 double last_round(double walk, double end, double used, double walk_idle, double end_idle) {   // (idle: of the time, where few CUs are busy)
   return used > 0 ? walk * (walk_idle + (1 - walk_idle) * used) + end * (end_idle + (1 - end_idle) * used) : 0;
 }
-double own_time(OwnProduct own, int64_t M, int64_t N, int64_t K) {
-  struct Form {
-    int64_t tile, groups;
-    double start, trip, end, walk_idle, end_idle;
-  };
-  static constexpr Form forms[] = {{64, 1, 2.82, 0.29, 0.17, 0.84, 0.00}, {64, 2, 1.87, 0.49, 1.26, 0.86, 0.84},
-                                   {128, 1, 3.44, 0.55, 1.45, 1.00, 0.08}, {128, 2, 2.76, 1.12, 2.92, 0.78, 0.30}};
-  for (const Form& f : forms) {
-    if (f.tile != own.tile || f.groups != own.groups) continue;
-    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
-    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
-    return f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
-  }
-  return 0;
-}
-// Whether a product goes to the package's kernel for products that fill the GPU (pico_product_large), in which tiles and in how
-// many pieces of the contraction (parts 0: no).
-//
-// The kernel's own time follows from its rounds: 256 workgroups take a tile each, a step of 64 of contraction costs 1.0 .. 1.4
-// us (less while part of the GPU idles), a tile's end 2 .. 5 us; and from what it reads and writes, at 4.8 TB/s.  Over 39000 timed
-// (shape, tile, pieces) the estimate has an error of 7 % (standard deviation).  Against it stands what the product would take
-// otherwise: pico_product's time, estimated to 3 .. 8 %, or the library's, whose choices are not monotone in any size and cannot be estimated
-// to better than 11 .. 34 %.  So the lines ask for a margin where the library is good, and for none where it never is.  Layers drawn over 64 .. 8192
-// rows, 64 .. 4096 columns on one side, up to 22016 on the other, and vocabularies of 24576 .. 151936, other ones than those that the lines were
-// drawn from, took, over the time without this kernel, in the geometric mean (slower than 1.05, at most):
-//   TN: 0.71 of the library's time (1768 products; 1, 1.07; [4096 x 4096]^T [4096 x 4096] 137 -> 103 us), 0.84 of pico_product's (216; 0, 1.01; under
-//     640 of contraction that one stays ahead but for a vocabulary's width).  A vocabulary's weight gradient of up to 768 columns over
-//     4000 rows (576: 3000) stays in the library, with an operand transposed: 0.95 .. 1.03 of that, one in four over 1.05 ([6080 x 49152]^T
-//     [6080 x 576] 333 us, here 387);
-//   NN: 0.82 whole (399; 0, 1.01; [2242 x 10880] @ [10880 x 4096] 248 -> 178) and 0.71 in pieces (421; 2, 1.08), see cut_limit;
-//   NT: 0.74 (912; 1, 1.07): the library's best layout ([4096 x 2048] @ [16384 x 2048]^T 194 us, here 203), except for large
-//     outputs of a short contraction ([3832 x 512] @ [49152 x 512]^T 315 -> 218) and where its tiles fit badly ([1790 x 16384] @ [4096 x
-//     16384]^T 424 -> 206).  Logits of up to 768 columns always ([680 x 576] @ [32000 x 576]^T 57 -> 29 us), unless they are short (256)
-//     and their rows no whole lines ([6912 x 192] @ [73448 x 192]^T 419, here 508).
-struct LargeProduct {
-  int64_t tile_m = 0, tile_n = 0, parts = 0;
-};
 // `work` us of products beside a walk through the operands and the result at `rate` TB/s: the longer one, and more where both are long
 double with_memory(double work, int64_t M, int64_t N, int64_t K, double rate) {
   const double memory = 2e-6 / rate * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N);
   return std::sqrt(std::sqrt(work * work * work * work + memory * memory * memory * memory));
 }
+double own_time(Product kind, OwnProduct own, int64_t M, int64_t N, int64_t K) {
+  struct Form {
+    int64_t tile, groups;
+    double start, trip, end, walk_idle, end_idle;
+  };
+  static constexpr Form forms[] = {{64, 1, 3.07, 0.26, 0.16, 0.84, 0.00}, {64, 2, 2.12, 0.54, 1.18, 0.86, 0.84},
+                                   {128, 1, 3.69, 0.52, 1.36, 1.00, 0.08}, {128, 2, 3.01, 1.14, 2.73, 0.78, 0.30}};
+  for (const Form& f : forms) {
+    if (f.tile != own.tile || f.groups != own.groups) continue;
+    const int64_t tiles = ((M + f.tile - 1) / f.tile) * ((N + f.tile - 1) / f.tile), steps = (K + 63) / 64;
+    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
+    const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
+    const double layout = kind == Product::TN ? 1.04 : f.tile == 64 ? (kind == Product::NT ? 0.93 : 1.04) : f.groups == 1 ? 0.95 : 1.0;
+    return with_memory(layout * t, M, N, K, 5.3);
+  }
+  return 0;
+}
+// The time of pico_product_large, the package's kernel for products that fill the GPU, and the tiles and pieces of the contraction that
+// take least.
+//
+// It follows from the rounds: 256 workgroups take a tile each, a step of 64 of contraction costs 1.1 .. 1.4 us (less while part of the
+// GPU idles), a tile's end 2 .. 5 us; and from what is read and written, at 4.4 TB/s.  Unit of all estimates here: a timed call, the
+// geometric mean of one with operands from memory and one with operands in the caches, over 1.07, less 3 us that any call shows.
+// Over 2900 timed (shape, tiles, pieces) the estimate has an error of 6 % (standard deviation).
+struct LargeProduct {
+  int64_t tile_m = 0, tile_n = 0, parts = 0;
+};
 double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
   struct Form {
     int64_t m, n;
     double step, end;
   };
-  static constexpr Form forms[] = {{256, 256, 1.43, 4.8}, {256, 192, 1.18, 5.6}, {192, 256, 1.2, 3.2}, {256, 128, 0.99, 2.4}, {128, 256, 1.0, 1.6}};
+  static constexpr Form forms[] = {{256, 256, 1.44, 4.6}, {256, 192, 1.31, 4.6}, {192, 256, 1.27, 2.9}, {256, 128, 1.13, 2.7}, {128, 256, 1.09, 1.9}};
   const int64_t steps = (K + 63) / 64;
   double least = 1e30;
   for (const Form& f : forms) {
@@ -212,18 +202,18 @@ double large_time(int64_t M, int64_t N, int64_t K, LargeProduct& best) {
       if (parts > 1 && (tiles * parts > 300 || steps < 8 * parts)) break;
       const int64_t full = tiles * parts / 256, rest = tiles * parts % 256, length = (steps + parts - 1) / parts;
       const double used = rest / 256.0;   // of the GPU, in the last round
-      double t = 5 + full * (length * f.step + f.end);
+      double t = 3.6 + full * (length * f.step + f.end);
       if (rest) t += length * f.step * (0.7 + 0.3 * used) + f.end * (0.45 + 0.55 * used);
-      if (parts > 1) t += 3.8 + 1e-6 * M * N * (0.63 * parts + 0.16);   // the pieces in fp32, and their sum
+      if (parts > 1) t += 5 + 1e-6 * M * N * (0.84 * parts - 0.4);   // the pieces in fp32, and their sum
       if (t < least) {
         least = t;
         best = {f.m, f.n, parts};
       }
     }
   }
-  return with_memory(least, M, N, K, 4.8);
+  return with_memory(least, M, N, K, 4.4);
 }
-// the same in the library (TN: 1.5 times this at the median, hardly ever less)
+// The library's at its best: hardly ever less, 1.0 .. 1.9 times this in the mean of a class of sizes, see library_cost
 double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
   struct Form {
     int64_t m, n;
@@ -240,6 +230,8 @@ double other_time(Product kind, int64_t M, int64_t N, int64_t K) {
   }
   return start[k] + least;
 }
+// (the library takes its largest tiles where their pieces fill the GPU)
+bool fills(int64_t M, int64_t N, int64_t parts) { return ((M + 255) / 256) * ((N + 255) / 256) * parts >= 256; }
 // The library's time for an input gradient that it would get in `parts` pieces (contraction_parts), at its best: whole tiles of a
 // contraction that divides evenly.
 double cut_time(int64_t M, int64_t N, int64_t K, int64_t parts) {
@@ -248,45 +240,15 @@ double cut_time(int64_t M, int64_t N, int64_t K, int64_t parts) {
     double step;
   };
   static constexpr Form forms[] = {{256, 256, 1.44}, {256, 128, 0.71}, {128, 256, 0.71}, {128, 128, 0.35}};
+  const bool full = fills(M, N, parts);
   double least = 1e30;
   for (const Form& f : forms) {
     const int64_t rounds = (((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n) * parts + 255) / 256;
+    if (f.m * f.n < 65536 && full) continue;
     least = std::min(least, rounds * (K / 64.0 / parts * f.step + 1.6));
   }
   return 2 + with_memory(least, M, N, K, 6.8) + 1.53e-6 * M * N * parts;
 }
-// What a kernel of the package's has to promise to get it.  Over 4000 timed products the library took, over cut_time, 0.98 .. 1.48 (a tenth and
-// nine tenths of them) with columns a multiple of 256 and a contraction of 1024, elsewhere 1.1 .. 2.0: there few kernels of its
-// do not fit.  A line of its own for vocabularies had [1536 x 49152] @ [49152 x 2048] at 262 -> 314 us, [3584 x 32768] @ [32768 x 512]
-// 120 -> 158; now 0.71 (large) and 0.55 (mid) of the library's time, as before, and 10 of 1460 over 1.05.  (Two pieces
-// need no margin: 20 of those products, none over 1.05; [4096 x 16384] @ [16384 x 2048] with operands from memory 225 us, here 218.)
-double cut_limit(int64_t M, int64_t N, int64_t K, int64_t parts) {
-  return (N % 256 != 0 || K % 1024 != 0 ? 1.3 : parts == 2 ? 1.0 : 0.92) * cut_time(M, N, K, parts);
-}
-LargeProduct large_product(Product kind, int64_t M, int64_t N, int64_t K) {
-  static_assert(static_cast<int>(Product::NT) == 0 && static_cast<int>(Product::NN) == 1 && static_cast<int>(Product::TN) == 2);
-  const int64_t narrow = std::min(M, N), wide = std::max(M, N);
-  LargeProduct best;
-  if (M < 1 || N < 1 || K < 128 || narrow < 192 || (wide >= 24576 && narrow < 256)) return {};
-  const double time = large_time(M, N, K, best), ideal = 2e-9 * M * N * K;   // (us at 1 PFLOP/s)
-  const OwnProduct own = own_product(kind, M, N, K);
-  bool take = false;
-  const bool vocabulary = wide >= 24576;
-  if (own.groups > 0) {
-    take = kind == Product::TN && (vocabulary ? narrow >= 384 && K >= 200 : K >= 640) && time < 0.9 * own_time(own, M, N, K);
-  } else if (kind == Product::TN) {
-    take = !vocabulary || narrow > 768 || K < (narrow > 576 ? 4000 : 3000);
-  } else if (kind == Product::NT) {
-    if (vocabulary && K <= 768) take = N % 64 == 0 || K > 256;
-    else take = time >= 14 && (time < (best.parts >= 6 ? 0.7 : 0.8) * other_time(kind, M, N, K) || (K <= 800 && time < 5 + ideal));
-  } else if (const int64_t parts = contraction_parts(kind, M, N, K); parts > 1) {
-    take = time < cut_limit(M, N, K, parts);
-  } else {
-    take = time >= 14 && (time < (best.parts >= 4 || time < 32 ? 0.75 : 0.85) * other_time(kind, M, N, K) || (best.parts < 4 && time < 5 + ideal / 1.05));
-  }
-  return take ? best : LargeProduct{};
-}
-
 // own_product's choice where the kernel takes the operands as they lie in memory; the library takes any row pitch
 OwnProduct own_product(Product kind, const ProductSizes& n) {
   const OwnProduct own = own_product(kind, n.M, n.N, n.K);
@@ -294,128 +256,144 @@ OwnProduct own_product(Product kind, const ProductSizes& n) {
   return own;
 }
 
-LargeProduct large_product(Product kind, const ProductSizes& n) {
-  const LargeProduct large = large_product(kind, n.M, n.N, n.K);
-  const bool takes = large.parts > 0 && pico_product_large_takes(n.M, n.N, n.K, n.lda, n.ldb, kind == Product::TN, kind != Product::NT,
-                                                                 static_cast<int>(large.parts));
-  return takes ? large : LargeProduct{};
-}
-
-// Whether a product goes to pico_product_mid and in which tiles (tile_m 0: no).
+// The time of pico_product_mid and the tiles that take least (tile_m 0: none).
 //
-// Its time follows from its rounds: 256 workgroups take a tile each, a trip (64 of contraction for each group of waves) costs `trip`,
-// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy; reading and writing go on beside, at 5.6 TB/s.
-// Over 27000 timed (shape, tiles) the estimate has an error of 7 .. 10 % (standard deviation), the larger one along a slow axis.  Against
-// it stands pico_product's or pico_product_large's own time, estimated alike, or the library's (other_time).  Of the drawn layers above those that
-// go here take, over the time without it, in the geometric mean (slower than 1.05, at most),
-//   NN 0.87 of pico_product's (2978 products; 1, 1.05; [512 x 3072] @ [3072 x 576] 12.9 -> 8.7 us) and 0.66 of the library's (1221; 4, 1.06; [2331 x
-//     3072] @ [3072 x 576] 27.7 -> 15.8),
-//   TN 0.75 of pico_product's (3570; 0, 1.05; [2331 x 3072]^T [2331 x 576] 23.7 -> 15.8) and 0.57 of the library's (503; 0),
-//   NT 0.94 of pico_product's (362; 0, 1.03) and 0.69 of the library's (3554; 10, 1.18; [2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5).  The forward's layout
-//     leaves pico_product only for a clear gain: tiles of 64 run level there.
-// Contractions that the library or pico_product_large would cut are cut here where that promises more than cut_limit (NN) or 0.88 of
-// pico_product_large's estimate: 0.54 of the library's time in its pieces (NN, 1039; 8, 1.28; [1063 x 8192] @ [8192 x 192] 20.7 -> 14.3 us, [145 x 49152] @
-// [49152 x 576] 37 -> 23) and 0.31 (TN, 424; 0).  And where a whole walk goes here, pieces that promise 0.9 of it ([208 x 5440] @ [256 x
-// 5440]^T 13.3 -> 10.3, [12232 x 288]^T [12232 x 576] 22.4 -> 14.9; with 0.95 two pieces of large outputs lost, [3584 x 3072]^T [3584 x 1024] 29.7 -> 35.8).
+// It follows from the rounds: 256 workgroups take a tile each, a trip (64 of contraction for each group of waves) costs `trip`,
+// a tile's start and end `end`, and in the last round both depend on how much of the GPU is busy; reading and writing go on beside, at 4.8 TB/s.
+// Over 7000 timed (shape, tiles) the estimate has an error of 4 .. 10 % (standard deviation), small tiles the larger one.
 struct MidProduct {
   int64_t tile_m = 0, tile_n = 0, parts = 1;
 };
 double mid_time(Product kind, int64_t M, int64_t N, int64_t K, MidProduct& best) {
   struct Form {
     int64_t m, n, groups;
-    double start, trip, end, walk_idle, end_idle;
+    double start, trip[3], end, walk_idle, end_idle;   // (trip: NT, NN, TN)
   };
   static constexpr Form forms[] = {
-      {32, 32, 4, 1.54, 0.50, 1.46, 0.47, 1.12},   {32, 64, 4, 1.37, 0.62, 1.78, 0.64, 1.09},   {64, 32, 4, 1.36, 0.68, 1.71, 0.58, 1.15},
-      {64, 64, 2, 1.51, 0.43, 1.98, 0.80, 0.83},   {64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81},   {96, 64, 2, 1.54, 0.56, 2.29, 0.82, 0.75},
-      {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73},  {128, 64, 2, 1.59, 0.67, 2.58, 0.86, 0.70},
-      {128, 96, 2, 1.31, 1.01, 2.83, 0.71, 0.79},  {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60}, {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45},
-      {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37}, {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36}};
+      {32, 32, 4, 1.89, {0.67, 0.69, 0.87}, 1.14, 0.47, 1.12}, {32, 64, 4, 1.72, {0.83, 0.88, 1.01}, 1.39, 0.64, 1.09},
+      {64, 32, 4, 1.71, {0.90, 1.20, 1.12}, 1.33, 0.58, 1.15}, {64, 64, 2, 1.86, {0.52, 0.57, 0.56}, 1.54, 0.80, 0.83},
+      {64, 96, 2, 1.84, {0.66, 0.71, 0.68}, 1.76, 0.78, 0.81}, {96, 64, 2, 1.89, {0.73, 0.67, 0.68}, 1.79, 0.82, 0.75},
+      {96, 96, 2, 1.84, {0.83, 0.85, 0.88}, 2.18, 0.82, 0.75}, {64, 128, 2, 1.88, {0.81, 0.83, 0.80}, 1.98, 0.84, 0.73},
+      {128, 64, 2, 1.94, {0.82, 0.80, 0.87}, 2.01, 0.86, 0.70}, {128, 96, 2, 1.66, {1.20, 1.28, 1.21}, 2.21, 0.71, 0.79},
+      {128, 128, 2, 1.98, {1.35, 1.36, 1.23}, 2.68, 0.84, 0.60}, {128, 192, 1, 2.24, {0.79, 0.77, 0.77}, 3.06, 0.90, 0.45},
+      {192, 128, 1, 2.52, {0.88, 0.83, 0.84}, 2.85, 0.90, 0.37}, {128, 256, 1, 2.52, {1.03, 0.92, 0.96}, 3.53, 0.89, 0.36}};
   const int64_t steps = (K + 63) / 64;
   double least = 1e30;
   for (const Form& f : forms) {
     const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n);
-    // (long walks along a slow axis in rows of 64 or 128 bytes take up to twice that)
-    if (tiles > 1024 || (f.m == 32 && ((f.n == 32 && steps > 48) || (kind != Product::NT && steps > 64)))) continue;
-    const double walk = (steps + f.groups - 1) / f.groups * f.trip;
+    // (long walks along a slow axis in rows of 64 bytes take up to twice that: [4819 x 232]^T [4819 x 184] 36 us in tiles of 64 x 32, 14 in pieces)
+    if (tiles > 1024 || (f.m == 32 && f.n == 32 && steps > 48) || (std::min(f.m, f.n) == 32 && kind != Product::NT && steps > 64)) continue;
+    const double walk = (steps + f.groups - 1) / f.groups * f.trip[static_cast<int>(kind)];
     const double t = f.start + tiles / 256 * (walk + f.end) + last_round(walk, f.end, tiles % 256 / 256.0, f.walk_idle, f.end_idle);
     if (t < least) {
       least = t;
       best = {f.m, f.n, 1};
     }
   }
-  return with_memory(least, M, N, K, 5.6);
+  return with_memory(least, M, N, K, 4.8);
 }
-// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces' sum: 10 % error over
-// 11000 timed (shape, tiles, pieces).
+// The same for a contraction that is cut into pieces, one round of workgroups of one piece each, and the pieces' sum: 6 .. 7 % error over
+// 2100 timed (shape, tiles, pieces).  (1.5 us of it are for the second launch, which costs more where the operands are in the caches.)
 double mid_parts_time(int64_t M, int64_t N, int64_t K, MidProduct& best) {
   struct Form {
     int64_t m, n, groups;
-    double start, trip, end, walk_idle, end_idle, share;   // (share: of a trip's time in mid_time)
+    double start, trip, end, walk_idle, end_idle;
   };
-  static constexpr Form forms[] = {{64, 96, 2, 1.49, 0.56, 2.25, 0.78, 0.81, 0.86},   {64, 128, 2, 1.53, 0.66, 2.54, 0.84, 0.73, 0.90},
-                                   {96, 96, 2, 1.49, 0.73, 2.80, 0.82, 0.75, 0.88},   {128, 128, 2, 1.63, 1.06, 3.43, 0.84, 0.60, 0.93},
-                                   {128, 192, 1, 1.89, 0.71, 3.92, 0.90, 0.45, 0.95}, {192, 128, 1, 2.17, 0.75, 3.66, 0.90, 0.37, 0.93},
-                                   {128, 256, 1, 2.17, 0.87, 4.53, 0.89, 0.36, 0.95}};
+  static constexpr Form forms[] = {
+      {64, 96, 2, 5.19, 0.69, 2.25, 0.78, 0.81}, {64, 128, 2, 5.23, 0.82, 2.54, 0.84, 0.73}, {96, 96, 2, 5.19, 0.85, 2.80, 0.82, 0.75},
+      {128, 128, 2, 5.33, 1.27, 3.43, 0.84, 0.60}, {128, 192, 1, 5.59, 0.72, 3.92, 0.90, 0.45}, {192, 128, 1, 5.87, 0.70, 3.66, 0.90, 0.37},
+      {128, 256, 1, 5.87, 0.83, 4.53, 0.89, 0.36}};
   const int64_t steps = (K + 63) / 64;
   double least = 1e30;
   for (const Form& f : forms) {
     const int64_t tiles = ((M + f.m - 1) / f.m) * ((N + f.n - 1) / f.n), most = 256 / tiles;
-    for (const int64_t parts : {most, 2 * most / 3, most / 2}) {
-      if (parts < 2 || parts > 64 || steps < 2 * parts) continue;
+    for (const int64_t wanted : {most, 2 * most / 3, most / 2}) {
+      const int64_t parts = std::min<int64_t>({wanted, 64, steps / 2});
+      if (parts < 2) continue;
       const double walk = ((steps + parts - 1) / parts + f.groups - 1) / f.groups * f.trip;
-      const double t = f.start + last_round(f.share * walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 4.8 + 1e-6 * M * N * (1.41 * parts - 0.9);
+      const double t = f.start + last_round(walk, f.end, tiles * parts / 256.0, f.walk_idle, f.end_idle) + 1e-6 * M * N * (1.82 * parts - 1.13);
       if (t < least) {
         least = t;
         best = {f.m, f.n, parts};
       }
     }
   }
-  return with_memory(least, M, N, K, 5.6);
+  return with_memory(least, M, N, K, 4.6);
 }
-MidProduct mid_product(Product kind, const ProductSizes& n, const LargeProduct& large, const OwnProduct& own) {
-  const auto [M, N, K, lda, ldb] = n;
-  if (M < 1 || N < 1 || K < 1 || !pico_product_mid_takes(M, N, K, lda, ldb, kind == Product::TN, kind != Product::NT)) return {};
-  // With few tiles the library deals out a contraction that divides evenly: [128 x 3328] @ [832 x 3328]^T 6.9 us, here 9.0; over 300 such
-  // products whole walks here took 1.06 .. 1.3 of its time, and 0.6 .. 0.9 with other contractions or more tiles.
-  const bool dealt = kind == Product::NT && K > 3072 && (K % 256 == 0 ? K <= 8192 : K % 128 == 0 && K <= 4352) && ((M + 31) / 32) * ((N + 63) / 64) <= 128;
-  MidProduct best, cut;
-  LargeProduct same;
-  const double time = mid_time(kind, M, N, K, best), pieces = mid_parts_time(M, N, K, cut), least = std::min(time, pieces);
-  const int64_t library_parts = own.groups > 0 ? 1 : contraction_parts(kind, M, N, K);
-  if (kind == Product::NN && library_parts > 1) {
-    const bool take = large.parts > 0 ? least < large_time(M, N, K, same) : least < cut_limit(M, N, K, library_parts);
-    return !take ? MidProduct{} : pieces < time ? cut : best;
-  }
-  if ((large.parts > 0 || library_parts > 1) && pieces < time && pieces < 0.88 * large_time(M, N, K, same)) return cut;
-  bool take;
-  if (large.parts > 0) take = time < 0.9 * large_time(M, N, K, same);
-  else if (own.groups > 0) {   // (margins that the estimates' errors need: along one slow axis and in tiles of 128 x 256 they are larger)
-    const int64_t area = best.tile_m * best.tile_n;
-    take = time < (kind == Product::NT ? 0.9 : area < 6144 ? 0.97 : kind == Product::NN ? 0.9 : area < 32768 ? 0.94 : 0.92) * own_time(own, M, N, K);
-  }
-  else {   // (a margin that grows with the work: a wrong choice between two full GPUs costs more than it can gain)
-    const double gflop = 2e-9 * M * N * K;
-    take = library_parts == 1 && turned_operand(kind, n) == 0 && time < (kind == Product::NN ? (gflop < 20 ? 0.97 : 0.87) : gflop < 6 ? 0.9 : 0.84) * other_time(kind, M, N, K);
-  }
-  if (!take) return {};
-  return pieces < 0.9 * time ? cut : dealt ? MidProduct{} : best;
-}
-
 // The route of a product: the library whole or in `parts` pieces of the contraction, with operand `turn` (1: a, 2: b) transposed first;
 // pico_product (a square tile, groups), pico_product_mid or pico_product_large (tiles, pieces).
 struct ProductRoute {
   enum Kernel { Library, Own, Mid, Large } kernel = Library;
   int64_t tile_m = 0, tile_n = 0, groups = 0, parts = 1, turn = 0;
 };
+// What the library promises for a product: what it took, over its time at its best, where the package's kernels were as fast, by classes of sizes.  Its
+// choice of tiles is not monotone in any size, and it has few kernels for contractions that are no multiple of 64 and for rows that are no whole lines
+// (over other_time: NN 1.0 and 1.3, NT 1.0 and 1.35; in pieces, over cut_time, 1.3 and 1.9), so a class spreads over 12 .. 28 %.  Forward products with much
+// work are its best: there the line is on its side ([4096 x 4096] @ [4096 x 4096]^T 93 us, pico_product_large 103; [4096 x 2048] @ [16384 x 2048]^T 192, 206),
+// but for short contractions ([3832 x 512] @ [49152 x 512]^T 315, 218).  A vocabulary's logits of up to 768 columns leave always ([680 x 576] @ [32000 x
+// 576]^T 57 -> 29), unless they are short (256) and their rows no whole lines ([6912 x 192] @ [73448 x 192]^T 433, 523).  Weight gradients are its slowest
+// layout, unless an operand is transposed first.
+double library_cost(Product kind, const ProductSizes& n, int64_t parts, int64_t turn) {
+  const auto [M, N, K, lda, ldb] = n;
+  const bool odd_k = K % 64 != 0, odd_n = N % 64 != 0;
+  if (parts > 1 && kind == Product::NN) {
+    const bool few = ((M + 127) / 128) * ((N + 127) / 128) * parts <= 256;
+    return (K / parts % 64 != 0 ? 1.6 : odd_n ? 1.55 : N % 256 != 0 ? 1.45 : few ? 1.6 : fills(M, N, parts) ? 1.0 : 1.15) * cut_time(M, N, K, parts);
+  }
+  const double whole = other_time(kind, M, N, K);
+  if (kind == Product::TN && turn != 0) return (odd_k ? 1.15 : odd_n ? 1.1 : std::min(M, N) < 256 ? 1.1 : 0.75) * whole;
+  if (kind == Product::TN) return 1.5 * whole;
+  const double gflop = 2e-9 * M * N * K;
+  if (kind == Product::NT && N >= 24576 && K <= 768) return (odd_n && K <= 256 ? 0.65 : 2) * whole;
+  if (kind == Product::NT) return (odd_k ? (gflop >= 40 ? 1.25 : 1.5) : K <= 800 && gflop >= 16 ? 1.2 : odd_n ? (gflop >= 40 ? 1.05 : 1.2) : gflop >= 40 ? 0.9 : 1.0) * whole;
+  return (odd_k ? 1.45 : odd_n ? 1.35 : K % 1024 != 0 ? 1.25 : 1.2) * (K >= 24576 ? 1.25 : 1.0) * whole;
+}
+// The kernel that promises least.  (Lines that compared the kernels in pairs, with a margin each, sent products past kernels that the next pair would have
+// taken: [1025 x 32000] @ [32000 x 336] 54 us in pico_product_large, 104 in the library's pieces.)  Of 4958 products of drawn
+// layers (64 .. 8192 rows, 64 .. 4096 columns, up to 22016 on the other side, four vocabularies) the choice takes 1.019 of the fastest kernel's time in the
+// geometric mean and 0.823 of the time without pico_product_mid and pico_product_large; 100 are over 1.05 of that, 1.22 at most.  With and without, us:
+//   NT: 0.81 of the library's time in pico_product_large, 0.71 in pico_product_mid ([2331 x 1536] @ [576 x 1536]^T 12.0 -> 9.5);
+//   NN: 0.81 in pico_product_large ([2242 x 10880] @ [10880 x 4096] 248 -> 178; in pieces [4096 x 49152] @ [49152 x 2048] 663 -> 635), 0.67 in pico_product_mid ([2331
+//     x 3072] @ [3072 x 576] 27.7 -> 15.8; [145 x 49152] @ [49152 x 576] 37 -> 23), 0.93 of pico_product's ([512 x 3072] @ [3072 x 576] 12.9 -> 8.7);
+//   TN: 0.80 in pico_product_large ([4096 x 4096]^T [4096 x 4096] 137 -> 103), 0.63 in pico_product_mid; 0.88 of pico_product's ([451 x 9792]^T [451 x 3264] 49.7 -> 38.8; [2331 x 3072]^T [2331 x 576] 23.7 -> 15.8).
 ProductRoute choose_route(Product kind, const ProductSizes& n) {
-  const LargeProduct large = large_product(kind, n);
+  const auto [M, N, K, lda, ldb] = n;
+  const int a_slow = kind == Product::TN, b_slow = kind != Product::NT;
   const OwnProduct own = own_product(kind, n);
-  const MidProduct mid = mid_product(kind, n, large, own);
-  if (mid.tile_m > 0) return {ProductRoute::Mid, mid.tile_m, mid.tile_n, 0, mid.parts, 0};
-  if (large.parts > 0) return {ProductRoute::Large, large.tile_m, large.tile_n, 0, large.parts, 0};
-  if (own.groups > 0) return {ProductRoute::Own, own.tile, own.tile, own.groups, 1, 0};
-  return {ProductRoute::Library, 0, 0, 0, contraction_parts(kind, n.M, n.N, n.K), turned_operand(kind, n)};
+  ProductRoute route;
+  double least;
+  if (own.groups > 0) {
+    route = {ProductRoute::Own, own.tile, own.tile, own.groups, 1, 0};
+    least = own_time(kind, own, M, N, K);
+  } else {
+    route = {ProductRoute::Library, 0, 0, 0, contraction_parts(kind, M, N, K), turned_operand(kind, n)};
+    least = 1.5 + library_cost(kind, n, route.parts, route.turn);   // (1.5 us: its calls take the host longer)
+  }
+  auto consider = [&](double cost, const ProductRoute& other) {
+    if (cost >= least) return;
+    least = cost;
+    route = other;
+  };
+  if (M < 1 || N < 1 || K < 1) return route;
+  // A step of many products with much work runs at the GPU's limit of power, where what moves more per product is slower than it is by itself:
+  // pico_product_mid and narrow tiles ([5640 x 12288]^T [5640 x 1536] by itself 211 us in mid, 226 in large; in a training step 234 and 197).
+  const double gflop = std::min(M, N) >= 512 ? 2e-9 * M * N * K : 0, narrow = gflop >= 60 ? 1.15 : gflop >= 25 ? 1.1 : 1.0, mid = gflop >= 60 ? 1.25 : 1.0;
+  // (rows that start in the same memory channel: [3584 x 32768] @ [32768 x 512] 131 us in the library's pieces, 178 in this kernel's)
+  const bool strided = kind == Product::NN && lda % 32768 == 0 && N <= 1024;
+  LargeProduct large;
+  const double large_cost = large_time(M, N, K, large);
+  if (K >= 128 && std::min(M, N) >= 192 && pico_product_large_takes(M, N, K, lda, ldb, a_slow, b_slow, static_cast<int>(large.parts)))
+    consider((strided ? 1.35 : large.tile_m * large.tile_n < 65536 ? narrow : 1.0) * large_cost, {ProductRoute::Large, large.tile_m, large.tile_n, 0, large.parts, 0});
+  if (pico_product_mid_takes(M, N, K, lda, ldb, a_slow, b_slow)) {
+    MidProduct whole, cut;
+    const double whole_cost = mid * mid_time(kind, M, N, K, whole), cut_cost = mid * mid_parts_time(M, N, K, cut);
+    // With few tiles the library deals out a contraction that divides evenly: [128 x 3328] @ [832 x 3328]^T 6.9 us, here 9.0; over 300 such
+    // products whole walks here took 1.06 .. 1.3 of its time, and 0.6 .. 0.9 with other contractions or more tiles.
+    const bool dealt = kind == Product::NT && K > 3072 && (K % 256 == 0 ? K <= 8192 : K % 128 == 0 && K <= 4352) && ((M + 31) / 32) * ((N + 63) / 64) <= 128;
+    if (whole.tile_m > 0 && !dealt) consider(whole_cost, {ProductRoute::Mid, whole.tile_m, whole.tile_n, 0, 1, 0});
+    if (cut.parts > 1 && !dealt) consider(cut_cost, {ProductRoute::Mid, cut.tile_m, cut.tile_n, 0, cut.parts, 0});
+  }
+  return route;
 }
 
 // The rules go through some thirty tiles each, 0.4 .. 1.3 us a call on the side that paces a small model's step (13 us of a two-layer
@@ -495,8 +473,11 @@ GradientTiles choose_gradient_tiles(int64_t rows, int64_t out, int64_t in) {
         best = {{x.m, x.n, 1}, {w.m, w.n, 1}};
       }
     }
-  MidProduct alone;
-  return least < 0.94 * (mid_time(Product::NN, rows, in, out, alone) + mid_time(Product::TN, out, in, rows, alone)) ? best : GradientTiles{};
+  auto alone = [](Product kind, int64_t M, int64_t N, int64_t K) {
+    MidProduct tiles;
+    return std::min(mid_time(kind, M, N, K, tiles), mid_parts_time(M, N, K, tiles));
+  };
+  return least < 0.85 * (alone(Product::NN, rows, in, out) + alone(Product::TN, out, in, rows)) ? best : GradientTiles{};
 }
 GradientTiles gradient_tiles(int64_t rows, int64_t out, int64_t in) {
   static thread_local RouteTable<GradientTiles> table;

@@ -92,7 +92,7 @@ def test_row_pitches_the_kernels_refuse_go_to_the_library():
     """The sizes route to the package's kernels; the pitch (no multiple of 8, or rows too far apart) sends them past, to the library
     or, where only the operand that stays as it is does not fit, to the library with the other one transposed."""
     run('''
-for kind, M, N, K, want in (("NT", 512, 576, 576, "own 64 in 2 groups"), ("NN", 512, 1024, 1024, "mid 32x64"), ("TN", 576, 960, 512, "own 64 in 2 groups"),
+for kind, M, N, K, want in (("NT", 512, 576, 576, "own 64 in 2 groups"), ("NN", 512, 1024, 1024, "mid 32x64"), ("TN", 2048, 2048, 4096, "own 128 in 2 groups"),
                             ("TN", 49152, 2048, 4096, "large 256x256"), ("TN", 2048, 49152, 4096, "large 256x256")):
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     for pad_a, pad_b in ((0, 0), (8, 0), (0, 24), (4, 0), (0, 4), (1, 1), (4, 24), (0, 1 << 24), (1 << 24, 0)):
@@ -204,23 +204,27 @@ for kind, M, N, K, want in (("TN", 4096, 4096, 4096, "large 256x256"),       # 1
                             ("TN", 6144, 2048, 4096, "large 192x256"),       # 101, 91
                             ("TN", 16384, 2048, 4096, "large 256x256"),      # 216, 199
                             ("TN", 49152, 576, 512, "large 192x256"),        # 45, 40
-                            ("TN", 32000, 256, 512, "own 128 in 1 group"),   # (level in the large kernel)
+                            ("TN", 32000, 256, 512, "mid 128x256"),          # own 17.2, 16.5
                             ("TN", 49152, 128, 7358, "turned"),              # 161, large 179
-                            ("TN", 2048, 2048, 4096, "mid 128x128"),         # 42, 39, large 51
+                            ("TN", 2048, 2048, 4096, "own 128 in 2 groups"), # 42, mid 39 .. 57 (operands from the caches, from memory), large 51
                             ("NN", 2242, 10880, 4096, "large 256x256"),      # 248, 178
                             ("NN", 608, 576, 49152, "mid 128x192 in 17"),    # 84, large 55
                             ("NN", 4548, 1024, 1024, "mid 128x192"),         # 17, large 20
                             ("NN", 2886, 3072, 49152, "library in 4"),       # 785, large 846
+                            ("NN", 4096, 2048, 49152, "large 256x256 in 2"), # 663, 635
+                            ("NN", 5108, 2816, 21504, "large 256x256"),      # 751, 472
+                            ("NN", 4608, 3840, 16384, "library in 2"),       # 475, large 605
                             ("NT", 3832, 49152, 512, "large 256x256"),       # 315, 218
                             ("NT", 5856, 6144, 768, "large 192x256"),        # 79, 52
                             ("NT", 4096, 16384, 2048, "library"),            # 194, large 203
-                            ("NT", 512, 49152, 576, "large 128x256"),        # 41, 34
-                            ("NT", 512, 576, 576, "own 64 in 2 groups"),
+                            ("NT", 512, 49152, 576, "large 256x256"),        # 41, 34, in 128 x 256 46
+                            ("NT", 512, 576, 576, "own 64 in 2 groups"),     # mid level
                             ("NN", 512, 576, 3072, "mid 32x64"),             # own 12.9, 8.7
-                            ("NN", 2331, 576, 3072, "mid 64x96"),            # 27.7, 15.8
+                            ("NN", 2331, 576, 3072, "mid 96x64"),            # 27.7, 15.8
                             ("TN", 3072, 576, 2331, "mid 64x128"),
                             ("NT", 2331, 576, 1536, "mid 64x96"),            # 12.0, 9.5
-                            ("NT", 128, 2048, 8192, "mid 64x96 in 5")):      # 14.9 in the library
+                            ("NT", 256, 4096, 10880, "large 128x256 in 8"),  # 53.3, 42.9
+                            ("NT", 128, 2048, 8192, "library in 8")):
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
     assert got == want, (kind, M, N, K, got)
@@ -254,18 +258,26 @@ def test_products_stay_where_the_other_kernels_lose():
     """Sizes of every kind that an own kernel, or another one, took and lost at: us where they go, us where they had gone."""
     run('''
 for kind, M, N, K, want in (("NN", 1536, 2048, 49152, "library in 4"),       # 262, large 314
-                            ("NN", 3584, 512, 32768, "library in 8"),        # 120, large 158
-                            ("NN", 1974, 1536, 12288, "library in 4"),       # 82, mid in pieces 90
+                            ("NN", 3584, 512, 32768, "library in 8"),        # 131, large 178, mid 145
+                            ("NN", 1974, 1536, 12288, "library in 4"),       # 81, large 78, mid in pieces 90
+                            ("NN", 1317, 4096, 49152, "large 192x256 in 2"), # 535, library in pieces 686
+                            ("NN", 1025, 336, 32000, "mid 192x128 in 14"),  # 54, library in pieces 104
+                            ("NN", 538, 768, 32000, "mid 192x128 in 14"),   # 55, library in pieces 104
+                            ("NN", 6144, 1520, 344, "large 192x256"),        # 24, library 35
+                            ("TN", 232, 184, 4819, "mid 64x96 in 21"),       # 14, mid in tiles of 64 x 32 36
+                            ("TN", 32000, 192, 1987, "mid 128x192"),         # 49, library with an operand transposed 64
+                            ("NT", 4096, 4096, 4096, "library"),             # 93, large 103
+                            ("NT", 4096, 49152, 2048, "library"),            # 575, large 624
                             ("NN", 3274, 920, 2384, "own 128 in 2 groups"),  # 25.3, mid 28.5
                             ("NN", 64, 1784, 5376, "mid 64x96 in 6"),        # 11, mid 32x64 18
                             ("TN", 49152, 576, 6080, "turned"),              # 333, large 387
                             ("TN", 50304, 384, 243, "own 128 in 1 group"),   # 19.4, large 23.6
                             ("TN", 3072, 1024, 3584, "own 128 in 2 groups"), # 31.9, mid in pieces 35.8
-                            ("TN", 2048, 2048, 5624, "own 128 in 2 groups"), # 56, mid 61
-                            ("TN", 9792, 3264, 451, "own 128 in 1 group"),   # 43.9, mid 50.4
+                            ("TN", 2048, 2048, 5624, "large 256x256 in 4"),  # 60, own 59, mid 61
+                            ("TN", 9792, 3264, 451, "large 256x256"),        # 38.8, own 49.7, mid 50.4
                             ("NT", 128, 832, 3328, "library"),               # 6.9, mid 9.0
                             ("NT", 6912, 73448, 192, "library"),             # 419, large 508
-                            ("NT", 256, 2112, 2112, "own 64 in 2 groups"),   # 9.0, mid 9.8
+                            ("NT", 256, 2112, 2112, "own 64 in 2 groups"),   # 9.0, mid 9.4
                             ("NT", 64, 2688, 8064, "mid 64x96 in 9")):       # 0.57 of the library's time
     (ra, ca), (rb, cb) = ((K, M) if kind == "TN" else (M, K)), ((N, K) if kind == "NT" else (K, N))
     got = host.product_route(operand(ra, ca), operand(rb, cb), kind)
