@@ -319,7 +319,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       kt.fragments(region, lane, kf);
       vt.fragments(region, lane, vf);
     } else {
-      // the first wave of each pair leaves both tiles in the pair's piece of LDS
+      // the first of the waves that share these keys leaves both tiles in their piece of LDS
       kt.fragments(split_k, lane, kf);
       vt.fragments(split_v, lane, vf);
     }
@@ -944,10 +944,8 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc) {
           const bf16x8 dsf = pack8(dp_acc[mb], 8 * cc);
-          const int krow = 32 * mb + 16 * cc + 4 * h + (lane % 16) / 4;
 #pragma unroll
           for (int db = 0; db < D / 32; ++db) {
-            const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
             const bf16x8 ktf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
             dq[db] = mfma32(ktf, dsf, dq[db]);
           }

@@ -33,16 +33,8 @@ __device__ __forceinline__ s16x4 lds_read_tr(const __bf16* p) {
 }
 
 // Two transposed reads -> the 8 k-slots of an MFMA operand.  Slots 0-3 come from rows
-// row0 .. row0+3, slots 4-7 from rows row0+8 .. row0+11 (the register order of a C tile).
-__device__ __forceinline__ bf16x8 lds_read_tr_pair(const __bf16* p, int ld) {
-  s16x4 lo = lds_read_tr(p);
-  s16x4 hi = lds_read_tr(p + 8 * ld);
-  typedef __attribute__((ext_vector_type(8))) short s16x8;
-  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
-}
-
-// the same with the second read `step` elements after the first (tiles whose rows are not evenly spaced)
+// row0 .. row0+3, slots 4-7 from rows row0+8 .. row0+11 (the register order of a C tile): the second read lies `step` elements
+// after the first (rows need not be evenly spaced).
 __device__ __forceinline__ bf16x8 lds_read_tr_pair_step(const __bf16* p, int step) {
   s16x4 lo = lds_read_tr(p);
   s16x4 hi = lds_read_tr(p + step);

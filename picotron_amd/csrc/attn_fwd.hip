@@ -355,10 +355,8 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
 #pragma unroll
           for (int cc = 0; cc < 2; ++cc) {
             const bf16x8 pf = pack8(s_acc[mb], 8 * cc);
-            const int krow = 32 * mb + 16 * cc + 4 * h + (lane % 16) / 4;
 #pragma unroll
             for (int db = 0; db < D / 32; ++db) {
-              const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
               const bf16x8 vf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
               o[qb][db] = mfma32(vf, pf, o[qb][db]);
             }

@@ -399,7 +399,7 @@ void launch_dw_reduce(const float* partial, void* dweight, int dweight_dtype, in
 // Few rows: dx and dweight in one launch.  There a backward takes the time of its two launches (the second one waits for the
 // partial sums of the first), so dweight has workgroups of its own, which read dy and x once more instead
 // of waiting for anybody: 32 columns of all rows each, they come first in the grid, the rows' waves after them.  The same fp32 products
-// as above, added in the order of 128 interleaved row lists.  bf16 with residual, us: [512 x 576] 6.3 -> 3.2, [64 x 2048] 7.4 -> 3.7,
+// as above, added in the order of 128 (fp32: 64) interleaved row lists.  bf16 with residual, us: [512 x 576] 6.3 -> 3.2, [64 x 2048] 7.4 -> 3.7,
 // [1024 x 576] 6.6 -> 4.3, [1024 x 4096] 13.5 -> 11.5.  Up to 1024 rows nothing loses (64 .. 1024 rows of 192 .. 4096, both types); with 1536 rows of
 // 2048 the second reading costs what the launch saves (11.6, 11.8), with 2048 of 192 as well (6.0, 6.4).
 constexpr int kFewThreads = 512, kFewCols = 32, kFewRows = 1024;
