@@ -72,14 +72,13 @@ struct KvCfg {
   // pieces of 4 consecutive rows tile the banks (transposed reads at their minimum of 2 requests per bank; at a pitch
   // of D + 8 they take 3-4), and the 4-word skew per 4 rows spreads 16 consecutive rows over all multiples of 4 words
   // (row reads at their minimum of 4).
-  // QS > 1: the tiles are filled by loads that go to LDS directly, 1 KiB of consecutive addresses per wave, so their rows are
-  // dense; the 16-byte pieces of a row change places instead (tile_twist), which spreads both kinds of read as evenly.
+  // QS > 1: the tiles are filled by loads that go to LDS directly and lie as TileLayout says.
   // (The loop is paced by LDS reads and their latency, the matrix cores are busy for half of it: without the LDS writes and
   // with more of K in registers B1 H32 S4096 281 -> 271 us, H32/8 S8192 1000 -> 950.  At head_dim 64 a wave's two sub-blocks take
-  // all 256 registers, and the flipped addresses of this layout end up in scratch: S4096 143 -> 156 us, so it keeps the pitch.)
+  // nearly all 256 registers.)
   static constexpr int LDQ = kSplit ? D : D + 32;
   static constexpr int kSkew = kSplit ? 0 : 8;
-  static constexpr int kTileElems = BM * LDQ + kSkew * (BM / 4);       // one tile
+  static constexpr int kTileElems = kSplit ? TileLayout<D>::bytes(BM) / 2 : BM * LDQ + kSkew * (BM / 4);       // one tile
   static constexpr int kTrStep = 8 * LDQ + 2 * kSkew;                  // 8 rows further down
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kQLoads = BM * kVecPerRow / kThreads;
@@ -156,6 +155,7 @@ __host__ __device__ constexpr int dkdv_piece_floats(int D) { return 2 * (D / 32)
 template <int D, int QS, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int ktile, const int part = 0, const int parts = 1) {
   using C = KvCfg<D, QS>;
+  using L = TileLayout<D>;
   constexpr bool kSplit = C::kSplit;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -226,7 +226,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
   for (int i = 0; i < C::kQLoads; ++i) {
     const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = kSplit ? idx % C::kVecPerRow ^ tile_twist<D>(r) : idx % C::kVecPerRow;
+    const int r = kSplit ? L::row(wave_id + C::NW * i, lane) : idx / C::kVecPerRow, cv = kSplit ? L::column(lane) / 8 : idx % C::kVecPerRow;
     q_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.qs[2] + cv * 8) * 2);
     do_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.os[2] + cv * 8) * 2);
   }
@@ -264,14 +264,14 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   // QS > 1: the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
   auto request_tile = [&](uint32_t buf_off) {
     const u32x4 qb = request_window(reinterpret_cast<uint64_t>(cur.q), cur.q_left), dob = request_window(reinterpret_cast<uint64_t>(cur.dout), cur.do_left);
-    const uint32_t to = buf_off + __builtin_amdgcn_readfirstlane(wave_id) * 1024;
+    const uint32_t to = buf_off + __builtin_amdgcn_readfirstlane(wave_id) * L::kPitch;
     each_load<C::kQLoads>([&](auto load) {
       constexpr int i = decltype(load)::value;
-      request16_to<i * C::kThreads * 16>(to, qb, q_off[i]);
+      request16_to<i * C::NW * L::kPitch>(to, qb, q_off[i]);
     });
     each_load<C::kQLoads>([&](auto load) {
       constexpr int i = decltype(load)::value;
-      request16_to<C::kTileElems * 2 + i * C::kThreads * 16>(to, dob, do_off[i]);
+      request16_to<C::kTileElems * 2 + i * C::NW * L::kPitch>(to, dob, do_off[i]);
     });
   };
   auto prefetch = [&]() {  // the tile under the cursor
@@ -336,6 +336,11 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   // NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
+  // (QS > 1) the lane's places in the wave's sub-block of a tile, and in its keys' K and V
+  const int sub_block = query_sb / 2 * L::kRows64 + query_sb % 2 * L::kRows32;
+  uint32_t row_first = sub_block + L::row_place(lane), tr_first = sub_block + L::column_place(lane);
+  uint32_t lse_first = 2 * C::kTileElems * 2 + (32 * query_sb + 4 * h) * 4, kv_at = C::kTileBytes + wave * 2 * WaveTile<D>::kRegionBytes + n * kFragPitch + 16 * h;
+  if constexpr (kSplit) asm volatile("" : "+v"(row_first), "+v"(tr_first), "+v"(lse_first), "+v"(kv_at));
   const int kw0 = key0 + 32 * wave;
   int tile = tile_first;     // query tile (within its head) of the trip being computed
   uint32_t buf_off = 0;      // byte offset of the LDS buffer being read
@@ -356,9 +361,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     const __bf16* sdO = sQ + C::kTileElems;
     const float* sL = reinterpret_cast<const float*>(sdO + C::kTileElems);
     const float* sDelta = sL + BM;
-    // (QS > 1) this lane's place in the tile of this trip: other pieces are reached by flipping bits of the address
-    const uint32_t row_lane = buf_off + row_place<D>(lane), tr_lane = buf_off + column_place<D>(lane);
-    static_assert(!kSplit || C::kBufBytes % 256 == 0);
+    // (QS > 1) this lane's places in the tile of this trip and its rows' lse and -delta
+    const uint32_t row_lane = buf_off + row_first, tr_lane = buf_off + tr_first, lse_lane = buf_off + lse_first;
 
     // The three phases of a 32-query sub-block.
     // products(): S = Q K^T and dP = dO V^T (C tile: lane = key, registers = queries); the dP accumulator starts at
@@ -366,7 +370,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     auto products = [&](int sb, f32x16& s_acc, f32x16& dp_acc) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDelta[32 * sb + 8 * j + 4 * h]);
+        const f32x4 d4 = kSplit ? lds_at<f32x4>(lse_lane + (BM + 8 * j) * 4) : *reinterpret_cast<const f32x4*>(&sDelta[32 * sb + 8 * j + 4 * h]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) { s_acc[4 * j + t] = 0.f; dp_acc[4 * j + t] = d4[t]; }
       }
@@ -377,10 +381,10 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         constexpr int kSteps = D / 16, kAhead = 2;
         bf16x8 qa[kSteps], da[kSteps], kb[kSteps], vb[kSteps];
         auto fetch = [&](int j) {
-          qa[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2);
-          if (j >= kKRegs) kb[j] = *reinterpret_cast<const bf16x8*>(split_k + n * kFragPitch + (16 * j + 8 * h) * 2);
-          da[j] = *reinterpret_cast<const bf16x8*>(smem_raw + (row_lane ^ 32 * j) + 32 * sb * D * 2 + C::kTileElems * 2);
-          vb[j] = *reinterpret_cast<const bf16x8*>(split_v + n * kFragPitch + (16 * j + 8 * h) * 2);
+          qa[j] = lds_at<bf16x8>(row_lane + 32 * j);
+          if (j >= kKRegs) kb[j] = lds_at<bf16x8>(kv_at + 32 * j);
+          da[j] = lds_at<bf16x8>(row_lane + (C::kTileElems * 2 + 32 * j));
+          vb[j] = lds_at<bf16x8>(kv_at + (WaveTile<D>::kRegionBytes + 32 * j));
         };
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) fetch(j);
@@ -410,7 +414,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       const int key_rel = kw0 + n - qs_pos - 4 * h;  // key is masked for row (8j + 4h + t) iff key_rel > 8j + t
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&sL[32 * sb + 8 * j + 4 * h]);
+        const f32x4 l4 = kSplit ? lds_at<f32x4>(lse_lane + 32 * j) : *reinterpret_cast<const f32x4*>(&sL[32 * sb + 8 * j + 4 * h]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int i = 4 * j + t;
@@ -432,10 +436,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         bf16x8 dof[kSlots], qf[kSlots];
         auto fetch = [&](int idx) {
           const int cc = idx / (D / 32), db = idx % (D / 32);
-          // rows 8 further down have their pieces at other places
-          const unsigned char *lo = smem_raw + (tr_lane ^ 64 * db) + (32 * sb + 16 * cc) * D * 2, *hi = smem_raw + (tr_lane ^ (64 * db + 32)) + (32 * sb + 16 * cc + 8) * D * 2;
-          dof[idx] = lds_read_tr_two(lo + C::kTileElems * 2, hi + C::kTileElems * 2);
-          qf[idx] = lds_read_tr_two(lo, hi);
+          dof[idx] = lds_tr_at<D>(tr_lane + (C::kTileElems * 2 + cc * L::kRows16 + db * 64));
+          qf[idx] = lds_tr_at<D>(tr_lane + (cc * L::kRows16 + db * 64));
         };
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) fetch(j);
@@ -721,13 +723,13 @@ struct DqCfg {
   static constexpr int kKT = KT;
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;
-  static constexpr int kTileElems = 2 * KT * D;   // K, then V
+  static constexpr int kSideBytes = TileLayout<D>::bytes(KT);   // a tile's K, or V; two of K, then two of V
   // workgroups that share a CU: the register budget and the plan go by it (at head_dim 128 a lane needs more than the 256
   // registers that two would leave it: with some in scratch 77 -> 121 us at one head of 3000 rows)
   static constexpr int kPerCu = NW <= 4 && D <= 64 ? 2 : 1;
   // the tiles, double-buffered; the Q / dO fragments pass through LDS behind them where there is room, so that the first tile is
   // requested at once, and through the tile buffers otherwise
-  static constexpr size_t kTiles = 2 * kTileElems * sizeof(__bf16), kFragmentBytes = NW * WaveTile<D>::kRegionBytes;
+  static constexpr size_t kTiles = 4 * kSideBytes, kFragmentBytes = NW * WaveTile<D>::kRegionBytes;
   static constexpr bool kBehind = kPerCu * (kTiles + kFragmentBytes) <= 160 * 1024;
   static constexpr size_t kFragments = kBehind ? kTiles : 0, kLdsBytes = kTiles + (kBehind ? kFragmentBytes : 0);
   static_assert(kFragmentBytes <= kLdsBytes);
@@ -757,6 +759,7 @@ __device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* regi
 template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) void attn_bwd_dq_kernel(const BwdParams p) {
   using C = DqCfg<D, NW, KT, KS>;
+  using L = TileLayout<D>;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
@@ -795,10 +798,9 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   uint32_t k_off[C::kLoads], v_off[C::kLoads];
 #pragma unroll
   for (int i = 0; i < C::kLoads; ++i) {
-    const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow ^ tile_twist<D>(r);
-    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
-    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
+    const int r = L::row(wave + NW * i, lane), cv = L::column(lane);
+    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv) * 2);
+    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv) * 2);
   }
   // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
   KvCursor<D> cur;
@@ -808,11 +810,11 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   // the next tile goes to LDS buffer `buf`
   auto request_tile = [&](int buf) {
     const u32x4 kb = request_window(reinterpret_cast<uint64_t>(cur.k), cur.k_left), vb = request_window(reinterpret_cast<uint64_t>(cur.v), cur.v_left);
-    const uint32_t to = static_cast<uint32_t>(buf) * (C::kTileElems * 2) + wave * 1024;
+    const uint32_t to = static_cast<uint32_t>(buf) * C::kSideBytes + wave * L::kPitch;
     each_load<C::kLoads>([&](auto load) {
       constexpr int i = decltype(load)::value;
-      request16_to<i * C::kThreads * 16>(to, kb, k_off[i]);
-      request16_to<KT * D * 2 + i * C::kThreads * 16>(to, vb, v_off[i]);
+      request16_to<i * NW * L::kPitch>(to, kb, k_off[i]);
+      request16_to<2 * C::kSideBytes + i * NW * L::kPitch>(to, vb, v_off[i]);
     });
     cur.next(a);
   };
@@ -877,20 +879,16 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
 
-  uint32_t row_at[D / 16], tr_at[D / 16];   // the lane's places in a tile (see the forward kernel)
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s) {
-    row_at[s] = row_place<D>(lane) ^ 32 * s;
-    tr_at[s] = column_place<D>(lane) ^ 32 * s;
-    asm volatile("" : "+v"(row_at[s]), "+v"(tr_at[s]));   // (kept, not computed again in front of every read)
-  }
+  // the lane's places in the K and V tiles
+  uint32_t row_at = L::row_place(lane), v_row_at = 2 * C::kSideBytes + L::row_place(lane), tr_at = L::column_place(lane);
+  asm volatile("" : "+v"(row_at), "+v"(v_row_at), "+v"(tr_at));   // (kept, not computed again in front of the reads)
 
   const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
   const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
   // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
   auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
-    constexpr uint32_t kAt = decltype(parity)::value * C::kTileElems * 2;
-    static_assert(kAt + C::kTileElems * 2 <= 65536, "offsets of LDS reads");
+    constexpr uint32_t kAt = decltype(parity)::value * C::kSideBytes;
+    static_assert(kAt + L::rows(KT - 32) + L::kRows16 + L::kRows8 + 2 * D <= 65535, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
     if (t + 1 < ntiles) request_tile(1 - decltype(parity)::value);
@@ -898,8 +896,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
       const int k0 = tile_key0 + sub * BN;
-      if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
-      if (a.causal && k0 > blk_q_lo + 31) continue;  // the wave's whole 32x64 block is in the future
+      if (kCut && KT > BN && k0 >= keys_end) break;
       f32x16 s_acc[BN / 32], dp_acc[BN / 32];
       // the compiler's scheduler is asked for its MFMA / LDS-read interleaving of this block (-1 to -5 %; the key-split
       // variant is better off without)
@@ -911,8 +908,8 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
         for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }
 #pragma unroll
         for (int s = 0; s < D / 16; ++s) {
-          const unsigned char* row = smem_raw + row_at[s] + (kAt + (sub * BN + 32 * mb) * D * 2);
-          const bf16x8 ka = *reinterpret_cast<const bf16x8*>(row), va = *reinterpret_cast<const bf16x8*>(row + KT * D * 2);
+          const uint32_t at = kAt + L::rows(sub * BN + 32 * mb) + s * 32;
+          const bf16x8 ka = lds_at<bf16x8>(row_at + at), va = lds_at<bf16x8>(v_row_at + at);
           s_acc[mb] = mfma32(ka, qf[s], s_acc[mb]);
           dp_acc[mb] = mfma32(va, dof[s], dp_acc[mb]);
         }
@@ -946,7 +943,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
           const bf16x8 dsf = pack8(dp_acc[mb], 8 * cc);
 #pragma unroll
           for (int db = 0; db < D / 32; ++db) {
-            const bf16x8 ktf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
+            const bf16x8 ktf = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * mb) + cc * L::kRows16 + db * 64));
             dq[db] = mfma32(ktf, dsf, dq[db]);
           }
         }
@@ -954,10 +951,20 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
     wait_requests<0>();
     __syncthreads();
   };
-  for (int t = 0; t < ntiles;) {
+  // the tiles that the wave's queries see come first; with the others it only helps (see the forward kernel)
+  const int see = (a.causal && blk_q_lo + 32 < kv_end ? blk_q_lo + 32 : kv_end) - BN * ks;
+  int mine = (see > 0 ? tiles_before(a.kv, see, KT) : 0) - t_first;
+  mine = mine < 0 ? 0 : mine < ntiles ? mine : ntiles;
+  int t = 0;
+  while (t < mine) {
     trip(std::integral_constant<int, 0>(), t++);
-    if (t >= ntiles) break;
+    if (t >= mine) break;
     trip(std::integral_constant<int, 1>(), t++);
+  }
+  for (; t < ntiles; ++t) {
+    if (t + 1 < ntiles) request_tile((t + 1) % 2);
+    wait_requests<0>();
+    __syncthreads();
   }
 
   // ---- key split: the partial sums of the waves ks > 0 are added to the wave ks == 0 of the same queries through LDS

@@ -43,15 +43,6 @@ __device__ __forceinline__ bf16x8 lds_read_tr_pair_step(const __bf16* p, int ste
   return __builtin_bit_cast(bf16x8, v);
 }
 
-// the same from two addresses
-__device__ __forceinline__ bf16x8 lds_read_tr_two(const unsigned char* a, const unsigned char* b) {
-  s16x4 lo = lds_read_tr(reinterpret_cast<const __bf16*>(a));
-  s16x4 hi = lds_read_tr(reinterpret_cast<const __bf16*>(b));
-  typedef __attribute__((ext_vector_type(8))) short s16x8;
-  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
-}
-
 // s_waitcnt immediate for "vmcnt(0)" with the other counters left at their maxima (gfx9 encoding:
 // vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
 constexpr int kWaitVmcnt0 = 0x0F70;
@@ -111,26 +102,52 @@ __device__ __forceinline__ u32x4 request_window(uint64_t base, uint32_t bytes) {
   return r;
 }
 
-// K, V, Q and dO tiles lie in LDS as dense rows of D elements (the direct loads write consecutive addresses), and the 16-byte pieces
-// of a row change places: piece p of row r lies at place p ^ tile_twist<D>(r).  Both kinds of read are then free of bank
-// conflicts: 16 consecutive rows put one piece at 16 different places of the 64 banks, and four consecutive rows put the four
-// pieces of 32 columns at 16 places.  Other pieces of a lane's row are reached by flipping bits 5 and up of its address, rows
-// a multiple of 16 further down by adding.
+// How K, V, Q and dO tiles lie in LDS, 64 rows at a time.  A request puts 1 KiB of consecutive addresses there, lane after lane, and
+// every lane can ask for any 16 bytes of the tile; the KiBs lie 16 bytes further apart than they are long.  Rows share a KiB such that
+// 16 consecutive ones start at 16 different places of the 64 banks, so reads by rows (16 lanes at a time: one piece of 16 rows) have no
+// bank conflicts, and rows 4 g .. 4 g + 3 a quarter of the banks apart, so transposing ones (32 lanes at a time: 4 rows x 64 bytes) have
+// none either.  And a lane's piece of any group of rows, any columns, lies at a constant distance from its first: one register per
+// kind of read holds all addresses.  Before, dense rows whose pieces changed places with the row: eight addresses per kind of read
+// at head_dim 128, kept in registers or flipped anew, and an addition in front of every read.  Forward at head_dim 128 221 -> 171
+// registers, 16 of 180 vector instructions per trip less: B1 H32 S4096 136.2 -> 133.3 us (D64 86.5 -> 84.3), its dK/dV 19 % fewer
+// of them and 257 -> 250 us (matrix work at the power limit: 4 % fewer cycles); small launches gain more, B3 H9/3 S777 D64 12.4 -> 10.7,
+// one rank's B1 H32 256 x 1024 13.3 -> 11.0.
+// (Counted conflicts say how LDS takes a read: 16 lanes of a 16-byte one at a time, 32 of an 8-byte one.  A layout that spread the
+// requests only over all 64 lanes doubled the pipe's cycles.)
 template <int D>
-__host__ __device__ constexpr int tile_twist(int r) {
-  return D == 128 ? (r & 3) << 2 | (r >> 2 & 3) : (r >> 1 & 1) << 2 | (r >> 2 & 3);
+struct TileLayout {
+  static constexpr int kBlocks = D / 8, kPitch = 1024 + 16;   // KiBs of 64 rows, and from one to the next
+  static constexpr int kRows64 = kBlocks * kPitch, kRows32 = 512, kRows16 = 256, kRows8 = 2 * kPitch;   // so many rows further
+  static constexpr int rows(int n) { return n / 64 * kRows64 + n % 64 / 32 * kRows32; }
+  static constexpr int bytes(int n) { return n / 64 * kRows64; }
+  // the row and first column of what lane `lane` of the request of KiB `block` brings
+  static __device__ __forceinline__ int row(int block, int lane) {
+    const int at = block % kBlocks, slot = lane / (D / 8), r = D == 128 ? 16 * slot : 16 * (slot / 2) + 2 * (slot % 2);
+    return block / kBlocks * 64 + at / 4 + 4 * (at % 4) + r;
+  }
+  static __device__ __forceinline__ int column(int lane) { return lane % (D / 8) * 8; }
+  static __device__ __forceinline__ uint32_t place(int r) {   // of a row, of the first 64
+    return D == 128 ? (r % 4 * 4 + r / 4 % 4) * kPitch + r / 16 * 256 : (r % 2 * 4 + r / 4 % 4) * kPitch + r / 16 * 256 + r % 4 / 2 * 128;
+  }
+  // the lane's place for reads by rows: row lane % 32, columns 8 (lane / 32) ..+7 (32 bytes further: the next 16 columns)
+  static __device__ __forceinline__ uint32_t row_place(int lane) { return place(lane % 32) + lane / 32 * 16; }
+  // ... and for transposing reads: row 4 (lane / 32) + lane % 16 / 4, columns 16 (lane / 16 % 2) + 4 (lane % 4) ..+3 (64 bytes further:
+  // the next 32 columns)
+  static __device__ __forceinline__ uint32_t column_place(int lane) { return place(4 * (lane / 32) + lane % 16 / 4) + lane / 16 % 2 * 32 + lane % 4 * 8; }
+};
+// LDS at a byte offset (the kernels' LDS starts at 0, see request16): through a pointer to the array the compiler adds its address,
+// which it does not know to be 0, to every lane offset
+template <typename T>
+__device__ __forceinline__ T lds_at(uint32_t off) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) T*>(off);
 }
-// the lane's place in a tile for reads by rows: piece h = lane / 32 of row lane % 32 (piece 2 s + h: ^ 32 s)
+// the 8 k-slots of an MFMA operand by two transposing reads: 4 rows at `off`, and 4 at 8 rows further
 template <int D>
-__device__ __forceinline__ uint32_t row_place(int lane) {
-  return lane % 32 * D * 2 + (lane / 32 ^ tile_twist<D>(lane % 32)) * 16;
-}
-// ... and for transposing reads: row 4 h + lane % 16 / 4, its columns 16 (lane / 16 % 2) + 4 (lane % 4) ..+3 (32 columns further: ^ 64;
-// 8 rows further down: ^ 32 besides the rows)
-template <int D>
-__device__ __forceinline__ uint32_t column_place(int lane) {
-  const int r = 4 * (lane / 32) + lane % 16 / 4;
-  return r * D * 2 + (tile_twist<D>(r) ^ (2 * (lane / 16 % 2) + lane % 4 / 2)) * 16 + lane % 2 * 8;
+__device__ __forceinline__ bf16x8 lds_tr_at(uint32_t off) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off + TileLayout<D>::kRows8));
+  typedef __attribute__((ext_vector_type(8))) short s16x8;
+  return __builtin_bit_cast(bf16x8, static_cast<s16x8>(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
 }
 
 // fn(integral_constant) for 0 .. N - 1

@@ -44,7 +44,7 @@ struct FwdCfg {
   static constexpr int kKDepth = D >= 128 ? 2 : 0;  // K fragments in flight from LDS ahead of the MFMA that uses them (0: compiler's order)
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;  // 16-byte loads per thread per tensor
-  static constexpr int kTileElems = 2 * KT * D;   // K, then V
+  static constexpr int kSideBytes = TileLayout<D>::bytes(KT);   // a tile's K, or V; two of K, then two of V
   // workgroups that share a CU: eight waves at head_dim 128 and with split keys have it to themselves.  The kernel's register
   // budget is this number's, and the plan counts on it.  (Left to the whole file, four waves at head_dim 128 took 290 and one
   // workgroup fitted: B1 H20 S3000 100 -> 68 us with the budget, 0.84 in the geometric mean of 93 drawn launches; at head_dim
@@ -52,7 +52,7 @@ struct FwdCfg {
   static constexpr int kPerCu = NW == 8 && (D >= 128 || KS > 1) ? 1 : 2;
   // the Q fragments pass through LDS behind the tile buffers where there is room, so that the first tile is requested at once, and
   // through the tile buffers otherwise
-  static constexpr size_t kTiles = 2 * kTileElems * sizeof(__bf16), kFragmentBytes = NW * QB * WaveTile<D>::kRegionBytes;
+  static constexpr size_t kTiles = 4 * kSideBytes, kFragmentBytes = NW * QB * WaveTile<D>::kRegionBytes;
   static constexpr bool kBehind = kPerCu * (kTiles + kFragmentBytes) <= 160 * 1024;
   static constexpr size_t kFragments = kBehind ? kTiles : 0, kLdsBytes = kTiles + (kBehind ? kFragmentBytes : 0);
   static_assert(NW * QB * kRowRegionBytes <= kLdsBytes, "the epilogue reuses the tile buffers");
@@ -95,6 +95,7 @@ __device__ __forceinline__ void fwd_epilogue(const FwdParams& p, unsigned char* 
 template <int D, int QB, int NW, int KT, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 4)) void attn_fwd_kernel(const FwdParams p) {
   using C = FwdCfg<D, QB, NW, KT, KS>;
+  using L = TileLayout<D>;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
@@ -136,15 +137,14 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
 
   // ---- staging of one K/V tile of KT keys: a wave-uniform window per tile (first key row, bytes left in the
   //      sequence) plus per-lane byte offsets that are computed once; rows past Sk read as zeros.  A lane asks for the
-  //      piece that belongs at its place of LDS (tile_twist).  The loop body holds no wait for memory other than the
+  //      piece that belongs at its place of LDS (TileLayout).  The loop body holds no wait for memory other than the
   //      one in front of the barrier that ends a trip, a whole tile after the requests.
   uint32_t k_off[C::kLoads], v_off[C::kLoads];
 #pragma unroll
   for (int i = 0; i < C::kLoads; ++i) {
-    const int idx = tid + i * C::kThreads;
-    const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow ^ tile_twist<D>(r);
-    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv * 8) * 2);
-    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv * 8) * 2);
+    const int r = L::row(wave + NW * i, lane), cv = L::column(lane);
+    k_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.ks[2] + cv) * 2);
+    v_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.vs[2] + cv) * 2);
   }
   // a cursor walks the key tiles in order (and from chunk to chunk): stepping it is a few scalar adds
   KvCursor<D> cur;
@@ -154,11 +154,11 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
   // the next tile goes to LDS buffer `buf`
   auto request_tile = [&](int buf) {
     const u32x4 kb = request_window(reinterpret_cast<uint64_t>(cur.k), cur.k_left), vb = request_window(reinterpret_cast<uint64_t>(cur.v), cur.v_left);
-    const uint32_t to = static_cast<uint32_t>(buf) * (C::kTileElems * 2) + wave * 1024;
+    const uint32_t to = static_cast<uint32_t>(buf) * C::kSideBytes + wave * L::kPitch;
     each_load<C::kLoads>([&](auto load) {
       constexpr int i = decltype(load)::value;
-      request16_to<i * C::kThreads * 16>(to, kb, k_off[i]);
-      request16_to<KT * D * 2 + i * C::kThreads * 16>(to, vb, v_off[i]);
+      request16_to<i * NW * L::kPitch>(to, kb, k_off[i]);
+      request16_to<2 * C::kSideBytes + i * NW * L::kPitch>(to, vb, v_off[i]);
     });
     cur.next(a);
   };
@@ -234,20 +234,13 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
 
-  // the lane's places in a tile (flipping bits of one address for every read takes the issue slots that the direct loads save:
-  // B1 H32 S4096 D128 147 -> 158 us that way)
-  uint32_t row_at[D / 16], tr_at[D / 16];
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s) {
-    row_at[s] = row_place<D>(lane) ^ 32 * s;
-    tr_at[s] = column_place<D>(lane) ^ 32 * s;
-    asm volatile("" : "+v"(row_at[s]), "+v"(tr_at[s]));   // (kept, not computed again in front of every read)
-  }
+  uint32_t row_at = L::row_place(lane), tr_at = 2 * C::kSideBytes + L::column_place(lane);   // the lane's places in the K and V tiles
+  asm volatile("" : "+v"(row_at), "+v"(tr_at));   // (kept, not computed again in front of the reads)
 
   // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
   auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
-    constexpr uint32_t kAt = decltype(parity)::value * C::kTileElems * 2;
-    static_assert(kAt + C::kTileElems * 2 <= 65536, "offsets of LDS reads");
+    constexpr uint32_t kAt = decltype(parity)::value * C::kSideBytes;
+    static_assert(kAt + L::rows(KT - 32) + L::kRows16 + L::kRows8 + 2 * D <= 65535, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
     // tile t+1 goes into the other buffer (its readers finished before the barrier that ended trip t-1)
@@ -257,11 +250,10 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
       const int k0 = tile_key0 + sub * BN;
-      if (k0 >= kv_end || (kCut && k0 >= keys_end)) break;
+      if (kCut && KT > BN && k0 >= keys_end) break;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
         const int blk_q_lo = a.q_offset + q0 + (qw * QB + qb) * 32;  // position of the block's first query
-        if (a.causal && k0 > blk_q_lo + 31) continue;                  // whole 32x64 block is in the future
         // ---- S^T[key][query] for 64 keys x 32 queries
         f32x16 s_acc[BN / 32];
         // Where no order is pinned by hand (head_dim 64), the compiler's scheduler is asked for its MFMA / LDS-read
@@ -276,7 +268,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
           bf16x8 kf[kSteps];
 #pragma unroll
           for (int j = 0; j < kSteps; ++j)
-            kf[j] = *reinterpret_cast<const bf16x8*>(smem_raw + row_at[j % (D / 16)] + (kAt + (sub * BN + 32 * (j / (D / 16))) * D * 2));
+            kf[j] = lds_at<bf16x8>(row_at + (kAt + L::rows(sub * BN + 32 * (j / (D / 16))) + j % (D / 16) * 32));
 #pragma unroll
           for (int mb = 0; mb < BN / 32; ++mb) {
 #pragma unroll
@@ -299,7 +291,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
             for (int i = 0; i < 16; ++i) s_acc[mb][i] = 0.f;
 #pragma unroll
             for (int s = 0; s < D / 16; ++s) {
-              const bf16x8 kf = *reinterpret_cast<const bf16x8*>(smem_raw + row_at[s] + (kAt + (sub * BN + 32 * mb) * D * 2));
+              const bf16x8 kf = lds_at<bf16x8>(row_at + (kAt + L::rows(sub * BN + 32 * mb) + s * 32));
               s_acc[mb] = mfma32(kf, qf[qb][s], s_acc[mb]);
             }
           }
@@ -357,7 +349,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
             const bf16x8 pf = pack8(s_acc[mb], 8 * cc);
 #pragma unroll
             for (int db = 0; db < D / 32; ++db) {
-              const bf16x8 vf = lds_read_tr_two(smem_raw + tr_at[2 * db] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc) * D * 2), smem_raw + tr_at[2 * db + 1] + (kAt + (KT + sub * BN + 32 * mb + 16 * cc + 8) * D * 2));
+              const bf16x8 vf = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * mb) + cc * L::kRows16 + db * 64));
               o[qb][db] = mfma32(vf, pf, o[qb][db]);
             }
           }
@@ -366,10 +358,22 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     wait_requests<0>();
     __syncthreads();  // all waves are done with buffer t&1 (it is refilled in trip t+1) and tile t+1 is visible
   };
-  for (int t = 0; t < ntiles;) {
+  // The tiles (its step of them) that the wave's queries see come first; with the others it only helps.  (A test inside the trip
+  // made the accumulators' registers depend on it, and the compiler copied all of them in some orders of the trip.)
+  static_assert(QB == 1);
+  const int see = (a.causal && a.q_offset + q0 + 32 * qw + 32 < kv_end ? a.q_offset + q0 + 32 * qw + 32 : kv_end) - BN * ks;
+  int mine = (see > 0 ? tiles_before(a.kv, see, KT) : 0) - t_first;
+  mine = mine < 0 ? 0 : mine < ntiles ? mine : ntiles;
+  int t = 0;
+  while (t < mine) {
     trip(std::integral_constant<int, 0>(), t++);
-    if (t >= ntiles) break;
+    if (t >= mine) break;
     trip(std::integral_constant<int, 1>(), t++);
+  }
+  for (; t < ntiles; ++t) {
+    if (t + 1 < ntiles) request_tile((t + 1) % 2);
+    wait_requests<0>();
+    __syncthreads();
   }
 
   // ---- key split: the waves ks > 0 hand their partial state to the wave ks == 0 of the same queries through LDS
