@@ -65,33 +65,23 @@ struct KvCfg {
   static constexpr int kThreads = 64 * NW;
   static constexpr int BN = 32 * kKeyWaves;  // keys per workgroup
   static constexpr int BM = QS > 2 ? 32 * QS : 64;   // queries per trip
-  // Q and dO tiles: rows of D elements at a pitch of LDQ elements, plus kSkew elements after every 4 rows.  Every
-  // tile is read both by rows (16 bytes per lane, 32 consecutive rows per instruction) and transposed (8 bytes per
-  // lane: 4 rows x 32 bytes per 16 lanes, rows 4 apart for the two wave halves).  An LDS instruction takes as many
-  // cycles as its busiest bank (64 banks of 4 bytes) has requests.  With the pitch = 16 (mod 32) words the 16-word
-  // pieces of 4 consecutive rows tile the banks (transposed reads at their minimum of 2 requests per bank; at a pitch
-  // of D + 8 they take 3-4), and the 4-word skew per 4 rows spreads 16 consecutive rows over all multiples of 4 words
-  // (row reads at their minimum of 4).
-  // QS > 1: the tiles are filled by loads that go to LDS directly and lie as TileLayout says.
-  // (The loop is paced by LDS reads and their latency, the matrix cores are busy for half of it: without the LDS writes and
-  // with more of K in registers B1 H32 S4096 281 -> 271 us, H32/8 S8192 1000 -> 950.  At head_dim 64 a wave's two sub-blocks take
-  // nearly all 256 registers.)
-  static constexpr int LDQ = kSplit ? D : D + 32;
-  static constexpr int kSkew = kSplit ? 0 : 8;
-  static constexpr int kTileElems = kSplit ? TileLayout<D>::bytes(BM) / 2 : BM * LDQ + kSkew * (BM / 4);       // one tile
-  static constexpr int kTrStep = 8 * LDQ + 2 * kSkew;                  // 8 rows further down
+  // Q and dO tiles are filled by loads that go to LDS directly and lie as TileLayout says.  (The loop is paced by LDS reads and their
+  // latency, the matrix cores are busy for half of it: without the LDS writes and with more of K in registers B1 H32 S4096 D128
+  // 281 -> 271 us, H32/8 S8192 1000 -> 950; at head_dim 64, which needs the constant distances of TileLayout for it, 244 -> 220 registers
+  // and, with dQ, B1 H32 S4096 252 -> 248.5, B8 H32/8 S512 83.8 -> 81, B3 H9/3 S777 41.3 -> 40.2.)
+  static constexpr int kTileElems = TileLayout<D>::bytes(BM) / 2;      // one tile
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kQLoads = BM * kVecPerRow / kThreads;
   static constexpr int kBufElems = 2 * kTileElems;                     // Q + dO tile of one stage (bf16)
   static constexpr size_t kBufBytes = kBufElems * sizeof(__bf16) + 2 * BM * sizeof(float);
   static constexpr size_t kTileBytes = 2 * kBufBytes;  // the two Q / dO tile buffers
-  // QS > 1: the K and V fragments of the key waves stay in LDS behind the tile buffers instead of in registers
-  static constexpr size_t kKvBytes = kSplit ? static_cast<size_t>(kKeyWaves) * 2 * WaveTile<D>::kRegionBytes : 0;
+  // the K and V fragments of the key waves pass through LDS behind the tile buffers, one after the other; QS > 1: both stay there
+  // instead of in registers
+  static constexpr size_t kKvBytes = static_cast<size_t>(kKeyWaves) * (kSplit ? 2 : 1) * WaveTile<D>::kRegionBytes;
   static constexpr size_t kLdsBytes = kTileBytes + kKvBytes;
   static constexpr int kPerCu = kSplit ? 1 : 2;         // workgroups that share a CU
   static_assert(kPerCu * kLdsBytes <= 160 * 1024, "the workgroups of a CU share its LDS");
   static_assert(NW * kRowRegionBytes <= kTileBytes, "the epilogue reuses the tile buffers");
-  static_assert(kSplit || NW * WaveTile<D>::kRegionBytes <= kBufBytes, "the K / V fragments pass through the second tile buffer");
   // QS > 1: one accumulator set (D/32 x 16 registers x 64 lanes of fp32) of every wave but the key waves' first passes through LDS at a time
   static constexpr size_t kExchangeBytes = static_cast<size_t>(D / 32) * 16 * 64 * 4;
   static_assert(!kSplit || (QS - 1) * kKeyWaves * kExchangeBytes <= kTileBytes, "the exchange reuses the tile buffers");
@@ -159,7 +149,6 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   constexpr bool kSplit = C::kSplit;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  auto tile_row = [](int r) { return r * C::LDQ + C::kSkew * (r >> 2); };   // element offset of a tile row
 
   const AttnParams& a = p.a;
   const int hkv = blockIdx.x % a.Hkv, b = blockIdx.x / a.Hkv;
@@ -169,7 +158,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   if (p.dk[chunk] == nullptr && p.dk_final[chunk] == nullptr) return;   // this chunk's gradient is not wanted (uniform over the workgroup)
   const int tid = threadIdx.x, wave_id = tid / 64, lane = tid % 64;
   // wave: which 32 keys of the tile; query_sb (QS > 1 only): which 32-query sub-block of every query tile
-  const int wave = kSplit ? __builtin_amdgcn_readfirstlane(wave_id % C::kKeyWaves) : wave_id;
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id % C::kKeyWaves);
   const int query_sb = kSplit ? __builtin_amdgcn_readfirstlane(wave_id / C::kKeyWaves) : 0;
   const int n = lane % 32, h = lane / 32;
   const float c = a.sm_scale * kLog2e;
@@ -178,8 +167,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   const __bf16* vbase = a.kv.v[chunk] + b * a.vs[0] + hkv * a.vs[1];
 
   // ---- K, V fragments of this wave's 32 keys (B operand: lane = key, 8 consecutive d per k step), fetched
-  //      row-major and turned into fragments through the wave's piece of the SECOND tile buffer, which nothing
-  //      else writes before the end of the first trip, a barrier later.  The loads are issued here; the first
+  //      row-major and turned into fragments through the wave's piece of LDS behind the tiles.  The loads are issued here; the first
   //      Q / dO tile's loads follow them further down before anything waits, so that the two latencies overlap.
   bf16x8 kf[D / 16], vf[D / 16];
   constexpr int kKRegs = kSplitKRegs < D / 16 ? kSplitKRegs : D / 16;
@@ -215,20 +203,18 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     tile_first += t0 - skip * tiles_per_head;
   }
 
-  // Loads of a Q / dO tile (+ lse, delta) into registers, QS > 1: of the tile straight to LDS.  A cursor (wave-uniform:
+  // Loads of a Q / dO tile straight to LDS, of its lse and delta through registers.  A cursor (wave-uniform:
   // it lives in scalar registers) walks the trip space; stepping to the next tile of the same head is a few
   // scalar adds, only a change of head recomputes addresses.  The per-lane byte offsets are computed once,
   // and rows past Sq read as zeros because they lie past the end of the buffer window.  Every instruction
   // of a wave costs an issue slot, scalar ones included, so the per-trip bookkeeping is kept this small.
-  u32x4 qreg[C::kQLoads], doreg[C::kQLoads];
   float lreg = 0.f, dreg = 0.f;
   uint32_t q_off[C::kQLoads], do_off[C::kQLoads];
 #pragma unroll
   for (int i = 0; i < C::kQLoads; ++i) {
-    const int idx = tid + i * C::kThreads;
-    const int r = kSplit ? L::row(wave_id + C::NW * i, lane) : idx / C::kVecPerRow, cv = kSplit ? L::column(lane) / 8 : idx % C::kVecPerRow;
-    q_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.qs[2] + cv * 8) * 2);
-    do_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.os[2] + cv * 8) * 2);
+    const int r = L::row(wave_id + C::NW * i, lane), cv = L::column(lane);
+    q_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.qs[2] + cv) * 2);
+    do_off[i] = static_cast<uint32_t>((static_cast<int64_t>(r) * a.os[2] + cv) * 2);
   }
   const uint32_t row_off = static_cast<uint32_t>((tid % BM) * 4);
   const uint32_t q_step = static_cast<uint32_t>(BM * a.qs[2] * 2), do_step = static_cast<uint32_t>(BM * a.os[2] * 2);
@@ -261,7 +247,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       cur.lse += BM;  cur.delta += BM;  cur.rows_left -= BM * 4;
     }
   };
-  // QS > 1: the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
+  // the tile under the cursor goes to the LDS buffer at buf_off (its lse and delta rows through registers, see stage)
   auto request_tile = [&](uint32_t buf_off) {
     const u32x4 qb = request_window(reinterpret_cast<uint64_t>(cur.q), cur.q_left), dob = request_window(reinterpret_cast<uint64_t>(cur.dout), cur.do_left);
     const uint32_t to = buf_off + __builtin_amdgcn_readfirstlane(wave_id) * L::kPitch;
@@ -274,32 +260,14 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       request16_to<C::kTileElems * 2 + i * C::NW * L::kPitch>(to, dob, do_off[i]);
     });
   };
-  auto prefetch = [&]() {  // the tile under the cursor
+  auto prefetch = [&]() {  // lse and delta of the tile under the cursor
     const buffer_rsrc lb = make_buffer(cur.lse, cur.rows_left), db = make_buffer(cur.delta, cur.rows_left);
-    if constexpr (!kSplit) {
-      const buffer_rsrc qb = make_buffer(cur.q, cur.q_left), dob = make_buffer(cur.dout, cur.do_left);
-#pragma unroll
-      for (int i = 0; i < C::kQLoads; ++i) {
-        qreg[i] = buffer_load_b128(qb, q_off[i]);
-        doreg[i] = buffer_load_b128(dob, do_off[i]);
-      }
-    }
     lreg = buffer_load_f32(lb, row_off);
     dreg = buffer_load_f32(db, row_off);
   };
-  auto stage = [&](int buf) {  // the prefetched tile (still under the cursor) goes to LDS buffer `buf`
-    __bf16* sQ = reinterpret_cast<__bf16*>(smem_raw + buf * C::kBufBytes);
-    __bf16* sdO = sQ + C::kTileElems;
-    float* sL = reinterpret_cast<float*>(sdO + C::kTileElems);
+  auto stage = [&](uint32_t buf_off) {  // ... (still under the cursor) go to the LDS buffer there
+    float* sL = reinterpret_cast<float*>(smem_raw + buf_off + 2 * C::kTileElems * sizeof(__bf16));
     float* sDelta = sL + BM;
-    if constexpr (!kSplit)
-#pragma unroll
-      for (int i = 0; i < C::kQLoads; ++i) {
-        const int idx = tid + i * C::kThreads;
-        const int r = idx / C::kVecPerRow, cv = idx % C::kVecPerRow;
-        *reinterpret_cast<u32x4*>(&sQ[tile_row(r) + cv * 8]) = qreg[i];
-        *reinterpret_cast<u32x4*>(&sdO[tile_row(r) + cv * 8]) = doreg[i];
-      }
     if (tid < BM) {
       // rows past Sq, and rows whose lse is -inf (they saw no key), get lse = +inf so that P = 0
       const bool live = static_cast<uint32_t>(tid) * 4u < cur.rows_left && lreg != -INFINITY;
@@ -311,11 +279,11 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
   if (n_iter > 0) {
     seek(head_first, tile_first);
     prefetch();
-    if constexpr (QS > 1) request_tile(0);
+    request_tile(0);
   }
   if (loads_kv) {
     if constexpr (!kSplit) {
-      unsigned char* region = smem_raw + C::kBufBytes + wave * WaveTile<D>::kRegionBytes;
+      unsigned char* region = smem_raw + C::kTileBytes + wave * WaveTile<D>::kRegionBytes;
       kt.fragments(region, lane, kf);
       vt.fragments(region, lane, vf);
     } else {
@@ -331,38 +299,37 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     for (int j = 0; j < kKRegs; ++j) kf[j] = *reinterpret_cast<const bf16x8*>(split_k + n * kFragPitch + (16 * j + 8 * h) * 2);
   }
   if (n_iter > 0) stage(0);
-  // All loads above are complete from here on (QS > 1: also the first tile, which the barrier publishes).  Saying so
+  // All loads above are complete from here on (also the first tile, which the barrier publishes).  Saying so
   // keeps the compiler from putting a vmcnt(0) wait in front of the loop's first MFMAs, where it would wait for the
   // NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
-  // (QS > 1) the lane's places in the wave's sub-block of a tile, and in its keys' K and V
+  // the lane's places in a tile (QS > 1: in the wave's sub-block of it), in its rows' lse and -delta, and (QS > 1) in its keys' K and V
   const int sub_block = query_sb / 2 * L::kRows64 + query_sb % 2 * L::kRows32;
   uint32_t row_first = sub_block + L::row_place(lane), tr_first = sub_block + L::column_place(lane);
   uint32_t lse_first = 2 * C::kTileElems * 2 + (32 * query_sb + 4 * h) * 4, kv_at = C::kTileBytes + wave * 2 * WaveTile<D>::kRegionBytes + n * kFragPitch + 16 * h;
-  if constexpr (kSplit) asm volatile("" : "+v"(row_first), "+v"(tr_first), "+v"(lse_first), "+v"(kv_at));
+  asm volatile("" : "+v"(row_first), "+v"(tr_first), "+v"(lse_first), "+v"(kv_at));   // (kept, not computed again)
   const int kw0 = key0 + 32 * wave;
   int tile = tile_first;     // query tile (within its head) of the trip being computed
   uint32_t buf_off = 0;      // byte offset of the LDS buffer being read
-  for (int it = 0; it < n_iter; ++it) {
-    // tile it+1 travels global -> registers while this trip computes; it goes to the other LDS buffer at
-    // the end of the trip (that buffer's readers finished before the barrier that ended trip it-1)
-    const bool has_next = it + 1 < n_iter;
-    // QS > 1: it goes there directly, and is requested at the top of the trip
-    if (has_next) advance();
-    if constexpr (QS > 1) {
-      if (has_next) {
-        prefetch();
-        request_tile(buf_off ^ static_cast<uint32_t>(C::kBufBytes));
-      }
+  // a trip; kOff: every pair of it is visible to this wave
+  auto trip = [&](auto off_c, const bool has_next) __attribute__((always_inline)) {
+    constexpr bool kOff = decltype(off_c)::value;
+    // the next tile travels to the other LDS buffer while this trip computes (that buffer's readers finished before the barrier that
+    // ended the last trip)
+    if (has_next) {
+      advance();
+      prefetch();
+      request_tile(buf_off ^ static_cast<uint32_t>(C::kBufBytes));
     }
     const int q0 = tile * BM;
-    const __bf16* sQ = reinterpret_cast<const __bf16*>(smem_raw + buf_off);
-    const __bf16* sdO = sQ + C::kTileElems;
-    const float* sL = reinterpret_cast<const float*>(sdO + C::kTileElems);
-    const float* sDelta = sL + BM;
-    // (QS > 1) this lane's places in the tile of this trip and its rows' lse and -delta
+    // this lane's places in the tile of this trip and its rows' lse and -delta
     const uint32_t row_lane = buf_off + row_first, tr_lane = buf_off + tr_first, lse_lane = buf_off + lse_first;
+    constexpr int kDo = C::kTileElems * 2;   // from Q's tile to dO's
+    // 32-query sub-block sb of the wave's (QS > 1: it has one, where its places point)
+    auto sub = [](int sb) { return kSplit ? 0 : sb * L::kRows32; };
+    auto lse_row = [&](int sb, int j) { return lds_at<f32x4>(lse_lane + (kSplit ? 32 * j : 32 * (4 * sb + j))); };
+    auto delta_row = [&](int sb, int j) { return lds_at<f32x4>(lse_lane + (BM * 4 + (kSplit ? 32 * j : 32 * (4 * sb + j)))); };
 
     // The three phases of a 32-query sub-block.
     // products(): S = Q K^T and dP = dO V^T (C tile: lane = key, registers = queries); the dP accumulator starts at
@@ -370,7 +337,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     auto products = [&](int sb, f32x16& s_acc, f32x16& dp_acc) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 d4 = kSplit ? lds_at<f32x4>(lse_lane + (BM + 8 * j) * 4) : *reinterpret_cast<const f32x4*>(&sDelta[32 * sb + 8 * j + 4 * h]);
+        const f32x4 d4 = delta_row(sb, j);
 #pragma unroll
         for (int t = 0; t < 4; ++t) { s_acc[4 * j + t] = 0.f; dp_acc[4 * j + t] = d4[t]; }
       }
@@ -383,7 +350,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         auto fetch = [&](int j) {
           qa[j] = lds_at<bf16x8>(row_lane + 32 * j);
           if (j >= kKRegs) kb[j] = lds_at<bf16x8>(kv_at + 32 * j);
-          da[j] = lds_at<bf16x8>(row_lane + (C::kTileElems * 2 + 32 * j));
+          da[j] = lds_at<bf16x8>(row_lane + (kDo + 32 * j));
           vb[j] = lds_at<bf16x8>(kv_at + (WaveTile<D>::kRegionBytes + 32 * j));
         };
 #pragma unroll
@@ -399,8 +366,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       } else {
 #pragma unroll
         for (int s = 0; s < D / 16; ++s) {
-          const bf16x8 qa = *reinterpret_cast<const bf16x8*>(&sQ[tile_row(32 * sb + n) + 16 * s + 8 * h]);
-          const bf16x8 da = *reinterpret_cast<const bf16x8*>(&sdO[tile_row(32 * sb + n) + 16 * s + 8 * h]);
+          const bf16x8 qa = lds_at<bf16x8>(row_lane + (sub(sb) + 32 * s)), da = lds_at<bf16x8>(row_lane + (kDo + sub(sb) + 32 * s));
           s_acc = mfma32(qa, kf[s], s_acc);
           dp_acc = mfma32(da, vf[s], dp_acc);
         }
@@ -414,7 +380,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       const int key_rel = kw0 + n - qs_pos - 4 * h;  // key is masked for row (8j + 4h + t) iff key_rel > 8j + t
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 l4 = kSplit ? lds_at<f32x4>(lse_lane + 32 * j) : *reinterpret_cast<const f32x4*>(&sL[32 * sb + 8 * j + 4 * h]);
+        const f32x4 l4 = lse_row(sb, j);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int i = 4 * j + t;
@@ -436,7 +402,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         bf16x8 dof[kSlots], qf[kSlots];
         auto fetch = [&](int idx) {
           const int cc = idx / (D / 32), db = idx % (D / 32);
-          dof[idx] = lds_tr_at<D>(tr_lane + (C::kTileElems * 2 + cc * L::kRows16 + db * 64));
+          dof[idx] = lds_tr_at<D>(tr_lane + (kDo + cc * L::kRows16 + db * 64));
           qf[idx] = lds_tr_at<D>(tr_lane + (cc * L::kRows16 + db * 64));
         };
 #pragma unroll
@@ -456,24 +422,20 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
-        // registers 8cc+4jj+t hold queries 32sb + 16cc + 8jj + 4h + t: fetch dO / Q rows in that order
+        // registers 8cc+4jj+t hold queries 32sb + 16cc + 8jj + 4h + t: dO / Q rows are fetched in that order
         const bf16x8 pf = pack8(s_acc, 8 * cc);
         const bf16x8 dsf = pack8(dp_acc, 8 * cc);
-        const int qr = 32 * sb + 16 * cc + 4 * h + (lane % 16) / 4;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db) {
-          const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
-          const bf16x8 dof = lds_read_tr_pair_step(&sdO[tile_row(qr) + col], C::kTrStep);
-          const bf16x8 qf = lds_read_tr_pair_step(&sQ[tile_row(qr) + col], C::kTrStep);
+          const uint32_t at = sub(sb) + cc * L::kRows16 + db * 64;
+          const bf16x8 dof = lds_tr_at<D>(tr_lane + (kDo + at)), qf = lds_tr_at<D>(tr_lane + at);
           dv_acc[db] = mfma32(dof, pf, dv_acc[db]);
           dk_acc[db] = mfma32(qf, dsf, dk_acc[db]);
         }
       }
     };
 
-    const bool off_diagonal = !kSplit && (!a.causal || kw0 + 31 <= a.q_offset + q0);
-    if (!kSplit && has_next && !off_diagonal) prefetch();
-    if (off_diagonal) {
+    if constexpr (kOff && !kSplit) {
       // Every pair of this trip is visible to this wave (all trips off the diagonal): straight-line code in an order
       // that lets the wave's own phases overlap -- the matrix pipe works on the second sub-block's S / dP while the
       // vector pipe does the first one's softmax, and on the first one's dV / dK during the second one's softmax.
@@ -506,29 +468,26 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
         // lse rows of sub-block 0 are fetched a slot ahead of the elements that need them (kPer elements per slot)
         constexpr int kPer = 16 / kPairs;
         f32x4 l4[4];
-        auto lse_row = [&](int r) {
-          l4[r] = *reinterpret_cast<const f32x4*>(&sL[8 * r + 4 * h]);
-        };
-        lse_row(0);
+        l4[0] = lse_row(0, 0);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDelta[32 + 8 * j + 4 * h]);
+          const f32x4 d4 = delta_row(1, j);
 #pragma unroll
           for (int t = 0; t < 4; ++t) { s1[4 * j + t] = 0.f; d1[4 * j + t] = d4[t]; }
         }
         bf16x8 qa[kPairs], da[kPairs];
         auto fetch = [&](int j) {
-          qa[j] = *reinterpret_cast<const bf16x8*>(&sQ[tile_row(32 + n) + 16 * j + 8 * h]);
-          da[j] = *reinterpret_cast<const bf16x8*>(&sdO[tile_row(32 + n) + 16 * j + 8 * h]);
+          qa[j] = lds_at<bf16x8>(row_lane + (sub(1) + 32 * j));
+          da[j] = lds_at<bf16x8>(row_lane + (kDo + sub(1) + 32 * j));
         };
-        constexpr int kAhead = D >= 128 ? 2 : 1;   // fragment pairs in flight ahead of their MFMAs
+        constexpr int kAhead = 1;   // fragment pairs in flight ahead of their MFMAs
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) fetch(j);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < kPairs; ++j) {
           if (j + kAhead < kPairs) fetch(j + kAhead);
-          if (((j + 1) * kPer) % 4 == 0 && (j + 1) * kPer < 16) lse_row((j + 1) * kPer / 4);
+          if (((j + 1) * kPer) % 4 == 0 && (j + 1) * kPer < 16) l4[(j + 1) * kPer / 4] = lse_row(0, (j + 1) * kPer / 4);
           s1 = mfma32(qa[j], kf[j], s1);
           d1 = mfma32(da[j], vf[j], d1);
           softmax_part(s0, d0, l4, j * kPer, kPer);
@@ -539,17 +498,13 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       {
         constexpr int kPer = 16 / kSlots;
         f32x4 l4[4];
-        auto lse_row = [&](int r) {
-          l4[r] = *reinterpret_cast<const f32x4*>(&sL[32 + 8 * r + 4 * h]);
-        };
-        lse_row(0);
+        l4[0] = lse_row(1, 0);
         bf16x8 dof[kSlots], qf[kSlots];
         auto fetch = [&](int idx) {
           const int cc = idx / (D / 32), db = idx % (D / 32);
-          const int qr = 16 * cc + 4 * h + (lane % 16) / 4;
-          const int col = 32 * db + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
-          dof[idx] = lds_read_tr_pair_step(&sdO[tile_row(qr) + col], C::kTrStep);
-          qf[idx] = lds_read_tr_pair_step(&sQ[tile_row(qr) + col], C::kTrStep);
+          const uint32_t at = cc * L::kRows16 + db * 64;
+          dof[idx] = lds_tr_at<D>(tr_lane + (kDo + at));
+          qf[idx] = lds_tr_at<D>(tr_lane + at);
         };
         fetch(0);
         bf16x8 pf = pack8(s0, 0), dsf = pack8(d0, 0);
@@ -561,34 +516,45 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
           dv_acc[db] = mfma32(dof[idx], pf, dv_acc[db]);
           dk_acc[db] = mfma32(qf[idx], dsf, dk_acc[db]);
           if (idx + 1 == D / 32) { pf = pack8(s0, 8); dsf = pack8(d0, 8); }
-          if (((idx + 1) * kPer) % 4 == 0 && (idx + 1) * kPer < 16) lse_row((idx + 1) * kPer / 4);
+          if (((idx + 1) * kPer) % 4 == 0 && (idx + 1) * kPer < 16) l4[(idx + 1) * kPer / 4] = lse_row(1, (idx + 1) * kPer / 4);
           softmax_part(s1, d1, l4, idx * kPer, kPer);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      // stage D: dV / dK of sub-block 1; the next tile's global loads are issued here, not at the top of the trip:
-      // their registers are free until now
+      // stage D: dV / dK of sub-block 1
       __builtin_amdgcn_s_setprio(0);
-      if (has_next) prefetch();
       accumulate(1, s1, d1);
     } else {
 #pragma unroll
       for (int sbi = 0; sbi < (kSplit ? 1 : BM / 32); ++sbi) {
         const int sb = kSplit ? query_sb : sbi;
         const int qs_pos = a.q_offset + q0 + 32 * sb;       // position of the sub-block's first query
-        if (a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
+        if (!kOff && a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
         f32x16 s_acc, dp_acc;
         products(sb, s_acc, dp_acc);
-        if (a.causal && kw0 + 31 > qs_pos) softmax_grad(sb, s_acc, dp_acc, std::true_type{});
+        if (!kOff && a.causal && kw0 + 31 > qs_pos) softmax_grad(sb, s_acc, dp_acc, std::true_type{});
         else softmax_grad(sb, s_acc, dp_acc, std::false_type{});
         accumulate(sb, s_acc, dp_acc);
       }
     }
     buf_off ^= static_cast<uint32_t>(C::kBufBytes);
-    if (has_next) stage(buf_off != 0);
-    if constexpr (QS > 1) wait_requests<0>();
+    if (has_next) stage(buf_off);
+    wait_requests<0>();
     tile = tile + 1 == n_qtiles ? qt_start : tile + 1;
     __syncthreads();  // all waves are done with the buffer just read (refilled in the next trip) and the next tile is visible
+  };
+  // of every head the tiles on the wave's diagonal come first: loops of their own, as a branch inside the trip had the compiler move
+  // the accumulators from registers to registers
+  const int seen = kw0 + 31 - a.q_offset - 32 * query_sb;
+  const int first_off = a.causal && seen > 0 ? (seen + BM - 1) / BM : 0;
+  // (QS 4 has few trips and is better off with less code: B2 H9/3 S256 backward 22.6 -> 22.9 us with two loops)
+  for (int it = 0; it < n_iter;) {
+    if constexpr (QS > 2) {
+      trip(std::false_type(), ++it < n_iter);
+      continue;
+    }
+    for (; it < n_iter && tile < first_off; ++it) trip(std::false_type(), it + 1 < n_iter);
+    for (; it < n_iter && tile >= first_off; ++it) trip(std::true_type(), it + 1 < n_iter);
   }
 
   // ---- epilogue (LDS is free now: the loop ended on a barrier)
