@@ -7,26 +7,68 @@
 //                  fp32 and every stored value is rounded once.
 #include "common.h"
 
+#include <type_traits>
+
 namespace pico {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPerThread = 8;  // elements: one 16-byte bf16 vector, two 16-byte fp32 vectors per state
+constexpr int kPerThread = 8;
 
-__device__ __forceinline__ void load8(const float* p, float (&out)[8]) {
-  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+// What bounds a step is HBM, and what it reaches depends on how its streams meet there (22 bytes per parameter unless said):
+//   * Every access of a wave is one run of consecutive bytes, 16 per lane of the widest type.  An fp32 array read as two 16-byte halves
+//     of 32 bytes per lane touches every line twice, which streaming accesses pay for: 63 M parameters 250 us, streamed 265; this way 222.
+//   * Weights and moments are streamed past the caches, loads and stores, where the arrays are larger than the Infinity Cache: nothing
+//     is there when the next step reads it.  Gradients are not: the last of them are still there behind a backward pass (63 M parameters,
+//     the same gradients again: 214 us, with streamed gradients 240).  Smaller steps find everything in the cache: arrays of 218 MB
+//     58.2 us, streamed 62.9; arrays of 285 MB 124, streamed 106.
+//   * The XCDs take 16 neighbouring blocks each instead of every eighth (block_of_workgroup).  How much the runs give hangs on where the arrays
+//     lie: ten steps of 150 to 600 M parameters took 0.97 of the time before with single blocks, 0.99 with runs of 8, 0.94 with 16 (0.91 to
+//     0.99), 0.97 with 12, 14, 20, 24 and 32, 0.95 with 128.  Where all arrays are bf16 there is nothing in runs (669 M: 1640 us, with
+//     runs of 16 to 64 1700 to 1800).
+//   Before and after, us: 669 M parameters 2677 -> 2475 (5.9 TB/s), fp32 weights (28 bytes) 3520 -> 3310, bf16 moments (14 bytes) 1717 -> 1640;
+//   63 M 257 -> 212 (6.5 TB/s), 335 -> 280, 169 -> 165; 24 M 123 -> 105.  (Threads of 16 elements, or 512 of them, are 2 to 3 % behind.)
+constexpr int64_t kCacheBytes = int64_t(256) << 20;
+
+// N consecutive elements (8 or 16 bytes) as floats
+template <bool kStream, int N, typename T>
+__device__ __forceinline__ void load_piece(const T* p, float (&out)[kPerThread], int at) {
+  if constexpr (sizeof(T) == 4) {
+    static_assert(N == 4);
+    const f32x4* from = reinterpret_cast<const f32x4*>(p);
+    const f32x4 raw = kStream ? __builtin_nontemporal_load(from) : *from;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { out[i] = a[i]; out[4 + i] = b[i]; }
-}
-__device__ __forceinline__ void store8(float* p, const float (&in)[8]) {
-  f32x4 a, b;
+    for (int i = 0; i < 4; ++i) out[at + i] = raw[i];
+  } else {
+    using Raw = std::conditional_t<N == 8, u32x4, u32x2>;
+    const Raw* from = reinterpret_cast<const Raw*>(p);
+    const Raw raw = kStream ? __builtin_nontemporal_load(from) : *from;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { a[i] = in[i]; b[i] = in[4 + i]; }
-  *reinterpret_cast<f32x4*>(p) = a;
-  *reinterpret_cast<f32x4*>(p + 4) = b;
+    for (int i = 0; i < N / 2; ++i) {
+      out[at + 2 * i] = __uint_as_float(raw[i] << 16);
+      out[at + 2 * i + 1] = __uint_as_float(raw[i] & 0xffff0000u);
+    }
+  }
 }
-__device__ __forceinline__ void load8(const __bf16* p, float (&out)[8]) { io<__bf16>::load(p, out); }
-__device__ __forceinline__ void store8(__bf16* p, const float (&in)[8]) { io<__bf16>::store(p, in); }
+template <bool kStream, int N, typename T>
+__device__ __forceinline__ void store_piece(T* p, const float (&in)[kPerThread], int at) {
+  auto put = [&](auto raw) {
+    if constexpr (kStream) __builtin_nontemporal_store(raw, reinterpret_cast<decltype(raw)*>(p));
+    else *reinterpret_cast<decltype(raw)*>(p) = raw;
+  };
+  if constexpr (sizeof(T) == 4) {
+    static_assert(N == 4);
+    f32x4 raw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = in[at + i];
+    put(raw);
+  } else {
+    std::conditional_t<N == 8, u32x4, u32x2> raw;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) raw[i] = pack_bf16x2(in[at + 2 * i], in[at + 2 * i + 1]);
+    put(raw);
+  }
+}
 
 // The arithmetic follows torch.optim.AdamW's (non-amsgrad) order of operations so that fp32 states match it to
 // rounding: p *= 1 - lr*wd;  m = m + (g - m)*(1 - b1);  v = v*b2 + g*g*(1 - b2);
@@ -37,25 +79,46 @@ struct Hyper {
   float decay, one_minus_b1, b2, one_minus_b2, step_size, inv_sqrt_bc2, eps, grad_scale;
 };
 
+// elements of one access: 16 bytes of the widest type
 template <typename TW, typename TM, typename TG>
+constexpr int kPiece = sizeof(TW) == 2 && sizeof(TM) == 2 && sizeof(TG) == 2 ? 8 : 4;
+
+// The block of a workgroup: neighbouring workgroups run on different XCDs (they go round all eight), and each XCD takes kRun blocks in
+// a row.  What does not fill a round of runs is dealt block by block.
+template <int N>
+__device__ __forceinline__ unsigned block_of_workgroup(unsigned workgroup, unsigned count) {
+  constexpr unsigned kRun = N == 8 ? 1 : 16, kXcds = 8, kRound = kXcds * kRun;
+  const unsigned round = workgroup / kRound, in = workgroup % kRound;
+  return (round + 1) * kRound <= count ? round * kRound + in % kXcds * kRun + in / kXcds : workgroup;
+}
+
+template <bool kStream, typename TW, typename TM, typename TG>
 __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* __restrict__ master,
                                             const TG* __restrict__ grad, TM* __restrict__ exp_avg,
                                             TM* __restrict__ exp_avg_sq, int64_t n, int64_t block, const Hyper& h) {
-  const int64_t i0 = (block * kThreads + threadIdx.x) * kPerThread;
+  constexpr int N = kPiece<TW, TM, TG>, kPieces = kPerThread / N;
+  const int64_t i0 = block * (kThreads * kPerThread) + threadIdx.x * N;
   if (i0 >= n) return;
+  auto at = [&](int j) { return i0 + j * (kThreads * N); };
   float g[kPerThread], p[kPerThread], m[kPerThread], v[kPerThread];
-  if (i0 + kPerThread <= n) {
-    load8(grad + i0, g);
-    load8(master + i0, p);
-    load8(exp_avg + i0, m);
-    load8(exp_avg_sq + i0, v);
+  const bool whole = at(kPieces - 1) + N <= n;
+  if (whole) {
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) {
+      load_piece<false, N>(grad + at(j), g, j * N);
+      load_piece<kStream, N>(master + at(j), p, j * N);
+      load_piece<kStream, N>(exp_avg + at(j), m, j * N);
+      load_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
+    }
   } else {
+#pragma unroll
     for (int e = 0; e < kPerThread; ++e) {
-      const bool in = i0 + e < n;
-      g[e] = in ? static_cast<float>(grad[i0 + e]) : 0.f;
-      p[e] = in ? static_cast<float>(master[i0 + e]) : 0.f;
-      m[e] = in ? static_cast<float>(exp_avg[i0 + e]) : 0.f;
-      v[e] = in ? static_cast<float>(exp_avg_sq[i0 + e]) : 0.f;
+      const int64_t i = at(e / N) + e % N;
+      const bool in = i < n;
+      g[e] = in ? static_cast<float>(grad[i]) : 0.f;
+      p[e] = in ? static_cast<float>(master[i]) : 0.f;
+      m[e] = in ? static_cast<float>(exp_avg[i]) : 0.f;
+      v[e] = in ? static_cast<float>(exp_avg_sq[i]) : 0.f;
     }
   }
 #pragma unroll
@@ -67,26 +130,32 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
     const float denom = __builtin_sqrtf(v[e]) * h.inv_sqrt_bc2 + h.eps;
     p[e] = p[e] - h.step_size * (m[e] / denom);
   }
-  if (i0 + kPerThread <= n) {
-    store8(master + i0, p);
-    store8(exp_avg + i0, m);
-    store8(exp_avg_sq + i0, v);
-    if (param_lp) io<__bf16>::store(param_lp + i0, p);
+  if (whole) {
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) {
+      store_piece<kStream, N>(master + at(j), p, j * N);
+      store_piece<kStream, N>(exp_avg + at(j), m, j * N);
+      store_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
+      if (param_lp) store_piece<kStream, N>(param_lp + at(j), p, j * N);
+    }
   } else {
-    for (int e = 0; e < kPerThread && i0 + e < n; ++e) {
-      master[i0 + e] = static_cast<TW>(p[e]);
-      exp_avg[i0 + e] = static_cast<TM>(m[e]);
-      exp_avg_sq[i0 + e] = static_cast<TM>(v[e]);
-      if (param_lp) param_lp[i0 + e] = static_cast<__bf16>(p[e]);
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e) {
+      const int64_t i = at(e / N) + e % N;
+      if (i >= n) continue;
+      master[i] = static_cast<TW>(p[e]);
+      exp_avg[i] = static_cast<TM>(m[e]);
+      exp_avg_sq[i] = static_cast<TM>(v[e]);
+      if (param_lp) param_lp[i] = static_cast<__bf16>(p[e]);
     }
   }
 }
 
-template <typename TW, typename TM, typename TG>
+template <bool kStream, typename TW, typename TM, typename TG>
 __global__ __launch_bounds__(kThreads) void adamw_kernel(__bf16* __restrict__ param_lp, TW* __restrict__ master,
                                                          const TG* __restrict__ grad, TM* __restrict__ exp_avg,
                                                          TM* __restrict__ exp_avg_sq, int64_t n, Hyper h) {
-  adamw_block<TW, TM, TG>(param_lp, master, grad, exp_avg, exp_avg_sq, n, blockIdx.x, h);
+  adamw_block<kStream, TW, TM, TG>(param_lp, master, grad, exp_avg, exp_avg_sq, n, block_of_workgroup<kPiece<TW, TM, TG>>(blockIdx.x, gridDim.x), h);
 }
 
 // Many tensors in one launch: the pointers travel in the kernel arguments (no table in device memory to keep alive),
@@ -103,15 +172,15 @@ struct TensorTable {
   int count;
 };
 
-template <typename TW, typename TM, typename TG>
+template <bool kStream, typename TW, typename TM, typename TG>
 __global__ __launch_bounds__(kThreads) void adamw_multi_kernel(TensorTable t, Hyper h) {
-  const unsigned bid = blockIdx.x;
+  const unsigned bid = block_of_workgroup<kPiece<TW, TM, TG>>(blockIdx.x, gridDim.x);
   int lo = 0, hi = t.count;   // block_start[lo] <= bid < block_start[hi]
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (bid >= t.block_start[mid]) lo = mid; else hi = mid;
   }
-  adamw_block<TW, TM, TG>(static_cast<__bf16*>(t.param_lp[lo]), static_cast<TW*>(t.weight[lo]),
+  adamw_block<kStream, TW, TM, TG>(static_cast<__bf16*>(t.param_lp[lo]), static_cast<TW*>(t.weight[lo]),
                           static_cast<const TG*>(t.grad[lo]), static_cast<TM*>(t.exp_avg[lo]),
                           static_cast<TM*>(t.exp_avg_sq[lo]), t.n[lo], bid - t.block_start[lo], h);
 }
@@ -149,6 +218,21 @@ Hyper make_hyper(float lr, float beta1, float beta2, float eps, float weight_dec
 constexpr int64_t kPerBlock = static_cast<int64_t>(kThreads) * kPerThread;
 
 template <typename TW, typename TM>
+int64_t state_bytes(int grad_dtype, bool copy) {   // per parameter, each array once
+  return static_cast<int64_t>(sizeof(TW) + 2 * sizeof(TM)) + (grad_dtype == PICO_BF16 ? 2 : 4) + (copy ? 2 : 0);
+}
+bool streams(int64_t bytes) { return bytes > kCacheBytes; }
+template <typename Fn>
+void with_kernel_types(int grad_dtype, bool stream, const Fn& fn) {
+  auto by_grad = [&](auto stream_it) {
+    if (grad_dtype == PICO_BF16) fn(stream_it, __bf16());
+    else fn(stream_it, float());
+  };
+  if (stream) by_grad(std::true_type());
+  else by_grad(std::false_type());
+}
+
+template <typename TW, typename TM>
 int adamw_launch(const char* who, void* param_lp, TW* master, const void* grad, int grad_dtype, TM* exp_avg,
                  TM* exp_avg_sq, int64_t n, float lr, float beta1, float beta2, float eps, float weight_decay,
                  int64_t step, float grad_scale, void* stream) {
@@ -162,12 +246,11 @@ int adamw_launch(const char* who, void* param_lp, TW* master, const void* grad, 
   const Hyper h = make_hyper(lr, beta1, beta2, eps, weight_decay, step, grad_scale);
   const unsigned grid = static_cast<unsigned>((n + kPerBlock - 1) / kPerBlock);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (grad_dtype == PICO_BF16)
-    hipLaunchKernelGGL((adamw_kernel<TW, TM, __bf16>), dim3(grid), dim3(kThreads), 0, s, static_cast<__bf16*>(param_lp),
-                       master, static_cast<const __bf16*>(grad), exp_avg, exp_avg_sq, n, h);
-  else
-    hipLaunchKernelGGL((adamw_kernel<TW, TM, float>), dim3(grid), dim3(kThreads), 0, s, static_cast<__bf16*>(param_lp),
-                       master, static_cast<const float*>(grad), exp_avg, exp_avg_sq, n, h);
+  with_kernel_types(grad_dtype, streams(n * state_bytes<TW, TM>(grad_dtype, param_lp != nullptr)), [&](auto stream_it, auto grad_type) {
+    using TG = decltype(grad_type);
+    hipLaunchKernelGGL((adamw_kernel<decltype(stream_it)::value, TW, TM, TG>), dim3(grid), dim3(kThreads), 0, s, static_cast<__bf16*>(param_lp),
+                       master, static_cast<const TG*>(grad), exp_avg, exp_avg_sq, n, h);
+  });
   return check_launch(who);
 }
 
@@ -188,16 +271,18 @@ int adamw_multi_launch(int count, void* const* weights, void* const* param_lps, 
     if ((sizes[i] + kPerBlock - 1) / kPerBlock > 0x7fffffff)
       return fail(PICO_ERR_SHAPE, "%s: tensor %d is too large for one launch", who, i);
   }
+  int64_t elements = 0;
+  for (int i = 0; i < count; ++i) elements += sizes[i];
+  const bool stream_all = streams(elements * state_bytes<TW, TM>(grad_dtype, param_lps != nullptr));
   TensorTable t;
   t.count = 0;
   t.block_start[0] = 0;
   auto flush = [&]() -> int {
     if (t.count == 0) return PICO_OK;
     const unsigned grid = t.block_start[t.count];
-    if (grad_dtype == PICO_BF16)
-      hipLaunchKernelGGL((adamw_multi_kernel<TW, TM, __bf16>), dim3(grid), dim3(kThreads), 0, s, t, h);
-    else
-      hipLaunchKernelGGL((adamw_multi_kernel<TW, TM, float>), dim3(grid), dim3(kThreads), 0, s, t, h);
+    with_kernel_types(grad_dtype, stream_all, [&](auto stream_it, auto grad_type) {
+      hipLaunchKernelGGL((adamw_multi_kernel<decltype(stream_it)::value, TW, TM, decltype(grad_type)>), dim3(grid), dim3(kThreads), 0, s, t, h);
+    });
     t.count = 0;
     return check_launch(who);
   };
