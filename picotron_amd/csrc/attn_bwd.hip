@@ -53,8 +53,8 @@ constexpr bool kStreamGrads = true;
 //     lets the head_dim 128 kernel fit 256 registers, i.e. two waves per SIMD.
 //   QS 4: for launches that leave most CUs idle, whose time is that of one workgroup's chain of trips: twice the workgroups
 //     (64 keys each), and a trip takes 128 queries in the time of 32.
-// QS > 1: K fragments (of D / 16) that stay in registers; the others are read from LDS.  As many as fit: 4 -> 7 with the registers
-// that staging the tiles took, 3 % at B1 H32 S4096.
+// QS > 1: K fragments (of D / 16) that stay in registers; the others are read from LDS.  As many as fit (two of V beside them do not):
+// 4 -> 7 with the registers that staging the tiles took, 3 % at B1 H32 S4096.
 constexpr int kSplitKRegs = 7;
 
 template <int D, int QS>
@@ -341,35 +341,11 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
         for (int t = 0; t < 4; ++t) { s_acc[4 * j + t] = 0.f; dp_acc[4 * j + t] = d4[t]; }
       }
-      if constexpr (QS > 1) {
-        // both operands of every MFMA come from LDS: they are requested kAhead steps before the MFMAs that use them, and
-        // the scheduling barriers keep that order (left alone, the compiler reuses one set of registers and every MFMA
-        // waits for an LDS round trip)
-        constexpr int kSteps = D / 16, kAhead = 2;
-        bf16x8 qa[kSteps], da[kSteps], kb[kSteps], vb[kSteps];
-        auto fetch = [&](int j) {
-          qa[j] = lds_at<bf16x8>(row_lane + 32 * j);
-          if (j >= kKRegs) kb[j] = lds_at<bf16x8>(kv_at + 32 * j);
-          da[j] = lds_at<bf16x8>(row_lane + (kDo + 32 * j));
-          vb[j] = lds_at<bf16x8>(kv_at + (WaveTile<D>::kRegionBytes + 32 * j));
-        };
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) fetch(j);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < kSteps; ++j) {
-          if (j + kAhead < kSteps) fetch(j + kAhead);
-          s_acc = mfma32(qa[j], j < kKRegs ? kf[j] : kb[j], s_acc);
-          dp_acc = mfma32(da[j], vb[j], dp_acc);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < D / 16; ++s) {
-          const bf16x8 qa = lds_at<bf16x8>(row_lane + (sub(sb) + 32 * s)), da = lds_at<bf16x8>(row_lane + (kDo + sub(sb) + 32 * s));
-          s_acc = mfma32(qa, kf[s], s_acc);
-          dp_acc = mfma32(da, vf[s], dp_acc);
-        }
+      for (int s = 0; s < D / 16; ++s) {
+        const bf16x8 qa = lds_at<bf16x8>(row_lane + (sub(sb) + 32 * s)), da = lds_at<bf16x8>(row_lane + (kDo + sub(sb) + 32 * s));
+        s_acc = mfma32(qa, kf[s], s_acc);
+        dp_acc = mfma32(da, vf[s], dp_acc);
       }
     };
     // softmax_grad(): P = exp2(S*c - lse*log2e), dS = P * (dP - delta) [already in the accumulator]; the mask test
@@ -397,29 +373,6 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // d, which is what lets the epilogue write whole 16-byte pieces of a row); P / dS come from the registers,
     // dO^T / Q^T from the row-major LDS tiles through transposing reads.
     auto accumulate = [&](int sb, const f32x16& s_acc, const f32x16& dp_acc) {
-      if constexpr (QS > 1) {
-        constexpr int kSlots = 2 * (D / 32), kAhead = 2;
-        bf16x8 dof[kSlots], qf[kSlots];
-        auto fetch = [&](int idx) {
-          const int cc = idx / (D / 32), db = idx % (D / 32);
-          dof[idx] = lds_tr_at<D>(tr_lane + (kDo + cc * L::kRows16 + db * 64));
-          qf[idx] = lds_tr_at<D>(tr_lane + (cc * L::kRows16 + db * 64));
-        };
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) fetch(j);
-        bf16x8 pf = pack8(s_acc, 0), dsf = pack8(dp_acc, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int idx = 0; idx < kSlots; ++idx) {
-          const int db = idx % (D / 32);
-          if (idx + kAhead < kSlots) fetch(idx + kAhead);
-          dv_acc[db] = mfma32(dof[idx], pf, dv_acc[db]);
-          dk_acc[db] = mfma32(qf[idx], dsf, dk_acc[db]);
-          if (idx + 1 == D / 32) { pf = pack8(s_acc, 8); dsf = pack8(dp_acc, 8); }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        return;
-      }
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
         // registers 8cc+4jj+t hold queries 32sb + 16cc + 8jj + 4h + t: dO / Q rows are fetched in that order
@@ -435,7 +388,80 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
     };
 
-    if constexpr (kOff && !kSplit) {
+    // The same for the one sub-block of a wave with QS > 1, product after product: exp2 and P need S alone and are dealt out between
+    // the MFMAs of dP, dS between those of dV, so that the vector pipe works in the shadow of every product but S and dK.  Both operands come from
+    // LDS: they are requested kAhead MFMAs before the one that uses them, across the products, and the scheduling barriers keep
+    // that order (left alone, the compiler reuses one set of registers and every MFMA waits for an LDS round trip).  Forward and backward of a
+    // ring of 8 x 4096 rows, 32 / 8 heads of 128, 33.19 -> 32.89 ms, B1 H32 S2048 D128 125.0 -> 124.0 us (nearly all of a wave's vector work
+    // is hidden already by the other wave of its SIMD; LDS reads and power remain).
+    auto one_block = [&](auto mask_c) __attribute__((always_inline)) {
+      constexpr bool kMask = decltype(mask_c)::value;
+      constexpr int kSteps = D / 16, kPer = 16 / kSteps, kAhead = D == 64 ? 3 : 2, kAll = 4 * kSteps;   // (2 * (D / 32) MFMAs of dV and of dK, as many as of S and of dP)
+      // (key is masked for row (8j + 4h + t) iff key_rel > 8j + t)
+      const int key_rel = a.causal ? kw0 + n - (a.q_offset + q0 + 32 * query_sb) - 4 * h : -1;
+      f32x16 s_acc, dp_acc;
+      f32x4 l4[4];
+      bf16x8 left[kAll], right[2 * kSteps], pf[2], dsf[2];
+      auto fetch = [&](int i) {
+        const int j = i % kSteps;
+        if (i < kSteps) {
+          left[i] = lds_at<bf16x8>(row_lane + 32 * j);
+          if (j >= kKRegs) right[i] = lds_at<bf16x8>(kv_at + 32 * j);
+        } else if (i < 2 * kSteps) {
+          left[i] = lds_at<bf16x8>(row_lane + (kDo + 32 * j));
+          right[i] = lds_at<bf16x8>(kv_at + (WaveTile<D>::kRegionBytes + 32 * j));
+        } else {
+          left[i] = lds_tr_at<D>(tr_lane + ((i < 3 * kSteps ? kDo : 0) + j / (D / 32) * L::kRows16 + j % (D / 32) * 64));
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s_acc[i] = 0.f;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) fetch(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kAll; ++i) {
+        const int j = i % kSteps;
+        if (i + kAhead < kAll) fetch(i + kAhead);
+        const int rows = i - 3 * kSteps / 4;   // lse of the rows whose exp2 is kSteps / 4 MFMAs away
+        if (rows >= 0 && rows < kSteps && rows % (kSteps / 4) == 0) l4[rows * 4 / kSteps] = lse_row(query_sb, rows * 4 / kSteps);
+        if (i < kSteps) {
+          s_acc = mfma32(left[i], j < kKRegs ? kf[j] : right[i], s_acc);
+          if (2 * j >= kSteps) {   // dP starts at -delta of its rows
+#pragma unroll
+            for (int r = (2 * j - kSteps) * 4 / kSteps; r < (2 * j + 2 - kSteps) * 4 / kSteps; ++r) {
+              const f32x4 d4 = delta_row(query_sb, r);
+#pragma unroll
+              for (int t = 0; t < 4; ++t) dp_acc[4 * r + t] = d4[t];
+            }
+          }
+        } else if (i < 2 * kSteps) {
+          dp_acc = mfma32(left[i], right[i], dp_acc);
+#pragma unroll
+          for (int e = j * kPer; e < (j + 1) * kPer; ++e) {
+            s_acc[e] = fast_exp2(s_acc[e] * c - l4[e / 4][e % 4]);
+            if (kMask && key_rel > 8 * (e / 4) + e % 4) s_acc[e] = 0.f;
+          }
+          if (2 * (j + 1) == kSteps) pf[0] = pack8(s_acc, 0);
+          if (j + 1 == kSteps) pf[1] = pack8(s_acc, 8);
+        } else if (i < 3 * kSteps) {
+          dv_acc[j % (D / 32)] = mfma32(left[i], pf[j / (D / 32)], dv_acc[j % (D / 32)]);
+#pragma unroll
+          for (int e = j * kPer; e < (j + 1) * kPer; ++e) dp_acc[e] = s_acc[e] * dp_acc[e];
+          if (2 * (j + 1) == kSteps) dsf[0] = pack8(dp_acc, 0);
+          if (j + 1 == kSteps) dsf[1] = pack8(dp_acc, 8);
+        } else {
+          dk_acc[j % (D / 32)] = mfma32(left[i], dsf[j / (D / 32)], dk_acc[j % (D / 32)]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+
+    if constexpr (kSplit) {
+      const int qs_pos = a.q_offset + q0 + 32 * query_sb;   // position of the sub-block's first query
+      if constexpr (kOff) one_block(std::false_type());
+      else if (!a.causal || kw0 <= qs_pos + 31) one_block(std::true_type());   // (else every pair is masked; the mask changes nothing off the diagonal)
+    } else if constexpr (kOff) {
       // Every pair of this trip is visible to this wave (all trips off the diagonal): straight-line code in an order
       // that lets the wave's own phases overlap -- the matrix pipe works on the second sub-block's S / dP while the
       // vector pipe does the first one's softmax, and on the first one's dV / dK during the second one's softmax.
@@ -526,13 +552,12 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       accumulate(1, s1, d1);
     } else {
 #pragma unroll
-      for (int sbi = 0; sbi < (kSplit ? 1 : BM / 32); ++sbi) {
-        const int sb = kSplit ? query_sb : sbi;
+      for (int sb = 0; sb < BM / 32; ++sb) {
         const int qs_pos = a.q_offset + q0 + 32 * sb;       // position of the sub-block's first query
-        if (!kOff && a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
+        if (a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
         f32x16 s_acc, dp_acc;
         products(sb, s_acc, dp_acc);
-        if (!kOff && a.causal && kw0 + 31 > qs_pos) softmax_grad(sb, s_acc, dp_acc, std::true_type{});
+        if (a.causal && kw0 + 31 > qs_pos) softmax_grad(sb, s_acc, dp_acc, std::true_type{});
         else softmax_grad(sb, s_acc, dp_acc, std::false_type{});
         accumulate(sb, s_acc, dp_acc);
       }

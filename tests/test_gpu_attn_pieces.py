@@ -120,3 +120,25 @@ def test_ragged_chunk_lists(device, B, Hq, Hkv, W, Sc, D, causal):
                                                             (1, 3, 1, 127, 64, False, 0), (4, 32, 32, 96, 96, True, 0)])
 def test_short_chains(device, B, Hq, Hkv, Sq, Sk, causal, q_offset):
     test_attention_in_pieces(device, B, Hq, Hkv, Sq, Sk, 64, causal, q_offset, (False, False))
+
+
+# the backward kernels' orders of work: masked and unmasked trips, offsets of the diagonal that are no multiple of a tile, no mask at all
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,q_offset", [
+    (2, 9, 3, 256, 256, 64, False, 0),       # few workgroups, every key visible
+    (1, 4, 4, 97, 161, 64, True, 31),        # few workgroups, queries behind the keys' start
+    (1, 4, 4, 130, 700, 64, True, 570),      # split keys: all tiles but the last unmasked
+    (2, 6, 2, 333, 333, 64, True, 0),
+    (1, 4, 2, 200, 641, 128, True, 441),
+    (1, 4, 2, 289, 400, 128, True, 111),     # diagonal through tiles, keys that end inside one
+    (1, 2, 2, 500, 300, 128, True, 0),       # queries past all keys
+    (1, 3, 3, 65, 193, 128, False, 0),
+])
+def test_backward_masked_and_unmasked_trips(device, B, Hq, Hkv, Sq, Sk, D, causal, q_offset):
+    from picotron_amd import ops
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, Sk, D)
+    scale = 1 / math.sqrt(D)
+    want = reference(q, k, v, scale, q_offset, causal, do)
+    out, lse = ops.attn_fwd(q, k, v, scale, causal, q_offset)
+    dq, dk, dv = (torch.empty_like(t) for t in (q, k, v))
+    ops.attn_bwd(do, q, k, v, lse, None, scale, causal, q_offset, dq=dq, dk=dk, dv=dv, out=out)
+    check((out, lse, dq, dk, dv), want, "bf16 results")   # (bf16 operands and probabilities: the bounds of the tests above)
