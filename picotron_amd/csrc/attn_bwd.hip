@@ -877,12 +877,58 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
   const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
   // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
-  auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
+  auto trip = [&](auto parity, auto plain_c, int t) __attribute__((always_inline)) {
     constexpr uint32_t kAt = decltype(parity)::value * C::kSideBytes;
+    constexpr bool kPlain = decltype(plain_c)::value;   // no key of the wave's step is masked
     static_assert(kAt + L::rows(KT - 32) + L::kRows16 + L::kRows8 + 2 * D <= 65535, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
     if (t + 1 < ntiles) request_tile(1 - decltype(parity)::value);
+    if constexpr (kPlain) {
+      // Straight-line code in an order that lets the wave's own phases overlap: exp2 needs S alone and is dealt out between the MFMAs of S
+      // (second 32 keys) and dP, dS between those of dP and dQ (first 32).  The fragments are requested kAhead MFMAs ahead and the scheduling
+      // barriers keep the order.  Forward and backward, us: B1 H4 S3000 D64 83.0 -> 81.8, B1 H32 S512 D64 49.6 -> 48.5, B1 H4 S3000 D128 85.8 -> 84,
+      // B2 H32 S1024 D64 71.3 -> 70.5; four MFMAs ahead is level.  (Without the order, the loop without masks alone: level with the loop it replaces.)
+      constexpr int kSteps = D / 16, kAll = 6 * kSteps, kAhead = 2;
+      static_assert(KT == BN * KS && BN == 64);
+      const uint32_t step_at = KS > 1 ? static_cast<uint32_t>(ks) * L::kRows64 : 0;
+      const uint32_t row_lane = row_at + step_at, v_row_lane = v_row_at + step_at, tr_lane = tr_at + step_at;
+      f32x16 s_acc[2], dp_acc[2];
+      bf16x8 from[kAll], dsf[4];
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }
+      auto fetch = [&](int i) {
+        const int j = i % (2 * kSteps), mb = j / kSteps;   // MFMA of its product, 32-key block
+        if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * mb) + j % kSteps * 32));
+        else from[i] = lds_tr_at<D>(tr_lane + (kAt + L::rows(32 * mb) + j % kSteps / (D / 32) * L::kRows16 + j % (D / 32) * 64));
+      };
+      auto probability = [&](int e) { s_acc[e / 16][e % 16] = fast_exp2(s_acc[e / 16][e % 16] * c - lse2); };
+      auto ds = [&](int e) { dp_acc[e / 16][e % 16] = s_acc[e / 16][e % 16] * dp_acc[e / 16][e % 16]; };
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) fetch(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kAll; ++i) {
+        const int j = i % (2 * kSteps), mb = j / kSteps, s = j % kSteps;
+        if (i + kAhead < kAll) fetch(i + kAhead);
+        if (i < 2 * kSteps) s_acc[mb] = mfma32(from[i], qf[s], s_acc[mb]);
+        else if (i < 4 * kSteps) dp_acc[mb] = mfma32(from[i], dof[s], dp_acc[mb]);
+        else dq[j % (D / 32)] = mfma32(from[i], dsf[j / (D / 32)], dq[j % (D / 32)]);
+        if (i >= kSteps && i < 4 * kSteps) {
+#pragma unroll
+          for (int e = (i - kSteps) * 32 / (3 * kSteps); e < (i + 1 - kSteps) * 32 / (3 * kSteps); ++e) probability(e);
+        }
+        if (i >= 3 * kSteps && i < 5 * kSteps) {
+#pragma unroll
+          for (int e = (i - 3 * kSteps) * 16 / kSteps; e < (i + 1 - 3 * kSteps) * 16 / kSteps; ++e) ds(e);
+          const int done = (i + 1 - 3 * kSteps) * 16 / kSteps;
+          if (done % 8 == 0) dsf[done / 8 - 1] = pack8(dp_acc[(done / 8 - 1) / 2], (done / 8 - 1) % 2 * 8);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
 #pragma unroll
     for (int sub = 0; sub < KT / BN; ++sub) {
       if (KS > 1 && sub != ks) continue;
@@ -939,6 +985,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
           }
         }
     }
+    }
     wait_requests<0>();
     __syncthreads();
   };
@@ -946,11 +993,21 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   const int see = (a.causal && blk_q_lo + 32 < kv_end ? blk_q_lo + 32 : kv_end) - BN * ks;
   int mine = (see > 0 ? tiles_before(a.kv, see, KT) : 0) - t_first;
   mine = mine < 0 ? 0 : mine < ntiles ? mine : ntiles;
+  // ... and of those the tiles that no mask touches (a loop of their own, for the same reason)
+  const int unmasked = (a.causal && blk_q_lo + 1 < a.Sk ? blk_q_lo + 1 : a.Sk) - BN * (ks + 1);
+  int plain = unmasked >= 0 && !ends_inside_tile(a.kv, KT) ? unmasked / KT + 1 - t_first : 0;
+  plain = plain < 0 ? 0 : plain < mine ? plain : mine;
   int t = 0;
+  while (t < plain) {
+    trip(std::integral_constant<int, 0>(), std::true_type(), t++);
+    if (t >= plain) break;
+    trip(std::integral_constant<int, 1>(), std::true_type(), t++);
+  }
+  if (t % 2 == 1 && t < mine) trip(std::integral_constant<int, 1>(), std::false_type(), t++);
   while (t < mine) {
-    trip(std::integral_constant<int, 0>(), t++);
+    trip(std::integral_constant<int, 0>(), std::false_type(), t++);
     if (t >= mine) break;
-    trip(std::integral_constant<int, 1>(), t++);
+    trip(std::integral_constant<int, 1>(), std::false_type(), t++);
   }
   for (; t < ntiles; ++t) {
     if (t + 1 < ntiles) request_tile((t + 1) % 2);
