@@ -332,6 +332,39 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
         }
         const float m_use = (m_run[qb] == -INFINITY) ? 0.f : m_run[qb];
         float psum = 0.f;
+        if constexpr (D == 128 && NW == 4) {
+          // O^T += V^T P^T, eight keys of a lane at a time, exp2 of the next eight dealt out between the MFMAs: a wave issues in order, and
+          // vector work that stands in front of a product leaves the matrix pipe idle.  B1 H20 S1500 37.8 -> 32.5 us, B4 H8 S900 25.2 -> 21.9, B1 H8
+          // S700 18.1 -> 15.7.  (Eight waves lose by it, B1 H32 S4096 150 -> 152: their launches draw the power that the clock has
+          // to fall for.  At head_dim 64 a product is too short to cover the exponentials: B4 H32 S1024 28.5 -> 29.2.)
+          constexpr int kDb = D / 32, kAll = 4 * kDb, kPer = 8 / kDb, kAhead = 2;
+          auto probability = [&](int e) {
+            const float pv = fast_exp2(s_acc[e / 16][e % 16] * c - m_use);
+            s_acc[e / 16][e % 16] = pv;
+            psum += pv;
+          };
+          bf16x8 vf[kAll], pf[4];
+          auto fetch = [&](int i) { vf[i] = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * (i / (2 * kDb))) + i / kDb % 2 * L::kRows16 + i % kDb * 64)); };
+#pragma unroll
+          for (int i = 0; i < kAhead; ++i) fetch(i);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) probability(e);
+          pf[0] = pack8(s_acc[0], 0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < kAll; ++i) {
+            const int step = i / kDb, db = i % kDb;
+            if (i + kAhead < kAll) fetch(i + kAhead);
+            o[qb][db] = mfma32(vf[i], pf[step], o[qb][db]);
+            if (step < 3) {
+#pragma unroll
+              for (int e = 0; e < kPer; ++e) probability(8 * (step + 1) + kPer * db + e);
+              if (db + 1 == kDb) pf[step + 1] = pack8(s_acc[(step + 1) / 2], (step + 1) % 2 * 8);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          l_run[qb] += psum;
+        } else {
 #pragma unroll
         for (int mb = 0; mb < BN / 32; ++mb)
 #pragma unroll
@@ -353,6 +386,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
               o[qb][db] = mfma32(vf, pf, o[qb][db]);
             }
           }
+        }
       }
     }
     wait_requests<0>();
