@@ -673,7 +673,18 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
     }
   } else {
     // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
-    plan.kernel = groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
+    // Eight waves share each staged tile among 256 queries and have a CU to themselves; four waves do 128, two workgroups to a CU, and lose
+    // 3 to 8 % where both fill the GPU evenly (B1 H32 S4096 150.5 us, four waves 161; 256 equal workgroups 70.5, 76; 384 causal ones
+    // 50.2, 52.7).  Four waves win where eight leave CUs idle: up to 352 workgroups of 256 queries, most of which run alone on the second
+    // round (B1 H32 S2048 58.0, four waves 48.0; S2500 76.0, 65.5; B2 H16 S2100 60.6, 52.4; from 360 on 1.04 times at the worst); just over
+    // two rounds of equal ones (540: 295, 268; 624: 423, 384); and where a tenth of the queries of 256 do not exist (B8 H32 S300 30.0,
+    // 22.0; B4 H32 S777 46.8, 39.0), unless the launch has many workgroups and the tiles' traffic counts (2304: 570, 628).  From 8192 keys on
+    // a head's K and V leave an XCD's L2 no room, and twice the traffic costs what the CUs gain (312 of 52184 keys: 1952, 2076).
+    const bool rectangular = !a.causal || a.q_offset >= a.Sq;   // (workgroups of about equal length)
+    const int64_t wide = groups(256), narrow = groups(128);
+    const bool idle = wide <= 352 && !(rectangular && wide == 256), third = rectangular && wide > 512 && wide <= 640;
+    const bool padded = narrow <= 1024 && 10 * narrow <= 18 * wide;
+    plan.kernel = wide < 256 || (a.Sk <= 8192 && (idle || third || padded)) ? FwdPlan::kWaves4 : FwdPlan::kWaves8;
     if (plan.kernel == FwdPlan::kWaves8) use(FwdCfg<128, 1, 8, 64>(), 1.6, 2.13, 1.0);
     else use(FwdCfg<128, 1, 4, 64>(), 1.66, 0.96, 1.19);
   }

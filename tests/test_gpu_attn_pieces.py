@@ -142,3 +142,27 @@ def test_backward_masked_and_unmasked_trips(device, B, Hq, Hkv, Sq, Sk, D, causa
     dq, dk, dv = (torch.empty_like(t) for t in (q, k, v))
     ops.attn_bwd(do, q, k, v, lse, None, scale, causal, q_offset, dq=dq, dk=dk, dv=dv, out=out)
     check((out, lse, dq, dk, dv), want, "bf16 results")   # (bf16 operands and probabilities: the bounds of the tests above)
+
+
+# head_dim 128: workgroups of four waves below, at and above the lines to those of eight (in workgroups of 256 queries)
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,q_offset", [
+    (1, 32, 8, 2048, 2048, True, 0),     # 256, causal: four
+    (1, 32, 8, 2048, 2048, False, 0),    # 256 equal ones: eight
+    (8, 32, 8, 257, 257, True, 0),       # 512, nearly half of them padding: four
+    (8, 11, 11, 901, 901, True, 0),      # 352: four
+    (8, 32, 8, 385, 385, True, 0),       # 512 without padding: eight
+    (6, 30, 10, 640, 1280, True, 640),   # 540 equal ones: four
+])
+def test_forward_on_both_sides_of_the_lines_at_head_dim_128(device, B, Hq, Hkv, Sq, Sk, causal, q_offset):
+    """The whole launch equals launches of one batch and kv head at a time (always four waves) to the rounding of bf16 results: the
+    kernels add the same keys in the same order."""
+    from picotron_amd import ops
+    q, k, v, _ = inputs(device, B, Hq, Hkv, Sq, Sk, 128)
+    scale, group = 1 / math.sqrt(128), Hq // Hkv
+    out, lse = ops.attn_fwd(q, k, v, scale, causal, q_offset)
+    for b in range(0, B, 5):
+        for h in range(0, Hkv, 7):
+            o, l = ops.attn_fwd(q[b:b + 1, h * group:(h + 1) * group], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], scale, causal, q_offset)
+            # one unit in the last place of bf16 beside sums in another order (pieces of a cut launch)
+            assert (o.float() - out[b:b + 1, h * group:(h + 1) * group].float()).abs().max().item() <= 2 ** -7 * max(1.0, out.float().abs().max().item())
+            assert (l - lse[b:b + 1, h * group:(h + 1) * group]).abs().max().item() <= 1e-5 * max(1.0, lse.abs().max().item())
