@@ -715,9 +715,10 @@ struct DqCfg {
   static constexpr int kVecPerRow = D / 8;
   static constexpr int kLoads = KT * kVecPerRow / kThreads;
   static constexpr int kSideBytes = TileLayout<D>::bytes(KT);   // a tile's K, or V; two of K, then two of V
-  // workgroups that share a CU: the register budget and the plan go by it (at head_dim 128 a lane needs more than the 256
-  // registers that two would leave it: with some in scratch 77 -> 121 us at one head of 3000 rows)
-  static constexpr int kPerCu = NW <= 4 && D <= 64 ? 2 : 1;
+  // workgroups that share a CU: the register budget and the plan go by it (at head_dim 128 a lane has 241 of the 256 registers that
+  // two leave it; one of 332 registers was slower: 154 drawn launches of under 256 workgroups of eight waves take 0.885 of its time, B1 H12/3
+  // S912 24.5 -> 21.9 us)
+  static constexpr int kPerCu = NW <= 4 ? 2 : 1;
   // the tiles, double-buffered; the Q / dO fragments pass through LDS behind them where there is room, so that the first tile is
   // requested at once, and through the tile buffers otherwise
   static constexpr size_t kTiles = 4 * kSideBytes, kFragmentBytes = NW * WaveTile<D>::kRegionBytes;
@@ -1261,9 +1262,15 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
       case DqPlan::kSplit4: use(DqCfg<64, 4, 128, 2>(), 1.25, 0.8, 1.0); break;
     }
   } else {
-    plan.kernel = groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
+    // The forward's rule (see there), with other lines.  Four waves and eight, us: up to 384 workgroups of eight waves B8 H8 S769 27, 32, B1 H32 S1918
+    // 55, 65, B8 H8 S1418 without a mask 96, 114, B4 H8 S3063 109, 111.5; then eight (432: 97, 96; 448: 145, 135); just over two rounds B8 H12 S1403
+    // 78, 87, B4 H8 S4386 205, 214; beyond them by a few percent one way or the other (B8 H32 S5246 2918, 2610).
+    const bool rectangular = !a.causal || a.q_offset >= a.Sq;
+    const int64_t wide = groups(256), narrow = groups(128);
+    const bool idle = wide <= 384 && !(rectangular && wide == 256), third = wide > 512 && wide <= 640, padded = narrow <= 1024 && 10 * narrow <= 18 * wide;
+    plan.kernel = wide < 256 || (a.Sk <= 8192 && (idle || third || padded)) ? DqPlan::kWaves4 : DqPlan::kWaves8;
     if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 1.15, 2.81, 1.01);
-    else use(DqCfg<128, 4, 64>(), 2.45, 0.78, 1.05);
+    else use(DqCfg<128, 4, 64>(), 1.4, 0.9, 1.15);
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);

@@ -166,3 +166,26 @@ def test_forward_on_both_sides_of_the_lines_at_head_dim_128(device, B, Hq, Hkv, 
             # one unit in the last place of bf16 beside sums in another order (pieces of a cut launch)
             assert (o.float() - out[b:b + 1, h * group:(h + 1) * group].float()).abs().max().item() <= 2 ** -7 * max(1.0, out.float().abs().max().item())
             assert (l - lse[b:b + 1, h * group:(h + 1) * group]).abs().max().item() <= 1e-5 * max(1.0, lse.abs().max().item())
+
+
+# dQ at head_dim 128 on both sides of its lines (in workgroups of 256 queries), alone: no other gradient is asked for
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,q_offset", [
+    (1, 32, 8, 2048, 2048, False, 0),    # 256 equal ones: eight waves
+    (8, 32, 8, 257, 257, True, 0),       # 512, nearly half of them padding: four
+    (8, 24, 8, 511, 511, True, 0),       # 384: four
+    (7, 29, 29, 385, 385, True, 0),      # 406: eight
+    (6, 32, 8, 640, 900, True, 130),     # 576: four
+])
+def test_dq_on_both_sides_of_the_lines_at_head_dim_128(device, B, Hq, Hkv, Sq, Sk, causal, q_offset):
+    """Against the fp32 reference of a batch and kv head at a time, with the bound of bf16 operands that the tests above have."""
+    from picotron_amd import ops
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, Sk, 128)
+    scale, group = 1 / math.sqrt(128), Hq // Hkv
+    out, lse = ops.attn_fwd(q, k, v, scale, causal, q_offset)
+    dq = torch.empty_like(q)
+    ops.attn_bwd_chunks(do, q, [k], [v], lse, scale, causal, q_offset, dq=dq, dks=[None], dvs=[None], out=out)
+    for b in range(0, B, 5):
+        for h in range(0, Hkv, 7):
+            part = slice(h * group, (h + 1) * group)
+            want = reference(q[b:b + 1, part], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], scale, q_offset, causal, do[b:b + 1, part])
+            assert rel_l2(dq[b:b + 1, part], want[2]) <= 1e-2, (b, h)
