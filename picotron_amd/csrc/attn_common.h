@@ -465,7 +465,8 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
 // kernels: of 16714 launches 22 run over 1.03 of the whole launch's time, 1.07 at worst, where they would be level.  The lengths chosen
 // run within 0.5 to 1.8 % of the best ones in the geometric mean, dK/dV at head_dim 64 4 %: constants that come nearer there make every
 // twentieth launch 3 to 12 % slower than these do.  The four-wave dQ at head_dim 64 is never faster cut, which its own loss, 1.18, says: with
-// 1.02 it was cut eight times in 218, B2 H8 S4096 64.1 whole, 71.1.)
+// 1.02 it was cut eight times in 218, B2 H8 S4096 64.1 whole, 71.1.  The four-wave dQ at head_dim 128, whose workgroups came to share a CU
+// later, has costs of its own: 117 drawn launches of under 256 workgroups of eight waves, 0.87 of the time, one 1.11, all others under 1.03.)
 struct TripCost {
   double alone_us, full_us, cut;
   int per_cu;
