@@ -101,19 +101,50 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
   if (i0 >= n) return;
   auto at = [&](int j) { return i0 + j * (kThreads * N); };
   float g[kPerThread], p[kPerThread], m[kPerThread], v[kPerThread];
-  const bool whole = at(kPieces - 1) + N <= n;
-  if (whole) {
-#pragma unroll
-    for (int j = 0; j < kPieces; ++j) {
-      load_piece<false, N>(grad + at(j), g, j * N);
-      load_piece<kStream, N>(master + at(j), p, j * N);
-      load_piece<kStream, N>(exp_avg + at(j), m, j * N);
-      load_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
-    }
-  } else {
+  auto load = [&](int j) {
+    load_piece<false, N>(grad + at(j), g, j * N);
+    load_piece<kStream, N>(master + at(j), p, j * N);
+    load_piece<kStream, N>(exp_avg + at(j), m, j * N);
+    load_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
+  };
+  auto store = [&](int j) {
+    store_piece<kStream, N>(master + at(j), p, j * N);
+    store_piece<kStream, N>(exp_avg + at(j), m, j * N);
+    store_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
+    if (param_lp) store_piece<kStream, N>(param_lp + at(j), p, j * N);
+  };
+  // (the FMAs are written out: left to the compiler, which of two products it takes into one differs from block to last block)
+  auto update = [&]() {
 #pragma unroll
     for (int e = 0; e < kPerThread; ++e) {
-      const int64_t i = at(e / N) + e % N;
+      const float ge = g[e] * h.grad_scale;
+      m[e] = __builtin_fmaf(__builtin_fmaf(g[e], h.grad_scale, -m[e]), h.one_minus_b1, m[e]);
+      v[e] = __builtin_fmaf(v[e], h.b2, ge * ge * h.one_minus_b2);
+      const float denom = __builtin_fmaf(__builtin_sqrtf(v[e]), h.inv_sqrt_bc2, h.eps);
+      p[e] = __builtin_fmaf(p[e], h.decay, -(h.step_size * (m[e] / denom)));
+    }
+  };
+  if ((block + 1) * (kThreads * kPerThread) <= n) {
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) load(j);
+    update();
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) store(j);
+    return;
+  }
+  // A tensor's last block has code of its own, in which every access is judged by itself and only the one that the tensor ends in goes
+  // element by element.  Where all accesses of a thread had to be there for any to be whole (a thread's two lie 1024 elements apart), 48 tensors of 576
+  // elements took 4.5 us and take 3.8, 80 drawn lists of 0.2 to 13 M parameters 0.89 of the time, 28 bytes 0.92, 14 bytes 0.95.  (One update
+  // for both: 1.01 and, at 28 bytes, 1.04 times on lists past the caches.  As it is 0.98 and 1.01.)
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) {
+    if (at(j) + N <= n) {
+      load(j);
+      continue;
+    }
+#pragma unroll
+    for (int e = j * N; e < (j + 1) * N; ++e) {
+      const int64_t i = at(j) + e % N;
       const bool in = i < n;
       g[e] = in ? static_cast<float>(grad[i]) : 0.f;
       p[e] = in ? static_cast<float>(master[i]) : 0.f;
@@ -121,27 +152,16 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
       v[e] = in ? static_cast<float>(exp_avg_sq[i]) : 0.f;
     }
   }
+  update();
 #pragma unroll
-  for (int e = 0; e < kPerThread; ++e) {
-    const float ge = g[e] * h.grad_scale;
-    p[e] = p[e] * h.decay;
-    m[e] = m[e] + (ge - m[e]) * h.one_minus_b1;
-    v[e] = v[e] * h.b2 + ge * ge * h.one_minus_b2;
-    const float denom = __builtin_sqrtf(v[e]) * h.inv_sqrt_bc2 + h.eps;
-    p[e] = p[e] - h.step_size * (m[e] / denom);
-  }
-  if (whole) {
-#pragma unroll
-    for (int j = 0; j < kPieces; ++j) {
-      store_piece<kStream, N>(master + at(j), p, j * N);
-      store_piece<kStream, N>(exp_avg + at(j), m, j * N);
-      store_piece<kStream, N>(exp_avg_sq + at(j), v, j * N);
-      if (param_lp) store_piece<kStream, N>(param_lp + at(j), p, j * N);
+  for (int j = 0; j < kPieces; ++j) {
+    if (at(j) + N <= n) {
+      store(j);
+      continue;
     }
-  } else {
 #pragma unroll
-    for (int e = 0; e < kPerThread; ++e) {
-      const int64_t i = at(e / N) + e % N;
+    for (int e = j * N; e < (j + 1) * N; ++e) {
+      const int64_t i = at(j) + e % N;
       if (i >= n) continue;
       master[i] = static_cast<TW>(p[e]);
       exp_avg[i] = static_cast<TM>(m[e]);

@@ -628,6 +628,35 @@ def test_adamw_multi_equals_one_call_per_tensor(ops, device, state_dtype, moment
         ops.adamw_multi_(w1, gr[:-1], m1, v1, *hyper)
 
 
+ADAMW_TYPES = [(torch.bfloat16, torch.float32, torch.bfloat16), (torch.float32, torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16, torch.bfloat16),
+               (torch.bfloat16, torch.bfloat16, torch.float32), (torch.bfloat16, torch.float32, torch.float32), (torch.float32, torch.float32, torch.float32)]
+
+
+@pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", ADAMW_TYPES)
+def test_adamw_ends_of_tensors(ops, device, weight_dtype, moment_dtype, grad_dtype):
+    """A tensor's last block judges every access by itself (they are 4 or 8 elements, the accesses of a thread 1024 apart): for lengths around
+    the ends of both, every state is bit-identical to the same elements inside a whole block, and nothing behind the tensor is touched."""
+    g = torch.Generator(device=device).manual_seed(23)
+    sizes = [1, 3, 4, 5, 7, 8, 9, 576, 1020, 1023, 1024, 1025, 1027, 1028, 1031, 1032, 2040, 2043, 2044, 2047, 2048 + 4, 2048 + 1023, 2048 + 1026]
+    hyper = (3, 2e-3, 0.9, 0.95, 1e-8, 0.1, 0.5)
+    dtypes = (weight_dtype, grad_dtype, moment_dtype, moment_dtype)
+    copies = weight_dtype == torch.float32
+    whole = [[torch.randn(4096, generator=g, device=device).to(dt) for _ in sizes] for dt in dtypes]
+    whole[3] = [v.abs() for v in whole[3]]
+    parts = [[t.clone() for t in ts] for ts in whole]
+    before = [[t.clone() for t in ts] for ts in whole]
+    lp_whole, lp_parts = ([torch.full((4096,), -7.0, dtype=torch.bfloat16, device=device) for _ in sizes] for _ in range(2))
+    ops.adamw_multi_(*whole, *hyper, param_lps=lp_whole if copies else None)
+    ops.adamw_multi_(*[[t[:n] for t, n in zip(ts, sizes)] for ts in parts], *hyper,
+                     param_lps=[t[:n] for t, n in zip(lp_parts, sizes)] if copies else None)
+    for what in range(4):
+        for i, n in enumerate(sizes):
+            assert torch.equal(parts[what][i][:n], whole[what][i][:n]), (what, n)
+            assert torch.equal(parts[what][i][n:], before[what][i][n:]), (what, n)
+    for i, n in enumerate(sizes if copies else []):
+        assert torch.equal(lp_parts[i][:n], lp_whole[i][:n]) and (lp_parts[i][n:] == -7.0).all(), n
+
+
 @pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", [(torch.bfloat16, torch.float32, torch.bfloat16), (torch.float32, torch.float32, torch.bfloat16),
                                                                   (torch.bfloat16, torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("sizes", [[2048 * 255 + 2047], [2048 * 256, 3], [2048 * 300 + 5, 1, 2048 * 212 + 2044], [2048 * 256 * 38 + 2051, 6, 2048 * 77 + 1]])
