@@ -657,27 +657,39 @@ def test_adamw_ends_of_tensors(ops, device, weight_dtype, moment_dtype, grad_dty
         assert torch.equal(lp_parts[i][:n], lp_whole[i][:n]) and (lp_parts[i][n:] == -7.0).all(), n
 
 
-@pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", [(torch.bfloat16, torch.float32, torch.bfloat16), (torch.float32, torch.float32, torch.bfloat16),
-                                                                  (torch.bfloat16, torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.bfloat16, torch.float32)])
-@pytest.mark.parametrize("sizes", [[2048 * 255 + 2047], [2048 * 256, 3], [2048 * 300 + 5, 1, 2048 * 212 + 2044], [2048 * 256 * 38 + 2051, 6, 2048 * 77 + 1]])
+@pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", ADAMW_TYPES)
+@pytest.mark.parametrize("sizes", [[2048 * 255 + 2047], [2048 * 256, 3], [2048 * 300 + 5, 1, 2048 * 212 + 2044], "past the caches", "past the caches, one tensor"])
 def test_adamw_blocks_in_any_order_equal_short_calls(ops, device, sizes, weight_dtype, moment_dtype, grad_dtype):
-    """Blocks are dealt to the XCDs in runs, and steps of more than 256 MiB (the last list of sizes) stream past the caches: every state is
-    bit-identical to calls over 100 blocks of a tensor at a time, which do neither."""
+    """Blocks are dealt to the XCDs in runs, and steps of more than 256 MiB stream past the caches, in the kernel for many tensors and in
+    the one for a single tensor: every state is bit-identical to calls over 100 blocks of a tensor at a time, which do neither."""
+    copies = weight_dtype == torch.float32
+    per = weight_dtype.itemsize + 2 * moment_dtype.itemsize + grad_dtype.itemsize + (2 if copies else 0)   # bytes of a parameter's arrays
+    assert per * 2048 * 100 < 2 ** 28
+    single = sizes == "past the caches, one tensor"
+    if isinstance(sizes, str):
+        big = 2 ** 28 // per + 2051
+        sizes = [big] if single else [big - 2048 * 70, 6, 2048 * 77 + 1]
+        assert per * sum(sizes) > 2 ** 28
     g = torch.Generator(device=device).manual_seed(19)
     mk = lambda n, dt: torch.randn(n, generator=g, device=device).to(dt)
     w1, m1, v1 = [mk(n, weight_dtype) for n in sizes], [mk(n, moment_dtype) for n in sizes], [mk(n, moment_dtype).abs() for n in sizes]
     gr = [mk(n, grad_dtype) for n in sizes]
     w2, m2, v2 = ([t.clone() for t in ts] for ts in (w1, m1, v1))
-    lp = [None] * len(sizes) if weight_dtype == torch.bfloat16 else [torch.empty(n, dtype=torch.bfloat16, device=device) for n in sizes]
+    lp = [torch.empty(n, dtype=torch.bfloat16, device=device) if copies else None for n in sizes]
     hyper = (3, 2e-3, 0.9, 0.95, 1e-8, 0.1, 0.5)
-    ops.adamw_multi_(w1, gr, m1, v1, *hyper, param_lps=None if weight_dtype == torch.bfloat16 else lp)
+    if not single:
+        ops.adamw_multi_(w1, gr, m1, v1, *hyper, param_lps=lp if copies else None)
+    elif copies:
+        ops.adamw_(lp[0], w1[0], gr[0], m1[0], v1[0], *hyper)
+    else:
+        ops.adamw_lp_(w1[0], gr[0], m1[0], v1[0], *hyper)
     for i, n in enumerate(sizes):
         for a in range(0, n, 2048 * 100):
             part = [t[i][a:a + 2048 * 100] for t in (w2, gr, m2, v2)]
-            if weight_dtype == torch.bfloat16:
-                ops.adamw_lp_(*part, *hyper)
-            else:
+            if copies:
                 ops.adamw_(None, *part, *hyper)
+            else:
+                ops.adamw_lp_(*part, *hyper)
         assert torch.equal(w1[i], w2[i]) and torch.equal(m1[i], m2[i]) and torch.equal(v1[i], v2[i]), n
         assert lp[i] is None or torch.equal(lp[i], w2[i].bfloat16())
 
