@@ -15,19 +15,23 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kPerThread = 8;
 
-// What bounds a step is HBM, and what it reaches depends on how its streams meet there (22 bytes per parameter unless said):
-//   * Every access of a wave is one run of consecutive bytes, 16 per lane of the widest type.  An fp32 array read as two 16-byte halves
-//     of 32 bytes per lane touches every line twice, which streaming accesses pay for: 63 M parameters 250 us, streamed 265; this way 222.
+// What bounds a step is HBM, and what it reaches depends on how its streams meet there (22 bytes per parameter unless said).  Times as shares
+// of a kernel that read fp32 arrays as two 16-byte halves of 32 bytes per lane, through the caches, single blocks; lists of a model's
+// tensors, every kernel on the same arrays:
+//   * Every access of a wave is one run of consecutive bytes, 16 per lane of the widest type; the halves touch every line twice, which streaming
+//     accesses pay for (63 M parameters 250 us, streamed 265).  By itself it gives nothing past the caches: 36 lists of 0.3 to 11 GiB 1.03
+//     of the time, 28 bytes 1.01, 14 bytes 1.00.
 //   * Weights and moments are streamed past the caches, loads and stores, where the arrays are larger than the Infinity Cache: nothing
-//     is there when the next step reads it.  Gradients are not: the last of them are still there behind a backward pass (63 M parameters,
-//     the same gradients again: 214 us, with streamed gradients 240).  Smaller steps find everything in the cache: arrays of 218 MB
-//     58.2 us, streamed 62.9; arrays of 285 MB 124, streamed 106.
-//   * The XCDs take 16 neighbouring blocks each instead of every eighth (block_of_workgroup).  How much the runs give hangs on where the arrays
-//     lie: ten steps of 150 to 600 M parameters took 0.97 of the time before with single blocks, 0.99 with runs of 8, 0.94 with 16 (0.91 to
-//     0.99), 0.97 with 12, 14, 20, 24 and 32, 0.95 with 128.  Where all arrays are bf16 there is nothing in runs (669 M: 1640 us, with
-//     runs of 16 to 64 1700 to 1800).
-//   Before and after, us: 669 M parameters 2677 -> 2475 (5.9 TB/s), fp32 weights (28 bytes) 3520 -> 3310, bf16 moments (14 bytes) 1717 -> 1640;
-//   63 M 257 -> 212 (6.5 TB/s), 335 -> 280, 169 -> 165; 24 M 123 -> 105.  (Threads of 16 elements, or 512 of them, are 2 to 3 % behind.)
+//     is there when the next step reads it.  With whole lines the same lists take 0.91, 0.86 and 0.97.  Gradients are not streamed: the last of
+//     them are still there behind a backward pass (63 M parameters, the same gradients again: 214 us, with streamed gradients 240).
+//     Smaller steps find everything in the cache: arrays of 218 MB 58.2 us, streamed 62.9; arrays of 285 MB 124, streamed 106.
+//   * The XCDs take 16 neighbouring blocks each instead of every eighth (block_of_workgroup): 60 lists 0.977 of the time with single blocks,
+//     28 bytes 0.979 (0.93 to 1.02).  It hangs on where the arrays lie, and what sets 16 apart is not known: runs of 8, 12, 20, 24 and 32 on the
+//     same lists 0.986 to 0.992, 28 bytes 0.989 to 1.00.  Where all arrays are bf16 there is nothing in runs (669 M: 1640 us, with runs of 16 to
+//     64 1700 to 1800).
+//   Before and after, us: 669 M parameters 2677 -> 2475 (5.9 TB/s) on one card and 2707 -> 2628 (5.6) on another, fp32 weights (28 bytes)
+//   3520 -> 3310, bf16 moments (14 bytes) 1717 -> 1640; 63 M, the same gradients again, 258 -> 210, 335 -> 284, 168 -> 160.  (Threads of 16 elements, or
+//   512 of them, are 2 to 3 % behind.)
 constexpr int64_t kCacheBytes = int64_t(256) << 20;
 
 // N consecutive elements (8 or 16 bytes) as floats
