@@ -331,7 +331,9 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     auto lse_row = [&](int sb, int j) { return lds_at<f32x4>(lse_lane + (kSplit ? 32 * j : 32 * (4 * sb + j))); };
     auto delta_row = [&](int sb, int j) { return lds_at<f32x4>(lse_lane + (BM * 4 + (kSplit ? 32 * j : 32 * (4 * sb + j)))); };
 
-    // The three phases of a 32-query sub-block.
+    // The three phases of a 32-query sub-block (and of the one that a wave with QS 4 has: S beside dP and dV beside dK are two chains at a time, which
+    // its few trips wait for.  Product after product, as with QS 2 below, it lost 2 to 4 %: dK/dV of B2 H9/3 S256 11.6 us, 11.9 so;
+    // B8 H9/3 S512 18.0, 18.8; B1 H8 S700 11.5, 12.0).
     // products(): S = Q K^T and dP = dO V^T (C tile: lane = key, registers = queries); the dP accumulator starts at
     // -delta of its row (sDelta holds the negated value), so dP - delta comes out of the MFMA.
     auto products = [&](int sb, f32x16& s_acc, f32x16& dp_acc) {
@@ -341,11 +343,34 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 #pragma unroll
         for (int t = 0; t < 4; ++t) { s_acc[4 * j + t] = 0.f; dp_acc[4 * j + t] = d4[t]; }
       }
+      if constexpr (kSplit) {
+        // V comes from LDS as well: the operands are requested kAhead steps before the MFMAs that use them, and the scheduling barriers
+        // keep that order (left alone, the compiler reuses one set of registers and every MFMA waits for an LDS round trip)
+        constexpr int kSteps = D / 16, kAhead = 2;
+        static_assert(QS == 2 || kKRegs == kSteps);
+        bf16x8 qa[kSteps], da[kSteps], vb[kSteps];
+        auto fetch = [&](int j) {
+          qa[j] = lds_at<bf16x8>(row_lane + 32 * j);
+          da[j] = lds_at<bf16x8>(row_lane + (kDo + 32 * j));
+          vb[j] = lds_at<bf16x8>(kv_at + (WaveTile<D>::kRegionBytes + 32 * j));
+        };
 #pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        const bf16x8 qa = lds_at<bf16x8>(row_lane + (sub(sb) + 32 * s)), da = lds_at<bf16x8>(row_lane + (kDo + sub(sb) + 32 * s));
-        s_acc = mfma32(qa, kf[s], s_acc);
-        dp_acc = mfma32(da, vf[s], dp_acc);
+        for (int j = 0; j < kAhead; ++j) fetch(j);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) {
+          if (j + kAhead < kSteps) fetch(j + kAhead);
+          s_acc = mfma32(qa[j], kf[j], s_acc);
+          dp_acc = mfma32(da[j], vb[j], dp_acc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s) {
+          const bf16x8 qa = lds_at<bf16x8>(row_lane + (sub(sb) + 32 * s)), da = lds_at<bf16x8>(row_lane + (kDo + sub(sb) + 32 * s));
+          s_acc = mfma32(qa, kf[s], s_acc);
+          dp_acc = mfma32(da, vf[s], dp_acc);
+        }
       }
     };
     // softmax_grad(): P = exp2(S*c - lse*log2e), dS = P * (dP - delta) [already in the accumulator]; the mask test
@@ -373,6 +398,29 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // d, which is what lets the epilogue write whole 16-byte pieces of a row); P / dS come from the registers,
     // dO^T / Q^T from the row-major LDS tiles through transposing reads.
     auto accumulate = [&](int sb, const f32x16& s_acc, const f32x16& dp_acc) {
+      if constexpr (kSplit) {
+        constexpr int kSlots = 2 * (D / 32), kAhead = 2;
+        bf16x8 dof[kSlots], qf[kSlots];
+        auto fetch = [&](int idx) {
+          const int at = idx / (D / 32) * L::kRows16 + idx % (D / 32) * 64;
+          dof[idx] = lds_tr_at<D>(tr_lane + (kDo + at));
+          qf[idx] = lds_tr_at<D>(tr_lane + at);
+        };
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) fetch(j);
+        bf16x8 pf = pack8(s_acc, 0), dsf = pack8(dp_acc, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int idx = 0; idx < kSlots; ++idx) {
+          const int db = idx % (D / 32);
+          if (idx + kAhead < kSlots) fetch(idx + kAhead);
+          dv_acc[db] = mfma32(dof[idx], pf, dv_acc[db]);
+          dk_acc[db] = mfma32(qf[idx], dsf, dk_acc[db]);
+          if (idx + 1 == D / 32) { pf = pack8(s_acc, 8); dsf = pack8(dp_acc, 8); }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+      }
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
         // registers 8cc+4jj+t hold queries 32sb + 16cc + 8jj + 4h + t: dO / Q rows are fetched in that order
@@ -388,7 +436,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
     };
 
-    // The same for the one sub-block of a wave with QS > 1, product after product: exp2 and P need S alone and are dealt out between
+    // The same for the one sub-block of a wave with QS 2, product after product: exp2 and P need S alone and are dealt out between
     // the MFMAs of dP, dS between those of dV, so that the vector pipe works in the shadow of every product but S and dK.  Both operands come from
     // LDS: they are requested kAhead MFMAs before the one that uses them, across the products, and the scheduling barriers keep
     // that order (left alone, the compiler reuses one set of registers and every MFMA waits for an LDS round trip).  Forward and backward of a
@@ -396,7 +444,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
     // is hidden already by the other wave of its SIMD; LDS reads and power remain).
     auto one_block = [&](auto mask_c) __attribute__((always_inline)) {
       constexpr bool kMask = decltype(mask_c)::value;
-      constexpr int kSteps = D / 16, kPer = 16 / kSteps, kAhead = D == 64 ? 3 : 2, kAll = 4 * kSteps;   // (2 * (D / 32) MFMAs of dV and of dK, as many as of S and of dP)
+      constexpr int kSteps = D / 16, kPer = 16 / kSteps, kAhead = 2, kAll = 4 * kSteps;   // (2 * (D / 32) MFMAs of dV and of dK, as many as of S and of dP)
       // (key is masked for row (8j + 4h + t) iff key_rel > 8j + t)
       const int key_rel = a.causal ? kw0 + n - (a.q_offset + q0 + 32 * query_sb) - 4 * h : -1;
       f32x16 s_acc, dp_acc;
@@ -457,7 +505,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       }
     };
 
-    if constexpr (kSplit) {
+    if constexpr (QS == 2) {
       const int qs_pos = a.q_offset + q0 + 32 * query_sb;   // position of the sub-block's first query
       if constexpr (kOff) one_block(std::false_type());
       else if (!a.causal || kw0 <= qs_pos + 31) one_block(std::true_type());   // (else every pair is masked; the mask changes nothing off the diagonal)
@@ -552,7 +600,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
       accumulate(1, s1, d1);
     } else {
 #pragma unroll
-      for (int sb = 0; sb < BM / 32; ++sb) {
+      for (int sbi = 0; sbi < (kSplit ? 1 : BM / 32); ++sbi) {
+        const int sb = kSplit ? query_sb : sbi;
         const int qs_pos = a.q_offset + q0 + 32 * sb;       // position of the sub-block's first query
         if (a.causal && kw0 > qs_pos + 31) continue;        // every (query, key) pair of this block is masked
         f32x16 s_acc, dp_acc;
