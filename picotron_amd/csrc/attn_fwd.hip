@@ -228,14 +228,20 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     __syncthreads();  // every wave has its Q fragments: the tile buffers may be filled
     if (ntiles > 0) request_tile(0);
   }
+  // While tile 0 is on its way: the lane's places in the K and V tiles, and how many tiles the wave's queries see.  Those come first in
+  // its loop; with the others it only helps.  (A test inside the trip made the accumulators' registers depend on it, and the compiler
+  // copied all of them in some orders of the trip.  Counted behind the barrier, with a division for chunks that only kCut has inside tiles,
+  // a launch of one key tile paid 0.2 us for it: B8 H16/4 S17 D128 5.44 -> 5.78, this way 5.5.)
+  static_assert(QB == 1);
+  uint32_t row_at = L::row_place(lane), tr_at = 2 * C::kSideBytes + L::column_place(lane);
+  const int see = max(min(a.causal ? a.q_offset + q0 + 32 * qw + 32 : kv_end, kv_end) - BN * ks, 0);
+  int mine = min(max((kCut ? tiles_before(a.kv, see, KT) : (see + KT - 1) / KT) - t_first, 0), ntiles);
+  asm volatile("" : "+v"(row_at), "+v"(tr_at), "+s"(mine));   // (kept, not computed again in front of the reads)
   // Every load issued so far (Q fragments, the merge state, tile 0) is complete from here on.  Without this the
   // barrier would publish a tile that is still on its way, and the compiler would put a vmcnt(0) wait in front of the
   // loop's first MFMAs, where it would wait for the NEXT tile on every trip.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
-
-  uint32_t row_at = L::row_place(lane), tr_at = 2 * C::kSideBytes + L::column_place(lane);   // the lane's places in the K and V tiles
-  asm volatile("" : "+v"(row_at), "+v"(tr_at));   // (kept, not computed again in front of the reads)
 
   // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
   auto trip = [&](auto parity, int t) __attribute__((always_inline)) {
@@ -392,12 +398,6 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
     wait_requests<0>();
     __syncthreads();  // all waves are done with buffer t&1 (it is refilled in trip t+1) and tile t+1 is visible
   };
-  // The tiles (its step of them) that the wave's queries see come first; with the others it only helps.  (A test inside the trip
-  // made the accumulators' registers depend on it, and the compiler copied all of them in some orders of the trip.)
-  static_assert(QB == 1);
-  const int see = (a.causal && a.q_offset + q0 + 32 * qw + 32 < kv_end ? a.q_offset + q0 + 32 * qw + 32 : kv_end) - BN * ks;
-  int mine = (see > 0 ? tiles_before(a.kv, see, KT) : 0) - t_first;
-  mine = mine < 0 ? 0 : mine < ntiles ? mine : ntiles;
   int t = 0;
   while (t < mine) {
     trip(std::integral_constant<int, 0>(), t++);
