@@ -915,149 +915,110 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
     __syncthreads();  // every wave has its Q / dO fragments: the tile buffers may be filled
     if (ntiles > 0) request_tile(0);
   }
+  // While the first tile is on its way: the lane's places in the K and V tiles, and how many tiles the wave's queries see (they come
+  // first, with the others it only helps, see the forward kernel).  The tiles that no mask touches have trips of their own, in loops of
+  // their own, for the same reason.
+  const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
+  const int see = max(min(a.causal ? blk_q_lo + 32 : kv_end, kv_end) - BN * ks, 0);
+  int mine = min(max((kCut ? tiles_before(a.kv, see, KT) : (see + KT - 1) / KT) - t_first, 0), ntiles);
+  // the wave's step of a tile is unmasked up to this first key of the tile, where keys end at `end`
+  auto unmasked_end = [&](int end) { return min(a.causal ? blk_q_lo + 1 : end, end) - BN * (ks + 1); };
+  int plain = unmasked_end(a.Sk);
+  plain = plain >= 0 ? min(plain / KT + 1, mine) : 0;
+  uint32_t row_at = L::row_place(lane), v_row_at = 2 * C::kSideBytes + L::row_place(lane), tr_at = L::column_place(lane);
+  asm volatile("" : "+v"(row_at), "+v"(v_row_at), "+v"(tr_at), "+s"(mine), "+s"(plain));   // (kept, not computed again in front of the reads)
   // all loads so far are complete, the first tile among them (the barrier publishes it); stating it also keeps a
   // vmcnt(0) wait, which would hit the next tile's requests, out of the loop body
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
 
-  // the lane's places in the K and V tiles
-  uint32_t row_at = L::row_place(lane), v_row_at = 2 * C::kSideBytes + L::row_place(lane), tr_at = L::column_place(lane);
-  asm volatile("" : "+v"(row_at), "+v"(v_row_at), "+v"(tr_at));   // (kept, not computed again in front of the reads)
-
-  const int blk_q_lo = a.q_offset + q0 + qw * 32;  // position of this wave's first query
   const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
-  // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip
+  // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip (kCut, whose runs of tiles begin
+  // anywhere: on buffer t % 2)
   auto trip = [&](auto parity, auto plain_c, int t) __attribute__((always_inline)) {
     constexpr uint32_t kAt = decltype(parity)::value * C::kSideBytes;
+    const uint32_t moved = kCut ? t % 2 * C::kSideBytes : 0;
     constexpr bool kPlain = decltype(plain_c)::value;   // no key of the wave's step is masked
     static_assert(kAt + L::rows(KT - 32) + L::kRows16 + L::kRows8 + 2 * D <= 65535, "offsets of LDS reads");
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
-    if (t + 1 < ntiles) request_tile(1 - decltype(parity)::value);
-    if constexpr (kPlain) {
-      // Straight-line code in an order that lets the wave's own phases overlap: exp2 needs S alone and is dealt out between the MFMAs of S
-      // (second 32 keys) and dP, dS between those of dP and dQ (first 32).  The fragments are requested kAhead MFMAs ahead and the scheduling
-      // barriers keep the order.  Forward and backward, us: B1 H4 S3000 D64 83.0 -> 81.8, B1 H32 S512 D64 49.6 -> 48.5, B1 H4 S3000 D128 85.8 -> 84,
-      // B2 H32 S1024 D64 71.3 -> 70.5; four MFMAs ahead is level.  (Without the order, the loop without masks alone: level with the loop it replaces.)
-      constexpr int kSteps = D / 16, kAll = 6 * kSteps, kAhead = 2;
-      static_assert(KT == BN * KS && BN == 64);
-      const uint32_t step_at = KS > 1 ? static_cast<uint32_t>(ks) * L::kRows64 : 0;
-      const uint32_t row_lane = row_at + step_at, v_row_lane = v_row_at + step_at, tr_lane = tr_at + step_at;
-      f32x16 s_acc[2], dp_acc[2];
-      bf16x8 from[kAll], dsf[4];
+    if (t + 1 < ntiles) request_tile(kCut ? 1 - t % 2 : 1 - decltype(parity)::value);
+    // Straight-line code in an order that lets the wave's own phases overlap: exp2 needs S alone and is dealt out between the MFMAs of S
+    // (second 32 keys) and dP, dS between those of dP and dQ (first 32).  The fragments are requested kAhead MFMAs ahead and the scheduling
+    // barriers keep the order.  Forward and backward, us: B1 H4 S3000 D64 83.0 -> 81.8, B1 H32 S512 D64 49.6 -> 48.5, B1 H4 S3000 D128 85.8 -> 84,
+    // B2 H32 S1024 D64 71.3 -> 70.5; four MFMAs ahead is level.  Masked trips go by it as well (in the compiler's order every MFMA waited for an LDS
+    // round trip): dQ alone B1 H8 S293 D64 8.0 -> 7.6, B4 H4/1 S1287 D128 29.2 -> 28.7.
+    constexpr int kSteps = D / 16, kAll = 6 * kSteps, kAhead = 2;
+    static_assert(KT == BN * KS && BN == 64);
+    const uint32_t step_at = moved + (KS > 1 ? static_cast<uint32_t>(ks) * L::kRows64 : 0);
+    const uint32_t row_lane = row_at + step_at, v_row_lane = v_row_at + step_at, tr_lane = tr_at + step_at;
+    // keys past the diagonal or the end of their chunk are masked (the rows read past a chunk are zero, but P of a zero score need
+    // not be finite beside a very negative lse): one compare with a constant per element
+    const int last = (qpos < keys_end ? qpos : keys_end - 1) - (tile_key0 + BN * ks) - 4 * h;
+    f32x16 s_acc[2], dp_acc[2];
+    bf16x8 from[kAll], dsf[4];
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }
-      auto fetch = [&](int i) {
-        const int j = i % (2 * kSteps), mb = j / kSteps;   // MFMA of its product, 32-key block
-        if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * mb) + j % kSteps * 32));
-        else from[i] = lds_tr_at<D>(tr_lane + (kAt + L::rows(32 * mb) + j % kSteps / (D / 32) * L::kRows16 + j % (D / 32) * 64));
-      };
-      auto probability = [&](int e) { s_acc[e / 16][e % 16] = fast_exp2(s_acc[e / 16][e % 16] * c - lse2); };
-      auto ds = [&](int e) { dp_acc[e / 16][e % 16] = s_acc[e / 16][e % 16] * dp_acc[e / 16][e % 16]; };
+      for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }   // dP - delta comes out of the MFMA
+    auto fetch = [&](int i) {
+      const int j = i % (2 * kSteps), mb = j / kSteps;   // MFMA of its product, 32-key block
+      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * mb) + j % kSteps * 32));
+      else from[i] = lds_tr_at<D>(tr_lane + (kAt + L::rows(32 * mb) + j % kSteps / (D / 32) * L::kRows16 + j % (D / 32) * 64));
+    };
+    auto probability = [&](int e) {
+      float s = s_acc[e / 16][e % 16];
+      if (!kPlain && 32 * (e / 16) + 8 * (e % 16 / 4) + e % 4 > last) s = -INFINITY;   // exp2(-inf) = 0
+      s_acc[e / 16][e % 16] = fast_exp2(s * c - lse2);
+    };
+    auto ds = [&](int e) { dp_acc[e / 16][e % 16] = s_acc[e / 16][e % 16] * dp_acc[e / 16][e % 16]; };
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) fetch(i);
+    for (int i = 0; i < kAhead; ++i) fetch(i);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kAll; ++i) {
+      const int j = i % (2 * kSteps), mb = j / kSteps, s = j % kSteps;
+      if (i + kAhead < kAll) fetch(i + kAhead);
+      if (i < 2 * kSteps) s_acc[mb] = mfma32(from[i], qf[s], s_acc[mb]);
+      else if (i < 4 * kSteps) dp_acc[mb] = mfma32(from[i], dof[s], dp_acc[mb]);
+      else dq[j % (D / 32)] = mfma32(from[i], dsf[j / (D / 32)], dq[j % (D / 32)]);
+      if (i >= kSteps && i < 4 * kSteps) {
+#pragma unroll
+        for (int e = (i - kSteps) * 32 / (3 * kSteps); e < (i + 1 - kSteps) * 32 / (3 * kSteps); ++e) probability(e);
+      }
+      if (i >= 3 * kSteps && i < 5 * kSteps) {
+#pragma unroll
+        for (int e = (i - 3 * kSteps) * 16 / kSteps; e < (i + 1 - 3 * kSteps) * 16 / kSteps; ++e) ds(e);
+        const int done = (i + 1 - 3 * kSteps) * 16 / kSteps;
+        if (done % 8 == 0) dsf[done / 8 - 1] = pack8(dp_acc[(done / 8 - 1) / 2], (done / 8 - 1) % 2 * 8);
+      }
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < kAll; ++i) {
-        const int j = i % (2 * kSteps), mb = j / kSteps, s = j % kSteps;
-        if (i + kAhead < kAll) fetch(i + kAhead);
-        if (i < 2 * kSteps) s_acc[mb] = mfma32(from[i], qf[s], s_acc[mb]);
-        else if (i < 4 * kSteps) dp_acc[mb] = mfma32(from[i], dof[s], dp_acc[mb]);
-        else dq[j % (D / 32)] = mfma32(from[i], dsf[j / (D / 32)], dq[j % (D / 32)]);
-        if (i >= kSteps && i < 4 * kSteps) {
-#pragma unroll
-          for (int e = (i - kSteps) * 32 / (3 * kSteps); e < (i + 1 - kSteps) * 32 / (3 * kSteps); ++e) probability(e);
-        }
-        if (i >= 3 * kSteps && i < 5 * kSteps) {
-#pragma unroll
-          for (int e = (i - 3 * kSteps) * 16 / kSteps; e < (i + 1 - 3 * kSteps) * 16 / kSteps; ++e) ds(e);
-          const int done = (i + 1 - 3 * kSteps) * 16 / kSteps;
-          if (done % 8 == 0) dsf[done / 8 - 1] = pack8(dp_acc[(done / 8 - 1) / 2], (done / 8 - 1) % 2 * 8);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma unroll
-    for (int sub = 0; sub < KT / BN; ++sub) {
-      if (KS > 1 && sub != ks) continue;
-      const int k0 = tile_key0 + sub * BN;
-      if (kCut && KT > BN && k0 >= keys_end) break;
-      f32x16 s_acc[BN / 32], dp_acc[BN / 32];
-      // the compiler's scheduler is asked for its MFMA / LDS-read interleaving of this block (-1 to -5 %; the key-split
-      // variant is better off without)
-      if constexpr (KS == 1) __builtin_amdgcn_iglp_opt(0);
-#pragma unroll
-      for (int mb = 0; mb < BN / 32; ++mb) {
-        // dP - delta comes out of the MFMA
-#pragma unroll
-        for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }
-#pragma unroll
-        for (int s = 0; s < D / 16; ++s) {
-          const uint32_t at = kAt + L::rows(sub * BN + 32 * mb) + s * 32;
-          const bf16x8 ka = lds_at<bf16x8>(row_at + at), va = lds_at<bf16x8>(v_row_at + at);
-          s_acc[mb] = mfma32(ka, qf[s], s_acc[mb]);
-          dp_acc[mb] = mfma32(va, dof[s], dp_acc[mb]);
-        }
-      }
-      // dS^T = P^T * (dP^T - delta); keys past the diagonal or the end of their chunk are masked only in tiles that
-      // straddle it (the rows read past a chunk are zero, but P of a zero score need not be finite beside a very
-      // negative lse)
-      const bool need_mask = (a.causal && k0 + BN - 1 > blk_q_lo) || k0 + BN > keys_end;
-      if (need_mask) {
-        // the asm statement keeps this a real (wave-uniform) branch instead of per-element selects
-        asm volatile("; masked tile" ::: "memory");
-        const int last = (qpos < keys_end ? qpos : keys_end - 1) - k0 - 4 * h;   // (one compare with a constant per element)
-#pragma unroll
-        for (int mb = 0; mb < BN / 32; ++mb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (32 * mb + 8 * (i / 4) + i % 4 > last) s_acc[mb][i] = -INFINITY;   // exp2(-inf) = 0
-      }
-#pragma unroll
-      for (int mb = 0; mb < BN / 32; ++mb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float pv = fast_exp2(s_acc[mb][i] * c - lse2);
-          dp_acc[mb][i] = pv * dp_acc[mb][i];
-        }
-      // ---- dQ^T[d][query] += K^T[d][key] dS^T[key][query]
-#pragma unroll
-      for (int mb = 0; mb < BN / 32; ++mb)
-#pragma unroll
-        for (int cc = 0; cc < 2; ++cc) {
-          const bf16x8 dsf = pack8(dp_acc[mb], 8 * cc);
-#pragma unroll
-          for (int db = 0; db < D / 32; ++db) {
-            const bf16x8 ktf = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * mb) + cc * L::kRows16 + db * 64));
-            dq[db] = mfma32(ktf, dsf, dq[db]);
-          }
-        }
-    }
     }
     wait_requests<0>();
     __syncthreads();
   };
-  // the tiles that the wave's queries see come first; with the others it only helps (see the forward kernel)
-  const int see = (a.causal && blk_q_lo + 32 < kv_end ? blk_q_lo + 32 : kv_end) - BN * ks;
-  int mine = (see > 0 ? tiles_before(a.kv, see, KT) : 0) - t_first;
-  mine = mine < 0 ? 0 : mine < ntiles ? mine : ntiles;
-  // ... and of those the tiles that no mask touches (a loop of their own, for the same reason)
-  const int unmasked = (a.causal && blk_q_lo + 1 < a.Sk ? blk_q_lo + 1 : a.Sk) - BN * (ks + 1);
-  int plain = unmasked >= 0 && !ends_inside_tile(a.kv, KT) ? unmasked / KT + 1 - t_first : 0;
-  plain = plain < 0 ? 0 : plain < mine ? plain : mine;
   int t = 0;
-  while (t < plain) {
-    trip(std::integral_constant<int, 0>(), std::true_type(), t++);
-    if (t >= plain) break;
-    trip(std::integral_constant<int, 1>(), std::true_type(), t++);
-  }
-  if (t % 2 == 1 && t < mine) trip(std::integral_constant<int, 1>(), std::false_type(), t++);
-  while (t < mine) {
-    trip(std::integral_constant<int, 0>(), std::false_type(), t++);
-    if (t >= mine) break;
-    trip(std::integral_constant<int, 1>(), std::false_type(), t++);
+  if constexpr (kCut) {
+    // Chunk after chunk, whose last tile may be a partial one.  (With masked trips alone where chunks end inside tiles, 150 drawn launches took
+    // 1.12 of the time at head_dim 64 and 1.07 at 128: B4 H9/3 S1582 of 4 x 1582 keys D64 160.6 -> 139.5 us, B1 H32 S2275 of 4 x 568 45.9 -> 42.4.)
+    while (t < mine) {
+      int run = unmasked_end(pos.end) - pos.key0;
+      run = run >= 0 ? min(t + run / KT + 1, mine) : t;
+      if (t >= run) trip(std::integral_constant<int, 0>(), std::false_type(), t++);
+      while (t < run) trip(std::integral_constant<int, 0>(), std::true_type(), t++);
+    }
+  } else {
+    while (t < plain) {
+      trip(std::integral_constant<int, 0>(), std::true_type(), t++);
+      if (t >= plain) break;
+      trip(std::integral_constant<int, 1>(), std::true_type(), t++);
+    }
+    if (t % 2 == 1 && t < mine) trip(std::integral_constant<int, 1>(), std::false_type(), t++);
+    while (t < mine) {
+      trip(std::integral_constant<int, 0>(), std::false_type(), t++);
+      if (t >= mine) break;
+      trip(std::integral_constant<int, 1>(), std::false_type(), t++);
+    }
   }
   for (; t < ntiles; ++t) {
     if (t + 1 < ntiles) request_tile((t + 1) % 2);

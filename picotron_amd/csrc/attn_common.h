@@ -623,7 +623,7 @@ __host__ __device__ inline int query_tile_trips(const AttnParams& a, int qtile, 
 }
 
 // do chunks end inside key tiles of KT rows that further chunks follow?
-__host__ __device__ inline bool ends_inside_tile(const KvChunks& kv, int KT) { return kv.count > 1 && kv.len % KT != 0; }
+inline bool ends_inside_tile(const KvChunks& kv, int KT) { return kv.count > 1 && kv.len % KT != 0; }
 
 // A cursor over the key tiles of KT keys, in order, across the chunks: wave-uniform, so it lives in scalar registers;
 // stepping inside a chunk is four adds, a new chunk re-reads its base addresses from the kernel arguments.

@@ -144,6 +144,32 @@ def test_backward_masked_and_unmasked_trips(device, B, Hq, Hkv, Sq, Sk, D, causa
     check((out, lse, dq, dk, dv), want, "bf16 results")   # (bf16 operands and probabilities: the bounds of the tests above)
 
 
+# chunks of several whole key tiles and a partial one: dQ's masked and unmasked trips follow each other chunk after chunk, in every kernel
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,W,Sc,D,causal,q_offset", [
+    (1, 4, 2, 300, 3, 449, 64, False, 0),       # split keys, four waves, cut
+    (1, 4, 2, 300, 3, 449, 64, True, 700),
+    (2, 32, 8, 512, 2, 833, 64, True, 1154),    # split keys, eight waves
+    (8, 32, 32, 768, 3, 257, 64, True, 3),      # four waves
+    (4, 32, 32, 1024, 2, 577, 64, True, 130),   # eight waves
+    (1, 4, 2, 300, 3, 449, 128, True, 1047),    # four waves, cut
+    (1, 4, 2, 300, 4, 191, 128, False, 0),
+    (8, 32, 8, 512, 2, 353, 128, True, 194),    # eight waves
+])
+def test_backward_over_chunks_that_end_inside_tiles(device, B, Hq, Hkv, Sq, W, Sc, D, causal, q_offset):
+    from picotron_amd import ops
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, W * Sc, D)
+    scale = 1 / math.sqrt(D)
+    ks, vs = ([c.contiguous() for c in t.chunk(W, dim=2)] for t in (k, v))
+    out, lse, _ = ops.attn_fwd_chunks(q, ks, vs, scale, causal, q_offset)
+    dq, dks, dvs = torch.empty_like(q), [torch.empty_like(t) for t in ks], [torch.empty_like(t) for t in vs]
+    ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, causal, q_offset, dq=dq, dks=dks, dvs=dvs, out=out)
+    for b in range(0, B, 5):
+        for h in range(0, Hkv, 7):
+            part, kv = slice(h * Hq // Hkv, (h + 1) * Hq // Hkv), slice(h, h + 1)
+            got = (out[b:b + 1, part], lse[b:b + 1, part], dq[b:b + 1, part], torch.cat(dks, 2)[b:b + 1, kv], torch.cat(dvs, 2)[b:b + 1, kv])
+            check(got, reference(q[b:b + 1, part], k[b:b + 1, kv], v[b:b + 1, kv], scale, q_offset, causal, do[b:b + 1, part]), (b, h))
+
+
 # head_dim 128: workgroups of four waves below, at and above the lines to those of eight (in workgroups of 256 queries)
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,q_offset", [
     (1, 32, 8, 2048, 2048, True, 0),     # 256, causal: four
