@@ -304,6 +304,10 @@ int pico_attn_bwd_chunks(const pico_attn_desc* desc, const void* q, const pico_k
 #define PICO_ATTN_MAX_WORKSPACE (256ll << 20)
 int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count);
 int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count);
+/* How the forward's and dQ's launches for a descriptor are run: plan[0] waves per workgroup, plan[1] the waves that share 32 queries (1, or 2 that
+ * take turns in the keys), plan[2] the key tiles of a piece where query tiles are cut (0: not cut).  PICO_ERR_SHAPE for a descriptor that has no launch. */
+int pico_attn_fwd_plan(const pico_attn_desc* desc, int chunk_count, int32_t* plan);
+int pico_attn_dq_plan(const pico_attn_desc* desc, int chunk_count, int32_t* plan);
 int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out, float* lse,
                             int out_dtype, int merge, const pico_rope_tables* rope, int q_pos_offset, void* q_rot,
                             const int64_t* q_rot_stride, void* workspace, int64_t workspace_bytes, void* stream);

@@ -1518,15 +1518,37 @@ extern "C" int pico_attn_bwd_rope(const pico_attn_desc* desc, const void* q_rot,
                           dkv_stride, dkv_dtype, stream, &r);
 }
 
-extern "C" int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
+namespace {
+
+// what a plan is made from, without operands; false: there is nothing to launch
+bool plan_params(const pico_attn_desc* desc, int chunk_count, AttnParams& a) {
   if (!desc || chunk_count < 1 || (desc->D != 64 && desc->D != 128) || desc->B <= 0 || desc->Hkv <= 0 || desc->Hq % desc->Hkv != 0 ||
       desc->Hq <= 0 || desc->Sq <= 0 || desc->Sk <= 0)
-    return 0;
-  AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
+    return false;
+  a = make_params(desc, nullptr, nullptr, nullptr);
   a.kv.count = chunk_count;
   a.kv.len = desc->Sk / chunk_count;
+  return true;
+}
+
+}  // namespace
+
+extern "C" int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
+  AttnParams a;
+  if (!plan_params(desc, chunk_count, a)) return 0;
   const int64_t dkdv = desc->D == 64 ? plan_dkdv<64>(a).ws_bytes : plan_dkdv<128>(a).ws_bytes;
   return std::max(dkdv, plan_dq(a, desc->D).ws_bytes);   // (the two kernels run one after the other)
+}
+
+extern "C" int pico_attn_dq_plan(const pico_attn_desc* desc, int chunk_count, int32_t* out) {
+  if (!out) return fail(PICO_ERR_NULL, "pico_attn_dq_plan: the plan is NULL");
+  AttnParams a;
+  if (!plan_params(desc, chunk_count, a)) return fail(PICO_ERR_SHAPE, "pico_attn_dq_plan: no launch for this descriptor");
+  const DqPlan& plan = plan_dq(a, desc->D);
+  out[0] = plan.kernel == DqPlan::kWaves8 || plan.kernel == DqPlan::kSplit8 ? 8 : 4;
+  out[1] = plan.kernel == DqPlan::kSplit4 || plan.kernel == DqPlan::kSplit8 ? 2 : 1;
+  out[2] = plan.len;
+  return PICO_OK;
 }
 
 extern "C" int pico_attn_bwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, const void* dout,

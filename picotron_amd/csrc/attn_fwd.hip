@@ -778,12 +778,32 @@ extern "C" int pico_attn_fwd_rope(const pico_attn_desc* desc, const void* q, con
   return run_fwd("pico_attn_fwd_rope", desc, q, &kv, out, lse, out_dtype, merge, rope, q_pos_offset, q_rot, q_rot_stride, stream);
 }
 
-extern "C" int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
-  if (!desc || chunk_count < 1 || (desc->D != 64 && desc->D != 128) || desc->B <= 0 || desc->Hq <= 0 || desc->Sq <= 0 || desc->Sk <= 0) return 0;
+namespace {
+
+// the plan for a descriptor without its operands; nullptr: there is nothing to launch
+const FwdPlan* plan_fwd(const pico_attn_desc* desc, int chunk_count) {
+  if (!desc || chunk_count < 1 || (desc->D != 64 && desc->D != 128) || desc->B <= 0 || desc->Hq <= 0 || desc->Sq <= 0 || desc->Sk <= 0) return nullptr;
   AttnParams a = make_params(desc, nullptr, nullptr, nullptr);
   a.kv.count = chunk_count;
   a.kv.len = desc->Sk / chunk_count;
-  return plan_fwd(a, desc->D).ws_bytes;
+  return &plan_fwd(a, desc->D);
+}
+
+}  // namespace
+
+extern "C" int64_t pico_attn_fwd_workspace_bytes(const pico_attn_desc* desc, int chunk_count) {
+  const FwdPlan* plan = plan_fwd(desc, chunk_count);
+  return plan ? plan->ws_bytes : 0;
+}
+
+extern "C" int pico_attn_fwd_plan(const pico_attn_desc* desc, int chunk_count, int32_t* out) {
+  if (!out) return fail(PICO_ERR_NULL, "pico_attn_fwd_plan: the plan is NULL");
+  const FwdPlan* plan = plan_fwd(desc, chunk_count);
+  if (!plan) return fail(PICO_ERR_SHAPE, "pico_attn_fwd_plan: no launch for this descriptor");
+  out[0] = plan->kernel == FwdPlan::kWaves8 || plan->kernel == FwdPlan::kSplit8 ? 8 : 4;
+  out[1] = plan->kernel == FwdPlan::kSplit4 || plan->kernel == FwdPlan::kSplit8 ? 2 : 1;
+  out[2] = plan->len;
+  return PICO_OK;
 }
 
 extern "C" int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out,
