@@ -1280,7 +1280,14 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     const bool idle = wide <= 384 && !(rectangular && wide == 256), third = wide > 512 && wide <= 640, padded = narrow <= 1024 && 10 * narrow <= 18 * wide;
     plan.kernel = wide < 256 || (a.Sk <= 8192 && (idle || third || padded)) ? DqPlan::kWaves4 : DqPlan::kWaves8;
     if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 1.15, 2.81, 1.01);
-    else use(DqCfg<128, 4, 64>(), 1.4, 0.9, 1.15);
+    else {
+      // The estimates put short walks in pieces 2 to 7 us too high (what the second kernel adds up is still in L2), so half of the time of a launch
+      // is asked for.  That cuts 27 of 589 drawn launches more, walks of 11 to 22 key tiles, to 0.76 to 0.98 of their time (one 1.024): B2 H4 S1168
+      // 25.2 us whole, 19.0 cut; B4 H2 S480 x 960 20.9, 16.9; B1 H4 S877 20.2, 17.0.  (2.0 would cut heads in eights of 14 tiles as well, whose sums
+      // stay on their XCD, B1 H8 S859 20.1, 16.8, but also B1 H9/3 S890 19.7, 21.2.)
+      use(DqCfg<128, 4, 64>(), 1.4, 0.9, 1.15);
+      cost.launch_us = 2.5;
+    }
   }
   const int n_qtiles = (a.Sq + bm - 1) / bm;
   cost.piece_bytes = 4.0 * (bm / 32) * dq_piece_floats(D);

@@ -471,6 +471,7 @@ struct TripCost {
   double alone_us, full_us, cut;
   int per_cu;
   double piece_bytes;
+  double launch_us = 5.0;   // by how much a cut has to win by the estimate (see choose_pieces)
 };
 // When the last of a launch's workgroups ends: they are dealt in grid order, tile by tile, to whichever place is free first.
 struct Places {
@@ -537,9 +538,8 @@ int choose_pieces(int64_t heads, int n_tiles, const TripCost& c, bool pairs, con
   // a cut has to win 5 % by the estimate (so that few of the launches above lose) and the time in which a
   // host launches the second kernel: where the host is the slower side a shorter kernel gains nothing (B2 H9/3 S256 D64, forward and backward: 33 us
   // of kernels cut to 29 took 38 us for 35)
-  constexpr double kLaunchUs = 5.0;
   const double uncut_us = launch_us(heads, n_tiles, c, 0, pairs, trips_of);
-  double best_us = std::min(0.95 * uncut_us, uncut_us - kLaunchUs);
+  double best_us = std::min(0.95 * uncut_us, uncut_us - c.launch_us);
   int best = 0, longest = 0;
   for (int i = 0; i < n_tiles; ++i) longest = std::max(longest, trips_of(i));
   for (int len : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {

@@ -56,6 +56,18 @@ def test_waves_at_head_dim_128(sizes, wide, narrow, fwd, dq):
     assert plan("fwd", *sizes)[:2] == (fwd, 1) and plan("dq", *sizes)[:2] == (dq, 1)
 
 
+@pytest.mark.parametrize("sizes,piece", [
+    ((2, 4, 1168, 1168, True, 0), 6),       # us whole and cut: 25.2, 19.0
+    ((4, 2, 480, 960, True, 480), 4),       # 20.9, 16.9
+    ((1, 4, 877, 877, True, 0), 4),         # 20.2, 17.0
+    ((1, 4, 903, 903, False, 0), 6),        # 20.8, 17.4
+    ((2, 4, 620, 620, True, 0), 0),         # a walk too short for it
+    ((1, 9, 890, 890, True, 0), 0),         # 19.7, 21.2
+])
+def test_short_walks_of_dq_in_pieces(sizes, piece):
+    assert plan("dq", *sizes) == (4, 1, piece)
+
+
 def test_a_descriptor_without_a_launch_has_no_plan():
     for which in ("fwd", "dq"):
         for sizes in ((0, 4, 64, 64, True, 0), (1, 4, 0, 64, True, 0), (1, 4, 64, 0, True, 0)):
