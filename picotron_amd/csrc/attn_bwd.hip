@@ -1274,11 +1274,12 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
   } else {
     // The forward's rule (see there), with other lines.  Four waves and eight, us: up to 384 workgroups of eight waves B8 H8 S769 27, 32, B1 H32 S1918
     // 55, 65, B8 H8 S1418 without a mask 96, 114, B4 H8 S3063 109, 111.5; then eight (432: 97, 96; 448: 145, 135); just over two rounds B8 H12 S1403
-    // 78, 87, B4 H8 S4386 205, 214; beyond them by a few percent one way or the other (B8 H32 S5246 2918, 2610).
+    // 78, 87, B4 H8 S4386 205, 214; beyond them by a few percent one way or the other (B8 H32 S5246 2918, 2610).  One workgroup to a head either way:
+    // B64 H32 S128 70, 103; B128 H32/8 S64 67, 122; B48 H32/8 128 x 4096 518, 930.
     const bool rectangular = !a.causal || a.q_offset >= a.Sq;
     const int64_t wide = groups(256), narrow = groups(128);
     const bool idle = wide <= 384 && !(rectangular && wide == 256), third = wide > 512 && wide <= 640, padded = narrow <= 1024 && 10 * narrow <= 18 * wide;
-    plan.kernel = wide < 256 || (a.Sk <= 8192 && (idle || third || padded)) ? DqPlan::kWaves4 : DqPlan::kWaves8;
+    plan.kernel = wide < 256 || narrow == wide || (a.Sk <= 8192 && (idle || third || padded)) ? DqPlan::kWaves4 : DqPlan::kWaves8;
     if (plan.kernel == DqPlan::kWaves8) use(DqCfg<128, 8, 64>(), 1.15, 2.81, 1.01);
     else {
       // The estimates put short walks in pieces 2 to 7 us too high (what the second kernel adds up is still in L2), so half of the time of a launch

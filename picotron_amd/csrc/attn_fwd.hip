@@ -678,13 +678,15 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
     // 50.2, 52.7).  Four waves win where eight leave CUs idle: up to 352 workgroups of 256 queries, most of which run alone on the second
     // round (B1 H32 S2048 58.0, four waves 48.0; S2500 76.0, 65.5; B2 H16 S2100 60.6, 52.4; from 360 on 1.04 times at the worst); just over
     // two rounds of equal ones (540: 295, 268; 624: 423, 384); and where a tenth of the queries of 256 do not exist (B8 H32 S300 30.0,
-    // 22.0; B4 H32 S777 46.8, 39.0), unless the launch has many workgroups and the tiles' traffic counts (2304: 570, 628).  From 8192 keys on
-    // a head's K and V leave an XCD's L2 no room, and twice the traffic costs what the CUs gain (312 of 52184 keys: 1952, 2076).
+    // 22.0; B4 H32 S777 46.8, 39.0), unless the launch has many workgroups and the tiles' traffic counts (2304: 570, 628).  It never does for up to
+    // 128 queries, one workgroup to a head either way, where half of eight waves and more have no query at all: B64 H32 S128 67.5, 45.1;
+    // B128 H32/8 S64 88.5, 48.3; B48 H32/8 128 x 4096 762, 461.
+    // From 8192 keys on a head's K and V leave an XCD's L2 no room, and twice the traffic costs what the CUs gain (312 of 52184 keys: 1952, 2076).
     const bool rectangular = !a.causal || a.q_offset >= a.Sq;   // (workgroups of about equal length)
     const int64_t wide = groups(256), narrow = groups(128);
     const bool idle = wide <= 352 && !(rectangular && wide == 256), third = rectangular && wide > 512 && wide <= 640;
     const bool padded = narrow <= 1024 && 10 * narrow <= 18 * wide;
-    plan.kernel = wide < 256 || (a.Sk <= 8192 && (idle || third || padded)) ? FwdPlan::kWaves4 : FwdPlan::kWaves8;
+    plan.kernel = wide < 256 || narrow == wide || (a.Sk <= 8192 && (idle || third || padded)) ? FwdPlan::kWaves4 : FwdPlan::kWaves8;
     if (plan.kernel == FwdPlan::kWaves8) use(FwdCfg<128, 1, 8, 64>(), 1.6, 2.13, 1.0);
     else use(FwdCfg<128, 1, 4, 64>(), 1.66, 0.96, 1.19);
   }

@@ -42,6 +42,10 @@ LINES = [
     ((1, 342, 300, 300, True, 0), 684, 1026, 8, 8),         # ... in many workgroups
     ((1, 100, 1153, 1153, True, 0), 500, 1000, 8, 8),       # narrow = 2 wide: none missing
     ((1, 100, 1100, 1100, True, 0), 500, 900, 4, 4),
+    ((33, 32, 128, 128, True, 0), 1056, 1056, 4, 4),        # one workgroup to a head either way
+    ((64, 32, 16, 512, True, 496), 2048, 2048, 4, 4),
+    ((33, 32, 128, 9000, False, 0), 1056, 1056, 4, 4),
+    ((33, 32, 129, 129, True, 0), 1056, 2112, 8, 8),
     ((1, 9, 8192, 8192, True, 0), 288, 576, 4, 4),          # keys past which the tiles' traffic counts
     ((1, 9, 8192, 8193, True, 0), 288, 576, 8, 8),
     ((1, 180, 768, 8193, False, 0), 540, 1080, 8, 8),
