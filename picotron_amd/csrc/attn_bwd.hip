@@ -1145,7 +1145,7 @@ DkdvPlan make_dkdv_plan(const AttnParams& a) {
   const int64_t heads = static_cast<int64_t>(a.Hkv) * a.B;
   const int n_ktiles = tiles_before(a.kv, a.Sk, C::BN);
   // pairs only when they still fill most of the GPU (two workgroups per CU for D = 64, one for D = 128; at D = 64 three
-  // quarters of the places are enough: rank 2 of 4 at configs[1], 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
+  // quarters of the places are enough: rank 2 of 4 of B4 H32 S1024, 384 pairs, 21.2 -> 20.3 us; with 256 pairs single tiles
   // are up to 30 % faster)
   // Few workgroups with short chains: the kernel whose chain is a quarter as long.  It takes 6.6 us + 0.92 per trip (of 128
   // queries) while its workgroups have a CU each, the usual one 5.3 + 1.25 per trip (of 64): B2 H9/3 S256 20.3 -> 12.1, B2 H32
@@ -1262,7 +1262,7 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     if (groups(256) >= 768 && visible_keys <= 1536) plan.kernel = DqPlan::kWaves4;
     else if (groups(256) >= 512) plan.kernel = DqPlan::kWaves8;
     else if (groups(128) >= 512) plan.kernel = rectangular && groups(256) >= 256 ? DqPlan::kWaves8 : DqPlan::kWaves4;
-    // few waves in all: two waves per 32 queries, 64 keys of every 128 each (rank 3 of 4 at configs[1] with eight waves
+    // few waves in all: two waves per 32 queries, 64 keys of every 128 each (rank 3 of 4 of B4 H32 S1024 with eight waves
     // per workgroup: 18.8 -> 17.9 us)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? DqPlan::kSplit8 : DqPlan::kSplit4;
     switch (plan.kernel) {
@@ -1275,7 +1275,9 @@ DqPlan make_dq_plan(const AttnParams& a, int D) {
     // The forward's rule (see there), with other lines.  Four waves and eight, us: up to 384 workgroups of eight waves B8 H8 S769 27, 32, B1 H32 S1918
     // 55, 65, B8 H8 S1418 without a mask 96, 114, B4 H8 S3063 109, 111.5; then eight (432: 97, 96; 448: 145, 135); just over two rounds B8 H12 S1403
     // 78, 87, B4 H8 S4386 205, 214; beyond them by a few percent one way or the other (B8 H32 S5246 2918, 2610).  One workgroup to a head either way:
-    // B64 H32 S128 70, 103; B128 H32/8 S64 67, 122; B48 H32/8 128 x 4096 518, 930.
+    // B64 H32 S128 70, 103; B128 H32/8 S64 67, 122; B48 H32/8 128 x 4096 518, 930.  The line at 8192 keys is the forward's and costs less on either
+    // side (288 workgroups of 8192 x 10240 498, 521, x 16384 767, 825, shifted 612, 587, x 32768 1560, 1549), and so does its absence under one
+    // round of workgroups of eight (12 heads of 4096 x 16384 484, 443; 9 of 4096 x 8192 172, 171; whole sequences of 14 heads 99, 112).
     const bool rectangular = !a.causal || a.q_offset >= a.Sq;
     const int64_t wide = groups(256), narrow = groups(128);
     const bool idle = wide <= 384 && !(rectangular && wide == 256), third = wide > 512 && wide <= 640, padded = narrow <= 1024 && 10 * narrow <= 18 * wide;

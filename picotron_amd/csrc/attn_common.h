@@ -109,7 +109,7 @@ __device__ __forceinline__ u32x4 request_window(uint64_t base, uint32_t bytes) {
 // none either.  And a lane's piece of any group of rows, any columns, lies at a constant distance from its first: one register per
 // kind of read holds all addresses.  Before, dense rows whose pieces changed places with the row: eight addresses per kind of read
 // at head_dim 128, kept in registers or flipped anew, and an addition in front of every read.  Forward at head_dim 128 221 -> 171
-// registers, 16 of 180 vector instructions per trip less: B1 H32 S4096 136.2 -> 133.3 us (D64 86.5 -> 84.3), its dK/dV 19 % fewer
+// registers, 16 of 180 vector instructions per trip less: B1 H32 S4096 136.2 -> 133.3 us in a long row of launches (D64 86.5 -> 84.3), its dK/dV 19 % fewer
 // of them and 257 -> 250 us (matrix work at the power limit: 4 % fewer cycles); small launches gain more, B3 H9/3 S777 D64 12.4 -> 10.7,
 // one rank's B1 H32 256 x 1024 13.3 -> 11.0.
 // (Counted conflicts say how LDS takes a read: 16 lanes of a 16-byte one at a time, 32 of an 8-byte one.  A layout that spread the

@@ -341,7 +341,7 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
         if constexpr (D == 128 && NW == 4) {
           // O^T += V^T P^T, eight keys of a lane at a time, exp2 of the next eight dealt out between the MFMAs: a wave issues in order, and
           // vector work that stands in front of a product leaves the matrix pipe idle.  B1 H20 S1500 37.8 -> 32.5 us, B4 H8 S900 25.2 -> 21.9, B1 H8
-          // S700 18.1 -> 15.7.  (Eight waves lose by it, B1 H32 S4096 150 -> 152: their launches draw the power that the clock has
+          // S700 18.1 -> 15.7.  (Eight waves lose by it, B1 H32 S4096 150 -> 152 right after a pause: their launches draw the power that the clock has
           // to fall for.  At head_dim 64 a product is too short to cover the exponentials: B4 H32 S1024 28.5 -> 29.2.)
           constexpr int kDb = D / 32, kAll = 4 * kDb, kPer = 8 / kDb, kAhead = 2;
           auto probability = [&](int e) {
@@ -372,26 +372,26 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
           l_run[qb] += psum;
         } else {
 #pragma unroll
-        for (int mb = 0; mb < BN / 32; ++mb)
+          for (int mb = 0; mb < BN / 32; ++mb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float pv = fast_exp2(s_acc[mb][i] * c - m_use);
-            s_acc[mb][i] = pv;
-            psum += pv;
-          }
-        l_run[qb] += psum;
-        // ---- O^T[d][query] += V^T[d][key] P^T[key][query]
-#pragma unroll
-        for (int mb = 0; mb < BN / 32; ++mb)
-#pragma unroll
-          for (int cc = 0; cc < 2; ++cc) {
-            const bf16x8 pf = pack8(s_acc[mb], 8 * cc);
-#pragma unroll
-            for (int db = 0; db < D / 32; ++db) {
-              const bf16x8 vf = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * mb) + cc * L::kRows16 + db * 64));
-              o[qb][db] = mfma32(vf, pf, o[qb][db]);
+            for (int i = 0; i < 16; ++i) {
+              const float pv = fast_exp2(s_acc[mb][i] * c - m_use);
+              s_acc[mb][i] = pv;
+              psum += pv;
             }
-          }
+          l_run[qb] += psum;
+          // ---- O^T[d][query] += V^T[d][key] P^T[key][query]
+#pragma unroll
+          for (int mb = 0; mb < BN / 32; ++mb)
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc) {
+              const bf16x8 pf = pack8(s_acc[mb], 8 * cc);
+#pragma unroll
+              for (int db = 0; db < D / 32; ++db) {
+                const bf16x8 vf = lds_tr_at<D>(tr_at + (kAt + L::rows(sub * BN + 32 * mb) + cc * L::kRows16 + db * 64));
+                o[qb][db] = mfma32(vf, pf, o[qb][db]);
+              }
+            }
         }
       }
     }
@@ -662,7 +662,7 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
     // (measured at B8, 256 queries x 1024 keys of every head: 26.9 us with eight waves, 30.1 us with four)
     else if (groups(128) >= 512) plan.kernel = rectangular && groups(256) >= 256 ? FwdPlan::kWaves8 : FwdPlan::kWaves4;
     // few waves in all: two waves per 32 queries, 64 keys of every 128 each -- in workgroups of eight waves (128 queries)
-    // when those still cover the CUs and the launch is rectangular (one rank's share of configs[1]: 19.8 -> 16.9 us for
+    // when those still cover the CUs and the launch is rectangular (one rank's share of B4 H32 S1024 in a ring of four: 19.8 -> 16.9 us for
     // rank 3 of 4; on a whole causal sequence, or with 256 keys, the smaller workgroups are a few percent faster)
     else plan.kernel = groups(128) >= 256 && rectangular && visible_keys >= 512 ? FwdPlan::kSplit8 : FwdPlan::kSplit4;
     switch (plan.kernel) {
@@ -674,14 +674,19 @@ FwdPlan make_fwd_plan(const AttnParams& a, int D) {
   } else {
     // (64-key staged tiles: 0.5-4 % faster than 128-key ones at every size measured)
     // Eight waves share each staged tile among 256 queries and have a CU to themselves; four waves do 128, two workgroups to a CU, and lose
-    // 3 to 8 % where both fill the GPU evenly (B1 H32 S4096 150.5 us, four waves 161; 256 equal workgroups 70.5, 76; 384 causal ones
+    // 3 to 8 % where both fill the GPU evenly (B1 H32 S4096 130 us in a long row of launches, four waves 142, 150 and 161 right after a pause; 256 equal workgroups 70.5, 76; 384 causal ones
     // 50.2, 52.7).  Four waves win where eight leave CUs idle: up to 352 workgroups of 256 queries, most of which run alone on the second
     // round (B1 H32 S2048 58.0, four waves 48.0; S2500 76.0, 65.5; B2 H16 S2100 60.6, 52.4; from 360 on 1.04 times at the worst); just over
     // two rounds of equal ones (540: 295, 268; 624: 423, 384); and where a tenth of the queries of 256 do not exist (B8 H32 S300 30.0,
     // 22.0; B4 H32 S777 46.8, 39.0), unless the launch has many workgroups and the tiles' traffic counts (2304: 570, 628).  It never does for up to
     // 128 queries, one workgroup to a head either way, where half of eight waves and more have no query at all: B64 H32 S128 67.5, 45.1;
     // B128 H32/8 S64 88.5, 48.3; B48 H32/8 128 x 4096 762, 461.
-    // From 8192 keys on a head's K and V leave an XCD's L2 no room, and twice the traffic costs what the CUs gain (312 of 52184 keys: 1952, 2076).
+    // From somewhere past 8192 keys on a head's K and V leave an XCD's L2 no room, and twice the traffic costs what the CUs gain.  The line
+    // is a cut through launches that go both ways (288 workgroups, eight and four: 9 heads of 8192 x 8192 179, 174, without a mask 344, 362; x 10240
+    // 403, 389, shifted 256, 234; x 12288 473, 460, shifted 314, 339; x 16384 618, 600, shifted 450, 491); at 32768 four lose in most (1207,
+    // 1382; 36 heads of 2048 1374, 1662; 312 of 52184 1952, 2076).  Under one round of workgroups of eight the line does not hold them back,
+    // which loses where the workgroups are about equal and few more than half a round (12 heads of 4096 x 16384 340, 387, x 32768 693, 852; 9 of
+    // 4096 x 8192 131, 143), is level at 128 and 240 (466, 487; 937, 950) and pays for whole causal sequences (10 heads of 4096 65, 68; 14 heads 89, 77).
     const bool rectangular = !a.causal || a.q_offset >= a.Sq;   // (workgroups of about equal length)
     const int64_t wide = groups(256), narrow = groups(128);
     const bool idle = wide <= 352 && !(rectangular && wide == 256), third = rectangular && wide > 512 && wide <= 640;
