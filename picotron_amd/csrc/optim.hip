@@ -57,8 +57,13 @@ __device__ __forceinline__ void load_piece(const T* p, float (&out)[kPerThread],
 template <bool kStream, int N, typename T>
 __device__ __forceinline__ void store_piece(T* p, const float (&in)[kPerThread], int at) {
   auto put = [&](auto raw) {
-    if constexpr (kStream) __builtin_nontemporal_store(raw, reinterpret_cast<decltype(raw)*>(p));
-    else *reinterpret_cast<decltype(raw)*>(p) = raw;
+    if constexpr (kStream) {
+      // (as it is: otherwise the compiler rebuilds the 16 bytes of eight bf16 values into a vector of its own and stores that without the hint)
+      asm("" : "+v"(raw));
+      __builtin_nontemporal_store(raw, reinterpret_cast<decltype(raw)*>(p));
+    } else {
+      *reinterpret_cast<decltype(raw)*>(p) = raw;
+    }
   };
   if constexpr (sizeof(T) == 4) {
     static_assert(N == 4);

@@ -192,3 +192,18 @@ extern "C" __global__ void parted(uint64_t base, uint32_t bytes, uint32_t to) {
         body = assembly[assembly.index(f"\n{name}:"):]
         seen = re.findall(r"s_mov_b32 m0, 40|s_sendmsg|s_add_u32 m0|offen lds", body[:body.index("s_endpgm")])
         assert seen == ["s_mov_b32 m0, 40", "s_sendmsg", "s_add_u32 m0", "offen lds", "s_mov_b32 m0, 40", "s_sendmsg"], (name, seen)
+
+
+def test_streaming_optimizer_kernels_store_past_the_caches():
+    """Every vector store of the AdamW kernels for arrays larger than the caches carries the streaming hint, and none of the others does;
+    of the loads all but the gradient's do."""
+    _, text = compiled(csrc("optim.hip"))
+    seen = 0
+    for name, body in re.findall(r"^(_Z\w*adamw\w*):\s*;.*?$(.*?)s_endpgm", text, flags=re.S | re.M):
+        streams = re.search(r"kernelILb([01])E", name).group(1) == "1"
+        loads, stores = (re.findall(r"^\s*global_%s_dwordx[24] .*$" % what, body, flags=re.M) for what in ("load", "store"))
+        assert loads and stores, name
+        assert all((" nt" in line) == streams for line in stores), name
+        assert sum(" nt" in line for line in loads) == (3 * len(loads) // 4 if streams else 0), name
+        seen += 1
+    assert seen == 24   # one and many tensors, streaming or not, six combinations of types
