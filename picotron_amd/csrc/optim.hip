@@ -13,7 +13,9 @@ namespace pico {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPerThread = 8;
+// elements of a thread: one access of each array where the step streams past the caches, otherwise two (one where all arrays are bf16)
+template <bool kStream>
+constexpr int kPerThread = kStream ? 4 : 8;
 
 // What bounds a step is HBM, and what it reaches depends on how its streams meet there (22 bytes per parameter unless said).  Times as shares
 // of a kernel that read fp32 arrays as two 16-byte halves of 32 bytes per lane, through the caches, single blocks; lists of a model's
@@ -22,21 +24,24 @@ constexpr int kPerThread = 8;
 //     accesses pay for (63 M parameters 250 us, streamed 265).  By itself it gives nothing past the caches: 36 lists of 0.3 to 11 GiB 1.03
 //     of the time, 28 bytes 1.01, 14 bytes 1.00.
 //   * Weights and moments are streamed past the caches, loads and stores, where the arrays are larger than the Infinity Cache: nothing
-//     is there when the next step reads it.  With whole lines the same lists take 0.91, 0.86 and 0.97.  Gradients are not streamed: the last of
-//     them are still there behind a backward pass (63 M parameters, the same gradients again: 214 us, with streamed gradients 240).
-//     Smaller steps find everything in the cache: arrays of 218 MB 58.2 us, streamed 62.9; arrays of 285 MB 124, streamed 106.
-//   * The XCDs take 16 neighbouring blocks each instead of every eighth (block_of_workgroup): 60 lists 0.977 of the time with single blocks,
-//     28 bytes 0.979 (0.93 to 1.02).  It hangs on where the arrays lie, and what sets 16 apart is not known: runs of 8, 12, 20, 24 and 32 on the
-//     same lists 0.986 to 0.992, 28 bytes 0.989 to 1.00.  Where all arrays are bf16 there is nothing in runs (669 M: 1640 us, with runs of 16 to
-//     64 1700 to 1800).
-//   Before and after, us: 669 M parameters 2677 -> 2475 (5.9 TB/s) on one card and 2707 -> 2628 (5.6) on another, fp32 weights (28 bytes)
-//   3520 -> 3310, bf16 moments (14 bytes) 1717 -> 1640; 63 M, the same gradients again, 258 -> 210, 335 -> 284, 168 -> 160.  (Threads of 16 elements, or
-//   512 of them, are 2 to 3 % behind.)
+//     is there when the next step reads it.  Gradients are not: the last of them are still there behind a backward pass (63 M parameters,
+//     the same gradients again: 214 us, with streamed gradients 240).  Smaller steps find everything in the cache: arrays of 218 MB
+//     58.2 us, streamed 62.9; arrays of 285 MB 124, streamed 106.
+//   * A thread of a streamed step has one access of each array, 4 elements.  With two (one of 8 where all arrays are bf16), how far apart the
+//     compiler laid loads, arithmetic and stores moved the time by up to 8 % either way (28 bytes: all eight loads first 1.07 of the time that the
+//     loads around the first wait took).  30 lists of 0.1 to 1.6 G parameters: 0.892 of the time with one, 0.902 with two; 28 bytes 0.910, 0.921;
+//     14 bytes 0.836, 0.938.  Steps in the cache keep two: 30 lists of 0.5 to 23 M parameters took 1.001 to 1.008 of the time with one, up to 1.09.
+//   * The XCDs take runs of neighbouring blocks instead of every eighth (block_of_workgroup), of 32 K elements.  It hangs on where the arrays lie,
+//     and what sets this length apart is not known: 24 lists with runs of 32 blocks 0.966 of the time of two accesses and runs of 16, 64 blocks
+//     0.974, single ones 0.961; 28 bytes 0.990, 1.000, 0.999; 14 bytes 0.897, 0.893, 0.911.  In the cache 60 lists with two accesses took 0.977 of
+//     the time of single blocks.  Where all arrays are bf16 and in the cache there is nothing in runs.
+//   Before all of it and now, on one card, us: 667 M parameters 2694 -> 2478 (5.9 TB/s), fp32 weights (28 bytes) 3502 -> 3249, bf16 moments (14
+//   bytes) 1702 -> 1491 (6.3 TB/s); 64 M, the same gradients again, 263 -> 210, 342 -> 279, 174 -> 135.  (512 threads are 2 to 3 % behind.)
 constexpr int64_t kCacheBytes = int64_t(256) << 20;
 
 // N consecutive elements (8 or 16 bytes) as floats
 template <bool kStream, int N, typename T>
-__device__ __forceinline__ void load_piece(const T* p, float (&out)[kPerThread], int at) {
+__device__ __forceinline__ void load_piece(const T* p, float* out, int at) {
   if constexpr (sizeof(T) == 4) {
     static_assert(N == 4);
     const f32x4* from = reinterpret_cast<const f32x4*>(p);
@@ -55,7 +60,7 @@ __device__ __forceinline__ void load_piece(const T* p, float (&out)[kPerThread],
   }
 }
 template <bool kStream, int N, typename T>
-__device__ __forceinline__ void store_piece(T* p, const float (&in)[kPerThread], int at) {
+__device__ __forceinline__ void store_piece(T* p, const float* in, int at) {
   auto put = [&](auto raw) {
     if constexpr (kStream) {
       // (as it is: otherwise the compiler rebuilds the 16 bytes of eight bf16 values into a vector of its own and stores that without the hint)
@@ -88,15 +93,16 @@ struct Hyper {
   float decay, one_minus_b1, b2, one_minus_b2, step_size, inv_sqrt_bc2, eps, grad_scale;
 };
 
-// elements of one access: 16 bytes of the widest type
-template <typename TW, typename TM, typename TG>
-constexpr int kPiece = sizeof(TW) == 2 && sizeof(TM) == 2 && sizeof(TG) == 2 ? 8 : 4;
+// elements of one access: 16 bytes of the widest type, at most a thread's
+template <bool kStream, typename TW, typename TM, typename TG>
+constexpr int kPiece = !kStream && sizeof(TW) == 2 && sizeof(TM) == 2 && sizeof(TG) == 2 ? 8 : 4;
 
 // The block of a workgroup: neighbouring workgroups run on different XCDs (they go round all eight), and each XCD takes kRun blocks in
 // a row.  What does not fill a round of runs is dealt block by block.
-template <int N>
+template <bool kStream, int N>
 __device__ __forceinline__ unsigned block_of_workgroup(unsigned workgroup, unsigned count) {
-  constexpr unsigned kRun = N == 8 ? 1 : 16, kXcds = 8, kRound = kXcds * kRun;
+  constexpr unsigned kRun = kStream ? 32 : N == 8 ? 1 : 16, kXcds = 8, kRound = kXcds * kRun;
+  if constexpr (kRun == 1) return workgroup;
   const unsigned round = workgroup / kRound, in = workgroup % kRound;
   return (round + 1) * kRound <= count ? round * kRound + in % kXcds * kRun + in / kXcds : workgroup;
 }
@@ -105,11 +111,11 @@ template <bool kStream, typename TW, typename TM, typename TG>
 __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* __restrict__ master,
                                             const TG* __restrict__ grad, TM* __restrict__ exp_avg,
                                             TM* __restrict__ exp_avg_sq, int64_t n, int64_t block, const Hyper& h) {
-  constexpr int N = kPiece<TW, TM, TG>, kPieces = kPerThread / N;
-  const int64_t i0 = block * (kThreads * kPerThread) + threadIdx.x * N;
+  constexpr int N = kPiece<kStream, TW, TM, TG>, kMine = kPerThread<kStream>, kPieces = kMine / N;
+  const int64_t i0 = block * (kThreads * kMine) + threadIdx.x * N;
   if (i0 >= n) return;
   auto at = [&](int j) { return i0 + j * (kThreads * N); };
-  float g[kPerThread], p[kPerThread], m[kPerThread], v[kPerThread];
+  float g[kMine], p[kMine], m[kMine], v[kMine];
   auto load = [&](int j) {
     load_piece<false, N>(grad + at(j), g, j * N);
     load_piece<kStream, N>(master + at(j), p, j * N);
@@ -125,7 +131,7 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
   // (the FMAs are written out: left to the compiler, which of two products it takes into one differs from block to last block)
   auto update = [&]() {
 #pragma unroll
-    for (int e = 0; e < kPerThread; ++e) {
+    for (int e = 0; e < kMine; ++e) {
       const float ge = g[e] * h.grad_scale;
       m[e] = __builtin_fmaf(__builtin_fmaf(g[e], h.grad_scale, -m[e]), h.one_minus_b1, m[e]);
       v[e] = __builtin_fmaf(v[e], h.b2, ge * ge * h.one_minus_b2);
@@ -133,7 +139,7 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
       p[e] = __builtin_fmaf(p[e], h.decay, -(h.step_size * (m[e] / denom)));
     }
   };
-  if ((block + 1) * (kThreads * kPerThread) <= n) {
+  if ((block + 1) * (kThreads * kMine) <= n) {
 #pragma unroll
     for (int j = 0; j < kPieces; ++j) load(j);
     update();
@@ -143,8 +149,7 @@ __device__ __forceinline__ void adamw_block(__bf16* __restrict__ param_lp, TW* _
   }
   // A tensor's last block has code of its own, in which every access is judged by itself and only the one that the tensor ends in goes
   // element by element.  Where all accesses of a thread had to be there for any to be whole (a thread's two lie 1024 elements apart), 48 tensors of 576
-  // elements took 4.5 us and take 3.8, 80 drawn lists of 0.2 to 13 M parameters 0.89 of the time, 28 bytes 0.92, 14 bytes 0.95.  (One update
-  // for both: 1.01 and, at 28 bytes, 1.04 times on lists past the caches.  As it is 0.98 and 1.01.)
+  // elements took 4.5 us and take 3.8, 80 drawn lists of 0.2 to 13 M parameters 0.89 of the time, 28 bytes 0.92, 14 bytes 0.95.
 #pragma unroll
   for (int j = 0; j < kPieces; ++j) {
     if (at(j) + N <= n) {
@@ -184,7 +189,7 @@ template <bool kStream, typename TW, typename TM, typename TG>
 __global__ __launch_bounds__(kThreads) void adamw_kernel(__bf16* __restrict__ param_lp, TW* __restrict__ master,
                                                          const TG* __restrict__ grad, TM* __restrict__ exp_avg,
                                                          TM* __restrict__ exp_avg_sq, int64_t n, Hyper h) {
-  adamw_block<kStream, TW, TM, TG>(param_lp, master, grad, exp_avg, exp_avg_sq, n, block_of_workgroup<kPiece<TW, TM, TG>>(blockIdx.x, gridDim.x), h);
+  adamw_block<kStream, TW, TM, TG>(param_lp, master, grad, exp_avg, exp_avg_sq, n, block_of_workgroup<kStream, kPiece<kStream, TW, TM, TG>>(blockIdx.x, gridDim.x), h);
 }
 
 // Many tensors in one launch: the pointers travel in the kernel arguments (no table in device memory to keep alive),
@@ -203,7 +208,7 @@ struct TensorTable {
 
 template <bool kStream, typename TW, typename TM, typename TG>
 __global__ __launch_bounds__(kThreads) void adamw_multi_kernel(TensorTable t, Hyper h) {
-  const unsigned bid = block_of_workgroup<kPiece<TW, TM, TG>>(blockIdx.x, gridDim.x);
+  const unsigned bid = block_of_workgroup<kStream, kPiece<kStream, TW, TM, TG>>(blockIdx.x, gridDim.x);
   int lo = 0, hi = t.count;   // block_start[lo] <= bid < block_start[hi]
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
@@ -244,7 +249,12 @@ Hyper make_hyper(float lr, float beta1, float beta2, float eps, float weight_dec
   return h;
 }
 
-constexpr int64_t kPerBlock = static_cast<int64_t>(kThreads) * kPerThread;
+int64_t blocks_of(int64_t n, bool stream) {
+  const int64_t per_block = kThreads * (stream ? kPerThread<true> : kPerThread<false>);
+  return (n + per_block - 1) / per_block;
+}
+// A launch has less than 2^32 threads; tensors of more than this many elements (a whole number of blocks) go in slices.
+constexpr int64_t kMostBlocks = 0xffffffff / kThreads, kSlice = int64_t(1) << 31;
 
 template <typename TW, typename TM>
 int64_t state_bytes(int grad_dtype, bool copy) {   // per parameter, each array once
@@ -273,14 +283,19 @@ int adamw_launch(const char* who, void* param_lp, TW* master, const void* grad, 
   if (!aligned16(param_lp) || !aligned16(master) || !aligned16(grad) || !aligned16(exp_avg) || !aligned16(exp_avg_sq))
     return fail(PICO_ERR_ALIGN, "%s: pointers must be 16-byte aligned", who);
   const Hyper h = make_hyper(lr, beta1, beta2, eps, weight_decay, step, grad_scale);
-  const unsigned grid = static_cast<unsigned>((n + kPerBlock - 1) / kPerBlock);
+  const bool stream_all = streams(n * state_bytes<TW, TM>(grad_dtype, param_lp != nullptr));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  with_kernel_types(grad_dtype, streams(n * state_bytes<TW, TM>(grad_dtype, param_lp != nullptr)), [&](auto stream_it, auto grad_type) {
-    using TG = decltype(grad_type);
-    hipLaunchKernelGGL((adamw_kernel<decltype(stream_it)::value, TW, TM, TG>), dim3(grid), dim3(kThreads), 0, s, static_cast<__bf16*>(param_lp),
-                       master, static_cast<const TG*>(grad), exp_avg, exp_avg_sq, n, h);
-  });
-  return check_launch(who);
+  for (int64_t at = 0; at < n; at += kSlice) {
+    const int64_t count = std::min(n - at, kSlice);
+    with_kernel_types(grad_dtype, stream_all, [&](auto stream_it, auto grad_type) {
+      using TG = decltype(grad_type);
+      hipLaunchKernelGGL((adamw_kernel<decltype(stream_it)::value, TW, TM, TG>), dim3(static_cast<unsigned>(blocks_of(count, stream_all))), dim3(kThreads), 0, s,
+                         param_lp ? static_cast<__bf16*>(param_lp) + at : nullptr, master + at, static_cast<const TG*>(grad) + at, exp_avg + at,
+                         exp_avg_sq + at, count, h);
+    });
+    if (int rc = check_launch(who)) return rc;
+  }
+  return PICO_OK;
 }
 
 template <typename TW, typename TM>
@@ -297,7 +312,7 @@ int adamw_multi_launch(int count, void* const* weights, void* const* param_lps, 
     if (!aligned16(weights[i]) || !aligned16(grads[i]) || !aligned16(exp_avgs[i]) || !aligned16(exp_avg_sqs[i]) ||
         (param_lps && !aligned16(param_lps[i])))
       return fail(PICO_ERR_ALIGN, "%s: tensor %d: pointers must be 16-byte aligned", who, i);
-    if ((sizes[i] + kPerBlock - 1) / kPerBlock > 0x7fffffff)
+    if (blocks_of(sizes[i], false) > 0x7fffffff)
       return fail(PICO_ERR_SHAPE, "%s: tensor %d is too large for one launch", who, i);
   }
   int64_t elements = 0;
@@ -317,17 +332,19 @@ int adamw_multi_launch(int count, void* const* weights, void* const* param_lps, 
   };
   for (int i = 0; i < count; ++i) {
     if (sizes[i] == 0) continue;
-    const uint64_t blocks = static_cast<uint64_t>((sizes[i] + kPerBlock - 1) / kPerBlock);
-    if (t.count == kMaxTensors || t.block_start[t.count] + blocks > 0x7fffffffu)
-      if (int rc = flush()) return rc;
-    const int j = t.count++;
-    t.weight[j] = weights[i];
-    t.param_lp[j] = param_lps ? param_lps[i] : nullptr;
-    t.grad[j] = grads[i];
-    t.exp_avg[j] = exp_avgs[i];
-    t.exp_avg_sq[j] = exp_avg_sqs[i];
-    t.n[j] = sizes[i];
-    t.block_start[j + 1] = t.block_start[j] + static_cast<unsigned>(blocks);
+    for (int64_t at = 0; at < sizes[i]; at += kSlice) {
+      const int64_t n = std::min(sizes[i] - at, kSlice), blocks = blocks_of(n, stream_all);
+      if (t.count == kMaxTensors || t.block_start[t.count] + blocks > kMostBlocks)
+        if (int rc = flush()) return rc;
+      const int j = t.count++;
+      t.weight[j] = static_cast<TW*>(weights[i]) + at;
+      t.param_lp[j] = param_lps && param_lps[i] ? static_cast<__bf16*>(param_lps[i]) + at : nullptr;
+      t.grad[j] = static_cast<const char*>(grads[i]) + at * (grad_dtype == PICO_BF16 ? 2 : 4);
+      t.exp_avg[j] = static_cast<TM*>(exp_avgs[i]) + at;
+      t.exp_avg_sq[j] = static_cast<TM*>(exp_avg_sqs[i]) + at;
+      t.n[j] = n;
+      t.block_start[j + 1] = t.block_start[j] + static_cast<unsigned>(blocks);
+    }
   }
   return flush();
 }

@@ -634,8 +634,8 @@ ADAMW_TYPES = [(torch.bfloat16, torch.float32, torch.bfloat16), (torch.float32, 
 
 @pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", ADAMW_TYPES)
 def test_adamw_ends_of_tensors(ops, device, weight_dtype, moment_dtype, grad_dtype):
-    """A tensor's last block judges every access by itself (they are 4 or 8 elements, the accesses of a thread 1024 apart): for lengths around
-    the ends of both, every state is bit-identical to the same elements inside a whole block, and nothing behind the tensor is touched."""
+    """A tensor's last block judges every access by itself (they are 4 or 8 elements, a thread's two 1024 apart): for lengths around the
+    ends of both, every state is bit-identical to the same elements inside a whole block, and nothing behind the tensor is touched."""
     g = torch.Generator(device=device).manual_seed(23)
     sizes = [1, 3, 4, 5, 7, 8, 9, 576, 1020, 1023, 1024, 1025, 1027, 1028, 1031, 1032, 2040, 2043, 2044, 2047, 2048 + 4, 2048 + 1023, 2048 + 1026]
     hyper = (3, 2e-3, 0.9, 0.95, 1e-8, 0.1, 0.5)
@@ -655,6 +655,30 @@ def test_adamw_ends_of_tensors(ops, device, weight_dtype, moment_dtype, grad_dty
             assert torch.equal(parts[what][i][n:], before[what][i][n:]), (what, n)
     for i, n in enumerate(sizes if copies else []):
         assert torch.equal(lp_parts[i][:n], lp_whole[i][:n]) and (lp_parts[i][n:] == -7.0).all(), n
+
+
+@pytest.mark.parametrize("many", [False, True])
+def test_adamw_of_a_tensor_that_goes_in_slices(ops, device, many):
+    """Tensors of more than 2^31 elements take a launch (or an entry of its table) for every 2^31: on both sides of that line and at both
+    ends every state is bit-identical to a short call over the same elements."""
+    if torch.cuda.get_device_properties(device).total_memory < 40 * 2 ** 30:
+        pytest.skip("needs 17 GiB for the arrays and as much again to make them")
+    n, hyper = 2 ** 31 + 2051, (3, 2e-3, 0.9, 0.95, 1e-8, 0.1, 0.5)
+    g = torch.Generator(device=device).manual_seed(29)
+    some = torch.randn(2 ** 22 + 7, generator=g, device=device).bfloat16()
+    make = lambda shift: some.roll(shift).repeat(n // some.numel() + 1)[:n]   # noqa: E731
+    w, gr, m, v = make(0), make(11), make(23), make(37).abs_()
+    parts = [slice(0, 4096), slice(2 ** 31 - 4096, 2 ** 31 + 2051), slice(2 ** 30, 2 ** 30 + 2048)]
+    want = [[t[part].clone() for t in (w, gr, m, v)] for part in parts]
+    if many:
+        small = [t[:5].clone() for t in (w, gr, m, v)]
+        ops.adamw_multi_([small[0], w], [small[1], gr], [small[2], m], [small[3], v], *hyper)
+    else:
+        ops.adamw_lp_(w, gr, m, v, *hyper)
+    for part, short in zip(parts, want):
+        ops.adamw_lp_(*short, *hyper)
+        for got, right in zip((w, gr, m, v), short):
+            assert torch.equal(got[part], right), part
 
 
 @pytest.mark.parametrize("weight_dtype,moment_dtype,grad_dtype", ADAMW_TYPES)
