@@ -461,12 +461,14 @@ __device__ __forceinline__ int first_piece(int tile, int len, const F& trips_of)
 // Host: the piece length for a launch, from what its workgroups cost.  A trip takes `alone_us` in a workgroup that has its
 // CU to itself and `full_us` of a CU's time where `per_cu` workgroups share each, `cut` times that in the kernel that can cut
 // (see kCut of the forward); `per_cu` is the number the kernel's registers and LDS are budgeted for.
-// (Fitted to every piece length of some thousand launches, 1 to 256 heads and 200 to 8192 rows, and held against 5752 others with today's
-// kernels: of 16714 launches 22 run over 1.03 of the whole launch's time, 1.07 at worst, where they would be level.  The lengths chosen
-// run within 0.5 to 1.8 % of the best ones in the geometric mean, dK/dV at head_dim 64 4 %: constants that come nearer there make every
-// twentieth launch 3 to 12 % slower than these do.  The four-wave dQ at head_dim 64 is never faster cut, which its own loss, 1.18, says: with
-// 1.02 it was cut eight times in 218, B2 H8 S4096 64.1 whole, 71.1.  The four-wave dQ at head_dim 128, whose workgroups came to share a CU
-// later, has costs of its own: 117 drawn launches of under 256 workgroups of eight waves, 0.87 of the time, one 1.11, all others under 1.03.)
+// (Fitted to every piece length of some thousand launches, 1 to 256 heads and 200 to 8192 rows; of 16714 others 22 ran over 1.03 of the whole
+// launch's time, 1.07 at worst, where they would be level.  Since then the uncut kernels gained more than the cutting ones: of 6179 launches of
+// 2136 drawn shapes 62 are over 1.03 now, the worst forwards of few heads at head_dim 64 (B1 H6/2 S4629 35.7 us whole, 44.1 cut; both were
+// slower before, 46.6 and 48.8).  The lengths chosen run within 0.1 to 2.5 % of the best ones in the geometric mean, dK/dV at head_dim 64 4 %:
+// constants that came nearer there made every twentieth launch 3 to 12 % slower than these did.  The four-wave dQ at head_dim 64 is
+// never faster cut, which its own loss, 1.18, says: with 1.02 it was cut eight times in 218, B2 H8 S4096 64.1 whole, 71.1.  The four-wave dQ at
+// head_dim 128, whose workgroups came to share a CU later, has costs of its own: over 589 launches and every length within 1.6 % of the best, 6
+// over 1.03 of the whole launch; of 180 other sets of its three costs the twelve that come within 1.45 % have 8 to 21 there, 1.17 at worst.)
 struct TripCost {
   double alone_us, full_us, cut;
   int per_cu;
