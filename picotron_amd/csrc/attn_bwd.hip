@@ -682,6 +682,10 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const BwdParams& p, const int
 // is 1 to 2 % slower with the pieces' bookkeeping around it (in the forward and in dQ up to 10 %).
 template <int D, int QS, bool kCut>
 __device__ __forceinline__ void attn_bwd_dkdv_body(const BwdParams& p) {
+  const Arguments<offsetof(BwdParams, dk), offsetof(BwdParams, dk_final), offsetof(BwdParams, dv), offsetof(BwdParams, dv_final), offsetof(BwdParams, dkfs),
+                  sizeof(BwdParams) - 4> gradients;
+  AttnArguments().arrive();
+  gradients.arrive();
   using C = KvCfg<D, QS>;
   if constexpr (kCut) {
     const Piece at = find_piece(blockIdx.y, tiles_before(p.a.kv, p.a.Sk, C::BN), p.a.pieces.len, [&](int i) { return dkdv_trips(p.a, i, C::BN, C::BM); });
@@ -804,6 +808,8 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
+  const Arguments<offsetof(BwdParams, dq), offsetof(BwdParams, dqs), sizeof(BwdParams) - 4> late;   // (what the epilogue uses)
+  AttnArguments().arrive();
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
   // same dispatch order as the forward kernel: every head's last (longest) query tile first
@@ -927,6 +933,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   plain = plain >= 0 ? min(plain / KT + 1, mine) : 0;
   uint32_t row_at = L::row_place(lane), v_row_at = 2 * C::kSideBytes + L::row_place(lane), tr_at = L::column_place(lane);
   asm volatile("" : "+v"(row_at), "+v"(v_row_at), "+v"(tr_at), "+s"(mine), "+s"(plain));   // (kept, not computed again in front of the reads)
+  late.arrive();
   // all loads so far are complete, the first tile among them (the barrier publishes it); stating it also keeps a
   // vmcnt(0) wait, which would hit the next tile's requests, out of the loop body
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
