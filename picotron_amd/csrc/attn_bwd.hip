@@ -772,6 +772,7 @@ struct DqCfg {
   // two leave it; one of 332 registers was slower: 154 drawn launches of under 256 workgroups of eight waves take 0.885 of its time, B1 H12/3
   // S912 24.5 -> 21.9 us)
   static constexpr int kPerCu = NW <= 4 ? 2 : 1;
+  static constexpr bool kSmall = D == 128 && NW == 8;   // products of 16 x 16 x 32 (see DqWave)
   // the tiles, double-buffered; the Q / dO fragments pass through LDS behind them where there is room, so that the first tile is
   // requested at once, and through the tile buffers otherwise
   static constexpr size_t kTiles = 4 * kSideBytes, kFragmentBytes = NW * WaveTile<D>::kRegionBytes;
@@ -788,23 +789,266 @@ struct DqCfg {
 // what a wave of a piece leaves: its dQ^T accumulators
 __host__ __device__ constexpr int dq_piece_floats(int D) { return (D / 32) * 16 * kWave; }
 
-// the wave's 32 dQ rows leave through its piece of LDS as whole lines
+// A wave's part of dQ: 32 queries, their fragments and sums, and a trip over 64 keys, with products of 32 x 32 x 16 or of 16 x 16 x 32.
+// The smaller ones take a seventh less power for the same work (a loop of products alone on normal values 1820 and 2080 TFLOP/s, on
+// zeros 2475 and 2440), and as many more issue slots.  So they are for the launches that run at the power limit, eight waves at head_dim 128:
+// dQ of B1 H32 S4096 169.1 -> 158.8 us, of 4096 queries and 32768 keys, 32 / 8 heads, 2264 -> 2126, of B8 H32 S1024 without a mask 197 -> 189.
+// The others wait for latencies and issue slots: at head_dim 64 level (0.98 to 1.02), four waves at head_dim 128, B1 H12 S1111 without a mask 24.8
+// us and 27.7, B1 H8/2 S700 16.9 and 18.7.
+//
+// A trip is straight-line code in an order that lets the wave's own phases overlap: exp2 needs S alone and is dealt out between the MFMAs of S
+// (second 32 keys) and dP, dS between those of dP and dQ (first 32).  The fragments are requested kAhead MFMAs of 32 x 32 x 16 ahead and the scheduling
+// barriers keep the order.  Forward and backward, us: B1 H4 S3000 D64 83.0 -> 81.8, B1 H32 S512 D64 49.6 -> 48.5, B1 H4 S3000 D128 85.8 -> 84,
+// B2 H32 S1024 D64 71.3 -> 70.5; four MFMAs ahead is level.  Masked trips go by it as well (in the compiler's order every MFMA waited for an LDS
+// round trip): dQ alone B1 H8 S293 D64 8.0 -> 7.6, B4 H4/1 S1287 D128 29.2 -> 28.7.
+template <int D, bool kDelta>
+struct DqOperands {   // a wave's rows of Q, dO and O, on their way
+  WaveTile<D> qt, dt, ot;
+  __device__ __forceinline__ void issue(const BwdParams& p, int b, int hq, int row0, int lane) {
+    const AttnParams& a = p.a;
+    const int64_t q_at = b * a.qs[0] + hq * a.qs[1] + static_cast<int64_t>(row0) * a.qs[2], o_at = b * a.os[0] + hq * a.os[1] + static_cast<int64_t>(row0) * a.os[2];
+    const buffer_rsrc qb = make_buffer(a.q + q_at, span_bytes(a.Sq - row0, a.qs[2], D)), db = make_buffer(p.dout + o_at, span_bytes(a.Sq - row0, a.os[2], D));
+    const buffer_rsrc ob = kDelta ? make_buffer(p.out + o_at, span_bytes(a.Sq - row0, a.os[2], D)) : db;
+    qt.issue(qb, a.qs[2], lane);
+    dt.issue(db, a.os[2], lane);
+    if constexpr (kDelta) ot.issue(ob, a.os[2], lane);
+  }
+};
+
+template <int D, bool kSmall> struct DqWave;
 template <int D>
-__device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* region, f32x16 (&dq)[D / 32], int b, int hq, int row0, int lane) {
+struct DqWave<D, false> {   // lane = query lane % 32, registers = keys
+  using L = TileLayout<D>;
+  static constexpr int kSteps = D / 16;
+  bf16x8 qf[D / 16], dof[D / 16];
+  float lse2, delta;
+  int pos, first_key;   // position of the lane's query; the first of its keys of 32
+  f32x16 dq[D / 32];
+  static __device__ __forceinline__ uint32_t row_place(int lane) { return L::row_place(lane); }
+  static __device__ __forceinline__ uint32_t column_place(int lane) { return L::column_place(lane); }
+  static __device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
+  }
+  // the fragments of the rows from row0, their lse, and delta = sum_d dO * O (context_parallel.py:145): each half of the wave holds half of
+  // a row's columns; with `writes` it goes to memory, for the dK/dV kernel that is launched after this one
+  template <bool kDelta>
+  __device__ __forceinline__ void load(const BwdParams& p, unsigned char* region, int64_t lse_row0, int b, int hq, int row0, bool writes, int lane) {
+    DqOperands<D, kDelta> rows;
+    rows.issue(p, b, hq, row0, lane);
+    const int qrow = row0 + lane % 32, h = lane / 32;
+    const int64_t gi = lse_row0 + qrow;
+    pos = p.a.causal ? p.a.q_offset + qrow : 0x7fffff00;   // (past every key)
+    first_key = 4 * h;
+    const uint32_t left = static_cast<uint32_t>(max(p.a.Sq - row0, 0)) * 4u, at = lane % 32 * 4u;
+    const float l = buffer_load_f32(make_buffer(p.lse + lse_row0 + row0, left), at);
+    delta = kDelta ? 0.f : buffer_load_f32(make_buffer(p.delta + lse_row0 + row0, left), at);
+    rows.qt.fragments(region, lane, qf);
+    rows.dt.fragments(region, lane, dof);
+    lse2 = qrow < p.a.Sq && l != -INFINITY ? l * kLog2e : INFINITY;   // (a row that saw no key contributes nothing)
+    if constexpr (kDelta) {
+      bf16x8 of[D / 16];
+      rows.ot.fragments(region, lane, of);
+      float part = 0.f;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part += static_cast<float>(dof[s][e]) * static_cast<float>(of[s][e]);
+      delta = half_sum(part);
+      if (qrow < p.a.Sq && h == 0 && writes) p.delta_w[gi] = delta;
+    }
+  }
+  // the 64 keys from position key0, whose rows lie at the three places (+ kAt); kPlain: none of them is masked, otherwise those past the
+  // query and from keys_end on are
+  template <uint32_t kAt, bool kPlain>
+  __device__ __forceinline__ void trip(uint32_t row_lane, uint32_t v_row_lane, uint32_t tr_lane, int key0, int keys_end, float c) {
+    constexpr int kAll = 6 * kSteps, kAhead = 2;
+    // (the rows read past a chunk are zero, but P of a zero score need not be finite beside a very negative lse): one compare with a constant per
+    // element
+    const int last = min(pos, keys_end - 1) - key0 - first_key;
+    f32x16 s_acc[2], dp_acc[2];
+    bf16x8 from[kAll], dsf[4];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }   // dP - delta comes out of the MFMA
+    auto fetch = [&](int i) {
+      const int j = i % (2 * kSteps), mb = j / kSteps;   // MFMA of its product, 32-key block
+      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * mb) + j % kSteps * 32));
+      else from[i] = lds_tr_at<D>(tr_lane + (kAt + L::rows(32 * mb) + j % kSteps / (D / 32) * L::kRows16 + j % (D / 32) * 64));
+    };
+    auto probability = [&](int e) {
+      float s = s_acc[e / 16][e % 16];
+      if (!kPlain && 32 * (e / 16) + 8 * (e % 16 / 4) + e % 4 > last) s = -INFINITY;   // exp2(-inf) = 0
+      s_acc[e / 16][e % 16] = fast_exp2(s * c - lse2);
+    };
+    auto ds = [&](int e) { dp_acc[e / 16][e % 16] = s_acc[e / 16][e % 16] * dp_acc[e / 16][e % 16]; };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) fetch(i);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kAll; ++i) {
+      const int j = i % (2 * kSteps), mb = j / kSteps, s = j % kSteps;
+      if (i + kAhead < kAll) fetch(i + kAhead);
+      if (i < 2 * kSteps) s_acc[mb] = mfma32(from[i], qf[s], s_acc[mb]);
+      else if (i < 4 * kSteps) dp_acc[mb] = mfma32(from[i], dof[s], dp_acc[mb]);
+      else dq[j % (D / 32)] = mfma32(from[i], dsf[j / (D / 32)], dq[j % (D / 32)]);
+      if (i >= kSteps && i < 4 * kSteps) {
+#pragma unroll
+        for (int e = (i - kSteps) * 32 / (3 * kSteps); e < (i + 1 - kSteps) * 32 / (3 * kSteps); ++e) probability(e);
+      }
+      if (i >= 3 * kSteps && i < 5 * kSteps) {
+#pragma unroll
+        for (int e = (i - 3 * kSteps) * 16 / kSteps; e < (i + 1 - 3 * kSteps) * 16 / kSteps; ++e) ds(e);
+        const int done = (i + 1 - 3 * kSteps) * 16 / kSteps;
+        if (done % 8 == 0) dsf[done / 8 - 1] = pack8(dp_acc[(done / 8 - 1) / 2], (done / 8 - 1) % 2 * 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
+template <int D>
+struct DqWave<D, true> {   // lane = queries lane % 16 and 16 + lane % 16, registers = keys group_row(lane / 16) ..+3 of every 16
+  using L = TileLayout<D>;
+  static constexpr int kSteps = D / 16;
+  bf16x8 qf[2][D / 32], dof[2][D / 32];
+  float lse2[2], delta[2];
+  int pos, first_key;   // position of the lane's first query; the first of its keys of 16
+  f32x4 dq[D / 16][2];
+  static __device__ __forceinline__ uint32_t row_place(int lane) { return L::row_place16(lane); }
+  static __device__ __forceinline__ uint32_t column_place(int lane) { return L::column_place16(lane); }
+  static __device__ __forceinline__ void clear(f32x4 (&acc)[D / 16][2]) {
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) acc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  template <bool kDelta>   // (a quarter of a row's columns in each lane of it)
+  __device__ __forceinline__ void load(const BwdParams& p, unsigned char* region, int64_t lse_row0, int b, int hq, int row0, bool writes, int lane) {
+    DqOperands<D, kDelta> rows;
+    rows.issue(p, b, hq, row0, lane);
+    const int qrow = row0 + lane % 16;
+    const int64_t gi = lse_row0 + qrow;
+    pos = p.a.causal ? p.a.q_offset + qrow : 0x7fffff00;
+    first_key = L::group_row(lane / 16);
+    const uint32_t left = static_cast<uint32_t>(max(p.a.Sq - row0, 0)) * 4u;
+    const buffer_rsrc lb = make_buffer(p.lse + lse_row0 + row0, left), eb = make_buffer((kDelta ? p.lse : p.delta) + lse_row0 + row0, left);
+    float l[2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      l[qb] = buffer_load_f32(lb, (lane % 16 + 16 * qb) * 4u);
+      delta[qb] = kDelta ? 0.f : buffer_load_f32(eb, (lane % 16 + 16 * qb) * 4u);
+    }
+    rows.qt.fragments16(region, lane, qf);
+    rows.dt.fragments16(region, lane, dof);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) lse2[qb] = qrow + 16 * qb < p.a.Sq && l[qb] != -INFINITY ? l[qb] * kLog2e : INFINITY;
+    if constexpr (kDelta) {
+      bf16x8 of[2][D / 32];
+      rows.ot.fragments16(region, lane, of);
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        float part = 0.f;
+#pragma unroll
+        for (int s = 0; s < D / 32; ++s)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) part += static_cast<float>(dof[qb][s][e]) * static_cast<float>(of[qb][s][e]);
+        delta[qb] = group_sum(part);
+        if (qrow + 16 * qb < p.a.Sq && lane < 16 && writes) p.delta_w[gi + 16 * qb] = delta[qb];
+      }
+    }
+  }
+  template <uint32_t kAt, bool kPlain>
+  __device__ __forceinline__ void trip(uint32_t row_lane, uint32_t v_row_lane, uint32_t tr_lane, int key0, int keys_end, float c) {
+    constexpr int kAll = 6 * kSteps, kAhead = 2;
+    int last[2];
+    f32x4 s_acc[4][2], dp_acc[4][2];   // [16 keys][16 queries]
+    bf16x8 from[kAll], dsf[4];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      last[qb] = min(pos + 16 * qb, keys_end - 1) - key0 - first_key;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        s_acc[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        dp_acc[kb][qb] = f32x4{-delta[qb], -delta[qb], -delta[qb], -delta[qb]};   // dP - delta comes out of the MFMA
+      }
+    }
+    auto fetch = [&](int i) {
+      const int j = i % (2 * kSteps);   // fragment of its product
+      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * (j / kSteps)) + j % kSteps / (D / 32) * L::kRows16 + L::column16(j % (D / 32)) * 2));
+      else from[i] = lds_tr16_at<D>(tr_lane + (kAt + L::rows(32 * (j / kSteps)) + j % kSteps * 32));
+    };
+    // element e of a lane's 32: 16 keys, 16 queries, key
+    auto probability = [&](int e) {
+      const int kb = e / 8, qb = e / 4 % 2;
+      float s = s_acc[kb][qb][e % 4];
+      if (!kPlain && 16 * kb + e % 4 > last[qb]) s = -INFINITY;   // exp2(-inf) = 0
+      s_acc[kb][qb][e % 4] = fast_exp2(s * c - lse2[qb]);
+    };
+    auto ds = [&](int e) {
+      const int kb = e / 8, qb = e / 4 % 2;
+      dp_acc[kb][qb][e % 4] = s_acc[kb][qb][e % 4] * dp_acc[kb][qb][e % 4];
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) fetch(i);
+    __builtin_amdgcn_sched_barrier(0);
+    each_load<2 * kAll>([&](auto which) __attribute__((always_inline)) {   // the MFMAs: every fragment has one for each 16 queries
+      constexpr int m = decltype(which)::value, i = m / 2, qb = m % 2, j = i % (2 * kSteps), kb = j / (D / 32), s = j % (D / 32);
+      if constexpr (qb == 0 && i + kAhead < kAll) fetch(i + kAhead);
+      if constexpr (i < 2 * kSteps) s_acc[kb][qb] = mfma16(from[i], qf[qb][s], s_acc[kb][qb]);
+      else if constexpr (i < 4 * kSteps) dp_acc[kb][qb] = mfma16(from[i], dof[qb][s], dp_acc[kb][qb]);
+      else dq[j % kSteps][qb] = mfma16(from[i], dsf[j / kSteps * 2 + qb], dq[j % kSteps][qb]);
+      // exp2 from the first 16 keys' S on, dS from the first 32 keys' dP on
+      constexpr int kExp = kSteps, kDs = 6 * kSteps, kEnd = 19 * kSteps / 2;
+      if constexpr (m >= kExp && m < kDs) {
+#pragma unroll
+        for (int e = (m - kExp) * 32 / (kDs - kExp); e < (m + 1 - kExp) * 32 / (kDs - kExp); ++e) probability(e);
+      } else if constexpr (m >= kDs && m < kEnd) {
+        constexpr int from_e = (m - kDs) * 32 / (kEnd - kDs), to_e = (m + 1 - kDs) * 32 / (kEnd - kDs);
+#pragma unroll
+        for (int e = from_e; e < to_e; ++e) ds(e);
+        each_load<4>([&](auto operand) __attribute__((always_inline)) {   // 32 keys, 16 queries
+          constexpr int at = decltype(operand)::value, last_e = at / 2 * 16 + 12 + at % 2 * 4;   // (all before it and its 4 are there)
+          if constexpr (from_e < last_e && to_e >= last_e) dsf[at] = pack8(dp_acc[at / 2 * 2][at % 2], dp_acc[at / 2 * 2 + 1][at % 2]);
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+};
+// the wave's 32 dQ rows leave through its piece of LDS as whole lines
+__device__ __forceinline__ int dq_position(const BwdParams& p, int row) { return row < p.a.Sq ? p.rope.q_pos0 + row : 0; }
+template <int D>
+__device__ __forceinline__ void dq_unrotate(const BwdParams& p, f32x16 (&dq)[D / 32], int row0, int lane) {
+  rope_unrotate_acc<D>(dq, p.rope, dq_position(p, row0 + lane % 32), lane / 32);
+}
+template <int D>
+__device__ __forceinline__ void dq_unrotate(const BwdParams& p, f32x4 (&dq)[D / 16][2], int row0, int lane) {
+  const int pos[2] = {dq_position(p, row0 + lane % 16), dq_position(p, row0 + 16 + lane % 16)};
+  rope_unrotate_acc<D>(RowPair<0, D / 16, 2>{dq}, p.rope, pos, lane);
+}
+template <int N>
+__device__ __forceinline__ const f32x16 (&rows_of(f32x16 (&acc)[N]))[N] { return acc; }
+template <int N>
+__device__ __forceinline__ RowPair<0, N, 2> rows_of(f32x4 (&acc)[N][2]) { return {acc}; }
+template <int D, typename Acc>
+__device__ __forceinline__ void dq_store(const BwdParams& p, unsigned char* region, Acc& dq, int b, int hq, int row0, int lane) {
   const AttnParams& a = p.a;
-  const int qrow = row0 + lane % 32, h = lane / 32;
   const int64_t off = b * p.dqs[0] + hq * p.dqs[1] + static_cast<int64_t>(row0) * p.dqs[2];
-  if (p.rope.cos != nullptr) rope_unrotate_acc<D>(dq, p.rope, qrow < a.Sq ? p.rope.q_pos0 + qrow : 0, h);
+  if (p.rope.cos != nullptr) dq_unrotate<D>(p, dq, row0, lane);
   if (p.dq_f32)
-    wave_store_rows<D, true>(region, dq, a.sm_scale, static_cast<float*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, p.dq_accumulate, false);
+    wave_store_rows<D, true>(region, rows_of(dq), a.sm_scale, static_cast<float*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, p.dq_accumulate, false);
   else
-    wave_store_rows<D, false>(region, dq, a.sm_scale, static_cast<__bf16*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, false, kStreamGrads);
+    wave_store_rows<D, false>(region, rows_of(dq), a.sm_scale, static_cast<__bf16*>(p.dq) + off, p.dqs[2], a.Sq - row0, lane, false, kStreamGrads);
 }
 
 template <int D, int NW, int KT, bool kDelta, int KS, bool kCut>
 __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) void attn_bwd_dq_kernel(const BwdParams p) {
   using C = DqCfg<D, NW, KT, KS>;
   using L = TileLayout<D>;
+  using W = DqWave<D, C::kSmall>;
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
@@ -822,7 +1066,6 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   const int q0 = qtile * BM;
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);   // (a scalar: the buffer windows below are built in scalar registers)
-  const int n = lane % 32, h = lane / 32;
   const int qw = wave % C::kQWaves, ks = wave / C::kQWaves;   // which queries, which 64-key step of a staged tile
   const float c = a.sm_scale * kLog2e;
 
@@ -870,52 +1113,12 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
     if (ntiles > 0) request_tile(0);
   }
 
-  // ---- per-lane query: Q and dO fragments (B operands: fetched row-major, turned into fragments through the
+  // ---- the wave's queries: Q and dO fragments (B operands: fetched row-major, turned into fragments through the
   //      wave's piece of LDS; the tile buffers are filled only after the barrier below), lse and delta
-  const int qrow = q0 + qw * 32 + n;
-  const bool qlive = qrow < a.Sq;
-  bf16x8 qf[D / 16], dof[D / 16];
-  float lse2 = INFINITY, delta = 0.f;
-  {
-    const int row0 = q0 + qw * 32;
-    WaveTile<D> qt, dt;
-    qt.issue(make_buffer(a.q + b * a.qs[0] + hq * a.qs[1] + static_cast<int64_t>(row0) * a.qs[2],
-                         span_bytes(a.Sq - row0, a.qs[2], D)), a.qs[2], lane);
-    dt.issue(make_buffer(p.dout + b * a.os[0] + hq * a.os[1] + static_cast<int64_t>(row0) * a.os[2],
-                         span_bytes(a.Sq - row0, a.os[2], D)), a.os[2], lane);
-    WaveTile<D> ot;
-    if constexpr (kDelta)
-      ot.issue(make_buffer(p.out + b * a.os[0] + hq * a.os[1] + static_cast<int64_t>(row0) * a.os[2],
-                           span_bytes(a.Sq - row0, a.os[2], D)), a.os[2], lane);
-    const int64_t gi = (static_cast<int64_t>(b) * a.Hq + hq) * a.Sq + qrow;
-    if (qlive) {
-      const float l = p.lse[gi];
-      lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;  // a row that saw no key contributes nothing
-      if constexpr (!kDelta) delta = p.delta[gi];
-    }
-    unsigned char* region = smem_raw + C::kFragments + wave * WaveTile<D>::kRegionBytes;
-    qt.fragments(region, lane, qf);
-    dt.fragments(region, lane, dof);
-    if constexpr (kDelta) {
-      // delta = sum_d dO * O of the lane's row (context_parallel.py:145): each half of the wave holds half of the
-      // row's columns in its fragments; the dK/dV kernel, launched after this one, reads the result from memory
-      bf16x8 of[D / 16];
-      ot.fragments(region, lane, of);
-      float part = 0.f;
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) part += static_cast<float>(dof[s][e]) * static_cast<float>(of[s][e]);
-      delta = half_sum(part);
-      if (qlive && h == 0 && ks == 0 && piece.part == 0) p.delta_w[gi] = delta;
-    }
-  }
-
-  f32x16 dq[D / 32];
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dq[db][i] = 0.f;
+  W w;
+  w.template load<kDelta>(p, smem_raw + C::kFragments + wave * WaveTile<D>::kRegionBytes, (static_cast<int64_t>(b) * a.Hq + hq) * a.Sq, b, hq,
+                          q0 + qw * 32, ks == 0 && piece.part == 0, lane);
+  W::clear(w.dq);
 
   if constexpr (!C::kBehind) {
     __syncthreads();  // every wave has its Q / dO fragments: the tile buffers may be filled
@@ -931,7 +1134,7 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   auto unmasked_end = [&](int end) { return min(a.causal ? blk_q_lo + 1 : end, end) - BN * (ks + 1); };
   int plain = unmasked_end(a.Sk);
   plain = plain >= 0 ? min(plain / KT + 1, mine) : 0;
-  uint32_t row_at = L::row_place(lane), v_row_at = 2 * C::kSideBytes + L::row_place(lane), tr_at = L::column_place(lane);
+  uint32_t row_at = W::row_place(lane), v_row_at = 2 * C::kSideBytes + W::row_place(lane), tr_at = W::column_place(lane);
   asm volatile("" : "+v"(row_at), "+v"(v_row_at), "+v"(tr_at), "+s"(mine), "+s"(plain));   // (kept, not computed again in front of the reads)
   late.arrive();
   // all loads so far are complete, the first tile among them (the barrier publishes it); stating it also keeps a
@@ -939,7 +1142,6 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
 
-  const int qpos = a.causal ? a.q_offset + qrow : 0x7fffffff;
   // a trip on the LDS buffer `parity`, a constant, so that a lane's addresses are the same in every trip (kCut, whose runs of tiles begin
   // anywhere: on buffer t % 2)
   auto trip = [&](auto parity, auto plain_c, int t) __attribute__((always_inline)) {
@@ -950,57 +1152,9 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
     const int tile_key0 = kCut ? pos.key0 : t * KT, keys_end = kCut ? pos.end : a.Sk;
     if constexpr (kCut) pos.next(a.kv, KT);
     if (t + 1 < ntiles) request_tile(kCut ? 1 - t % 2 : 1 - decltype(parity)::value);
-    // Straight-line code in an order that lets the wave's own phases overlap: exp2 needs S alone and is dealt out between the MFMAs of S
-    // (second 32 keys) and dP, dS between those of dP and dQ (first 32).  The fragments are requested kAhead MFMAs ahead and the scheduling
-    // barriers keep the order.  Forward and backward, us: B1 H4 S3000 D64 83.0 -> 81.8, B1 H32 S512 D64 49.6 -> 48.5, B1 H4 S3000 D128 85.8 -> 84,
-    // B2 H32 S1024 D64 71.3 -> 70.5; four MFMAs ahead is level.  Masked trips go by it as well (in the compiler's order every MFMA waited for an LDS
-    // round trip): dQ alone B1 H8 S293 D64 8.0 -> 7.6, B4 H4/1 S1287 D128 29.2 -> 28.7.
-    constexpr int kSteps = D / 16, kAll = 6 * kSteps, kAhead = 2;
     static_assert(KT == BN * KS && BN == 64);
     const uint32_t step_at = moved + (KS > 1 ? static_cast<uint32_t>(ks) * L::kRows64 : 0);
-    const uint32_t row_lane = row_at + step_at, v_row_lane = v_row_at + step_at, tr_lane = tr_at + step_at;
-    // keys past the diagonal or the end of their chunk are masked (the rows read past a chunk are zero, but P of a zero score need
-    // not be finite beside a very negative lse): one compare with a constant per element
-    const int last = (qpos < keys_end ? qpos : keys_end - 1) - (tile_key0 + BN * ks) - 4 * h;
-    f32x16 s_acc[2], dp_acc[2];
-    bf16x8 from[kAll], dsf[4];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) { s_acc[mb][i] = 0.f; dp_acc[mb][i] = -delta; }   // dP - delta comes out of the MFMA
-    auto fetch = [&](int i) {
-      const int j = i % (2 * kSteps), mb = j / kSteps;   // MFMA of its product, 32-key block
-      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * mb) + j % kSteps * 32));
-      else from[i] = lds_tr_at<D>(tr_lane + (kAt + L::rows(32 * mb) + j % kSteps / (D / 32) * L::kRows16 + j % (D / 32) * 64));
-    };
-    auto probability = [&](int e) {
-      float s = s_acc[e / 16][e % 16];
-      if (!kPlain && 32 * (e / 16) + 8 * (e % 16 / 4) + e % 4 > last) s = -INFINITY;   // exp2(-inf) = 0
-      s_acc[e / 16][e % 16] = fast_exp2(s * c - lse2);
-    };
-    auto ds = [&](int e) { dp_acc[e / 16][e % 16] = s_acc[e / 16][e % 16] * dp_acc[e / 16][e % 16]; };
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) fetch(i);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < kAll; ++i) {
-      const int j = i % (2 * kSteps), mb = j / kSteps, s = j % kSteps;
-      if (i + kAhead < kAll) fetch(i + kAhead);
-      if (i < 2 * kSteps) s_acc[mb] = mfma32(from[i], qf[s], s_acc[mb]);
-      else if (i < 4 * kSteps) dp_acc[mb] = mfma32(from[i], dof[s], dp_acc[mb]);
-      else dq[j % (D / 32)] = mfma32(from[i], dsf[j / (D / 32)], dq[j % (D / 32)]);
-      if (i >= kSteps && i < 4 * kSteps) {
-#pragma unroll
-        for (int e = (i - kSteps) * 32 / (3 * kSteps); e < (i + 1 - kSteps) * 32 / (3 * kSteps); ++e) probability(e);
-      }
-      if (i >= 3 * kSteps && i < 5 * kSteps) {
-#pragma unroll
-        for (int e = (i - 3 * kSteps) * 16 / kSteps; e < (i + 1 - 3 * kSteps) * 16 / kSteps; ++e) ds(e);
-        const int done = (i + 1 - 3 * kSteps) * 16 / kSteps;
-        if (done % 8 == 0) dsf[done / 8 - 1] = pack8(dp_acc[(done / 8 - 1) / 2], (done / 8 - 1) % 2 * 8);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    w.template trip<kAt, kPlain>(row_at + step_at, v_row_at + step_at, tr_at + step_at, tile_key0 + BN * ks, keys_end, c);
     wait_requests<0>();
     __syncthreads();
   };
@@ -1037,35 +1191,23 @@ __global__ __launch_bounds__(64 * NW, (DqCfg<D, NW, KT, KS>::kPerCu * NW / 4)) v
   //      (the loop ended on a barrier: the tile buffers are free; the store pieces used below lie in front of the
   //      exchange areas of the ks > 0 waves)
   if constexpr (KS > 1) {
-    float* xo = reinterpret_cast<float*>(smem_raw + wave * C::kExchangeBytes);
-    if (ks > 0) {
-#pragma unroll
-      for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) xo[(db * 16 + i) * 64 + lane] = dq[db][i];
-    }
+    if (ks > 0) put_acc(reinterpret_cast<float*>(smem_raw + wave * C::kExchangeBytes), w.dq, lane);
     __syncthreads();
     if (ks > 0) return;
 #pragma unroll
-    for (int j = 1; j < KS; ++j) {
-      const float* oo = reinterpret_cast<const float*>(smem_raw + (qw + j * C::kQWaves) * C::kExchangeBytes);
-#pragma unroll
-      for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dq[db][i] += oo[(db * 16 + i) * 64 + lane];
-    }
+    for (int j = 1; j < KS; ++j) add_acc(w.dq, reinterpret_cast<const float*>(smem_raw + (qw + j * C::kQWaves) * C::kExchangeBytes), lane);
     static_assert(kRowRegionBytes <= C::kExchangeBytes, "store pieces lie below the exchange areas read above");
   }
 
   if (kCut && piece.parts > 1) {   // one piece of several: the sums leave as they are
-    put_acc<D / 32>(a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * dq_piece_floats(D), dq, lane);
+    put_acc(a.pieces.ws + ((static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * C::kQWaves + qw) * dq_piece_floats(D), w.dq, lane);
     return;
   }
-  dq_store<D>(p, smem_raw + wave * kRowRegionBytes, dq, b, hq, q0 + qw * 32, lane);
+  dq_store<D>(p, smem_raw + wave * kRowRegionBytes, w.dq, b, hq, q0 + qw * 32, lane);
 }
 
 // The pieces of every cut query tile put together (see attn_bwd_dkdv_join_kernel).
-template <int D, int QW, int KT>
+template <int D, int QW, int KT, bool kSmall>
 __global__ __launch_bounds__(64 * QW) void attn_bwd_dq_join_kernel(const BwdParams p, const int pieces_per_head) {
   __shared__ __attribute__((aligned(16))) unsigned char smem_raw[QW * kRowRegionBytes];
   const AttnParams& a = p.a;
@@ -1079,19 +1221,9 @@ __global__ __launch_bounds__(64 * QW) void attn_bwd_dq_join_kernel(const BwdPara
   const int64_t first = static_cast<int64_t>(blockIdx.x) * pieces_per_head + first_piece(tile, a.pieces.len, trips_of);
   const float* src = a.pieces.ws + (first * QW + wave) * dq_piece_floats(D);
   constexpr int64_t kStep = static_cast<int64_t>(QW) * dq_piece_floats(D);
-  f32x16 dq[D / 32];
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dq[db][i] = 0.f;
-  for (int j = 0; j < parts; ++j) {
-    f32x4 raw[D / 32][4];
-    get_acc<D / 32>(src + j * kStep, raw, lane);
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dq[db][i] += raw[db][i / 4][i % 4];
-  }
+  decltype(DqWave<D, kSmall>::dq) dq;
+  DqWave<D, kSmall>::clear(dq);
+  for (int j = 0; j < parts; ++j) add_acc(dq, src + j * kStep, lane);
   dq_store<D>(p, smem_raw + wave * kRowRegionBytes, dq, b, hq, (n_qtiles - 1 - tile) * BM + wave * 32, lane);
 }
 
@@ -1228,7 +1360,7 @@ int launch_dq_impl(const BwdParams& p, hipStream_t s) {
   const int n = count_pieces(n_qtiles, len, [&](int i) { return query_tile_trips(p.a, n_qtiles - 1 - i, C::BM, KT); });
   hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NW, KT, kDelta, KS, kCut>), dim3(heads, n), dim3(C::kThreads), C::kLdsBytes, s, p);
   if (kCut && len > 0)
-    hipLaunchKernelGGL((attn_bwd_dq_join_kernel<D, C::kQWaves, KT>), dim3(heads, n_qtiles), dim3(64 * C::kQWaves), 0, s, p, n);
+    hipLaunchKernelGGL((attn_bwd_dq_join_kernel<D, C::kQWaves, KT, C::kSmall>), dim3(heads, n_qtiles), dim3(64 * C::kQWaves), 0, s, p, n);
   return PICO_OK;
 }
 

@@ -25,6 +25,9 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
 
 // 4 rows x 1 column of a row-major bf16 tile in LDS, transposed into the lane (see header comment).
 // `p` must point at tile[row0 + (lane%16)/4][col0 + 4*(lane%4)].
@@ -134,6 +137,18 @@ struct TileLayout {
   // ... and for transposing reads: row 4 (lane / 32) + lane % 16 / 4, columns 16 (lane / 16 % 2) + 4 (lane % 4) ..+3 (64 bytes further:
   // the next 32 columns)
   static __device__ __forceinline__ uint32_t column_place(int lane) { return place(4 * (lane / 32) + lane % 16 / 4) + lane / 16 % 2 * 32 + lane % 4 * 8; }
+  // For products of 16 x 16 x 32, whose results have rows 4 (lane / 16) ..+3 in a lane: there the four groups of lanes stand for the rows from
+  // 0, 8, 4 and 12, so that the 32 lanes of a transposing read, which fetch 8 rows x 32 bytes, have no bank conflicts (rows 0 .. 7 would share banks
+  // in twos).  A 16-byte read is taken 16 lanes at a time, lanes 0-3, 12-15, 20-27 and 4-11, 16-19, 28-31 of each half: it has none if lanes 16 apart
+  // read columns 32 apart, so a fragment's 32 columns of the contraction are 0-7, 32-39, 8-15, 40-47 (the next one's 16 further on), in both operands.
+  // (With 32 consecutive columns every such read took eight cycles instead of four.)
+  static __device__ __forceinline__ int group_row(int group) { return group % 2 * 8 + group / 2 * 4; }
+  static __device__ __forceinline__ int group_column(int group) { return group % 2 * 32 + group / 2 * 8; }
+  static constexpr int column16(int s) { return s / 2 * 64 + s % 2 * 16; }   // fragment s: columns column16(s) + group_column(lane / 16) ..+7
+  // the lane's row of a read by rows; the first of its rows in a result is group_row(lane / 16); and of a transposing read, columns 4 (lane % 4) ..+3
+  // (32 bytes further: the next 16 columns)
+  static __device__ __forceinline__ uint32_t row_place16(int lane) { return place(group_row(lane / 4 % 4) + lane % 4) + group_column(lane / 16) * 2; }
+  static __device__ __forceinline__ uint32_t column_place16(int lane) { return place(group_row(lane / 16) + lane % 16 / 4) + lane % 4 * 8; }
 };
 // LDS at a byte offset (the kernels' LDS starts at 0, see request16): through a pointer to the array the compiler adds its address,
 // which it does not know to be 0, to every lane offset
@@ -146,6 +161,15 @@ template <int D>
 __device__ __forceinline__ bf16x8 lds_tr_at(uint32_t off) {
   const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off));
   const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off + TileLayout<D>::kRows8));
+  typedef __attribute__((ext_vector_type(8))) short s16x8;
+  return __builtin_bit_cast(bf16x8, static_cast<s16x8>(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
+}
+
+// ... of a 16 x 16 x 32 product: 16 rows at `off`, 4 of each lane, and the 16 rows after them
+template <int D>
+__device__ __forceinline__ bf16x8 lds_tr16_at(uint32_t off) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(off + TileLayout<D>::kRows16));
   typedef __attribute__((ext_vector_type(8))) short s16x8;
   return __builtin_bit_cast(bf16x8, static_cast<s16x8>(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
 }
@@ -166,6 +190,13 @@ __device__ __forceinline__ bf16x8 pack8(const f32x16& c, int base) {
   return r;
 }
 
+__device__ __forceinline__ bf16x8 pack8(const f32x4& lo, const f32x4& hi) {
+  bf16x8 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { r[e] = static_cast<__bf16>(lo[e]); r[4 + e] = static_cast<__bf16>(hi[e]); }
+  return r;
+}
+
 // max / sum of a value across the two 32-lane halves of a wave (lane l with lane l^32)
 __device__ __forceinline__ float half_max(float v) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -174,6 +205,16 @@ __device__ __forceinline__ float half_max(float v) {
 __device__ __forceinline__ float half_sum(float v) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// ... across the four groups of 16 lanes (lanes l, l^16, l^32, l^48)
+__device__ __forceinline__ float group_max(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return half_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float group_sum(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return half_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
 // ---- reading a wave's 32 x D operand tile as MFMA fragments.  Fetched straight in fragment layout (lane =
@@ -186,24 +227,37 @@ struct WaveTile {
   static constexpr int kChunks = D / 16;                 // 16-byte pieces per lane
   static constexpr int kRegionBytes = 32 * (D + 8) * 2;
   u32x4 raw[kChunks];
+  template <int kSecond = 16>   // where the second 16 rows are, counted from the first
   __device__ __forceinline__ void issue(buffer_rsrc window, int64_t row_stride, int lane) {
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
-      const int idx = lane + 64 * i, r = idx / (D / 8), cv = idx % (D / 8);
+      const int idx = lane + 64 * i, r = idx / (D / 8) + (2 * i >= kChunks ? kSecond - 16 : 0), cv = idx % (D / 8);
       raw[i] = buffer_load_b128(window, static_cast<uint32_t>((static_cast<int64_t>(r) * row_stride + cv * 8) * 2));
     }
   }
-  __device__ __forceinline__ void fragments(unsigned char* region, int lane, bf16x8 (&frag)[D / 16]) const {
-    constexpr int kPitch = (D + 8) * 2;
+  static constexpr int kPitch = (D + 8) * 2;
+  __device__ __forceinline__ void put(unsigned char* region, int lane) const {
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
       const int idx = lane + 64 * i, r = idx / (D / 8), cv = idx % (D / 8);
       *reinterpret_cast<u32x4*>(region + r * kPitch + cv * 16) = raw[i];
     }
+  }
+  __device__ __forceinline__ void fragments(unsigned char* region, int lane, bf16x8 (&frag)[D / 16]) const {
+    put(region, lane);
     const int n = lane % 32, h = lane / 32;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s)
       frag[s] = *reinterpret_cast<const bf16x8*>(region + n * kPitch + (16 * s + 8 * h) * 2);
+  }
+  // ... of 16 x 16 x 32 products: frag[b][s] holds row 16 b + lane % 16, eight columns as TileLayout says
+  __device__ __forceinline__ void fragments16(unsigned char* region, int lane, bf16x8 (&frag)[2][D / 32]) const {
+    put(region, lane);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int s = 0; s < D / 32; ++s)
+        frag[b][s] = *reinterpret_cast<const bf16x8*>(region + (16 * b + lane % 16) * kPitch + (TileLayout<D>::column16(s) + TileLayout<D>::group_column(lane / 16)) * 2);
   }
 };
 
@@ -217,39 +271,56 @@ struct WaveTile {
 //   accumulate (fp32 only) adds to what is there; all its reads are issued before the first write.
 //   streaming marks bf16 stores non-temporal (the data is not read again by the kernels that follow soon).
 constexpr int kRowRegionBytes = 32 * 144;
-template <int D, bool kF32>
-__device__ __forceinline__ void wave_store_rows(unsigned char* region, const f32x16 (&acc)[D / 32], float scale,
+// columns c0 .. c0 + kCols - 1 of the 32 rows, scaled, to the wave's piece of LDS
+template <bool kF32>
+__device__ __forceinline__ void put_columns(unsigned char* region, int row, int col, f32x4 v4, float scale) {
+  if constexpr (kF32) {
+    *reinterpret_cast<f32x4*>(region + row * 144 + col * 4) = f32x4{v4[0] * scale, v4[1] * scale, v4[2] * scale, v4[3] * scale};
+  } else {
+    bf16x4 b4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) b4[t] = static_cast<__bf16>(v4[t] * scale);
+    *reinterpret_cast<bf16x4*>(region + row * 144 + col * 2) = b4;
+  }
+}
+template <bool kF32, int kCols, int N>   // products of 32 x 32
+__device__ __forceinline__ void put_rows(unsigned char* region, const f32x16 (&acc)[N], float scale, int c0, int lane) {
+#pragma unroll
+  for (int db = c0 / 32; db < (c0 + kCols) / 32; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      put_columns<kF32>(region, lane % 32, 32 * db + 8 * j + 4 * (lane / 32) - c0,
+                        f32x4{acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]}, scale);
+}
+// of 16 x 16: acc[db][kFrom + b] holds row 16 b + lane % 16, columns 16 db + 4 (lane / 16) ..+3
+template <int kFrom, int N, int M>
+struct RowPair {
+  f32x4 (&acc)[N][M];
+};
+template <bool kF32, int kCols, int kFrom, int N, int M>
+__device__ __forceinline__ void put_rows(unsigned char* region, const RowPair<kFrom, N, M>& rows, float scale, int c0, int lane) {
+#pragma unroll
+  for (int db = c0 / 16; db < (c0 + kCols) / 16; ++db)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) put_columns<kF32>(region, 16 * b + lane % 16, 16 * db + 4 * (lane / 16) - c0, rows.acc[db][kFrom + b], scale);
+}
+// (kSecond: where the second 16 rows are, counted from the first)
+template <int D, bool kF32, int kSecond = 16, typename Acc>
+__device__ __forceinline__ void wave_store_rows(unsigned char* region, const Acc& acc, float scale,
                                                 void* dst_row0, int64_t row_stride, int rows_live, int lane,
                                                 bool accumulate, bool streaming) {
   constexpr int kPitch = 144;
   constexpr int kColsPerPass = kF32 ? 32 : 64;
-  const int n = lane % 32, h = lane / 32;
 #pragma unroll
   for (int c0 = 0; c0 < D; c0 += kColsPerPass) {
-#pragma unroll
-    for (int db = c0 / 32; db < (c0 + kColsPerPass) / 32; ++db)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = 32 * db + 8 * j + 4 * h - c0;
-        if constexpr (kF32) {
-          f32x4 v4;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) v4[t] = acc[db][4 * j + t] * scale;
-          *reinterpret_cast<f32x4*>(region + n * kPitch + col * 4) = v4;
-        } else {
-          bf16x4 v4;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) v4[t] = static_cast<__bf16>(acc[db][4 * j + t] * scale);
-          *reinterpret_cast<bf16x4*>(region + n * kPitch + col * 2) = v4;
-        }
-      }
+    put_rows<kF32, kColsPerPass>(region, acc, scale, c0, lane);
     // 32 rows x 8 pieces of 16 bytes = 4 pieces per lane; 8 consecutive lanes cover one row's line
     unsigned char* g[4];
     u32x4 v[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int idx = lane + 64 * t, r = idx / 8, ch = idx % 8;
-      v[t] = *reinterpret_cast<const u32x4*>(region + r * kPitch + ch * 16);
+      const int idx = lane + 64 * t, ch = idx % 8, r = idx / 8 + t / 2 * (kSecond - 16);
+      v[t] = *reinterpret_cast<const u32x4*>(region + idx / 8 * kPitch + ch * 16);
       g[t] = r < rows_live ? static_cast<unsigned char*>(dst_row0) +
                                  (static_cast<int64_t>(r) * row_stride + c0) * (kF32 ? 4 : 2) + ch * 16
                            : nullptr;
@@ -280,30 +351,22 @@ __device__ __forceinline__ void wave_store_rows(unsigned char* region, const f32
 // The same rows as the sum of an fp32 buffer and the accumulators, rounded once to bf16 and written somewhere else:
 // the last block of a ring adds itself to the travelling fp32 sums (`old_row0`, nullptr: nothing to add) and hands
 // the total back in the dtype of the inputs.  32 columns per pass (fp32 staging), 8-byte bf16 pieces per lane.
-template <int D>
-__device__ __forceinline__ void wave_store_rows_total(unsigned char* region, const f32x16 (&acc)[D / 32], float scale,
+template <int D, int kSecond = 16, typename Acc>
+__device__ __forceinline__ void wave_store_rows_total(unsigned char* region, const Acc& acc, float scale,
                                                       const float* old_row0, int64_t old_stride, __bf16* dst_row0,
                                                       int64_t dst_stride, int rows_live, int lane) {
   constexpr int kPitch = 144;
-  const int n = lane % 32, h = lane / 32;
 #pragma unroll
   for (int c0 = 0; c0 < D; c0 += 32) {
-    const int db = c0 / 32;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f32x4 v4;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) v4[t] = acc[db][4 * j + t] * scale;
-      *reinterpret_cast<f32x4*>(region + n * kPitch + (8 * j + 4 * h) * 4) = v4;
-    }
+    put_rows<true, 32>(region, acc, scale, c0, lane);
     f32x4 v[4], old[4];
     int row[4], piece[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int idx = lane + 64 * t;
-      row[t] = idx / 8;
+      row[t] = idx / 8 + t / 2 * (kSecond - 16);
       piece[t] = idx % 8;
-      v[t] = *reinterpret_cast<const f32x4*>(region + row[t] * kPitch + piece[t] * 16);
+      v[t] = *reinterpret_cast<const f32x4*>(region + idx / 8 * kPitch + piece[t] * 16);
       old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (old_row0 != nullptr && row[t] < rows_live)
         old[t] = *reinterpret_cast<const f32x4*>(old_row0 + static_cast<int64_t>(row[t]) * old_stride + c0 + piece[t] * 4);
@@ -387,6 +450,26 @@ __device__ __forceinline__ void rope_unrotate_acc(f32x16 (&acc)[D / 32], const R
     }
 }
 
+// ... of 16 x 16 products, whose rows are at positions pos[b]
+template <int D, int kFrom, int N, int M>
+__device__ __forceinline__ void rope_unrotate_acc(const RowPair<kFrom, N, M>& rows, const RopeArgs& r, const int (&pos)[2], int lane) {
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      f32x4 &first = rows.acc[db][kFrom + b], &second = rows.acc[db + D / 32][kFrom + b];
+      float c[4], sn[4];
+      rope_load<4>(r, r.cos, pos[b], 16 * db + 4 * (lane / 16), c);
+      rope_load<4>(r, r.sin, pos[b], 16 * db + 4 * (lane / 16), sn);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float lo = first[t], hi = second[t];
+        first[t] = lo * c[t] + hi * sn[t];
+        second[t] = hi * c[t] - lo * sn[t];
+      }
+    }
+}
+
 // K / V as a list of equally long chunks that lie one after another along the key axis: key j of the launch is row
 // j % len of chunk j / len.  One chunk of len = Sk is the plain case.  A staged key tile belongs to one chunk: with a len
 // that is no multiple of the tile the last tile of every chunk is a partial one (its rows past the chunk read as zeros and
@@ -421,6 +504,13 @@ struct AttnParams {
 
 __host__ __device__ inline int pieces_of(int trips, int len) { return len <= 0 || trips <= len ? 1 : (trips + len - 1) / len; }
 
+// The lane, counted anew where it is used: kept in a register (threadIdx is one) it costs the kernels that need all of theirs.
+__device__ __forceinline__ int lane_here() {
+  uint32_t all = ~0u;
+  asm volatile("" : "+s"(all));
+  return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
 // Which (tile, piece) workgroup `y` of a head is, tiles in order, and how many pieces its tile has.  64 tiles at a time, one
 // per lane: a prefix sum over their numbers of pieces and a ballot.  All lanes of the wave take part.
 struct Piece {
@@ -428,7 +518,7 @@ struct Piece {
 };
 template <typename F>
 __device__ __forceinline__ Piece find_piece(int y, int n_tiles, int len, const F& trips_of) {
-  const int lane = threadIdx.x % kWave;
+  const int lane = lane_here();
   for (int base = 0; base < n_tiles; base += kWave) {
     const int mine = base + lane < n_tiles ? pieces_of(trips_of(base + lane), len) : 0;
     int sum = mine;
@@ -605,6 +695,40 @@ __device__ __forceinline__ void get_acc(const float* src, f32x4 (&raw)[N][4], in
   for (int db = 0; db < N; ++db)
 #pragma unroll
     for (int j = 0; j < 4; ++j) raw[db][j] = *reinterpret_cast<const f32x4*>(src + ((db * 4 + j) * kWave + lane) * 4);
+}
+
+template <int N, int M>   // of 16 x 16 products
+__device__ __forceinline__ void put_acc(float* dst, const f32x4 (&acc)[N][M], int lane) {
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int b = 0; b < M; ++b) *reinterpret_cast<f32x4*>(dst + ((db * M + b) * kWave + lane) * 4) = acc[db][b];
+}
+template <int N, int M>
+__device__ __forceinline__ void get_acc(const float* src, f32x4 (&raw)[N][M], int lane) {
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int b = 0; b < M; ++b) raw[db][b] = *reinterpret_cast<const f32x4*>(src + ((db * M + b) * kWave + lane) * 4);
+}
+// what put_acc left, added
+template <int N>
+__device__ __forceinline__ void add_acc(f32x16 (&acc)[N], const float* src, int lane) {
+  f32x4 raw[N][4];
+  get_acc<N>(src, raw, lane);
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[db][i] += raw[db][i / 4][i % 4];
+}
+template <int N, int M>
+__device__ __forceinline__ void add_acc(f32x4 (&acc)[N][M], const float* src, int lane) {
+  f32x4 raw[N][M];
+  get_acc(src, raw, lane);
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+#pragma unroll
+    for (int b = 0; b < M; ++b) acc[db][b] += raw[db][b];
 }
 
 // How many key tiles of KT keys lie in front of position `end`, counted chunk by chunk.

@@ -231,3 +231,27 @@ def test_dq_on_both_sides_of_the_lines_at_head_dim_128(device, B, Hq, Hkv, Sq, S
             part = slice(h * group, (h + 1) * group)
             want = reference(q[b:b + 1, part], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], scale, q_offset, causal, do[b:b + 1, part])
             assert rel_l2(dq[b:b + 1, part], want[2]) <= 1e-2, (b, h)
+
+
+# head_dim 128: gradients of rotated q and k, added to what is there, of eight and of four waves
+@pytest.mark.parametrize("B,Hq,Hkv,S,waves", [(8, 16, 16, 1000, 8), (11, 32, 16, 417, 8), (1, 4, 2, 300, 4)])
+def test_gradients_leave_unrotated_and_added_at_head_dim_128(device, B, Hq, Hkv, S, waves):
+    """The rotation's backward and the sum in the kernels' epilogues equal the two on their fp32 results: eight roundings of products of
+    two elements of a pair, and the sum's."""
+    from picotron_amd import ops
+    assert plan("dq", B, Hq, S, S, True, 0, Hkv=Hkv)[0] == waves
+    q, k, v, do = inputs(device, B, Hq, Hkv, S, S, 128)
+    scale = 1 / math.sqrt(128)
+    cos, sin = (t.to(device) for t in OL.get_cos_sin(S + 5, 128, 10000.0, torch.float32))
+    out, lse = ops.attn_fwd(q, k, v, scale, True, 0)
+    plain = ops.attn_bwd(do, q, k, v, lse, None, scale, True, 0, out=out)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    bases = [torch.randn(t.shape, generator=g, device=device) for t in plain]
+    got = [t.clone() for t in bases]
+    ops.attn_bwd_rope(do, q, k, v, out, lse, cos, sin, scale, True, *got, 0, q_pos_offset=5, k_pos_offset=5, dq_accumulate=True, dkv_accumulate=True)
+    c, s = cos[5:5 + S, :64], sin[5:5 + S, :64]
+    for i, (a, b, base) in enumerate(zip(got, plain, bases)):
+        lo, hi = b[..., :64], b[..., 64:]
+        turned = b if i == 2 else torch.cat((lo * c + hi * s, hi * c - lo * s), -1)
+        size = (lo.abs() + hi.abs()).repeat(1, 1, 1, 2) + base.abs()
+        assert ((a - (base + turned)).abs() <= 9 * 2 ** -24 * size).all(), i
