@@ -308,6 +308,8 @@ int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int chunk_coun
  * take turns in the keys), plan[2] the key tiles of a piece where query tiles are cut (0: not cut).  PICO_ERR_SHAPE for a descriptor that has no launch. */
 int pico_attn_fwd_plan(const pico_attn_desc* desc, int chunk_count, int32_t* plan);
 int pico_attn_dq_plan(const pico_attn_desc* desc, int chunk_count, int32_t* plan);
+/* ... and dK/dV's: plan[0] keys of a key tile, plan[1] key tiles of a workgroup, plan[2] the trips of a piece where key tiles are cut (0: not cut). */
+int pico_attn_dkdv_plan(const pico_attn_desc* desc, int chunk_count, int32_t* plan);
 int pico_attn_fwd_chunks_ws(const pico_attn_desc* desc, const void* q, const pico_kv_chunks* kv, void* out, float* lse,
                             int out_dtype, int merge, const pico_rope_tables* rope, int q_pos_offset, void* q_rot,
                             const int64_t* q_rot_stride, void* workspace, int64_t workspace_bytes, void* stream);

@@ -66,6 +66,7 @@ SIGNATURES = {
     "pico_attn_bwd_workspace_bytes": (_I64, [POINTER(AttnDesc), c_int]),
     "pico_attn_fwd_plan": (c_int, [POINTER(AttnDesc), c_int, POINTER(c_int32)]),
     "pico_attn_dq_plan": (c_int, [POINTER(AttnDesc), c_int, POINTER(c_int32)]),
+    "pico_attn_dkdv_plan": (c_int, [POINTER(AttnDesc), c_int, POINTER(c_int32)]),
     "pico_attn_fwd_chunks_ws": (c_int, [POINTER(AttnDesc), _P, POINTER(KvChunks), _P, _P, c_int, c_int, POINTER(RopeTables), c_int, _P,
                                         POINTER(c_int64), _P, _I64, _P]),
     "pico_attn_bwd_chunks_ws": (c_int, [POINTER(AttnDesc), _P, POINTER(KvChunks), _P, _P, c_int, _P, _P, _P, POINTER(c_int64), c_int, c_int,

@@ -20,7 +20,7 @@ OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libpicotron_amd.so")
 HOST = os.path.join(HERE, "_host.so")
 
-SOURCES = ["common.hip", "norm.hip", "pointwise.hip", "optim.hip", "loss.hip", "embedding.hip", "product.hip", "product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip"]
+SOURCES = ["common.hip", "norm.hip", "pointwise.hip", "optim.hip", "loss.hip", "embedding.hip", "product.hip", "product_mid.hip", "product_large.hip", "attn_fwd.hip", "attn_bwd.hip", "attn_bwd_roles.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
     # packed fp32 VALU forms are kept out of the generated code on purpose
@@ -33,7 +33,7 @@ FLAGS = [
 # an addition per request).  And they wait for a count of their own memory operations: an access to scratch memory would be
 # counted with them, and the wait would end before what it waits for is there.
 REQUESTING = {"product_mid.hip": "_kernel", "product_large.hip": "_kernel", "attn_fwd.hip": "attn_fwd_kernel",
-              "attn_bwd.hip": "dkdv_kernel|dkdv_few_kernel|dq_kernel"}
+              "attn_bwd.hip": "dkdv_kernel|dkdv_few_kernel|dq_kernel", "attn_bwd_roles.hip": "roles_kernel"}
 RESOURCES = "-Rpass-analysis=kernel-resource-usage"
 
 

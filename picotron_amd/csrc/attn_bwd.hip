@@ -15,38 +15,14 @@
 //
 // Recomputing S and dP in the second kernel costs 2 of 7 MFMA products; a single-kernel version that
 // accumulated dQ with fp32 atomics was bound by the atomic rate of the memory system (measured).
-#include "attn_common.h"
+#include "attn_bwd.h"
 
 #include <type_traits>
 
 namespace pico {
 namespace {
 
-struct BwdParams {
-  AttnParams a;
-  const __bf16* dout;
-  const float* lse;
-  const float* delta;
-  const __bf16* out;   // fused-delta mode of the dQ kernel: the forward output, addressed like dout
-  float* delta_w;      //   ... and where that kernel writes delta = sum_d dO * O for the dK/dV kernel
-  void* dq;
-  void* dk[kMaxChunks];      // per K / V chunk; nullptr: that chunk's gradient is not wanted
-  void* dv[kMaxChunks];
-  __bf16* dk_final[kMaxChunks];   // per chunk, optional: the chunk's total (fp32 dk[c] if its accumulate bit is set, plus this
-  __bf16* dv_final[kMaxChunks];   //   launch's block) leaves here in bf16; dk[c] / dv[c] are only read
-  int64_t dkfs[3];                // element strides (b, h, s) of dk_final / dv_final
-  uint32_t dkv_accumulate;   // bit c: chunk c's dk / dv are added to (fp32)
-  int dq_f32, dq_accumulate;
-  int dkv_f32;
-  int pair_ktiles;                  // > 0: every workgroup does key tile blockIdx.y and this number - 1 - blockIdx.y
-  int64_t dqs[3];  // element strides (b, h, s) of dq
-  int64_t dks[3];  // element strides (b, h, s) of dk and dv
-  RopeArgs rope;   // rope.cos != nullptr: q and k are rotated tensors; dq and dk leave un-rotated (RoPE's backward)
-};
-
 // =====================================================================================  dK / dV
-// bf16 gradients leave with streaming (non-temporal) stores: nothing on this GPU reads them back soon
-constexpr bool kStreamGrads = true;
 // QS > 1: eight waves instead of four, QS of them own the same 32 keys and split every query tile between them, one
 // 32-query sub-block each, with accumulators of their own that are added through LDS at the end of the key tile.
 //   QS 2 (waves w and w + 4, which share a SIMD): a wave holds one sub-block's S / dP tiles instead of two, which is what
@@ -89,26 +65,6 @@ struct KvCfg {
 
 // (per head_dim, where the launch is not tiny)
 template <int D> constexpr int kUsualSplit = D == 128 ? 2 : 1;
-
-// key tile `ktile` (counted chunk by chunk): its chunk, its first row there and that row's position in the launch
-struct KeyTile {
-  int chunk, row0, key0;
-};
-__host__ __device__ inline KeyTile key_tile(const KvChunks& kv, int ktile, int BN) {
-  if (kv.count == 1) return {0, ktile * BN, ktile * BN};
-  const int per = (kv.len + BN - 1) / BN, chunk = ktile / per, row0 = (ktile - chunk * per) * BN;
-  return {chunk, row0, chunk * kv.len + row0};
-}
-// first query tile of BM queries that sees position key0
-__host__ __device__ inline int first_query_tile(const AttnParams& a, int key0, int BM) {
-  const int first_q = a.causal ? key0 - a.q_offset : 0;
-  return first_q > 0 ? first_q / BM : 0;
-}
-// trips of a key tile: (query heads of the group) x (query tiles that see it)
-__host__ __device__ inline int dkdv_trips(const AttnParams& a, int ktile, int BN, int BM) {
-  const int n = (a.Sq + BM - 1) / BM, start = first_query_tile(a, key_tile(a.kv, ktile, BN).key0, BM);
-  return n > start ? (n - start) * (a.Hq / a.Hkv) : 0;
-}
 
 // the rows of dK (kDk) and / or dV (kDv) that a wave's accumulators hold: 32 keys from row `row0` of their chunk, position
 // `key0`, through the wave's piece of LDS.  bf16 gradients are written with streaming stores: nothing on this GPU reads them
@@ -1273,6 +1229,7 @@ __global__ __launch_bounds__(256) void attn_bwd_preprocess_kernel(const __bf16* 
 // How the dK/dV launch is run: key tiles singly, in pairs, or cut into pieces.
 struct DkdvPlan {
   bool few = false;    // attn_bwd_dkdv_few_kernel
+  bool roles = false;  // attn_bwd_roles.hip
   bool pair = false;
   int len = 0;
   int64_t ws_bytes = 0;
@@ -1303,6 +1260,21 @@ DkdvPlan make_dkdv_plan(const AttnParams& a) {
   cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
   auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
   plan.len = choose_pieces(heads, n_ktiles, cost, plan.pair, trips_of);
+  // Key tiles of 256 (attn_bwd_roles.hip) where the estimate says so, by a sixth: 58 of 70 drawn launches, 0.59 to 0.99 of the time of the others and one
+  // 1.05 (B8 H6/2 S2057 without a mask); of the twelve that come closer two are 1.03 and 1.05, five 0.95 to 0.99, five 0.81 to 0.84.  (And B4 H16 S1100
+  // causal, which comes to 0.844, stays bit for bit equal to its halves.)  Few workgroups lose, and are cut: B1 H32 S1024 28.6 us, 46.4 so; B1 H32 S2048
+  // causal, one round of unequal lengths, 71.8 and 92.9.  A trip (64 queries) takes 2.6 us with half of the GPU idle and 3.15 with all of it busy.
+  if constexpr (D == 128) {
+    using R = RoleTiles;
+    auto role_trips = [&](int i) { return dkdv_trips(a, i, R::BN, R::BM); };
+    const double us = launch_us(heads, n_ktiles, cost, plan.len, plan.len == 0 && plan.pair, trips_of);
+    const double roles_us = launch_us(heads, tiles_before(a.kv, a.Sk, R::BN), {2.6, 3.15, 1.0, R::kPerCu, 0.0}, 0, false, role_trips);
+    if (roles_us < 0.84 * us) {
+      plan = DkdvPlan();
+      plan.roles = true;
+      return plan;
+    }
+  }
   if (plan.len > 0) plan.ws_bytes = static_cast<int64_t>(heads * count_pieces(n_ktiles, plan.len, trips_of) * cost.piece_bytes);
   return plan;
 }
@@ -1336,6 +1308,9 @@ int launch_dkdv(const BwdParams& p, float* ws, int64_t ws_bytes, hipStream_t s) 
       hipLaunchKernelGGL(attn_bwd_dkdv_few_kernel, dim3(p.a.Hkv * p.a.B, tiles_before(p.a.kv, p.a.Sk, F::BN)), dim3(F::kThreads), F::kLdsBytes, s, q);
       return PICO_OK;
     }
+  }
+  if constexpr (D == 128) {
+    if (plan.roles) return launch_dkdv_roles(p, s);
   }
   const int n_ktiles = tiles_before(p.a.kv, p.a.Sk, C::BN);
   BwdParams q = p;
@@ -1687,6 +1662,17 @@ extern "C" int64_t pico_attn_bwd_workspace_bytes(const pico_attn_desc* desc, int
   if (!plan_params(desc, chunk_count, a)) return 0;
   const int64_t dkdv = desc->D == 64 ? plan_dkdv<64>(a).ws_bytes : plan_dkdv<128>(a).ws_bytes;
   return std::max(dkdv, plan_dq(a, desc->D).ws_bytes);   // (the two kernels run one after the other)
+}
+
+extern "C" int pico_attn_dkdv_plan(const pico_attn_desc* desc, int chunk_count, int32_t* out) {
+  if (!out) return fail(PICO_ERR_NULL, "pico_attn_dkdv_plan: the plan is NULL");
+  AttnParams a;
+  if (!plan_params(desc, chunk_count, a)) return fail(PICO_ERR_SHAPE, "pico_attn_dkdv_plan: no launch for this descriptor");
+  const DkdvPlan& plan = desc->D == 64 ? plan_dkdv<64>(a) : plan_dkdv<128>(a);
+  out[0] = plan.roles ? RoleTiles::BN : plan.few ? KvCfg<64, 4>::BN : 128;
+  out[1] = plan.pair && plan.len == 0 ? 2 : 1;
+  out[2] = plan.len;
+  return PICO_OK;
 }
 
 extern "C" int pico_attn_dq_plan(const pico_attn_desc* desc, int chunk_count, int32_t* out) {

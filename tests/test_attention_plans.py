@@ -19,6 +19,18 @@ def plan(which, B, H, Sq, Sk, causal, q_offset, D=128, Hkv=None):
     return tuple(out)
 
 
+def dkdv_plan(B, H, Sq, Sk, causal, q_offset, D=128, Hkv=None, chunks=1):
+    """(keys of a key tile, key tiles of a workgroup, trips of a piece)"""
+    from picotron_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here (python -m picotron_amd.build)")
+    d = _lib.AttnDesc()
+    d.B, d.Hq, d.Hkv, d.Sq, d.Sk, d.D, d.causal, d.q_offset, d.sm_scale = B, H, Hkv or H, Sq, Sk, D, int(causal), q_offset, D ** -0.5
+    out = (ctypes.c_int32 * 3)()
+    _lib.check(_lib.lib().pico_attn_dkdv_plan(ctypes.byref(d), chunks, out))
+    return tuple(out)
+
+
 # (B, H, Sq, Sk, causal, q_offset), workgroups of 256 queries and of 128, waves of the forward, waves of dQ
 LINES = [
     ((1, 32, 1792, 1792, True, 0), 224, 448, 4, 4),         # under one round
@@ -79,3 +91,17 @@ def test_a_descriptor_without_a_launch_has_no_plan():
                 plan(which, *sizes)
         with pytest.raises(RuntimeError, match="no launch"):
             plan(which, 1, 4, 64, 64, True, 0, D=96)
+
+
+@pytest.mark.parametrize("sizes,kv_heads,want", [   # us of key tiles of 128 (as planned without the other kernel) and of 256
+    ((1, 32, 2048, 2048, False, 0), 32, (256, 1, 0)),       # 129, 111: one round of equal ones
+    ((1, 32, 2048, 2048, True, 0), 32, (128, 2, 0)),        # 72, 93: of unequal ones
+    ((1, 32, 4096, 4096, True, 0), 32, (256, 1, 0)),        # 243, 220
+    ((3, 32, 777, 777, True, 0), 32, (256, 1, 0)),          # 64, 44
+    ((1, 32, 1024, 1024, False, 0), 32, (128, 1, 0)),       # 36, 50: half a round
+    ((2, 32, 1531, 1531, True, 0), 8, (128, 1, 48)),        # 90, 95 uncut: few workgroups
+    ((3, 16, 2769, 2769, False, 0), 16, (128, 1, 0)),       # 383, 396: just over two rounds
+    ((4, 32, 1281, 1281, True, 0), 32, (256, 1, 0)),       # (as drawn: 0.85 of the time)
+])
+def test_key_tiles_at_head_dim_128(sizes, kv_heads, want):
+    assert dkdv_plan(*sizes, Hkv=kv_heads) == want

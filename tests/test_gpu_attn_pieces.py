@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import layers as OL
-from test_attention_plans import plan
+from test_attention_plans import dkdv_plan, plan
 from test_gpu_sweep import reference, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -255,3 +255,57 @@ def test_gradients_leave_unrotated_and_added_at_head_dim_128(device, B, Hq, Hkv,
         turned = b if i == 2 else torch.cat((lo * c + hi * s, hi * c - lo * s), -1)
         size = (lo.abs() + hi.abs()).repeat(1, 1, 1, 2) + base.abs()
         assert ((a - (base + turned)).abs() <= 9 * 2 ** -24 * size).all(), i
+
+
+# dK/dV at head_dim 128 in key tiles of 256, whose waves have dV or dK of 64 keys, 16 of every 64
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,W,Sc,causal,q_offset", [
+    (8, 32, 32, 97, 1, 129, False, 0),       # keys that end in the third block of 64 of some waves and the second of others
+    (8, 32, 32, 200, 1, 193, False, 0),
+    (8, 32, 32, 256, 1, 256, False, 0),
+    (3, 32, 32, 777, 1, 777, True, 0),       # every number of blocks on the diagonal, ragged ends of both
+    (4, 16, 16, 922, 1, 922, False, 0),
+    (8, 32, 32, 128, 1, 512, True, 384),     # queries behind the keys
+    (16, 16, 8, 300, 1, 520, True, 219),     # two query heads to a walk, a diagonal that no block begins on
+    (16, 32, 16, 150, 1, 200, False, 0),
+    (13, 20, 10, 520, 1, 600, True, 80),
+    (8, 32, 8, 257, 2, 449, True, 641),      # chunks that end inside key tiles
+])
+def test_key_tiles_of_256(device, B, Hq, Hkv, Sq, W, Sc, causal, q_offset):
+    """Gradients against the fp32 reference of a batch and kv head at a time, with the bound of bf16 operands; then the forms that a
+    chunk's gradients leave in: added to fp32 sums, their rounded total, not at all."""
+    from picotron_amd import ops
+    assert dkdv_plan(B, Hq, Sq, W * Sc, causal, q_offset, Hkv=Hkv, chunks=W)[0] == 256
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, W * Sc, 128)
+    scale, group = 1 / math.sqrt(128), Hq // Hkv
+    ks, vs = ([c.contiguous() for c in t.chunk(W, dim=2)] for t in (k, v))
+    out, lse, _ = ops.attn_fwd_chunks(q, ks, vs, scale, causal, q_offset)
+
+    def run(make, **more):
+        dks, dvs = [make() for _ in range(W)], [make() for _ in range(W)]
+        ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, causal, q_offset, dks=dks, dvs=dvs, out=out, **more)
+        return dks, dvs
+
+    dks, dvs = run(lambda: torch.full_like(ks[0], float("nan"), dtype=torch.float32))
+    for b in range(0, B, 5):
+        for h in range(0, Hkv, 7):
+            part = slice(h * group, (h + 1) * group)
+            want = reference(q[b:b + 1, part], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], scale, q_offset, causal, do[b:b + 1, part])
+            for got, w in ((torch.cat(dks, 2), want[3]), (torch.cat(dvs, 2), want[4])):
+                assert rel_l2(got[b:b + 1, h:h + 1], w) <= 1e-2, (b, h)
+                for r in range(0, W * Sc, 64):
+                    assert rel_l2(got[b:b + 1, h:h + 1, r:r + 64], w[:, :, r:r + 64]) <= 2e-2 or w[:, :, r:r + 64].norm() < 0.05 * w.norm(), (b, h, r)
+    base = torch.randn(ks[0].shape, generator=torch.Generator(device="cuda").manual_seed(1), device=device)
+    added = run(base.clone, dkv_accumulate=[True] * W)
+    for got, one in zip(added[0] + added[1], dks + dvs):
+        assert torch.equal(got, base + one)
+    totals = [torch.empty_like(t) for t in ks], [torch.empty_like(t) for t in ks]
+    kept = run(base.clone, dkv_accumulate=[True] * W, dk_finals=totals[0], dv_finals=totals[1])
+    for total, got, read in zip(totals[0] + totals[1], added[0] + added[1], kept[0] + kept[1]):
+        assert torch.equal(total, got.to(torch.bfloat16)) and torch.equal(read, base)
+    rounded = run(lambda: torch.empty_like(ks[0]))
+    for got, one in zip(rounded[0] + rounded[1], dks + dvs):
+        assert torch.equal(got, one.to(torch.bfloat16))
+    if W > 1:
+        some = [None, torch.empty_like(dks[1])], [None, torch.empty_like(dks[1])]
+        ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, causal, q_offset, dks=some[0], dvs=some[1], out=out)
+        assert torch.equal(some[0][1], dks[1]) and torch.equal(some[1][1], dvs[1])

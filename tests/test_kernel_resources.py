@@ -207,3 +207,12 @@ def test_streaming_optimizer_kernels_store_past_the_caches():
         assert sum(" nt" in line for line in loads) == (3 * len(loads) // 4 if streams else 0), name
         seen += 1
     assert seen == 24   # one and many tensors, streaming or not, six combinations of types
+
+
+def test_the_kernel_of_two_roles_fits_a_cu():
+    """Eight waves share a CU, with no register in scratch memory and no LDS of their own (its requests count from 0)."""
+    kernels = compiled(csrc("attn_bwd_roles.hip"))[0]
+    assert len(kernels) == 1
+    for name, r in kernels.items():
+        assert "attn_bwd_roles_kernel" in name and r["Occupancy"] >= 2
+        assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0 and r["LDS Size"] == 0, (name, r)
