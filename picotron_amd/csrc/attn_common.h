@@ -811,26 +811,9 @@ struct KvPosition {
   }
 };
 
-// A launch's first workgroups find none of its arguments in the caches, and the compiler loads them where they are used, line after line with a wait
-// for each.  These request one word of every line that a launch of one chunk uses, together; the loads that follow hit.  Forward, dQ, dK/dV alone, us:
-// B4 H32 256 x 1024 D64 15.3 -> 14.8, 18.0 -> 17.7, 25.3 -> 23.6; B2 H9/3 S256 D64 5.9 -> 5.7, 6.5 -> 6.3, 11.5 -> 11.1; B4 H32 S1024 D64 27.4 ->
-// 26.3, 36.8 -> 36.4, 42.7 -> 42.6.  (All 18 lines of the backward's arguments, or loads that the compiler may move behind others, gain less, and the
-// forward lost up to 4 %.)  kAt: offsets of what lies 64 bytes or more from the one before.
-template <int... kAt>
-struct Arguments {
-  uint32_t word[sizeof...(kAt)];
-  __device__ __forceinline__ Arguments() {
-    const auto* args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int at[] = {kAt...};
-#pragma unroll
-    for (int i = 0; i < static_cast<int>(sizeof...(kAt)); ++i) word[i] = args[at[i] / 4];
-  }
-  __device__ __forceinline__ void arrive() const {   // (what keeps the loads)
-#pragma unroll
-    for (int i = 0; i < static_cast<int>(sizeof...(kAt)); ++i) asm volatile("" ::"s"(word[i]));
-    __builtin_amdgcn_sched_barrier(0);
-  }
-};
+// The arguments of a launch of one chunk (see Arguments).  Forward, dQ, dK/dV alone, us: B4 H32 256 x 1024 D64 15.3 -> 14.8, 18.0 -> 17.7, 25.3 -> 23.6;
+// B2 H9/3 S256 D64 5.9 -> 5.7, 6.5 -> 6.3, 11.5 -> 11.1; B4 H32 S1024 D64 27.4 -> 26.3, 36.8 -> 36.4, 42.7 -> 42.6.  (All 18 lines of the backward's
+// arguments, or loads that the compiler may move behind others, gain less, and the forward lost up to 4 %.)
 using AttnArguments = Arguments<0, offsetof(AttnParams, kv.v), offsetof(AttnParams, kv.count), offsetof(AttnParams, kv.count) + 64, sizeof(AttnParams) + 4>;
 
 int check_attn_desc(const char* fn, const pico_attn_desc* d);

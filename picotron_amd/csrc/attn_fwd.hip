@@ -99,7 +99,9 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
+  const Arguments<sizeof(FwdParams) - 4> rope;
   AttnArguments().arrive();
+  rope.arrive();
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
   // key tiles that the queries of a tile see (the last of a head's query tiles comes first in the order below)

@@ -148,4 +148,21 @@ inline bool reserve_lds_once(LdsOnce& once, const void* kernel, size_t bytes) {
   return true;
 }
 
+// A launch's first workgroups find none of its arguments in the caches, and the compiler loads them where they are used, line after line with a wait
+// for each.  These request one word of every line, together; the loads that follow hit.  kAt: offsets of what lies 64 bytes or more from the one before.
+template <int... kAt>
+struct Arguments {
+  uint32_t word[sizeof...(kAt)];
+  __device__ __forceinline__ Arguments() {
+    const auto* args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int at[] = {kAt...};
+#pragma unroll
+    for (int i = 0; i < static_cast<int>(sizeof...(kAt)); ++i) word[i] = args[at[i] / 4];
+  }
+  __device__ __forceinline__ void arrive() const {   // (what keeps the loads)
+#pragma unroll
+    for (int i = 0; i < static_cast<int>(sizeof...(kAt)); ++i) asm volatile("" ::"s"(word[i]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
 }  // namespace pico

@@ -48,6 +48,7 @@ __global__ __launch_bounds__(kFwdThreads) void rmsnorm_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y, float* __restrict__ rstd,
     const T* __restrict__ res_in, T* __restrict__ res_out, int64_t rows, int hidden, float eps,
     int cast_then_scale) {
+  Arguments<0, 64>().arrive();
   constexpr int V = io<T>::kVec;
   __shared__ float smem[8];
   const int gid = threadIdx.x / G;
@@ -407,6 +408,7 @@ template <typename T, typename TW, int NV, bool kRes>
 __global__ __launch_bounds__(kFewThreads) void rmsnorm_bwd_few_kernel(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ rstd, const T* dres, T* dx,
     TW* __restrict__ dweight, int rows, int hidden, int dw_blocks) {
+  Arguments<0, 64>().arrive();
   constexpr int V = io<T>::kVec;
   auto unpack = [](const u32x4& raw, float (&out)[V]) {
     if constexpr (V == 8) {

@@ -21,6 +21,7 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(
     const T* __restrict__ x, T* __restrict__ y, const TT* __restrict__ cos_t, const TT* __restrict__ sin_t,
     int64_t total, int H, int S, int D, int64_t xsb, int64_t xsh, int64_t xss, int64_t ysb, int64_t ysh,
     int64_t yss, int64_t table_ld, int64_t pos_offset, int inverse, int s_outer) {
+  Arguments<0, 64>().arrive();
   constexpr int V = io<T>::kVec;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (idx >= total) return;
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_kernel(const T* __restric
                                                               T* __restrict__ dup, int64_t total, int vpr,
                                                               int64_t dyld, int64_t gld, int64_t uld, int64_t dgld,
                                                               int64_t duld) {
+  Arguments<0, 64>().arrive();
   constexpr int V = io<T>::kVec;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (idx >= total) return;
