@@ -931,9 +931,16 @@ struct DqWave<D, true> {   // lane = queries lane % 16 and 16 + lane % 16, regis
         dp_acc[kb][qb] = f32x4{-delta[qb], -delta[qb], -delta[qb], -delta[qb]};   // dP - delta comes out of the MFMA
       }
     }
+    // Fragment i of S and dP: which 16 keys, which 32 columns.  S goes through one 16 keys after the other, so that exp2 can begin early; dP, which dS
+    // waits for by 32 keys, takes two 16 keys of the same columns in turn and the queries of the second the other way round, so that the fragment of dO stays
+    // (an operand that does not change takes less power).  us, dP like S and so: B1 H32 S4096 161.0, 160.1; 4096 queries and 32768 keys with 32 / 8 heads
+    // 2180, 2152; B8 H32 S1024 no mask 181.3, 179.5; 17 launches, 14 of them drawn, 0.981 to 1.001 of the time, 0.993 over all.  (S like dP, with exp2 six
+    // MFMAs later, 2134.8 -> 2146.1 in the second of these; the queries of dQ's products there and back, level.)
+    auto keys_of = [](int i) constexpr { return i < 2 * kSteps ? i / (D / 32) : i % (2 * kSteps) / kSteps * 2 + i % 2; };
+    auto step_of = [](int i) constexpr { return i < 2 * kSteps ? i % (D / 32) : i % kSteps / 2; };
     auto fetch = [&](int i) {
       const int j = i % (2 * kSteps);   // fragment of its product
-      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * (j / kSteps)) + j % kSteps / (D / 32) * L::kRows16 + L::column16(j % (D / 32)) * 2));
+      if (i < 4 * kSteps) from[i] = lds_at<bf16x8>((i < 2 * kSteps ? row_lane : v_row_lane) + (kAt + L::rows(32 * (keys_of(i) / 2)) + keys_of(i) % 2 * L::kRows16 + L::column16(step_of(i)) * 2));
       else from[i] = lds_tr16_at<D>(tr_lane + (kAt + L::rows(32 * (j / kSteps)) + j % kSteps * 32));
     };
     // element e of a lane's 32: 16 keys, 16 queries, key
@@ -951,8 +958,9 @@ struct DqWave<D, true> {   // lane = queries lane % 16 and 16 + lane % 16, regis
     for (int i = 0; i < kAhead; ++i) fetch(i);
     __builtin_amdgcn_sched_barrier(0);
     each_load<2 * kAll>([&](auto which) __attribute__((always_inline)) {   // the MFMAs: every fragment has one for each 16 queries
-      constexpr int m = decltype(which)::value, i = m / 2, qb = m % 2, j = i % (2 * kSteps), kb = j / (D / 32), s = j % (D / 32);
-      if constexpr (qb == 0 && i + kAhead < kAll) fetch(i + kAhead);
+      constexpr int m = decltype(which)::value, i = m / 2, j = i % (2 * kSteps), kb = keys_of(i), s = step_of(i);
+      constexpr int qb = i >= 2 * kSteps && i < 4 * kSteps && i % 2 ? 1 - m % 2 : m % 2;
+      if constexpr (m % 2 == 0 && i + kAhead < kAll) fetch(i + kAhead);
       if constexpr (i < 2 * kSteps) s_acc[kb][qb] = mfma16(from[i], qf[qb][s], s_acc[kb][qb]);
       else if constexpr (i < 4 * kSteps) dp_acc[kb][qb] = mfma16(from[i], dof[qb][s], dp_acc[kb][qb]);
       else dq[j % kSteps][qb] = mfma16(from[i], dsf[j / kSteps * 2 + qb], dq[j % kSteps][qb]);
