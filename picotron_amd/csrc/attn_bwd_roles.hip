@@ -292,8 +292,13 @@ __device__ __forceinline__ void role_walk(const BwdParams& p, const KeyTile& at,
         if constexpr (db == 2) move_on();
         if constexpr (db == 6) tr_at += rows;
         if constexpr (db == 6 && kDk) first_fetch();
+        // (key blocks there and back: from each product to the next one operand stays.  17 launches 0.998 of the time, 4096 queries and 32768 keys with
+        // 32 / 8 heads 3060 -> 3045 us)
 #pragma unroll
-        for (int kb = 0; kb < kKb; ++kb) acc[db][kb] = mfma16(tr[db], __builtin_bit_cast(bf16x8, right[kb]), acc[db][kb]);
+        for (int to = 0; to < kKb; ++to) {
+          const int kb = db % 2 ? kKb - 1 - to : to;
+          acc[db][kb] = mfma16(tr[db], __builtin_bit_cast(bf16x8, right[kb]), acc[db][kb]);
+        }
         __builtin_amdgcn_sched_barrier(0);
       });
     }
