@@ -932,8 +932,8 @@ struct DqWave<D, true> {   // lane = queries lane % 16 and 16 + lane % 16, regis
       }
     }
     // Fragment i of S and dP: which 16 keys, which 32 columns.  S goes through one 16 keys after the other, so that exp2 can begin early; dP, which dS
-    // waits for by 32 keys, takes two 16 keys of the same columns in turn and the queries of the second the other way round, so that the fragment of dO stays
-    // (an operand that does not change takes less power).  us, dP like S and so: B1 H32 S4096 161.0, 160.1; 4096 queries and 32768 keys with 32 / 8 heads
+    // waits for by 32 keys, takes two 16 keys of the same columns in turn and the queries of the second the other way round, so that a sum's products are four
+    // MFMAs apart instead of two and the fragment of dO stays (in the second launch below 1.5 % fewer cycles).  us, dP like S and so: B1 H32 S4096 161.0, 160.1; 4096 queries and 32768 keys with 32 / 8 heads
     // 2180, 2152; B8 H32 S1024 no mask 181.3, 179.5; 17 launches, 14 of them drawn, 0.981 to 1.001 of the time, 0.993 over all.  (S like dP, with exp2 six
     // MFMAs later, 2134.8 -> 2146.1 in the second of these; the queries of dQ's products there and back, level.)
     auto keys_of = [](int i) constexpr { return i < 2 * kSteps ? i / (D / 32) : i % (2 * kSteps) / kSteps * 2 + i % 2; };
