@@ -1268,10 +1268,12 @@ DkdvPlan make_dkdv_plan(const AttnParams& a) {
   cost.piece_bytes = 4.0 * C::kKeyWaves * dkdv_piece_floats(D);
   auto trips_of = [&](int i) { return dkdv_trips(a, i, C::BN, C::BM); };
   plan.len = choose_pieces(heads, n_ktiles, cost, plan.pair, trips_of);
-  // Key tiles of 256 (attn_bwd_roles.hip) where the estimate says so, by a sixth: 58 of 70 drawn launches, 0.59 to 0.99 of the time of the others and one
-  // 1.05 (B8 H6/2 S2057 without a mask); of the twelve that come closer two are 1.03 and 1.05, five 0.95 to 0.99, five 0.81 to 0.84.  (And B4 H16 S1100
-  // causal, which comes to 0.844, stays bit for bit equal to its halves.)  Few workgroups lose, and are cut: B1 H32 S1024 28.6 us, 46.4 so; B1 H32 S2048
-  // causal, one round of unequal lengths, 71.8 and 92.9.  A trip (64 queries) takes 2.6 us with half of the GPU idle and 3.15 with all of it busy.
+  // Key tiles of 256 (attn_bwd_roles.hip) where the estimate says so, by a sixth: the line lies under the first launch that loses.  Of 115 launches whose estimate
+  // is under the others' (113 of them drawn), the 72 below the line take 0.69 to 0.993 of the time of the others, 0.86 in the mean.  The first above it is at
+  // 0.844 and loses (B8 H6/2 S2057 without a mask 263 -> 269 us; B4 H16 S1100 causal, at 0.844 too, would gain, 63 -> 58), and from there to 1 so do 16 of 43, up to
+  // 1.06 (0.96 in the mean: masked and unmasked trips have one price here, and an estimate that tells them apart could take more).  Few workgroups lose, and are cut: B1
+  // H32 S1024 28.6 us, 46.4 so; B1 H32 S2048 causal, one round of unequal lengths, 71.8 and 92.9.  A trip (64 queries) takes 2.6 us with half of the GPU idle and 3.15 with
+  // all of it busy.
   if constexpr (D == 128) {
     using R = RoleTiles;
     auto role_trips = [&](int i) { return dkdv_trips(a, i, R::BN, R::BM); };

@@ -105,3 +105,11 @@ def test_a_descriptor_without_a_launch_has_no_plan():
 ])
 def test_key_tiles_at_head_dim_128(sizes, kv_heads, want):
     assert dkdv_plan(*sizes, Hkv=kv_heads) == want
+
+
+def test_key_tiles_of_128_where_the_estimates_are_close():
+    """Both just above the line (0.844): one that the other kernel would slow down, 263 -> 269 us, and one that is compared bit for bit with
+    its halves as paired and single key tiles of one kernel."""
+    assert dkdv_plan(8, 6, 2057, 2057, False, 0, Hkv=2) == (128, 1, 48)
+    assert dkdv_plan(4, 16, 1100, 1100, True, 0) == (128, 2, 0)
+    assert dkdv_plan(2, 16, 1100, 1100, True, 0) == (128, 1, 0)
