@@ -309,3 +309,83 @@ def test_key_tiles_of_256(device, B, Hq, Hkv, Sq, W, Sc, causal, q_offset):
         some = [None, torch.empty_like(dks[1])], [None, torch.empty_like(dks[1])]
         ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, causal, q_offset, dks=some[0], dvs=some[1], out=out)
         assert torch.equal(some[0][1], dks[1]) and torch.equal(some[1][1], dvs[1])
+
+
+# ... whose last tiles have 9, 76 and 200 rows: ends in a wave's first, second and fourth block of 16, the rows n and n + 64 that leave together
+@pytest.mark.parametrize("B,Hq,Hkv,S,waves", [(3, 32, 32, 777, 4), (5, 16, 16, 1100, 4), (6, 16, 16, 968, 4), (8, 32, 16, 712, 8)])
+def test_gradients_leave_unrotated_and_added_in_key_tiles_of_256(device, B, Hq, Hkv, S, waves):
+    assert dkdv_plan(B, Hq, S, S, True, 0, Hkv=Hkv) == (256, 1, 0)
+    test_gradients_leave_unrotated_and_added_at_head_dim_128(device, B, Hq, Hkv, S, waves)
+
+
+def test_chunks_in_key_tiles_of_256_leave_unrotated(device):
+    """Chunks that end inside key tiles: the rotation's backward on the fp32 results (eight roundings of products of two elements of a pair, and
+    the sum's), and the rounded totals are those sums rounded."""
+    from picotron_amd import ops
+    B, Hq, Hkv, Sq, W, Sc, offset, k_first = 8, 32, 8, 257, 2, 449, 641, 7
+    assert dkdv_plan(B, Hq, Sq, W * Sc, True, offset, Hkv=Hkv, chunks=W) == (256, 1, 0)
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, W * Sc, 128)
+    scale = 1 / math.sqrt(128)
+    ks, vs = ([c.contiguous() for c in t.chunk(W, dim=2)] for t in (k, v))
+    cos, sin = (t.to(device) for t in OL.get_cos_sin(W * Sc + k_first, 128, 10000.0, torch.float32))
+    out, lse, _ = ops.attn_fwd_chunks(q, ks, vs, scale, True, offset)
+
+    def run(make, **more):
+        dks, dvs = [make() for _ in range(W)], [make() for _ in range(W)]
+        ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, True, offset, dks=dks, dvs=dvs, out=out, **more)
+        return dks, dvs
+
+    plain = run(lambda: torch.empty(ks[0].shape, device=device))
+    base = torch.randn(ks[0].shape, generator=torch.Generator(device="cuda").manual_seed(1), device=device)
+    turning = dict(rope=(cos, sin), q_pos_offset=offset, k_pos_offset=k_first, dkv_accumulate=[True] * W)
+    added = run(base.clone, **turning)
+    for c in range(W):
+        at = slice(k_first + c * Sc, k_first + (c + 1) * Sc)
+        lo, hi = plain[0][c][..., :64], plain[0][c][..., 64:]
+        turned = torch.cat((lo * cos[at, :64] + hi * sin[at, :64], hi * cos[at, :64] - lo * sin[at, :64]), -1)
+        size = (lo.abs() + hi.abs()).repeat(1, 1, 1, 2) + base.abs()
+        assert ((added[0][c] - (base + turned)).abs() <= 9 * 2 ** -24 * size).all(), c
+        assert torch.equal(added[1][c], base + plain[1][c]), c
+    totals = [torch.empty_like(t) for t in ks], [torch.empty_like(t) for t in ks]
+    run(base.clone, dk_finals=totals[0], dv_finals=totals[1], **turning)
+    for total, got in zip(totals[0] + totals[1], added[0] + added[1]):
+        assert torch.equal(total, got.to(torch.bfloat16))
+
+
+def test_key_tiles_of_256_that_no_query_sees(device):
+    """Nine of them, and the last blocks of the one before: zeros where the gradients are written, what was there where they are added; the others against
+    the fp32 reference."""
+    from picotron_amd import ops
+    B, H, Sq, Sk, q_offset = 8, 8, 1201, 3782, 100
+    assert dkdv_plan(B, H, Sq, Sk, True, q_offset) == (256, 1, 0)
+    q, k, v, do = inputs(device, B, H, H, Sq, Sk, 128)
+    scale, seen = 1 / math.sqrt(128), q_offset + Sq
+    out, lse = ops.attn_fwd(q, k, v, scale, True, q_offset)
+    dk, dv = (torch.full(k.shape, float("nan"), device=device) for _ in range(2))
+    dq, _, _ = ops.attn_bwd(do, q, k, v, lse, None, scale, True, q_offset, None, dk, dv, out=out)
+    assert (dk[:, :, seen:] == 0).all() and (dv[:, :, seen:] == 0).all()
+    for b, h in ((0, 0), (B // 2, H - 1), (B - 1, 3)):
+        want = reference(*(t[b:b + 1, h:h + 1] for t in (q, k, v)), scale, q_offset, True, do[b:b + 1, h:h + 1])
+        for got, w in ((dq, want[2]), (dk, want[3]), (dv, want[4])):
+            assert rel_l2(got[b:b + 1, h:h + 1], w) <= 1e-2, (b, h)
+    base = torch.randn(k.shape, generator=torch.Generator(device="cuda").manual_seed(1), device=device)
+    added = base.clone(), base.clone()
+    ops.attn_bwd(do, q, k, v, lse, None, scale, True, q_offset, None, *added, out=out, dkv_accumulate=True)
+    assert torch.equal(added[0], base + dk) and torch.equal(added[1], base + dv)
+
+
+def test_rows_without_keys_in_key_tiles_of_256(device):
+    """Rows whose lse is -inf add nothing, as rows without a gradient do: bit for bit."""
+    from picotron_amd import ops
+    B, H, S = 3, 32, 777
+    assert dkdv_plan(B, H, S, S, True, 0) == (256, 1, 0)
+    q, k, v, do = inputs(device, B, H, H, S, S, 128)
+    scale = 1 / math.sqrt(128)
+    out, lse = ops.attn_fwd(q, k, v, scale, True, 0)
+    rows = torch.zeros(S, dtype=torch.bool, device=device)
+    rows[[0, 31, 776]] = True
+    rows[100:175] = True
+    got = ops.attn_bwd(do, q, k, v, lse.masked_fill(rows, -math.inf), None, scale, True, 0, out=out)
+    want = ops.attn_bwd(do.masked_fill(rows[:, None], 0.0), q, k, v, lse, None, scale, True, 0, out=out)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
