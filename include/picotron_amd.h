@@ -199,8 +199,10 @@ int pico_attn_bwd_preprocess(const pico_attn_desc* desc, const void* dout, const
 
 /* replaces: ring_attention_backward  context_parallel.py:130-155 and the fp32 accumulation of
  *           RingAttentionFunc.backward  context_parallel.py:85-93.
- * Two kernels are enqueued: dK/dV (one workgroup per 128 keys) and dQ (one workgroup per query tile);
- * neither uses atomics, so results are deterministic.
+ * Two kernels are enqueued: dK/dV (a workgroup owns 64, 128 or 256 keys) and dQ (one workgroup per query tile);
+ * neither uses atomics: equal calls give equal bits.  Which kernels a call gets, and whether they cut their tiles, follows from
+ * all sizes of the descriptor, the batch among them (pico_attn_*_plan), and their fp32 sums have other orders: a batch and its
+ * parts in calls of their own agree to rounding, not bit for bit.
  * lse, delta: [B,Hq,Sq] fp32 (lse is the FINAL merged lse, as in the reference).
  * dq:     [B,Hq,Sq,D] addressed by dq_stride (element strides for b, h, s, multiples of 4; NULL = contiguous);
  *         dq_dtype PICO_F32 with dq_accumulate = 1 adds into the buffer (the running sum over ring steps),

@@ -389,3 +389,20 @@ def test_rows_without_keys_in_key_tiles_of_256(device):
     want = ops.attn_bwd(do.masked_fill(rows[:, None], 0.0), q, k, v, lse, None, scale, True, 0, out=out)
     for x, y in zip(got, want):
         assert torch.equal(x, y)
+
+
+def test_a_batch_and_its_halves_at_head_dim_128(device):
+    """The whole batch and its halves go to other kernels of dQ and of dK/dV, whose sums of 128 products have other orders: they differ by under 2^-17 of
+    themselves, so that at most one value of P and dS in 2^9 is rounded to bf16 the other way, by at most 2^-7 of it: 2^-11.5 in rel. L2."""
+    from picotron_amd import ops
+    B, H, S = 8, 32, 1100
+    assert plan("dq", B, H, S, S, True, 0)[0] == 8 and plan("dq", B // 2, H, S, S, True, 0)[0] == 4
+    assert dkdv_plan(B, H, S, S, True, 0) == (128, 2, 0) and dkdv_plan(B // 2, H, S, S, True, 0) == (256, 1, 0)
+    q, k, v, do = inputs(device, B, H, H, S, S, 128)
+    scale = 1 / math.sqrt(128)
+    out, lse = ops.attn_fwd(q, k, v, scale, True, 0)
+    whole = ops.attn_bwd(do, q, k, v, lse, None, scale, True, 0, out=out)
+    for half in (slice(0, B // 2), slice(B // 2, B)):
+        part = ops.attn_bwd(do[half], q[half], k[half], v[half], lse[half], None, scale, True, 0, out=out[half])
+        for x, y in zip(whole, part):
+            assert rel_l2(y, x[half]) <= 2 ** -11.5
