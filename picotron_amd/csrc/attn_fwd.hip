@@ -99,9 +99,16 @@ __global__ __launch_bounds__(64 * NW, (FwdCfg<D, QB, NW, KT, KS>::kPerCu * NW / 
   constexpr int BM = C::BM, BN = C::BN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
-  const Arguments<sizeof(FwdParams) - 4> rope;
-  AttnArguments().arrive();
-  rope.arrive();
+  // (whole tiles at head_dim 64 leave the rotation's line out: us of launches behind each other, with it and without, B2 H9/3 S256 6.08, 6.02, rotated 7.07,
+  // 7.00, B8 H3 S1314 15.47, 15.33; replayed from a graph, whose arguments stay in the caches, 5.50, 5.45, and 5.45 without any of this.  The others gain by it:
+  // head_dim 128 B4 H1 S153 7.22, 7.17, B8 H2 S182 7.40, 7.34; cut at head_dim 64 B2 H1 S5778 29.83, 29.72)
+  if constexpr (D == 128 || kCut) {
+    const Arguments<sizeof(FwdParams) - 4> rope;
+    AttnArguments().arrive();
+    rope.arrive();
+  } else {
+    AttnArguments().arrive();
+  }
   const AttnParams& a = p.a;
   const int n_qtiles = (a.Sq + BM - 1) / BM;
   // key tiles that the queries of a tile see (the last of a head's query tiles comes first in the order below)
