@@ -8,9 +8,10 @@
 //
 // What this split gives over waves that have all four products of 32 keys (attn_bwd_dkdv_kernel_d128), us: B1 H32 S4096 causal 239 -> 216, 4096 queries and
 // 32768 keys with 32 / 8 heads 3470 -> 3010, B8 H32 S1024 without a mask 279 -> 240, B3 H32 S777 64 -> 44; 70 drawn launches 0.874 of the time.
-// LDS: 34 reads and 4 writes of 16 bytes (counting a transposing pair as one) for 64 MFMAs of 16 x 16 x 32, where there were 57 for 32 of twice the
-// work each; products of 16 x 16 x 32 take a seventh less power (see DqWave).  The clock rose from 1.77 to 2.2 GHz by it, at 0.55 of the cycles with the
-// matrix pipe busy instead of 0.60: what is left is the length of the two waves' own chains, 2700 and 2400 of a step's 3400 cycles when the other wave does
+// LDS: 22 reads and 4 writes of 16 bytes (a transposing pair is one) for 64 MFMAs of 16 x 16 x 32, 34 instructions, where there were 49 reads, 65 instructions,
+// for 32 of twice the work each; products of 16 x 16 x 32 take a seventh less power (see DqWave).  For 4096 queries and 32768 keys the clock rose from 1.77 to 2.16 GHz
+// by it (dQ, whose matrix pipe is fuller, 1.88), with the matrix pipe busy for 0.61 of the cycles instead of 0.65: what is left is the length of the two waves' own
+// chains, 2700 and 2400 of a step's 3400 cycles when the other wave does
 // nothing (LDS latency behind the barrier 100 to 180, exp2 and what waits for P 1000 to 1300, dV or dK 600, the step's scalar work 160).
 // Taken out one at a time from B8 H32 S1024, us: P's way through LDS 250 -> 231, exp2 243, requests 216, most of dV and dK 194.
 // Two bodies in turn for the halves of a tile, or a branch between them, spill: the walk has 256 registers and needs 250 to 256 in every form.
@@ -331,7 +332,7 @@ __device__ __forceinline__ void role_walk(const BwdParams& p, const KeyTile& at,
     first_fetch();
   }
   while (true) {
-    const int end = min(2 * walk.n_qtiles, u + 2 * left + 2);   // (heads and pieces begin and end with a tile)
+    const int end = min(2 * walk.n_qtiles, u + 2 * left + 2);   // (a head begins and ends with a tile)
     steps(std::integral_constant<int, 0>(), std::true_type(), min(from_step(1), end));
     steps(std::integral_constant<int, 1>(), std::true_type(), min(from_step(2), end));
     steps(std::integral_constant<int, 2>(), std::true_type(), min(from_step(3), end));
