@@ -1,4 +1,4 @@
-// Pieces shared by the attention forward and backward kernels (gfx950, wave64, MFMA 32x32x16 bf16).
+// Pieces shared by the attention forward and backward kernels (gfx950, wave64, MFMA 32x32x16 and 16x16x32 bf16).
 //
 // MFMA 32x32x16 operand layout (verified on hardware): lane l, half h = l / 32, n = l % 32
 //   A[m][k]  : lane holds m = n, k = 8h .. 8h+7          (8 bf16)
@@ -8,6 +8,13 @@
 // C tile can be fed back as the k-operand of the next MFMA straight from registers: registers
 // 8c .. 8c+7 of a lane hold rows {16c + 8jj + 4h + t : jj < 2, t < 4}, and the partner operand is
 // fetched with that same row order.
+//
+// MFMA 16x16x32: lane l, group g = l / 16, n = l % 16
+//   A[m][k]  : lane holds m = n, k = 8g .. 8g+7          (8 bf16)
+//   B[k][n]  : lane holds n,     k = 8g .. 8g+7          (8 bf16)
+//   C[m][n]  : lane holds column n, register i holds row 4g + i                   (4 fp32)
+// Two C tiles' registers are 8 slots k of the next product, 4 rows of the one and 4 of the other.  Which row and which columns of a tile in
+// LDS stand for m and k is TileLayout's (group_row, column16 and group_column, the same in A and B).
 //
 // ds_read_b64_tr_b16 (verified on hardware): within a group of 16 lanes, lane p supplies the address
 // of 4 consecutive 16-bit elements; lane p receives element p%4 of lanes {p/4, 4 + p/4, 8 + p/4, 12 + p/4}.
@@ -208,10 +215,6 @@ __device__ __forceinline__ float half_sum(float v) {
 }
 
 // ... across the four groups of 16 lanes (lanes l, l^16, l^32, l^48)
-__device__ __forceinline__ float group_max(float v) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return half_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
-}
 __device__ __forceinline__ float group_sum(float v) {
   auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return half_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
@@ -271,7 +274,7 @@ struct WaveTile {
 //   accumulate (fp32 only) adds to what is there; all its reads are issued before the first write.
 //   streaming marks bf16 stores non-temporal (the data is not read again by the kernels that follow soon).
 constexpr int kRowRegionBytes = 32 * 144;
-// columns c0 .. c0 + kCols - 1 of the 32 rows, scaled, to the wave's piece of LDS
+// four columns of a row, scaled, to the wave's piece of LDS
 template <bool kF32>
 __device__ __forceinline__ void put_columns(unsigned char* region, int row, int col, f32x4 v4, float scale) {
   if constexpr (kF32) {
@@ -283,6 +286,7 @@ __device__ __forceinline__ void put_columns(unsigned char* region, int row, int 
     *reinterpret_cast<bf16x4*>(region + row * 144 + col * 2) = b4;
   }
 }
+// columns c0 .. c0 + kCols - 1 of the 32 rows
 template <bool kF32, int kCols, int N>   // products of 32 x 32
 __device__ __forceinline__ void put_rows(unsigned char* region, const f32x16 (&acc)[N], float scale, int c0, int lane) {
 #pragma unroll
