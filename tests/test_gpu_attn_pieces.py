@@ -406,3 +406,31 @@ def test_a_batch_and_its_halves_at_head_dim_128(device):
         part = ops.attn_bwd(do[half], q[half], k[half], v[half], lse[half], None, scale, True, 0, out=out[half])
         for x, y in zip(whole, part):
             assert rel_l2(y, x[half]) <= 2 ** -11.5
+
+
+# dQ of eight waves at head_dim 128 in pieces: 264 and 288 workgroups, over a round of one per CU, beside over 8192 keys
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,W,Sc,q_offset", [(11, 12, 1, 274, 2, 4199, 8124), (9, 16, 1, 262, 1, 8413, 8151)])
+def test_dq_of_eight_waves_in_pieces_at_head_dim_128(device, B, Hq, Hkv, Sq, W, Sc, q_offset):
+    """Against the fp32 reference of a batch at a time, with the bound of bf16 operands; un-rotated and added, equal to the two on that result: eight
+    roundings of products of two elements of a pair, and the sum's."""
+    from picotron_amd import _lib, ops
+    q, k, v, do = inputs(device, B, Hq, Hkv, Sq, W * Sc, 128)
+    scale = 1 / math.sqrt(128)
+    ks, vs = ([c.contiguous() for c in t.chunk(W, dim=2)] for t in (k, v))
+    how = (ctypes.c_int32 * 3)()
+    _lib.check(_lib.lib().pico_attn_dq_plan(ctypes.byref(ops._chunk_desc(q, ks, vs, q, scale, True, q_offset)), W, how))
+    assert how[0] == 8 and how[2] > 0
+    out, lse, _ = ops.attn_fwd_chunks(q, ks, vs, scale, True, q_offset)
+    dq = torch.full(q.shape, float("nan"), device=device)
+    ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, True, q_offset, dq=dq, dks=[None] * W, dvs=[None] * W, out=out)
+    for b in (0, B // 2, B - 1):
+        want = reference(*(t[b:b + 1] for t in (q, k, v)), scale, q_offset, True, do[b:b + 1])[2]
+        for r in range(0, Sq, 32):
+            assert rel_l2(dq[b:b + 1, :, r:r + 32], want[:, :, r:r + 32]) <= 1e-2, (b, r)
+    cos, sin = (t.to(device) for t in OL.get_cos_sin(W * Sc + 5, 128, 10000.0, torch.float32))
+    base = torch.randn(q.shape, generator=torch.Generator(device="cuda").manual_seed(3), device=device)
+    got = base.clone()
+    ops.attn_bwd_chunks(do, q, ks, vs, lse, scale, True, q_offset, dq=got, dks=[None] * W, dvs=[None] * W, out=out, rope=(cos, sin), q_pos_offset=5, dq_accumulate=True)
+    c, s, lo, hi = cos[5:5 + Sq, :64], sin[5:5 + Sq, :64], dq[..., :64], dq[..., 64:]
+    size = (lo.abs() + hi.abs()).repeat(1, 1, 1, 2) + base.abs()
+    assert ((got - (base + torch.cat((lo * c + hi * s, hi * c - lo * s), -1))).abs() <= 9 * 2 ** -24 * size).all()
